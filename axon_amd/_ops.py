@@ -843,7 +843,7 @@ class HeadBlocks:
     """One step of the head as blocks of consecutive tokens (``axon_lmhead_block_*``): forward of a block over
     the whole vocabulary with a stash, then (by the caller) the loss on the block's positions, then the block's
     backward from the stash, then the next block.  Holds the step's operands and everything the blocks share:
-    the stash and the workspaces (sized for the largest block, allocated once), the transposed weight, the
+    the stash and the workspaces (sized for the largest block, allocated once), the
     fp32 accumulator of the weight gradient, and the whole-stream outputs.
 
     ``hidden`` ``[N, H]`` and ``weight`` ``[V, H]`` bf16; ``labels`` ``[N]`` (with ``seq_start``: the packed id
@@ -885,7 +885,7 @@ class HeadBlocks:
             raise _lib.AxonAmdError(f"HeadBlocks: unsupported shape tokens={n_max} hidden={self.h} vocab={self.v}")
         self.fwd_ws = torch.empty(self.fwd_ws_bytes, device=dev, dtype=torch.uint8)
         self.bwd_ws = torch.empty(self.bwd_ws_bytes, device=dev, dtype=torch.uint8)
-        self.stash_bytes = max(lmhead_stash_bytes(b - a, self.h, self.v) for a, b in self.ranges) if stash else 0
+        self.stash_bytes = self._stash_bytes(n_max) if stash else 0
         self.stash = torch.empty(self.stash_bytes, device=dev, dtype=torch.uint8) if self.stash_bytes else None
         self.stats = torch.empty(2, n_max, device=dev, dtype=torch.float32)  # lse, entropy_b of the current block
         # whole-stream outputs; position 0 is a sequence start (the aligned layout writes it from the last row)
@@ -895,7 +895,6 @@ class HeadBlocks:
         self.one_block = self.n_groups == 1  # one weight-gradient GEMM: no partial sums to carry
         self.dw_acc_bytes = 0 if self.one_block else int(self.lib.axon_lmhead_block_dw_acc_bytes(self.h, self.v))
         self.dw_acc = torch.empty(self.dw_acc_bytes // 4, device=dev, dtype=torch.float32) if self.dw_acc_bytes else None
-        self.wt_ready = False
         self.block_stash_bytes = 0
         self.workspace_bytes = self.fwd_ws_bytes + self.bwd_ws_bytes + self.stash_bytes + self.dw_acc_bytes
 
@@ -906,6 +905,9 @@ class HeadBlocks:
     @property
     def entropy(self):
         return self.out[1][: self.n]
+
+    def _stash_bytes(self, n):
+        return int(self.lib.axon_lmhead_block_stash_bytes(n, self.h, self.v))
 
     def _block(self, k):
         n0, n1 = self.ranges[k]
@@ -922,7 +924,7 @@ class HeadBlocks:
         stream reaches the point after the call."""
         n0, n1, last_dst = self._block(k)
         nb = n1 - n0
-        self.block_stash_bytes = lmhead_stash_bytes(nb, self.h, self.v) if self.stash is not None else 0
+        self.block_stash_bytes = self._stash_bytes(nb) if self.stash is not None else 0
         check(self.lib.axon_lmhead_block_fwd(
             self.hidden.data_ptr() + n0 * self.h * 2, ptr(self.weight), self._at(self.labels, n0),
             int(self.labels.dtype == torch.int64), nb, self.h, self.v, self.inv_t, self.softcap,
@@ -943,10 +945,6 @@ class HeadBlocks:
             raise ValueError("HeadBlocks.backward: dentropy must be a contiguous fp32 array over the whole stream")
         st = stream_ptr()
         th = self.timing.handle if self.timing else None
-        if not self.wt_ready:
-            check(self.lib.axon_lmhead_block_begin(ptr(self.weight), self.h, self.v, self.chunk, ptr(self.bwd_ws),
-                                                   self.bwd_ws_bytes, st, th), "axon_lmhead_block_begin")
-            self.wt_ready = True
         group, pos, dw_now = self.place[k]
         mode = (DW_STORE if self.one_block else DW_FIRST if group == 0
                 else DW_LAST if group == self.n_groups - 1 else DW_ADD)

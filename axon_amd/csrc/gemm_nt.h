@@ -18,17 +18,22 @@
 // TFLOP/s), which is worth more than the larger block's operand reuse.
 //
 // Two main loops:
-//  * DmaLoopT<kAT, kBT>, DmaLoop = DmaLoopT<false, false>  (the fast path; needs
-//      m_rows >= 256, n_rows >= 256, k % 64 == 0; kAT / kBT: that side is K-major)
+//  * DmaLoopT<kAT, kBT>, DmaLoop = DmaLoopT<false, false>  (the fast path; any number of
+//      rows; k % 64 == 0 where a side is K-contiguous; kAT / kBT: that side is K-major)
 //      global -> LDS by `buffer_load_dwordx4 ... lds` (no VGPR staging), 32 KB
 //      slots of 256 x 64 bf16 (three for A, two for B), 16-byte chunks
 //      XOR-swizzled by row; fragment reads for k-step kk+1 are issued under the
-//      MFMAs of k-step kk; A is fetched two k-tiles ahead, B one.  Edge tiles are
-//      shifted back inside the matrix (uniform addressing, no per-lane clamps);
-//      the rows that then belong to the neighbouring tile are masked by the
-//      epilogue through `m_lo` / `n_lo`.
-//  * RegLoop<32>  (any shape with k % 32 == 0): loads through registers with
-//      per-row clamping.  Used for small or odd shapes.
+//      MFMAs of k-step kk; A is fetched two k-tiles ahead, B one.  Rows of an edge
+//      tile beyond the matrix (and k-rows of a K-major operand beyond its last one)
+//      read as zeros: the buffer descriptor of each operand ends with the tile's last
+//      valid row, and a load beyond it lands as 0 in LDS without touching memory
+//      (uniform addressing, no per-lane clamps, and no smallest matrix).
+//      Shifting edge tiles back inside the matrix instead needed 256 rows on both
+//      sides (a forward over 187 tokens, 896 x 151936, ran on RegLoop: 355 us per call
+//      against 108 now) and token counts in fours for the head's stash (16381 tokens,
+//      2880 x 201088: half of a step recomputed its logits, 51.2 ms against 45.4 now).
+//  * RegLoop<32>  (k % 64 == 32, which the 64-wide k-tiles above do not divide):
+//      loads through registers with per-row clamping.
 //
 // Accumulator layout of one 16x16 block (four floats, index r):
 //   m = 4*(lane/16) + r,   n = lane%16.
@@ -60,11 +65,10 @@ struct GemmOperands {
   int k;               // reduction length
 };
 
-// Where a workgroup's tile sits.  (m0, n0) is the first row/column actually
-// computed; rows with tile-relative index < m_lo (columns < n_lo) duplicate the
-// previous tile and must be ignored by the epilogue.
+// Where a workgroup's tile sits: its first row / column.  Rows of an edge tile beyond the matrix
+// hold zeros (DmaLoop) or the last valid row's values (RegLoop) and are dropped by the epilogue.
 struct TilePos {
-  int m0, n0, m_lo, n_lo;
+  int m0, n0;
 };
 
 // Position of this lane inside the workgroup tile.
@@ -132,6 +136,13 @@ struct DmaSide {
   int vo[kVariants];   // per-lane source byte offset of a DMA instruction, by variant(j)
   int step;            // source bytes from DMA instruction j to j + 1
   int64_t kt_bytes;    // source bytes from one k-tile to the next
+  // Bytes from a k-tile's first element to the end of what belongs to this tile; the descriptor's size: loads
+  // beyond it land as zeros.  K-contiguous: the tile's valid rows (the row stride covers a whole k-tile, so
+  // the limit is the same for every k-tile).  K-major: the k-rows of the k-tile, of which the last may have
+  // fewer than 64 (`rec_last`, which ends with the matrix's last column, rounded up to a 16-byte vector: ld is a
+  // multiple of 8).  What a K-major side reads beyond the matrix's last COLUMN elsewhere is the next k-row: values
+  // of rows that the epilogue drops.
+  int rec, rec_last;
   const __bf16* base;  // the tile's first element of k-tile 0
   int frag[kFrag];     // per-lane fragment offsets inside a slot: by k-step (row-major) or by block (K-major)
 
@@ -142,8 +153,8 @@ struct DmaSide {
   // what is left to add per read (the slot: a scalar; block, k-step, half: constants) fits the 16-bit offset
   // field of the LDS instructions: a constant beyond it costs a vector addition right before the read that
   // needs its result, and every such pair delays the MFMA behind it.
-  __device__ __forceinline__ void init(const __bf16* p, int64_t ld, int row0, int sub, const LanePos& lp,
-                                       int lds_base) {
+  __device__ __forceinline__ void init(const __bf16* p, int64_t ld, int rows, int k, int row0, int sub,
+                                       const LanePos& lp, int lds_base) {
     if (!T) {
       // One DMA instruction fills 1 KB of LDS = 8 rows x 128 B; wave w owns rows [64w, 64w+64) of the
       // operand (8 instructions).  Lane i lands on row i/8, chunk slot i%8, and therefore fetches
@@ -157,6 +168,7 @@ struct DmaSide {
       step = (int)ld * 16;
       kt_bytes = 128;
       base = p + (int64_t)row0 * ld;
+      rec = rec_last = min(rows - row0, kTile) * (int)ld * 2;
       // fragment addressing: row = 128*sub + 16*i + l16, chunk = 4*kk + lq, swizzle = (l16/2)%8.
       // Sixteen lanes (one chunk column of sixteen rows) cover all 64 banks once.
       const int sw = (lp.l16 >> 1) & 7;
@@ -177,6 +189,8 @@ struct DmaSide {
       step = (int)ld * 4;
       kt_bytes = (int64_t)ld * 128;
       base = p + row0;
+      rec = (int)ld * 128;
+      rec_last = ((k - 1) & 63) * (int)ld * 2 + (rows - row0 + 7) / 8 * 16;
       // fragment of block i, k-step kk, half h: k-row 32kk + 8lq + 4h + l16/4, elements
       // 128*sub + 16i + 4*(l16%4) ..+3: granule 16*sub + 2i + (l16%4)/2, second half of it for odd l16.
       const int s15 = (2 * (lp.l16 >> 2) + 8 * lp.lq) & 15;
@@ -186,37 +200,26 @@ struct DmaSide {
       for (int i = 0; i < kBlocks; ++i) frag[i] = lds_base + fb + ((i << 5) ^ (s15 << 4));
     }
   }
-  // source byte offset of k-tile kt; past the end: refetches the last tile, never consumed
-  __device__ __forceinline__ int64_t k_off(int kt, int kt_n) const { return (int64_t)min(kt, kt_n - 1) * kt_bytes; }
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_at(int64_t ko) const {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)(reinterpret_cast<const char*>(base) + ko), 0, 0x7fffffff,
-                                             0x00020000);
+  // k-tile kt as a descriptor; past the end: the last tile again, never consumed
+  __device__ __forceinline__ const char* k_ptr(int kt, int kt_n) const {
+    return reinterpret_cast<const char*>(base) + (int64_t)min(kt, kt_n - 1) * kt_bytes;
+  }
+  __device__ __forceinline__ int k_rec(int kt, int kt_n) const { return (T && kt >= kt_n - 1) ? rec_last : rec; }
+  __device__ static __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const char* p, int rec) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, rec, 0x00020000);
   }
 };
 
-template <bool kAT, bool kBT>
+// kNarrow: the K-major A operand's rows are shorter than 512 bytes (see dma_kb).
+template <bool kAT, bool kBT, bool kNarrow = false>
 struct DmaLoopT {
   static constexpr int kBK = 64;
   static constexpr int kRowBytes = 128;
   static constexpr int kOperandBytes = kTile * kRowBytes;  // 32 KB
   static constexpr int kBBase = 3 * kOperandBytes;         // A slots at 0/32/64 KB, B slots at 96/128 KB
-  static constexpr bool kShiftsEdgeTiles = true;
   static constexpr int kReadsA = kAT ? 2 : 1, kReadsB = kBT ? 2 : 1;  // LDS reads per fragment
 
-  __device__ static __forceinline__ bool supports(const GemmOperands& g) {
-    return g.m_rows >= kTile && g.n_rows >= kTile && (g.k % kBK) == 0;
-  }
-
-  // Edge tiles are shifted back inside the matrix; the epilogue skips the duplicated rows.
-  __device__ static __forceinline__ TilePos place(const GemmOperands& g, int tm, int tn) {
-    TilePos t;
-    const int m0 = tm * kTile, n0 = tn * kTile;
-    t.m0 = min(m0, g.m_rows - kTile);
-    t.n0 = min(n0, g.n_rows - kTile);
-    t.m_lo = m0 - t.m0;
-    t.n_lo = n0 - t.n0;
-    return t;
-  }
+  __device__ static __forceinline__ TilePos place(int tm, int tn) { return TilePos{tm * kTile, tn * kTile}; }
 
   // One DMA instruction: 16 bytes per lane, LDS destination = lds + IMM + 16 * lane
   // (wave-contiguous), memory source = base + voffset + soffset + IMM.  The instruction's immediate
@@ -230,6 +233,9 @@ struct DmaLoopT {
   // instruction j of an operand tile (the wave's j-th kilobyte of the slot): lds = tile base of the wave
   __device__ static __forceinline__ void dma_kb(__amdgpu_buffer_rsrc_t rsrc, int voffset, int step_bytes,
                                                 char* lds, int j) {
+    // With rows shorter than what one instruction steps over in LDS the offset below would be negative, which
+    // the descriptor's bounds do not allow: one M0 value per instruction then.
+    if (kNarrow) return dma16<0>(rsrc, voffset, j * step_bytes, lds + j * 1024);
     char* const l = lds + (j >> 2) * 4096;
     const int so = j * step_bytes - (j & 3) * 1024;
     switch (j & 3) {
@@ -263,8 +269,8 @@ struct DmaLoopT {
     const LanePos lp;
     DmaSide<kAT> sa;
     DmaSide<kBT> sb;
-    sa.init(g.a, g.lda, t.m0, lp.wm, lp, 0);
-    sb.init(g.b, g.ldb, t.n0, lp.wn, lp, kBBase);
+    sa.init(g.a, g.lda, g.m_rows, g.k, t.m0, lp.wm, lp, 0);
+    sb.init(g.b, g.ldb, g.n_rows, g.k, t.n0, lp.wn, lp, kBBase);
     // wave-uniform, so the LDS destination of every DMA instruction is scalar arithmetic into M0
     char* const dst = smem + __builtin_amdgcn_readfirstlane(lp.wave) * 8192;
 
@@ -272,7 +278,7 @@ struct DmaLoopT {
     // fragments of two k-steps: whole (one 16-byte read) or as the two halves of a transpose read
     bf16x8 af[2][kBlocks], bf[2][kBlocks];
     i16x4 aft[2][kBlocks][2], bft[2][kBlocks][2];
-    const int kt_n = g.k / kBK;
+    const int kt_n = (g.k + kBK - 1) / kBK;
     auto dma_a = [&](int slot_off, const __amdgpu_buffer_rsrc_t& r, int j) {
       dma_kb(r, sa.vo[DmaSide<kAT>::variant(j)], sa.step, dst + slot_off, j);
     };
@@ -357,12 +363,14 @@ struct DmaLoopT {
 
     // prologue: tiles 0 and 1 whole (A slots 0, 1; B slots 0, 1)
     {
-      const __amdgpu_buffer_rsrc_t ra = sa.rsrc_at(0), rb = sb.rsrc_at(0);
+      const __amdgpu_buffer_rsrc_t ra = sa.rsrc_of(sa.k_ptr(0, kt_n), sa.k_rec(0, kt_n));
+      const __amdgpu_buffer_rsrc_t rb = sb.rsrc_of(sb.k_ptr(0, kt_n), sb.k_rec(0, kt_n));
 #pragma unroll
       for (int j = 0; j < 8; ++j) dma_a(0, ra, j);
 #pragma unroll
       for (int j = 0; j < 8; ++j) dma_b(0, rb, j);
-      const __amdgpu_buffer_rsrc_t ra1 = sa.rsrc_at(sa.k_off(1, kt_n)), rb1 = sb.rsrc_at(sb.k_off(1, kt_n));
+      const __amdgpu_buffer_rsrc_t ra1 = sa.rsrc_of(sa.k_ptr(1, kt_n), sa.k_rec(1, kt_n));
+      const __amdgpu_buffer_rsrc_t rb1 = sb.rsrc_of(sb.k_ptr(1, kt_n), sb.k_rec(1, kt_n));
 #pragma unroll
       for (int j = 0; j < 8; ++j) dma_a(kOperandBytes, ra1, j);
 #pragma unroll
@@ -392,15 +400,13 @@ struct DmaLoopT {
     auto next_a_slot = [](int slot) { return (slot == 2 * kOperandBytes) ? 0 : slot + kOperandBytes; };
     auto pin = [](auto& x) { asm volatile("" : "+s"(x)); };
     int a_nxt = kOperandBytes, a_fill = 2 * kOperandBytes, b_cur = 0;
-    const char* pa = reinterpret_cast<const char*>(sa.base) + sa.k_off(2, kt_n);
-    const char* pb = reinterpret_cast<const char*>(sb.base) + sb.k_off(2, kt_n);
-    auto rsrc_of = [](const char* p) {
-      return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000);
-    };
+    const char* pa = sa.k_ptr(2, kt_n);
+    const char* pb = sb.k_ptr(2, kt_n);
+    int rec_a = sa.k_rec(2, kt_n), rec_b = sb.k_rec(2, kt_n);
     auto k_tile = [&](int kt) {
       // first k-step: A of tile kt+2; the fragments of this tile's second k-step are read (the addresses stand
       // for this tile's slots), then the addresses move on to the next tile's slots
-      step(1, 0, a_fill, I8{}, 0, I0{}, rsrc_of(pa), [](auto) {}, std::integral_constant<int, kLateAdr ? 1 : 0>{},
+      step(1, 0, a_fill, I8{}, 0, I0{}, sa.rsrc_of(pa, rec_a), [](auto) {}, std::integral_constant<int, kLateAdr ? 1 : 0>{},
            a_nxt, b_cur ^ kOperandBytes);
       // second k-step: tile kt+1 must have landed for every wave (the eight younger instructions are
       // A of tile kt+2) and every wave must be done reading this tile's B slot before it is refilled
@@ -413,13 +419,22 @@ struct DmaLoopT {
         for (int q = 0; q < kAddrB; ++q) set_adr_b(q, b_cur ^ kOperandBytes);
       }
       const bool more = kt + 3 < kt_n;  // else: past the end, the last tile is fetched again and never consumed
-      step(0, 1, 0, I0{}, b_cur, I8{}, rsrc_of(pb),
+      const bool whole = kt + 4 < kt_n;  // K-major: k-tile kt+3 is not the last one
+      step(0, 1, 0, I0{}, b_cur, I8{}, sb.rsrc_of(pb, rec_b),
            [&](auto part) {
              constexpr int kPart = decltype(part)::value;
              if (kPart == 0) { a_nxt = next_a_slot(a_nxt); pin(a_nxt); }
              if (kPart == 1) { a_fill = next_a_slot(a_nxt); pin(a_fill); }
-             if (kPart == 2) { pa += more ? sa.kt_bytes : 0; pin(pa); }
-             if (kPart == 3) { pb += more ? sb.kt_bytes : 0; pin(pb); }
+             if (kPart == 2) {
+               pa += more ? sa.kt_bytes : 0;
+               pin(pa);
+               if (kAT) { rec_a = whole ? sa.rec : sa.rec_last; pin(rec_a); }
+             }
+             if (kPart == 3) {
+               pb += more ? sb.kt_bytes : 0;
+               pin(pb);
+               if (kBT) { rec_b = whole ? sb.rec : sb.rec_last; pin(rec_b); }
+             }
              if (kPart == 4) { b_cur ^= kOperandBytes; pin(b_cur); }
            },
            I0{}, 0, 0);
@@ -457,9 +472,7 @@ struct RegLoop {
     return row * kRowBytes + ((chunk ^ sw) << 4);
   }
 
-  __device__ static __forceinline__ TilePos place(const GemmOperands&, int tm, int tn) {
-    return TilePos{tm * kTile, tn * kTile, 0, 0};
-  }
+  __device__ static __forceinline__ TilePos place(int tm, int tn) { return TilePos{tm * kTile, tn * kTile}; }
 
   __device__ static __forceinline__ void run(const GemmOperands& g, const TilePos& t, AccTile& acc,
                                              char* smem) {

@@ -7,13 +7,12 @@
 // Backward   per vocab chunk:
 //   B1  recompute the logits tile (or decode the forward's stash), form dlogit in
 //       registers, write it as bf16 dl[token][vocab];
-//   B2  dHidden[token][h] (+)= sum_v dl[token][v]  * WT[h][v]
+//   B2  dHidden[token][h] (+)= sum_v dl[token][v]  * W[v][h]
 //   B3  dWeight[v][h]      =  sum_t dl[t][v]       * hiddenT[h][t]
-// WT and hiddenT are bf16 transposes made once per call: B2 runs on the
-// K-contiguous main loop of gemm_nt.h, B3 on its variant that reads dl, K-major
-// for this product, as it lies.  Shapes that variant does not take (hidden < 256,
-// a vocabulary that is no multiple of 8) get a second, vocab-major copy
-// dlT[vocab][token] from B1 and the K-contiguous loop.
+// hiddenT is a bf16 transpose made once per call.  B2 reads the weight and B3 reads
+// dl as they lie, K-major for these products (gemm_nt.h).  Small hidden sizes and
+// vocabularies that are no multiple of 8 get a second, vocab-major copy
+// dlT[vocab][token] from B1 for B3.
 #include "common.h"
 #include "gemm_nt.h"
 #include <vector>
@@ -55,8 +54,7 @@ struct FwdParams {
 // gradient.  Each wavefront's 128 x 128 sub-tile is stored in accumulator order, 16 bytes per lane
 // and store (two 16-row blocks), every store one contiguous kilobyte:
 //   uint4 index = ((tile * 4 + wave) * 32 + j * 4 + i / 2) * 64 + lane,   tile = tm * tiles_n + tn.
-// Elements that do not count in their tile (duplicates of the neighbouring tile, rows beyond the
-// matrix) are stored as 0 and never read.
+// Vocabulary rows beyond the matrix are stored as 0.
 constexpr int64_t kStashTileBytes = 131072;
 constexpr int kStashWaveVecs = 2048;  // uint4 per wavefront sub-tile
 
@@ -110,8 +108,7 @@ __device__ __forceinline__ float rows_all_reduce(float v, Op op) {
 }
 
 // Fold one 256x256 logits tile into per-token partials.  MASKED: some rows of the tile
-// do not count (beyond the vocabulary, or duplicates of the neighbouring tile); they are
-// excluded by predicate — their accumulators hold finite values.  STASH: also store every
+// lie beyond the vocabulary; they are excluded by predicate — their accumulators hold finite values.  STASH: also store every
 // 2^(y - M) for the backward (`stash_wave`: this wavefront's 32 KB, already offset by the lane).
 template <bool MASKED, bool STASH>
 __device__ __forceinline__ void fwd_epilogue(AccTile& acc, const FwdParams& p, const LanePos& lp,
@@ -125,7 +122,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTile& acc, const FwdParams& p, c
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int mr = lp.m(i, r);
-        const bool ok = !MASKED || (mr >= t.m_lo && t.m0 + mr < p.vocab);
+        const bool ok = !MASKED || t.m0 + mr < p.vocab;
         mx = ok ? fmaxf(mx, acc[i][j][r]) : mx;
       }
     // the four lanes that hold the same token (lane ^ 16, lane ^ 32) share one reference
@@ -139,7 +136,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTile& acc, const FwdParams& p, c
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int mr = lp.m(i, r);
-        const bool ok = !MASKED || (mr >= t.m_lo && t.m0 + mr < p.vocab);
+        const bool ok = !MASKED || t.m0 + mr < p.vocab;
         const float y = fmaf(acc[i][j][r], p.c, -M);  // scaled logit relative to the max, <= 0
         w[r] = ok ? fast_exp2(y) : 0.f;
         s += w[r];
@@ -163,7 +160,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTile& acc, const FwdParams& p, c
     e = rows_all_reduce(e, [](float a, float b) { return a + b; });
     const int nr = lp.n(j);
     const int n = t.n0 + nr;
-    if (lp.lq == 0 && nr >= t.n_lo && n < p.n_tokens) {
+    if (lp.lq == 0 && n < p.n_tokens) {
       const int64_t o = (int64_t)part * p.n_tokens + n;
       p.pm[o] = M;
       p.ps[o] = s;
@@ -179,7 +176,7 @@ __device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams&
   extern __shared__ __align__(16) char smem[];
   int tm, tn;
   tile_coords<8>(tiles_m, tiles_n, tm, tn);
-  const TilePos t = Loop::place(g, tm, tn);
+  const TilePos t = Loop::place(tm, tn);
   AccTile acc;
   Loop::run(g, t, acc, smem);
   if (SOFTCAP) {
@@ -193,7 +190,7 @@ __device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams&
   const LanePos lp;
   uint4* const stash_wave =
       STASH ? p.stash + ((int64_t)(tm * tiles_n + tn) * 4 + lp.wave) * kStashWaveVecs + lp.lane : nullptr;
-  if (t.m_lo > 0 || t.m0 + kTile > p.vocab)
+  if (t.m0 + kTile > p.vocab)
     fwd_epilogue<true, STASH>(acc, p, lp, t, tm, stash_wave);
   else
     fwd_epilogue<false, STASH>(acc, p, lp, t, tm, stash_wave);
@@ -439,7 +436,6 @@ __device__ __forceinline__ void dlogit_stage(AccTile& acc, const DlogitParams& p
         float v = pr * fmaf(k.cb, raw, k.ca);
         if (mrel == k.lab_rel) v += k.gl;
         if (SOFTCAP) v *= dcap;
-        // rows shared with the neighbouring tile keep their (identical) values
         d[r] = (!MASKED || mrel < m_end) ? v : 0.f;
       }
       uint2 w;
@@ -453,8 +449,8 @@ __device__ __forceinline__ void dlogit_stage(AccTile& acc, const DlogitParams& p
 // The same from a forward's stash (see StashLayout above FwdParams): softmax = w * 2^(M - lse), scaled
 // logit = log2(w) + M.  One call covers 64 tokens (four 16-token blocks, j0 .. j0 + 3) x 128 vocabulary
 // rows of a wavefront's sub-tile; staged row = token - 16 * j0.  SOFTCAP: the stash describes the capped
-// logit, whose derivative factor is 1 - (capped / cap)^2.  EDGE: entries that do not count in this tile
-// are staged as zeros.
+// logit, whose derivative factor is 1 - (capped / cap)^2.  EDGE: entries beyond the last token or the last
+// vocabulary row are staged as zeros.
 constexpr int kStashHalfBlocks = kBlocks / 2;
 template <bool SOFTCAP, bool EDGE>
 __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashHalfBlocks], int j0,
@@ -469,7 +465,7 @@ __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashH
     const TokenCoef k(p, t.n0 + nr, (int64_t)p.v_begin + t.m0);
     const float Mp = pm[(int64_t)part * p.n_tokens + k.nn];
     const float scale = fast_exp2(Mp - k.lse2);
-    const bool n_counts = !EDGE || (k.n_ok && nr >= t.n_lo);
+    const bool n_counts = !EDGE || k.n_ok;
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
       const uint4 q = st[jl * 4 + (i >> 1)];
@@ -488,7 +484,7 @@ __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashH
           const float th = raw * p.inv_cap;
           v *= fmaf(-th, th, 1.f);
         }
-        const bool ok = !EDGE || (n_counts && mrel >= t.m_lo && p.v_begin + t.m0 + mrel < p.vocab);
+        const bool ok = !EDGE || (n_counts && p.v_begin + t.m0 + mrel < p.vocab);
         d[r] = ok ? v : 0.f;
       }
       uint2 w;
@@ -502,20 +498,16 @@ __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashH
 // A staged 64 x 128 half sub-tile (tokens 16 * j0 .. of the wavefront's sub-tile) -> dl and dlT.  Token-major
 // as in dlogit_copy_out (below); vocab-major: sixteen lanes cover the 64 tokens of one vocabulary row (one
 // 128-byte line), the four lane groups take units u, u + 8, u + 16, u + 24, whose permuted slots differ in
-// a bit that the rows' swizzles (a set with that bit fixed) cannot cancel.  EDGE: entries that duplicate the
-// neighbouring tile (tile-relative token < n_lo, vocabulary row < m_lo; both multiples of 4) are left to it.
-template <bool EDGE>
+// a bit that the rows' swizzles (a set with that bit fixed) cannot cancel.
 __device__ __forceinline__ void dlogit_copy_out_half(const char* stage, int j0, const DlogitParams& p,
                                                      const LanePos& lp, const TilePos& t) {
   const int l32 = lp.lane & 31, lhi = lp.lane >> 5;
   const int m_base = t.m0 + lp.wm * kWaveTile;
   const int n_base = t.n0 + lp.wn * kWaveTile + j0 * kBlk;
-  const int m_skip = t.m_lo - lp.wm * kWaveTile, n_skip = t.n_lo - lp.wn * kWaveTile - j0 * kBlk;
   {
     const int unit = l32;
     char* d = reinterpret_cast<char*>(p.dl + (int64_t)(n_base + lhi) * p.ld_dl + m_base + unit * 4);
     const int64_t dstep = p.ld_dl * 4;  // two rows of bf16
-    const bool col_ok = !EDGE || unit * 4 >= m_skip;
 #pragma unroll 1
     for (int nw0 = lhi; nw0 < kStashHalfBlocks * kBlk; nw0 += 16) {
       uint2 v[8];
@@ -523,7 +515,7 @@ __device__ __forceinline__ void dlogit_copy_out_half(const char* stage, int j0, 
       for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const uint2*>(stage + stage_off(nw0 + 2 * u, unit));
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        if (col_ok && (!EDGE || nw0 + 2 * u >= n_skip)) *reinterpret_cast<uint2*>(d) = v[u];
+        *reinterpret_cast<uint2*>(d) = v[u];
         d += dstep;
       }
     }
@@ -532,7 +524,6 @@ __device__ __forceinline__ void dlogit_copy_out_half(const char* stage, int j0, 
     const int nq = lp.lane & 15, grp = lp.lane >> 4;
     const int64_t rstep = p.ld_dlT * 2;  // one row of bf16
     char* d = reinterpret_cast<char*>(p.dlT + (int64_t)(m_base + grp * 32) * p.ld_dlT + n_base + nq * 4);
-    const bool tok_ok = !EDGE || nq * 4 >= n_skip;
 #pragma unroll 2
     for (int u8 = 0; u8 < 8; ++u8) {
       const int unit = grp * 8 + u8;
@@ -542,10 +533,8 @@ __device__ __forceinline__ void dlogit_copy_out_half(const char* stage, int j0, 
         rws[f] = *reinterpret_cast<const uint2*>(stage + stage_off(nq * 4 + f, unit));
       uint2 o[4];
       transpose_4x4_bf16(rws, o);
-      if (tok_ok && (!EDGE || unit * 4 >= m_skip)) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) *reinterpret_cast<uint2*>(d + e * rstep) = o[e];
-      }
+      for (int e = 0; e < 4; ++e) *reinterpret_cast<uint2*>(d + e * rstep) = o[e];
       d += 4 * rstep;
     }
   }
@@ -602,7 +591,7 @@ __device__ __forceinline__ void dlogit_body(const GemmOperands& g, const DlogitP
   extern __shared__ __align__(16) char smem[];
   int tm, tn;
   tile_coords(tiles_m, tiles_n, tm, tn);
-  const TilePos t = Loop::place(g, tm, tn);  // t.m0 is relative to the chunk
+  const TilePos t = Loop::place(tm, tn);  // t.m0 is relative to the chunk
   AccTile acc;
   Loop::run(g, t, acc, smem);
   __syncthreads();  // every wave is past its last main-loop LDS access
@@ -633,13 +622,12 @@ __global__ __launch_bounds__(kGemmThreads) void lmhead_dlogit_softcap_kernel(Gem
 // Backward B1 without the recompute: one wavefront per workgroup turns half (64 tokens x 128 rows) of a
 // sub-tile that a stashing forward stored into bf16 dlogits in both orientations (16 KB of LDS and few
 // registers: ten wavefronts per CU hide the latency of the loads and of the per-token operands).  A streaming kernel: 2 bytes
-// read and 4 written per logit.  Tiles are the forward's (same shifted or clamped placement), so
-// `tm0` is the forward tile row of the chunk's first vocabulary row and t.m0 is made chunk-relative
-// only after the edge tests; it is negative only for rows that the tile does not own.
+// read and 4 written per logit.  Tiles are the forward's: `tm0` is the forward tile row of the chunk's
+// first vocabulary row, and t.m0 is made chunk-relative after the edge tests.
 struct StashSource {
   const uint4* stash;
   const float* pm;
-  int tiles_n, tm0, shifted;
+  int tiles_n, tm0;
 };
 
 template <bool SOFTCAP>
@@ -647,13 +635,7 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_stash_kernel(DlogitParams p,
   __shared__ __align__(16) char stage[kStashHalfBlocks * kBlk * 256];  // 64 tokens x 128 bf16
   const int half = blockIdx.x & 1, wave = (blockIdx.x >> 1) & 3, tile = blockIdx.x >> 3;
   const int tm = src.tm0 + tile / src.tiles_n, tn = tile % src.tiles_n;
-  TilePos t{tm * kTile, tn * kTile, 0, 0};
-  if (src.shifted) {
-    t.m0 = min(t.m0, p.vocab - kTile);
-    t.n0 = min(t.n0, p.n_tokens - kTile);
-    t.m_lo = tm * kTile - t.m0;
-    t.n_lo = tn * kTile - t.n0;
-  }
+  TilePos t{tm * kTile, tn * kTile};
   LanePos lp;
   lp.wave = wave;
   lp.wm = wave >> 1;
@@ -668,16 +650,15 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_stash_kernel(DlogitParams p,
     const u32x4 x = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(sv + q * 64));
     st[q] = make_uint4(x[0], x[1], x[2], x[3]);
   }
-  const bool edge = t.m_lo > 0 || t.n_lo > 0 || t.m0 + kTile > p.vocab || t.n0 + kTile > p.n_tokens;
+  const bool edge = t.m0 + kTile > p.vocab || t.n0 + kTile > p.n_tokens;
   t.m0 -= p.v_begin;
   const int part = tm * 2 + lp.wm;
   if (edge) {
     dlogit_stage_stash<SOFTCAP, true>(st, j0, src.pm, part, p, lp, t, stage);
-    dlogit_copy_out_half<true>(stage, j0, p, lp, t);
   } else {
     dlogit_stage_stash<SOFTCAP, false>(st, j0, src.pm, part, p, lp, t, stage);
-    dlogit_copy_out_half<false>(stage, j0, p, lp, t);
   }
+  dlogit_copy_out_half(stage, j0, p, lp, t);
 }
 
 // ----------------------------------------------------------------------------
@@ -704,7 +685,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
   extern __shared__ __align__(16) char smem[];
   int tm, tn;
   tile_coords(tiles_m, tiles_n, tm, tn);
-  const TilePos t = Loop::place(g, tm, tn);
+  const TilePos t = Loop::place(tm, tn);
   AccTile acc;
   Loop::run(g, t, acc, smem);
   const LanePos lp;
@@ -737,13 +718,12 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
   for (int j = 0; j < kBlocks; ++j) {
     const int nr = lp.n(j);
     const int n = t.n0 + nr;
-    if (nr < t.n_lo || n >= p.n_valid) continue;
+    if (n >= p.n_valid) continue;
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
       const int mr = lp.m(i, 0);
       const int m = t.m0 + mr;
-      // m_valid % 4 == 0 and tile shifts are multiples of 4: a quad is all in or all out
-      if (mr < t.m_lo || m >= p.m_valid) continue;
+      if (m >= p.m_valid) continue;  // m_valid % 4 == 0: a quad is all in or all out
       float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
       if (p.out_f32) {
         float4* dst = reinterpret_cast<float4*>(p.out_f32 + (int64_t)n * p.ld_f32 + m);
@@ -806,16 +786,6 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t* __r
     }
   }
 }
-
-// zero the bf16 columns [col0, col0 + ncols) of `rows` rows (reduction padding of dl / dlT)
-__global__ __launch_bounds__(256) void zero_cols_bf16_kernel(uint16_t* p, int64_t ld, int rows,
-                                                             int col0, int ncols) {
-  const int64_t total = (int64_t)rows * ncols;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[(i / ncols) * ld + col0 + (i % ncols)] = 0;
-}
-
 
 // ----------------------------------------------------------------------------
 // Rows without an upstream gradient (prompt positions, masked or clipped tokens)
@@ -941,9 +911,10 @@ constexpr int64_t kDefaultVocabChunk = 32768;
 constexpr int64_t kAlign = 256;
 using SlowLoop = RegLoop<32>;
 
+// Leading dimensions whose byte offsets inside a tile (256 rows K-contiguous, 64 K-major) stay below 2^30
+constexpr int64_t kMaxLd = 1 << 21, kMaxLdKMajor = 1 << 23;
 inline bool dma_ok(const GemmOperands& g) {
-  return g.m_rows >= kTile && g.n_rows >= kTile && (g.k % DmaLoop::kBK) == 0 &&
-         g.lda < (1 << 21) && g.ldb < (1 << 21);  // byte offsets inside a tile stay below 2^31
+  return (g.k % DmaLoop::kBK) == 0 && g.lda < kMaxLd && g.ldb < kMaxLd;
 }
 
 template <typename K>
@@ -997,17 +968,12 @@ FwdWs fwd_ws(int64_t n, int64_t vocab, void* base) {
 struct StashWs {
   uint4* tiles;
   float* pm;
-  int tiles_m, tiles_n, shifted;
-  int64_t bytes;  // 0: this shape cannot be stashed
+  int tiles_m, tiles_n;
+  int64_t bytes;
 };
-StashWs stash_ws(int64_t n, int64_t h, int64_t v, void* base) {
+StashWs stash_ws(int64_t n, int64_t v, void* base) {
   StashWs w{};
   if (n <= 0) return w;
-  GemmOperands g{};
-  g.lda = g.ldb = h;  g.m_rows = (int)v;  g.n_rows = (int)n;  g.k = (int)h;
-  w.shifted = dma_ok(g);
-  // shifted edge tiles hand their duplicated rows to the neighbouring tile in groups of four
-  if (w.shifted && ((v % 4) != 0 || (n % 4) != 0)) return w;
   w.tiles_m = (int)(round_up(v, kTile) / kTile);
   w.tiles_n = (int)(round_up(n, kTile) / kTile);
   const int64_t tile_bytes = (int64_t)w.tiles_m * w.tiles_n * kStashTileBytes;
@@ -1016,25 +982,27 @@ StashWs stash_ws(int64_t n, int64_t h, int64_t v, void* base) {
   w.bytes = tile_bytes + round_up((int64_t)w.tiles_m * 2 * n * 4, kAlign);
   return w;
 }
+// The whole-call operator (axon_lmhead_fwd / _bwd) keeps a stash for the shapes its callers have always got
+// one for; the block entry points take any shape.
+bool stash_of_all_tokens(int64_t n, int64_t h, int64_t v) {
+  return n > 0 && (h % 64 != 0 || n < kTile || v < kTile || (n % 4 == 0 && v % 4 == 0));
+}
 
 struct BwdWs {
-  __bf16 *wT, *hT, *dl, *dlT;
+  __bf16 *hT, *dl, *dlT;
   float* dh_acc;
   int64_t v_pad, n_pad, chunk, bytes;
-  int64_t ld_v, ld_n, ld_c;  // leading dimensions of wT, hT/dlT, dl: padded by kLdPad elements
+  int64_t ld_n, ld_c;  // leading dimensions of hT/dlT, dl: padded by kLdPad elements
   int chunks;
   // The dWeight GEMM reads dl [token][vocab] as it lies, as its K-major operand: no vocab-major copy
-  // (dlT is null).  Needs the DMA loop for every chunk's GEMM and 16-byte vectors along the vocabulary.
+  // (dlT is null).
   bool dl_kmajor;
-  // The dHidden GEMM reads the weight [vocab][hidden] as it lies, as its K-major operand: no transposed
-  // copy (wT is null).  Needs the DMA loop (fewer than 256 tokens are padded to 256 with zero dlogit rows)
-  // and a reduction that ends with the weight's last row (vocab % 64 == 0).
-  bool w_kmajor;
 };
 // Rows a power of two apart land on the same L2 sets and memory channels; 128 bytes of padding
 // per row moves consecutive rows to consecutive cache lines (+5..13 % on a stand-alone GEMM with
 // power-of-two leading dimensions, within noise on the whole backward).
 constexpr int64_t kLdPad = 64;
+constexpr int64_t kMaxVocabChunk = 1 << 20;  // keeps dl's leading dimension inside kMaxLd
 // `n`: the tokens the workspace holds (one call's, or the span of a group of blocks whose weight
 // gradient is formed by one GEMM)
 BwdWs bwd_ws(int64_t n, int64_t h, int64_t vocab, int64_t chunk, void* base) {
@@ -1043,20 +1011,14 @@ BwdWs bwd_ws(int64_t n, int64_t h, int64_t vocab, int64_t chunk, void* base) {
   w.n_pad = round_up(n, kTile);
   w.chunk = (chunk <= 0) ? kDefaultVocabChunk : chunk;
   if (w.chunk > w.v_pad) w.chunk = w.v_pad;
+  if (w.chunk > kMaxVocabChunk) w.chunk = kMaxVocabChunk;
   w.chunks = (int)((vocab + w.chunk - 1) / w.chunk);
-  w.ld_v = w.v_pad + kLdPad;
   w.ld_n = w.n_pad + kLdPad;
   w.ld_c = w.chunk + kLdPad;
   const int64_t last_rows = vocab - (int64_t)(w.chunks - 1) * w.chunk;
-  w.dl_kmajor = h >= kTile && last_rows >= kTile && vocab % 8 == 0 && w.ld_n < (1 << 21) && w.ld_c < (1 << 21);
-  w.w_kmajor = h >= kTile && vocab % 64 == 0 && h < (1 << 21) && w.ld_c < (1 << 21);
+  w.dl_kmajor = h >= kTile && last_rows >= kTile && vocab % 8 == 0 && w.ld_n < kMaxLd;
   char* p = static_cast<char*>(base);
   int64_t off = 0;
-  w.wT = nullptr;
-  if (!w.w_kmajor) {
-    w.wT = reinterpret_cast<__bf16*>(p + off);
-    off += round_up(h * w.ld_v * 2, kAlign);
-  }
   w.hT = reinterpret_cast<__bf16*>(p + off);  off += round_up(h * w.ld_n * 2, kAlign);
   w.dl = reinterpret_cast<__bf16*>(p + off);  off += round_up(w.n_pad * w.ld_c * 2, kAlign);
   w.dlT = nullptr;
@@ -1129,10 +1091,10 @@ int launch_store(const GemmOperands& g, const StoreParams& sp, hipStream_t st) {
 }
 
 // The same with operands that are K-major ([k][rows], see DmaLoopT): the rows are fetched as 16-byte
-// vectors, so the row count (edge tiles are shifted back by it), the leading dimension and the base are
-// multiples of 8 elements.  The DMA loop only: the caller keeps a K-contiguous copy for other shapes.
-inline bool kmajor_ok(const void* p, int64_t ld, int rows) {
-  return rows % 8 == 0 && ld % 8 == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+// vectors, so the leading dimension and the base are multiples of 8 elements.  The DMA loop only.  A
+// K-contiguous side beside a K-major one is readable, and zero, up to the next multiple of 64 of k.
+inline bool kmajor_ok(const void* p, int64_t ld) {
+  return ld % 8 == 0 && ld < kMaxLdKMajor && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 template <class Loop>
 int launch_store_loop(const GemmOperands& g, const StoreParams& sp, hipStream_t st) {
@@ -1143,14 +1105,14 @@ int launch_store_loop(const GemmOperands& g, const StoreParams& sp, hipStream_t 
   AXON_CHECK_LAUNCH();
   return AXON_OK;
 }
-bool store_kmajor_ok(const GemmOperands& g, bool a_kmajor, bool b_kmajor) {
-  return dma_ok(g) && (!a_kmajor || kmajor_ok(g.a, g.lda, g.m_rows)) && (!b_kmajor || kmajor_ok(g.b, g.ldb, g.n_rows));
-}
 int launch_store_kmajor(const GemmOperands& g, const StoreParams& sp, bool a_kmajor, bool b_kmajor,
                         hipStream_t st) {
   if (!a_kmajor && !b_kmajor) return launch_store(g, sp, st);
-  if (!store_kmajor_ok(g, a_kmajor, b_kmajor)) return AXON_ERR_SHAPE;
+  if (b_kmajor && (g.ldb < kTile || (a_kmajor && g.lda < kTile))) return AXON_ERR_SHAPE;
+  if (!(a_kmajor ? kmajor_ok(g.a, g.lda) : g.lda < kMaxLd) || !(b_kmajor ? kmajor_ok(g.b, g.ldb) : g.ldb < kMaxLd))
+    return AXON_ERR_SHAPE;
   if (a_kmajor && b_kmajor) return launch_store_loop<DmaLoopT<true, true>>(g, sp, st);
+  if (a_kmajor && g.lda < kTile) return launch_store_loop<DmaLoopT<true, false, true>>(g, sp, st);
   if (a_kmajor) return launch_store_loop<DmaLoopT<true, false>>(g, sp, st);
   return launch_store_loop<DmaLoopT<false, true>>(g, sp, st);
 }
@@ -1164,17 +1126,6 @@ int launch_transpose(const void* in, int64_t ld_in, int rows, int cols, void* ou
   hipLaunchKernelGGL(transpose_bf16_kernel, grid, dim3(256), 0, st,
                      static_cast<const uint16_t*>(in), ld_in, rows, cols,
                      static_cast<uint16_t*>(out), ld_out, rows_pad);
-  AXON_CHECK_LAUNCH();
-  return AXON_OK;
-}
-
-int launch_zero_cols(void* p, int64_t ld, int rows, int col0, int ncols, hipStream_t st) {
-  if (ncols <= 0 || rows <= 0) return AXON_OK;
-  const int64_t total = (int64_t)rows * ncols;
-  const int64_t blocks = (total + 255) / 256;
-  const int grid = (int)(blocks < 2048 ? blocks : 2048);
-  hipLaunchKernelGGL(zero_cols_bf16_kernel, dim3(grid), dim3(256), 0, st, static_cast<uint16_t*>(p),
-                     ld, rows, col0, ncols);
   AXON_CHECK_LAUNCH();
   return AXON_OK;
 }
@@ -1199,8 +1150,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
   StashWs sw{};
   if (stash) {
     if (reinterpret_cast<uintptr_t>(stash) & 15) return AXON_ERR_ARG;
-    sw = stash_ws(n, h, v, stash);
-    if (sw.bytes == 0) return AXON_ERR_SHAPE;
+    sw = stash_ws(n, v, stash);
     if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
     w.pm = sw.pm;  // the backward needs the per-part maxima: they live in the stash
   }
@@ -1249,13 +1199,11 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
 }
 
 // A backward over a block of consecutive tokens of a longer stream (one call per block, one stream):
-// where the last row's label and gradients live (aligned_pos), whether the workspace already holds the
-// transposed weight (written by the step's first call), and how this block's share of the weight
+// where the last row's label and gradients live (aligned_pos), and how this block's share of the weight
 // gradient leaves: the blocks of a step add up in one fp32 array, the last one rounds the sum to bf16.
 enum { kDwStore = 0, kDwFirst = 1, kDwAdd = 2, kDwLast = 3 };
 struct BlockArgs {
   int64_t last_dst = 0;
-  int wt_ready = 0;
   int dw_mode = kDwStore;
   float* dw_acc = nullptr;  // axon_lmhead_block_dw_acc_bytes of fp32 partial sums, tile order (modes other than kDwStore)
   // Several consecutive blocks may share ONE weight-gradient GEMM (a longer reduction, fewer passes over
@@ -1302,18 +1250,13 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   StashWs sw{};
   if (stash) {
     if (reinterpret_cast<uintptr_t>(stash) & 15) return AXON_ERR_ARG;
-    sw = stash_ws(n, h, v, const_cast<void*>(stash));
-    if (sw.bytes == 0) return AXON_ERR_SHAPE;
+    sw = stash_ws(n, v, const_cast<void*>(stash));
     if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
   }
 
-  // K-contiguous copies for the two output GEMMs
+  // the hidden states K-contiguous for the weight gradient, zeros up to the tile border
   {
     Span span(timer, 0);
-    if (!blk.wt_ready && !w.w_kmajor) {
-      rc = launch_transpose(weight, h, (int)v, (int)h, w.wT, w.ld_v, (int)w.v_pad, st);
-      if (rc != AXON_OK) return rc;
-    }
     rc = launch_transpose(hidden, h, (int)n, (int)h, w.hT + pos, w.ld_n, (int)n_tile, st);
     if (rc != AXON_OK) return rc;
   }
@@ -1324,8 +1267,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   for (int ci = 0; ci < w.chunks; ++ci) {
     const int64_t v0 = (int64_t)ci * w.chunk;
     const int64_t vc = (v - v0 < w.chunk) ? (v - v0) : w.chunk;  // valid vocab rows in this chunk
-    const int64_t vc_red = round_up(vc, 64);                      // reduction length of B2
-    // B1: dlogit for vocab rows [v0, v0 + vc)
+    // B1: dlogit for vocab rows [v0, v0 + vc); whole tiles, zeros beyond the last token and vocabulary row
     {
       Span span(timer, 1);
       GemmOperands g;
@@ -1341,7 +1283,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       p.is_start = is_start;
       p.last_dst = (int)blk.last_dst;
       if (stash) {
-        const StashSource src{sw.tiles, sw.pm, sw.tiles_n, (int)(v0 / kTile), sw.shifted};
+        const StashSource src{sw.tiles, sw.pm, sw.tiles_n, (int)(v0 / kTile)};
         const unsigned blocks = (unsigned)(round_up(vc, kTile) / kTile) * (unsigned)sw.tiles_n * 8u;
         if (softcap > 0.f)
           hipLaunchKernelGGL(lmhead_dlogit_stash_kernel<true>, dim3(blocks), dim3(64), 0, st, p, src);
@@ -1353,36 +1295,21 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       } else {
         AXON_LAUNCH_GEMM(lmhead_dlogit_kernel, g, p, st);
       }
-      // reduction padding the tiles did not cover (the shifted-tile path writes no padding; the
-      // clamped path writes zeros there already, the extra fill is then redundant but harmless)
-      rc = launch_zero_cols(dl, w.ld_c, (int)n, (int)vc, (int)(vc_red - vc), st);
-      if (rc != AXON_OK) return rc;
-      // the token rows up to the next tile boundary: reduction padding of B3 when it reads dl K-major, and
-      // rows of B2's operand when fewer than 256 tokens run on the DMA loop
-      if (w.dl_kmajor || (w.w_kmajor && n < kTile))
-        rc = launch_zero_cols(dl + n * w.ld_c, w.ld_c, (int)(n_tile - n), 0, (int)vc_red, st);
-      if (rc == AXON_OK && !w.dl_kmajor)
-        rc = launch_zero_cols(w.dlT, w.ld_n, (int)vc, (int)n, (int)(n_red - n), st);
-      if (rc != AXON_OK) return rc;
     }
-    // B2: dHidden[n][h] (+)= sum_v dl[n][v] * W[v0 + v][h]  (the weight read K-major where it lies, or its
-    // transposed copy wT[h][v0 + v])
+    // B2: dHidden[n][h] (+)= sum_v dl[n][v] * W[v0 + v][h], the weight read K-major where it lies
     {
       Span span(timer, 2);
       GemmOperands g;
-      if (w.w_kmajor) { g.a = static_cast<const __bf16*>(weight) + v0 * h;  g.lda = h; }
-      else            { g.a = w.wT + v0;                                     g.lda = w.ld_v; }
-      g.m_rows = (int)h;
-      // fewer than 256 tokens: the zero rows up to 256 are part of the operand, the stores stop at n
-      g.b = dl;  g.ldb = w.ld_c;  g.n_rows = (int)((w.w_kmajor && n < kTile) ? kTile : n);
-      g.k = (int)vc_red;
+      g.a = static_cast<const __bf16*>(weight) + v0 * h;  g.lda = h;  g.m_rows = (int)h;
+      g.b = dl;  g.ldb = w.ld_c;  g.n_rows = (int)n;
+      g.k = (int)vc;
       StoreParams sp;
       const bool last = (ci == w.chunks - 1);
       sp.out_f32 = (w.chunks > 1) ? w.dh_acc : nullptr;  sp.ld_f32 = h;
       sp.out_bf16 = last ? static_cast<__bf16*>(d_hidden) : nullptr;  sp.ld_bf16 = h;
       sp.m_valid = (int)h; sp.n_valid = (int)n; sp.accumulate = (ci > 0); sp.keep_f32 = 1;
       sp.tile_acc = nullptr;
-      rc = launch_store_kmajor(g, sp, w.w_kmajor, false, st);
+      rc = launch_store_kmajor(g, sp, true, false, st);
       if (rc != AXON_OK) return rc;
     }
     // B3: dWeight[v0 + v][h] = sum_t dl[t][v] * hT[h][t] over the tokens the workspace holds up to this
@@ -1496,7 +1423,12 @@ extern "C" int64_t axon_lmhead_fwd_workspace_bytes(int64_t n, int64_t h, int64_t
 
 extern "C" int64_t axon_lmhead_stash_bytes(int64_t n, int64_t h, int64_t v) {
   if (check_head_shape(n, h, v) != AXON_OK) return -1;
-  return stash_ws(n, h, v, nullptr).bytes;
+  return stash_of_all_tokens(n, h, v) ? stash_ws(n, v, nullptr).bytes : 0;
+}
+
+extern "C" int64_t axon_lmhead_block_stash_bytes(int64_t n, int64_t h, int64_t v) {
+  if (check_head_shape(n, h, v) != AXON_OK) return -1;
+  return stash_ws(n, v, nullptr).bytes;
 }
 
 extern "C" int axon_lmhead_fwd(const void* hidden, const void* weight, const void* labels,
@@ -1591,6 +1523,12 @@ extern "C" int axon_gemm_nt_bf16(const void* a, int64_t lda, const void* b, int6
   return launch_store(g, sp, (hipStream_t)stream);
 }
 
+// The K-major forms of the plain GEMM keep the domain their documentation states.
+static bool gemm_kmajor_domain(const GemmOperands& g, bool a_kmajor, bool b_kmajor) {
+  return (!a_kmajor && !b_kmajor) || (g.m_rows >= kTile && g.n_rows >= kTile && g.k % 64 == 0 &&
+                                      (!a_kmajor || g.m_rows % 8 == 0) && (!b_kmajor || g.n_rows % 8 == 0));
+}
+
 extern "C" int axon_gemm_bf16(const void* a, int64_t lda, int a_kmajor, const void* b, int64_t ldb,
                               int b_kmajor, float* out, int64_t ldo, int64_t m, int64_t n, int64_t k,
                               void* stream) {
@@ -1602,6 +1540,7 @@ extern "C" int axon_gemm_bf16(const void* a, int64_t lda, int a_kmajor, const vo
   g.a = static_cast<const __bf16*>(a);  g.lda = lda;  g.m_rows = (int)m;
   g.b = static_cast<const __bf16*>(b);  g.ldb = ldb;  g.n_rows = (int)n;
   g.k = (int)k;
+  if (!gemm_kmajor_domain(g, a_kmajor != 0, b_kmajor != 0)) return AXON_ERR_SHAPE;
   StoreParams sp;
   sp.out_f32 = out; sp.ld_f32 = ldo; sp.out_bf16 = nullptr; sp.ld_bf16 = 0;
   sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 1; sp.tile_acc = nullptr;
@@ -1642,20 +1581,13 @@ extern "C" int axon_lmhead_block_can_group(int64_t h, int64_t v, int64_t chunk) 
 }
 
 extern "C" int axon_lmhead_block_begin(const void* weight, int64_t h, int64_t v, int64_t chunk,
-                                       void* workspace, int64_t ws_bytes, void* stream, void* timer) {
+                                       void* workspace, int64_t /*ws_bytes*/, void* stream, void* timer) {
   int rc = check_head_shape(0, h, v);
   if (rc != AXON_OK) return rc;
   if (chunk < 0 || chunk % kTile != 0) return AXON_ERR_ARG;
   if (!weight || !workspace || (reinterpret_cast<uintptr_t>(weight) & 15)) return AXON_ERR_ARG;
-  PhaseTimer* t = block_timer(timer, stream, 4, &rc);
-  if (rc != AXON_OK) return rc;
-  char* base = reinterpret_cast<char*>(round_up(reinterpret_cast<int64_t>(workspace), kAlign));
-  const BwdWs w = bwd_ws(0, h, v, chunk, base);
-  if (w.w_kmajor) return AXON_OK;  // the dHidden GEMM reads the weight where it lies
-  if ((base - static_cast<char*>(workspace)) + round_up(h * w.ld_v * 2, kAlign) > ws_bytes)
-    return AXON_ERR_WORKSPACE;
-  Span span(t, 0);
-  return launch_transpose(weight, h, (int)v, (int)h, w.wT, w.ld_v, (int)w.v_pad, (hipStream_t)stream);
+  (void)block_timer(timer, stream, 4, &rc);
+  return rc;
 }
 
 extern "C" int axon_lmhead_block_fwd(const void* hidden, const void* weight, const void* labels,
@@ -1677,7 +1609,7 @@ extern "C" int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentro
                                      const float* lse, const float* entropy_b, int64_t n, int64_t h,
                                      int64_t v, float inv_temp, float softcap,
                                      const uint8_t* seq_start, int64_t last_dst, void* d_hidden,
-                                     void* d_weight, float* dw_acc, int dw_mode, int wt_ready,
+                                     void* d_weight, float* dw_acc, int dw_mode, int /*wt_ready*/,
                                      int64_t group_pos, int dw_now, int64_t ws_tokens,
                                      int64_t chunk, void* workspace, int64_t ws_bytes,
                                      const void* stash, int64_t stash_bytes, void* stream,
@@ -1688,7 +1620,6 @@ extern "C" int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentro
   if (rc != AXON_OK) return rc;
   BlockArgs blk;
   blk.last_dst = last_dst;
-  blk.wt_ready = wt_ready != 0;
   blk.dw_mode = dw_mode;
   blk.dw_acc = dw_acc;
   blk.group_pos = group_pos;

@@ -114,13 +114,7 @@ class _BlockedHeadLoss(torch.autograd.Function):
 
         if seq_mode:
             row_blocks = spec["row_blocks"]
-            # hidden rows of a block: its sequences, lengthened to a multiple of four rows (the stash needs it);
-            # the up to three rows borrowed from the next block carry a zero gradient here and are done again there
-            ranges = []
-            for r0, r1 in row_blocks:
-                a, b = cu_host[r0], cu_host[r1]
-                ranges.append((a, min(n, a + (b - a + 3) // 4 * 4)))
-            slots = [(cu_host[r0], cu_host[r1]) for r0, r1 in row_blocks]
+            ranges = slots = [(cu_host[r0], cu_host[r1]) for r0, r1 in row_blocks]  # a block's sequences
         else:
             ranges = token_blocks(n, spec["block_tokens"])
             # hidden row r writes position r + 1: a block of rows [a, b) owns positions a + 1 .. b

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define AXON_AMD_ABI_VERSION 20
+#define AXON_AMD_ABI_VERSION 21
 
 enum {
   AXON_OK = 0,
@@ -92,9 +92,10 @@ const char* axon_amd_error_string(int code);
  *        the logit; numerators below 2^-24 of their part's maximum read back as 0.
  * Constraints: hidden % 32 == 0, hidden >= 32, vocab >= 1, n_tokens >= 0. */
 int64_t axon_lmhead_fwd_workspace_bytes(int64_t n_tokens, int64_t hidden, int64_t vocab);
-/* Bytes of the forward's stash for this shape; 0 if the shape cannot be stashed (tiles that are
- * shifted back inside the matrix need n_tokens % 4 == 0 and vocab % 4 == 0), -1 for an invalid
- * shape.  The layout is private to the library and depends on the shape only. */
+/* Bytes of the forward's stash for this shape; 0 for the shapes for which this operator keeps none
+ * (n_tokens, vocab >= 256 with hidden % 64 == 0 and n_tokens or vocab no multiple of 4: their backward
+ * recomputes the logits; a block of a step has one for any shape, axon_lmhead_block_stash_bytes), -1 for
+ * an invalid shape.  The layout is private to the library and depends on the shape only. */
 int64_t axon_lmhead_stash_bytes(int64_t n_tokens, int64_t hidden, int64_t vocab);
 /* flags[p] = 1 where a non-empty sequence of cu_seqlens[n_seqs + 1] begins, else 0.
  * `flags` holds n_tokens bytes rounded up to a multiple of 4. */
@@ -204,11 +205,9 @@ int axon_lmhead_bwd_timed(const float* dlogprobs, const float* dentropy, const v
  *        then read and written at index n_tokens of the block-offset arrays, i.e. the next block's
  *        first position), and minus the block's first position when the block ends the stream (index 0
  *        of the whole arrays, a sequence start).  0 is the whole-stream call, as axon_lmhead_fwd.
- *   axon_lmhead_block_begin: once per step, before the first backward: the transposed weight into
- *        `workspace` (the same workspace, of axon_lmhead_bwd_workspace_bytes(largest block, ...) bytes,
- *        must then be handed to every axon_lmhead_block_bwd of the step, with wt_ready = 1).  For
- *        hidden >= 256 and vocab % 64 == 0 the backward reads the weight where it lies: the call then
- *        launches nothing and the workspace holds no transposed weight.
+ *   axon_lmhead_block_stash_bytes: the stash of a block of n_tokens rows; any shape the head takes.
+ *   axon_lmhead_block_begin: checks its arguments and launches nothing (the backward reads the weight
+ *        where it lies); kept for callers that open a step with it.
  *   axon_lmhead_block_bwd: d_hidden rows of the block (bf16, complete: a row sums over the vocabulary
  *        only).  The weight gradient sums over all blocks: dw_mode 0 = this block is the whole step,
  *        d_weight (bf16) is written; 1 = first block, dw_acc (fp32 partial sums,
@@ -222,6 +221,7 @@ int axon_lmhead_bwd_timed(const float* dlogprobs, const float* dentropy, const v
  * nothing when it is exactly 1 (the step's gradients are finished before autograd hands over the
  * factor of the loss, which is 1 unless the caller scaled the loss); n % 8 == 0, x on a 16-byte boundary. */
 int64_t axon_lmhead_block_dw_acc_bytes(int64_t hidden, int64_t vocab);
+int64_t axon_lmhead_block_stash_bytes(int64_t n_tokens, int64_t hidden, int64_t vocab);
 int axon_lmhead_block_begin(const void* weight_bf16, int64_t hidden, int64_t vocab, int64_t vocab_chunk,
                             void* workspace, int64_t workspace_bytes, void* stream, void* timer);
 int axon_lmhead_block_fwd(const void* hidden_bf16, const void* weight_bf16, const void* labels,

@@ -827,3 +827,30 @@ def test_default_backward_has_no_readback_and_replays_in_a_hip_graph(from_stash)
             with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=side):
                 _ops.lmhead_backward(g_lp, g_en, hd, wd, ld, lse, eb, 1.0, skip_zero_rows=True)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("n,h,v", [
+    (1, 64, 5), (3, 128, 257), (255, 192, 511),      # fewer rows than a tile on either side, hidden < 256
+    (256, 256, 256), (257, 320, 513),                # one row more than a tile
+    (130, 256, 1003), (511, 896, 1031),              # odd vocabularies: the reduction over the vocabulary ends inside a k-tile
+    (515, 256, 1000),
+])
+def test_ragged_tile_edges_of_the_dma_loop_vs_oracle(n, h, v):
+    """Rows beyond an operand's last one read as zeros (descriptor bounds): forward, recompute backward, and a block
+    of a step with its stash, at sizes where no dimension is a multiple of the tile."""
+    hid, w, lab = W.lmhead_inputs(n, h, v, seed=n + h + v)
+    w = (w.float() * 8).bfloat16()
+    hd, wd, ld = hid.to(DEV), w.to(DEV), lab.to(DEV)
+    g = torch.Generator().manual_seed(9)
+    g_lp, g_en = torch.randn(n, generator=g) / n, torch.randn(n, generator=g) / n
+    ref_lp, ref_ent = OM.forward(hid, w, lab)
+    ref_dh, ref_dw = OM.backward(g_lp, g_en, hid, w, lab)
+    lp, ent, lse, eb = _ops.lmhead_forward(hd, wd, ld, 1.0)
+    assert (lp.cpu() - ref_lp).abs().max() < 1e-3 and (ent.cpu() - ref_ent).abs().max() < 1e-3
+    dh, dw = _ops.lmhead_backward(g_lp.to(DEV), g_en.to(DEV), hd, wd, ld, lse, eb, 1.0)
+    assert rel_l2(dh, ref_dh) < 2e-2 and rel_l2(dw, ref_dw) < 2e-2
+    hb = _ops.HeadBlocks(hd, wd, ld, 1.0, [(0, n)])
+    hb.forward(0)
+    assert hb.block_stash_bytes > 0 and torch.equal(hb.logprobs, lp) and torch.equal(hb.entropy, ent)
+    hb.backward(0, g_lp.to(DEV), g_en.to(DEV))
+    assert rel_l2(hb.d_hidden, ref_dh) < 2e-2 and rel_l2(hb.d_weight, ref_dw) < 2e-2
