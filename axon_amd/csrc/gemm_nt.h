@@ -214,6 +214,7 @@ struct DmaSide {
 template <bool kAT, bool kBT, bool kNarrow = false>
 struct DmaLoopT {
   static constexpr int kBK = 64;
+  static constexpr bool kAMajor = kAT, kBMajor = kBT;
   static constexpr int kRowBytes = 128;
   static constexpr int kOperandBytes = kTile * kRowBytes;  // 32 KB
   static constexpr int kBBase = 3 * kOperandBytes;         // A slots at 0/32/64 KB, B slots at 96/128 KB
@@ -461,6 +462,7 @@ template <int BK>
 struct RegLoop {
   static_assert(BK == 32, "one 16x16x32 k-step per staged tile");
   static constexpr int kBK = BK;
+  static constexpr bool kAMajor = false, kBMajor = false;
   static constexpr int kChunks = BK / 8;                 // 16-byte chunks per row
   static constexpr int kRowBytes = BK * 2;
   static constexpr int kRowsPerLine = 256 / kRowBytes;   // rows per 256-byte bank line
@@ -550,19 +552,21 @@ struct RegLoop {
   }
 };
 
-// Workgroup id -> (tile_m, tile_n).  Consecutive workgroup ids land on
-// different XCDs (round-robin over 8), so ids are first regrouped so that each
-// XCD walks a contiguous range, and inside that range tiles are visited in
-// bands of `kBand` n-tiles so that concurrently resident workgroups of one XCD
-// share A and B tiles in its L2 (32 workgroups per XCD: 8 x 4 tiles at kBand = 4, 4 x 8 at kBand = 8; the
-// forward, whose A operand is the weight, is 1.7 % faster with 8, the output GEMMs 2.3 % faster with 4).
-template <int kBand = 4>
-__device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, int& tn) {
+// Workgroup id -> place in the walk over `total` units of work.  Consecutive workgroup ids land on
+// different XCDs (round-robin over 8), so ids are regrouped so that each XCD walks a contiguous range.
+__device__ __forceinline__ int xcd_order(int total) {
   constexpr int kXcd = 8;
-  const int total = tiles_m * tiles_n;
-  int pid = blockIdx.x;
+  const int pid = blockIdx.x;
   const int per = total / kXcd;  // ids beyond kXcd*per keep their natural position
-  if (pid < per * kXcd) pid = (pid % kXcd) * per + pid / kXcd;
+  return pid < per * kXcd ? (pid % kXcd) * per + pid / kXcd : pid;
+}
+
+// Place in the walk -> (tile_m, tile_n): tiles are visited in bands of `kBand` n-tiles so that
+// concurrently resident workgroups of one XCD share A and B tiles in its L2 (32 workgroups per XCD: 8 x 4
+// tiles at kBand = 4, 4 x 8 at kBand = 8; the forward, whose A operand is the weight, is 1.7 % faster with
+// 8, the output GEMMs 2.3 % faster with 4).
+template <int kBand = 4>
+__device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int band_sz = kBand * tiles_m;
   const int band = pid / band_sz;
   const int first_n = band * kBand;

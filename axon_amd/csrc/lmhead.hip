@@ -175,7 +175,7 @@ __device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams&
                                          int tiles_n) {
   extern __shared__ __align__(16) char smem[];
   int tm, tn;
-  tile_coords<8>(tiles_m, tiles_n, tm, tn);
+  tile_coords<8>(xcd_order(tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
   const TilePos t = Loop::place(tm, tn);
   AccTile acc;
   Loop::run(g, t, acc, smem);
@@ -590,7 +590,7 @@ __device__ __forceinline__ void dlogit_body(const GemmOperands& g, const DlogitP
                                             int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) char smem[];
   int tm, tn;
-  tile_coords(tiles_m, tiles_n, tm, tn);
+  tile_coords(xcd_order(tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
   const TilePos t = Loop::place(tm, tn);  // t.m0 is relative to the chunk
   AccTile acc;
   Loop::run(g, t, acc, smem);
@@ -665,17 +665,20 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_stash_kernel(DlogitParams p,
 // Backward B2/B3 and the plain GEMM: store the tile as out[n][m]
 // ----------------------------------------------------------------------------
 struct StoreParams {
-  float* out_f32;     // [n][ld_f32] fp32 accumulator / output (may be null)
+  float* out_f32;     // [n][ld_f32] fp32 output (may be null)
   __bf16* out_bf16;   // [n][ld_bf16] (may be null)
   int64_t ld_f32, ld_bf16;
   int m_valid, n_valid;
-  int accumulate;     // add the previous contents of out_f32 (or tile_acc) first
-  int keep_f32;       // write the sum back to out_f32 / tile_acc (0: it is only read, the sum leaves as bf16)
-  // fp32 partial sums that only this kernel ever reads back (the weight gradient carried from one token
-  // block to the next): kept per tile in the order the accumulators lie in the registers, so that every
+  int accumulate;     // add the previous contents of tile_acc first
+  int keep_f32;       // write the sum back to tile_acc (0: it is only read, the sum leaves as bf16)
+  // fp32 partial sums (the weight gradient carried from one token block to the next, dHidden carried from one
+  // vocabulary chunk to the next or formed in parts): kept per tile in the order the accumulators lie in the registers, so that every
   // wavefront load and store is one contiguous kilobyte.  float4 index =
   // ((tile * 4 + wave) * 64 + i * 8 + j) * 64 + lane, tile = tm * tiles_n + tn.  Null: not used.
   float4* tile_acc;
+  // Split reduction: `splits` workgroups per tile, each over `k_split` (a multiple of 64) of the k; they leave their
+  // partial sums in tile_acc, one array of tiles after the other, for split_sum_kernel.
+  int splits, k_split;
 };
 constexpr int64_t kTileAccVecs = 4 * kBlocks * kBlocks * 64;  // float4 per tile (256 KB)
 
@@ -684,7 +687,14 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
                                                                   int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) char smem[];
   int tm, tn;
-  tile_coords(tiles_m, tiles_n, tm, tn);
+  const int tiles = tiles_m * tiles_n;
+  const int pid = xcd_order(tiles * p.splits);
+  const int split = pid / tiles;  // the tiles of one part of k side by side: they share operand slices
+  tile_coords(pid - split * tiles, tiles_m, tiles_n, tm, tn);
+  const int64_t k0 = (int64_t)split * p.k_split;
+  g.a += Loop::kAMajor ? k0 * g.lda : k0;
+  g.b += Loop::kBMajor ? k0 * g.ldb : k0;
+  g.k = min(g.k - (int)k0, p.k_split);
   const TilePos t = Loop::place(tm, tn);
   AccTile acc;
   Loop::run(g, t, acc, smem);
@@ -692,7 +702,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
   if (p.tile_acc) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     f32x4* ta = reinterpret_cast<f32x4*>(p.tile_acc) +
-                ((int64_t)(tm * tiles_n + tn) * 4 + lp.wave) * (kBlocks * kBlocks * 64) + lp.lane;
+                (((int64_t)split * tiles + tm * tiles_n + tn) * 4 + lp.wave) * (kBlocks * kBlocks * 64) + lp.lane;
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
       f32x4 old[kBlocks];
@@ -726,12 +736,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
       if (m >= p.m_valid) continue;  // m_valid % 4 == 0: a quad is all in or all out
       float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
       if (p.out_f32) {
-        float4* dst = reinterpret_cast<float4*>(p.out_f32 + (int64_t)n * p.ld_f32 + m);
-        if (p.accumulate) {
-          const float4 old = *dst;
-          v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
-        }
-        if (p.keep_f32) *dst = v;
+        *reinterpret_cast<float4*>(p.out_f32 + (int64_t)n * p.ld_f32 + m) = v;
       }
       if (p.out_bf16) {
         uint2 w;
@@ -741,6 +746,37 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
       }
     }
   }
+}
+
+// out[n][m] = the sum over the parts of a split reduction, rounded to bf16: a streaming kernel, one thread per
+// four accumulators (read as whole kilobytes per wavefront, in the order of the parts).
+__global__ __launch_bounds__(256) void split_sum_kernel(const float4* __restrict__ parts, int splits, int tiles_m,
+                                                        int tiles_n, int m_valid, int n_valid,
+                                                        __bf16* __restrict__ out, int64_t ld) {
+  const int64_t stride = (int64_t)tiles_m * tiles_n * kTileAccVecs;
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;  // lane, then block (i, j), wavefront, tile
+  const float4* src = parts + q;
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  int s = 0;
+  for (; s + 4 <= splits; s += 4) {
+    float4 x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = src[(s + u) * stride];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { v.x += x[u].x; v.y += x[u].y; v.z += x[u].z; v.w += x[u].w; }
+  }
+  for (; s < splits; ++s) {
+    const float4 x = src[s * stride];
+    v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
+  }
+  const int lane = (int)(q & 63), ij = (int)(q >> 6) & 63, wave = (int)(q >> 12) & 3, tile = (int)(q >> 14);
+  const int m = (tile / tiles_n) * kTile + (wave >> 1) * kWaveTile + (ij >> 3) * kBlk + 4 * (lane >> 4);
+  const int n = (tile % tiles_n) * kTile + (wave & 1) * kWaveTile + (ij & 7) * kBlk + (lane & 15);
+  if (m >= m_valid || n >= n_valid) return;
+  uint2 w;
+  w.x = pack_bf16(v.x, v.y);
+  w.y = pack_bf16(v.z, v.w);
+  *reinterpret_cast<uint2*>(out + (int64_t)n * ld + m) = w;
 }
 
 // out[c][r] = in[r][c] for r < rows, c < cols; zero for r in [rows, rows_pad).
@@ -905,9 +941,11 @@ using namespace axon;
 namespace {
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
-// bf16 dlogits of one chunk exist in both orientations (2 x 2.1 GB at 32768 tokens); every chunk costs one
-// read-modify-write pass over the fp32 dHidden accumulator, so fewer, larger chunks are cheaper
+// Vocabulary chunk of a backward that is not told one: every chunk costs one read-modify-write pass over the fp32
+// dHidden partial sums and its own launches, so as much of the vocabulary as keeps a chunk's bf16 dlogits within
+// the 2 GiB that 32768 columns take at 32768 tokens.
 constexpr int64_t kDefaultVocabChunk = 32768;
+constexpr int64_t kDefaultChunkElems = int64_t(1) << 30;
 constexpr int64_t kAlign = 256;
 using SlowLoop = RegLoop<32>;
 
@@ -988,9 +1026,36 @@ bool stash_of_all_tokens(int64_t n, int64_t h, int64_t v) {
   return n > 0 && (h % 64 != 0 || n < kTile || v < kTile || (n % 4 == 0 && v % 4 == 0));
 }
 
+// How many workgroups share a tile's reduction.  dHidden has few tiles (tokens x hidden) and a long reduction (the
+// vocabulary): with one workgroup per tile 700 tokens x 4096 keep 48 of the 256 CUs busy and 6007 x 896 keep 96.
+// The plan minimises an estimate in thirds of a microsecond.  A k-tile takes 1.33 us per workgroup when all CUs work
+// (the part is power-limited then) and 1.0 us when few do; a round of workgroups costs 6 us beside its k-tiles
+// (first loads, epilogue); a tile part costs 0.1 us of memory time (256 KB written, then read by
+// split_sum_kernel).  Measured (sums included): 48 tiles, K = 151936, 2396 us with one part and 579 with 5; 96
+// tiles 2475 and 1183 with 8; 384 tiles (8192 x 2880), K = 201088, 7662 and 6525 with 2; 512 tiles (8192 x 4096)
+// stay whole.
+// At most kMaxUnits tile parts (three rounds, 200 MB of partial sums, which the Infinity Cache holds).
+// A part has at least kMinPartTiles k-tiles: below that its first loads and its epilogue are a quarter of its time.
+constexpr int kCus = 256, kMaxSplits = 64, kMaxUnits = 3 * kCus, kMinPartTiles = 32;
+struct SplitPlan { int splits, k_split; };
+SplitPlan split_plan(int64_t tiles, int64_t k) {
+  const int64_t kt = (k + 63) / 64;
+  SplitPlan best{1, (int)(kt * 64)};
+  int64_t best_cost = INT64_MAX;
+  for (int s = 1; s <= kMaxSplits && (s == 1 || (s * kMinPartTiles <= kt && tiles * s <= kMaxUnits)); ++s) {
+    const int64_t per = (kt + s - 1) / s, parts = (kt + per - 1) / per;  // every part gets k-tiles
+    if (parts != s) continue;
+    const int64_t units = tiles * s, full = units / kCus, rem = units % kCus;
+    const int64_t cost = per * 4 * full + (rem ? per * 3 + per * rem / kCus : 0) + 18 * (full + (rem ? 1 : 0)) +
+                         (s > 1 ? units / 3 : 0);
+    if (cost < best_cost) { best_cost = cost; best = SplitPlan{s, (int)(per * 64)}; }
+  }
+  return best;
+}
+
 struct BwdWs {
   __bf16 *hT, *dl, *dlT;
-  float* dh_acc;
+  float4* dh_acc;  // dHidden partial sums in tile order: the parts of a split reduction, or carried over the chunks
   int64_t v_pad, n_pad, chunk, bytes;
   int64_t ld_n, ld_c;  // leading dimensions of hT/dlT, dl: padded by kLdPad elements
   int chunks;
@@ -1009,7 +1074,11 @@ BwdWs bwd_ws(int64_t n, int64_t h, int64_t vocab, int64_t chunk, void* base) {
   BwdWs w;
   w.v_pad = round_up(vocab, kTile);
   w.n_pad = round_up(n, kTile);
-  w.chunk = (chunk <= 0) ? kDefaultVocabChunk : chunk;
+  w.chunk = chunk;
+  if (w.chunk <= 0) {
+    const int64_t fit = kDefaultChunkElems / (w.n_pad > 0 ? w.n_pad : kTile) / kTile * kTile;
+    w.chunk = fit > kDefaultVocabChunk ? fit : kDefaultVocabChunk;
+  }
   if (w.chunk > w.v_pad) w.chunk = w.v_pad;
   if (w.chunk > kMaxVocabChunk) w.chunk = kMaxVocabChunk;
   w.chunks = (int)((vocab + w.chunk - 1) / w.chunk);
@@ -1026,8 +1095,14 @@ BwdWs bwd_ws(int64_t n, int64_t h, int64_t vocab, int64_t chunk, void* base) {
     w.dlT = reinterpret_cast<__bf16*>(p + off);
     off += round_up(w.chunk * w.ld_n * 2, kAlign);
   }
-  w.dh_acc = reinterpret_cast<float*>(p + off);
-  if (w.chunks > 1) off += round_up(n * h * 4, kAlign);
+  const int64_t dh_tiles = (round_up(h, kTile) / kTile) * (w.n_pad / kTile);
+  // room for the parts of any call over at most n tokens (split_plan), or for one part per tile
+  const int64_t longest = vocab / (64 * kMinPartTiles);
+  const int64_t max_splits = longest < kMaxSplits ? longest : kMaxSplits;
+  int64_t parts = max_splits < 2 ? 0 : dh_tiles * max_splits < kMaxUnits ? dh_tiles * max_splits : kMaxUnits;
+  if (w.chunks > 1 && parts < dh_tiles) parts = dh_tiles;
+  w.dh_acc = reinterpret_cast<float4*>(p + off);
+  off += parts * kTileAccVecs * 16;
   w.bytes = off;
   return w;
 }
@@ -1100,7 +1175,7 @@ template <class Loop>
 int launch_store_loop(const GemmOperands& g, const StoreParams& sp, hipStream_t st) {
   const int tiles_m = (g.m_rows + kTile - 1) / kTile, tiles_n = (g.n_rows + kTile - 1) / kTile;
   if (set_lds(gemm_store_kernel<Loop>) != AXON_OK) return AXON_ERR_LAUNCH;
-  hipLaunchKernelGGL(gemm_store_kernel<Loop>, dim3(tiles_m * tiles_n), dim3(kGemmThreads), kGemmLdsBytes, st, g,
+  hipLaunchKernelGGL(gemm_store_kernel<Loop>, dim3(tiles_m * tiles_n * sp.splits), dim3(kGemmThreads), kGemmLdsBytes, st, g,
                      sp, tiles_m, tiles_n);
   AXON_CHECK_LAUNCH();
   return AXON_OK;
@@ -1262,6 +1337,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   }
   const int64_t n_red = round_up(n, 64);  // reduction length of B3 (from this block's first token)
   const int64_t tiles_h = round_up(h, kTile) / kTile;
+  const SplitPlan plan = split_plan(tiles_h * (n_tile / kTile), w.chunks > 1 ? w.chunk : v);
   __bf16* const dl = w.dl + pos * w.ld_c;  // this block's rows
 
   for (int ci = 0; ci < w.chunks; ++ci) {
@@ -1303,14 +1379,25 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       g.a = static_cast<const __bf16*>(weight) + v0 * h;  g.lda = h;  g.m_rows = (int)h;
       g.b = dl;  g.ldb = w.ld_c;  g.n_rows = (int)n;
       g.k = (int)vc;
+      const bool last = (ci == w.chunks - 1), split = plan.splits > 1;
       StoreParams sp;
-      const bool last = (ci == w.chunks - 1);
-      sp.out_f32 = (w.chunks > 1) ? w.dh_acc : nullptr;  sp.ld_f32 = h;
-      sp.out_bf16 = last ? static_cast<__bf16*>(d_hidden) : nullptr;  sp.ld_bf16 = h;
-      sp.m_valid = (int)h; sp.n_valid = (int)n; sp.accumulate = (ci > 0); sp.keep_f32 = 1;
-      sp.tile_acc = nullptr;
+      sp.out_f32 = nullptr;  sp.ld_f32 = 0;
+      sp.out_bf16 = (last && !split) ? static_cast<__bf16*>(d_hidden) : nullptr;  sp.ld_bf16 = h;
+      sp.m_valid = (int)h; sp.n_valid = (int)n;
+      sp.tile_acc = (w.chunks > 1 || split) ? w.dh_acc : nullptr;
+      sp.accumulate = (ci > 0); sp.keep_f32 = split || !last;
+      // a shorter last chunk reaches the first parts only
+      sp.k_split = plan.k_split;
+      sp.splits = (int)((vc + sp.k_split - 1) / sp.k_split);
       rc = launch_store_kmajor(g, sp, true, false, st);
       if (rc != AXON_OK) return rc;
+      if (last && split) {
+        const int tiles_m = (int)tiles_h, tiles_n = (int)(n_tile / kTile);
+        hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)(tiles_m * tiles_n * (kTileAccVecs / 256))), dim3(256), 0, st,
+                           w.dh_acc, plan.splits, tiles_m, tiles_n, (int)h, (int)n,
+                           static_cast<__bf16*>(d_hidden), h);
+        AXON_CHECK_LAUNCH();
+      }
     }
     // B3: dWeight[v0 + v][h] = sum_t dl[t][v] * hT[h][t] over the tokens the workspace holds up to this
     // block's end (dl read as the K-major operand, or its vocab-major copy dlT[v][t])
@@ -1331,6 +1418,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       sp.m_valid = (int)h; sp.n_valid = (int)vc;
       sp.accumulate = blk.dw_mode == kDwAdd || blk.dw_mode == kDwLast;
       sp.keep_f32 = blk.dw_mode != kDwLast;
+      sp.splits = 1; sp.k_split = g.k;
       rc = launch_store_kmajor(g, sp, false, w.dl_kmajor, st);
       if (rc != AXON_OK) return rc;
     }
@@ -1519,7 +1607,8 @@ extern "C" int axon_gemm_nt_bf16(const void* a, int64_t lda, const void* b, int6
   g.k = (int)k;
   StoreParams sp;
   sp.out_f32 = out; sp.ld_f32 = ldo; sp.out_bf16 = nullptr; sp.ld_bf16 = 0;
-  sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 1; sp.tile_acc = nullptr;
+  sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 0; sp.tile_acc = nullptr;
+  sp.splits = 1; sp.k_split = (int)k;
   return launch_store(g, sp, (hipStream_t)stream);
 }
 
@@ -1543,7 +1632,8 @@ extern "C" int axon_gemm_bf16(const void* a, int64_t lda, int a_kmajor, const vo
   if (!gemm_kmajor_domain(g, a_kmajor != 0, b_kmajor != 0)) return AXON_ERR_SHAPE;
   StoreParams sp;
   sp.out_f32 = out; sp.ld_f32 = ldo; sp.out_bf16 = nullptr; sp.ld_bf16 = 0;
-  sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 1; sp.tile_acc = nullptr;
+  sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 0; sp.tile_acc = nullptr;
+  sp.splits = 1; sp.k_split = (int)k;
   return launch_store_kmajor(g, sp, a_kmajor != 0, b_kmajor != 0, (hipStream_t)stream);
 }
 
@@ -1571,12 +1661,12 @@ extern "C" int64_t axon_lmhead_block_dw_acc_bytes(int64_t h, int64_t v) {
 
 extern "C" int axon_lmhead_bwd_dlogit_copies(int64_t h, int64_t v, int64_t chunk) {
   if (check_head_shape(0, h, v) != AXON_OK || chunk < 0 || chunk % kTile != 0) return -1;
-  return bwd_ws(kTile, h, v, chunk, nullptr).dl_kmajor ? 1 : 2;
+  return bwd_ws(kTile, h, v, chunk > 0 ? chunk : kDefaultVocabChunk, nullptr).dl_kmajor ? 1 : 2;
 }
 
 extern "C" int axon_lmhead_block_can_group(int64_t h, int64_t v, int64_t chunk) {
   if (check_head_shape(0, h, v) != AXON_OK || chunk < 0 || chunk % kTile != 0) return 0;
-  const BwdWs w = bwd_ws(kTile, h, v, chunk, nullptr);
+  const BwdWs w = bwd_ws(kTile, h, v, chunk > 0 ? chunk : kDefaultVocabChunk, nullptr);
   return (w.dl_kmajor && w.chunks == 1) ? 1 : 0;
 }
 

@@ -854,3 +854,23 @@ def test_ragged_tile_edges_of_the_dma_loop_vs_oracle(n, h, v):
     assert hb.block_stash_bytes > 0 and torch.equal(hb.logprobs, lp) and torch.equal(hb.entropy, ent)
     hb.backward(0, g_lp.to(DEV), g_en.to(DEV))
     assert rel_l2(hb.d_hidden, ref_dh) < 2e-2 and rel_l2(hb.d_weight, ref_dw) < 2e-2
+
+
+@pytest.mark.parametrize("n,h,v,chunk", [
+    (5, 64, 4096, 0), (70, 256, 4100, 0),            # the shortest vocabulary that is reduced in parts (64 k-tiles)
+    (300, 256, 9001, 0), (513, 320, 20000, 0),       # a shorter last part, several tiles
+    (200, 256, 8192 + 136, 4096), (40, 128, 13000, 6144),  # chunks: the last one reaches the first parts only
+])
+def test_split_reduction_of_d_hidden_vs_oracle(n, h, v, chunk):
+    """dHidden over a long vocabulary and few tokens: several workgroups share a tile's reduction."""
+    hid, w, lab = W.lmhead_inputs(n, h, v, seed=n + h + v)
+    w = (w.float() * 8).bfloat16()
+    hd, wd, ld = hid.to(DEV), w.to(DEV), lab.to(DEV)
+    g = torch.Generator().manual_seed(10)
+    g_lp = torch.randn(n, generator=g) / n
+    _, _, lse, eb = _ops.lmhead_forward(hd, wd, ld, 1.0)
+    dh, dw = _ops.lmhead_backward(g_lp.to(DEV), None, hd, wd, ld, lse, eb, 1.0, vocab_chunk=chunk)
+    again = _ops.lmhead_backward(g_lp.to(DEV), None, hd, wd, ld, lse, eb, 1.0, vocab_chunk=chunk)
+    assert torch.equal(dh, again[0]) and torch.equal(dw, again[1])  # the parts are added in a fixed order
+    ref_dh, ref_dw = OM.backward(g_lp, None, hid, w, lab)
+    assert rel_l2(dh, ref_dh) < 2e-2 and rel_l2(dw, ref_dw) < 2e-2
