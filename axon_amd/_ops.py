@@ -596,7 +596,7 @@ TIMING: "Timer | None" = None
 # vocab chunk of the LM-head backward used when the caller passes 0 (0 = library default)
 DEFAULT_VOCAB_CHUNK = 0
 
-_PHASES = ("fwd/logits_stats", "fwd/merge", "fwd/label", "fwd/unused",
+_PHASES = ("fwd/logits_stats", "fwd/merge", "fwd/unused2", "fwd/unused3",
            "bwd/transpose", "bwd/dlogit", "bwd/dhidden", "bwd/dweight")
 
 

@@ -247,94 +247,115 @@ __global__ __launch_bounds__(256) void seq_start_kernel(const int32_t* __restric
   if (s0 >= 0 && s0 < n_tokens && cu[i + 1] > s0) is_start[s0] = 1;  // empty sequences own no position
 }
 
-// Merge partials: lse, entropy_b, entropy.  A workgroup owns kMergeTokens consecutive tokens; its
-// kMergeGroups thread groups each fold every kMergeGroups-th partial of a token (four loads ahead of the
-// fold), then the first group folds the groups' results in group order.
-constexpr int kMergeTokens = 32;
-constexpr int kMergeGroups = 8;
-
-__global__ __launch_bounds__(kMergeTokens * kMergeGroups) void lmhead_merge_kernel(
+// The last kernel of the forward: folds a token's partials into lse, entropy_b and entropy, forms the label's
+// logit and with it logprob[n] = softcap(hidden[n] . W[label[n]]) / T - lse[n].
+// A workgroup of 1024 threads owns 16 * PER consecutive tokens (a thread PER of them, 16 apart); its 64 thread groups each fold every 64th partial of a
+// token (four loads ahead of the fold), so that the chain of dependent folds is 19 long for 151936 vocabulary
+// rows (149 with eight groups of 32 tokens).  Groups of one wavefront are folded by lane exchanges, the wavefronts
+// through LDS in order: the same order whatever the number of tokens.  The label dots (one wavefront per token) run
+// before the barrier, beside the folds of the other wavefronts.  PER = 2 (both halves of a 128-byte line by the same
+// thread) once a workgroup per 16 tokens would be more than one per CU.
+// 187 tokens x 896 x 151936: 11.0 us where separate merge and label kernels took 18.7 + 5.2; 700 x 4096: 19.4 for
+// 26.0 + 7.4; 8192 x 4096: 51 for 33.2 + 23.3.
+constexpr int kFinishTokens = 16;
+template <int PER, typename LabelT>
+__global__ __launch_bounds__(1024) void lmhead_finish_kernel(
     const float* __restrict__ pm, const float* __restrict__ ps, const float* __restrict__ pe,
-    int parts, int n_tokens, float* __restrict__ lse, float* __restrict__ entropy_b,
-    float* __restrict__ entropy, float* __restrict__ fin_max, float* __restrict__ fin_log2s,
-    const uint8_t* __restrict__ is_start, int last_dst) {
-  __shared__ float red[3][kMergeGroups][kMergeTokens];
-  const int tok = threadIdx.x % kMergeTokens, grp = threadIdx.x / kMergeTokens;
-  const int n = blockIdx.x * kMergeTokens + tok;
-  const int nc = n < n_tokens ? n : n_tokens - 1;  // a valid token; its result is dropped below
-  float M = 0.f, s = 0.f, e = 0.f;
-  bool any = false;  // a group beyond the number of partials folds nothing
-  auto fold = [&](float M2, float s2, float e2) {
-    if (!any) { M = M2; s = s2; e = e2; any = true; return; }
-    const float Mn = fmaxf(M, M2);
-    merge_stats(M, s, e, M2, s2, e2, Mn);
-    M = Mn;
+    int parts, const __bf16* __restrict__ hidden, const __bf16* __restrict__ weight,
+    const LabelT* __restrict__ labels, int n_tokens, int hidden_sz, int vocab, float inv_temp, float cap,
+    float* __restrict__ lse, float* __restrict__ entropy_b, float* __restrict__ entropy,
+    float* __restrict__ logprobs, const uint8_t* __restrict__ is_start, int last_dst) {
+  constexpr int TOK = kFinishTokens * PER, kGroups = 1024 / kFinishTokens, kWaves = 16;
+  __shared__ float red[3][kWaves][TOK];
+  __shared__ float dots[TOK];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int grp = threadIdx.x / kFinishTokens;
+  int nc[PER];
+#pragma unroll
+  for (int t = 0; t < PER; ++t)  // a valid token; the results of those beyond the last are dropped below
+    nc[t] = min(blockIdx.x * TOK + t * kFinishTokens + (int)(threadIdx.x % kFinishTokens), n_tokens - 1);
+  // a group beyond the number of partials holds an empty set (s = 0 below any reference)
+  float M[PER], s[PER], e[PER];
+#pragma unroll
+  for (int t = 0; t < PER; ++t) { M[t] = kEmptyMax; s[t] = 0.f; e[t] = 0.f; }
+  auto fold = [](float& M1, float& s1, float& e1, float M2, float s2, float e2) {
+    const float Mn = fmaxf(M1, M2);
+    merge_stats(M1, s1, e1, M2, s2, e2, Mn);
+    M1 = Mn;
   };
   int q = grp;
-  for (; q + 3 * kMergeGroups < parts; q += 4 * kMergeGroups) {
-    float M2[4], s2[4], e2[4];
+  for (; q + 3 * kGroups < parts; q += 4 * kGroups) {
+    float M2[4][PER], s2[4][PER], e2[4][PER];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t o = (int64_t)(q + u * kMergeGroups) * n_tokens + nc;
-      M2[u] = pm[o]; s2[u] = ps[o]; e2[u] = pe[o];
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < PER; ++t) {
+        const int64_t o = (int64_t)(q + u * kGroups) * n_tokens + nc[t];
+        M2[u][t] = pm[o]; s2[u][t] = ps[o]; e2[u][t] = pe[o];
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < PER; ++t) fold(M[t], s[t], e[t], M2[u][t], s2[u][t], e2[u][t]);
+  }
+  for (; q < parts; q += kGroups) {
+#pragma unroll
+    for (int t = 0; t < PER; ++t) {
+      const int64_t o = (int64_t)q * n_tokens + nc[t];
+      fold(M[t], s[t], e[t], pm[o], ps[o], pe[o]);
     }
+  }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) fold(M2[u], s2[u], e2[u]);
+  for (int t = 0; t < PER; ++t) {
+#pragma unroll
+    for (int off = kFinishTokens; off < 64; off <<= 1)
+      fold(M[t], s[t], e[t], __shfl_xor(M[t], off), __shfl_xor(s[t], off), __shfl_xor(e[t], off));
+    if (lane < kFinishTokens) {
+      const int tok = t * kFinishTokens + lane;
+      red[0][wave][tok] = M[t]; red[1][wave][tok] = s[t]; red[2][wave][tok] = e[t];
+    }
   }
-  for (; q < parts; q += kMergeGroups) {
-    const int64_t o = (int64_t)q * n_tokens + nc;
-    fold(pm[o], ps[o], pe[o]);
-  }
-  red[0][grp][tok] = M; red[1][grp][tok] = s; red[2][grp][tok] = e;
-  __syncthreads();
-  if (grp != 0 || n >= n_tokens) return;
-  for (int g2 = 1; g2 < kMergeGroups && g2 < parts; ++g2)
-    fold(red[0][g2][tok], red[1][g2][tok], red[2][g2][tok]);
-  // log2 units: logsumexp = M + L, sum softmax*logit = M + e/s; differences are taken
-  // before adding M so that large logits do not cancel
-  const float L = __log2f(s);
-  const float d = e / s;
-  lse[n] = (M + L) * kLn2;
-  entropy_b[n] = (M + d) * kLn2;
-  const int dst = aligned_pos(n, n_tokens, is_start, last_dst);
-  entropy[dst] = (is_start && is_start[dst]) ? 0.f : (L - d) * kLn2;
-  fin_max[n] = M;
-  fin_log2s[n] = L;
-}
 
-// logprob[n] = softcap(hidden[n] . W[label[n]]) / T - lse[n].  One wave per token.
-template <typename LabelT>
-__global__ __launch_bounds__(256) void lmhead_label_kernel(
-    const __bf16* __restrict__ hidden, const __bf16* __restrict__ weight,
-    const LabelT* __restrict__ labels, int n_tokens, int hidden_sz, int vocab, float inv_temp,
-    float cap, const float* __restrict__ fin_max, const float* __restrict__ fin_log2s,
-    float* __restrict__ logprobs, const uint8_t* __restrict__ is_start, int last_dst) {
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= n_tokens) return;
-  const int lane = threadIdx.x & 63;
-  const int dst = aligned_pos(n, n_tokens, is_start, last_dst);
-  const int64_t lab = (int64_t)labels[dst];
-  float dot = 0.f;
-  if (lab >= 0 && lab < vocab) {
-    const uint4* h = reinterpret_cast<const uint4*>(hidden + (int64_t)n * hidden_sz);
-    const uint4* w = reinterpret_cast<const uint4*>(weight + lab * hidden_sz);
-    for (int c = lane; c < hidden_sz / 8; c += 64) {
-      const uint4 hv = h[c], wv = w[c];
-      const uint32_t hs[4] = {hv.x, hv.y, hv.z, hv.w}, ws[4] = {wv.x, wv.y, wv.z, wv.w};
+  for (int k = wave; k < TOK; k += kWaves) {  // label dots
+    const int nk = blockIdx.x * TOK + k;
+    if (nk >= n_tokens) break;
+    const int64_t lab = (int64_t)labels[aligned_pos(nk, n_tokens, is_start, last_dst)];
+    float dot = 0.f;
+    if (lab >= 0 && lab < vocab) {
+      const uint4* h = reinterpret_cast<const uint4*>(hidden + (int64_t)nk * hidden_sz);
+      const uint4* w = reinterpret_cast<const uint4*>(weight + lab * hidden_sz);
+#pragma unroll 4
+      for (int c = lane; c < hidden_sz / 8; c += 64) {
+        const uint4 hv = h[c], wv = w[c];
+        const uint32_t hs[4] = {hv.x, hv.y, hv.z, hv.w}, ws[4] = {wv.x, wv.y, wv.z, wv.w};
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        dot = fmaf(__uint_as_float(hs[k] << 16), __uint_as_float(ws[k] << 16), dot);
-        dot = fmaf(__uint_as_float(hs[k] & 0xffff0000u), __uint_as_float(ws[k] & 0xffff0000u), dot);
+        for (int i = 0; i < 4; ++i) {
+          dot = fmaf(__uint_as_float(hs[i] << 16), __uint_as_float(ws[i] << 16), dot);
+          dot = fmaf(__uint_as_float(hs[i] & 0xffff0000u), __uint_as_float(ws[i] & 0xffff0000u), dot);
+        }
       }
     }
+    dot = wave_sum(dot);
+    if (cap != 0.f) dot = cap * fast_tanh(dot / cap);
+    if (lane == 0) dots[k] = dot;
   }
-  dot = wave_sum(dot);
-  if (cap != 0.f) dot = cap * fast_tanh(dot / cap);
+  __syncthreads();
+  const int tok = threadIdx.x, n = blockIdx.x * TOK + tok;
+  if (tok >= TOK || n >= n_tokens) return;
+  float Mt = red[0][0][tok], st = red[1][0][tok], et = red[2][0][tok];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) fold(Mt, st, et, red[0][w][tok], red[1][w][tok], red[2][w][tok]);
+  // log2 units: logsumexp = M + L, sum softmax*logit = M + e/s; differences are taken
+  // before adding M so that large logits do not cancel
+  const float L = __log2f(st);
+  const float d = et / st;
+  lse[n] = (Mt + L) * kLn2;
+  entropy_b[n] = (Mt + d) * kLn2;
+  const int dst = aligned_pos(n, n_tokens, is_start, last_dst);
+  const bool start = is_start && is_start[dst];
+  entropy[dst] = start ? 0.f : (L - d) * kLn2;
   // (logit*c - M) is formed in one rounding, then log2(sum) is subtracted: no cancellation
-  if (lane == 0) {
-    const float lpv = (fmaf(dot, inv_temp * kLog2e, -fin_max[n]) - fin_log2s[n]) * kLn2;
-    logprobs[dst] = (is_start && is_start[dst]) ? 0.f : lpv;
-  }
+  logprobs[dst] = start ? 0.f : (fmaf(dots[tok], inv_temp * kLog2e, -Mt) - L) * kLn2;
 }
 
 // ----------------------------------------------------------------------------
@@ -947,6 +968,7 @@ inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 constexpr int64_t kDefaultVocabChunk = 32768;
 constexpr int64_t kDefaultChunkElems = int64_t(1) << 30;
 constexpr int64_t kAlign = 256;
+constexpr int kCus = 256;
 using SlowLoop = RegLoop<32>;
 
 // Leading dimensions whose byte offsets inside a tile (256 rows K-contiguous, 64 K-major) stay below 2^30
@@ -982,7 +1004,6 @@ int set_lds(K kernel) {
 
 struct FwdWs {
   float *pm, *ps, *pe;
-  float *fin_max, *fin_log2s;  // [n] merged max and log2(sum), for the label kernel
   int parts;
   int64_t bytes;
 };
@@ -994,10 +1015,7 @@ FwdWs fwd_ws(int64_t n, int64_t vocab, void* base) {
   w.pm = reinterpret_cast<float*>(p);
   w.ps = reinterpret_cast<float*>(p + one);
   w.pe = reinterpret_cast<float*>(p + 2 * one);
-  const int64_t fin = round_up(n * 4, kAlign);
-  w.fin_max = reinterpret_cast<float*>(p + 3 * one);
-  w.fin_log2s = reinterpret_cast<float*>(p + 3 * one + fin);
-  w.bytes = 3 * one + 2 * fin;
+  w.bytes = 3 * one;
   return w;
 }
 
@@ -1036,7 +1054,7 @@ bool stash_of_all_tokens(int64_t n, int64_t h, int64_t v) {
 // stay whole.
 // At most kMaxUnits tile parts (three rounds, 200 MB of partial sums, which the Infinity Cache holds).
 // A part has at least kMinPartTiles k-tiles: below that its first loads and its epilogue are a quarter of its time.
-constexpr int kCus = 256, kMaxSplits = 64, kMaxUnits = 3 * kCus, kMinPartTiles = 32;
+constexpr int kMaxSplits = 64, kMaxUnits = 3 * kCus, kMinPartTiles = 32;
 struct SplitPlan { int splits, k_split; };
 SplitPlan split_plan(int64_t tiles, int64_t k) {
   const int64_t kt = (k + 63) / 64;
@@ -1249,26 +1267,19 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
       AXON_LAUNCH_GEMM(lmhead_fwd_kernel, g, p, st);
     }
   }
-  {
-    Span span(timer, 1);
-    hipLaunchKernelGGL(lmhead_merge_kernel, dim3((unsigned)((n + kMergeTokens - 1) / kMergeTokens)),
-                       dim3(kMergeTokens * kMergeGroups), 0, st,
-                       w.pm, w.ps, w.pe, w.parts, (int)n, lse, entropy_b, entropy, w.fin_max,
-                       w.fin_log2s, is_start, (int)last_dst);
+  Span span(timer, 1);
+#define AXON_FINISH(PER, LabelT)                                                                                 \
+  hipLaunchKernelGGL((lmhead_finish_kernel<PER, LabelT>),                                                        \
+                     dim3((unsigned)((n + kFinishTokens * PER - 1) / (kFinishTokens * PER))), dim3(1024), 0, st, \
+                     w.pm, w.ps, w.pe, w.parts, static_cast<const __bf16*>(hidden),                              \
+                     static_cast<const __bf16*>(weight), static_cast<const LabelT*>(labels), (int)n, (int)h,     \
+                     (int)v, inv_temp, softcap, lse, entropy_b, entropy, logprobs, is_start, (int)last_dst)
+  if (n > kFinishTokens * kCus) {
+    if (labels_i64) AXON_FINISH(2, int64_t); else AXON_FINISH(2, int32_t);
+  } else {
+    if (labels_i64) AXON_FINISH(1, int64_t); else AXON_FINISH(1, int32_t);
   }
-  AXON_CHECK_LAUNCH();
-  const dim3 lg((unsigned)((n + 3) / 4));
-  Span span(timer, 2);
-  if (labels_i64)
-    hipLaunchKernelGGL(lmhead_label_kernel<int64_t>, lg, dim3(256), 0, st,
-                       static_cast<const __bf16*>(hidden), static_cast<const __bf16*>(weight),
-                       static_cast<const int64_t*>(labels), (int)n, (int)h, (int)v, inv_temp,
-                       softcap, w.fin_max, w.fin_log2s, logprobs, is_start, (int)last_dst);
-  else
-    hipLaunchKernelGGL(lmhead_label_kernel<int32_t>, lg, dim3(256), 0, st,
-                       static_cast<const __bf16*>(hidden), static_cast<const __bf16*>(weight),
-                       static_cast<const int32_t*>(labels), (int)n, (int)h, (int)v, inv_temp,
-                       softcap, w.fin_max, w.fin_log2s, logprobs, is_start, (int)last_dst);
+#undef AXON_FINISH
   AXON_CHECK_LAUNCH();
   return AXON_OK;
 }

@@ -166,7 +166,7 @@ int axon_lmhead_scatter_rows(const void* d_hidden_c_bf16, const int32_t* row_ran
  * axon_timer_collect synchronises the timer's stream, ADDS the elapsed milliseconds
  * and launch counts of everything recorded since the last collect to the two HOST
  * arrays of 8 entries (zero them first) and forgets the spans:
- *   [0] forward logits+statistics kernel, [1] merge, [2] label logit, [3] unused,
+ *   [0] forward logits+statistics kernel, [1] merge of the statistics and label logit, [2], [3] unused,
  *   [4] backward transposes, [5] dlogit (recompute, or decode of the stash), [6] dHidden GEMM, [7] dWeight GEMM.
  * The timer creates and destroys events and owns host memory (the exception to
  * "never allocates"); `stream` of a timed call must be the timer's.
