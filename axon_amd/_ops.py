@@ -181,6 +181,35 @@ def row_broadcast_mask(row_scalar, mask, rows: Rows, clamp_abs=0.0):
     return out
 
 
+GROUP_ADVANTAGE_MAX_GROUPS = 2048  # the groups' sums live in a workgroup's LDS
+
+
+def group_advantage(rewards, mask, gidx, n_groups, rows: Rows, *, eps, mode, clamp_abs=0.0):
+    """Row scores, group statistics, per-row scalar (``mode``: axon_group_stats' norm_by_std) and broadcast over the
+    mask.  Two launches (axon_group_advantage) unless the rows are very short or long on average or there are more
+    groups than fit in LDS; the row pass, group kernel and broadcast one by one then."""
+    if 0 < n_groups <= GROUP_ADVANTAGE_MAX_GROUPS and _own_rows(rows):
+        lib = _lib.load()
+        require_device(rewards, "group_advantage")
+        _same_len("group_advantage", rows.n_slots, rewards=rewards, mask=mask)
+        _same_len("group_advantage", rows.n_rows, gidx=gidx)
+        dev = rewards.device
+        rw = f32(rewards)
+        mk, kind = mask_arg(mask)
+        scratch = torch.empty(2 * rows.n_rows, device=dev, dtype=torch.float32)
+        out = torch.empty(rows.shape, device=dev, dtype=torch.float32)
+        check(
+            lib.axon_group_advantage(ptr(rw), ptr(mk), kind, rows.cu_ptr, rows.n_rows, rows.n_slots, rows.uniform_len,
+                                     ptr(gidx), int(n_groups), float(eps), int(mode), float(clamp_abs), ptr(scratch),
+                                     ptr(out), ptr(_partials(rows.n_slots, dev)), stream_ptr()),
+            "axon_group_advantage",
+        )
+        return out
+    _, scores, _ = row_stats(rewards, None, None, rows, want_cnt=False)
+    _, _, _, scalar = group_stats(scores, gidx, n_groups, eps, mode)
+    return row_broadcast_mask(scalar, mask, rows, clamp_abs=clamp_abs)
+
+
 SCAN_GAE, SCAN_GAE_RESPONSE_ONLY, SCAN_DISCOUNTED, SCAN_SUFFIX_SUM = 0, 1, 2, 3
 
 

@@ -168,6 +168,26 @@ __global__ __launch_bounds__(kBlock) void row_stats_kernel(
   }
 }
 
+struct GroupCfg {
+  int64_t n_groups;
+  float eps;
+  int mode;  // 0 centred, 1 centred and divided by the standard deviation, 2 RLOO, 3 GPG
+};
+
+// GRPO / RLOO / GPG scalar of a row with score x in a group of c rows with mean mu and deviation sd (advantage.py:78-146,
+// 336-371); alpha: rows over rows with a non-zero score.
+__device__ __forceinline__ float group_scalar_of(const GroupCfg& g, float x, float c, float mu, float sd, float alpha) {
+  float v;
+  if (g.mode == 2) {  // (n*s - S) / (n - 1), S = n * mean
+    v = (c * x - c * mu) / fmaxf(c - 1.f, 1.f);
+  } else if (g.mode == 3) {  // alpha * (s - mean) / f_norm, eps carries f_norm; singletons have mean 0 and keep their score
+    return alpha * (x - mu) / g.eps;
+  } else {
+    v = g.mode ? (x - mu) / (sd + g.eps) : (x - mu);
+  }
+  return v * ((c > 1.f) ? 1.f : 0.f);
+}
+
 // group_mean_std + GRPO scalar, one workgroup.
 __global__ __launch_bounds__(1024) void group_stats_kernel(
     const float* __restrict__ scores, const int64_t* __restrict__ gidx, int64_t n_rows,
@@ -206,19 +226,94 @@ __global__ __launch_bounds__(1024) void group_stats_kernel(
     const int64_t g = gidx[i];
     if (g < 0 || g >= n_groups) { scalar[i] = 0.f; continue; }
     const float x = scores[i];
-    const float c = count[g];
-    float v;
-    if (norm_by_std == 2) {  // RLOO / LOOP: (n*s - S) / (n - 1), S = n * mean (advantage.py:112-146)
-      v = (c * x - c * mean[g]) / fmaxf(c - 1.f, 1.f);
-    } else if (norm_by_std == 3) {  // GPG: alpha * (s - mean) / f_norm, eps carries f_norm (:336-371)
-      const float alpha = (float)n_rows / (float)max(nonzero, 1);
-      scalar[i] = alpha * (x - mean[g]) / eps;  // singleton groups have mean 0 and keep their score
-      continue;
-    } else {
-      v = norm_by_std ? (x - mean[g]) / (stdv[g] + eps) : (x - mean[g]);
+    const float alpha = (float)n_rows / (float)max(nonzero, 1);
+    scalar[i] = group_scalar_of(GroupCfg{n_groups, eps, norm_by_std}, x, count[g], mean[g], stdv[g], alpha);
+  }
+}
+
+// Row sums and, in the workgroup that ends last, the group statistics and the per-row scalar of the group-based
+// estimators: with row_broadcast_kernel behind it an advantage is two launches, no zero fills and no float atomics
+// in memory.  A wavefront owns a row (double accumulators per lane, then a fixed tree), four 16-byte loads in flight;
+// the grid is bounded so that its tickets stay cheap.  The groups' sums are formed in LDS (double, so that the order
+// in which the rows arrive does not show in the fp32 results).
+// 128 x 1024 slots, 16 groups: 8.3 us where fill, row pass, finish and group kernel took 6.9 + 1.3 + 10.9 and two fills;
+// 8.4 M slots in 9000 rows, 1150 groups: 40 for 27 + 4.7 + 80.
+constexpr int kScoreGroups = 2048;  // 40 KB of LDS
+constexpr int kScoreBlocks = 1024;
+
+__global__ __launch_bounds__(1024) void group_scores_kernel(
+    const float* __restrict__ a, const int32_t* __restrict__ cu, int64_t n_rows, int64_t n_slots, int64_t uniform_len,
+    const int64_t* __restrict__ gidx, GroupCfg g, float* scores, float* __restrict__ scalar, unsigned* ticket) {
+  __shared__ double sums[kScoreGroups][2];
+  __shared__ int count[kScoreGroups];
+  __shared__ int last, nonzero;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
+  for (int64_t r = (int64_t)blockIdx.x * waves + wave; r < n_rows; r += (int64_t)gridDim.x * waves) {
+    int64_t t0 = uniform_len > 0 ? r * uniform_len : (int64_t)cu[r];
+    int64_t t1 = uniform_len > 0 ? t0 + uniform_len : (int64_t)cu[r + 1];
+    t0 = min(max(t0, (int64_t)0), n_slots);
+    t1 = min(max(t1, t0), n_slots);
+    double acc = 0.0;
+    const int64_t b0 = min((t0 + 3) & ~(int64_t)3, t1), b1 = max(t1 & ~(int64_t)3, b0);  // whole vectors
+    if (lane < b0 - t0) acc += (double)a[t0 + lane];
+    if (lane < t1 - b1) acc += (double)a[b1 + lane];
+    int64_t p = b0 + lane * kVec;
+    for (; p + 3 * kWave * kVec < b1; p += 4 * kWave * kVec) {
+      float v[4][4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) load4(a, p + u * kWave * kVec, v[u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc += ((double)v[u][0] + (double)v[u][1]) + ((double)v[u][2] + (double)v[u][3]);
     }
-    v = v * ((c > 1.f) ? 1.f : 0.f);
-    scalar[i] = v;
+    for (; p < b1; p += kWave * kVec) {
+      float v[4];
+      load4(a, p, v);
+      acc += ((double)v[0] + (double)v[1]) + ((double)v[2] + (double)v[3]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, kWave);
+    if (lane == 0) __hip_atomic_store(scores + r, (float)acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // the scores' write-through stores are acknowledged before the workgroup draws its ticket (publish_row_take_ticket)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0)
+  __syncthreads();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  if (threadIdx.x == 0) {
+    const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = (t == gridDim.x - 1);
+    if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+    nonzero = 0;
+  }
+  const int n_groups = (int)g.n_groups;
+  for (int i = threadIdx.x; i < n_groups; i += blockDim.x) { sums[i][0] = 0.0; sums[i][1] = 0.0; count[i] = 0; }
+  __syncthreads();
+  if (!last) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  for (int64_t i = threadIdx.x; i < n_rows; i += blockDim.x) {
+    const int64_t k = gidx[i];
+    const float x = scores[i];
+    if (g.mode == 3 && x != 0.f) atomicAdd(&nonzero, 1);
+    if (k < 0 || k >= n_groups) continue;
+    atomicAdd(&count[k], 1);
+    atomicAdd(&sums[k][0], (double)x);
+    atomicAdd(&sums[k][1], (double)x * (double)x);
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < n_groups; k += blockDim.x) {  // sums -> mean and deviation, singletons 0 and 1
+    const double c = (double)count[k], cc = fmax(c, 1.0);
+    const double s1 = sums[k][0], s2 = sums[k][1];
+    const float var = (float)((s2 - s1 * s1 / cc) / fmax(c - 1.0, 1.0));
+    const bool one = count[k] <= 1;
+    sums[k][0] = one ? 0.0 : s1 / cc;
+    sums[k][1] = one ? 1.0 : (double)sqrtf(fmaxf(var, g.eps));
+  }
+  __syncthreads();
+  const float alpha = (float)n_rows / (float)max(nonzero, 1);
+  for (int64_t i = threadIdx.x; i < n_rows; i += blockDim.x) {
+    const int64_t k = gidx[i];
+    const bool ok = k >= 0 && k < n_groups;
+    scalar[i] = ok ? group_scalar_of(g, scores[i], (float)count[k], (float)sums[k][0], (float)sums[k][1], alpha) : 0.f;
   }
 }
 
@@ -404,6 +499,27 @@ extern "C" int axon_group_stats(const float* scores, const int64_t* gidx, int64_
                      n_rows, n_groups, eps, norm_by_std, mean, stdv, count, scalar);
   AXON_CHECK_LAUNCH();
   return AXON_OK;
+}
+
+extern "C" int axon_group_advantage(const float* rewards, const void* mask, int mask_kind, const int32_t* cu,
+                                    int64_t n_rows, int64_t n_slots, int64_t uniform_len, const int64_t* gidx,
+                                    int64_t n_groups, float eps, int mode, float clamp_abs, float* row_scratch,
+                                    float* out, float* partials, void* stream) {
+  int rc = check_rows(cu, n_rows, n_slots, uniform_len);
+  if (rc != AXON_OK) return rc;
+  if (n_slots == 0 || n_rows == 0) return AXON_OK;
+  if (n_groups <= 0 || n_groups > kScoreGroups) return AXON_ERR_SHAPE;
+  if (!rewards || !gidx || !row_scratch || !out || !partials || mode < 0 || mode > 3) return AXON_ERR_ARG;
+  if (reinterpret_cast<uintptr_t>(rewards) & 15) return AXON_ERR_ARG;
+  constexpr int kWaves = 1024 / kWave;
+  const int64_t blocks = (n_rows + kWaves - 1) / kWaves;
+  hipLaunchKernelGGL(group_scores_kernel, dim3((unsigned)(blocks < kScoreBlocks ? blocks : kScoreBlocks)), dim3(1024), 0,
+                     (hipStream_t)stream, rewards, cu, n_rows, n_slots, uniform_len, gidx,
+                     GroupCfg{n_groups, eps, mode}, row_scratch, row_scratch + n_rows,
+                     reinterpret_cast<unsigned*>(partials + kTicketsOffset));
+  AXON_CHECK_LAUNCH();
+  return axon_row_broadcast_mask(row_scratch + n_rows, mask, mask_kind, cu, n_rows, n_slots, uniform_len, clamp_abs, out,
+                                 stream);
 }
 
 extern "C" int axon_row_broadcast_mask(const float* row_scalar, const void* mask, int mask_kind,

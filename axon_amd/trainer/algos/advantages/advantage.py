@@ -2,7 +2,7 @@
 
 ``grpo_advantage_fn`` follows advantage.py:78-109: score = sum_t token_level_rewards, per-uid mean/std
 (Bessel, std floored at sqrt(eps), then +eps again in the divide), singleton groups -> 0, broadcast over
-``response_mask``.  Three launches: ragged row sum, one-workgroup group statistics, masked broadcast.  The
+``response_mask``.  Two launches: row sums with the group statistics behind them, masked broadcast.  The
 other group-based estimators differ in the per-row scalar only.  The return-based estimators (GAE,
 REINFORCE++, ReMax) run their time recurrence as a wavefront scan per row, then the global masked
 whitening where the reference has one.  Group labels are ranked on the host (they are strings); nothing
@@ -94,8 +94,6 @@ def _group_advantage(data, mode: int, eps: float, clamp_abs: float):
     rewards, home = _stage(data.batch["token_level_rewards"])
     mask, _ = _stage(data.batch["response_mask"])
     uid = data.non_tensor_batch["uid"]
-    norm = mode
-
     cu = data.meta_info.get("cu_seqlens", None) if data.meta_info else None
     rows = _ops.rows_of(rewards, cu)
     # group ids are ranked on the host (labels are strings); the group count is read there as well, so
@@ -103,9 +101,7 @@ def _group_advantage(data, mode: int, eps: float, clamp_abs: float):
     gidx_host, n_groups, gidx = _ranked_groups(uid, rewards.device)
     if gidx_host.numel() != rows.n_rows:
         raise ValueError(f"uid has {gidx_host.numel()} entries, batch has {rows.n_rows} rows")
-    _, scores, _ = _ops.row_stats(rewards, None, None, rows, want_cnt=False)
-    _, _, _, scalar = _ops.group_stats(scores, gidx, n_groups, eps, norm)
-    adv = _ops.row_broadcast_mask(scalar, mask, rows, clamp_abs=clamp_abs)
+    adv = _ops.group_advantage(rewards, mask, gidx, n_groups, rows, eps=eps, mode=mode, clamp_abs=clamp_abs)
     if home is not None:
         adv = adv.to(home)
     return adv, adv

@@ -1161,3 +1161,33 @@ def test_all_padding_micro_batch_is_a_no_op_before_any_validation():
             S.compute_sampler_correction_and_rejection_mask(z, z, torch.ones_like(z), **kw)
     proto, mask, m = S.compute_sampler_correction_and_rejection_mask(z, torch.zeros(2, 5, device=DEV), z)
     assert proto is None and m == {}
+
+
+@pytest.mark.parametrize("name", ["grpo", "rloo", "gpg"])
+@pytest.mark.parametrize("rows,t,group", [
+    (3, 67, 2), (64, 257, 8), (130, 1031, 1),   # rows off 16-byte boundaries, a short last group, singletons only
+    (17, 4096, 5), (1030, 64, 4), (4100, 64, 2), (4096, 65, 2), (5000, 64, 2),  # 2050 and 2500 groups: the separate kernels
+])
+def test_group_advantage_in_two_launches_vs_oracle(name, rows, t, group):
+    """Row sums with the group statistics in the last workgroup, against the oracle, padded and packed, and the same
+    bits on every run."""
+    g = torch.Generator().manual_seed(rows + t)
+    rew = torch.zeros(rows, t)
+    # Scores are integers up to 7: their sums and squares are exact in fp32, so the two sides differ by the rounding of
+    # a square root and two divisions, 4 * 2^-24 relative.  (With continuous scores two close ones of a group of
+    # two make the oracle's own fp32 variance, sum of squares minus square of the sum, wrong by 2^-24 * s2 / var.)
+    rew[torch.arange(rows), torch.randint(0, t, (rows,), generator=g)] = torch.randint(0, 8, (rows,), generator=g).float()
+    mask = (torch.rand(rows, t, generator=g) < 0.7).float()
+    uid = W.uids_for(rows, group)
+    gidx = T(np.unique(uid, return_inverse=True)[1])
+    fn = {"grpo": OA.grpo_advantage, "rloo": OA.rloo_advantage, "gpg": OA.gpg_advantage}[name]
+    ref = fn(rew, mask, gidx)
+    out = compute_advantage(_grpo_proto(rew, mask, uid), {"advantage": name}).batch["advantages"]
+    assert torch.allclose(out.cpu(), ref, rtol=1e-6, atol=1e-6)
+    cu = torch.arange(0, rows * t + 1, t, dtype=torch.int32)
+    packed = _grpo_proto(rew.reshape(-1), mask.reshape(-1), uid, meta={"cu_seqlens": cu.to(DEV)})
+    got = compute_advantage(packed, {"advantage": name}).batch["advantages"]
+    assert torch.equal(got.view(rows, t), out)
+    if len(np.unique(uid)) <= 2048:
+        again = compute_advantage(_grpo_proto(rew, mask, uid), {"advantage": name}).batch["advantages"]
+        assert torch.equal(again, out)
