@@ -151,59 +151,68 @@ __device__ __forceinline__ bool publish_row_take_ticket(float* row, const float 
   return true;
 }
 
-// The sums finished inside the launch, in two levels.  Every workgroup publishes its row and takes a
-// ticket of its group of kFinishGroup workgroups; the workgroup that draws a group's last ticket adds
-// the group's rows (one wavefront: lane l takes row l, then the fixed tree of wave_sum), publishes
-// the group row and takes a ticket of the grid; the workgroup that draws the last of those adds the
-// group rows (thread t takes group t, then the fixed tree of block_sum) and hands the eight totals
-// to `fin` in its thread 0.  The order of every addition is fixed by the grid size alone.  The
-// counters must be zero when the kernel starts and are zero again when it ends.
+// The sums finished inside the launch.  A grid of at most kOneLevelGrid workgroups: every workgroup publishes its row and takes
+// a ticket of the grid; the workgroup that draws the last one adds the rows (thread t takes rows t, t + 256, ..., then
+// the fixed tree of block_sum) and hands the eight totals to `fin` in its thread 0.  A larger grid does it in two levels, groups of
+// kFinishGroup workgroups first (one wavefront adds a group: lane l takes row l, then the fixed tree of wave_sum), so
+// that no counter is drawn from by thousands; the second level costs 3.5 us (its own stores, ticket and loads at the
+// level the XCDs share), as much as everything else in a launch over a micro-batch.  The order of every addition is
+// fixed by the grid size alone.  The counters must be zero when the kernel starts and are zero again when it ends.
+constexpr unsigned kOneLevelGrid = 1024;
 template <int NV, class Fin>
 __device__ __forceinline__ void grid_finish(float (&v)[NV], float* lds /* [8 * 4] */, float* ws,
                                             Fin&& fin) {
   static_assert(NV <= kPartialStride, "partials row too small");
   __shared__ int s_stage;
   unsigned* tickets = reinterpret_cast<unsigned*>(ws + kTicketsOffset);
+  const bool one_level = gridDim.x <= kOneLevelGrid;
   const unsigned group = blockIdx.x / kFinishGroup;
   const unsigned n_groups = (gridDim.x + kFinishGroup - 1) / kFinishGroup;
   const unsigned first = group * kFinishGroup;
   const unsigned in_group = min((unsigned)kFinishGroup, gridDim.x - first);
+  auto read_row = [](const float* rows, unsigned i, bool ok, float (&t)[kPartialStride]) {
+    const float* row = rows + (size_t)(ok ? i : 0) * kPartialStride;
+    const float4 lo4 = *reinterpret_cast<const float4*>(row), hi4 = *reinterpret_cast<const float4*>(row + 4);
+    t[0] = ok ? lo4.x : 0.f; t[1] = ok ? lo4.y : 0.f; t[2] = ok ? lo4.z : 0.f; t[3] = ok ? lo4.w : 0.f;
+    t[4] = ok ? hi4.x : 0.f; t[5] = ok ? hi4.y : 0.f; t[6] = ok ? hi4.z : 0.f; t[7] = ok ? hi4.w : 0.f;
+  };
   block_sum<NV>(v, lds);
   if (threadIdx.x == 0) {
     float row[kPartialStride];
 #pragma unroll
     for (int k = 0; k < kPartialStride; ++k) row[k] = (k < NV) ? v[k < NV ? k : 0] : 0.f;
-    s_stage = publish_row_take_ticket(ws + (size_t)blockIdx.x * kPartialStride, row, tickets + 1 + group,
-                                      in_group) ? 1 : 0;
+    s_stage = publish_row_take_ticket(ws + (size_t)blockIdx.x * kPartialStride, row,
+                                      one_level ? tickets : tickets + 1 + group,
+                                      one_level ? gridDim.x : in_group) ? 1 : 0;
   }
   __syncthreads();
   if (s_stage == 0) return;
-  // every row of the group was acknowledged at the shared level before its ticket was drawn; drop
+  // every row was acknowledged at the shared level before its ticket was drawn; drop
   // what this XCD's caches may still hold of those addresses (an earlier launch), then read them
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  if (threadIdx.x < kWave) {
-    float t[kPartialStride];
-    const bool ok = threadIdx.x < in_group;
-    const float* row = ws + (size_t)(first + (ok ? threadIdx.x : 0)) * kPartialStride;
-    const float4 lo4 = *reinterpret_cast<const float4*>(row), hi4 = *reinterpret_cast<const float4*>(row + 4);
-    t[0] = ok ? lo4.x : 0.f; t[1] = ok ? lo4.y : 0.f; t[2] = ok ? lo4.z : 0.f; t[3] = ok ? lo4.w : 0.f;
-    t[4] = ok ? hi4.x : 0.f; t[5] = ok ? hi4.y : 0.f; t[6] = ok ? hi4.z : 0.f; t[7] = ok ? hi4.w : 0.f;
+  if (!one_level) {
+    if (threadIdx.x < kWave) {
+      float t[kPartialStride];
+      read_row(ws, first + threadIdx.x, threadIdx.x < in_group, t);
 #pragma unroll
-    for (int k = 0; k < kPartialStride; ++k) t[k] = wave_sum(t[k]);
-    if (threadIdx.x == 0)
-      s_stage = publish_row_take_ticket(ws + kGroupRowsOffset + (size_t)group * kPartialStride, t, tickets,
-                                        n_groups) ? 2 : 1;
+      for (int k = 0; k < kPartialStride; ++k) t[k] = wave_sum(t[k]);
+      if (threadIdx.x == 0)
+        s_stage = publish_row_take_ticket(ws + kGroupRowsOffset + (size_t)group * kPartialStride, t, tickets,
+                                          n_groups) ? 2 : 1;
+    }
+    __syncthreads();
+    if (s_stage != 2) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
-  __syncthreads();
-  if (s_stage != 2) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   float t[kPartialStride];
-  {
-    const bool ok = threadIdx.x < n_groups;  // n_groups <= kBlock
-    const float* row = ws + kGroupRowsOffset + (size_t)(ok ? threadIdx.x : 0) * kPartialStride;
-    const float4 lo4 = *reinterpret_cast<const float4*>(row), hi4 = *reinterpret_cast<const float4*>(row + 4);
-    t[0] = ok ? lo4.x : 0.f; t[1] = ok ? lo4.y : 0.f; t[2] = ok ? lo4.z : 0.f; t[3] = ok ? lo4.w : 0.f;
-    t[4] = ok ? hi4.x : 0.f; t[5] = ok ? hi4.y : 0.f; t[6] = ok ? hi4.z : 0.f; t[7] = ok ? hi4.w : 0.f;
+  const unsigned n_rows = one_level ? gridDim.x : n_groups;
+  const float* rows = one_level ? ws : ws + kGroupRowsOffset;
+  read_row(rows, threadIdx.x, threadIdx.x < n_rows, t);
+  for (unsigned i = threadIdx.x + kBlock; i < n_rows; i += kBlock) {
+    float u[kPartialStride];
+    read_row(rows, i, true, u);
+#pragma unroll
+    for (int k = 0; k < kPartialStride; ++k) t[k] += u[k];
   }
   block_sum<kPartialStride>(t, lds);  // the barriers above separate this use of `lds` from the first
   if (threadIdx.x == 0) fin(t);
@@ -211,11 +220,13 @@ __device__ __forceinline__ void grid_finish(float (&v)[NV], float* lds /* [8 * 4
 
 // Workgroups of a streaming launch: beyond this many chunks a workgroup walks several (every
 // workgroup publishes a row of partial sums and takes a ticket when it ends, which costs more than
-// the walk; 6144 measured best between 1024 and 16384 at 2^26 tokens).
+// the walk; 6144 measured best between 1024 and 16384 at 2^26 tokens; up to 2^24 tokens 1024, whose sums are
+// finished in one level: 8.4 M tokens 44.0 us against 46.3 with 2048).
 constexpr int kStreamGridCap = 6144;
-inline unsigned stream_grid(int64_t n_slots) {
-  const int64_t chunks = (n_slots + kChunk - 1) / kChunk;
-  return (unsigned)(chunks < kStreamGridCap ? chunks : kStreamGridCap);
+inline unsigned stream_grid(int64_t n_slots, int64_t chunk = kChunk) {
+  const int64_t chunks = (n_slots + chunk - 1) / chunk;
+  if (chunks > 4 * (int64_t)kOneLevelGrid) return (unsigned)(chunks < kStreamGridCap ? chunks : kStreamGridCap);
+  return (unsigned)(chunks < kOneLevelGrid ? chunks : kOneLevelGrid);
 }
 
 // 16-byte streaming accesses.  Every input of these kernels is read once and every output

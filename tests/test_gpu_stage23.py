@@ -1191,3 +1191,27 @@ def test_group_advantage_in_two_launches_vs_oracle(name, rows, t, group):
     if len(np.unique(uid)) <= 2048:
         again = compute_advantage(_grpo_proto(rew, mask, uid), {"advantage": name}).batch["advantages"]
         assert torch.equal(again, out)
+
+
+@pytest.mark.parametrize("n", [5, 1024, 1025, 262144, 262145, 524288, 524293, 4 * 1024 * 1024, 4 * 1024 * 1024 + 4097,
+                               16 * 1024 * 1024 + 3])
+def test_launch_shapes_of_the_streaming_loss(n):
+    """Vectors per thread, workgroup counts and the one- and two-level finishing of the sums change with the number of
+    slots: REINFORCE, whose loss and gradient are plain products, at the borders against float64."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    lp, adv = (torch.randn(1, n, generator=g, device=DEV) for _ in range(2))
+    mask = (torch.rand(1, n, generator=g, device=DEV) < 0.8).float()
+    rows = _ops.rows_of(lp)
+    kw = dict(token_reduce="sum", batch_reduce="token-mean", ratio_lo=0.8, ratio_hi=1.2, clip_c=3.0)
+    acc, grad = _ops.policy_loss(2, lp, lp, adv, mask, None, rows, **kw)
+    again, grad2 = _ops.policy_loss(2, lp, lp, adv, mask, None, rows, **kw)
+    assert torch.equal(acc, again) and torch.equal(grad, grad2)  # fixed order of every addition
+    assert torch.equal(grad, -adv * mask)
+    prod = -(adv.double() * lp.double() * mask.double())
+    # fp32 sums of n products: a thread's run of at most 2^14, then trees; each addition rounds by 2^-24 of the running sum
+    bound = 2.0 ** -24 * 32 * prod.abs().sum() / mask.sum()
+    assert (acc[0].double() - prod.sum() / mask.sum().double()).abs() <= bound + 1e-12
+    assert acc[4] == mask.sum(dtype=torch.float64).float()
+    ent, w, _ = _ops.side_terms(lp, None, None, mask, rows, token_reduce="sum", batch_reduce="token-mean")
+    assert torch.equal(w, mask) and (ent[0].double() - (lp.double() * mask).sum() / mask.sum().double()).abs() <= (
+        2.0 ** -24 * 32 * (lp.double().abs() * mask).sum() / mask.sum() + 1e-12)
