@@ -1044,11 +1044,13 @@ def logits_forward(logits, labels=None, want_entropy=True):
     n, v, ld = _logits_operands("logits_forward", logits, labels)
     dev = logits.device
     out = torch.empty(3, max(n, 1), device=dev, dtype=torch.float32)
+    ws_bytes = lib.axon_logits_fwd_workspace_bytes(_LOGITS_DTYPES[logits.dtype], n, v) if v > 0 else 0
+    ws = torch.empty(ws_bytes // 4, device=dev, dtype=torch.float32) if ws_bytes > 0 else None
     check(
-        lib.axon_logits_fwd(ptr(logits), _LOGITS_DTYPES[logits.dtype], ld, n, v, ptr(labels),
-                            int(labels is not None and labels.dtype == torch.int64),
-                            ptr(out[0]) if labels is not None else None, ptr(out[1]) if want_entropy else None,
-                            ptr(out[2]), stream_ptr()),
+        lib.axon_logits_fwd_ws(ptr(logits), _LOGITS_DTYPES[logits.dtype], ld, n, v, ptr(labels),
+                               int(labels is not None and labels.dtype == torch.int64),
+                               ptr(out[0]) if labels is not None else None, ptr(out[1]) if want_entropy else None,
+                               ptr(out[2]), ptr(ws), stream_ptr()),
         "axon_logits_fwd",
     )
     return (out[0][:n] if labels is not None else None), (out[1][:n] if want_entropy else None), out[2][:n]

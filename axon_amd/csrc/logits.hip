@@ -13,10 +13,13 @@ constexpr float kLn2 = 0.6931471805599453f;
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ float bf16_to_f32(unsigned short h) { return __uint_as_float((uint32_t)h << 16); }
-__device__ __forceinline__ unsigned short f32_to_bf16(float f) {  // round to nearest even, NaN kept
-  const uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40);
-  return (unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+// two floats to bf16, round to nearest even, NaN kept (one v_cvt_pk_bf16_f32; in integer arithmetic eight
+// instructions per value, which is what held the gradient kernel back)
+__device__ __forceinline__ uint32_t f32x2_to_bf16(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const f32x2 v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
 template <typename T> struct Row;
@@ -42,12 +45,12 @@ template <> struct Row<unsigned short> {
   }
   __device__ static float one(const unsigned short* p) { return bf16_to_f32(*p); }
   __device__ static void store(unsigned short* p, const float (&v)[8]) {
-    u16x8 x;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = f32_to_bf16(v[j]);
-    __builtin_nontemporal_store(x, reinterpret_cast<u16x8*>(p));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 x = {f32x2_to_bf16(v[0], v[1]), f32x2_to_bf16(v[2], v[3]), f32x2_to_bf16(v[4], v[5]),
+                     f32x2_to_bf16(v[6], v[7])};
+    __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(p));
   }
-  __device__ static void store_one(unsigned short* p, float v) { *p = f32_to_bf16(v); }
+  __device__ static void store_one(unsigned short* p, float v) { *p = (unsigned short)f32x2_to_bf16(v, 0.f); }
 };
 
 // Running statistics of a set of logits y (log2 units): M >= every y, s = sum 2^(y-M), e = sum 2^(y-M)(y-M).
@@ -92,31 +95,68 @@ __device__ __forceinline__ Stats merge(Stats a, Stats b) {
 }
 constexpr float kFloor = -1e30f;  // below any logit; finite, so that differences stay finite
 
-// One workgroup per token row.  VEC_OK: every row starts on a 16-byte boundary.
+// What one workgroup does of a row: the 16-byte vectors [q_lo, q_hi) of the row's aligned middle, counted from
+// element `head` on, and its share of the n_scalar elements outside it (before `head`, then behind the last vector).  An odd vocabulary puts every row on another boundary, so a row's first vector starts at its first
+// 16-byte boundary and not at its first element.
+struct RowSpan {
+  int head, n_vec, n_scalar, q_lo, q_hi;
+  template <typename T>
+  __device__ __forceinline__ RowSpan(const T* row, int vocab, bool vec_ok, int part, int parts) {
+    constexpr int kPer = Row<T>::kPer;
+    const int off = (int)((reinterpret_cast<uintptr_t>(row) & 15) / sizeof(T));
+    head = min((kPer - off) & (kPer - 1), vocab);
+    n_vec = vec_ok ? (vocab - head) / kPer : 0;
+    n_scalar = vocab - n_vec * kPer;
+    q_lo = (int)((int64_t)n_vec * part / parts);
+    q_hi = (int)((int64_t)n_vec * (part + 1) / parts);
+  }
+  template <typename T>
+  __device__ __forceinline__ int scalar(int i) const { return i < head ? i : i + n_vec * Row<T>::kPer; }
+};
+
+template <typename T, typename LabelT>
+__device__ __forceinline__ void write_stats(Stats st, int t, const T* row, int vocab, const LabelT* labels,
+                                            float* logprob, float* entropy, float* lse) {
+  const float L = __log2f(st.s), d = st.e / st.s;
+  const float lse_v = (st.M + L) * kLn2;
+  lse[t] = lse_v;
+  if (entropy != nullptr) entropy[t] = (L - d) * kLn2;  // lse - sum p z, the common max cancelled
+  if (logprob != nullptr) {
+    const int64_t lab = (int64_t)labels[t];
+    logprob[t] = (lab >= 0 && lab < vocab) ? Row<T>::one(row + lab) - lse_v : 0.f;
+  }
+}
+
+// Workgroup (part, row): blockIdx.x = row * parts + part.  One part writes the row's results, several leave their
+// statistics in ws[row][part][3] for logits_merge_kernel.  Bound by memory, 6.0 to 6.6 TB/s from 1100 rows on.
+// 2047 x 50257 bf16 39 us for 81 (rows off a 16-byte boundary), 187 x 151936 bf16 20 for 31, 300 x 151936 fp32 32 for 58.
 template <typename T, typename LabelT>
 __global__ __launch_bounds__(kBlock) void logits_stats_kernel(
     const T* __restrict__ logits, int64_t ld, int vocab, const LabelT* __restrict__ labels,
-    float* __restrict__ logprob, float* __restrict__ entropy, float* __restrict__ lse, int vec_ok) {
+    float* __restrict__ logprob, float* __restrict__ entropy, float* __restrict__ lse, int parts,
+    float* __restrict__ ws) {
   __shared__ float red[3][kBlock / kWave];
-  const T* row = logits + (int64_t)blockIdx.x * ld;
+  const int t = blockIdx.x / parts, part = blockIdx.x - t * parts;
+  const T* row = logits + (int64_t)t * ld;
   constexpr int kPer = Row<T>::kPer;
+  const RowSpan sp(row, vocab, true, part, parts);
   Stats st{kFloor, 0.f, 0.f};
-  const int n_vec = vec_ok ? vocab / kPer : 0;
-  int q = threadIdx.x;
-  for (; q + kBlock < n_vec; q += 2 * kBlock) {  // two loads in flight per thread
+  const T* body = row + sp.head;
+  int q = sp.q_lo + threadIdx.x;
+  for (; q + kBlock < sp.q_hi; q += 2 * kBlock) {  // two loads in flight per thread
     float v0[8], v1[8];
-    Row<T>::load(row + (int64_t)q * kPer, v0);
-    Row<T>::load(row + (int64_t)(q + kBlock) * kPer, v1);
+    Row<T>::load(body + (uint32_t)q * kPer, v0);
+    Row<T>::load(body + (uint32_t)(q + kBlock) * kPer, v1);
     fold<kPer>(st, v0);
     fold<kPer>(st, v1);
   }
-  for (; q < n_vec; q += kBlock) {
+  for (; q < sp.q_hi; q += kBlock) {
     float v[8];
-    Row<T>::load(row + (int64_t)q * kPer, v);
+    Row<T>::load(body + (uint32_t)q * kPer, v);
     fold<kPer>(st, v);
   }
-  for (int i = n_vec * kPer + threadIdx.x; i < vocab; i += kBlock) {
-    const float v[8] = {Row<T>::one(row + i)};
+  for (int i = part * kBlock + threadIdx.x; i < sp.n_scalar; i += parts * kBlock) {
+    const float v[8] = {Row<T>::one(row + sp.scalar<T>(i))};
     fold<1>(st, v);
   }
 #pragma unroll
@@ -132,49 +172,98 @@ __global__ __launch_bounds__(kBlock) void logits_stats_kernel(
   __syncthreads();
   if (threadIdx.x != 0) return;
   for (int w = 1; w < kBlock / kWave; ++w) st = merge(st, Stats{red[0][w], red[1][w], red[2][w]});
-  const float L = __log2f(st.s), d = st.e / st.s;
-  const float lse_v = (st.M + L) * kLn2;
-  lse[blockIdx.x] = lse_v;
-  if (entropy != nullptr) entropy[blockIdx.x] = (L - d) * kLn2;  // lse - sum p z, the common max cancelled
-  if (logprob != nullptr) {
-    const int64_t lab = (int64_t)labels[blockIdx.x];
-    logprob[blockIdx.x] = (lab >= 0 && lab < vocab) ? Row<T>::one(row + lab) - lse_v : 0.f;
+  if (parts > 1) {
+    float* o = ws + (int64_t)blockIdx.x * 3;
+    o[0] = st.M; o[1] = st.s; o[2] = st.e;
+    return;
   }
+  write_stats(st, t, row, vocab, labels, logprob, entropy, lse);
+}
+
+// One wavefront per row folds the row's parts (at most kMaxParts), in a fixed tree.
+constexpr int kMaxParts = 64;
+template <typename T, typename LabelT>
+__global__ __launch_bounds__(kWave) void logits_merge_kernel(
+    const float* __restrict__ ws, int parts, const T* __restrict__ logits, int64_t ld, int vocab,
+    const LabelT* __restrict__ labels, float* __restrict__ logprob, float* __restrict__ entropy,
+    float* __restrict__ lse) {
+  const int t = blockIdx.x, lane = threadIdx.x;
+  Stats st{kFloor, 0.f, 0.f};
+  if (lane < parts) {
+    const float* o = ws + ((int64_t)t * parts + lane) * 3;
+    st = Stats{o[0], o[1], o[2]};
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    Stats o;
+    o.M = __shfl_down(st.M, off, kWave);
+    o.s = __shfl_down(st.s, off, kWave);
+    o.e = __shfl_down(st.e, off, kWave);
+    st = merge(st, o);
+  }
+  if (lane == 0) write_stats(st, t, logits + (int64_t)t * ld, vocab, labels, logprob, entropy, lse);
 }
 
 // dlogits[j] = g_lp (onehot_j - p_j) - g_ent p_j (log p_j + H),  p_j = exp(z_j - lse).
 // dlogits may be the logits' own storage: every element is read before it is written by the same thread.
+// Rows, and the vectors of a row, are walked from the last to the first: the end of what the forward read last is
+// still in the 256 MB cache in front of the memory.  Bound by memory (read + write 5.1 TB/s, a device copy 5.3): 2047 x 151936
+// bf16 244 us for 250; where a short batch is split into parts 32 x 151936 takes 9.3 us for 53, 187 x 151936 24 for 78;
+// rows of an odd vocabulary, read from their first 16-byte boundary on, 2047 x 50257 bf16 93 us for 166.
 template <typename T, typename LabelT>
 __global__ __launch_bounds__(kBlock) void logits_grad_kernel(
     const T* logits, int64_t ld, int vocab, const LabelT* __restrict__ labels,
     const float* __restrict__ lse, const float* __restrict__ entropy, const float* __restrict__ g_logprob,
-    const float* __restrict__ g_entropy, T* dlogits, int64_t ld_d, int vec_ok) {
-  const T* row = logits + (int64_t)blockIdx.x * ld;
-  T* out = dlogits + (int64_t)blockIdx.x * ld_d;
+    const float* __restrict__ g_entropy, T* dlogits, int64_t ld_d, int vec_ok, int parts) {
+  const int b = gridDim.x - 1 - blockIdx.x;
+  const int t = b / parts, part = b - t * parts;
+  const T* row = logits + (int64_t)t * ld;
+  T* out = dlogits + (int64_t)t * ld_d;
   constexpr int kPer = Row<T>::kPer;
-  const float lse_v = lse[blockIdx.x];
-  const float g_lp = g_logprob ? g_logprob[blockIdx.x] : 0.f;
-  const float g_en = g_entropy ? g_entropy[blockIdx.x] : 0.f;
-  const float H = g_entropy ? entropy[blockIdx.x] : 0.f;
-  const int64_t lab = g_logprob ? (int64_t)labels[blockIdx.x] : -1;
-  auto grad = [&](int64_t j, float z) {
+  const float lse_v = lse[t];
+  const float g_lp = g_logprob ? g_logprob[t] : 0.f;
+  const float g_en = g_entropy ? g_entropy[t] : 0.f;
+  const float H = g_entropy ? entropy[t] : 0.f;
+  const int64_t lab64 = g_logprob ? (int64_t)labels[t] : -1;
+  const int lab = (lab64 >= 0 && lab64 < vocab) ? (int)lab64 : -1;
+  auto grad = [&](float z) {
     const float lp = z - lse_v;
     const float p = __expf(lp);
-    float g = -g_lp * p;
-    if (g_en != 0.f) g -= (p > 0.f) ? g_en * p * (lp + H) : 0.f;
-    if (j == lab) g += g_lp;
-    return g;
+    // a probability of 0 takes nothing from the entropy, also where its log is -inf
+    return p * ((p > 0.f) ? fmaf(-g_en, lp + H, -g_lp) : -g_lp);
   };
-  const int n_vec = vec_ok ? vocab / kPer : 0;
-  for (int q = threadIdx.x; q < n_vec; q += kBlock) {
-    float v[8], o[8];
-    Row<T>::load(row + (int64_t)q * kPer, v);
+  // vec_ok: the row of dlogits sits on the same offset from a 16-byte boundary as the row of logits
+  const RowSpan sp(row, vocab, vec_ok != 0, part, parts);
+  const T* body = row + sp.head;
+  T* body_out = out + sp.head;
+  const int lab_b = lab < sp.head ? -1 : lab - sp.head;
+  auto finish = [&](int q, float (&v)[8]) {
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) o[j] = grad((int64_t)q * kPer + j, v[j]);
-    Row<T>::store(out + (int64_t)q * kPer, o);
+    for (int j = 0; j < kPer; ++j) v[j] = grad(v[j]);
+    const int in_vec = lab_b - q * kPer;
+    if ((unsigned)in_vec < (unsigned)kPer) {
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) v[j] += (j == in_vec) ? g_lp : 0.f;
+    }
+    Row<T>::store(body_out + (uint32_t)q * kPer, v);
+  };
+  int q = sp.q_hi - 1 - (int)threadIdx.x;
+  for (; q - kBlock >= sp.q_lo; q -= 2 * kBlock) {  // two loads in flight per thread
+    float v0[8], v1[8];
+    Row<T>::load(body + (uint32_t)q * kPer, v0);
+    Row<T>::load(body + (uint32_t)(q - kBlock) * kPer, v1);
+    finish(q, v0);
+    finish(q - kBlock, v1);
   }
-  for (int i = n_vec * kPer + threadIdx.x; i < vocab; i += kBlock)
-    Row<T>::store_one(out + i, grad(i, Row<T>::one(row + i)));
+  for (; q >= sp.q_lo; q -= kBlock) {
+    float v[8];
+    Row<T>::load(body + (uint32_t)q * kPer, v);
+    finish(q, v);
+  }
+  for (int i = part * kBlock + threadIdx.x; i < sp.n_scalar; i += parts * kBlock) {
+    const int j = sp.scalar<T>(i);
+    Row<T>::store_one(out + j, grad(Row<T>::one(row + j)) + (j == lab ? g_lp : 0.f));
+  }
 }
 
 }  // namespace axon
@@ -183,8 +272,21 @@ using namespace axon;
 
 namespace {
 
-bool rows_on_16_bytes(const void* p, int64_t ld, int elem_bytes) {
-  return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && (ld * elem_bytes) % 16 == 0;
+// Workgroups per row.  The part holds 2048 of these workgroups at once; from three quarters of that on a row is left
+// to one (2047 x 151936 bf16, forward + backward: 343 us with one, 343 with two, 353 with four).  Fewer rows are split
+// into about 8192 pieces, of at least eight vectors per thread each (1500 x 128264 bf16: 228 us for 242 with 4096
+// pieces and with one per row, 700 x 151936: 126 for 130 and 148, 300 x 151936 fp32: 104 for 110 and 187).
+int row_parts(int64_t n, int64_t vocab, int elem_bytes) {
+  if (n >= 1536) return 1;
+  const int64_t fill = 8192 / (n > 0 ? n : 1), work = vocab * elem_bytes / (8 * 16 * kBlock);
+  const int64_t p = fill < work ? fill : work;
+  return (int)(p < 1 ? 1 : (p < kMaxParts ? p : kMaxParts));
+}
+
+// every row of b sits on the same offset from a 16-byte boundary as the row of a
+bool same_offsets(const void* a, int64_t ld_a, const void* b, int64_t ld_b, int64_t n, int elem_bytes) {
+  const uintptr_t d = reinterpret_cast<uintptr_t>(a) ^ reinterpret_cast<uintptr_t>(b);
+  return (d & 15) == 0 && (n <= 1 || ((ld_a - ld_b) * elem_bytes) % 16 == 0);
 }
 
 int check_logits(const void* logits, int dtype, int64_t ld, int64_t n, int64_t v) {
@@ -197,20 +299,32 @@ int check_logits(const void* logits, int dtype, int64_t ld, int64_t n, int64_t v
 
 }  // namespace
 
-extern "C" int axon_logits_fwd(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
-                               const void* labels, int labels_i64, float* logprob, float* entropy,
-                               float* lse, void* stream) {
+extern "C" int64_t axon_logits_fwd_workspace_bytes(int dtype, int64_t n, int64_t vocab) {
+  if (n < 0 || vocab <= 0 || (dtype != AXON_LOGITS_F32 && dtype != AXON_LOGITS_BF16)) return AXON_ERR_ARG;
+  const int parts = row_parts(n, vocab, dtype == AXON_LOGITS_F32 ? 4 : 2);
+  return parts > 1 ? n * parts * 3 * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
+                                  const void* labels, int labels_i64, float* logprob, float* entropy,
+                                  float* lse, float* workspace, void* stream) {
   int rc = check_logits(logits, dtype, ld, n, vocab);
   if (rc != AXON_OK) return rc;
   if (n == 0) return AXON_OK;
   if (!lse || (logprob && !labels)) return AXON_ERR_ARG;
   const hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)n), blk(kBlock);
   const int eb = dtype == AXON_LOGITS_F32 ? 4 : 2;
-  const int vec_ok = rows_on_16_bytes(logits, ld, eb);
-#define AXON_STATS(T, L)                                                                           \
-  hipLaunchKernelGGL((logits_stats_kernel<T, L>), grid, blk, 0, st, static_cast<const T*>(logits), ld, \
-                     (int)vocab, static_cast<const L*>(labels), logprob, entropy, lse, vec_ok)
+  const int parts = workspace ? row_parts(n, vocab, eb) : 1;
+  const dim3 grid((unsigned)(n * parts)), blk(kBlock);
+#define AXON_STATS(T, L)                                                                               \
+  do {                                                                                                 \
+    hipLaunchKernelGGL((logits_stats_kernel<T, L>), grid, blk, 0, st, static_cast<const T*>(logits), ld, \
+                       (int)vocab, static_cast<const L*>(labels), logprob, entropy, lse, parts, workspace); \
+    if (parts > 1)                                                                                     \
+      hipLaunchKernelGGL((logits_merge_kernel<T, L>), dim3((unsigned)n), dim3(kWave), 0, st, workspace, parts, \
+                         static_cast<const T*>(logits), ld, (int)vocab, static_cast<const L*>(labels), \
+                         logprob, entropy, lse);                                                       \
+  } while (0)
   if (dtype == AXON_LOGITS_F32) {
     if (labels_i64) AXON_STATS(float, int64_t); else AXON_STATS(float, int32_t);
   } else {
@@ -219,6 +333,12 @@ extern "C" int axon_logits_fwd(const void* logits, int dtype, int64_t ld, int64_
 #undef AXON_STATS
   AXON_CHECK_LAUNCH();
   return AXON_OK;
+}
+
+extern "C" int axon_logits_fwd(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
+                               const void* labels, int labels_i64, float* logprob, float* entropy,
+                               float* lse, void* stream) {
+  return axon_logits_fwd_ws(logits, dtype, ld, n, vocab, labels, labels_i64, logprob, entropy, lse, nullptr, stream);
 }
 
 extern "C" int axon_logits_bwd(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
@@ -231,13 +351,13 @@ extern "C" int axon_logits_bwd(const void* logits, int dtype, int64_t ld, int64_
   if (!lse || !dlogits || ld_d < vocab) return AXON_ERR_ARG;
   if ((g_logprob && !labels) || (g_entropy && !entropy)) return AXON_ERR_ARG;
   const hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)n), blk(kBlock);
   const int eb = dtype == AXON_LOGITS_F32 ? 4 : 2;
-  const int vec_ok = rows_on_16_bytes(logits, ld, eb) && rows_on_16_bytes(dlogits, ld_d, eb);
+  const int vec_ok = same_offsets(logits, ld, dlogits, ld_d, n, eb), parts = row_parts(n, vocab, eb);
+  const dim3 grid((unsigned)(n * parts)), blk(kBlock);
 #define AXON_GRAD(T, L)                                                                            \
   hipLaunchKernelGGL((logits_grad_kernel<T, L>), grid, blk, 0, st, static_cast<const T*>(logits), ld,  \
                      (int)vocab, static_cast<const L*>(labels), lse, entropy, g_logprob, g_entropy,    \
-                     static_cast<T*>(dlogits), ld_d, vec_ok)
+                     static_cast<T*>(dlogits), ld_d, vec_ok, parts)
   if (dtype == AXON_LOGITS_F32) {
     if (labels_i64) AXON_GRAD(float, int64_t); else AXON_GRAD(float, int32_t);
   } else {

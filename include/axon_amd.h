@@ -542,6 +542,13 @@ enum { AXON_LOGITS_F32 = 0, AXON_LOGITS_BF16 = 1 };
 int axon_logits_fwd(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
                     const void* labels, int labels_are_i64, float* logprob, float* entropy, float* lse,
                     void* stream);
+/* The same with `workspace` of axon_logits_fwd_workspace_bytes(dtype, n, vocab) bytes (4-byte aligned; its contents
+ * do not matter): a short batch, whose rows alone do not fill the part, is split into several workgroups per row.
+ * 0 bytes, or workspace NULL: one workgroup per row, as above. */
+int64_t axon_logits_fwd_workspace_bytes(int dtype, int64_t n, int64_t vocab);
+int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
+                       const void* labels, int labels_are_i64, float* logprob, float* entropy, float* lse,
+                       float* workspace, void* stream);
 
 /* Backward of the above in one read and one write of the rows:
  *   dlogits[t][j] = g_logprob[t] (onehot - p) - g_entropy[t] p (log p + entropy[t]),  p = exp(logits - lse)
