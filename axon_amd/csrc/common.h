@@ -56,12 +56,6 @@ __device__ __forceinline__ bool select_hit(const SelectState& s, uint32_t key, i
   return key > s.threshold || (key == s.threshold && i < s.index_limit);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, kWave);
-  return v;
-}
-
 // Sum over the wavefront by DPP row shifts and broadcasts (no LDS traffic); the total lands in lane 63.
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ float dpp_add(float v) {
@@ -78,6 +72,49 @@ __device__ __forceinline__ float wave_sum_to_last(float v) {
   v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
   return v;
 }
+
+// The same with the total in every lane.  All 64 lanes have to be active.  Each step is one vector instruction; a
+// shuffle is a trip through the LDS crossbar with a wait behind it, and the six of a sum one after the other are
+// 0.3 us: for the 8 to 70 values that a kernel ends with, most of a launch over a micro-batch.
+__device__ __forceinline__ float wave_sum(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wave_sum_to_last(v)), kWave - 1));
+}
+
+// The same order for doubles, and for the extrema (a lane without a source keeps its own value).
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ double dpp_add_d(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROW_MASK, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROW_MASK, 0xf, false);
+  return v + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double wave_sum_d(double v) {
+  v = dpp_add_d<0x111, 0xf>(v);
+  v = dpp_add_d<0x112, 0xf>(v);
+  v = dpp_add_d<0x114, 0xf>(v);
+  v = dpp_add_d<0x118, 0xf>(v);
+  v = dpp_add_d<0x142, 0xa>(v);
+  v = dpp_add_d<0x143, 0xc>(v);
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, kWave - 1);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), kWave - 1);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_or_own(float v) {
+  const int i = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, ROW_MASK, 0xf, false));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, dpp_or_own<0x111, 0xf>(v));
+  v = fmaxf(v, dpp_or_own<0x112, 0xf>(v));
+  v = fmaxf(v, dpp_or_own<0x114, 0xf>(v));
+  v = fmaxf(v, dpp_or_own<0x118, 0xf>(v));
+  v = fmaxf(v, dpp_or_own<0x142, 0xa>(v));
+  v = fmaxf(v, dpp_or_own<0x143, 0xc>(v));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), kWave - 1));
+}
+__device__ __forceinline__ float wave_min(float v) { return -wave_max(-v); }
 
 // Sum NV values over the workgroup; the total lands in thread 0.
 template <int NV>

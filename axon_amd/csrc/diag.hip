@@ -35,7 +35,7 @@ __global__ __launch_bounds__(kBlock) void sampler_diag_tokens_kernel(
     const float* __restrict__ oldp, const float* __restrict__ samp, const void* __restrict__ mask,
     const int32_t* __restrict__ cu, int64_t n_rows, int64_t n_slots, int64_t uniform_len,
     float is_lo, float is_hi, float rs_lo, float rs_hi, float rs_lr_lo, float rs_lr_hi,
-    float* row_vals, float* __restrict__ partials) {
+    int iters, float* row_vals, float* __restrict__ partials) {
   __shared__ int32_t lds_cu[kLdsRows];
   __shared__ float lds_red[kDiagSums * (kBlock / kWave)];
   __shared__ float lds_mm[kDiagMinMax * (kBlock / kWave)];
@@ -45,16 +45,16 @@ __global__ __launch_bounds__(kBlock) void sampler_diag_tokens_kernel(
   for (int k = 0; k < kDiagSums; ++k) a[k] = 0.f;
   float mx[3] = {-kInf, -kInf, -kInf}, mn[3] = {kInf, kInf, kInf};
 
-  const int64_t n_chunks = (n_slots + kChunk - 1) / kChunk;
+  const int64_t chunk_len = (int64_t)iters * kBlock * kVec, n_chunks = (n_slots + chunk_len - 1) / chunk_len;
 #pragma unroll 1
   for (int64_t chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
-    const int64_t c0 = chunk * kChunk;
-    const int64_t c1 = min(c0 + (int64_t)kChunk, n_slots);
+    const int64_t c0 = chunk * chunk_len;
+    const int64_t c1 = min(c0 + chunk_len, n_slots);
     __syncthreads();  // the previous chunk's row window is no longer read
     RowFinder rf;
     rf.init(cu, n_rows, uniform_len, c0, c1, lds_cu);
 #pragma unroll 1
-    for (int it = 0; it < kIter; ++it) {
+    for (int it = 0; it < iters; ++it) {
       const int64_t i = c0 + ((int64_t)it * kBlock + threadIdx.x) * kVec;
       DiagSeg s;
       s.row = -1;
@@ -141,11 +141,8 @@ __global__ __launch_bounds__(kBlock) void sampler_diag_tokens_kernel(
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      mx[k] = fmaxf(mx[k], __shfl_down(mx[k], off, kWave));
-      mn[k] = fminf(mn[k], __shfl_down(mn[k], off, kWave));
-    }
+    mx[k] = wave_max(mx[k]);
+    mn[k] = wave_min(mn[k]);
     if (lane == 0) {
       lds_mm[wave * kDiagMinMax + 2 * k] = mx[k];
       lds_mm[wave * kDiagMinMax + 2 * k + 1] = mn[k];
@@ -180,17 +177,13 @@ struct DiagCfg {
   float log_is_lo, log_is_hi, log_rs_lo, log_rs_hi;  // fp32 log of the same
 };
 
-__device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, kWave);
-  return v;
-}
-
 // Four wavefronts per workgroup: what a wavefront spends here is mostly the 50 + 20 reductions at the end,
 // which cost the same for one row per lane as for four, and sixteen wavefronts would queue four deep on a SIMD.
+// Those reductions by DPP moves instead of LDS shuffles: 65536 tokens in 90 rows 9.6 us for 17.3, 8.4 M in 9000 15.3 for 21.9.
 constexpr int kDiagRowThreads = 256;
 // Workgroup b of the grid takes token partials b, b + gridDim.x, ... and rows likewise, and leaves its
-// 70 sums / maxima / minima in out[b][kDiagOut]; sampler_diag_final_kernel folds the workgroups.
+// 70 sums / maxima / minima in out[b][kDiagOut]; sampler_diag_final_kernel folds the workgroups where there are
+// several (a single one writes the operator's output).
 __global__ __launch_bounds__(kDiagRowThreads) void sampler_diag_rows_kernel(
     const float* __restrict__ partials, int n_blocks, const float* __restrict__ row_vals,
     int64_t n_rows, DiagCfg cfg, double* __restrict__ out_all) {
@@ -295,12 +288,7 @@ __global__ __launch_bounds__(kDiagRowThreads) void sampler_diag_rows_kernel(
   }
 #pragma unroll
   for (int k = 0; k < kOutMM; ++k) {
-    float hi = mx[k], lo = mn[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      hi = fmaxf(hi, __shfl_down(hi, off, kWave));
-      lo = fminf(lo, __shfl_down(lo, off, kWave));
-    }
+    const float hi = wave_max(mx[k]), lo = wave_min(mn[k]);
     if (lane == 0) { red_mx[wave][k] = hi; red_mn[wave][k] = lo; }
   }
   __syncthreads();
@@ -351,9 +339,19 @@ static inline int diag_row_blocks(int64_t n_rows, int64_t token_blocks) {
   return (int)(b < 1 ? 1 : (b > 128 ? 128 : b));
 }
 
+// Steps of 1024 slots per workgroup of the token pass: one where longer chunks would leave compute units idle
+// (65536 slots in chunks of 4096 run on 16 of 256: 17.6 us, in chunks of 1024 8.6).
+static inline int diag_iters(int64_t n_slots) {
+  const int64_t steps = (n_slots + kBlock * kVec - 1) / (kBlock * kVec);
+  return steps <= 256 ? 1 : (steps <= 512 ? 2 : kIter);
+}
+static inline unsigned diag_grid(int64_t n_slots) {
+  return stream_grid(n_slots, (int64_t)diag_iters(n_slots) * kBlock * kVec);
+}
+
 extern "C" int64_t axon_sampler_diag_workspace_bytes(int64_t n_rows, int64_t n_slots) {
   if (n_rows < 0 || n_slots < 0) return AXON_ERR_ARG;
-  const int64_t blocks = n_slots > 0 ? (int64_t)stream_grid(n_slots) : 1;
+  const int64_t blocks = n_slots > 0 ? (int64_t)diag_grid(n_slots) : 1;
   // [6][n_rows] row sums (zero-filled by the caller), the per-workgroup token partials, then the
   // row pass's per-workgroup results (doubles, 8-byte aligned)
   const int64_t floats = kDiagRowVals * n_rows + blocks * kDiagStride;
@@ -377,16 +375,17 @@ extern "C" int axon_sampler_diag(const float* oldp, const float* samp, const voi
   if (mask_kind != AXON_MASK_F32 && mask_kind != AXON_MASK_I64) return AXON_ERR_ARG;
   float* row_vals = workspace;
   float* partials = workspace + kDiagRowVals * n_rows;
-  const dim3 g(stream_grid(n_slots)), blk(kBlock);
+  const dim3 g(diag_grid(n_slots)), blk(kBlock);
+  const int iters = diag_iters(n_slots);
   const hipStream_t st = (hipStream_t)stream;
   if (mask_kind == AXON_MASK_F32)
     hipLaunchKernelGGL(sampler_diag_tokens_kernel<AXON_MASK_F32>, g, blk, 0, st, oldp, samp, mask, cu,
                        n_rows, n_slots, uniform_len, is_lo, is_hi, rs_lo, rs_hi, rs_lr_lo, rs_lr_hi,
-                       row_vals, partials);
+                       iters, row_vals, partials);
   else
     hipLaunchKernelGGL(sampler_diag_tokens_kernel<AXON_MASK_I64>, g, blk, 0, st, oldp, samp, mask, cu,
                        n_rows, n_slots, uniform_len, is_lo, is_hi, rs_lo, rs_hi, rs_lr_lo, rs_lr_hi,
-                       row_vals, partials);
+                       iters, row_vals, partials);
   AXON_CHECK_LAUNCH();
   DiagCfg cfg;
   cfg.is_mode = is_mode; cfg.rs_mode = rs_mode;
@@ -397,8 +396,9 @@ extern "C" int axon_sampler_diag(const float* oldp, const float* samp, const voi
   double* parts = reinterpret_cast<double*>(workspace + (floats + 1) / 2 * 2);
   const int rb = diag_row_blocks(n_rows, g.x);
   hipLaunchKernelGGL(sampler_diag_rows_kernel, dim3(rb), dim3(kDiagRowThreads), 0, st, partials, (int)g.x, row_vals,
-                     n_rows, cfg, parts);
+                     n_rows, cfg, rb == 1 ? out : parts);
   AXON_CHECK_LAUNCH();
+  if (rb == 1) return AXON_OK;  // one workgroup's results are the totals
   hipLaunchKernelGGL(sampler_diag_final_kernel, dim3(1), dim3(1024), 0, st, parts, rb, out);
   AXON_CHECK_LAUNCH();
   return AXON_OK;

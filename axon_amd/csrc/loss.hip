@@ -627,8 +627,7 @@ __global__ __launch_bounds__(1024) void gmpo_rows_kernel(const float* __restrict
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int k = 0; k < 3; ++k) {
-    double v = t[k];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, kWave);
+    const double v = wave_sum_d(t[k]);
     if (lane == 0) red[wave][k] = v;
   }
   __syncthreads();

@@ -270,8 +270,7 @@ __global__ __launch_bounds__(1024) void group_scores_kernel(
       load4(a, p, v);
       acc += ((double)v[0] + (double)v[1]) + ((double)v[2] + (double)v[3]);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, kWave);
+    acc = wave_sum_d(acc);
     if (lane == 0) __hip_atomic_store(scores + r, (float)acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   // the scores' write-through stores are acknowledged before the workgroup draws its ticket (publish_row_take_ticket)
