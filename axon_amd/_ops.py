@@ -251,7 +251,7 @@ def masked_whiten(x, mask, *, remask=False, inplace=False, stats_only=False):
         out = None
     else:
         out = xf if (inplace and xf.data_ptr() == x.data_ptr()) else torch.empty_like(xf)
-    stats = _zeros(4, dev)
+    stats = torch.empty(4, device=dev, dtype=torch.float32)
     ws = torch.empty(max(lib.axon_masked_whiten_workspace_bytes(n) // 4, 8), device=dev, dtype=torch.float32)
     check(
         lib.axon_masked_whiten(ptr(xf), ptr(mk), kind, n, int(remask), ptr(out), ptr(stats), ptr(ws), stream_ptr()),

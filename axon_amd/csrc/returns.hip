@@ -188,16 +188,61 @@ __global__ __launch_bounds__(kBlock) void reverse_scan_kernel(
 // ---- masked whitening -------------------------------------------------------------------------
 // stats[0] mean, [1] n, [2] variance (times n/(n-1) when n > 1), [3] rsqrt(variance + 1e-8)
 
-// PASS 0: sum m x, sum m.   PASS 1: sum m (x - mean)^2.
+// Every workgroup that needs a pass's result adds the pass's at most kMomentBlocks partials itself, in the same fixed
+// order (32 KB out of L2), where a launch of one workgroup in between cost 3.6 us and the gaps around it.
+constexpr int kMomentBlocks = 1024;
+
+__device__ __forceinline__ void add_partials(const float* __restrict__ partials, int n_blocks, float (&a)[2], float* lds_red) {
+  float2 v[kMomentBlocks / kBlock];
+#pragma unroll
+  for (int u = 0; u < kMomentBlocks / kBlock; ++u) {
+    const int b = threadIdx.x + u * kBlock;
+    v[u] = *reinterpret_cast<const float2*>(partials + (size_t)(b < n_blocks ? b : 0) * kPartialStride);
+  }
+  a[0] = a[1] = 0.f;
+#pragma unroll
+  for (int u = 0; u < kMomentBlocks / kBlock; ++u) {
+    const bool ok = (int)threadIdx.x + u * kBlock < n_blocks;
+    a[0] += ok ? v[u].x : 0.f;
+    a[1] += ok ? v[u].y : 0.f;
+  }
+  block_sum<2>(a, lds_red);
+}
+
+// The statistics in thread 0, from the partials of pass 0 (mean, n) and of pass 1 (variance, 1 / deviation).
+__device__ __forceinline__ void finish_mean(const float (&a)[2], float* st) {
+  st[0] = a[0] / fmaxf(a[1], 1.f);
+  st[1] = a[1];
+}
+__device__ __forceinline__ void finish_var(const float (&a)[2], float n, float* st) {
+  float var = a[0] / fmaxf(n, 1.f);
+  if (n > 1.f) var = var * n / (n - 1.f);
+  st[2] = var;
+  st[3] = rsqrtf(var + 1e-8f);
+}
+
+// PASS 0: sum m x, sum m.   PASS 1: sum m (x - mean)^2, with the mean from pass 0's partials; its workgroup 0 leaves
+// mean and n in stats.
 template <int MK, int PASS>
 __global__ __launch_bounds__(kBlock) void masked_moments_kernel(const float* __restrict__ x,
                                                                 const void* __restrict__ mask,
                                                                 int64_t n_slots,
-                                                                const float* __restrict__ stats,
-                                                                float* partials) {
+                                                                const float* __restrict__ partials0,
+                                                                float* __restrict__ stats,
+                                                                float* __restrict__ partials) {
   __shared__ float lds_red[2 * (kBlock / kWave)];
-  const float mean = PASS == 1 ? stats[0] : 0.f;
-  float a[2] = {0.f, 0.f};
+  __shared__ float st[2];
+  float a[2] = {0.f, 0.f}, mean = 0.f;
+  if (PASS == 1) {
+    add_partials(partials0, (int)gridDim.x, a, lds_red);
+    if (threadIdx.x == 0) {
+      finish_mean(a, st);
+      if (blockIdx.x == 0) { stats[0] = st[0]; stats[1] = st[1]; }
+    }
+    __syncthreads();
+    mean = st[0];
+    a[0] = a[1] = 0.f;
+  }
   const int64_t n_vec = n_slots / kVec;
   for (int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x; q < n_vec;
        q += (int64_t)gridDim.x * kBlock) {
@@ -229,38 +274,31 @@ __global__ __launch_bounds__(kBlock) void masked_moments_kernel(const float* __r
   store_block_partials<2>(a, lds_red, partials);
 }
 
-// one workgroup adds the partials in a fixed order and finishes the statistics
-__global__ __launch_bounds__(kBlock) void masked_moments_finish_kernel(const float* __restrict__ partials,
-                                                                       int n_blocks, int pass,
-                                                                       float* __restrict__ stats) {
+// the variance where nobody else forms it (statistics only)
+__global__ __launch_bounds__(kBlock) void masked_var_finish_kernel(const float* __restrict__ partials,
+                                                                   int n_blocks, float* __restrict__ stats) {
   __shared__ float lds_red[2 * (kBlock / kWave)];
-  float a[2] = {0.f, 0.f};
-  for (int b = threadIdx.x; b < n_blocks; b += kBlock) {
-    a[0] += partials[(size_t)b * kPartialStride];
-    a[1] += partials[(size_t)b * kPartialStride + 1];
-  }
-  block_sum<2>(a, lds_red);
-  if (threadIdx.x == 0) {
-    if (pass == 0) {
-      stats[0] = a[0] / fmaxf(a[1], 1.f);
-      stats[1] = a[1];
-    } else {
-      const float n = stats[1];
-      float var = a[0] / fmaxf(n, 1.f);
-      if (n > 1.f) var = var * n / (n - 1.f);
-      stats[2] = var;
-      stats[3] = rsqrtf(var + 1e-8f);
-    }
-  }
+  float a[2];
+  add_partials(partials, n_blocks, a, lds_red);
+  if (threadIdx.x == 0) finish_var(a, stats[1], stats);
 }
 
 template <int MK>
 __global__ __launch_bounds__(kBlock) void whiten_kernel(const float* __restrict__ x,
                                                         const void* __restrict__ mask,
                                                         int64_t n_slots,
-                                                        const float* __restrict__ stats, int remask,
-                                                        float* __restrict__ out) {
-  const float mean = stats[0], rstd = stats[3];
+                                                        const float* __restrict__ partials, float* stats,
+                                                        int remask, float* __restrict__ out) {
+  __shared__ float lds_red[2 * (kBlock / kWave)];
+  __shared__ float st[4];
+  float a[2];
+  add_partials(partials, (int)gridDim.x, a, lds_red);
+  if (threadIdx.x == 0) {
+    finish_var(a, stats[1], st);
+    if (blockIdx.x == 0) { stats[2] = st[2]; stats[3] = st[3]; }
+  }
+  __syncthreads();
+  const float mean = stats[0], rstd = st[3];
   const int64_t n_vec = n_slots / kVec;
   for (int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x; q < n_vec;
        q += (int64_t)gridDim.x * kBlock) {
@@ -388,7 +426,7 @@ int launch_scan(int mode, const float* rewards, const float* values, const void*
 
 unsigned moments_grid(int64_t n_slots) {
   const int64_t blocks = (n_slots / kVec + kBlock - 1) / kBlock;
-  const int64_t cap = 2048;  // eight workgroups per compute unit walk the tokens
+  const int64_t cap = kMomentBlocks;  // four workgroups per compute unit walk the tokens
   return (unsigned)(blocks < 1 ? 1 : (blocks < cap ? blocks : cap));
 }
 
@@ -396,15 +434,14 @@ template <int MK>
 int launch_whiten(const float* x, const void* mask, int64_t n_slots, int remask, float* out,
                   float* stats, float* partials, hipStream_t st) {
   const dim3 grid(moments_grid(n_slots)), blk(kBlock);
-  hipLaunchKernelGGL((masked_moments_kernel<MK, 0>), grid, blk, 0, st, x, mask, n_slots, stats, partials);
-  hipLaunchKernelGGL(masked_moments_finish_kernel, dim3(1), blk, 0, st, partials, (int)grid.x, 0, stats);
-  hipLaunchKernelGGL((masked_moments_kernel<MK, 1>), grid, blk, 0, st, x, mask, n_slots, stats, partials);
-  hipLaunchKernelGGL(masked_moments_finish_kernel, dim3(1), blk, 0, st, partials, (int)grid.x, 1, stats);
+  float* partials1 = partials + (size_t)grid.x * kPartialStride;
+  hipLaunchKernelGGL((masked_moments_kernel<MK, 0>), grid, blk, 0, st, x, mask, n_slots, nullptr, stats, partials);
+  hipLaunchKernelGGL((masked_moments_kernel<MK, 1>), grid, blk, 0, st, x, mask, n_slots, partials, stats, partials1);
+  if (out != nullptr)
+    hipLaunchKernelGGL((whiten_kernel<MK>), grid, blk, 0, st, x, mask, n_slots, partials1, stats, remask, out);
+  else
+    hipLaunchKernelGGL(masked_var_finish_kernel, dim3(1), blk, 0, st, partials1, (int)grid.x, stats);
   AXON_CHECK_LAUNCH();
-  if (out != nullptr) {
-    hipLaunchKernelGGL((whiten_kernel<MK>), grid, blk, 0, st, x, mask, n_slots, stats, remask, out);
-    AXON_CHECK_LAUNCH();
-  }
   return AXON_OK;
 }
 
@@ -439,7 +476,7 @@ extern "C" int axon_reverse_scan(int mode, const float* rewards, const float* va
 
 extern "C" int64_t axon_masked_whiten_workspace_bytes(int64_t n_slots) {
   if (n_slots < 0) return AXON_ERR_ARG;
-  return (int64_t)moments_grid(n_slots) * kPartialStride * (int64_t)sizeof(float);
+  return 2 * (int64_t)moments_grid(n_slots) * kPartialStride * (int64_t)sizeof(float);  // one set per pass
 }
 
 extern "C" int axon_masked_whiten(const float* x, const void* mask, int mask_kind, int64_t n_slots,

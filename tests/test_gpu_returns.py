@@ -193,6 +193,90 @@ def test_masked_whiten_gpu():
     assert out.shape == (5, 7) and abs(out.mean().item()) < 1e-5
 
 
+@pytest.mark.parametrize("n", [1, 1021, 1024 * 1024, 1024 * 1024 + 1027, 3 * 1024 * 1024 + 1])
+def test_masked_whiten_statistics_at_the_edges_of_the_grid(n):
+    """One workgroup, as many as the launch has, and several trips of each, against float64; the statistics alone and
+    beside the output come out the same.  Sums of n positive terms in trees of at most 64 in a row: n-independent
+    relative error below 1e-5."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn(n, generator=g, device=DEV) + 2
+    m = (torch.rand(n, generator=g, device=DEV) > 0.3).float()
+    m[0] = 1.0
+    out, stats = _ops.masked_whiten(x, m)
+    _, alone = _ops.masked_whiten(x, m, stats_only=True)
+    assert torch.equal(stats, alone)
+    xd, md = x.double(), m.double()
+    mean = (xd * md).sum() / md.sum()
+    var = ((xd - mean) ** 2 * md).sum() / md.sum()
+    var = var * md.sum() / (md.sum() - 1) if md.sum() > 1 else var
+    ref = torch.stack([mean, md.sum(), var, (var + 1e-8).rsqrt()])
+    assert torch.allclose(stats.double(), ref, rtol=1e-5, atol=1e-7 if n == 1 else 0)
+    if n > 1:
+        assert rel_l2(out, (xd - mean) * ref[3]) < 1e-5
+
+
+@pytest.mark.parametrize("n_rows,mode", [(8192, 1), (8193, 2), (17001, 1), (8200, 3)])
+def test_group_advantage_with_more_rows_than_one_trip(n_rows, mode):
+    """The workgroup that ends last takes eight rows per thread and trip."""
+    g = torch.Generator(device=DEV).manual_seed(n_rows)
+    r = torch.randint(0, 3, (n_rows, 4), generator=g, device=DEV).float()
+    gidx = torch.arange(n_rows, device=DEV) // 16
+    n_groups = int(gidx[-1]) + 1
+    rows = _ops.rows_of(r)
+    adv = _ops.group_advantage(r, torch.ones_like(r), gidx, n_groups, rows, eps=1e-6, mode=mode)
+    _, scores, _ = _ops.row_stats(r, None, None, rows, want_cnt=False)
+    _, _, _, scalar = _ops.group_stats(scores, gidx, n_groups, 1e-6, mode)
+    # the other kernel adds the small whole-number scores of a group exactly too: the same quotients, one rounding apart
+    assert torch.allclose(adv[:, 0], scalar, rtol=1e-5, atol=2e-6) and torch.equal(adv[:, 0], adv[:, 3])
+
+
+@pytest.mark.parametrize("mask_dtype", [torch.float32, torch.int64])
+@pytest.mark.parametrize("mode", [_ops.SCAN_GAE, _ops.SCAN_GAE_RESPONSE_ONLY, _ops.SCAN_DISCOUNTED, _ops.SCAN_SUFFIX_SUM])
+def test_scan_by_workgroup_equals_scan_by_wavefront(mode, mask_dtype):
+    """Rows around the edges of a wavefront's 256 and a workgroup's 1024 tokens, on every offset from a 16-byte boundary.
+    Short rows behind them bring the mean length under a window, so the second launch gives each row one wavefront:
+    the same arithmetic in the same order, hence the same bits.  The first launch against a loop in float64."""
+    lens = [1, 255, 256, 257, 3, 1023, 1024, 1025, 2050, 4097, 0, 767, 770]
+    n = sum(lens)
+    g = torch.Generator().manual_seed(n + mode)
+    total = n + 4000
+    r, v = torch.randn(total, generator=g), torch.randn(total, generator=g)
+    m = (torch.rand(total, generator=g) < 0.8).to(mask_dtype)
+    cu = torch.tensor([0] + lens).cumsum(0).int()
+    base = torch.randn(len(lens), generator=g)
+    more = torch.cat([cu, n + 4 * torch.arange(1, 1001, dtype=torch.int32)])
+    kw = dict(gamma=0.99, lam=0.95)
+    suffix = mode == _ops.SCAN_SUFFIX_SUM
+
+    def run(k, offsets, b):
+        x = r[:k].to(DEV)
+        return _ops.reverse_scan(mode, x, v[:k].to(DEV), m[:k].to(DEV), _ops.rows_of(x, offsets.to(DEV)),
+                                 row_baseline=b.to(DEV) if suffix else None, **kw)
+
+    adv, ret = run(n, cu, base)
+    adv1, ret1 = run(total, more, torch.cat([base, torch.zeros(1000)]))
+    assert torch.equal(ret, ret1[:n]) and (adv is None or torch.equal(adv, adv1[:n]))
+    rd, vd, md = r.double().tolist(), v.double().tolist(), m.double().tolist()
+    ra, rr = [0.0] * n, [0.0] * n
+    for i, (a, b) in enumerate(zip(cu[:-1].tolist(), cu[1:].tolist())):
+        nv = last = 0.0
+        for t in range(b - 1, a - 1, -1):
+            if mode in (_ops.SCAN_GAE, _ops.SCAN_GAE_RESPONSE_ONLY):
+                if md[t] > 0:
+                    last = rd[t] + 0.99 * nv - vd[t] + 0.99 * 0.95 * last
+                    nv = vd[t]
+                keep = md[t] > 0 or mode == _ops.SCAN_GAE
+                ra[t], rr[t] = (last, last + vd[t]) if keep else (0.0, 0.0)
+            elif mode == _ops.SCAN_DISCOUNTED:
+                rr[t] = rd[t] + 0.99 * last
+                last = md[t] * rr[t]
+            else:
+                last += rd[t] * md[t]
+                rr[t], ra[t] = last, last - base[i].item() * md[t]
+    # sums of at most 4097 terms in trees: relative error of some 2^-24 * 2 log2(4097)
+    assert rel_l2(ret, T(rr)) < 5e-6 and (adv is None or rel_l2(adv, T(ra)) < 5e-6)
+
+
 # ---- group scalars ------------------------------------------------------------------------------------
 def _group_case(seed=7):
     d = W.c1_loss_only(seed, groups=6, samples=5, seqlen=200)
