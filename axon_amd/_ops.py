@@ -1043,17 +1043,19 @@ def logits_forward(logits, labels=None, want_entropy=True):
     require_device(logits, "logits_forward")
     n, v, ld = _logits_operands("logits_forward", logits, labels)
     dev = logits.device
-    out = torch.empty(3, max(n, 1), device=dev, dtype=torch.float32)
+    out = torch.empty(3, n, device=dev, dtype=torch.float32)
     ws_bytes = lib.axon_logits_fwd_workspace_bytes(_LOGITS_DTYPES[logits.dtype], n, v) if v > 0 else 0
     ws = torch.empty(ws_bytes // 4, device=dev, dtype=torch.float32) if ws_bytes > 0 else None
+    base = out.data_ptr()
     check(
         lib.axon_logits_fwd_ws(ptr(logits), _LOGITS_DTYPES[logits.dtype], ld, n, v, ptr(labels),
                                int(labels is not None and labels.dtype == torch.int64),
-                               ptr(out[0]) if labels is not None else None, ptr(out[1]) if want_entropy else None,
-                               ptr(out[2]), ptr(ws), stream_ptr()),
-        "axon_logits_fwd",
+                               base if labels is not None else None, base + 4 * n if want_entropy else None,
+                               base + 8 * n, ptr(ws), stream_ptr()),
+        "axon_logits_fwd_ws",
     )
-    return (out[0][:n] if labels is not None else None), (out[1][:n] if want_entropy else None), out[2][:n]
+    lp, ent, lse = out.unbind(0)
+    return (lp if labels is not None else None), (ent if want_entropy else None), lse
 
 
 def logits_backward(logits, labels, lse, entropy, g_logprob, g_entropy, inplace=False):

@@ -283,6 +283,12 @@ int row_parts(int64_t n, int64_t vocab, int elem_bytes) {
   return (int)(p < 1 ? 1 : (p < kMaxParts ? p : kMaxParts));
 }
 
+// The forward pays for a split with a second launch: rows of less than 128 KB, which one workgroup reads in about as
+// long, are left whole (32 x 151936 bf16, 300 KB, is split; 50257 and 32768 are not).
+int fwd_parts(int64_t n, int64_t vocab, int elem_bytes) {
+  return vocab * elem_bytes < 131072 ? 1 : row_parts(n, vocab, elem_bytes);
+}
+
 // every row of b sits on the same offset from a 16-byte boundary as the row of a
 bool same_offsets(const void* a, int64_t ld_a, const void* b, int64_t ld_b, int64_t n, int elem_bytes) {
   const uintptr_t d = reinterpret_cast<uintptr_t>(a) ^ reinterpret_cast<uintptr_t>(b);
@@ -301,7 +307,7 @@ int check_logits(const void* logits, int dtype, int64_t ld, int64_t n, int64_t v
 
 extern "C" int64_t axon_logits_fwd_workspace_bytes(int dtype, int64_t n, int64_t vocab) {
   if (n < 0 || vocab <= 0 || (dtype != AXON_LOGITS_F32 && dtype != AXON_LOGITS_BF16)) return AXON_ERR_ARG;
-  const int parts = row_parts(n, vocab, dtype == AXON_LOGITS_F32 ? 4 : 2);
+  const int parts = fwd_parts(n, vocab, dtype == AXON_LOGITS_F32 ? 4 : 2);
   return parts > 1 ? n * parts * 3 * (int64_t)sizeof(float) : 0;
 }
 
@@ -314,7 +320,7 @@ extern "C" int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int
   if (!lse || (logprob && !labels)) return AXON_ERR_ARG;
   const hipStream_t st = (hipStream_t)stream;
   const int eb = dtype == AXON_LOGITS_F32 ? 4 : 2;
-  const int parts = workspace ? row_parts(n, vocab, eb) : 1;
+  const int parts = workspace ? fwd_parts(n, vocab, eb) : 1;
   const dim3 grid((unsigned)(n * parts)), blk(kBlock);
 #define AXON_STATS(T, L)                                                                               \
   do {                                                                                                 \
