@@ -310,12 +310,13 @@ RS_MODES = {None: 0, "token": 1, "sequence": 2, "geometric": 3}
 
 
 def sampler_correction(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_threshold, rs_mode, rs_lr_lo, rs_lr_hi,
-                       log_veto):
+                       log_veto, acc=None):
     """Importance weights and rejection / veto mask.  Without a row-level quantity: one elementwise pass.  With
     one (veto, sequence or geometric level): one launch in which a workgroup owns whole rows, or (short rows, see
     ``OWNED_ROWS_MIN_MEAN_LEN``) a row-stats pass followed by an elementwise pass.
 
-    Returns (is_weights | None, new_mask fp32, acc[8] device tensor).
+    Returns (is_weights | None, new_mask fp32, acc[8] device tensor).  ``acc``: where the eight fp32 sums go (a
+    contiguous device tensor of at least 32 bytes; with no slots it is left as it is).
     """
     lib = _lib.load()
     require_device(old_lp, "sampler_correction")
@@ -327,7 +328,8 @@ def sampler_correction(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_thresho
     need_row = is_mode == 2 or rs_mode >= 2 or has_veto
     isw = torch.empty(rows.shape, device=dev, dtype=torch.float32) if is_mode else None
     new_mask = torch.empty(rows.shape, device=dev, dtype=torch.float32)
-    acc = _acc8(rows.n_slots, dev)
+    if acc is None:
+        acc = _acc8(rows.n_slots, dev)
     if need_row and _own_rows(rows):
         # a workgroup owns whole rows: one launch, one pass over the tokens, row sums in a fixed order
         check(
@@ -358,9 +360,9 @@ DIAG_OUT = 72
 
 
 def sampler_diag(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_lo, is_hi, rs_mode, rs_lo, rs_hi, rs_lr_lo,
-                 rs_lr_hi, log_is_lo, log_is_hi, log_rs_lo, log_rs_hi):
+                 rs_lr_hi, log_is_lo, log_is_hi, log_rs_lo, log_rs_hi, out=None):
     """All mismatch diagnostics as one float64 device tensor of DIAG_OUT raw sums / extrema
-    (layout: axon_sampler_diag in include/axon_amd.h).  No host synchronisation."""
+    (layout: axon_sampler_diag in include/axon_amd.h), ``out`` if given.  No host synchronisation."""
     lib = _lib.load()
     require_device(old_lp, "sampler_diag")
     _same_len("sampler_diag", rows.n_slots, old_log_probs=old_lp, sampler_log_probs=samp_lp, mask=mask)
@@ -368,9 +370,9 @@ def sampler_diag(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_lo, is_hi, rs
     old_lp, samp_lp = f32(old_lp), f32(samp_lp)
     mk, kind = mask_arg(mask)
     nbytes = lib.axon_sampler_diag_workspace_bytes(rows.n_rows, rows.n_slots)
-    ws = torch.empty(nbytes // 4, device=dev, dtype=torch.float32)
-    ws[: 6 * rows.n_rows].zero_()
-    out = torch.empty(DIAG_OUT, device=dev, dtype=torch.float64)
+    ws = torch.zeros(nbytes // 4, device=dev, dtype=torch.float32)  # the row sums start at zero
+    if out is None:
+        out = torch.empty(DIAG_OUT, device=dev, dtype=torch.float64)
     check(
         lib.axon_sampler_diag(ptr(old_lp), ptr(samp_lp), ptr(mk), kind, rows.cu_ptr, rows.n_rows, rows.n_slots,
                               rows.uniform_len, int(is_mode), float(is_lo), float(is_hi), int(rs_mode), float(rs_lo),

@@ -43,6 +43,25 @@ class _ClippedPolicyLoss(torch.autograd.Function):
         return _ops.scale_f32(grad, g_loss, acc[5]).to(ctx.in_dtype), None, None, None, None
 
 
+class _ValueLoss(torch.autograd.Function):
+    """Half the aggregated value loss; one launch where a product behind ``_ClippedPolicyLoss`` is a copy, a product
+    and an autograd node more."""
+
+    @staticmethod
+    def forward(ctx, vpreds, batch, rows, hp):
+        acc, grad = _ops.policy_loss(_KIND_VALUE, vpreds, batch["old_log_probs"], batch["advantages"],
+                                     batch["response_mask"], None, rows, **hp)
+        ctx.save_for_backward(grad, acc)
+        ctx.in_dtype = vpreds.dtype
+        ctx.mark_non_differentiable(acc)
+        return 0.5 * acc[0], acc
+
+    @staticmethod
+    def backward(ctx, g_loss, _g_acc):
+        grad, acc = ctx.saved_tensors
+        return _ops.scale_f32(grad, 0.5 * g_loss, acc[5]).to(ctx.in_dtype), None, None, None
+
+
 def _aggregation(b, config, default_token_reduce: str) -> dict:
     """The ``agg_loss`` arguments of a loss call (loss/utils.py:120-251), validated as the reference does."""
     token_reduce = config.get("token_reduce", default_token_reduce)
@@ -203,11 +222,9 @@ def value_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
     agg = _aggregation(b, config, "sum")
     _lib.require_device(vpreds, "value loss")
     rows = _ops.rows_of(vpreds, data.meta_info.get("cu_seqlens", None) if data.meta_info else None)
-    tensors = {"old_log_probs": b["values"], "advantages": b["returns"], "response_mask": b["response_mask"],
-               "sampler_is_weights": None}
+    tensors = {"old_log_probs": b["values"], "advantages": b["returns"], "response_mask": b["response_mask"]}
     hp = dict(ratio_lo=config.get("cliprange_value", 0.5), ratio_hi=0.0, clip_c=0.0, **agg)
-    raw, acc = _ClippedPolicyLoss.apply(vpreds, _KIND_VALUE, tensors, rows, hp)
-    loss = 0.5 * raw
+    loss, acc = _ValueLoss.apply(vpreds, tensors, rows, hp)
     sums = acc.tolist()
     denom = max(sums[4], 1.0)
     return loss, {"vf_loss": 0.5 * sums[0], "vf_clipfrac": sums[1] / denom, "vpred_mean": sums[2] / denom}

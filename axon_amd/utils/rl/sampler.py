@@ -246,11 +246,14 @@ def compute_sampler_correction_and_rejection_mask(
 
     _ops.require_device(old_log_prob, "compute_sampler_correction_and_rejection_mask")
     rows = _ops.rows_of(old_log_prob, cu_seqlens)
-    weights, new_mask, acc = _ops.sampler_correction(
+    # the eight fp32 sums of the correction (32 bytes), then the diagnostics: one buffer, one copy to the host
+    both = torch.zeros(4 + _ops.DIAG_OUT, device=old_log_prob.device, dtype=torch.float64) if rows.n_slots == 0 else \
+        torch.empty(4 + _ops.DIAG_OUT, device=old_log_prob.device, dtype=torch.float64)
+    weights, new_mask, _ = _ops.sampler_correction(
         old_log_prob, sampler_log_prob, response_mask, rows,
         is_mode=_ops.IS_MODES[sampler_is] if use_is else 0,
         is_threshold=sampler_is_threshold if use_is else 1.0,
-        rs_mode=_ops.RS_MODES[sampler_rs], rs_lr_lo=rs_lo, rs_lr_hi=rs_hi, log_veto=log_veto,
+        rs_mode=_ops.RS_MODES[sampler_rs], rs_lr_lo=rs_lo, rs_lr_hi=rs_hi, log_veto=log_veto, acc=both,
     )
     is_hi = float(sampler_is_threshold) if use_is else 1.0
     is_lo = 1.0 / is_hi
@@ -258,14 +261,14 @@ def compute_sampler_correction_and_rejection_mask(
     rs_lo_t = (float(sampler_rs_threshold_lower) if sampler_rs_threshold_lower is not None else 1.0 / rs_hi_t) \
         if sampler_rs is not None else 1.0
     tok_lo, tok_hi = (rs_lo, rs_hi) if sampler_rs == "token" else (-math.inf, math.inf)
-    diag = _ops.sampler_diag(
-        old_log_prob, sampler_log_prob, response_mask, rows,
+    _ops.sampler_diag(
+        old_log_prob, sampler_log_prob, response_mask, rows, out=both[4:],
         is_mode=_ops.IS_MODES[sampler_is] if use_is else 0, is_lo=is_lo, is_hi=is_hi,
         rs_mode=_ops.RS_MODES[sampler_rs], rs_lo=rs_lo_t, rs_hi=rs_hi_t, rs_lr_lo=tok_lo, rs_lr_hi=tok_hi,
         log_is_lo=_log32(is_lo), log_is_hi=_log32(is_hi), log_rs_lo=_log32(rs_lo_t), log_rs_hi=_log32(rs_hi_t),
     )
-    both = torch.cat([acc.double(), diag]).tolist()  # single readback: empty-mask test and every metric
-    sums, d = both[:8], both[8:]
+    host = both.cpu().numpy()  # single readback: empty-mask test and every metric
+    sums, d = host[:4].view(np.float32).tolist(), host[4:].tolist()
     n_valid = sums[0]
     if n_valid == 0:
         return None, response_mask, {}
