@@ -2,8 +2,8 @@
 // global masked whitening, and the per-group scalars of the estimators that need more than mean/std.
 //
 // A recurrence y[t] = b[t] + a[t] * y[t+1] is a scan over pairs (a, b) under the composition
-// (a2, b2) o (a1, b1) = (a2*a1, b2 + a2*b1).  One wavefront owns one row and walks it from the end in
-// windows of 256 tokens that are 4-aligned in the token array: a lane holds four consecutive tokens (one
+// (a2, b2) o (a1, b1) = (a2*a1, b2 + a2*b1).  One wavefront (or, for long rows, one workgroup, each wavefront
+// with a quarter of 1024 tokens) owns one row and walks it from the end in windows of 256 tokens that are 4-aligned in the token array: a lane holds four consecutive tokens (one
 // 16-byte access where the vector lies inside the row, guarded scalar accesses at the row's edges), lane 0
 // the last ones.  A lane composes its four elements, the wavefront scans the 64 composites with DPP row shifts and broadcasts,
 // and each lane then replays its four tokens from the value that enters it.  The loads of the next window
@@ -50,9 +50,25 @@ __device__ __forceinline__ Pair wave_scan(Pair p) {
 }
 
 // Scans the lanes' composites; returns the value that enters this lane (the recurrence at the token after the
-// lane's last one) and moves `carry` to the value that leaves lane 63.
-__device__ __forceinline__ float scan_enter(Pair lane_total, float& carry) {
+// lane's last one) and moves `carry` to the value that leaves the window.  W wavefronts with a quarter of the window
+// each: they exchange their totals through `tot` and pass the carry on in order, the arithmetic of one wavefront that
+// walks the quarters.  All threads of the workgroup call; one barrier, so consecutive calls need different `tot`.
+template <int W>
+__device__ __forceinline__ float scan_enter(Pair lane_total, float& carry, Pair* tot) {
   const Pair s = wave_scan(lane_total);
+  if (W > 1) {
+    const int wave = threadIdx.x / kWave;
+    if ((threadIdx.x & (kWave - 1)) == kWave - 1) tot[wave] = s;
+    __syncthreads();
+    float mine = carry;
+#pragma unroll
+    for (int u = 0; u < W; ++u) {
+      if (u == wave) mine = carry;
+      carry = tot[u].b + tot[u].a * carry;
+    }
+    const float leaves = s.b + s.a * mine;
+    return dpp_move<0x138, 0xf>(mine, leaves);  // wave_shr:1; lane 0 keeps what enters the wavefront
+  }
   const float leaves = s.b + s.a * carry;
   const float enters = dpp_move<0x138, 0xf>(carry, leaves);  // wave_shr:1; lane 0 keeps the carry
   carry = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, leaves), kWave - 1));
@@ -104,15 +120,20 @@ __device__ __forceinline__ void scan_load(ScanBlock& x, const float* __restrict_
 // MODE kScanGaeResponseOnly: the same over the tokens with mask > 0, 0 elsewhere.
 // MODE kScanDiscounted: Q[t] = m (r + gamma Q[t+1]);  ret = r + gamma Q[t+1].
 // MODE kScanSuffixSum:  ret[t] = sum_{s >= t} r m;  adv = ret - row_baseline * m.
-template <int MK, int MODE>
+// W = 1: a wavefront owns a row; W = 4: a workgroup does, in windows of 1024 tokens.
+template <int MK, int MODE, int W>
 __global__ __launch_bounds__(kBlock) void reverse_scan_kernel(
     const float* __restrict__ rewards, const float* __restrict__ values,
     const void* __restrict__ mask, const int32_t* __restrict__ cu, int64_t n_rows, int64_t n_slots,
     int64_t uniform_len, float gamma, float gamma_lam, const float* __restrict__ row_baseline,
     float* __restrict__ adv, float* __restrict__ ret, int vec_ok) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = (int64_t)blockIdx.x * (kBlock / kWave) + (threadIdx.x / kWave);
-  if (row >= n_rows) return;  // whole wavefronts leave together; no workgroup barrier below
+  static_assert(W == 1 || W == kBlock / kWave, "");
+  __shared__ Pair tot[2][2][kBlock / kWave];  // by recurrence and window parity: a slot is written again two barriers on
+  const int64_t row = W > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * (kBlock / kWave) + (threadIdx.x / kWave);
+  if (row >= n_rows) return;  // W = 1: whole wavefronts leave together, no workgroup barrier below; W = 4: the workgroup
+  const int64_t back = W > 1 ? (int64_t)(threadIdx.x / kWave) * kScanStep : 0;  // this wavefront's part of the window
+  int par = 0;
   int64_t begin = uniform_len > 0 ? row * uniform_len : (int64_t)cu[row];
   int64_t stop = uniform_len > 0 ? begin + uniform_len : (int64_t)cu[row + 1];
   begin = begin < 0 ? 0 : begin;              // offsets outside the arrays (caller error) touch nothing
@@ -122,23 +143,23 @@ __global__ __launch_bounds__(kBlock) void reverse_scan_kernel(
   float carry0 = 0.f, carry1 = 0.f;  // the recurrences' values at the token after the current window
   const int64_t last = (stop + kScanVec - 1) & ~(int64_t)(kScanVec - 1);
   ScanBlock cur, nxt;
-  scan_load<MK, MODE>(cur, rewards, values, mask, begin, stop, last, vec_ok);
-  for (int64_t end = last; end > begin; end -= kScanStep) {
-    const bool more = end - kScanStep > begin;
-    if (more) scan_load<MK, MODE>(nxt, rewards, values, mask, begin, stop, end - kScanStep, vec_ok);
+  scan_load<MK, MODE>(cur, rewards, values, mask, begin, stop, last - back, vec_ok);
+  for (int64_t end = last; end > begin; end -= W * kScanStep, par ^= 1) {
+    const bool more = end - W * kScanStep > begin;
+    if (more) scan_load<MK, MODE>(nxt, rewards, values, mask, begin, stop, end - W * kScanStep - back, vec_ok);
     float out_adv[kScanVec], out_ret[kScanVec];
     if (MODE <= kScanGaeResponseOnly) {
       Pair e[kScanVec];
 #pragma unroll
       for (int j = 0; j < kScanVec; ++j) e[j] = Pair{1.f - cur.m[j], cur.m[j] * cur.v[j]};
-      float nv = scan_enter(after(e[0], after(e[1], after(e[2], e[3]))), carry0);
+      float nv = scan_enter<W>(after(e[0], after(e[1], after(e[2], e[3]))), carry0, tot[0][par]);
 #pragma unroll
       for (int j = kScanVec - 1; j >= 0; --j) {
         const float delta = cur.r[j] + gamma * nv - cur.v[j];
         nv = e[j].b + e[j].a * nv;
         e[j] = Pair{cur.m[j] * gamma_lam + (1.f - cur.m[j]), cur.m[j] * delta};
       }
-      float l = scan_enter(after(e[0], after(e[1], after(e[2], e[3]))), carry1);
+      float l = scan_enter<W>(after(e[0], after(e[1], after(e[2], e[3]))), carry1, tot[1][par]);
 #pragma unroll
       for (int j = kScanVec - 1; j >= 0; --j) {
         l = e[j].b + e[j].a * l;
@@ -154,7 +175,7 @@ __global__ __launch_bounds__(kBlock) void reverse_scan_kernel(
         if (MODE == kScanDiscounted) e[j] = Pair{ok ? gamma * cur.m[j] : 1.f, cur.m[j] * cur.r[j]};
         else e[j] = Pair{1.f, cur.r[j] * cur.m[j]};
       }
-      float q = scan_enter(after(e[0], after(e[1], after(e[2], e[3]))), carry0);
+      float q = scan_enter<W>(after(e[0], after(e[1], after(e[2], e[3]))), carry0, tot[0][par]);
 #pragma unroll
       for (int j = kScanVec - 1; j >= 0; --j) {
         if (MODE == kScanDiscounted) {
@@ -168,7 +189,7 @@ __global__ __launch_bounds__(kBlock) void reverse_scan_kernel(
         }
       }
     }
-    const int64_t p0 = end - kScanVec * (lane + 1);
+    const int64_t p0 = end - back - kScanVec * (lane + 1);
     if (cur.ok == 15 && vec_ok) {
       if (adv != nullptr) store4(adv, p0, out_adv);
       store4(ret, p0, out_ret);
@@ -409,10 +430,21 @@ int launch_scan(int mode, const float* rewards, const float* values, const void*
   const int vec_ok = ((reinterpret_cast<uintptr_t>(rewards) | reinterpret_cast<uintptr_t>(values) |
                        reinterpret_cast<uintptr_t>(mask) | reinterpret_cast<uintptr_t>(adv) |
                        reinterpret_cast<uintptr_t>(ret)) & 15) == 0;
-  const dim3 grid((unsigned)((n_rows + (kBlock / kWave) - 1) / (kBlock / kWave))), blk(kBlock);
+  constexpr int kWaves = kBlock / kWave;
+  // A workgroup per row where rows are longer than two of a wavefront's windows on average: a launch lasts as long as
+  // its longest row's chain of windows, and a long batch of such rows is faster too.  Rows of 900 tokens on average, a
+  // wavefront / a workgroup each: 310 rows 16.5 / 9.2 us, 2308 35.6 / 20.5, 9223 57.2 / 39.7, 36647 164 / 127; 30000 rows of 576 tokens 59.5 / 56.8, of 448 44.9 / 50.7.
+  const bool wide = n_slots > 2 * kScanStep * n_rows;
+  const dim3 grid((unsigned)(wide ? n_rows : (n_rows + kWaves - 1) / kWaves)), blk(kBlock);
 #define AXON_SCAN(M)                                                                              \
-  hipLaunchKernelGGL((reverse_scan_kernel<MK, M>), grid, blk, 0, st, rewards, values, mask, cu,   \
-                     n_rows, n_slots, uniform_len, gamma, gamma_lam, row_baseline, adv, ret, vec_ok)
+  do {                                                                                            \
+    if (wide)                                                                                     \
+      hipLaunchKernelGGL((reverse_scan_kernel<MK, M, kWaves>), grid, blk, 0, st, rewards, values, mask, cu, \
+                         n_rows, n_slots, uniform_len, gamma, gamma_lam, row_baseline, adv, ret, vec_ok);   \
+    else                                                                                          \
+      hipLaunchKernelGGL((reverse_scan_kernel<MK, M, 1>), grid, blk, 0, st, rewards, values, mask, cu,      \
+                         n_rows, n_slots, uniform_len, gamma, gamma_lam, row_baseline, adv, ret, vec_ok);   \
+  } while (0)
   switch (mode) {
     case kScanGae: AXON_SCAN(kScanGae); break;
     case kScanGaeResponseOnly: AXON_SCAN(kScanGaeResponseOnly); break;

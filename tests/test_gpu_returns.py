@@ -234,7 +234,7 @@ def test_group_advantage_with_more_rows_than_one_trip(n_rows, mode):
 @pytest.mark.parametrize("mode", [_ops.SCAN_GAE, _ops.SCAN_GAE_RESPONSE_ONLY, _ops.SCAN_DISCOUNTED, _ops.SCAN_SUFFIX_SUM])
 def test_scan_by_workgroup_equals_scan_by_wavefront(mode, mask_dtype):
     """Rows around the edges of a wavefront's 256 and a workgroup's 1024 tokens, on every offset from a 16-byte boundary.
-    Short rows behind them bring the mean length under a window, so the second launch gives each row one wavefront:
+    Short rows behind them bring the mean length under two windows, so the second launch gives each row one wavefront:
     the same arithmetic in the same order, hence the same bits.  The first launch against a loop in float64."""
     lens = [1, 255, 256, 257, 3, 1023, 1024, 1025, 2050, 4097, 0, 767, 770]
     n = sum(lens)
