@@ -236,10 +236,10 @@ __global__ __launch_bounds__(1024) void group_stats_kernel(
 // in memory.  A wavefront owns a row (double accumulators per lane, then a fixed tree), four 16-byte loads in flight;
 // the grid is bounded so that its tickets stay cheap.  The groups' sums are formed in LDS (double, so that the order
 // in which the rows arrive does not show in the fp32 results).
-// 128 x 1024 slots, 16 groups: 8.3 us where fill, row pass, finish and group kernel took 6.9 + 1.3 + 10.9 and two fills;
-// 8.4 M slots in 9000 rows, 1150 groups: 40 for 27 + 4.7 + 80.
+// 128 x 1024 slots, 16 groups: 7.5 us where fill, row pass, finish and group kernel took 6.9 + 1.3 + 10.9 and two fills;
+// 8.4 M slots in 9000 rows, 1150 groups: 33 for 27 + 4.7 + 80 (40 with one row after the other in the last workgroup).
 constexpr int kScoreGroups = 2048;  // 40 KB of LDS
-constexpr int kScoreBlocks = 1024;
+constexpr int kScoreBlocks = 512;  // what fits the part at once: a wavefront with a short row takes another one
 
 __global__ __launch_bounds__(1024) void group_scores_kernel(
     const float* __restrict__ a, const int32_t* __restrict__ cu, int64_t n_rows, int64_t n_slots, int64_t uniform_len,
@@ -255,21 +255,19 @@ __global__ __launch_bounds__(1024) void group_scores_kernel(
     t1 = min(max(t1, t0), n_slots);
     double acc = 0.0;
     const int64_t b0 = min((t0 + 3) & ~(int64_t)3, t1), b1 = max(t1 & ~(int64_t)3, b0);  // whole vectors
-    if (lane < b0 - t0) acc += (double)a[t0 + lane];
-    if (lane < t1 - b1) acc += (double)a[b1 + lane];
-    int64_t p = b0 + lane * kVec;
-    for (; p + 3 * kWave * kVec < b1; p += 4 * kWave * kVec) {
+    // the row's edges and its first four vectors per lane are on their way before anything is added
+    const float e0 = lane < b0 - t0 ? a[t0 + lane] : 0.f, e1 = lane < t1 - b1 ? a[b1 + lane] : 0.f;
+    for (int64_t p = b0 + lane * kVec; p < b1; p += 4 * kWave * kVec) {
       float v[4][4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) load4(a, p + u * kWave * kVec, v[u]);
+      for (int u = 0; u < 4; ++u) load4(a, min(p + u * kWave * kVec, b1 - kVec), v[u]);  // a valid vector; dropped below
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc += ((double)v[u][0] + (double)v[u][1]) + ((double)v[u][2] + (double)v[u][3]);
+      for (int u = 0; u < 4; ++u) {
+        const double x = ((double)v[u][0] + (double)v[u][1]) + ((double)v[u][2] + (double)v[u][3]);
+        acc += p + u * kWave * kVec < b1 ? x : 0.0;
+      }
     }
-    for (; p < b1; p += kWave * kVec) {
-      float v[4];
-      load4(a, p, v);
-      acc += ((double)v[0] + (double)v[1]) + ((double)v[2] + (double)v[3]);
-    }
+    acc += (double)e0 + (double)e1;
     acc = wave_sum_d(acc);
     if (lane == 0) __hip_atomic_store(scores + r, (float)acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -289,15 +287,51 @@ __global__ __launch_bounds__(1024) void group_scores_kernel(
   __syncthreads();
   if (!last) return;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  for (int64_t i = threadIdx.x; i < n_rows; i += blockDim.x) {
-    const int64_t k = gidx[i];
-    const float x = scores[i];
-    if (g.mode == 3 && x != 0.f) atomicAdd(&nonzero, 1);
-    if (k < 0 || k >= n_groups) continue;
-    atomicAdd(&count[k], 1);
-    atomicAdd(&sums[k][0], (double)x);
-    atomicAdd(&sums[k][1], (double)x * (double)x);
-  }
+  // Up to 1024 rows: a thread has one.  More: eight consecutive rows per thread and trip, their loads all in flight (a
+  // load from behind a dropped cache is a microsecond).  Rows of a group lie next to one another as a rule: a thread adds
+  // up its run of a group in registers and adds to LDS once per run, and the threads of a wavefront rarely meet on one
+  // address.  (With 128 rows eight in a row per thread cost 2.5 us more than one.)
+  const int per = n_rows <= blockDim.x ? 1 : 8;
+  auto each_eight = [&](auto&& f) {
+    for (int64_t i0 = per * (int64_t)threadIdx.x; i0 < n_rows; i0 += 8 * (int64_t)blockDim.x) {
+      int64_t k[8];
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int64_t i = min(i0 + u, n_rows - 1);  // a valid row; dropped by f
+        k[u] = gidx[i];
+        x[u] = scores[i];
+      }
+      f(i0, k, x);
+    }
+  };
+  each_eight([&](int64_t i0, const int64_t (&k)[8], const float (&x)[8]) {
+    int run = -1, c = 0, nz = 0;
+    double s1 = 0.0, s2 = 0.0;
+    auto flush = [&]() {
+      if (run < 0) return;
+      atomicAdd(&count[run], c);
+      atomicAdd(&sums[run][0], s1);
+      atomicAdd(&sums[run][1], s2);
+    };
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (u >= per || i0 + u >= n_rows) break;
+      nz += x[u] != 0.f ? 1 : 0;
+      if (k[u] < 0 || k[u] >= n_groups) continue;
+      if ((int)k[u] != run) {
+        flush();
+        run = (int)k[u];
+        c = 0;
+        s1 = s2 = 0.0;
+      }
+      ++c;
+      s1 += (double)x[u];
+      s2 += (double)x[u] * (double)x[u];
+    }
+    flush();
+    if (g.mode == 3 && nz != 0) atomicAdd(&nonzero, nz);
+  });
   __syncthreads();
   for (int k = threadIdx.x; k < n_groups; k += blockDim.x) {  // sums -> mean and deviation, singletons 0 and 1
     const double c = (double)count[k], cc = fmax(c, 1.0);
@@ -309,11 +343,16 @@ __global__ __launch_bounds__(1024) void group_scores_kernel(
   }
   __syncthreads();
   const float alpha = (float)n_rows / (float)max(nonzero, 1);
-  for (int64_t i = threadIdx.x; i < n_rows; i += blockDim.x) {
-    const int64_t k = gidx[i];
-    const bool ok = k >= 0 && k < n_groups;
-    scalar[i] = ok ? group_scalar_of(g, scores[i], (float)count[k], (float)sums[k][0], (float)sums[k][1], alpha) : 0.f;
-  }
+  each_eight([&](int64_t i0, const int64_t (&k)[8], const float (&x)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (u >= per || i0 + u >= n_rows) break;
+      const bool ok = k[u] >= 0 && k[u] < n_groups;
+      const int q = ok ? (int)k[u] : 0;
+      const float v = group_scalar_of(g, x[u], (float)count[q], (float)sums[q][0], (float)sums[q][1], alpha);
+      scalar[i0 + u] = ok ? v : 0.f;
+    }
+  });
 }
 
 template <int MK>
