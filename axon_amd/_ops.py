@@ -886,7 +886,9 @@ class HeadBlocks:
     d_hidden; bf16 dlogits of block x vocab x 2 bytes), else a multiple of 256.  ``dw_group``: how many
     consecutive blocks share one weight-gradient GEMM (their dlogits stay in the workspace until the group's
     last block: a longer reduction and fewer passes over the fp32 partial sums for ``dw_group`` x the dlogit
-    memory); 1 where the shape does not allow it (``axon_lmhead_block_can_group``)."""
+    memory); 1 where the shape does not allow it (``axon_lmhead_block_can_group``).  ``stash``: whether the blocks'
+    dlogits are decoded from a stash (softmax numerators in 16 bits) or their logits recomputed in fp32, for all
+    blocks or one truth value per block."""
 
     def __init__(self, hidden, weight, labels, inv_temperature, ranges, *, softcap=0.0, seq_start=None,
                  vocab_chunk=0, stash=True, dw_group=2, timing: "Timer | None" = None):
@@ -916,7 +918,11 @@ class HeadBlocks:
             raise _lib.AxonAmdError(f"HeadBlocks: unsupported shape tokens={n_max} hidden={self.h} vocab={self.v}")
         self.fwd_ws = torch.empty(self.fwd_ws_bytes, device=dev, dtype=torch.uint8)
         self.bwd_ws = torch.empty(self.bwd_ws_bytes, device=dev, dtype=torch.uint8)
-        self.stash_bytes = self._stash_bytes(n_max) if stash else 0
+        self.keeps_stash = [bool(stash)] * len(self.ranges) if isinstance(stash, bool) else [bool(x) for x in stash]
+        if len(self.keeps_stash) != len(self.ranges):
+            raise ValueError(f"HeadBlocks: {len(self.keeps_stash)} stash choices for {len(self.ranges)} blocks")
+        self.stash_bytes = max((self._stash_bytes(b - a) for (a, b), keep in zip(self.ranges, self.keeps_stash) if keep),
+                               default=0)
         self.stash = torch.empty(self.stash_bytes, device=dev, dtype=torch.uint8) if self.stash_bytes else None
         self.stats = torch.empty(2, n_max, device=dev, dtype=torch.float32)  # lse, entropy_b of the current block
         # whole-stream outputs; position 0 is a sequence start (the aligned layout writes it from the last row)
@@ -955,7 +961,7 @@ class HeadBlocks:
         stream reaches the point after the call."""
         n0, n1, last_dst = self._block(k)
         nb = n1 - n0
-        self.block_stash_bytes = self._stash_bytes(nb) if self.stash is not None else 0
+        self.block_stash_bytes = self._stash_bytes(nb) if self.keeps_stash[k] else 0
         check(self.lib.axon_lmhead_block_fwd(
             self.hidden.data_ptr() + n0 * self.h * 2, ptr(self.weight), self._at(self.labels, n0),
             int(self.labels.dtype == torch.int64), nb, self.h, self.v, self.inv_t, self.softcap,

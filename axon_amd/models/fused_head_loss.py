@@ -62,6 +62,15 @@ def sequence_blocks(cu: list, block_tokens: int):
     return out
 
 
+def blocks_with_stash(ranges, n: int, h: int, v: int):
+    """Per block: whether its backward decodes the dlogits from the forward's stash, whose softmax numerators have
+    16 bits, or recomputes the logits in fp32.  The stash where the whole-call operator has one for such a shape
+    (``lmhead_stash_bytes``: large blocks need token count and vocabulary in fours); a block with others behind it counts
+    as rounded up to four rows, so that among the large blocks of such a vocabulary only the one that ends an odd
+    stream recomputes: one more product of its rows, and no bits that a caller did not give away."""
+    return [_ops.lmhead_stash_bytes(min(n - a, (b - a + 3) // 4 * 4), h, v) > 0 for a, b in ranges]
+
+
 def _global_count(mask, rows, batch_reduce, given):
     """The batch-wide denominator of ``agg_loss``'s batch reduction as a device scalar (loss/utils.py:190-214):
     the count the batch carries, else the number of mask tokens (token-mean) or of rows with any (step-mean)."""
@@ -122,7 +131,7 @@ class _BlockedHeadLoss(torch.autograd.Function):
 
         hb = _ops.HeadBlocks(hidden, weight, spec["ids"], spec["inv_t"], ranges, softcap=spec["softcap"],
                              seq_start=spec["seq_start"], vocab_chunk=spec["vocab_chunk"], dw_group=spec["dw_group"],
-                             timing=_ops.TIMING)
+                             stash=blocks_with_stash(ranges, n, hidden.shape[1], weight.shape[0]), timing=_ops.TIMING)
         g_lp = torch.zeros(n + 4, device=dev, dtype=torch.float32)
         want_ent_grad = side is not None and side["entropy_coef"] != 0
         g_en = torch.zeros(n + 4, device=dev, dtype=torch.float32) if want_ent_grad else None

@@ -286,6 +286,51 @@ def test_fused_step_odd_shapes_softcap_temperature_and_integer_operands(case):
         assert metrics[k] == pytest.approx(val, rel=1e-4, abs=1e-6), k
 
 
+@pytest.mark.parametrize("v", [2000, 1999])
+@pytest.mark.parametrize("case", ["ppo", "gspo"])
+def test_large_blocks_that_the_stash_is_not_kept_for_recompute_in_fp32(monkeypatch, case, v):
+    """Blocks of 256 rows and more whose tokens (the last one's) or vocabulary are no multiple of four recompute
+    their logits in fp32: the gradients are bit for bit those of a step that keeps no stash at all.  Where the other
+    blocks do keep one, the rows of the last block are."""
+    from axon_amd import _ops
+    from axon_amd.models.fused_head_loss import fused_head_loss
+    lens = [256, 301, 211, 256, 277]  # 1301 tokens; blocks of 512, or whole sequences of 557 and 467: the last has 277 rows
+    n, h = sum(lens), 128
+    name, args = {"ppo": ("ppo", PPO), "gspo": ("gspo", GSPO)}[case]
+    g = torch.Generator().manual_seed(17)
+    hid = torch.randn(n, h, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(v, h, generator=g) * 0.2).bfloat16().to(DEV)
+    ids = torch.randint(0, v, (n,), generator=g).to(DEV)
+    old, adv = (-8 + 0.1 * torch.randn(n, generator=g)).to(DEV), torch.randn(n, generator=g).to(DEV)
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(DEV)
+    real = _ops.HeadBlocks
+    kept = []
+
+    class Recording(real):
+        def forward(self, k):
+            super().forward(k)
+            kept.append(self.block_stash_bytes > 0)
+
+    def step(cls):
+        monkeypatch.setattr(_ops, "HeadBlocks", cls)
+        hd, wd = hid.clone().requires_grad_(True), w.clone().requires_grad_(True)
+        data = DataProto.from_dict(tensors={"old_log_probs": old, "advantages": adv,
+                                            "response_mask": torch.ones(n, device=DEV)})
+        loss, _ = fused_head_loss(hd, wd, ids, cu, data, {"loss_fn": name, "loss_fn_args": args, "temperature": 1.0,
+                                                          "dp_replicas": 1}, block_tokens=560 if case == "gspo" else 512)
+        loss.backward()
+        return hd.grad, wd.grad
+
+    dh, dw = step(Recording)
+    dh0, dw0 = step(lambda *a, **k: real(*a, **dict(k, stash=False)))
+    assert len(kept) == 3 and not kept[-1] and kept[:-1] == [v % 4 == 0] * 2
+    assert torch.equal(dh[1024:], dh0[1024:]) and dh[1024:].float().norm() > 0
+    if v % 4:
+        assert torch.equal(dh, dh0) and torch.equal(dw, dw0)
+    else:
+        assert rel_l2(dh, dh0) < 5e-3 and rel_l2(dw, dw0) < 5e-3
+
+
 def test_fused_step_falls_back_where_blocks_do_not_apply():
     """A loss that selects tokens across the whole batch, and a sequence longer than a block under a
     per-sequence loss, take the unfused path; the node refuses a second backward."""
