@@ -44,6 +44,7 @@ SIGNATURES: dict[str, tuple] = {
                                      _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
     "axon_lmhead_block_can_group": (_i32, [_i64, _i64, _i64]),
     "axon_lmhead_bwd_dlogit_copies": (_i32, [_i64, _i64, _i64]),
+    "axon_lmhead_bwd_dhidden_parts": (_i64, [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
     "axon_scale_bf16_unless_one": (_i32, [_ptr, _i64, _ptr, _ptr]),
     "axon_lmhead_active_rows": (_i32, [_ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr]),
     "axon_lmhead_gather_rows": (_i32, [_ptr, _ptr, _i32, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _i64,
@@ -102,7 +103,7 @@ SIGNATURES: dict[str, tuple] = {
                                         _ptr, _ptr, _f32, _i32, _ptr, _f32, _f32, _f32, _ptr, _ptr, _ptr]),
 }
 
-ABI_VERSION = 21
+ABI_VERSION = 22
 MASK_F32, MASK_I64 = 0, 1
 
 _lock = threading.Lock()

@@ -1085,11 +1085,17 @@ bool stash_of_all_tokens(int64_t n, int64_t h, int64_t v) {
 // A part has at least kMinPartTiles k-tiles: below that its first loads and its epilogue are a quarter of its time.
 constexpr int kMaxSplits = 64, kMaxUnits = 3 * kCus, kMinPartTiles = 32;
 struct SplitPlan { int splits, k_split; };
+// The most parts that a reduction of kt k-tiles is planned in, whatever the number of tiles: the plan's bound and
+// what the workspace has room for.
+int64_t max_splits(int64_t kt) {
+  const int64_t longest = kt / kMinPartTiles;
+  return longest < 1 ? 1 : longest < kMaxSplits ? longest : kMaxSplits;
+}
 SplitPlan split_plan(int64_t tiles, int64_t k) {
-  const int64_t kt = (k + 63) / 64;
+  const int64_t kt = (k + 63) / 64, most = max_splits(kt);
   SplitPlan best{1, (int)(kt * 64)};
   int64_t best_cost = INT64_MAX;
-  for (int s = 1; s <= kMaxSplits && (s == 1 || (s * kMinPartTiles <= kt && tiles * s <= kMaxUnits)); ++s) {
+  for (int s = 1; s <= most && (s == 1 || tiles * s <= kMaxUnits); ++s) {
     const int64_t per = (kt + s - 1) / s, parts = (kt + per - 1) / per;  // every part gets k-tiles
     if (parts != s) continue;
     const int64_t units = tiles * s, full = units / kCus, rem = units % kCus;
@@ -1103,6 +1109,7 @@ SplitPlan split_plan(int64_t tiles, int64_t k) {
 struct BwdWs {
   __bf16 *hT, *dl, *dlT;
   float4* dh_acc;  // dHidden partial sums in tile order: the parts of a split reduction, or carried over the chunks
+  int64_t dh_parts;  // how many 256 KB tile parts dh_acc holds
   int64_t v_pad, n_pad, chunk, bytes;
   int64_t ld_n, ld_c;  // leading dimensions of hT/dlT, dl: padded by kLdPad elements
   int chunks;
@@ -1143,15 +1150,23 @@ BwdWs bwd_ws(int64_t n, int64_t h, int64_t vocab, int64_t chunk, void* base) {
     off += round_up(w.chunk * w.ld_n * 2, kAlign);
   }
   const int64_t dh_tiles = (round_up(h, kTile) / kTile) * (w.n_pad / kTile);
-  // room for the parts of any call over at most n tokens (split_plan), or for one part per tile
-  const int64_t longest = vocab / (64 * kMinPartTiles);
-  const int64_t max_splits = longest < kMaxSplits ? longest : kMaxSplits;
-  int64_t parts = max_splits < 2 ? 0 : dh_tiles * max_splits < kMaxUnits ? dh_tiles * max_splits : kMaxUnits;
+  // room for the parts of any call over at most n tokens (dh_plan), or for one part per tile
+  const int64_t most = max_splits(((w.chunks > 1 ? w.chunk : vocab) + 63) / 64);
+  int64_t parts = most < 2 ? 0 : dh_tiles * most < kMaxUnits ? dh_tiles * most : kMaxUnits;
   if (w.chunks > 1 && parts < dh_tiles) parts = dh_tiles;
   w.dh_acc = reinterpret_cast<float4*>(p + off);
+  w.dh_parts = parts;
   off += parts * kTileAccVecs * 16;
   w.bytes = off;
   return w;
+}
+
+// dHidden of a call over `n` tokens: how its tiles' reductions are shared, and the tile parts that it keeps in dh_acc.
+struct DhPlan { SplitPlan split; int64_t parts; };
+DhPlan dh_plan(const BwdWs& w, int64_t n, int64_t h, int64_t v) {
+  const int64_t tiles = (round_up(h, kTile) / kTile) * (round_up(n, kTile) / kTile);
+  const SplitPlan split = split_plan(tiles, w.chunks > 1 ? w.chunk : v);
+  return DhPlan{split, (w.chunks > 1 || split.splits > 1) ? tiles * split.splits : 0};
 }
 
 // Optional per-phase timing with HIP events on the launch stream (used by the *_timed entry points
@@ -1360,6 +1375,9 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   char* base = reinterpret_cast<char*>(round_up(reinterpret_cast<int64_t>(workspace), kAlign));
   const BwdWs w = bwd_ws(ws_tokens, h, v, chunk, base);
   if ((base - static_cast<char*>(workspace)) + w.bytes > ws_bytes) return AXON_ERR_WORKSPACE;
+  const DhPlan dh = dh_plan(w, n, h, v);
+  const SplitPlan plan = dh.split;
+  if (dh.parts > w.dh_parts) return AXON_ERR_WORKSPACE;
   // blocks that share a weight-gradient GEMM keep their dlogits of the whole vocabulary side by side
   if ((pos > 0 || !blk.dw_now) && !(w.dl_kmajor && w.chunks == 1)) return AXON_ERR_ARG;
   StashWs sw{};
@@ -1377,7 +1395,6 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   }
   const int64_t n_red = round_up(n, 64);  // reduction length of B3 (from this block's first token)
   const int64_t tiles_h = round_up(h, kTile) / kTile;
-  const SplitPlan plan = split_plan(tiles_h * (n_tile / kTile), w.chunks > 1 ? w.chunk : v);
   __bf16* const dl = w.dl + pos * w.ld_c;  // this block's rows
 
   for (int ci = 0; ci < w.chunks; ++ci) {
@@ -1702,6 +1719,17 @@ extern "C" int64_t axon_lmhead_block_dw_acc_bytes(int64_t h, int64_t v) {
 extern "C" int axon_lmhead_bwd_dlogit_copies(int64_t h, int64_t v, int64_t chunk) {
   if (check_head_shape(0, h, v) != AXON_OK || chunk < 0 || chunk % kTile != 0) return -1;
   return bwd_ws(kTile, h, v, chunk > 0 ? chunk : kDefaultVocabChunk, nullptr).dl_kmajor ? 1 : 2;
+}
+
+extern "C" int64_t axon_lmhead_bwd_dhidden_parts(int64_t n, int64_t ws_tokens, int64_t h, int64_t v, int64_t chunk,
+                                                 int64_t* reserved) {
+  int rc = check_head_shape(n, h, v);
+  if (rc == AXON_OK) rc = check_head_shape(ws_tokens, h, v);
+  if (rc != AXON_OK) return rc;
+  if (!reserved || chunk < 0 || chunk % kTile != 0 || n > ws_tokens) return AXON_ERR_ARG;
+  const BwdWs w = bwd_ws(ws_tokens, h, v, chunk, nullptr);
+  *reserved = w.dh_parts;
+  return n > 0 ? dh_plan(w, n, h, v).parts : 0;
 }
 
 extern "C" int axon_lmhead_block_can_group(int64_t h, int64_t v, int64_t chunk) {

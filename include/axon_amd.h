@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define AXON_AMD_ABI_VERSION 21
+#define AXON_AMD_ABI_VERSION 22
 
 enum {
   AXON_OK = 0,
@@ -246,6 +246,11 @@ int axon_lmhead_block_can_group(int64_t hidden, int64_t vocab, int64_t vocab_chu
  * vocab-major (hidden < 256, vocab % 8 != 0, or a last vocabulary chunk of fewer than 256 rows).  vocab_chunk 0 is taken as 32768. For
  * byte accounting; negative for an unsupported shape.  No reference counterpart. */
 int axon_lmhead_bwd_dlogit_copies(int64_t hidden, int64_t vocab, int64_t vocab_chunk);
+/* How many 256 KB parts of fp32 partial sums the dHidden reduction of a backward over n_tokens keeps in a workspace
+ * of axon_lmhead_bwd_workspace_bytes(ws_tokens, ...), and in *reserved how many that workspace has room for: never
+ * fewer (a call would return AXON_ERR_WORKSPACE).  n_tokens <= ws_tokens; negative for an unsupported shape. */
+int64_t axon_lmhead_bwd_dhidden_parts(int64_t n_tokens, int64_t ws_tokens, int64_t hidden, int64_t vocab,
+                                      int64_t vocab_chunk, int64_t* reserved);
 int axon_scale_bf16_unless_one(void* x_bf16, int64_t n, const float* scale, void* stream);
 
 /* Plain bf16 NT GEMM on the same MFMA main loop, out[n][m] = sum_k A[m][k]*B[n][k]

@@ -888,6 +888,7 @@ def test_ragged_tile_edges_of_the_dma_loop_vs_oracle(n, h, v):
 @pytest.mark.parametrize("n,h,v,chunk", [
     (5, 64, 4096, 0), (70, 256, 4100, 0),            # the shortest vocabulary that is reduced in parts (64 k-tiles)
     (300, 256, 9001, 0), (513, 320, 20000, 0),       # a shorter last part, several tiles
+    (1, 64, 4033, 0), (5, 128, 4095, 0), (187, 1024, 30719, 0),  # the last k-tile of the last part is not a whole one
     (200, 256, 8192 + 136, 4096), (40, 128, 13000, 6144),  # chunks: the last one reaches the first parts only
 ])
 def test_split_reduction_of_d_hidden_vs_oracle(n, h, v, chunk):

@@ -311,6 +311,41 @@ def test_which_shapes_write_the_dlogits_once_and_may_group_blocks():
     assert group(256, 2048, 0) == 1 and group(128, 2048, 0) == 0 and group(256, 2044, 0) == 0
 
 
+def test_split_reduction_of_d_hidden_fits_its_workspace():
+    """The parts that the dHidden plan writes against the room the workspace reserves for them (host arithmetic, no GPU
+    call): vocabularies around every multiple of 2048 (32 k-tiles of 64, the shortest part), whole and in chunks,
+    several hidden sizes, and blocks shorter than the ones the workspace was sized for."""
+    import ctypes
+
+    from axon_amd import _lib
+    lib = _lib.load()
+    parts_of, room = lib.axon_lmhead_bwd_dhidden_parts, ctypes.c_int64()
+    seen_split = 0
+
+    def check(n, ws_n, h, v, chunk):
+        nonlocal seen_split
+        parts = parts_of(n, ws_n, h, v, chunk, ctypes.byref(room))
+        assert 0 <= parts <= room.value, (n, ws_n, h, v, chunk, parts, room.value)
+        assert room.value * 262144 <= lib.axon_lmhead_bwd_workspace_bytes(ws_n, h, v, chunk)
+        seen_split += parts > 0
+
+    for j in range(1, 67):
+        for v in (2048 * j - 64, 2048 * j - 63, 2048 * j - 17, 2048 * j - 1, 2048 * j, 2048 * j + 1):
+            for h in (64, 896, 4096):
+                for n in (1, 187, 700, 3001):
+                    check(n, n, h, v, 0)
+                check(300, 8192, h, v, 0)
+                check(300, 8192, h, v, 4096)
+                check(1, 513, h, v, (v + 255) // 256 * 256)
+    for v in (50257, 128264, 151936, 201088, 262143):
+        for n in (1, 255, 257, 2048, 6007, 8192, 16381, 32768, 40000):
+            for chunk in (0, 6144, 32768, (v + 255) // 256 * 256):
+                check(n, n, 2880, v, chunk)
+                check(n, 40000, 2880, v, chunk)
+    assert seen_split > 1000
+    assert parts_of(2, 1, 64, 4096, 0, ctypes.byref(room)) < 0 and parts_of(1, 1, 64, 4096, 100, ctypes.byref(room)) < 0
+
+
 def test_blocks_that_share_a_weight_gradient_gemm_are_placed_on_tile_borders():
     from axon_amd._ops import head_block_groups
     four = [(0, 8192), (8192, 16384), (16384, 24576), (24576, 32768)]
