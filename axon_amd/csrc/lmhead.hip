@@ -1002,8 +1002,14 @@ using SlowLoop = RegLoop<32>;
 
 // Leading dimensions whose byte offsets inside a tile (256 rows K-contiguous, 64 K-major) stay below 2^30
 constexpr int64_t kMaxLd = 1 << 21, kMaxLdKMajor = 1 << 23;
+// A K-contiguous operand of the DMA loop: 16-byte vectors, and rows at least a k-tile apart (the descriptor's end and
+// the scalar offsets of its instructions are multiples of the row stride; rows closer than that, an expanded or an
+// overlapping view, go through registers).
+inline bool kcontig_ok(const void* p, int64_t ld) {
+  return ld >= DmaLoop::kBK && ld < kMaxLd && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+}
 inline bool dma_ok(const GemmOperands& g) {
-  return (g.k % DmaLoop::kBK) == 0 && g.lda < kMaxLd && g.ldb < kMaxLd;
+  return (g.k % DmaLoop::kBK) == 0 && kcontig_ok(g.a, g.lda) && kcontig_ok(g.b, g.ldb);
 }
 
 template <typename K>
@@ -1246,7 +1252,8 @@ int launch_store_kmajor(const GemmOperands& g, const StoreParams& sp, bool a_kma
                         hipStream_t st) {
   if (!a_kmajor && !b_kmajor) return launch_store(g, sp, st);
   if (b_kmajor && (g.ldb < kTile || (a_kmajor && g.lda < kTile))) return AXON_ERR_SHAPE;
-  if (!(a_kmajor ? kmajor_ok(g.a, g.lda) : g.lda < kMaxLd) || !(b_kmajor ? kmajor_ok(g.b, g.ldb) : g.ldb < kMaxLd))
+  if (!(a_kmajor ? kmajor_ok(g.a, g.lda) : kcontig_ok(g.a, g.lda)) ||
+      !(b_kmajor ? kmajor_ok(g.b, g.ldb) : kcontig_ok(g.b, g.ldb)))
     return AXON_ERR_SHAPE;
   if (a_kmajor && b_kmajor) return launch_store_loop<DmaLoopT<true, true>>(g, sp, st);
   if (a_kmajor && g.lda < kTile) return launch_store_loop<DmaLoopT<true, false, true>>(g, sp, st);

@@ -265,7 +265,8 @@ int axon_gemm_nt_bf16(const void* a_bf16, int64_t lda, const void* b_bf16, int64
  * A K-major operand is read as it lies (no transposed copy) through the LDS transpose read of gfx950.
  * No reference counterpart (test and benchmark helper, like the above).  K-major operands only on the
  * DMA main loop: m, n >= 256, k % 64 == 0, and for a K-major operand a 16-byte aligned base and a row
- * count and leading dimension that are multiples of 8; AXON_ERR_SHAPE otherwise. */
+ * count and leading dimension that are multiples of 8, and a K-contiguous operand beside it on a 16-byte boundary
+ * with rows at least 64 elements apart; AXON_ERR_SHAPE otherwise. */
 int axon_gemm_bf16(const void* a_bf16, int64_t lda, int a_kmajor, const void* b_bf16, int64_t ldb,
                    int b_kmajor, float* out, int64_t ldo, int64_t m, int64_t n, int64_t k, void* stream);
 

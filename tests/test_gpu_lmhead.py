@@ -49,6 +49,23 @@ def test_gemm_nt_vs_fp32_matmul(m, n, k):
     assert out.shape == (n, m) and rel_l2(out, ref) < 1e-5
 
 
+@pytest.mark.parametrize("m,n", [(100, 77), (300, 260)])
+def test_gemm_nt_on_views_whose_rows_lie_closer_than_a_k_tile(m, n):
+    """One row for all (stride 0), overlapping windows (stride 8 of 64) and a base off the 16-byte boundary: what the
+    register loop takes and the descriptors of the DMA loop cannot describe."""
+    g = torch.Generator().manual_seed(m)
+    k = 64
+    base = torch.randn(m * 8 + n * 8 + 2 * k, generator=g).bfloat16().to(DEV)
+    whole = torch.randn(n, k, generator=g).bfloat16().to(DEV)
+    for a in (base[:k].expand(m, k), base.as_strided((m, k), (8, 1)), base[4:].as_strided((m, k), (8, 1), 4)):
+        for b in (whole, base.as_strided((n, k), (8, 1), 8)):
+            ref = b.cpu().float() @ a.cpu().float().t()
+            assert rel_l2(_ops.gemm_nt(a, b), ref) < 1e-5
+    off = torch.randn(m * k + 4, generator=g).bfloat16().to(DEV)[4:].view(m, k)  # 8 bytes off
+    assert off.data_ptr() % 16 == 8
+    assert rel_l2(_ops.gemm_nt(off, whole), whole.cpu().float() @ off.cpu().float().t()) < 1e-5
+
+
 def _stored(x, kmajor, pad):
     """The logical [rows][k] matrix `x` as the GEMM takes it: row-major, or K-major ([k][rows]), either with
     `pad` unused elements at the end of every stored row."""
