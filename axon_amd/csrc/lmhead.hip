@@ -1278,7 +1278,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
              int64_t h, int64_t v, float inv_temp, float softcap, const uint8_t* is_start,
              int64_t last_dst, float* logprobs, float* entropy, float* lse, float* entropy_b,
              void* workspace, int64_t ws_bytes, void* stash, int64_t stash_bytes, void* stream,
-             PhaseTimer* timer) {
+             PhaseTimer* timer, bool is_block = false) {
   int rc = check_head_shape(n, h, v);
   if (rc != AXON_OK) return rc;
   if (n == 0) return AXON_OK;
@@ -1294,6 +1294,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
   StashWs sw{};
   if (stash) {
     if (reinterpret_cast<uintptr_t>(stash) & 15) return AXON_ERR_ARG;
+    if (!is_block && !stash_of_all_tokens(n, h, v)) return AXON_ERR_SHAPE;
     sw = stash_ws(n, v, stash);
     if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
     w.pm = sw.pm;  // the backward needs the per-part maxima: they live in the stash
@@ -1340,6 +1341,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
 // gradient leaves: the blocks of a step add up in one fp32 array, the last one rounds the sum to bf16.
 enum { kDwStore = 0, kDwFirst = 1, kDwAdd = 2, kDwLast = 3 };
 struct BlockArgs {
+  bool is_block = false;  // a stash for any shape, as the caller decides; else the shapes of stash_of_all_tokens
   int64_t last_dst = 0;
   int dw_mode = kDwStore;
   float* dw_acc = nullptr;  // axon_lmhead_block_dw_acc_bytes of fp32 partial sums, tile order (modes other than kDwStore)
@@ -1390,6 +1392,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   StashWs sw{};
   if (stash) {
     if (reinterpret_cast<uintptr_t>(stash) & 15) return AXON_ERR_ARG;
+    if (!blk.is_block && !stash_of_all_tokens(n, h, v)) return AXON_ERR_SHAPE;
     sw = stash_ws(n, v, const_cast<void*>(stash));
     if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
   }
@@ -1766,7 +1769,7 @@ extern "C" int axon_lmhead_block_fwd(const void* hidden, const void* weight, con
   PhaseTimer* t = block_timer(timer, stream, 0, &rc);
   if (rc != AXON_OK) return rc;
   return fwd_impl(hidden, weight, labels, labels_i64, n, h, v, inv_temp, softcap, seq_start, last_dst,
-                  logprobs, entropy, lse, entropy_b, workspace, ws_bytes, stash, stash_bytes, stream, t);
+                  logprobs, entropy, lse, entropy_b, workspace, ws_bytes, stash, stash_bytes, stream, t, true);
 }
 
 extern "C" int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentropy, const void* hidden,
@@ -1784,6 +1787,7 @@ extern "C" int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentro
   PhaseTimer* t = block_timer(timer, stream, 4, &rc);
   if (rc != AXON_OK) return rc;
   BlockArgs blk;
+  blk.is_block = true;
   blk.last_dst = last_dst;
   blk.dw_mode = dw_mode;
   blk.dw_acc = dw_acc;

@@ -42,8 +42,8 @@ def test_workspace_queries_and_argument_errors_without_gpu():
     assert lib.axon_lmhead_fwd_workspace_bytes(16, 100, 50) == -1  # hidden % 32 != 0
     assert lib.axon_lmhead_bwd_workspace_bytes(64, 128, 1000, 100) == -1  # chunk % 256 != 0
     assert lib.axon_lmhead_bwd_workspace_bytes(64, 128, 1000, 256) > 0
-    # the forward's optional stash: 128 KB per 256 x 256 tile + the per-part maxima; 0 where shifted edge tiles
-    # could not hand rows over in fours; -1 for an invalid shape
+    # the forward's optional stash: 128 KB per 256 x 256 tile + the per-part maxima; 0 for large shapes whose tokens or
+    # vocabulary are no multiple of four (their backward recomputes in fp32); -1 for an invalid shape
     assert lib.axon_lmhead_stash_bytes(32768, 4096, 151936) == 594 * 128 * 131072 + 594 * 2 * 32768 * 4
     assert lib.axon_lmhead_stash_bytes(513, 256, 1500) == 0 and lib.axon_lmhead_stash_bytes(516, 256, 1502) == 0
     assert lib.axon_lmhead_stash_bytes(513, 96, 1501) == 3 * 6 * 131072 + 256 * ((6 * 2 * 513 * 4 + 255) // 256)
@@ -54,6 +54,17 @@ def test_workspace_queries_and_argument_errors_without_gpu():
                                 3.0, None, None, None, None) == -1
     assert lib.axon_reduce_partials_bytes(4097) == lib.axon_reduce_partials_bytes(1 << 30) == 16384 * 32 + 256 * 32 + 2048 and lib.axon_reduce_partials_bytes(-1) == -1
     assert lib.axon_fill_zero(None, 3, None) == -1
+
+
+def test_whole_call_head_refuses_a_stash_for_shapes_it_keeps_none_for():
+    """axon_lmhead_stash_bytes is 0 for these: a caller that hands a buffer over all the same gets AXON_ERR_SHAPE
+    before anything is launched (the addresses below are never read)."""
+    lib = _lib.load()
+    assert lib.axon_lmhead_stash_bytes(513, 256, 1500) == 0 < lib.axon_lmhead_block_stash_bytes(513, 256, 1500)
+    p, big = 1 << 20, 1 << 40
+    shape = (513, 256, 1500, 1.0, 0.0)
+    assert lib.axon_lmhead_fwd(p, p, p, 0, *shape, None, p, p, p, p, p, big, p, big, None) == -2
+    assert lib.axon_lmhead_bwd(p, None, p, p, p, 0, p, p, *shape, None, p, p, 0, p, big, p, big, None) == -2
 
 
 def test_cpu_tensors_fail_loudly():
