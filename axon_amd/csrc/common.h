@@ -257,13 +257,14 @@ __device__ __forceinline__ void grid_finish(float (&v)[NV], float* lds /* [8 * 4
 
 // Workgroups of a streaming launch: beyond this many chunks a workgroup walks several (every
 // workgroup publishes a row of partial sums and takes a ticket when it ends, which costs more than
-// the walk; 6144 measured best between 1024 and 16384 at 2^26 tokens; up to 2^24 tokens 1024, whose sums are
-// finished in one level: 8.4 M tokens 44.0 us against 46.3 with 2048).
+// the walk; 6144 measured best between 1024 and 16384 at 2^26 tokens).  Below it every chunk has its own
+// workgroup, so that a thread's fp32 sums are at most kVec * kIter slots long: walking several with 1024
+// workgroups, whose sums are finished in one level, is 5 % faster at 8.4 M tokens (44.0 us for 46.3) and doubles
+// the rounding of the sums.
 constexpr int kStreamGridCap = 6144;
 inline unsigned stream_grid(int64_t n_slots, int64_t chunk = kChunk) {
   const int64_t chunks = (n_slots + chunk - 1) / chunk;
-  if (chunks > 4 * (int64_t)kOneLevelGrid) return (unsigned)(chunks < kStreamGridCap ? chunks : kStreamGridCap);
-  return (unsigned)(chunks < kOneLevelGrid ? chunks : kOneLevelGrid);
+  return (unsigned)(chunks < kStreamGridCap ? chunks : kStreamGridCap);
 }
 
 // 16-byte streaming accesses.  Every input of these kernels is read once and every output

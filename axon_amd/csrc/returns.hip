@@ -210,8 +210,9 @@ __global__ __launch_bounds__(kBlock) void reverse_scan_kernel(
 // stats[0] mean, [1] n, [2] variance (times n/(n-1) when n > 1), [3] rsqrt(variance + 1e-8)
 
 // Every workgroup that needs a pass's result adds the pass's at most kMomentBlocks partials itself, in the same fixed
-// order (32 KB out of L2), where a launch of one workgroup in between cost 3.6 us and the gaps around it.
-constexpr int kMomentBlocks = 1024;
+// order (64 KB out of L2), where a launch of one workgroup in between cost 3.6 us and the gaps around it.  Half as many
+// workgroups would double the length of every thread's fp32 sums.
+constexpr int kMomentBlocks = 2048;
 
 __device__ __forceinline__ void add_partials(const float* __restrict__ partials, int n_blocks, float (&a)[2], float* lds_red) {
   float2 v[kMomentBlocks / kBlock];
@@ -458,7 +459,7 @@ int launch_scan(int mode, const float* rewards, const float* values, const void*
 
 unsigned moments_grid(int64_t n_slots) {
   const int64_t blocks = (n_slots / kVec + kBlock - 1) / kBlock;
-  const int64_t cap = kMomentBlocks;  // four workgroups per compute unit walk the tokens
+  const int64_t cap = kMomentBlocks;  // eight workgroups per compute unit walk the tokens
   return (unsigned)(blocks < 1 ? 1 : (blocks < cap ? blocks : cap));
 }
 

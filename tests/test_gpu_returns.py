@@ -193,7 +193,8 @@ def test_masked_whiten_gpu():
     assert out.shape == (5, 7) and abs(out.mean().item()) < 1e-5
 
 
-@pytest.mark.parametrize("n", [1, 1021, 1024 * 1024, 1024 * 1024 + 1027, 3 * 1024 * 1024 + 1])
+@pytest.mark.parametrize("n", [1, 1021, 1024 * 1024, 1024 * 1024 + 1027, 2 * 1024 * 1024, 2 * 1024 * 1024 + 1027,
+                               3 * 1024 * 1024 + 1, 5 * 1024 * 1024 + 1])
 def test_masked_whiten_statistics_at_the_edges_of_the_grid(n):
     """One workgroup, as many as the launch has, and several trips of each, against float64; the statistics alone and
     beside the output come out the same.  Sums of n positive terms in trees of at most 64 in a row: n-independent
@@ -213,6 +214,15 @@ def test_masked_whiten_statistics_at_the_edges_of_the_grid(n):
     assert torch.allclose(stats.double(), ref, rtol=1e-5, atol=1e-7 if n == 1 else 0)
     if n > 1:
         assert rel_l2(out, (xd - mean) * ref[3]) < 1e-5
+
+
+def test_masked_whiten_sums_at_most_sixteen_slots_per_thread_at_2_23():
+    """2^23 equal values: the partial sums of all threads are equal and every tree step doubles them exactly, so that
+    the mean is off by what a thread's own run of additions rounds.  0.1 added 16 times is 1.5e-7 too large, 32 times
+    3.0e-7 too small (fp32 additions, counted by hand)."""
+    x = torch.full((1 << 23,), 0.1, device=DEV)
+    _, stats = _ops.masked_whiten(x, torch.ones_like(x), stats_only=True)
+    assert abs(stats[0].item() / x[0].item() - 1) < 2e-7
 
 
 @pytest.mark.parametrize("n_rows,mode", [(8192, 1), (8193, 2), (17001, 1), (8200, 3)])

@@ -1215,3 +1215,19 @@ def test_launch_shapes_of_the_streaming_loss(n):
     ent, w, _ = _ops.side_terms(lp, None, None, mask, rows, token_reduce="sum", batch_reduce="token-mean")
     assert torch.equal(w, mask) and (ent[0].double() - (lp.double() * mask).sum() / mask.sum().double()).abs() <= (
         2.0 ** -24 * 32 * (lp.double().abs() * mask).sum() / mask.sum() + 1e-12)
+
+
+@pytest.mark.parametrize("chunks", [1025, 2048, 4096])
+def test_a_threads_run_in_the_streaming_losses_stays_at_sixteen_slots(chunks):
+    """Equal products: all threads' partial sums are equal, the trees double them (and add the four wavefronts and up
+    to 256 rows of equal sums, below 1e-7), so that the loss is off by what a thread's own run of additions rounds:
+    0.1 added 16 times in fp32 is 1.5e-7 too large, 32 times 3.0e-7 and 64 times 6.0e-7 too small."""
+    n = chunks * 4096
+    lp = torch.full((1, n), 0.1, device=DEV)
+    one = torch.ones_like(lp)
+    rows = _ops.rows_of(lp)
+    acc, _ = _ops.policy_loss(2, lp, lp, one, one, None, rows, token_reduce="sum", batch_reduce="token-mean",
+                              ratio_lo=0.8, ratio_hi=1.2, clip_c=3.0)
+    assert abs(-acc[0].item() / lp[0, 0].item() - 1) < 2.5e-7 and acc[4].item() == n
+    ent, _, _ = _ops.side_terms(lp, None, None, one, rows, token_reduce="sum", batch_reduce="token-mean")
+    assert abs(ent[0].item() / lp[0, 0].item() - 1) < 2.5e-7
