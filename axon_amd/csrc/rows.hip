@@ -233,43 +233,92 @@ __global__ __launch_bounds__(1024) void group_stats_kernel(
 
 // Row sums and, in the workgroup that ends last, the group statistics and the per-row scalar of the group-based
 // estimators: with row_broadcast_kernel behind it an advantage is two launches, no zero fills and no float atomics
-// in memory.  A wavefront owns a row (double accumulators per lane, then a fixed tree), four 16-byte loads in flight;
+// in memory.  A wavefront owns a row (double accumulators per lane, then a fixed tree; a workgroup a very long one), four 16-byte loads in flight;
 // the grid is bounded so that its tickets stay cheap.  The groups' sums are formed in LDS (double, so that the order
 // in which the rows arrive does not show in the fp32 results).
 // 128 x 1024 slots, 16 groups: 7.5 us where fill, row pass, finish and group kernel took 6.9 + 1.3 + 10.9 and two fills;
 // 8.4 M slots in 9000 rows, 1150 groups: 33 for 27 + 4.7 + 80 (40 with one row after the other in the last workgroup).
 constexpr int kScoreGroups = 2048;  // 40 KB of LDS
 constexpr int kScoreBlocks = 512;  // what fits the part at once: a wavefront with a short row takes another one
+// A row of more than kLongRow slots is summed by the whole workgroup of the wavefront that meets it (on its first 64
+// trips): a wavefront needs 0.5 us per 1024 slots, which a packed batch, of which the host knows the mean length only,
+// pays for its longest row alone.  Whole operator, 9000 rows of 500 slots and one of 2^20: 110 us, 593 with a wavefront per row
+// and 221 with the separate kernels; one of 65536: 42, 68 and 179.  Workgroups of many long rows take one after the other, so that
+// the line lies where half the rows of the longest mean length that comes here can be beyond it: from 8192 on, 512 rows
+// of 16384 took 48 us for 34.
+constexpr int kScoreThreads = 1024, kLongRow = 32768;
 
-__global__ __launch_bounds__(1024) void group_scores_kernel(
+__global__ __launch_bounds__(kScoreThreads) void group_scores_kernel(
     const float* __restrict__ a, const int32_t* __restrict__ cu, int64_t n_rows, int64_t n_slots, int64_t uniform_len,
     const int64_t* __restrict__ gidx, GroupCfg g, float* scores, float* __restrict__ scalar, unsigned* ticket) {
   __shared__ double sums[kScoreGroups][2];
   __shared__ int count[kScoreGroups];
   __shared__ int last, nonzero;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
-  for (int64_t r = (int64_t)blockIdx.x * waves + wave; r < n_rows; r += (int64_t)gridDim.x * waves) {
-    int64_t t0 = uniform_len > 0 ? r * uniform_len : (int64_t)cu[r];
-    int64_t t1 = uniform_len > 0 ? t0 + uniform_len : (int64_t)cu[r + 1];
+  constexpr int kWaves = kScoreThreads / kWave;
+  __shared__ double part[kWaves];
+  __shared__ uint64_t long_trips[kWaves];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  auto span = [&](int64_t r, int64_t& t0, int64_t& t1) {
+    t0 = uniform_len > 0 ? r * uniform_len : (int64_t)cu[r];
+    t1 = uniform_len > 0 ? t0 + uniform_len : (int64_t)cu[r + 1];
     t0 = min(max(t0, (int64_t)0), n_slots);
     t1 = min(max(t1, t0), n_slots);
+  };
+  // this thread's share of a row that `n` threads add up, `id` of them: whole vectors, and the row's edges
+  auto share = [&](int64_t t0, int64_t t1, int id, auto n_c) -> double {
+    constexpr int n = decltype(n_c)::value;
     double acc = 0.0;
     const int64_t b0 = min((t0 + 3) & ~(int64_t)3, t1), b1 = max(t1 & ~(int64_t)3, b0);  // whole vectors
-    // the row's edges and its first four vectors per lane are on their way before anything is added
-    const float e0 = lane < b0 - t0 ? a[t0 + lane] : 0.f, e1 = lane < t1 - b1 ? a[b1 + lane] : 0.f;
-    for (int64_t p = b0 + lane * kVec; p < b1; p += 4 * kWave * kVec) {
+    // the row's edges and its first four vectors per thread are on their way before anything is added
+    const float e0 = id < b0 - t0 ? a[t0 + id] : 0.f, e1 = id < t1 - b1 ? a[b1 + id] : 0.f;
+    for (int64_t p = b0 + id * kVec; p < b1; p += 4 * n * kVec) {
       float v[4][4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) load4(a, min(p + u * kWave * kVec, b1 - kVec), v[u]);  // a valid vector; dropped below
+      for (int u = 0; u < 4; ++u) load4(a, min(p + u * n * kVec, b1 - kVec), v[u]);  // a valid vector; dropped below
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const double x = ((double)v[u][0] + (double)v[u][1]) + ((double)v[u][2] + (double)v[u][3]);
-        acc += p + u * kWave * kVec < b1 ? x : 0.0;
+        acc += p + u * n * kVec < b1 ? x : 0.0;
       }
     }
-    acc += (double)e0 + (double)e1;
-    acc = wave_sum_d(acc);
-    if (lane == 0) __hip_atomic_store(scores + r, (float)acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return acc + ((double)e0 + (double)e1);
+  };
+  auto put = [&](int64_t r, double v) {
+    __hip_atomic_store(scores + r, (float)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto row_of = [&](int trip, int w) { return ((int64_t)trip * gridDim.x + blockIdx.x) * kWaves + w; };
+  uint64_t longs = 0;  // this wavefront's trips whose row is left to the whole workgroup
+  for (int trip = 0;; ++trip) {
+    const int64_t r = row_of(trip, wave);
+    if (r >= n_rows) break;
+    int64_t t0, t1;
+    span(r, t0, t1);
+    if (t1 - t0 > kLongRow && trip < 64) {
+      longs |= 1ull << trip;
+      continue;
+    }
+    const double acc = wave_sum_d(share(t0, t1, lane, std::integral_constant<int, kWave>{}));
+    if (lane == 0) put(r, acc);
+  }
+  if (lane == 0) long_trips[wave] = longs;
+  __syncthreads();
+  // the same rows for every thread of the workgroup
+  for (uint64_t with = __ballot(lane < kWaves && long_trips[lane % kWaves] != 0); with != 0; with &= with - 1) {
+    const int w = __builtin_ctzll(with);
+    for (uint64_t m = long_trips[w]; m != 0; m &= m - 1) {
+      const int64_t r = row_of(__builtin_ctzll(m), w);
+      int64_t t0, t1;
+      span(r, t0, t1);
+      const double acc = wave_sum_d(share(t0, t1, (int)threadIdx.x, std::integral_constant<int, kScoreThreads>{}));
+      if (lane == 0) part[wave] = acc;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        double sum = 0.0;
+        for (int u = 0; u < kWaves; ++u) sum += part[u];
+        put(r, sum);
+      }
+      __syncthreads();
+    }
   }
   // the scores' write-through stores are acknowledged before the workgroup draws its ticket (publish_row_take_ticket)
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -549,9 +598,9 @@ extern "C" int axon_group_advantage(const float* rewards, const void* mask, int 
   if (n_groups <= 0 || n_groups > kScoreGroups) return AXON_ERR_SHAPE;
   if (!rewards || !gidx || !row_scratch || !out || !partials || mode < 0 || mode > 3) return AXON_ERR_ARG;
   if (reinterpret_cast<uintptr_t>(rewards) & 15) return AXON_ERR_ARG;
-  constexpr int kWaves = 1024 / kWave;
+  constexpr int kWaves = kScoreThreads / kWave;
   const int64_t blocks = (n_rows + kWaves - 1) / kWaves;
-  hipLaunchKernelGGL(group_scores_kernel, dim3((unsigned)(blocks < kScoreBlocks ? blocks : kScoreBlocks)), dim3(1024), 0,
+  hipLaunchKernelGGL(group_scores_kernel, dim3((unsigned)(blocks < kScoreBlocks ? blocks : kScoreBlocks)), dim3(kScoreThreads), 0,
                      (hipStream_t)stream, rewards, cu, n_rows, n_slots, uniform_len, gidx,
                      GroupCfg{n_groups, eps, mode}, row_scratch, row_scratch + n_rows,
                      reinterpret_cast<unsigned*>(partials + kTicketsOffset));

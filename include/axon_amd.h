@@ -321,8 +321,8 @@ int axon_row_broadcast_mask(const float* row_scalar, const void* mask, int mask_
 
 /* The group-based advantage in two launches: score[r] = sum of the row's rewards, the group statistics and the scalar
  * of axon_group_stats (mode = its norm_by_std, 0..3), broadcast over the mask (axon_row_broadcast_mask).
- * n_groups <= 2048 (AXON_ERR_SHAPE beyond: use the separate entry points); a wavefront sums a row, so batches of
- * very long or very short rows are better served by axon_row_stats.  row_scratch: 2 * n_rows floats (scores, then
+ * n_groups <= 2048 (AXON_ERR_SHAPE beyond: use the separate entry points); a wavefront sums a row of up to
+ * 32768 slots, a workgroup a longer one, so batches of rows that are long or very short on average are better served by axon_row_stats.  row_scratch: 2 * n_rows floats (scores, then
  * scalars); partials: axon_reduce_partials_bytes, ticket counters zero (they are left zero).  rewards on a
  * 16-byte boundary. */
 int axon_group_advantage(const float* rewards, const void* mask, int mask_kind, const int32_t* cu_seqlens,

@@ -1193,6 +1193,35 @@ def test_group_advantage_in_two_launches_vs_oracle(name, rows, t, group):
         assert torch.equal(again, out)
 
 
+@pytest.mark.parametrize("lens,group", [
+    ([32768, 32769, 5, 0, 32771, 700, 64], 2),            # the longest row of a wavefront, the shortest of a workgroup
+    ([300] * 20 + [100003] + [301] * 20 + [65536, 32767], 4),  # several in one workgroup, off 16-byte boundaries
+    ([100] * 9000 + [40001] + [100] * 20, 8),             # met on a second trip
+    ([33001, 2, 3] * 20, 5),                              # eight or so in every workgroup
+])
+def test_group_advantage_with_rows_that_a_whole_workgroup_sums(lens, group):
+    """Packed rows of more than 32768 slots beside short ones, against float64, and the same bits on every run."""
+    n = sum(lens)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    r = torch.randn(n, generator=g, device=DEV)
+    cu = torch.tensor([0] + lens).cumsum(0)
+    rows = _ops.rows_of(r, cu.int().to(DEV))
+    gidx = torch.arange(len(lens), device=DEV) // group
+    n_groups = int(gidx[-1]) + 1
+    ones = torch.ones_like(r)
+    adv = _ops.group_advantage(r, ones, gidx, n_groups, rows, eps=1e-6, mode=0)
+    assert torch.equal(_ops.group_advantage(r, ones, gidx, n_groups, rows, eps=1e-6, mode=0), adv)
+    score = torch.stack([x.double().sum() for x in r.split(lens)]).float().double()
+    count = torch.bincount(gidx, minlength=n_groups)
+    mean = torch.zeros(n_groups, device=DEV, dtype=torch.float64).index_add_(0, gidx, score) / count
+    want = torch.where(count[gidx] > 1, score - mean[gidx], 0.0)
+    # sums in double; score and mean round to fp32 (2^-24 of their size) and so does their difference
+    bound = 2.0 ** -23 * (score.abs() + mean[gidx].abs()) + 1e-12
+    got = torch.stack([x[0] if len(x) else x.new_zeros(()) for x in adv.split(lens)]).double()
+    has = torch.tensor([l > 0 for l in lens], device=DEV)
+    assert ((got - want).abs() <= bound)[has].all()
+
+
 @pytest.mark.parametrize("n", [5, 1024, 1025, 262144, 262145, 524288, 524293, 4 * 1024 * 1024, 4 * 1024 * 1024 + 4097,
                                16 * 1024 * 1024 + 3])
 def test_launch_shapes_of_the_streaming_loss(n):
