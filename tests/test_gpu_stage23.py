@@ -1169,8 +1169,8 @@ def test_all_padding_micro_batch_is_a_no_op_before_any_validation():
     (17, 4096, 5), (1030, 64, 4), (4100, 64, 2), (4096, 65, 2), (5000, 64, 2),  # 2050 and 2500 groups: the separate kernels
 ])
 def test_group_advantage_in_two_launches_vs_oracle(name, rows, t, group):
-    """Row sums with the group statistics in the last workgroup, against the oracle, padded and packed, and the same
-    bits on every run."""
+    """Row sums with the group statistics in the last workgroup, against the oracle, padded and packed; the same bits
+    on every run, since these scores' sums are exact in any order."""
     g = torch.Generator().manual_seed(rows + t)
     rew = torch.zeros(rows, t)
     # Scores are integers up to 7: their sums and squares are exact in fp32, so the two sides differ by the rounding of
@@ -1191,6 +1191,25 @@ def test_group_advantage_in_two_launches_vs_oracle(name, rows, t, group):
     if len(np.unique(uid)) <= 2048:
         again = compute_advantage(_grpo_proto(rew, mask, uid), {"advantage": name}).batch["advantages"]
         assert torch.equal(again, out)
+
+
+@pytest.mark.parametrize("offset,spread", [(0.0, 1.0), (1000.0, 0.5), (-300.0, 0.1)])
+def test_group_statistics_of_continuous_scores_with_a_common_offset(offset, spread):
+    """Scores far from zero beside their deviation, where sums of squares in fp32 lose the variance, against float64
+    (offset / spread under 5000: the double sums cost less than the fp32 results' own rounding)."""
+    n_rows, t, group = 512, 70, 8
+    g = torch.Generator(device=DEV).manual_seed(5)
+    r = torch.zeros(n_rows, t, device=DEV)
+    r[:, 13] = offset + spread * torch.randn(n_rows, generator=g, device=DEV)
+    gidx = torch.arange(n_rows, device=DEV) // group
+    adv = _ops.group_advantage(r, torch.ones_like(r), gidx, n_rows // group, _ops.rows_of(r), eps=1e-6, mode=1)
+    x = r[:, 13].double().view(-1, group)
+    mean, sd = x.mean(1, keepdim=True), x.std(1, keepdim=True).clamp_min(1e-3)
+    want = (x - mean) / (sd + 1e-6)
+    # the mean leaves double rounded to fp32 (2^-24 of it, over the deviation); variance, root, sum and quotient: five
+    # roundings, and the double sums at most one more
+    bound = 2.0 ** -24 * mean.abs() / sd + 6 * 2.0 ** -24 * want.abs()
+    assert ((adv[:, 0].double().view(-1, group) - want).abs() <= bound).all()
 
 
 @pytest.mark.parametrize("lens,group", [
