@@ -27,7 +27,10 @@
 //      tile beyond the matrix (and k-rows of a K-major operand beyond its last one)
 //      read as zeros: the buffer descriptor of each operand ends with the tile's last
 //      valid row, and a load beyond it lands as 0 in LDS without touching memory
-//      (uniform addressing, no per-lane clamps, and no smallest matrix).
+//      (uniform addressing, no per-lane clamps, and no smallest matrix).  A load's scalar
+//      offset counts towards the bound, also where it alone lies beyond the end, as most
+//      instructions' of a tile with few valid rows do (checked with NaN behind the operands
+//      and on the accumulators of dropped rows).
 //      Shifting edge tiles back inside the matrix instead needed 256 rows on both
 //      sides (a forward over 187 tokens, 896 x 151936, ran on RegLoop: 355 us per call
 //      against 108 now) and token counts in fours for the head's stash (16381 tokens,

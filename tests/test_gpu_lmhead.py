@@ -80,7 +80,7 @@ def _stored(x, kmajor, pad):
                                    (4096, 1000, 192)])
 def test_gemm_with_k_major_operands_vs_fp32_matmul(m, n, k, a_kmajor, b_kmajor):
     """Operands stored [k][rows] are read as they lie (LDS transpose reads): same result as the NT form, on whole
-    tiles, on edge tiles shifted back by a multiple of 8 rows, with padded leading dimensions."""
+    tiles, on edge tiles that end with the buffer descriptor, with padded leading dimensions."""
     g = torch.Generator().manual_seed(3 * m + 5 * n + k)
     a = torch.randn(m, k, generator=g).bfloat16()
     b = torch.randn(n, k, generator=g).bfloat16()
@@ -882,8 +882,8 @@ def test_default_backward_has_no_readback_and_replays_in_a_hip_graph(from_stash)
     (515, 256, 1000),
 ])
 def test_ragged_tile_edges_of_the_dma_loop_vs_oracle(n, h, v):
-    """Rows beyond an operand's last one read as zeros (descriptor bounds): forward, recompute backward, and a block
-    of a step with its stash, at sizes where no dimension is a multiple of the tile."""
+    """Forward, recompute backward, and a block of a step with its stash, at sizes around and below the tile's.  (That
+    rows beyond an operand's last one come as zeros: the tests of operands inside larger ones below.)"""
     hid, w, lab = W.lmhead_inputs(n, h, v, seed=n + h + v)
     w = (w.float() * 8).bfloat16()
     hd, wd, ld = hid.to(DEV), w.to(DEV), lab.to(DEV)
@@ -921,3 +921,59 @@ def test_split_reduction_of_d_hidden_vs_oracle(n, h, v, chunk):
     assert torch.equal(dh, again[0]) and torch.equal(dw, again[1])  # the parts are added in a fixed order
     ref_dh, ref_dw = OM.backward(g_lp, None, hid, w, lab)
     assert rel_l2(dh, ref_dh) < 2e-2 and rel_l2(dw, ref_dw) < 2e-2
+
+
+def _leading_rows(x, extra=512):
+    """`x` as the first rows of a larger allocation whose other rows are NaN: what reads beyond x's last row stays inside
+    memory of this test's own, and shows."""
+    buf = torch.full((x.shape[0] + extra, x.shape[1]), float("nan"), dtype=x.dtype, device=DEV)
+    buf[: x.shape[0]] = x.to(DEV)
+    return buf[: x.shape[0]]
+
+
+@pytest.mark.parametrize("n,h,v", [
+    (1, 64, 65), (3, 128, 257), (1, 320, 1025), (257, 256, 1089),  # vocab % 64 == 1: the last k-tile holds one k-row
+    (130, 256, 1003), (70, 64, 1031), (511, 896, 1031), (33, 192, 4097), (300, 256, 8200),
+])
+def test_operands_are_not_read_beyond_their_last_row(n, h, v):
+    """dHidden contracts over the vocabulary with the weight K-major: the k-rows beyond its last one have to come as
+    zeros (the dlogits there are zeros too, but a zero times NaN is not).  Rows beyond the last token or vocabulary row
+    in the other products would show in the statistics or the gradients only if an epilogue let them through."""
+    hid, w, lab = W.lmhead_inputs(n, h, v, seed=n + h + v)
+    w = (w.float() * 8).bfloat16()
+    ld = lab.to(DEV)
+    g = torch.Generator().manual_seed(12)
+    g_lp, g_en = (torch.randn(n, generator=g) / n).to(DEV), (torch.randn(n, generator=g) / n).to(DEV)
+
+    def run(hd, wd):
+        lp, ent, lse, eb = _ops.lmhead_forward(hd, wd, ld, 1.0)
+        dh, dw = _ops.lmhead_backward(g_lp, g_en, hd, wd, ld, lse, eb, 1.0)
+        hb = _ops.HeadBlocks(hd, wd, ld, 1.0, [(0, n)])
+        hb.forward(0)
+        hb.backward(0, g_lp, g_en)
+        return lp, ent, lse, dh, dw, hb.logprobs, hb.d_hidden, hb.d_weight
+
+    plain = run(hid.to(DEV), w.to(DEV))
+    for a, b in zip(run(_leading_rows(hid), _leading_rows(w)), plain):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+def test_rows_of_an_edge_tile_beyond_the_operand_are_zeros_in_the_accumulators():
+    """The weight gradient's partial sums keep whole tiles, the rows that the epilogue drops among them.  hidden = 288
+    leaves 32 valid rows in the second tile, so that most of its load instructions start beyond the descriptor's
+    end by their scalar offset alone; what follows in the workspace are the dlogits, which are not zero."""
+    n, h, v = 512, 288, 1024
+    hid, w, lab = W.lmhead_inputs(n, h, v, seed=3)
+    hd, wd, ld = hid.to(DEV), (w.float() * 8).bfloat16().to(DEV), lab.to(DEV)
+    g_lp = torch.randn(n, generator=torch.Generator().manual_seed(4)).to(DEV)
+    hb = _ops.HeadBlocks(hd, wd, ld, 1.0, [(0, 256), (256, 512)], dw_group=1)
+    hb.forward(0)
+    hb.backward(0, g_lp, None)
+    # [tile_m, tile_n, wave_m, wave_n, block_m, block_n, lane / 16, lane % 16, m % 4] in the order of the registers
+    acc = hb.dw_acc.view(2, 4, 2, 2, 8, 8, 4, 16, 4)
+    m = acc.permute(0, 2, 4, 6, 8, 1, 3, 5, 7).reshape(512, 1024)  # m rows: hidden, padded to tiles; n: vocabulary
+    assert (m[288:] == 0).all() and (m[:288].abs().amax(1) > 0).all()
+    hb.forward(1)
+    hb.backward(1, g_lp, None)
+    ref_dh, ref_dw = OM.backward(g_lp.cpu(), None, hid, wd.cpu(), lab)
+    assert rel_l2(hb.d_weight, ref_dw) < 2e-2 and rel_l2(hb.d_hidden, ref_dh) < 2e-2
