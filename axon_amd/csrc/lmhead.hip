@@ -1141,6 +1141,9 @@ BwdWs bwd_ws(int64_t n, int64_t h, int64_t vocab, int64_t chunk, void* base) {
   }
   if (w.chunk > w.v_pad) w.chunk = w.v_pad;
   if (w.chunk > kMaxVocabChunk) w.chunk = kMaxVocabChunk;
+  // not so that a last chunk of less than a tile is left, which would need the second copy of the dlogits
+  if (chunk <= 0)
+    while (w.chunk > kDefaultVocabChunk && (vocab - 1) % w.chunk + 1 < kTile) w.chunk -= kTile;
   w.chunks = (int)((vocab + w.chunk - 1) / w.chunk);
   w.ld_n = w.n_pad + kLdPad;
   w.ld_c = w.chunk + kLdPad;
@@ -1173,6 +1176,18 @@ DhPlan dh_plan(const BwdWs& w, int64_t n, int64_t h, int64_t v) {
   const int64_t tiles = (round_up(h, kTile) / kTile) * (round_up(n, kTile) / kTile);
   const SplitPlan split = split_plan(tiles, w.chunks > 1 ? w.chunk : v);
   return DhPlan{split, (w.chunks > 1 || split.splits > 1) ? tiles * split.splits : 0};
+}
+
+// Bytes for a call over `n` tokens.  The default chunk shrinks in steps while n grows, so a shorter call can need a
+// little more: the most of any call over at most n tokens (beyond 32768 the chunk stays the same).
+int64_t bwd_ws_bytes(int64_t n, int64_t h, int64_t vocab, int64_t chunk) {
+  int64_t bytes = bwd_ws(n, h, vocab, chunk, nullptr).bytes;
+  if (chunk <= 0)
+    for (int64_t m = kTile; m < n && m <= kDefaultChunkElems / kDefaultVocabChunk; m += kTile) {
+      const int64_t b = bwd_ws(m, h, vocab, chunk, nullptr).bytes;
+      bytes = b > bytes ? b : bytes;
+    }
+  return bytes;
 }
 
 // Optional per-phase timing with HIP events on the launch stream (used by the *_timed entry points
@@ -1630,7 +1645,7 @@ extern "C" int64_t axon_lmhead_bwd_workspace_bytes(int64_t n, int64_t h, int64_t
                                                    int64_t chunk) {
   if (check_head_shape(n, h, v) != AXON_OK) return -1;
   if (chunk < 0 || chunk % kTile != 0) return -1;
-  return bwd_ws(n, h, v, chunk, nullptr).bytes + kAlign;
+  return bwd_ws_bytes(n, h, v, chunk) + kAlign;
 }
 
 extern "C" int axon_lmhead_bwd(const float* dlogprobs, const float* dentropy, const void* hidden,

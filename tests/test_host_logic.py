@@ -357,6 +357,23 @@ def test_split_reduction_of_d_hidden_fits_its_workspace():
     assert parts_of(2, 1, 64, 4096, 0, ctypes.byref(room)) < 0 and parts_of(1, 1, 64, 4096, 100, ctypes.byref(room)) < 0
 
 
+@pytest.mark.parametrize("h,v", [(896, 151936), (2880, 201088), (4096, 151936), (3072, 128264), (1024, 50257),
+                                 (2048, 102400), (256, 262144), (1024, 65800), (128, 40000), (512, 1310720)])
+def test_default_backward_workspace_grows_with_the_tokens_and_stays_bounded(h, v):
+    """A caller sizes the workspace once, for the longest batch: no shorter one may need more.  With hidden >= 256 and
+    vocab % 8 == 0 one copy of a chunk's dlogits is enough at every token count (host arithmetic, no GPU call)."""
+    from axon_amd import _lib
+    ws = _lib.load().axon_lmhead_bwd_workspace_bytes
+    need = [ws(n, h, v, 0) for n in range(0, 40000, 128)]
+    assert all(a <= b for a, b in zip(need, need[1:]))
+    copies = 1 if h >= 256 and v % 8 == 0 else 2
+    for n, b in zip(range(0, 40000, 128), need):
+        n_pad = (n + 255) // 256 * 256
+        elems = max(1 << 30, n_pad * 32768)
+        tiles = n_pad // 256 * ((h + 255) // 256)
+        assert b <= copies * 2 * (elems + 64 * max(n_pad, v + 255)) + 2 * h * (n_pad + 64) + max(768, tiles) * 262144 + 4096
+
+
 def test_blocks_that_share_a_weight_gradient_gemm_are_placed_on_tile_borders():
     from axon_amd._ops import head_block_groups
     four = [(0, 8192), (8192, 16384), (16384, 24576), (24576, 32768)]
