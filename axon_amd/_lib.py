@@ -44,6 +44,7 @@ SIGNATURES: dict[str, tuple] = {
                                      _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
     "axon_lmhead_block_can_group": (_i32, [_i64, _i64, _i64]),
     "axon_lmhead_bwd_dlogit_copies": (_i32, [_i64, _i64, _i64]),
+    "axon_lmhead_bwd_dlogit_copies_of": (_i32, [_i64, _i64, _i64, _i64]),
     "axon_lmhead_bwd_dhidden_parts": (_i64, [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
     "axon_scale_bf16_unless_one": (_i32, [_ptr, _i64, _ptr, _ptr]),
     "axon_lmhead_active_rows": (_i32, [_ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr]),

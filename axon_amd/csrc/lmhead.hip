@@ -1741,9 +1741,13 @@ extern "C" int64_t axon_lmhead_block_dw_acc_bytes(int64_t h, int64_t v) {
   return (round_up(h, kTile) / kTile) * (round_up(v, kTile) / kTile) * kTileAccVecs * 16;
 }
 
+extern "C" int axon_lmhead_bwd_dlogit_copies_of(int64_t n, int64_t h, int64_t v, int64_t chunk) {
+  if (check_head_shape(n, h, v) != AXON_OK || chunk < 0 || chunk % kTile != 0) return -1;
+  return bwd_ws(n, h, v, chunk, nullptr).dl_kmajor ? 1 : 2;
+}
+
 extern "C" int axon_lmhead_bwd_dlogit_copies(int64_t h, int64_t v, int64_t chunk) {
-  if (check_head_shape(0, h, v) != AXON_OK || chunk < 0 || chunk % kTile != 0) return -1;
-  return bwd_ws(kTile, h, v, chunk > 0 ? chunk : kDefaultVocabChunk, nullptr).dl_kmajor ? 1 : 2;
+  return axon_lmhead_bwd_dlogit_copies_of(kTile, h, v, chunk == 0 ? kDefaultVocabChunk : chunk);
 }
 
 extern "C" int64_t axon_lmhead_bwd_dhidden_parts(int64_t n, int64_t ws_tokens, int64_t h, int64_t v, int64_t chunk,

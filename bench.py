@@ -628,7 +628,7 @@ def kernel_table(timing, steps, n, h, v, stash_bytes, vocab_chunk=0):
     from axon_amd import _lib
 
     nhv = float(n) * h * v
-    copies = max(int(_lib.load().axon_lmhead_bwd_dlogit_copies(h, v, vocab_chunk)), 1)
+    copies = max(int(_lib.load().axon_lmhead_bwd_dlogit_copies_of(n, h, v, vocab_chunk)), 1)
     classes = [
         ("gemm_store_kernel (dHidden + dWeight GEMMs)", ("bwd/dhidden", "bwd/dweight"), 4 * nhv, 4 * nhv, 0.0),
         ("lmhead_fwd_stash_kernel (logits + online softmax statistics + stash)" if stash_bytes else

@@ -117,7 +117,7 @@ int axon_lmhead_fwd(const void* hidden_bf16, const void* weight_bf16, const void
  * (fused_linear.py:80-83).  dentropy may be NULL (treated as zeros).  vocab_chunk (multiple of 256, or 0
  * for the library default: as much of the vocabulary as keeps the bf16 dlogits of a chunk within 2 GiB, at least
  * 32768) bounds the bf16 dlogit scratch to n_tokens_padded * vocab_chunk * 2 bytes (twice that where
- * axon_lmhead_bwd_dlogit_copies says 2).  stash (may be NULL): what axon_lmhead_fwd left
+ * axon_lmhead_bwd_dlogit_copies_of says 2).  The workspace of a call over n_tokens serves every shorter one too.  stash (may be NULL): what axon_lmhead_fwd left
  * for the same operands, shape, temperature and softcap; the dlogits are then decoded from it by
  * a streaming kernel (2 bytes read, 4 written per logit) and the logits are not recomputed. */
 int64_t axon_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t hidden, int64_t vocab,
@@ -243,8 +243,11 @@ int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentropy, const v
 int axon_lmhead_block_can_group(int64_t hidden, int64_t vocab, int64_t vocab_chunk);
 /* How many bf16 copies of a chunk's dlogits the backward (axon_lmhead_bwd, axon_lmhead_block_bwd) writes for
  * this shape: 1 = token-major only (the weight-gradient GEMM reads it K-major), 2 = token-major and
- * vocab-major (hidden < 256, vocab % 8 != 0, or a last vocabulary chunk of fewer than 256 rows).  vocab_chunk 0 is taken as 32768. For
- * byte accounting; negative for an unsupported shape.  No reference counterpart. */
+ * vocab-major (hidden < 256, vocab % 8 != 0, or a last vocabulary chunk of fewer than 256 rows).  For
+ * byte accounting; negative for an unsupported shape.  The default chunk (vocab_chunk 0) depends on the token
+ * count: `_of` answers for a call over n_tokens, the other one for a chunk that is given, or (0) for the 32768
+ * columns that calls over 32768 tokens and more take.  No reference counterpart. */
+int axon_lmhead_bwd_dlogit_copies_of(int64_t n_tokens, int64_t hidden, int64_t vocab, int64_t vocab_chunk);
 int axon_lmhead_bwd_dlogit_copies(int64_t hidden, int64_t vocab, int64_t vocab_chunk);
 /* How many 256 KB parts of fp32 partial sums the dHidden reduction of a backward over n_tokens keeps in a workspace
  * of axon_lmhead_bwd_workspace_bytes(ws_tokens, ...), and in *reserved how many that workspace has room for: never

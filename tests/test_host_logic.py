@@ -316,9 +316,13 @@ def test_which_shapes_write_the_dlogits_once_and_may_group_blocks():
     assert copies(256, 1500, 512) == 2 and copies(192, 2048, 512) == 2             # vocab % 8, hidden < 256
     assert copies(4096, 151936, 100) < 0 and copies(4097, 151936, 0) < 0           # chunk % 256, hidden % 32
     assert group(4096, 151936, 152064) == 1 and group(4096, 151936, 0) == 0        # one chunk only
-    # with vocab % 64 == 0 the workspace holds no transposed weight either: hidden x (vocab + 64) x 2 bytes less
+    # the default chunk follows from the tokens: 33000 rows are one chunk of a short call, 32768 + 232 of a long one
+    of = lib.axon_lmhead_bwd_dlogit_copies_of
+    assert copies(256, 33000, 0) == of(32768, 256, 33000, 0) == 2 and of(700, 256, 33000, 0) == 1
+    assert of(700, 256, 1160, 512) == 2 and of(700, 256, 1160, 0) == 1 and of(700, 4097, 33000, 0) < 0
+    # the workspace holds no transposed weight, whatever the vocabulary's remainder: 8 rows more cost a tile of dlogits
     ws = lib.axon_lmhead_bwd_workspace_bytes
-    assert ws(8192, 256, 2048 + 8, 2304) - ws(8192, 256, 2048, 2048) > 256 * 2048 * 2
+    assert ws(8192, 256, 2048 + 8, 2304) - ws(8192, 256, 2048, 2048) == 8192 * 256 * 2
     assert group(256, 2048, 0) == 1 and group(128, 2048, 0) == 0 and group(256, 2044, 0) == 0
 
 
