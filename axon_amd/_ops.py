@@ -918,7 +918,7 @@ class HeadBlocks:
             raise _lib.AxonAmdError(f"HeadBlocks: unsupported shape tokens={n_max} hidden={self.h} vocab={self.v}")
         self.fwd_ws = torch.empty(self.fwd_ws_bytes, device=dev, dtype=torch.uint8)
         self.bwd_ws = torch.empty(self.bwd_ws_bytes, device=dev, dtype=torch.uint8)
-        self.keeps_stash = [bool(stash)] * len(self.ranges) if isinstance(stash, bool) else [bool(x) for x in stash]
+        self.keeps_stash = [bool(x) for x in (stash if isinstance(stash, (list, tuple)) else [stash] * len(self.ranges))]
         if len(self.keeps_stash) != len(self.ranges):
             raise ValueError(f"HeadBlocks: {len(self.keeps_stash)} stash choices for {len(self.ranges)} blocks")
         self.stash_bytes = max((self._stash_bytes(b - a) for (a, b), keep in zip(self.ranges, self.keeps_stash) if keep),

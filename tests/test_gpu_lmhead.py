@@ -958,6 +958,17 @@ def test_operands_are_not_read_beyond_their_last_row(n, h, v):
         assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
+def test_which_blocks_keep_a_stash():
+    """Any one truth value for all blocks, or a list of one per block."""
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(512, 64, 512, seed=2))
+    keeps = lambda stash: _ops.HeadBlocks(hid, w, lab, 1.0, [(0, 256), (256, 512)], stash=stash).keeps_stash
+    assert keeps(True) == keeps(1) == keeps([1, True]) == [True, True]
+    assert keeps(False) == keeps(0) == keeps(None) == keeps((0, False)) == [False, False]
+    assert keeps([False, True]) == [False, True]
+    with pytest.raises(ValueError, match="stash choices"):
+        keeps([True])
+
+
 def test_rows_of_an_edge_tile_beyond_the_operand_are_zeros_in_the_accumulators():
     """The weight gradient's partial sums keep whole tiles, the rows that the epilogue drops among them.  hidden = 288
     leaves 32 valid rows in the second tile, so that most of its load instructions start beyond the descriptor's
