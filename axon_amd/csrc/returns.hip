@@ -210,9 +210,11 @@ __global__ __launch_bounds__(kBlock) void reverse_scan_kernel(
 // stats[0] mean, [1] n, [2] variance (times n/(n-1) when n > 1), [3] rsqrt(variance + 1e-8)
 
 // Every workgroup that needs a pass's result adds the pass's at most kMomentBlocks partials itself, in the same fixed
-// order (64 KB out of L2), where a launch of one workgroup in between cost 3.6 us and the gaps around it.  Half as many
-// workgroups would double the length of every thread's fp32 sums.
-constexpr int kMomentBlocks = 2048;
+// order (32 KB out of L2), where a launch of one workgroup in between cost 3.6 us and the gaps around it.  With 2048
+// workgroups, 64 KB for each, the variance pass takes 8.8 us for 5.3 and the normalisation 8.7 for 5.7 at 2.1 M tokens, 42
+// for 40 and 51 for 44 at 33.5 M.  So that half the workgroups do not mean fp32 sums of twice the length, a thread adds its
+// vectors up in two sums in turn.
+constexpr int kMomentBlocks = 1024;
 
 __device__ __forceinline__ void add_partials(const float* __restrict__ partials, int n_blocks, float (&a)[2], float* lds_red) {
   float2 v[kMomentBlocks / kBlock];
@@ -265,23 +267,38 @@ __global__ __launch_bounds__(kBlock) void masked_moments_kernel(const float* __r
     mean = st[0];
     a[0] = a[1] = 0.f;
   }
-  const int64_t n_vec = n_slots / kVec;
-  for (int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x; q < n_vec;
-       q += (int64_t)gridDim.x * kBlock) {
-    float xv[4], mv[4];
-    load4(x, q * kVec, xv);
-    load_mask4<MK>(mask, q * kVec, mv);
+  const int64_t n_vec = n_slots / kVec, stride = (int64_t)gridDim.x * kBlock;
+  float b[2] = {0.f, 0.f};  // every other vector of the thread
+  auto add = [&](float (&s)[2], const float (&xv)[4], const float (&mv)[4]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (PASS == 0) {
-        a[0] += (mv[j] != 0.f) ? xv[j] * mv[j] : 0.f;
-        a[1] += mv[j];
+        s[0] += (mv[j] != 0.f) ? xv[j] * mv[j] : 0.f;
+        s[1] += mv[j];
       } else {
         const float d = xv[j] - mean;
-        a[0] += (mv[j] != 0.f) ? d * d * mv[j] : 0.f;
+        s[0] += (mv[j] != 0.f) ? d * d * mv[j] : 0.f;
       }
     }
+  };
+  int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  for (; q + stride < n_vec; q += 2 * stride) {
+    float x0[4], m0[4], x1[4], m1[4];
+    load4(x, q * kVec, x0);
+    load_mask4<MK>(mask, q * kVec, m0);
+    load4(x, (q + stride) * kVec, x1);
+    load_mask4<MK>(mask, (q + stride) * kVec, m1);
+    add(a, x0, m0);
+    add(b, x1, m1);
   }
+  if (q < n_vec) {
+    float x0[4], m0[4];
+    load4(x, q * kVec, x0);
+    load_mask4<MK>(mask, q * kVec, m0);
+    add(a, x0, m0);
+  }
+  a[0] += b[0];
+  a[1] += b[1];
   if (blockIdx.x == 0 && threadIdx.x < (int)(n_slots - n_vec * kVec)) {  // the ragged tail
     const int64_t p = n_vec * kVec + threadIdx.x;
     const float xv = x[p], m = load_mask1<MK>(mask, p);
@@ -459,7 +476,7 @@ int launch_scan(int mode, const float* rewards, const float* values, const void*
 
 unsigned moments_grid(int64_t n_slots) {
   const int64_t blocks = (n_slots / kVec + kBlock - 1) / kBlock;
-  const int64_t cap = kMomentBlocks;  // eight workgroups per compute unit walk the tokens
+  const int64_t cap = kMomentBlocks;  // four workgroups per compute unit walk the tokens
   return (unsigned)(blocks < 1 ? 1 : (blocks < cap ? blocks : cap));
 }
 
