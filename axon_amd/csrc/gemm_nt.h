@@ -2,10 +2,10 @@
 //
 // The 16x16x32 bf16 MFMA wants eight consecutive k of one row in every lane on
 // both sides.  K-contiguous operands ([row][k]) give that with one 16-byte LDS
-// read per fragment; the LM-head forward, its logit recompute and dHidden are
-// brought to this form (by pre-transposed copies of the weight and the hidden
-// states where needed).  An operand stored the other way round ([k][row],
-// "K-major": the dlogits in the dWeight product) is read as it lies with the LDS
+// read per fragment: both sides of the LM-head forward and of its logit recompute, the
+// dlogits in the dHidden product, the hidden states' transposed copy in the dWeight product.
+// An operand stored the other way round ([k][row], "K-major": the weight in the dHidden
+// product, the dlogits in the dWeight product) is read as it lies with the LDS
 // transpose read of gfx950, two 8-byte reads per fragment, at the same speed
 // within a per cent.  One main loop serves the whole path; the kernels differ
 // only in the epilogue.
@@ -33,9 +33,9 @@
 //      and on the accumulators of dropped rows).
 //      Shifting edge tiles back inside the matrix instead needed 256 rows on both
 //      sides (a forward over 187 tokens, 896 x 151936, ran on RegLoop: 355 us per call
-//      against 108 now) and token counts in fours for the head's stash (16381 tokens,
-//      2880 x 201088: half of a step recomputed its logits, 51.2 ms against 45.4 now).
-//  * RegLoop<32>  (k % 64 == 32, which the 64-wide k-tiles above do not divide):
+//      against 89 now).
+//  * RegLoop<32>  (k % 64 == 32, which the 64-wide k-tiles above do not divide, and operands whose
+//      rows lie closer together than a k-tile or off a 16-byte boundary):
 //      loads through registers with per-row clamping.
 //
 // Accumulator layout of one 16x16 block (four floats, index r):

@@ -216,7 +216,8 @@ int axon_lmhead_bwd_timed(const float* dlogprobs, const float* dentropy, const v
  *        tile by tile in register order, so that it streams at full width) is written;
  *        2 = a middle block, added to dw_acc; 3 = last block, dw_acc + this block's share is rounded
  *        to bf16 into d_weight and dw_acc is left as it was.  The same vocab_chunk in every call of a
- *        step.  stash may be NULL (the block's logits are then recomputed).
+ *        step.  stash may be NULL (the block's logits are then recomputed).  wt_ready is ignored (kept from the time
+ *        when the workspace held a transposed weight).
  *   timer: NULL, or an axon_timer_create object on `stream` (phases as below).
  * axon_scale_bf16_unless_one multiplies n bf16 values in place by the DEVICE scalar scale[0] and touches
  * nothing when it is exactly 1 (the step's gradients are finished before autograd hands over the

@@ -412,7 +412,7 @@ STASH_CASES = [
     (64, 128, 1000, 0, 0.0, False),
     (1, 32, 5, 0, 0.0, False),
     # hidden >= 256 and vocab % 8 == 0: the dlogits are written once and the weight gradient reads them K-major;
-    # chunks of 512 + 512 + 480 and 512 + 512 + 264 rows (edge tiles shifted back by 32 and 248 rows), one chunk,
+    # chunks of 512 + 512 + 480 and 512 + 512 + 264 rows (edge tiles of 224 and 8 rows), one chunk,
     # and a last chunk of 136 rows, which sends the whole call back to the two-copy path
     (516, 256, 1504, 512, 0.0, False),
     (772, 320, 1288, 512, 3.0, True),
@@ -461,10 +461,10 @@ def test_backward_from_stash_vs_recompute_and_oracle(n, h, v, chunk, cap, aligne
 
 
 def test_stash_policy_and_refusals():
-    """Shapes whose shifted tiles cannot hand rows over in fours have no stash and fall back to the recompute
+    """Large shapes whose tokens or vocabulary are no multiple of four have no stash and fall back to the recompute
     backward; the policy switch; a stash of another shape is refused."""
     assert _ops.lmhead_stash_bytes(513, 256, 1500) == 0 and _ops.lmhead_stash_bytes(516, 256, 1502) == 0
-    assert _ops.lmhead_stash_bytes(513, 96, 1501) > 0  # clamped tiles: any shape
+    assert _ops.lmhead_stash_bytes(513, 96, 1501) > 0  # hidden % 64 != 0: any shape
     assert _ops.lmhead_stash_bytes(32768, 4096, 151936) == 594 * 128 * 131072 + 594 * 2 * 32768 * 4
     hid, w, lab = W.lmhead_inputs(513, 256, 1500, seed=4)
     hd, wd, ld = hid.to(DEV), w.to(DEV), lab.to(DEV)
