@@ -42,6 +42,12 @@ SIGNATURES: dict[str, tuple] = {
     "axon_lmhead_block_bwd": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _i32, _ptr, _ptr, _i64, _i64, _i64,
                                      _f32, _f32, _ptr, _i64, _ptr, _ptr, _ptr, _i32, _i32, _i64, _i32, _i64,
                                      _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
+    "axon_lmhead_block_logits_bytes": (_i64, [_i64, _i64, _i64]),
+    "axon_lmhead_block_fwd_logits": (_i32, [_ptr, _ptr, _ptr, _i32, _i64, _i64, _i64, _f32, _f32, _ptr, _i64,
+                                            _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
+    "axon_lmhead_block_bwd_logits": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _i32, _ptr, _ptr, _i64, _i64, _i64,
+                                            _f32, _f32, _ptr, _i64, _ptr, _ptr, _ptr, _i32, _i32, _i64, _i32, _i64,
+                                            _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr]),
     "axon_lmhead_block_can_group": (_i32, [_i64, _i64, _i64]),
     "axon_lmhead_bwd_dlogit_copies": (_i32, [_i64, _i64, _i64]),
     "axon_lmhead_bwd_dlogit_copies_of": (_i32, [_i64, _i64, _i64, _i64]),

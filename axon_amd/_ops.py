@@ -887,11 +887,13 @@ class HeadBlocks:
     consecutive blocks share one weight-gradient GEMM (their dlogits stay in the workspace until the group's
     last block: a longer reduction and fewer passes over the fp32 partial sums for ``dw_group`` x the dlogit
     memory); 1 where the shape does not allow it (``axon_lmhead_block_can_group``).  ``stash``: whether the blocks'
-    dlogits are decoded from a stash (softmax numerators in 16 bits) or their logits recomputed in fp32, for all
-    blocks or one truth value per block."""
+    dlogits are decoded from a stash (softmax numerators in 16 bits) or formed from logits in fp32, for all
+    blocks or one truth value per block.  ``logits``: the same choice for the blocks without a stash, whether their fp32
+    logits are kept from the forward (4 bytes x block x vocab, shared by the blocks as the stash is) or recomputed:
+    the same bits either way.  Recomputed where the device has no memory for them."""
 
     def __init__(self, hidden, weight, labels, inv_temperature, ranges, *, softcap=0.0, seq_start=None,
-                 vocab_chunk=0, stash=True, dw_group=2, timing: "Timer | None" = None):
+                 vocab_chunk=0, stash=True, logits=False, dw_group=2, timing: "Timer | None" = None):
         self.lib = _lib.load()
         require_device(hidden, "HeadBlocks")
         self.n, self.h, self.v = _head_operands("HeadBlocks", hidden, weight, labels, seq_start)
@@ -918,12 +920,11 @@ class HeadBlocks:
             raise _lib.AxonAmdError(f"HeadBlocks: unsupported shape tokens={n_max} hidden={self.h} vocab={self.v}")
         self.fwd_ws = torch.empty(self.fwd_ws_bytes, device=dev, dtype=torch.uint8)
         self.bwd_ws = torch.empty(self.bwd_ws_bytes, device=dev, dtype=torch.uint8)
-        self.keeps_stash = [bool(x) for x in (stash if isinstance(stash, (list, tuple)) else [stash] * len(self.ranges))]
-        if len(self.keeps_stash) != len(self.ranges):
+        per_block = lambda x: [bool(y) for y in (x if isinstance(x, (list, tuple)) else [x] * len(self.ranges))]  # noqa: E731
+        self.keeps_stash, self.keeps_logits = per_block(stash), per_block(logits)
+        if len(self.keeps_stash) != len(self.ranges) or len(self.keeps_logits) != len(self.ranges):
             raise ValueError(f"HeadBlocks: {len(self.keeps_stash)} stash choices for {len(self.ranges)} blocks")
-        self.stash_bytes = max((self._stash_bytes(b - a) for (a, b), keep in zip(self.ranges, self.keeps_stash) if keep),
-                               default=0)
-        self.stash = torch.empty(self.stash_bytes, device=dev, dtype=torch.uint8) if self.stash_bytes else None
+        self.stash_bytes = self._keep_buffer(dev)
         self.stats = torch.empty(2, n_max, device=dev, dtype=torch.float32)  # lse, entropy_b of the current block
         # whole-stream outputs; position 0 is a sequence start (the aligned layout writes it from the last row)
         self.out = torch.zeros(2, max(self.n, 1), device=dev, dtype=torch.float32)
@@ -932,7 +933,7 @@ class HeadBlocks:
         self.one_block = self.n_groups == 1  # one weight-gradient GEMM: no partial sums to carry
         self.dw_acc_bytes = 0 if self.one_block else int(self.lib.axon_lmhead_block_dw_acc_bytes(self.h, self.v))
         self.dw_acc = torch.empty(self.dw_acc_bytes // 4, device=dev, dtype=torch.float32) if self.dw_acc_bytes else None
-        self.block_stash_bytes = 0
+        self.block_stash_bytes = self.block_logits_bytes = 0
         self.workspace_bytes = self.fwd_ws_bytes + self.bwd_ws_bytes + self.stash_bytes + self.dw_acc_bytes
 
     @property
@@ -945,6 +946,24 @@ class HeadBlocks:
 
     def _stash_bytes(self, n):
         return int(self.lib.axon_lmhead_block_stash_bytes(n, self.h, self.v))
+
+    def _logits_bytes(self, k):
+        n0, n1 = self.ranges[k]
+        keep = self.keeps_logits[k] and not self.keeps_stash[k]
+        return int(self.lib.axon_lmhead_block_logits_bytes(n1 - n0, self.h, self.v)) if keep else 0
+
+    def _keep_buffer(self, dev):
+        """Allocate what a block keeps from its forward to its backward, for the largest block; its size."""
+        stash = max((self._stash_bytes(b - a) for (a, b), keep in zip(self.ranges, self.keeps_stash) if keep), default=0)
+        size = max([stash] + [self._logits_bytes(k) for k in range(len(self.ranges))])
+        try:
+            self.stash = torch.empty(size, device=dev, dtype=torch.uint8) if size else None
+        except torch.OutOfMemoryError:
+            if size == stash:
+                raise
+            self.keeps_logits = [False] * len(self.ranges)  # as if nobody had asked: recomputed
+            return self._keep_buffer(dev)
+        return size
 
     def _block(self, k):
         n0, n1 = self.ranges[k]
@@ -962,13 +981,16 @@ class HeadBlocks:
         n0, n1, last_dst = self._block(k)
         nb = n1 - n0
         self.block_stash_bytes = self._stash_bytes(nb) if self.keeps_stash[k] else 0
-        check(self.lib.axon_lmhead_block_fwd(
+        self.block_logits_bytes = self._logits_bytes(k)
+        kept = self.block_stash_bytes or self.block_logits_bytes
+        fwd = self.lib.axon_lmhead_block_fwd_logits if self.block_logits_bytes else self.lib.axon_lmhead_block_fwd
+        check(fwd(
             self.hidden.data_ptr() + n0 * self.h * 2, ptr(self.weight), self._at(self.labels, n0),
             int(self.labels.dtype == torch.int64), nb, self.h, self.v, self.inv_t, self.softcap,
             self._at(self.seq_start, n0), last_dst, self._at(self.out[0], n0), self._at(self.out[1], n0),
             ptr(self.stats[0]), ptr(self.stats[1]), ptr(self.fwd_ws), self.fwd_ws_bytes,
-            ptr(self.stash) if self.block_stash_bytes else None, self.block_stash_bytes, stream_ptr(),
-            self.timing.handle if self.timing else None), "axon_lmhead_block_fwd")
+            ptr(self.stash) if kept else None, kept, stream_ptr(), self.timing.handle if self.timing else None),
+            "axon_lmhead_block_fwd")
 
     def backward(self, k, dlogprobs, dentropy):
         """Backward of block ``k`` (after its ``forward``; no other block's forward in between).  ``dlogprobs`` /
@@ -985,14 +1007,16 @@ class HeadBlocks:
         group, pos, dw_now = self.place[k]
         mode = (DW_STORE if self.one_block else DW_FIRST if group == 0
                 else DW_LAST if group == self.n_groups - 1 else DW_ADD)
-        check(self.lib.axon_lmhead_block_bwd(
+        kept = self.block_stash_bytes or self.block_logits_bytes
+        bwd = self.lib.axon_lmhead_block_bwd_logits if self.block_logits_bytes else self.lib.axon_lmhead_block_bwd
+        check(bwd(
             self._at(dlogprobs, n0), self._at(dentropy, n0), self.hidden.data_ptr() + n0 * self.h * 2,
             ptr(self.weight), self._at(self.labels, n0), int(self.labels.dtype == torch.int64),
             ptr(self.stats[0]), ptr(self.stats[1]), nb, self.h, self.v, self.inv_t, self.softcap,
             self._at(self.seq_start, n0), last_dst, self.d_hidden.data_ptr() + n0 * self.h * 2,
             ptr(self.d_weight), ptr(self.dw_acc), mode, 1, pos, int(dw_now), self.ws_tokens, self.chunk,
             ptr(self.bwd_ws), self.bwd_ws_bytes,
-            ptr(self.stash) if self.block_stash_bytes else None, self.block_stash_bytes, st, th),
+            ptr(self.stash) if kept else None, kept, st, th),
             "axon_lmhead_block_bwd")
 
 

@@ -43,8 +43,10 @@ struct FwdParams {
   int n_tokens, vocab;
   float c;     // inv_temperature * log2(e)
   float cap, inv_cap;  // logit soft-capping cap * tanh(logit / cap) (SOFTCAP kernels only)
-  uint4* stash;        // STASH kernels only: 128 KB per tile, see StashLayout
+  uint4* stash;        // kernels that keep something for the backward: the stash or the logits, see below
 };
+// What a forward leaves for its backward beside the statistics.
+enum Keep { kKeepNone, kKeepStash, kKeepLogits };
 
 // What a stashing forward leaves for the backward: for every logit, w = 2^(y - M) as fp16, where
 // y is the scaled logit in log2 units and M the maximum of y over the 128 vocabulary rows of the
@@ -57,6 +59,12 @@ struct FwdParams {
 // Vocabulary rows beyond the matrix are stored as 0.
 constexpr int64_t kStashTileBytes = 131072;
 constexpr int kStashWaveVecs = 2048;  // uint4 per wavefront sub-tile
+
+// kKeepLogits: the accumulators themselves (fp32, before temperature and soft-capping), so that the backward forms
+// the very dlogits that it would form from recomputed logits, without the product.  Accumulator order again, one
+// contiguous kilobyte per store:  uint4 index = ((tile * 4 + wave) * 64 + j * 8 + i) * 64 + lane.
+constexpr int64_t kLogitsTileBytes = 262144;
+constexpr int kLogitsWaveVecs = 4096;  // uint4 per wavefront sub-tile
 
 __device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -170,7 +178,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTile& acc, const FwdParams& p, c
 }
 
 // SOFTCAP: the logits go through cap * tanh(. / cap) before the statistics (fused_linear.py:19-23).
-template <class Loop, bool SOFTCAP, bool STASH>
+template <class Loop, bool SOFTCAP, Keep KEEP>
 __device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams& p, int tiles_m,
                                          int tiles_n) {
   extern __shared__ __align__(16) char smem[];
@@ -179,6 +187,16 @@ __device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams&
   const TilePos t = Loop::place(tm, tn);
   AccTile acc;
   Loop::run(g, t, acc, smem);
+  const LanePos lp;
+  if (KEEP == kKeepLogits) {  // written once, read once by the backward, long after: past the caches
+    float4* const out = reinterpret_cast<float4*>(p.stash) +
+                        ((int64_t)(tm * tiles_n + tn) * 4 + lp.wave) * kLogitsWaveVecs + lp.lane;
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+      for (int i = 0; i < kBlocks; ++i)
+        __builtin_nontemporal_store(acc[i][j], reinterpret_cast<acc4*>(out + (j * kBlocks + i) * 64));
+  }
   if (SOFTCAP) {
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i)
@@ -187,7 +205,7 @@ __device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams&
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[i][j][r] = p.cap * fast_tanh(acc[i][j][r] * p.inv_cap);
   }
-  const LanePos lp;
+  constexpr bool STASH = KEEP == kKeepStash;
   uint4* const stash_wave =
       STASH ? p.stash + ((int64_t)(tm * tiles_n + tn) * 4 + lp.wave) * kStashWaveVecs + lp.lane : nullptr;
   if (t.m0 + kTile > p.vocab)
@@ -199,20 +217,20 @@ __device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams&
 template <class Loop>
 __global__ __launch_bounds__(kGemmThreads) void lmhead_fwd_kernel(GemmOperands g, FwdParams p,
                                                                   int tiles_m, int tiles_n) {
-  fwd_body<Loop, false, false>(g, p, tiles_m, tiles_n);
+  fwd_body<Loop, false, kKeepNone>(g, p, tiles_m, tiles_n);
 }
 
 template <class Loop>
 __global__ __launch_bounds__(kGemmThreads) void lmhead_fwd_softcap_kernel(GemmOperands g,
                                                                           FwdParams p, int tiles_m,
                                                                           int tiles_n) {
-  fwd_body<Loop, true, false>(g, p, tiles_m, tiles_n);
+  fwd_body<Loop, true, kKeepNone>(g, p, tiles_m, tiles_n);
 }
 
 template <class Loop>
 __global__ __launch_bounds__(kGemmThreads) void lmhead_fwd_stash_kernel(GemmOperands g, FwdParams p,
                                                                         int tiles_m, int tiles_n) {
-  fwd_body<Loop, false, true>(g, p, tiles_m, tiles_n);
+  fwd_body<Loop, false, kKeepStash>(g, p, tiles_m, tiles_n);
 }
 
 template <class Loop>
@@ -220,7 +238,13 @@ __global__ __launch_bounds__(kGemmThreads) void lmhead_fwd_softcap_stash_kernel(
                                                                                 FwdParams p,
                                                                                 int tiles_m,
                                                                                 int tiles_n) {
-  fwd_body<Loop, true, true>(g, p, tiles_m, tiles_n);
+  fwd_body<Loop, true, kKeepStash>(g, p, tiles_m, tiles_n);
+}
+
+template <bool SOFTCAP>
+__global__ __launch_bounds__(kGemmThreads) void lmhead_fwd_logits_kernel(GemmOperands g, FwdParams p,
+                                                                         int tiles_m, int tiles_n) {
+  fwd_body<DmaLoop, SOFTCAP, kKeepLogits>(g, p, tiles_m, tiles_n);
 }
 
 // Token-aligned packed layout.  With `is_start` (one byte per packed position, 1 where a sequence
@@ -431,6 +455,22 @@ struct TokenCoef {
   }
 };
 
+// The dlogit of one logit (the accumulator, before temperature and soft-capping), row mrel of the tile.
+template <bool SOFTCAP>
+__device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef& k, const DlogitParams& p, float c) {
+  float dcap = 1.f;
+  if (SOFTCAP) {
+    const float th = fast_tanh(raw * p.inv_cap);
+    raw = p.cap * th;
+    dcap = fmaf(-th, th, 1.f);
+  }
+  const float pr = fast_exp2(fmaf(raw, c, -k.lse2));
+  float v = pr * fmaf(k.cb, raw, k.ca);
+  if (mrel == k.lab_rel) v += k.gl;
+  if (SOFTCAP) v *= dcap;
+  return v;
+}
+
 template <bool SOFTCAP, bool MASKED>
 __device__ __forceinline__ void dlogit_stage(AccTile& acc, const DlogitParams& p, const LanePos& lp,
                                              const TilePos& t, char* stage) {
@@ -446,17 +486,7 @@ __device__ __forceinline__ void dlogit_stage(AccTile& acc, const DlogitParams& p
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int mrel = lp.m(i, r);
-        float raw = acc[i][j][r];
-        float dcap = 1.f;
-        if (SOFTCAP) {
-          const float th = fast_tanh(raw * p.inv_cap);
-          raw = p.cap * th;
-          dcap = fmaf(-th, th, 1.f);
-        }
-        const float pr = fast_exp2(fmaf(raw, c, -k.lse2));
-        float v = pr * fmaf(k.cb, raw, k.ca);
-        if (mrel == k.lab_rel) v += k.gl;
-        if (SOFTCAP) v *= dcap;
+        const float v = dlogit_of<SOFTCAP>(acc[i][j][r], mrel, k, p, c);
         d[r] = (!MASKED || mrel < m_end) ? v : 0.f;
       }
       uint2 w;
@@ -507,6 +537,37 @@ __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashH
         }
         const bool ok = !EDGE || (n_counts && p.v_begin + t.m0 + mrel < p.vocab);
         d[r] = ok ? v : 0.f;
+      }
+      uint2 w;
+      w.x = pack_bf16(d[0], d[1]);
+      w.y = pack_bf16(d[2], d[3]);
+      *reinterpret_cast<uint2*>(stage + stage_off(nw, i * 4 + lp.lq)) = w;
+    }
+  }
+}
+
+// The same from the logits that a forward kept (kKeepLogits): the arithmetic of dlogit_stage on what the
+// accumulators held.
+template <bool SOFTCAP, bool EDGE>
+__device__ __forceinline__ void dlogit_stage_logits(const float4 (&x)[kStashHalfBlocks * kBlocks], int j0,
+                                                    const DlogitParams& p, const LanePos& lp, const TilePos& t,
+                                                    char* stage) {
+  const float c = p.inv_temp * kLog2e;
+#pragma unroll
+  for (int jl = 0; jl < kStashHalfBlocks; ++jl) {
+    const int nw = jl * kBlk + lp.l16;
+    const TokenCoef k(p, t.n0 + lp.wn * kWaveTile + j0 * kBlk + nw, (int64_t)p.v_begin + t.m0);
+    const int m_end = EDGE ? (k.n_ok ? p.vocab - p.v_begin - t.m0 : 0) : kTile;  // rows that count
+#pragma unroll
+    for (int i = 0; i < kBlocks; ++i) {
+      const float4 q = x[jl * kBlocks + i];
+      const float raw[4] = {q.x, q.y, q.z, q.w};
+      float d[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int mrel = lp.m(i, r);
+        const float v = dlogit_of<SOFTCAP>(raw[r], mrel, k, p, c);
+        d[r] = (!EDGE || mrel < m_end) ? v : 0.f;
       }
       uint2 w;
       w.x = pack_bf16(d[0], d[1]);
@@ -679,6 +740,35 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_stash_kernel(DlogitParams p,
   } else {
     dlogit_stage_stash<SOFTCAP, false>(st, j0, src.pm, part, p, lp, t, stage);
   }
+  dlogit_copy_out_half(stage, j0, p, lp, t);
+}
+
+// The same from kept logits: 4 bytes read and 2 written per logit.
+template <bool SOFTCAP>
+__global__ __launch_bounds__(64) void lmhead_dlogit_logits_kernel(DlogitParams p, StashSource src) {
+  __shared__ __align__(16) char stage[kStashHalfBlocks * kBlk * 256];  // 64 tokens x 128 bf16
+  const int half = blockIdx.x & 1, wave = (blockIdx.x >> 1) & 3, tile = blockIdx.x >> 3;
+  const int tm = src.tm0 + tile / src.tiles_n, tn = tile % src.tiles_n;
+  TilePos t{tm * kTile, tn * kTile};
+  LanePos lp;
+  lp.wave = wave;
+  lp.wm = wave >> 1;
+  lp.wn = wave & 1;
+  const int j0 = half * kStashHalfBlocks;
+  const uint4* sv = src.stash + ((int64_t)(tm * src.tiles_n + tn) * 4 + wave) * kLogitsWaveVecs +
+                    j0 * kBlocks * 64 + lp.lane;
+  float4 x[kStashHalfBlocks * kBlocks];
+#pragma unroll
+  for (int q = 0; q < kStashHalfBlocks * kBlocks; ++q) {  // read once
+    const acc4 v = __builtin_nontemporal_load(reinterpret_cast<const acc4*>(sv + q * 64));
+    x[q] = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  const bool edge = t.m0 + kTile > p.vocab || t.n0 + kTile > p.n_tokens;
+  t.m0 -= p.v_begin;
+  if (edge)
+    dlogit_stage_logits<SOFTCAP, true>(x, j0, p, lp, t, stage);
+  else
+    dlogit_stage_logits<SOFTCAP, false>(x, j0, p, lp, t, stage);
   dlogit_copy_out_half(stage, j0, p, lp, t);
 }
 
@@ -1073,6 +1163,11 @@ StashWs stash_ws(int64_t n, int64_t v, void* base) {
   w.bytes = tile_bytes + round_up((int64_t)w.tiles_m * 2 * n * 4, kAlign);
   return w;
 }
+// The logits that a block's forward keeps in fp32 (kKeepLogits), for the shapes of its main loop; 0 for others.
+int64_t logits_bytes(int64_t n, int64_t h, int64_t v) {
+  if (n <= 0 || h % DmaLoop::kBK != 0 || h >= kMaxLd) return 0;
+  return (round_up(v, kTile) / kTile) * (round_up(n, kTile) / kTile) * kLogitsTileBytes;
+}
 // The whole-call operator (axon_lmhead_fwd / _bwd) keeps a stash for the shapes its callers have always got
 // one for; the block entry points take any shape.
 bool stash_of_all_tokens(int64_t n, int64_t h, int64_t v) {
@@ -1289,11 +1384,22 @@ int launch_transpose(const void* in, int64_t ld_in, int rows, int cols, void* ou
   return AXON_OK;
 }
 
+template <bool SOFTCAP>
+int launch_fwd_logits(const GemmOperands& g, const FwdParams& p, hipStream_t st) {
+  const int tiles_m = (g.m_rows + kTile - 1) / kTile, tiles_n = (g.n_rows + kTile - 1) / kTile;
+  if (!dma_ok(g)) return AXON_ERR_SHAPE;
+  if (set_lds(lmhead_fwd_logits_kernel<SOFTCAP>) != AXON_OK) return AXON_ERR_LAUNCH;
+  hipLaunchKernelGGL(lmhead_fwd_logits_kernel<SOFTCAP>, dim3(tiles_m * tiles_n), dim3(kGemmThreads), kGemmLdsBytes, st,
+                     g, p, tiles_m, tiles_n);
+  AXON_CHECK_LAUNCH();
+  return AXON_OK;
+}
+
 int fwd_impl(const void* hidden, const void* weight, const void* labels, int labels_i64, int64_t n,
              int64_t h, int64_t v, float inv_temp, float softcap, const uint8_t* is_start,
              int64_t last_dst, float* logprobs, float* entropy, float* lse, float* entropy_b,
              void* workspace, int64_t ws_bytes, void* stash, int64_t stash_bytes, void* stream,
-             PhaseTimer* timer, bool is_block = false) {
+             PhaseTimer* timer, bool is_block = false, Keep keep = kKeepStash) {
   int rc = check_head_shape(n, h, v);
   if (rc != AXON_OK) return rc;
   if (n == 0) return AXON_OK;
@@ -1309,10 +1415,17 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
   StashWs sw{};
   if (stash) {
     if (reinterpret_cast<uintptr_t>(stash) & 15) return AXON_ERR_ARG;
-    if (!is_block && !stash_of_all_tokens(n, h, v)) return AXON_ERR_SHAPE;
-    sw = stash_ws(n, v, stash);
-    if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
-    w.pm = sw.pm;  // the backward needs the per-part maxima: they live in the stash
+    if (keep == kKeepLogits) {
+      const int64_t bytes = logits_bytes(n, h, v);
+      if (bytes == 0) return AXON_ERR_SHAPE;
+      if (bytes > stash_bytes) return AXON_ERR_WORKSPACE;
+      sw.tiles = static_cast<uint4*>(stash);
+    } else {
+      if (!is_block && !stash_of_all_tokens(n, h, v)) return AXON_ERR_SHAPE;
+      sw = stash_ws(n, v, stash);
+      if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
+      w.pm = sw.pm;  // the backward needs the per-part maxima: they live in the stash
+    }
   }
 
   GemmOperands g;
@@ -1323,7 +1436,10 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
               softcap > 0.f ? 1.f / softcap : 0.f, sw.tiles};
   {
     Span span(timer, 0);
-    if (stash) {
+    if (stash && keep == kKeepLogits) {
+      rc = softcap > 0.f ? launch_fwd_logits<true>(g, p, st) : launch_fwd_logits<false>(g, p, st);
+      if (rc != AXON_OK) return rc;
+    } else if (stash) {
       if (softcap > 0.f)
         AXON_LAUNCH_GEMM(lmhead_fwd_softcap_stash_kernel, g, p, st);
       else
@@ -1357,6 +1473,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
 enum { kDwStore = 0, kDwFirst = 1, kDwAdd = 2, kDwLast = 3 };
 struct BlockArgs {
   bool is_block = false;  // a stash for any shape, as the caller decides; else the shapes of stash_of_all_tokens
+  Keep keep = kKeepStash;  // what the buffer beside the forward's holds
   int64_t last_dst = 0;
   int dw_mode = kDwStore;
   float* dw_acc = nullptr;  // axon_lmhead_block_dw_acc_bytes of fp32 partial sums, tile order (modes other than kDwStore)
@@ -1409,7 +1526,9 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
     if (reinterpret_cast<uintptr_t>(stash) & 15) return AXON_ERR_ARG;
     if (!blk.is_block && !stash_of_all_tokens(n, h, v)) return AXON_ERR_SHAPE;
     sw = stash_ws(n, v, const_cast<void*>(stash));
-    if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
+    const int64_t bytes = blk.keep == kKeepLogits ? logits_bytes(n, h, v) : sw.bytes;
+    if (bytes == 0) return AXON_ERR_SHAPE;
+    if (bytes > stash_bytes) return AXON_ERR_WORKSPACE;
   }
 
   // the hidden states K-contiguous for the weight gradient, zeros up to the tile border
@@ -1443,10 +1562,10 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       if (stash) {
         const StashSource src{sw.tiles, sw.pm, sw.tiles_n, (int)(v0 / kTile)};
         const unsigned blocks = (unsigned)(round_up(vc, kTile) / kTile) * (unsigned)sw.tiles_n * 8u;
-        if (softcap > 0.f)
-          hipLaunchKernelGGL(lmhead_dlogit_stash_kernel<true>, dim3(blocks), dim3(64), 0, st, p, src);
-        else
-          hipLaunchKernelGGL(lmhead_dlogit_stash_kernel<false>, dim3(blocks), dim3(64), 0, st, p, src);
+        auto* const kernel = blk.keep == kKeepLogits
+                                 ? (softcap > 0.f ? lmhead_dlogit_logits_kernel<true> : lmhead_dlogit_logits_kernel<false>)
+                                 : (softcap > 0.f ? lmhead_dlogit_stash_kernel<true> : lmhead_dlogit_stash_kernel<false>);
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, st, p, src);
         AXON_CHECK_LAUNCH();
       } else if (softcap > 0.f) {
         AXON_LAUNCH_GEMM(lmhead_dlogit_softcap_kernel, g, p, st);
@@ -1777,36 +1896,60 @@ extern "C" int axon_lmhead_block_begin(const void* weight, int64_t h, int64_t v,
   return rc;
 }
 
-extern "C" int axon_lmhead_block_fwd(const void* hidden, const void* weight, const void* labels,
-                                     int labels_i64, int64_t n, int64_t h, int64_t v, float inv_temp,
-                                     float softcap, const uint8_t* seq_start, int64_t last_dst,
-                                     float* logprobs, float* entropy, float* lse, float* entropy_b,
-                                     void* workspace, int64_t ws_bytes, void* stash,
-                                     int64_t stash_bytes, void* stream, void* timer) {
+extern "C" int64_t axon_lmhead_block_logits_bytes(int64_t n, int64_t h, int64_t v) {
+  if (check_head_shape(n, h, v) != AXON_OK) return -1;
+  return logits_bytes(n, h, v);
+}
+
+static int block_fwd(const void* hidden, const void* weight, const void* labels, int labels_i64, int64_t n,
+                     int64_t h, int64_t v, float inv_temp, float softcap, const uint8_t* seq_start,
+                     int64_t last_dst, float* logprobs, float* entropy, float* lse, float* entropy_b,
+                     void* workspace, int64_t ws_bytes, void* stash, int64_t stash_bytes, void* stream,
+                     void* timer, Keep keep) {
   if (!last_dst_ok(last_dst, n)) return AXON_ERR_ARG;
   int rc;
   PhaseTimer* t = block_timer(timer, stream, 0, &rc);
   if (rc != AXON_OK) return rc;
   return fwd_impl(hidden, weight, labels, labels_i64, n, h, v, inv_temp, softcap, seq_start, last_dst,
-                  logprobs, entropy, lse, entropy_b, workspace, ws_bytes, stash, stash_bytes, stream, t, true);
+                  logprobs, entropy, lse, entropy_b, workspace, ws_bytes, stash, stash_bytes, stream, t, true, keep);
 }
 
-extern "C" int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentropy, const void* hidden,
-                                     const void* weight, const void* labels, int labels_i64,
-                                     const float* lse, const float* entropy_b, int64_t n, int64_t h,
-                                     int64_t v, float inv_temp, float softcap,
-                                     const uint8_t* seq_start, int64_t last_dst, void* d_hidden,
-                                     void* d_weight, float* dw_acc, int dw_mode, int /*wt_ready*/,
-                                     int64_t group_pos, int dw_now, int64_t ws_tokens,
-                                     int64_t chunk, void* workspace, int64_t ws_bytes,
-                                     const void* stash, int64_t stash_bytes, void* stream,
+extern "C" int axon_lmhead_block_fwd(const void* hidden, const void* weight, const void* labels, int labels_i64,
+                                     int64_t n, int64_t h, int64_t v, float inv_temp, float softcap,
+                                     const uint8_t* seq_start, int64_t last_dst, float* logprobs,
+                                     float* entropy, float* lse, float* entropy_b, void* workspace,
+                                     int64_t ws_bytes, void* stash, int64_t stash_bytes, void* stream,
                                      void* timer) {
+  return block_fwd(hidden, weight, labels, labels_i64, n, h, v, inv_temp, softcap, seq_start, last_dst,
+                   logprobs, entropy, lse, entropy_b, workspace, ws_bytes, stash, stash_bytes, stream, timer,
+                   kKeepStash);
+}
+
+extern "C" int axon_lmhead_block_fwd_logits(const void* hidden, const void* weight, const void* labels,
+                                            int labels_i64, int64_t n, int64_t h, int64_t v, float inv_temp,
+                                            float softcap, const uint8_t* seq_start, int64_t last_dst,
+                                            float* logprobs, float* entropy, float* lse, float* entropy_b,
+                                            void* workspace, int64_t ws_bytes, void* stash, int64_t stash_bytes,
+                                            void* stream, void* timer) {
+  return block_fwd(hidden, weight, labels, labels_i64, n, h, v, inv_temp, softcap, seq_start, last_dst,
+                   logprobs, entropy, lse, entropy_b, workspace, ws_bytes, stash, stash_bytes, stream, timer,
+                   kKeepLogits);
+}
+
+static int block_bwd(const float* dlogprobs, const float* dentropy, const void* hidden, const void* weight,
+                     const void* labels, int labels_i64, const float* lse, const float* entropy_b, int64_t n,
+                     int64_t h, int64_t v, float inv_temp, float softcap, const uint8_t* seq_start,
+                     int64_t last_dst, void* d_hidden, void* d_weight, float* dw_acc, int dw_mode,
+                     int /*wt_ready*/, int64_t group_pos, int dw_now, int64_t ws_tokens, int64_t chunk,
+                     void* workspace, int64_t ws_bytes, const void* stash, int64_t stash_bytes, void* stream,
+                     void* timer, Keep keep) {
   if (!last_dst_ok(last_dst, n) || n <= 0) return AXON_ERR_ARG;
   int rc;
   PhaseTimer* t = block_timer(timer, stream, 4, &rc);
   if (rc != AXON_OK) return rc;
   BlockArgs blk;
   blk.is_block = true;
+  blk.keep = keep;
   blk.last_dst = last_dst;
   blk.dw_mode = dw_mode;
   blk.dw_acc = dw_acc;
@@ -1816,6 +1959,34 @@ extern "C" int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentro
   return bwd_impl(dlogprobs, dentropy, hidden, weight, labels, labels_i64, lse, entropy_b, n, h, v,
                   inv_temp, softcap, seq_start, d_hidden, d_weight, chunk, workspace, ws_bytes, stash,
                   stash_bytes, stream, t, blk);
+}
+
+extern "C" int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentropy, const void* hidden,
+                                     const void* weight, const void* labels, int labels_i64, const float* lse,
+                                     const float* entropy_b, int64_t n, int64_t h, int64_t v, float inv_temp,
+                                     float softcap, const uint8_t* seq_start, int64_t last_dst, void* d_hidden,
+                                     void* d_weight, float* dw_acc, int dw_mode, int wt_ready,
+                                     int64_t group_pos, int dw_now, int64_t ws_tokens, int64_t chunk,
+                                     void* workspace, int64_t ws_bytes, const void* stash, int64_t stash_bytes,
+                                     void* stream, void* timer) {
+  return block_bwd(dlogprobs, dentropy, hidden, weight, labels, labels_i64, lse, entropy_b, n, h, v, inv_temp,
+                   softcap, seq_start, last_dst, d_hidden, d_weight, dw_acc, dw_mode, wt_ready, group_pos,
+                   dw_now, ws_tokens, chunk, workspace, ws_bytes, stash, stash_bytes, stream, timer,
+                   kKeepStash);
+}
+
+extern "C" int axon_lmhead_block_bwd_logits(const float* dlogprobs, const float* dentropy, const void* hidden,
+                                            const void* weight, const void* labels, int labels_i64,
+                                            const float* lse, const float* entropy_b, int64_t n, int64_t h,
+                                            int64_t v, float inv_temp, float softcap, const uint8_t* seq_start,
+                                            int64_t last_dst, void* d_hidden, void* d_weight, float* dw_acc,
+                                            int dw_mode, int wt_ready, int64_t group_pos, int dw_now,
+                                            int64_t ws_tokens, int64_t chunk, void* workspace, int64_t ws_bytes,
+                                            const void* stash, int64_t stash_bytes, void* stream, void* timer) {
+  return block_bwd(dlogprobs, dentropy, hidden, weight, labels, labels_i64, lse, entropy_b, n, h, v, inv_temp,
+                   softcap, seq_start, last_dst, d_hidden, d_weight, dw_acc, dw_mode, wt_ready, group_pos,
+                   dw_now, ws_tokens, chunk, workspace, ws_bytes, stash, stash_bytes, stream, timer,
+                   kKeepLogits);
 }
 
 extern "C" int axon_scale_bf16_unless_one(void* x, int64_t n, const float* scale, void* stream) {

@@ -34,6 +34,12 @@ from axon_amd.trainer.algos.loss.loss import POLICY_LOSS_KINDS, policy_loss_metr
 # vocab x hidden x 4 bytes per group.
 DEFAULT_BLOCK_TOKENS = 8192
 DEFAULT_DW_GROUP = 2
+# The blocks without a stash (blocks_with_stash) keep their fp32 logits from the forward to the backward, 4 bytes x
+# block x vocab, where the product that recomputes them costs more than writing and reading them: its time grows
+# with the hidden size, the traffic does not.  Head forward + backward of 6007 tokens x 151936, recomputed / kept:
+# hidden 256 2.85 / 3.01 ms, 512 4.00 / 3.83, 896 6.02 / 5.73; 8189 x 2880 x 201088 26.9 / 22.7, 8189 x 4096 x 151936
+# 27.3 / 22.3.
+KEEP_LOGITS_MIN_HIDDEN = 512
 _TILE = 256
 
 
@@ -64,10 +70,10 @@ def sequence_blocks(cu: list, block_tokens: int):
 
 def blocks_with_stash(ranges, n: int, h: int, v: int):
     """Per block: whether its backward decodes the dlogits from the forward's stash, whose softmax numerators have
-    16 bits, or recomputes the logits in fp32.  The stash where the whole-call operator has one for such a shape
+    16 bits, or forms them from fp32 logits (kept or recomputed).  The stash where the whole-call operator has one for such a shape
     (``lmhead_stash_bytes``: large blocks need token count and vocabulary in fours); a block with others behind it counts
     as rounded up to four rows, so that among the large blocks of such a vocabulary only the one that ends an odd
-    stream recomputes: one more product of its rows, and no bits that a caller did not give away."""
+    stream has fp32 logits, and no bits are lost that a caller did not give away."""
     return [_ops.lmhead_stash_bytes(min(n - a, (b - a + 3) // 4 * 4), h, v) > 0 for a, b in ranges]
 
 
@@ -131,7 +137,8 @@ class _BlockedHeadLoss(torch.autograd.Function):
 
         hb = _ops.HeadBlocks(hidden, weight, spec["ids"], spec["inv_t"], ranges, softcap=spec["softcap"],
                              seq_start=spec["seq_start"], vocab_chunk=spec["vocab_chunk"], dw_group=spec["dw_group"],
-                             stash=blocks_with_stash(ranges, n, hidden.shape[1], weight.shape[0]), timing=_ops.TIMING)
+                             stash=blocks_with_stash(ranges, n, hidden.shape[1], weight.shape[0]),
+                             logits=hidden.shape[1] >= KEEP_LOGITS_MIN_HIDDEN, timing=_ops.TIMING)
         g_lp = torch.zeros(n + 4, device=dev, dtype=torch.float32)
         want_ent_grad = side is not None and side["entropy_coef"] != 0
         g_en = torch.zeros(n + 4, device=dev, dtype=torch.float32) if want_ent_grad else None

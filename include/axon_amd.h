@@ -207,6 +207,11 @@ int axon_lmhead_bwd_timed(const float* dlogprobs, const float* dentropy, const v
  *        first position), and minus the block's first position when the block ends the stream (index 0
  *        of the whole arrays, a sequence start).  0 is the whole-stream call, as axon_lmhead_fwd.
  *   axon_lmhead_block_stash_bytes: the stash of a block of n_tokens rows; any shape the head takes.
+ *   axon_lmhead_block_fwd_logits / _bwd_logits: the same two calls with the block's logits kept in fp32
+ *        (axon_lmhead_block_logits_bytes bytes, 16-byte aligned, about 4 bytes x block tokens x vocab) in place of
+ *        the stash, whose softmax numerators have 16 bits: the gradients are those of a backward that recomputes
+ *        the logits, bit for bit, without the product.  hidden % 64 == 0 (the query answers 0 for other shapes,
+ *        the calls AXON_ERR_SHAPE).
  *   axon_lmhead_block_begin: checks its arguments and launches nothing (the backward reads the weight
  *        where it lies); kept for callers that open a step with it.
  *   axon_lmhead_block_bwd: d_hidden rows of the block (bf16, complete: a row sums over the vocabulary
@@ -241,6 +246,22 @@ int axon_lmhead_block_bwd(const float* dlogprobs, const float* dentropy, const v
                           int64_t group_pos, int dw_now, int64_t ws_tokens,
                           int64_t vocab_chunk, void* workspace, int64_t workspace_bytes,
                           const void* stash, int64_t stash_bytes, void* stream, void* timer);
+int64_t axon_lmhead_block_logits_bytes(int64_t n_tokens, int64_t hidden, int64_t vocab);
+int axon_lmhead_block_fwd_logits(const void* hidden_bf16, const void* weight_bf16, const void* labels,
+                                 int labels_are_i64, int64_t n_tokens, int64_t hidden, int64_t vocab,
+                                 float inv_temperature, float softcap, const uint8_t* seq_start,
+                                 int64_t last_dst, float* logprobs, float* entropy, float* lse,
+                                 float* entropy_b, void* workspace, int64_t workspace_bytes, void* logits,
+                                 int64_t logits_bytes, void* stream, void* timer);
+int axon_lmhead_block_bwd_logits(const float* dlogprobs, const float* dentropy, const void* hidden_bf16,
+                                 const void* weight_bf16, const void* labels, int labels_are_i64,
+                                 const float* lse, const float* entropy_b, int64_t n_tokens, int64_t hidden,
+                                 int64_t vocab, float inv_temperature, float softcap,
+                                 const uint8_t* seq_start, int64_t last_dst, void* d_hidden_bf16,
+                                 void* d_weight_bf16, float* dw_acc, int dw_mode, int wt_ready,
+                                 int64_t group_pos, int dw_now, int64_t ws_tokens,
+                                 int64_t vocab_chunk, void* workspace, int64_t workspace_bytes,
+                                 const void* logits, int64_t logits_bytes, void* stream, void* timer);
 int axon_lmhead_block_can_group(int64_t hidden, int64_t vocab, int64_t vocab_chunk);
 /* How many bf16 copies of a chunk's dlogits the backward (axon_lmhead_bwd, axon_lmhead_block_bwd) writes for
  * this shape: 1 = token-major only (the weight-gradient GEMM reads it K-major), 2 = token-major and

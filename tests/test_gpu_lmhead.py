@@ -988,3 +988,57 @@ def test_rows_of_an_edge_tile_beyond_the_operand_are_zeros_in_the_accumulators()
     hb.backward(1, g_lp, None)
     ref_dh, ref_dw = OM.backward(g_lp.cpu(), None, hid, wd.cpu(), lab)
     assert rel_l2(hb.d_weight, ref_dw) < 2e-2 and rel_l2(hb.d_hidden, ref_dh) < 2e-2
+
+
+@pytest.mark.parametrize("n,h,v,chunk,cap,lens", [
+    (257, 64, 256, 0, 0.0, None),              # one row into a second token tile, one vocabulary tile
+    (301, 128, 1999, 0, 0.0, None),            # ragged on both sides
+    (301, 320, 1999, 512, 5.0, None),          # vocabulary chunks, soft-capping
+    (515, 512, 1001, 0, 0.0, (100, 300, 115)),  # token-aligned layout, blocks that share a weight-gradient GEMM
+    (770, 256, 2000, 0, 5.0, (400, 370)),
+    (5, 64, 40, 0, 0.0, None),
+])
+def test_block_with_its_logits_kept_gives_the_bits_of_the_recompute(n, h, v, chunk, cap, lens):
+    """axon_lmhead_block_fwd_logits / _bwd_logits: the kept accumulators stand for the recomputed ones, so head
+    outputs and both gradients are equal bit for bit."""
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(n, h, v, seed=n))
+    w = (w.float() * 6).bfloat16()
+    g = torch.Generator().manual_seed(v)
+    g_lp, g_en = torch.randn(n + 4, generator=g).to(DEV), torch.randn(n + 4, generator=g).to(DEV)
+    flags, ranges = None, [(0, n)]
+    if lens:
+        flags = _ops.seq_start_flags(torch.tensor((0,) + lens).cumsum(0).int().to(DEV), n)
+        ranges = [(0, 256), (256, n)]
+
+    def run(logits):
+        hb = _ops.HeadBlocks(hid, w, lab, 1.0 / 0.7, ranges, softcap=cap, seq_start=flags, vocab_chunk=chunk, stash=False,
+                             logits=logits)
+        for k in range(len(ranges)):
+            hb.forward(k)
+            assert hb.block_stash_bytes == 0 and (hb.block_logits_bytes > 0) == logits
+            hb.backward(k, g_lp, g_en)
+        return hb.logprobs, hb.entropy, hb.d_hidden, hb.d_weight
+
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a, b) and a.float().norm() > 0
+
+
+def test_block_logits_are_recomputed_where_there_is_no_memory_or_no_kernel_for_them(monkeypatch):
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(301, 128, 1000, seed=2))
+    make = lambda h, w_, **kw: _ops.HeadBlocks(h, w_, lab, 1.0, [(0, 256), (256, 301)], logits=True, **kw)  # noqa: E731
+    need = make(hid, w, stash=False).stash_bytes
+    assert need == 4 * 262144  # four vocabulary tiles, one token tile
+    assert make(hid, w, stash=[False, True]).keeps_logits == [True, True]
+    assert make(hid[:, :96].contiguous(), w[:, :96].contiguous(), stash=False).stash is None  # hidden % 64 == 32
+    real = torch.empty
+
+    def short(*a, **k):
+        if a == (need,):
+            raise torch.OutOfMemoryError("no room")
+        return real(*a, **k)
+
+    monkeypatch.setattr(torch, "empty", short)
+    hb = make(hid, w, stash=False)
+    assert hb.stash is None and hb.stash_bytes == 0
+    hb.forward(0)
+    assert hb.block_logits_bytes == 0

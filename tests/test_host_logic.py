@@ -67,6 +67,21 @@ def test_whole_call_head_refuses_a_stash_for_shapes_it_keeps_none_for():
     assert lib.axon_lmhead_bwd(p, None, p, p, p, 0, p, p, *shape, None, p, p, 0, p, big, p, big, None) == -2
 
 
+def test_block_logits_room_and_refusals():
+    """256 KB per 256 x 256 tile for the shapes of the main loop, 0 and AXON_ERR_SHAPE for others, a short buffer is
+    AXON_ERR_WORKSPACE: before anything is launched (the addresses below are never read)."""
+    lib = _lib.load()
+    assert lib.axon_lmhead_block_logits_bytes(8189, 2880, 201088) == 32 * 786 * 262144
+    assert lib.axon_lmhead_block_logits_bytes(1, 64, 1) == 262144
+    assert lib.axon_lmhead_block_logits_bytes(513, 96, 1500) == 0 and lib.axon_lmhead_block_logits_bytes(16, 100, 50) == -1
+    p, big = 1 << 20, 1 << 40
+    for h, keep, want in ((96, big, -2), (128, 3 * 6 * 262144 - 1, -3)):
+        shape = (513, h, 1500, 1.0, 0.0, None, 0)
+        assert lib.axon_lmhead_block_fwd_logits(p, p, p, 0, *shape, p, p, p, p, p, big, p, keep, None, None) == want
+        assert lib.axon_lmhead_block_bwd_logits(p, None, p, p, p, 0, p, p, *shape, p, p, None, 0, 1, 0, 1, 513, 0,
+                                                p, big, p, keep, None, None) == want
+
+
 def test_cpu_tensors_fail_loudly():
     x = torch.zeros(2, 4)
     with pytest.raises(_lib.AxonAmdError, match="no CPU fallback"):
