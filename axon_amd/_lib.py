@@ -71,6 +71,7 @@ SIGNATURES: dict[str, tuple] = {
     "axon_logits_fwd": (_i32, [_ptr, _i32, _i64, _i64, _i64, _ptr, _i32, _ptr, _ptr, _ptr, _ptr]),
     "axon_logits_fwd_workspace_bytes": (_i64, [_i32, _i64, _i64]),
     "axon_logits_fwd_ws": (_i32, [_ptr, _i32, _i64, _i64, _i64, _ptr, _i32, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "axon_logits_fwd_train": (_i32, [_ptr, _i32, _i64, _i64, _i64, _ptr, _i32, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "axon_logits_bwd": (_i32, [_ptr, _i32, _i64, _i64, _i64, _ptr, _i32, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
     "axon_reverse_scan": (_i32, [_i32, _ptr, _ptr, _ptr, _i32, _ptr, _i64, _i64, _i64, _f32, _f32, _ptr, _ptr, _ptr,
                                  _ptr]),

@@ -1069,8 +1069,9 @@ def _logits_operands(what, logits, labels):
     return n, v, int(logits.stride(0)) if n > 1 else v
 
 
-def logits_forward(logits, labels=None, want_entropy=True):
-    """``(logprob | None, entropy | None, lse)`` fp32 [tokens] from materialised logits; see axon_logits_fwd."""
+def logits_forward(logits, labels=None, want_entropy=True, backward_follows=False):
+    """``(logprob | None, entropy | None, lse)`` fp32 [tokens] from materialised logits; see axon_logits_fwd and,
+    for ``backward_follows``, axon_logits_fwd_train."""
     lib = _lib.load()
     require_device(logits, "logits_forward")
     n, v, ld = _logits_operands("logits_forward", logits, labels)
@@ -1079,11 +1080,11 @@ def logits_forward(logits, labels=None, want_entropy=True):
     ws_bytes = lib.axon_logits_fwd_workspace_bytes(_LOGITS_DTYPES[logits.dtype], n, v) if v > 0 else 0
     ws = torch.empty(ws_bytes // 4, device=dev, dtype=torch.float32) if ws_bytes > 0 else None
     base = out.data_ptr()
+    fwd = lib.axon_logits_fwd_train if backward_follows else lib.axon_logits_fwd_ws
     check(
-        lib.axon_logits_fwd_ws(ptr(logits), _LOGITS_DTYPES[logits.dtype], ld, n, v, ptr(labels),
-                               int(labels is not None and labels.dtype == torch.int64),
-                               base if labels is not None else None, base + 4 * n if want_entropy else None,
-                               base + 8 * n, ptr(ws), stream_ptr()),
+        fwd(ptr(logits), _LOGITS_DTYPES[logits.dtype], ld, n, v, ptr(labels),
+            int(labels is not None and labels.dtype == torch.int64), base if labels is not None else None,
+            base + 4 * n if want_entropy else None, base + 8 * n, ptr(ws), stream_ptr()),
         "axon_logits_fwd_ws",
     )
     lp, ent, lse = out.unbind(0)

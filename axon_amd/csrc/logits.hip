@@ -4,6 +4,7 @@
 // more read and one write (in place when asked to).  HBM-bound: 2 or 4 bytes per logit forward, twice that
 // plus the write backward.
 #include "common.h"
+#include <type_traits>
 
 namespace axon {
 
@@ -25,8 +26,11 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16(float lo, float hi) {
 template <typename T> struct Row;
 template <> struct Row<float> {
   static constexpr int kPer = 4;
+  // CACHED: the vector stays in the caches behind (plain load) instead of passing them by
+  template <bool CACHED = false>
   __device__ static void load(const float* p, float (&v)[8]) {
-    const f32x4 x = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+    const f32x4* const q = reinterpret_cast<const f32x4*>(p);
+    const f32x4 x = CACHED ? *q : __builtin_nontemporal_load(q);
     v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
   }
   __device__ static float one(const float* p) { return *p; }
@@ -38,8 +42,10 @@ template <> struct Row<float> {
 };
 template <> struct Row<unsigned short> {
   static constexpr int kPer = 8;
+  template <bool CACHED = false>
   __device__ static void load(const unsigned short* p, float (&v)[8]) {
-    const u16x8 x = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(p));
+    const u16x8* const q = reinterpret_cast<const u16x8*>(p);
+    const u16x8 x = CACHED ? *q : __builtin_nontemporal_load(q);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = bf16_to_f32(x[j]);
   }
@@ -130,11 +136,14 @@ __device__ __forceinline__ void write_stats(Stats st, int t, const T* row, int v
 // Workgroup (part, row): blockIdx.x = row * parts + part.  One part writes the row's results, several leave their
 // statistics in ws[row][part][3] for logits_merge_kernel.  Bound by memory, 6.0 to 6.6 TB/s from 1100 rows on.
 // 2047 x 50257 bf16 39 us for 81 (rows off a 16-byte boundary), 187 x 151936 bf16 20 for 31, 300 x 151936 fp32 32 for 58.
+// Rows from `cached_from` on are left in the 256 MB cache in front of the memory, for the backward to find: a
+// non-temporal load does not allocate there.  The rows before them, which would be evicted again, pass it by (all
+// rows cached: 116 us for 106 at 2047 x 151936 bf16, for the lines that are written back to make room).
 template <typename T, typename LabelT>
 __global__ __launch_bounds__(kBlock) void logits_stats_kernel(
     const T* __restrict__ logits, int64_t ld, int vocab, const LabelT* __restrict__ labels,
     float* __restrict__ logprob, float* __restrict__ entropy, float* __restrict__ lse, int parts,
-    float* __restrict__ ws) {
+    float* __restrict__ ws, int cached_from) {
   __shared__ float red[3][kBlock / kWave];
   const int t = blockIdx.x / parts, part = blockIdx.x - t * parts;
   const T* row = logits + (int64_t)t * ld;
@@ -142,19 +151,23 @@ __global__ __launch_bounds__(kBlock) void logits_stats_kernel(
   const RowSpan sp(row, vocab, true, part, parts);
   Stats st{kFloor, 0.f, 0.f};
   const T* body = row + sp.head;
-  int q = sp.q_lo + threadIdx.x;
-  for (; q + kBlock < sp.q_hi; q += 2 * kBlock) {  // two loads in flight per thread
-    float v0[8], v1[8];
-    Row<T>::load(body + (uint32_t)q * kPer, v0);
-    Row<T>::load(body + (uint32_t)(q + kBlock) * kPer, v1);
-    fold<kPer>(st, v0);
-    fold<kPer>(st, v1);
-  }
-  for (; q < sp.q_hi; q += kBlock) {
-    float v[8];
-    Row<T>::load(body + (uint32_t)q * kPer, v);
-    fold<kPer>(st, v);
-  }
+  auto walk = [&](auto cached) {
+    constexpr bool kCached = decltype(cached)::value;
+    int q = sp.q_lo + threadIdx.x;
+    for (; q + kBlock < sp.q_hi; q += 2 * kBlock) {  // two loads in flight per thread
+      float v0[8], v1[8];
+      Row<T>::template load<kCached>(body + (uint32_t)q * kPer, v0);
+      Row<T>::template load<kCached>(body + (uint32_t)(q + kBlock) * kPer, v1);
+      fold<kPer>(st, v0);
+      fold<kPer>(st, v1);
+    }
+    for (; q < sp.q_hi; q += kBlock) {
+      float v[8];
+      Row<T>::template load<kCached>(body + (uint32_t)q * kPer, v);
+      fold<kPer>(st, v);
+    }
+  };
+  if (t >= cached_from) walk(std::true_type{}); else walk(std::false_type{});
   for (int i = part * kBlock + threadIdx.x; i < sp.n_scalar; i += parts * kBlock) {
     const float v[8] = {Row<T>::one(row + sp.scalar<T>(i))};
     fold<1>(st, v);
@@ -207,8 +220,9 @@ __global__ __launch_bounds__(kWave) void logits_merge_kernel(
 // dlogits[j] = g_lp (onehot_j - p_j) - g_ent p_j (log p_j + H),  p_j = exp(z_j - lse).
 // dlogits may be the logits' own storage: every element is read before it is written by the same thread.
 // Rows, and the vectors of a row, are walked from the last to the first: the end of what the forward read last is
-// still in the 256 MB cache in front of the memory.  Bound by memory (read + write 5.1 TB/s, a device copy 5.3): 2047 x 151936
-// bf16 244 us for 250; where a short batch is split into parts 32 x 151936 takes 9.3 us for 53, 187 x 151936 24 for 78;
+// still in the 256 MB cache in front of the memory (its cached_from), and the loads and stores here, which pass that
+// cache by, leave it there until it is read.  Bound by memory: 2047 x 151936 bf16 208 us for 247 with a forward that
+// leaves nothing, 4096 x 50257 151 for 186, 1600 x 151936 fp32 355 for 404; where a short batch is split into parts 32 x 151936 takes 9.3 us for 53, 187 x 151936 24 for 78;
 // rows of an odd vocabulary, read from their first 16-byte boundary on, 2047 x 50257 bf16 93 us for 166.
 template <typename T, typename LabelT>
 __global__ __launch_bounds__(kBlock) void logits_grad_kernel(
@@ -289,6 +303,11 @@ int fwd_parts(int64_t n, int64_t vocab, int elem_bytes) {
   return vocab * elem_bytes < 131072 ? 1 : row_parts(n, vocab, elem_bytes);
 }
 
+// How much of the rows a forward leaves in the cache in front of the memory for its backward: the size of that cache.
+// Forward + backward at 2047 x 151936 bf16: 354 us with nothing, 333 with 128 MB, 323 with 192, 316 with 224, 314 with
+// 256, 321 with 400; 4096 x 50257 (411 MB) 263, 246, 240, 233, 231, 232; a backward that does not come costs up to 2 us.
+constexpr int64_t kCacheBytes = int64_t(256) << 20;
+
 // every row of b sits on the same offset from a 16-byte boundary as the row of a
 bool same_offsets(const void* a, int64_t ld_a, const void* b, int64_t ld_b, int64_t n, int elem_bytes) {
   const uintptr_t d = reinterpret_cast<uintptr_t>(a) ^ reinterpret_cast<uintptr_t>(b);
@@ -311,9 +330,9 @@ extern "C" int64_t axon_logits_fwd_workspace_bytes(int dtype, int64_t n, int64_t
   return parts > 1 ? n * parts * 3 * (int64_t)sizeof(float) : 0;
 }
 
-extern "C" int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
-                                  const void* labels, int labels_i64, float* logprob, float* entropy,
-                                  float* lse, float* workspace, void* stream) {
+static int logits_fwd(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab, const void* labels,
+                      int labels_i64, float* logprob, float* entropy, float* lse, float* workspace, bool bwd_follows,
+                      void* stream) {
   int rc = check_logits(logits, dtype, ld, n, vocab);
   if (rc != AXON_OK) return rc;
   if (n == 0) return AXON_OK;
@@ -321,11 +340,13 @@ extern "C" int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int
   const hipStream_t st = (hipStream_t)stream;
   const int eb = dtype == AXON_LOGITS_F32 ? 4 : 2;
   const int parts = workspace ? fwd_parts(n, vocab, eb) : 1;
+  const int64_t cached = bwd_follows ? kCacheBytes / (vocab * eb) : 0;
+  const int cached_from = (int)(cached < n ? n - cached : 0);
   const dim3 grid((unsigned)(n * parts)), blk(kBlock);
 #define AXON_STATS(T, L)                                                                               \
   do {                                                                                                 \
     hipLaunchKernelGGL((logits_stats_kernel<T, L>), grid, blk, 0, st, static_cast<const T*>(logits), ld, \
-                       (int)vocab, static_cast<const L*>(labels), logprob, entropy, lse, parts, workspace); \
+                       (int)vocab, static_cast<const L*>(labels), logprob, entropy, lse, parts, workspace, cached_from); \
     if (parts > 1)                                                                                     \
       hipLaunchKernelGGL((logits_merge_kernel<T, L>), dim3((unsigned)n), dim3(kWave), 0, st, workspace, parts, \
                          static_cast<const T*>(logits), ld, (int)vocab, static_cast<const L*>(labels), \
@@ -339,6 +360,18 @@ extern "C" int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int
 #undef AXON_STATS
   AXON_CHECK_LAUNCH();
   return AXON_OK;
+}
+
+extern "C" int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
+                                  const void* labels, int labels_i64, float* logprob, float* entropy,
+                                  float* lse, float* workspace, void* stream) {
+  return logits_fwd(logits, dtype, ld, n, vocab, labels, labels_i64, logprob, entropy, lse, workspace, false, stream);
+}
+
+extern "C" int axon_logits_fwd_train(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
+                                     const void* labels, int labels_i64, float* logprob, float* entropy,
+                                     float* lse, float* workspace, void* stream) {
+  return logits_fwd(logits, dtype, ld, n, vocab, labels, labels_i64, logprob, entropy, lse, workspace, true, stream);
 }
 
 extern "C" int axon_logits_fwd(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,

@@ -31,7 +31,7 @@ class _LogitsHead(torch.autograd.Function):
     def forward(ctx, logits, labels, want_entropy, inplace_backward):
         flat = _rows(logits)
         lab = labels.reshape(-1).contiguous() if labels is not None else None
-        logprob, entropy, lse = _ops.logits_forward(flat, lab, want_entropy)
+        logprob, entropy, lse = _ops.logits_forward(flat, lab, want_entropy, ctx.needs_input_grad[0])
         ctx.save_for_backward(flat, lab, lse, entropy)
         ctx.shape = logits.shape
         # writing the gradient over the logits is only possible when `flat` is the caller's storage

@@ -580,6 +580,11 @@ int64_t axon_logits_fwd_workspace_bytes(int dtype, int64_t n, int64_t vocab);
 int axon_logits_fwd_ws(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
                        const void* labels, int labels_are_i64, float* logprob, float* entropy, float* lse,
                        float* workspace, void* stream);
+/* axon_logits_fwd_ws for a caller whose backward follows: the same results, and the rows read last stay in the cache
+ * in front of the memory, where axon_logits_bwd begins. */
+int axon_logits_fwd_train(const void* logits, int dtype, int64_t ld, int64_t n, int64_t vocab,
+                          const void* labels, int labels_are_i64, float* logprob, float* entropy, float* lse,
+                          float* workspace, void* stream);
 
 /* Backward of the above in one read and one write of the rows:
  *   dlogits[t][j] = g_logprob[t] (onehot - p) - g_entropy[t] p (log p + entropy[t]),  p = exp(logits - lse)

@@ -594,6 +594,17 @@ def test_logits_rows_in_parts_and_on_any_boundary(n, v, cut, dtype):
     assert torch.equal(_ops.logits_backward(over, labels, lse, en, g_lp, g_en, inplace=True), grad)
 
 
+@pytest.mark.parametrize("n,v,dtype", [(1100, 131072, torch.bfloat16), (3, 999, torch.float32), (40, 70001, torch.float32),
+                                       (1025, 65537, torch.float32)])
+def test_logits_forward_with_a_backward_to_come(n, v, dtype):
+    """Rows that are left in the cache for the backward (all, or those after the first ones of a batch beyond 256 MB) give
+    the same results as rows that are not."""
+    x = torch.randn(n, v, generator=torch.Generator(device=DEV).manual_seed(v), device=DEV, dtype=dtype)
+    labels = torch.arange(n, device=DEV) % v
+    for a, b in zip(_ops.logits_forward(x, labels, True, True), _ops.logits_forward(x, labels)):
+        assert torch.equal(a, b) and torch.isfinite(a).all()
+
+
 def test_logits_path_inplace_backward_shapes_and_strides():
     from axon_amd.utils.torch.ops import entropy_from_logits_with_chunking, logprobs_from_logits
     g = torch.Generator().manual_seed(5)
