@@ -425,10 +425,6 @@ __device__ __forceinline__ int stage_off(int nw, int unit) {
   return nw * 256 + ((pu ^ ((nw & 31) ^ (nw >> 5))) << 3);
 }
 
-// SOFTCAP: the recomputed logit goes through cap * tanh(. / cap) and the gradient is multiplied by
-// the derivative 1 - tanh^2 (fused_linear.py:80-83).
-// Accumulators -> bf16 dlogits in the wave's staging area.  MASKED: the tile reaches past the last
-// token or the last vocabulary row; those entries are written as zeros.
 // Per-token factors of dlogit = softmax * (ca + cb * logit) + onehot * gl for tile-relative token
 // row nr; lab_rel is the label's row inside the tile whose first vocabulary row is m0_abs (-1: not
 // in this tile).
@@ -436,6 +432,7 @@ struct TokenCoef {
   float ca, cb, gl, lse2;
   int lab_rel, nn;
   bool n_ok;
+  TokenCoef() = default;
   __device__ __forceinline__ TokenCoef(const DlogitParams& p, int n, int64_t m0_abs) {
     n_ok = n < p.n_tokens;
     nn = n_ok ? n : 0;
@@ -455,7 +452,9 @@ struct TokenCoef {
   }
 };
 
-// The dlogit of one logit (the accumulator, before temperature and soft-capping), row mrel of the tile.
+// The dlogit of one logit (the accumulator, before temperature and soft-capping), row mrel of the tile.  SOFTCAP:
+// the logit goes through cap * tanh(. / cap) and the gradient is multiplied by the derivative 1 - tanh^2
+// (fused_linear.py:80-83).
 template <bool SOFTCAP>
 __device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef& k, const DlogitParams& p, float c) {
   float dcap = 1.f;
@@ -471,28 +470,51 @@ __device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef&
   return v;
 }
 
+// Accumulators -> bf16 dlogits, token-major to dl through the wave's staging area, where they stay for the
+// vocab-major copy.  MASKED: the tile reaches past the last token or the last vocabulary row; those entries are
+// written as zeros.  Sixteen tokens at a time, and all tokens' scalars requested before the first: the main loop ends for
+// all workgroups of the chip at about the same time, so that this is a burst of 33 MB of stores, which the arithmetic
+// of the next sixteen tokens now runs under (whole sub-tile first, then its copy: 6007 x 896 x 151936 1.98 ms for
+// 1.79, 3001 x 1024 x 50257 0.408 for 0.380, 8192 x 4096 x 151936 7.43 for 7.27).
 template <bool SOFTCAP, bool MASKED>
-__device__ __forceinline__ void dlogit_stage(AccTile& acc, const DlogitParams& p, const LanePos& lp,
+__device__ __forceinline__ void dlogit_store(AccTile& acc, const DlogitParams& p, const LanePos& lp,
                                              const TilePos& t, char* stage) {
   const float c = p.inv_temp * kLog2e;
+  const int l32 = lp.lane & 31, lhi = lp.lane >> 5;
+  const int n_wave = t.n0 + lp.wn * kWaveTile;
+  // token-major: 32 lanes cover one 256-byte row of the sub-tile, two rows per store
+  char* d = reinterpret_cast<char*>(p.dl + (int64_t)(n_wave + lhi) * p.ld_dl + t.m0 + lp.wm * kWaveTile + l32 * 4);
+  const int64_t dstep = p.ld_dl * 4;  // two rows of bf16
+  TokenCoef k[kBlocks];
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j) k[j] = TokenCoef(p, n_wave + j * kBlk + lp.l16, (int64_t)p.v_begin + t.m0);
 #pragma unroll
   for (int j = 0; j < kBlocks; ++j) {
     const int nw = j * kBlk + lp.l16;  // token row inside the wave's sub-tile
-    const TokenCoef k(p, t.n0 + lp.wn * kWaveTile + nw, (int64_t)p.v_begin + t.m0);
-    const int m_end = MASKED ? (k.n_ok ? p.vocab - p.v_begin - t.m0 : 0) : kTile;  // rows that count
+    const int m_end = MASKED ? (k[j].n_ok ? p.vocab - p.v_begin - t.m0 : 0) : kTile;  // rows that count
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
-      float d[4];
+      float v[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int mrel = lp.m(i, r);
-        const float v = dlogit_of<SOFTCAP>(acc[i][j][r], mrel, k, p, c);
-        d[r] = (!MASKED || mrel < m_end) ? v : 0.f;
+        const float x = dlogit_of<SOFTCAP>(acc[i][j][r], mrel, k[j], p, c);
+        v[r] = (!MASKED || mrel < m_end) ? x : 0.f;
       }
       uint2 w;
-      w.x = pack_bf16(d[0], d[1]);
-      w.y = pack_bf16(d[2], d[3]);
+      w.x = pack_bf16(v[0], v[1]);
+      w.y = pack_bf16(v[2], v[3]);
       *reinterpret_cast<uint2*>(stage + stage_off(nw, i * 4 + lp.lq)) = w;
+    }
+    // these sixteen tokens are complete: their rows leave while the next sixteen are computed
+    uint2 o[kBlocks];
+#pragma unroll
+    for (int u = 0; u < kBlocks; ++u)
+      o[u] = *reinterpret_cast<const uint2*>(stage + stage_off(j * kBlk + 2 * u + lhi, l32));
+#pragma unroll
+    for (int u = 0; u < kBlocks; ++u) {
+      *reinterpret_cast<uint2*>(d) = o[u];
+      d += dstep;
     }
   }
 }
@@ -546,7 +568,7 @@ __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashH
   }
 }
 
-// The same from the logits that a forward kept (kKeepLogits): the arithmetic of dlogit_stage on what the
+// The same from the logits that a forward kept (kKeepLogits): the arithmetic of dlogit_store on what the
 // accumulators held.
 template <bool SOFTCAP, bool EDGE>
 __device__ __forceinline__ void dlogit_stage_logits(const float4 (&x)[kStashHalfBlocks * kBlocks], int j0,
@@ -578,7 +600,7 @@ __device__ __forceinline__ void dlogit_stage_logits(const float4 (&x)[kStashHalf
 }
 
 // A staged 64 x 128 half sub-tile (tokens 16 * j0 .. of the wavefront's sub-tile) -> dl and dlT.  Token-major
-// as in dlogit_copy_out (below); vocab-major: sixteen lanes cover the 64 tokens of one vocabulary row (one
+// 32 lanes cover one 256-byte row, eight rows per trip (reads before writes); vocab-major: sixteen lanes cover the 64 tokens of one vocabulary row (one
 // 128-byte line), the four lane groups take units u, u + 8, u + 16, u + 24, whose permuted slots differ in
 // a bit that the rows' swizzles (a set with that bit fixed) cannot cancel.
 __device__ __forceinline__ void dlogit_copy_out_half(const char* stage, int j0, const DlogitParams& p,
@@ -622,31 +644,13 @@ __device__ __forceinline__ void dlogit_copy_out_half(const char* stage, int j0, 
   }
 }
 
-// The wave's staged 128 x 128 bf16 sub-tile -> dl (token-major) and dlT (vocab-major).  The wave
+// The wave's staged 128 x 128 bf16 sub-tile -> dlT (vocab-major), where it is wanted.  The wave
 // reads back only what it wrote itself; LDS operations of one wave complete in order.
-__device__ __forceinline__ void dlogit_copy_out(const char* stage, const DlogitParams& p,
-                                                const LanePos& lp, const TilePos& t) {
+__device__ __forceinline__ void dlogit_copy_out_vocab(const char* stage, const DlogitParams& p,
+                                                      const LanePos& lp, const TilePos& t) {
   const int l32 = lp.lane & 31, lhi = lp.lane >> 5;
   const int m_base = t.m0 + lp.wm * kWaveTile;  // chunk-relative column of the sub-tile
   const int n_base = t.n0 + lp.wn * kWaveTile;
-  // token-major copy: 32 lanes cover one 256-byte row.  Eight rows per trip, reads before writes;
-  // destinations by running pointers (no 64-bit multiplies in the loop).
-  {
-    const int unit = l32;
-    char* d = reinterpret_cast<char*>(p.dl + (int64_t)(n_base + lhi) * p.ld_dl + m_base + unit * 4);
-    const int64_t dstep = p.ld_dl * 4;  // two rows of bf16
-#pragma unroll 1
-    for (int nw0 = lhi; nw0 < kWaveTile; nw0 += 16) {
-      uint2 v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const uint2*>(stage + stage_off(nw0 + 2 * u, unit));
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        *reinterpret_cast<uint2*>(d) = v[u];
-        d += dstep;
-      }
-    }
-  }
   // vocab-major copy: 4x4 blocks transposed in registers; 32 lanes cover 128 tokens of one vocab row
   if (p.dlT) {
     const int nq = l32;  // token quad
@@ -681,10 +685,10 @@ __device__ __forceinline__ void dlogit_body(const GemmOperands& g, const DlogitP
   const LanePos lp;
   char* const stage = smem + lp.wave * 32768;
   if (t.n0 + kTile > p.n_tokens || p.v_begin + t.m0 + kTile > p.vocab)
-    dlogit_stage<SOFTCAP, true>(acc, p, lp, t, stage);
+    dlogit_store<SOFTCAP, true>(acc, p, lp, t, stage);
   else
-    dlogit_stage<SOFTCAP, false>(acc, p, lp, t, stage);
-  dlogit_copy_out(stage, p, lp, t);
+    dlogit_store<SOFTCAP, false>(acc, p, lp, t, stage);
+  dlogit_copy_out_vocab(stage, p, lp, t);
 }
 
 template <class Loop>
