@@ -85,16 +85,20 @@ struct LanePos {
     wm = wave >> 1;
     wn = wave & 1;
   }
-  // tile-relative coordinates of accumulator (i, j, r)
-  __device__ __forceinline__ int m(int i, int r) const { return wm * kWaveTile + i * kBlk + 4 * lq + r; }
+  // tile-relative coordinates of accumulator (i, j, r); BM: block rows per wave
+  template <int BM = kBlocks>
+  __device__ __forceinline__ int m(int i, int r) const { return (wm * BM + i) * kBlk + 4 * lq + r; }
   __device__ __forceinline__ int n(int j) const { return wn * kWaveTile + j * kBlk + l16; }
 };
 
-typedef acc4 AccTile[kBlocks][kBlocks];
+template <int BM>
+using AccTileOf = acc4[BM][kBlocks];
+typedef AccTileOf<kBlocks> AccTile;
 
-__device__ __forceinline__ void zero_acc(AccTile& acc) {
+template <int BM>
+__device__ __forceinline__ void zero_acc(AccTileOf<BM>& acc) {
 #pragma unroll
-  for (int i = 0; i < kBlocks; ++i)
+  for (int i = 0; i < BM; ++i)
 #pragma unroll
     for (int j = 0; j < kBlocks; ++j)
 #pragma unroll
@@ -131,11 +135,11 @@ __device__ __forceinline__ void settle_acc() { asm volatile("s_nop 15\n\ts_nop 1
 typedef __attribute__((ext_vector_type(4))) short i16x4;
 typedef __attribute__((ext_vector_type(8))) short i16x8;
 
-// What the loop needs to know of one operand side.  T: the operand is K-major.
-template <bool T>
+// What the loop needs to know of one operand side.  T: the operand is K-major.  B: blocks per wave on this side.
+template <bool T, int B = kBlocks>
 struct DmaSide {
   static constexpr int kVariants = T ? 4 : 2;
-  static constexpr int kFrag = T ? kBlocks : 2;
+  static constexpr int kFrag = T ? B : 2;
   int vo[kVariants];   // per-lane source byte offset of a DMA instruction, by variant(j)
   int step;            // source bytes from DMA instruction j to j + 1
   int64_t kt_bytes;    // source bytes from one k-tile to the next
@@ -151,7 +155,7 @@ struct DmaSide {
 
   __device__ static __forceinline__ int variant(int j) { return T ? (j & 1) + 2 * (j >> 2) : (j & 1); }
 
-  // `row0`: first tile row (m0 or n0); `sub`: which half of the tile the wave computes (wm or wn);
+  // `row0`: first tile row (m0 or n0); `sub`: which half of the tile's rows the wave computes (wm or wn);
   // `lds_base`: where the operand's first slot begins.  It is part of the per-lane fragment offsets so that
   // what is left to add per read (the slot: a scalar; block, k-step, half: constants) fits the 16-bit offset
   // field of the LDS instructions: a constant beyond it costs a vector addition right before the read that
@@ -171,13 +175,16 @@ struct DmaSide {
       step = (int)ld * 16;
       kt_bytes = 128;
       base = p + (int64_t)row0 * ld;
-      rec = rec_last = min(rows - row0, kTile) * (int)ld * 2;
-      // fragment addressing: row = 128*sub + 16*i + l16, chunk = 4*kk + lq, swizzle = (l16/2)%8.
+      // (0 rows: the half of an edge tile that lies beyond the matrix.  A clamp on both sides is one vector instruction
+      // to the compiler, and a descriptor that passes through a vector register costs a loop around every DMA
+      // instruction: hence the scalar read.)
+      rec = rec_last = __builtin_amdgcn_readfirstlane(max(min(rows - row0, kTile), 0)) * (int)ld * 2;
+      // fragment addressing: row = 16*(B*sub + i) + l16, chunk = 4*kk + lq, swizzle = (l16/2)%8.
       // Sixteen lanes (one chunk column of sixteen rows) cover all 64 banks once.
       const int sw = (lp.l16 >> 1) & 7;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
-        frag[kk] = lds_base + (sub * kWaveTile + lp.l16) * 128 + (((kk * 4 + lp.lq) ^ sw) << 4);
+        frag[kk] = lds_base + (sub * B * kBlk + lp.l16) * 128 + (((kk * 4 + lp.lq) ^ sw) << 4);
     } else {
       // One DMA instruction fills 1 KB of LDS = 2 k-rows x 512 B; wave w owns k-rows [16w, 16w+16) of
       // the k-tile (8 instructions).  Lane i lands on k-row 2j + i/32, 16-byte granule i%32, and fetches
@@ -195,12 +202,11 @@ struct DmaSide {
       rec = (int)ld * 128;
       rec_last = ((k - 1) & 63) * (int)ld * 2 + (rows - row0 + 7) / 8 * 16;
       // fragment of block i, k-step kk, half h: k-row 32kk + 8lq + 4h + l16/4, elements
-      // 128*sub + 16i + 4*(l16%4) ..+3: granule 16*sub + 2i + (l16%4)/2, second half of it for odd l16.
-      const int s15 = (2 * (lp.l16 >> 2) + 8 * lp.lq) & 15;
-      const int fb = (8 * lp.lq + (lp.l16 >> 2)) * 512 + (((16 * sub) ^ (16 * (lp.lq >> 1))) << 4) +
-                     8 * (lp.l16 & 1) + (((lp.l16 & 3) >> 1) << 4);
+      // 16*(B*sub + i) + 4*(l16%4) ..+3: granule 2*(B*sub + i) + (l16%4)/2, second half of it for odd l16.
+      const int sw = 2 * (lp.l16 >> 2) + 8 * lp.lq;
+      const int fb = lds_base + (8 * lp.lq + (lp.l16 >> 2)) * 512 + 8 * (lp.l16 & 1) + (((lp.l16 & 3) >> 1) << 4);
 #pragma unroll
-      for (int i = 0; i < kBlocks; ++i) frag[i] = lds_base + fb + ((i << 5) ^ (s15 << 4));
+      for (int i = 0; i < B; ++i) frag[i] = fb + (((2 * (B * sub + i)) ^ sw) << 4);
     }
   }
   // k-tile kt as a descriptor; past the end: the last tile again, never consumed
@@ -214,8 +220,15 @@ struct DmaSide {
 };
 
 // kNarrow: the K-major A operand's rows are shorter than 512 bytes (see dma_kb).
-template <bool kAT, bool kBT, bool kNarrow = false>
+// BM: block rows per wave.  8 is the whole 256 x 256 tile; 4 computes its first 128 rows (64 per wave, half the matrix
+// instructions per k-tile) with the same slots and the same DMA instructions, of which those for the other rows
+// fetch nothing on a K-contiguous side (the descriptor ends): for the last tile of an m that fills at most half of it, and for
+// the tail of a walk whose tiles are halved to spread them over the compute units.
+template <bool kAT, bool kBT, bool kNarrow = false, int BM = kBlocks>
 struct DmaLoopT {
+  static_assert(BM == kBlocks || BM == kBlocks / 2, "");
+  typedef DmaLoopT<kAT, kBT, kNarrow, kBlocks / 2> Half;
+  static constexpr int kRows = 2 * BM * kBlk;  // tile rows computed
   static constexpr int kBK = 64;
   static constexpr bool kAMajor = kAT, kBMajor = kBT;
   static constexpr int kRowBytes = 128;
@@ -268,23 +281,23 @@ struct DmaLoopT {
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   }
 
-  __device__ static __forceinline__ void run(const GemmOperands& g, const TilePos& t, AccTile& acc,
+  __device__ static __forceinline__ void run(const GemmOperands& g, const TilePos& t, AccTileOf<BM>& acc,
                                              char* smem) {
     const LanePos lp;
-    DmaSide<kAT> sa;
+    DmaSide<kAT, BM> sa;
     DmaSide<kBT> sb;
-    sa.init(g.a, g.lda, g.m_rows, g.k, t.m0, lp.wm, lp, 0);
+    sa.init(g.a, g.lda, BM < kBlocks ? min(g.m_rows, t.m0 + kRows) : g.m_rows, g.k, t.m0, lp.wm, lp, 0);
     sb.init(g.b, g.ldb, g.n_rows, g.k, t.n0, lp.wn, lp, kBBase);
     // wave-uniform, so the LDS destination of every DMA instruction is scalar arithmetic into M0
     char* const dst = smem + __builtin_amdgcn_readfirstlane(lp.wave) * 8192;
 
-    zero_acc(acc);
+    zero_acc<BM>(acc);
     // fragments of two k-steps: whole (one 16-byte read) or as the two halves of a transpose read
-    bf16x8 af[2][kBlocks], bf[2][kBlocks];
-    i16x4 aft[2][kBlocks][2], bft[2][kBlocks][2];
+    bf16x8 af[2][BM], bf[2][kBlocks];
+    i16x4 aft[2][BM][2], bft[2][kBlocks][2];
     const int kt_n = (g.k + kBK - 1) / kBK;
     auto dma_a = [&](int slot_off, const __amdgpu_buffer_rsrc_t& r, int j) {
-      dma_kb(r, sa.vo[DmaSide<kAT>::variant(j)], sa.step, dst + slot_off, j);
+      dma_kb(r, sa.vo[DmaSide<kAT, BM>::variant(j)], sa.step, dst + slot_off, j);
     };
     auto dma_b = [&](int slot_off, const __amdgpu_buffer_rsrc_t& r, int j) {
       dma_kb(r, sb.vo[DmaSide<kBT>::variant(j)], sb.step, dst + kBBase + slot_off, j);
@@ -294,10 +307,15 @@ struct DmaLoopT {
     // behind the pair; sixteen such pairs per k-tile cost 3-4 % of the loop).  The reads under a tile's second
     // k-step (k-step 0 of the next tile) and under the next tile's first k-step (its k-step 1) go to the same
     // slots, so the addresses change once per k-tile: after the last read of a tile's first k-step.
-    constexpr int kAddrA = DmaSide<kAT>::kFrag, kAddrB = DmaSide<kBT>::kFrag;
+    constexpr int kAddrA = DmaSide<kAT, BM>::kFrag, kAddrB = DmaSide<kBT>::kFrag;
+    // The schedule of a k-step: its MFMAs, one DMA instruction every kDmaGap of them, the fragment reads one per two
+    // MFMAs (BM 4: in every MFMA gap without a DMA instruction), then the address additions, kAdrPer to a gap.
+    constexpr bool kWhole = BM == kBlocks;
+    constexpr int kMfmas = BM * kBlocks, kDmaGap = kMfmas / 8, kReads = BM * kReadsA + kBlocks * kReadsB;
+    constexpr int kFirstAdr = kWhole ? 2 * kReads : (4 * kReads + 2) / 3, kAdrPer = kWhole ? 1 : 2;
     // room for the additions behind the reads of a k-step (not with both operands K-major, whose reads fill it:
     // that form, which no kernel of the library uses, forms them in one piece after the barrier)
-    constexpr bool kLateAdr = 2 * kBlocks * (kReadsA + kReadsB) + kAddrA + kAddrB <= kBlocks * kBlocks;
+    constexpr bool kLateAdr = kFirstAdr + (kAddrA + kAddrB + kAdrPer - 1) / kAdrPer <= kMfmas;
     typedef __attribute__((address_space(3))) const char* LdsPtr;
     const uint32_t smem_lds = (uint32_t)(uintptr_t)(LdsPtr)smem;
     uint32_t adr_a[kAddrA], adr_b[kAddrB];
@@ -326,36 +344,38 @@ struct DmaLoopT {
       constexpr bool kAdr = decltype(adr_c)::value != 0;
       static_assert((NA == 0 || NA == 8) && (NB == 0 || NB == 8) && NA + NB <= 8, "");
       constexpr int RA = kReadsA, RB = kReadsB;
-      constexpr int kFirstAdr = 2 * kBlocks * (RA + RB);  // the MFMA after the last read
       static_assert(!kAdr || kLateAdr, "");
       const int rd_set = mm_set ^ 1;
 #pragma unroll
-      for (int i = 0; i < kBlocks; ++i) {
+      for (int i = 0; i < BM; ++i) {
 #pragma unroll
         for (int j = 0; j < kBlocks; ++j) {
           const int m = i * kBlocks + j;
           // scalar bookkeeping for the coming k-tile, in pieces of at most four instructions, in slots without
           // other work (a wavefront issues in order: a dozen scalar instructions in one MFMA gap hold up the
           // MFMA behind them); pieces 3 and 4 come behind the step's last DMA instruction
-          if (m == 37) mid(std::integral_constant<int, 0>{});
-          if (m == 39) mid(std::integral_constant<int, 1>{});
-          if (m == 41) mid(std::integral_constant<int, 2>{});
-          if (m == 61) mid(std::integral_constant<int, 3>{});
-          if (m == 63) mid(std::integral_constant<int, 4>{});
-          if ((m & 7) == 3) {
-            if (NB) dma_b(b_slot, rsrc, m >> 3);
-            if (NA) dma_a(a_slot, rsrc, m >> 3);
+          if (m == (kWhole ? 37 : 18)) mid(std::integral_constant<int, 0>{});
+          if (m == (kWhole ? 39 : 20)) mid(std::integral_constant<int, 1>{});
+          if (m == (kWhole ? 41 : 22)) mid(std::integral_constant<int, 2>{});
+          if (m == kMfmas - (kWhole ? 3 : 2)) mid(std::integral_constant<int, 3>{});
+          if (m == kMfmas - 1) mid(std::integral_constant<int, 4>{});
+          const bool dma_slot = (m % kDmaGap) == (kWhole ? 3 : 1);
+          if (dma_slot) {
+            if (NB) dma_b(b_slot, rsrc, m / kDmaGap);
+            if (NA) dma_a(a_slot, rsrc, m / kDmaGap);
           }
-          if ((m & 1) == 0) {
-            const int s = m >> 1;
+          if (kWhole ? (m & 1) == 0 : !dma_slot) {
+            const int s = kWhole ? m >> 1 : m - ((m + 2) >> 2);
             if (s < RA) read_a(rd_kk, rd_set, 0, s);
             else if (s < RA + kBlocks * RB) read_b(rd_kk, rd_set, (s - RA) / RB, (s - RA) % RB);
-            else if (s < kBlocks * (RA + RB))
+            else if (s < kReads)
               read_a(rd_kk, rd_set, 1 + (s - RA - kBlocks * RB) / RA, (s - RA - kBlocks * RB) % RA);
           }
-          if (kAdr && m >= kFirstAdr && m < kFirstAdr + kAddrA) set_adr_a(m - kFirstAdr, nxt_a);
-          if (kAdr && m >= kFirstAdr + kAddrA && m < kFirstAdr + kAddrA + kAddrB)
-            set_adr_b(m - kFirstAdr - kAddrA, nxt_b);
+#pragma unroll
+          for (int q = (m - kFirstAdr) * kAdrPer; q < (m - kFirstAdr + 1) * kAdrPer; ++q) {
+            if (kAdr && q >= 0 && q < kAddrA) set_adr_a(q, nxt_a);
+            if (kAdr && q >= kAddrA && q < kAddrA + kAddrB) set_adr_b(q - kAddrA, nxt_b);
+          }
           mfma_16x16x32(acc[i][j], kAT ? join(aft[mm_set][i][0], aft[mm_set][i][1]) : af[mm_set][i],
                         kBT ? join(bft[mm_set][j][0], bft[mm_set][j][1]) : bf[mm_set][j]);
           __builtin_amdgcn_sched_barrier(0);
@@ -389,7 +409,8 @@ struct DmaLoopT {
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
 #pragma unroll
-      for (int h = 0; h < kReadsA; ++h) read_a(0, 0, i, h);
+      for (int h = 0; h < kReadsA; ++h)
+        if (i < BM) read_a(0, 0, i, h);
 #pragma unroll
       for (int h = 0; h < kReadsB; ++h) read_b(0, 0, i, h);
     }
@@ -466,6 +487,7 @@ struct RegLoop {
   static_assert(BK == 32, "one 16x16x32 k-step per staged tile");
   static constexpr int kBK = BK;
   static constexpr bool kAMajor = false, kBMajor = false;
+  typedef void Half;  // whole tiles only
   static constexpr int kChunks = BK / 8;                 // 16-byte chunks per row
   static constexpr int kRowBytes = BK * 2;
   static constexpr int kRowsPerLine = 256 / kRowBytes;   // rows per 256-byte bank line
@@ -504,7 +526,7 @@ struct RegLoop {
       a_off[i] = offset(lp.wm * kWaveTile + i * kBlk + lp.l16, lp.lq);
       b_off[i] = kOperandBytes + offset(lp.wn * kWaveTile + i * kBlk + lp.l16, lp.lq);
     }
-    zero_acc(acc);
+    zero_acc<kBlocks>(acc);
 
     uint4 ra[kLoads], rb[kLoads];
     const int kt_n = g.k / BK;

@@ -44,6 +44,7 @@ struct FwdParams {
   float c;     // inv_temperature * log2(e)
   float cap, inv_cap;  // logit soft-capping cap * tanh(logit / cap) (SOFTCAP kernels only)
   uint4* stash;        // kernels that keep something for the backward: the stash or the logits, see below
+  int halved;          // the walk's last tiles that are computed in two halves of 128 vocabulary rows
 };
 // What a forward leaves for its backward beside the statistics.
 enum Keep { kKeepNone, kKeepStash, kKeepLogits };
@@ -115,40 +116,67 @@ __device__ __forceinline__ float rows_all_reduce(float v, Op op) {
   return op(c, d);
 }
 
-// Fold one 256x256 logits tile into per-token partials.  MASKED: some rows of the tile
-// lie beyond the vocabulary; they are excluded by predicate — their accumulators hold finite values.  STASH: also store every
-// 2^(y - M) for the backward (`stash_wave`: this wavefront's 32 KB, already offset by the lane).
-template <bool MASKED, bool STASH>
-__device__ __forceinline__ void fwd_epilogue(AccTile& acc, const FwdParams& p, const LanePos& lp,
-                                             const TilePos& t, int tm, uint4* stash_wave) {
-  const int part = tm * 2 + lp.wm;
-#pragma unroll
-  for (int j = 0; j < kBlocks; ++j) {
+// Fold a logits tile of 32 * BM vocabulary rows x 256 tokens into per-token partials, one per 128 rows.  BM 8: a whole
+// tile, whose wavefronts have a part each; BM 4: the half `half` of one, whose part the wavefronts 0 and 2 (1 and 3) share:
+// its maximum and its sums go through LDS, in the order in which one wavefront of a whole tile adds them up (a lane
+// adds the first four and the last four 16-row blocks apart), so that the results do not depend on how a tile was computed.
+// MASKED: some rows of the tile lie beyond the vocabulary; they are excluded by predicate — their accumulators hold finite
+// values.  STASH: also store every 2^(y - M) for the backward (`stash_wave`: the 32 KB of the part and these
+// tokens, already offset by the lane).
+template <bool MASKED, bool STASH, int BM>
+__device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams& p, const LanePos& lp,
+                                             const TilePos& t, int part, uint4* stash_wave, float* lds) {
+  constexpr bool kHalf = BM < kBlocks;
+  constexpr int kRun = kBlocks / 2;  // blocks that a lane adds up in one go
+  auto add = [](float a, float b) { return a + b; };
+  auto row_ok = [&](int i, int r) { return !MASKED || t.m0 + lp.m<BM>(i, r) < p.vocab; };
+  // the part's maximum over this wavefront's rows; the four lanes that hold the same token (lane ^ 16, lane ^ 32)
+  // share one reference
+  auto max_of = [&](int j) {
     float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i)
+    for (int i = 0; i < BM; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int mr = lp.m(i, r);
-        const bool ok = !MASKED || t.m0 + mr < p.vocab;
-        mx = ok ? fmaxf(mx, acc[i][j][r]) : mx;
-      }
-    // the four lanes that hold the same token (lane ^ 16, lane ^ 32) share one reference
-    mx = rows_all_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
+      for (int r = 0; r < 4; ++r) mx = row_ok(i, r) ? fmaxf(mx, acc[i][j][r]) : mx;
+    return rows_all_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
+  };
+  auto write = [&](int j, float M, float s, float e) {
+    s = rows_all_reduce(s, add);
+    e = rows_all_reduce(e, add);
+    const int n = t.n0 + lp.n(j);
+    if (lp.lq == 0 && n < p.n_tokens) {
+      const int64_t o = (int64_t)part * p.n_tokens + n;
+      p.pm[o] = M;
+      p.ps[o] = s;
+      p.pe[o] = e;
+    }
+  };
+  float* const mine = lds + lp.wave * 1024 + lp.lane;  // per wavefront: 8 x 64 of each of the two sums
+  const float* const other = lds + (lp.wave ^ 2) * 1024 + lp.lane;
+  float mxs[kBlocks];
+  if (kHalf) {
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j) mine[j * 64] = mxs[j] = max_of(j);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j) mxs[j] = fmaxf(mxs[j], other[j * 64]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j) {
+    const float mx = kHalf ? mxs[j] : max_of(j);
     const float M = (MASKED && mx == -INFINITY) ? kEmptyMax : mx * p.c;
-    float s = 0.f, e = 0.f;
-    uint32_t hw[kBlocks][2];
+    float s[2] = {0.f, 0.f}, e[2] = {0.f, 0.f};
+    uint32_t hw[BM][2];
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
+    for (int i = 0; i < BM; ++i) {
       float w[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int mr = lp.m(i, r);
-        const bool ok = !MASKED || t.m0 + mr < p.vocab;
         const float y = fmaf(acc[i][j][r], p.c, -M);  // scaled logit relative to the max, <= 0
-        w[r] = ok ? fast_exp2(y) : 0.f;
-        s += w[r];
-        e = fmaf(w[r], y, e);
+        w[r] = row_ok(i, r) ? fast_exp2(y) : 0.f;
+        s[i / kRun] += w[r];
+        e[i / kRun] = fmaf(w[r], y, e[i / kRun]);
       }
       if (STASH) {
         hw[i][0] = pack_f16(w[0], w[1]);
@@ -157,61 +185,87 @@ __device__ __forceinline__ void fwd_epilogue(AccTile& acc, const FwdParams& p, c
     }
     if (STASH) {
 #pragma unroll
-      for (int ip = 0; ip < kBlocks / 2; ++ip)
+      for (int ip = 0; ip < BM / 2; ++ip)
       {  // written once, read once by the backward: kept out of the way of the operand slices in L2
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
         const u32x4 x = {hw[2 * ip][0], hw[2 * ip][1], hw[2 * ip + 1][0], hw[2 * ip + 1][1]};
-        __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(stash_wave + (j * 4 + ip) * 64));
+        const int at = kHalf ? lp.wm * (BM / 2) + ip : ip;
+        __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(stash_wave + (j * 4 + at) * 64));
       }
     }
-    s = rows_all_reduce(s, [](float a, float b) { return a + b; });
-    e = rows_all_reduce(e, [](float a, float b) { return a + b; });
-    const int nr = lp.n(j);
-    const int n = t.n0 + nr;
-    if (lp.lq == 0 && n < p.n_tokens) {
-      const int64_t o = (int64_t)part * p.n_tokens + n;
-      p.pm[o] = M;
-      p.ps[o] = s;
-      p.pe[o] = e;
+    if (kHalf) {
+      mxs[j] = M;
+      mine[j * 64] = s[0];
+      mine[(kBlocks + j) * 64] = e[0];
+    } else {
+      write(j, M, s[0] + s[1], e[0] + e[1]);
+    }
+  }
+  if (kHalf) {
+    __syncthreads();
+    if (lp.wm == 0) {
+#pragma unroll
+      for (int j = 0; j < kBlocks; ++j)
+        write(j, mxs[j], mine[j * 64] + other[j * 64], mine[(kBlocks + j) * 64] + other[(kBlocks + j) * 64]);
     }
   }
 }
 
-// SOFTCAP: the logits go through cap * tanh(. / cap) before the statistics (fused_linear.py:19-23).
-template <class Loop, bool SOFTCAP, Keep KEEP>
-__device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams& p, int tiles_m,
-                                         int tiles_n) {
-  extern __shared__ __align__(16) char smem[];
-  int tm, tn;
-  tile_coords<8>(xcd_order(tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
-  const TilePos t = Loop::place(tm, tn);
-  AccTile acc;
+// One tile (BM 8), or the half `half` of one (BM 4: t.m0 is its first row).  SOFTCAP: the logits go through
+// cap * tanh(. / cap) before the statistics (fused_linear.py:19-23).
+template <class Loop, int BM, bool SOFTCAP, Keep KEEP>
+__device__ __forceinline__ void fwd_tile(const GemmOperands& g, const FwdParams& p, const TilePos& t, int tile, int part0,
+                                         int half, char* smem) {
+  constexpr bool kHalf = BM < kBlocks;
+  AccTileOf<BM> acc;
   Loop::run(g, t, acc, smem);
   const LanePos lp;
+  const int wm = kHalf ? half : lp.wm;  // the 128-row part of the tile, and with it the place of what is kept
+  const int64_t kept = (int64_t)tile * 4 + wm * 2 + lp.wn;
   if (KEEP == kKeepLogits) {  // written once, read once by the backward, long after: past the caches
-    float4* const out = reinterpret_cast<float4*>(p.stash) +
-                        ((int64_t)(tm * tiles_n + tn) * 4 + lp.wave) * kLogitsWaveVecs + lp.lane;
+    float4* const out = reinterpret_cast<float4*>(p.stash) + kept * kLogitsWaveVecs + lp.lane;
 #pragma unroll
     for (int j = 0; j < kBlocks; ++j)
 #pragma unroll
-      for (int i = 0; i < kBlocks; ++i)
-        __builtin_nontemporal_store(acc[i][j], reinterpret_cast<acc4*>(out + (j * kBlocks + i) * 64));
+      for (int i = 0; i < BM; ++i)
+        __builtin_nontemporal_store(
+            acc[i][j], reinterpret_cast<acc4*>(out + (j * kBlocks + (kHalf ? lp.wm * BM + i : i)) * 64));
   }
   if (SOFTCAP) {
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i)
+    for (int i = 0; i < BM; ++i)
 #pragma unroll
       for (int j = 0; j < kBlocks; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[i][j][r] = p.cap * fast_tanh(acc[i][j][r] * p.inv_cap);
   }
   constexpr bool STASH = KEEP == kKeepStash;
-  uint4* const stash_wave =
-      STASH ? p.stash + ((int64_t)(tm * tiles_n + tn) * 4 + lp.wave) * kStashWaveVecs + lp.lane : nullptr;
-  if (t.m0 + kTile > p.vocab)
-    fwd_epilogue<true, STASH>(acc, p, lp, t, tm, stash_wave);
+  uint4* const stash_wave = STASH ? p.stash + kept * kStashWaveVecs + lp.lane : nullptr;
+  float* const lds = reinterpret_cast<float*>(smem);
+  if (t.m0 + 2 * BM * kBlk > p.vocab)
+    fwd_epilogue<true, STASH, BM>(acc, p, lp, t, part0 + wm, stash_wave, lds);
   else
-    fwd_epilogue<false, STASH>(acc, p, lp, t, tm, stash_wave);
+    fwd_epilogue<false, STASH, BM>(acc, p, lp, t, part0 + wm, stash_wave, lds);
+}
+
+template <class Loop, bool SOFTCAP, Keep KEEP>
+__device__ __forceinline__ void fwd_body(const GemmOperands& g, const FwdParams& p, int tiles_m,
+                                         int tiles_n) {
+  extern __shared__ __align__(16) char smem[];
+  const int whole = tiles_m * tiles_n - p.halved;
+  int tm, tn;
+  if constexpr (!std::is_void_v<typename Loop::Half>) {
+    if ((int)blockIdx.x >= whole) {
+      const int h = blockIdx.x - whole;
+      tile_coords<8>(whole + (h >> 1), tiles_m, tiles_n, tm, tn);
+      TilePos t = Loop::place(tm, tn);
+      t.m0 += (h & 1) * (kTile / 2);
+      fwd_tile<typename Loop::Half, kBlocks / 2, SOFTCAP, KEEP>(g, p, t, tm * tiles_n + tn, tm * 2, h & 1, smem);
+      return;
+    }
+  }
+  tile_coords<8>(xcd_order(whole), tiles_m, tiles_n, tm, tn);
+  fwd_tile<Loop, kBlocks, SOFTCAP, KEEP>(g, p, Loop::place(tm, tn), tm * tiles_n + tn, tm * 2, 0, smem);
 }
 
 template <class Loop>
@@ -1116,12 +1170,14 @@ int set_lds(K kernel) {
 }
 
 // Launch kernel<DmaLoop> or kernel<SlowLoop> over all tiles of the problem.
-#define AXON_LAUNCH_GEMM(KERNEL, G, P, ST)                                                        \
+#define AXON_LAUNCH_GEMM(KERNEL, G, P, ST) AXON_LAUNCH_GEMM_PLUS(KERNEL, G, P, ST, 0)
+// with EXTRA workgroups more than tiles where the fast loop is taken
+#define AXON_LAUNCH_GEMM_PLUS(KERNEL, G, P, ST, EXTRA)                                            \
   do {                                                                                            \
     const int tiles_m_ = ((G).m_rows + kTile - 1) / kTile, tiles_n_ = ((G).n_rows + kTile - 1) / kTile; \
     if (dma_ok(G)) {                                                                              \
       if (set_lds(KERNEL<DmaLoop>) != AXON_OK) return AXON_ERR_LAUNCH;                            \
-      hipLaunchKernelGGL(KERNEL<DmaLoop>, dim3(tiles_m_ * tiles_n_), dim3(kGemmThreads),          \
+      hipLaunchKernelGGL(KERNEL<DmaLoop>, dim3(tiles_m_ * tiles_n_ + (EXTRA)), dim3(kGemmThreads), \
                          kGemmLdsBytes, ST, G, P, tiles_m_, tiles_n_);                            \
     } else {                                                                                      \
       if (set_lds(KERNEL<SlowLoop>) != AXON_OK) return AXON_ERR_LAUNCH;                           \
@@ -1388,13 +1444,22 @@ int launch_transpose(const void* in, int64_t ld_in, int rows, int cols, void* ou
   return AXON_OK;
 }
 
+// The forward's tiles that are computed in halves of 128 vocabulary rows: those of a last round that would occupy at
+// most half of the compute units, so that it takes half as long.  594 tiles, 2.3 rounds: 187 tokens x 896 x 151936 87 us
+// for 80, 187 x 4096 305 for 288; 128 tiles (250 x 2048 x 32768) 44 for 35.  A last round over more than half of
+// them would become two.
+int halved_tiles(int64_t n, int64_t v) {
+  const int64_t tiles = (round_up(v, kTile) / kTile) * (round_up(n, kTile) / kTile), rest = tiles % kCus;
+  return rest <= kCus / 2 ? (int)rest : 0;
+}
+
 template <bool SOFTCAP>
 int launch_fwd_logits(const GemmOperands& g, const FwdParams& p, hipStream_t st) {
   const int tiles_m = (g.m_rows + kTile - 1) / kTile, tiles_n = (g.n_rows + kTile - 1) / kTile;
   if (!dma_ok(g)) return AXON_ERR_SHAPE;
   if (set_lds(lmhead_fwd_logits_kernel<SOFTCAP>) != AXON_OK) return AXON_ERR_LAUNCH;
-  hipLaunchKernelGGL(lmhead_fwd_logits_kernel<SOFTCAP>, dim3(tiles_m * tiles_n), dim3(kGemmThreads), kGemmLdsBytes, st,
-                     g, p, tiles_m, tiles_n);
+  hipLaunchKernelGGL(lmhead_fwd_logits_kernel<SOFTCAP>, dim3(tiles_m * tiles_n + p.halved), dim3(kGemmThreads),
+                     kGemmLdsBytes, st, g, p, tiles_m, tiles_n);
   AXON_CHECK_LAUNCH();
   return AXON_OK;
 }
@@ -1437,7 +1502,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
   g.b = static_cast<const __bf16*>(hidden);  g.ldb = h;  g.n_rows = (int)n;
   g.k = (int)h;
   FwdParams p{w.pm, w.ps, w.pe, (int)n, (int)v, inv_temp * kLog2e, softcap,
-              softcap > 0.f ? 1.f / softcap : 0.f, sw.tiles};
+              softcap > 0.f ? 1.f / softcap : 0.f, sw.tiles, dma_ok(g) ? halved_tiles(n, v) : 0};
   {
     Span span(timer, 0);
     if (stash && keep == kKeepLogits) {
@@ -1445,13 +1510,13 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
       if (rc != AXON_OK) return rc;
     } else if (stash) {
       if (softcap > 0.f)
-        AXON_LAUNCH_GEMM(lmhead_fwd_softcap_stash_kernel, g, p, st);
+        AXON_LAUNCH_GEMM_PLUS(lmhead_fwd_softcap_stash_kernel, g, p, st, p.halved);
       else
-        AXON_LAUNCH_GEMM(lmhead_fwd_stash_kernel, g, p, st);
+        AXON_LAUNCH_GEMM_PLUS(lmhead_fwd_stash_kernel, g, p, st, p.halved);
     } else if (softcap > 0.f) {
-      AXON_LAUNCH_GEMM(lmhead_fwd_softcap_kernel, g, p, st);
+      AXON_LAUNCH_GEMM_PLUS(lmhead_fwd_softcap_kernel, g, p, st, p.halved);
     } else {
-      AXON_LAUNCH_GEMM(lmhead_fwd_kernel, g, p, st);
+      AXON_LAUNCH_GEMM_PLUS(lmhead_fwd_kernel, g, p, st, p.halved);
     }
   }
   Span span(timer, 1);

@@ -37,9 +37,9 @@ DEFAULT_DW_GROUP = 2
 # The blocks without a stash (blocks_with_stash) keep their fp32 logits from the forward to the backward, 4 bytes x
 # block x vocab, where the product that recomputes them costs more than writing and reading them: its time grows
 # with the hidden size, the traffic does not.  Head forward + backward of 6007 tokens x 151936, recomputed / kept:
-# hidden 256 2.85 / 3.01 ms, 512 4.00 / 3.83, 896 6.02 / 5.73; 8189 x 2880 x 201088 26.9 / 22.7, 8189 x 4096 x 151936
-# 27.3 / 22.3.
-KEEP_LOGITS_MIN_HIDDEN = 512
+# hidden 256 2.75 / 3.01 ms, 512 3.84 / 3.87, 768 5.05 / 4.97, 896 5.92 / 5.78; x 50257 1024 2.27 / 2.13; 8189 x 2880 x
+# 201088 26.9 / 22.7, 8189 x 4096 x 151936 27.1 / 22.3.
+KEEP_LOGITS_MIN_HIDDEN = 768
 _TILE = 256
 
 

@@ -1053,3 +1053,31 @@ def test_block_logits_are_recomputed_where_there_is_no_memory_or_no_kernel_for_t
     assert hb.stash is None and hb.stash_bytes == 0
     hb.forward(0)
     assert hb.block_logits_bytes == 0
+
+
+@pytest.mark.parametrize("h,v,cap", [(64, 25600, 0.0), (128, 99 * 256 + 1, 0.0), (192, 99 * 256 + 129, 5.0), (64, 256 * 356 - 3, 0.0)])
+def test_tiles_computed_in_halves_give_the_bits_of_whole_ones(h, v, cap):
+    """A forward of 200 tokens computes its last round of 100 vocabulary tiles in halves, one of 512 tokens (200 or 712
+    tiles) whole tiles: the statistics of the shared tokens are equal bit for bit, at vocabularies that end with
+    a tile's first row, in its second half and three rows before its end.  What a block keeps for its backward lies where a
+    whole tile leaves it: kept logits give the recompute's bits, the stash its gradients to the stash's rounding."""
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(512, h, v, seed=h))
+    w = (w.float() * 6).bfloat16()
+    lab[7], lab[11] = v - 1, v - v % 256 if v % 256 else 0
+    few, many = (_ops.lmhead_forward(hid[:n], w, lab[:n], 1.0, softcap=cap) for n in (200, 512))
+    for a, b in zip(few, many):
+        assert torch.equal(a, b[:200]) and torch.isfinite(a).all()
+    g_lp, g_en = torch.randn(2, 204, generator=torch.Generator().manual_seed(v)).to(DEV)
+
+    def run(**keep):
+        hb = _ops.HeadBlocks(hid[:200], w, lab[:200], 1.0, [(0, 200)], softcap=cap, **keep)
+        hb.forward(0)
+        hb.backward(0, g_lp, g_en)
+        return hb.logprobs, hb.entropy, hb.d_hidden, hb.d_weight
+
+    again = run(stash=False)
+    for a, b in zip(run(stash=False, logits=True), again):
+        assert torch.equal(a, b) and a.float().norm() > 0
+    lp, ent, dh, dw = run(stash=True)
+    assert torch.equal(lp, again[0]) and torch.equal(ent, again[1])
+    assert rel_l2(dh, again[2]) < 5e-3 and rel_l2(dw, again[3]) < 5e-3
