@@ -228,6 +228,7 @@ template <bool kAT, bool kBT, bool kNarrow = false, int BM = kBlocks>
 struct DmaLoopT {
   static_assert(BM == kBlocks || BM == kBlocks / 2, "");
   typedef DmaLoopT<kAT, kBT, kNarrow, kBlocks / 2> Half;
+  typedef std::conditional_t<kAT != kBT && !kNarrow, Half, void> HalfEdge;  // for the forms of the output products
   static constexpr int kRows = 2 * BM * kBlk;  // tile rows computed
   static constexpr int kBK = 64;
   static constexpr bool kAMajor = kAT, kBMajor = kBT;
@@ -487,7 +488,7 @@ struct RegLoop {
   static_assert(BK == 32, "one 16x16x32 k-step per staged tile");
   static constexpr int kBK = BK;
   static constexpr bool kAMajor = false, kBMajor = false;
-  typedef void Half;  // whole tiles only
+  typedef void Half, HalfEdge;  // whole tiles only
   static constexpr int kChunks = BK / 8;                 // 16-byte chunks per row
   static constexpr int kRowBytes = BK * 2;
   static constexpr int kRowsPerLine = 256 / kRowBytes;   // rows per 256-byte bank line

@@ -848,32 +848,44 @@ struct StoreParams {
   // Split reduction: `splits` workgroups per tile, each over `k_split` (a multiple of 64) of the k; they leave their
   // partial sums in tile_acc, one array of tiles after the other, for split_sum_kernel.
   int splits, k_split;
+  // The last tile of an m that fills at most half of it is computed as half a tile (DmaLoopT's BM).  Its rows lie in
+  // tile_acc where a whole tile leaves them, the other half of the tile is left as it was.
+  int half_edge;
 };
 constexpr int64_t kTileAccVecs = 4 * kBlocks * kBlocks * 64;  // float4 per tile (256 KB)
 
-template <class Loop>
-__global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g, StoreParams p,
-                                                                  int tiles_m, int tiles_n) {
-  extern __shared__ __align__(16) char smem[];
-  int tm, tn;
-  const int tiles = tiles_m * tiles_n;
-  const int pid = xcd_order(tiles * p.splits);
-  const int split = pid / tiles;  // the tiles of one part of k side by side: they share operand slices
-  tile_coords(pid - split * tiles, tiles_m, tiles_n, tm, tn);
-  const int64_t k0 = (int64_t)split * p.k_split;
-  g.a += Loop::kAMajor ? k0 * g.lda : k0;
-  g.b += Loop::kBMajor ? k0 * g.ldb : k0;
-  g.k = min(g.k - (int)k0, p.k_split);
-  const TilePos t = Loop::place(tm, tn);
-  AccTile acc;
+// U rows of staged bf16 values, kStep apart, to out_bf16: 16 bytes per lane and row.
+template <int U, int kStep>
+__device__ __forceinline__ void store_rows(const StoreParams& p, const char* stage, int row, int unit, int n, int m) {
+  uint2 v[U][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      v[u][q] = *reinterpret_cast<const uint2*>(stage + stage_off(row + kStep * u, unit + q));
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (n + kStep * u >= p.n_valid) continue;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 x = {v[u][0].x, v[u][0].y, v[u][1].x, v[u][1].y};  // read by nobody soon
+    __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(p.out_bf16 + (int64_t)(n + kStep * u) * p.ld_bf16 + m));
+  }
+}
+
+template <class Loop, int BM>
+__device__ __forceinline__ void store_tile(const GemmOperands& g, const StoreParams& p, const TilePos& t, int64_t tile,
+                                           char* smem) {
+  constexpr bool kHalf = BM < kBlocks;
+  AccTileOf<BM> acc;
   Loop::run(g, t, acc, smem);
   const LanePos lp;
   if (p.tile_acc) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     f32x4* ta = reinterpret_cast<f32x4*>(p.tile_acc) +
-                (((int64_t)split * tiles + tm * tiles_n + tn) * 4 + lp.wave) * (kBlocks * kBlocks * 64) + lp.lane;
+                (tile * 4 + (kHalf ? lp.wn : lp.wave)) * (kBlocks * kBlocks * 64) +
+                (kHalf ? lp.wm * BM * kBlocks * 64 : 0) + lp.lane;
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
+    for (int i = 0; i < BM; ++i) {
       f32x4 old[kBlocks];
       if (p.accumulate) {
 #pragma unroll
@@ -898,8 +910,8 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
       const int n = t.n0 + lp.n(j);
       if (n >= p.n_valid) continue;
 #pragma unroll
-      for (int i = 0; i < kBlocks; ++i) {
-        const int m = t.m0 + lp.m(i, 0);
+      for (int i = 0; i < BM; ++i) {
+        const int m = t.m0 + lp.m<BM>(i, 0);
         if (m >= p.m_valid) continue;  // m_valid % 4 == 0: a quad is all in or all out
         *reinterpret_cast<float4*>(p.out_f32 + (int64_t)n * p.ld_f32 + m) =
             make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
@@ -916,34 +928,50 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g
 #pragma unroll
   for (int j = 0; j < kBlocks; ++j)
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
+    for (int i = 0; i < BM; ++i) {
       uint2 w;
       w.x = pack_bf16(acc[i][j][0], acc[i][j][1]);
       w.y = pack_bf16(acc[i][j][2], acc[i][j][3]);
       *reinterpret_cast<uint2*>(stage + stage_off(j * kBlk + lp.l16, i * 4 + lp.lq)) = w;
     }
+  if (kHalf) {  // 64 values of m per wavefront: eight rows of 128 contiguous bytes per store instruction
+    const int row0 = lp.lane >> 3, col = lp.lane & 7, m = t.m0 + lp.wm * BM * kBlk + col * 8;
+    if (m >= p.m_valid) return;
+#pragma unroll 1
+    for (int r64 = 0; r64 < kWaveTile; r64 += 64)
+      store_rows<8, 8>(p, stage, r64 + row0, 2 * col, t.n0 + lp.wn * kWaveTile + r64 + row0, m);
+    return;
+  }
   const int m = t.m0 + lp.wm * kWaveTile + lp.l16 * 8;
   if (m >= p.m_valid) return;  // m_valid % 8 == 0: a vector of eight is all in or all out
-  const int row0 = (lp.lane >> 5) + 16 * (lp.lq & 1), n0 = t.n0 + lp.wn * kWaveTile + row0;
+  const int row0 = (lp.lane >> 5) + 16 * (lp.lq & 1);
 #pragma unroll 1
-  for (int r32 = 0; r32 < kWaveTile; r32 += 32) {
-    uint2 v[8][2];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        v[u][q] = *reinterpret_cast<const uint2*>(stage + stage_off(r32 + 2 * u + row0, 2 * lp.l16 + q));
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int n = n0 + r32 + 2 * u;
-      if (n < p.n_valid)
-        {  // read by nobody soon
-          typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-          const u32x4 x = {v[u][0].x, v[u][0].y, v[u][1].x, v[u][1].y};
-          __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(p.out_bf16 + (int64_t)n * p.ld_bf16 + m));
-        }
+  for (int r32 = 0; r32 < kWaveTile; r32 += 32)
+    store_rows<8, 2>(p, stage, r32 + row0, 2 * lp.l16, t.n0 + lp.wn * kWaveTile + r32 + row0, m);
+}
+
+template <class Loop>
+__global__ __launch_bounds__(kGemmThreads) void gemm_store_kernel(GemmOperands g, StoreParams p,
+                                                                  int tiles_m, int tiles_n) {
+  extern __shared__ __align__(16) char smem[];
+  int tm, tn;
+  const int tiles = tiles_m * tiles_n;
+  const int pid = xcd_order(tiles * p.splits);
+  const int split = pid / tiles;  // the tiles of one part of k side by side: they share operand slices
+  tile_coords(pid - split * tiles, tiles_m, tiles_n, tm, tn);
+  const int64_t k0 = (int64_t)split * p.k_split;
+  g.a += Loop::kAMajor ? k0 * g.lda : k0;
+  g.b += Loop::kBMajor ? k0 * g.ldb : k0;
+  g.k = min(g.k - (int)k0, p.k_split);
+  const TilePos t = Loop::place(tm, tn);
+  const int64_t tile = (int64_t)split * tiles + tm * tiles_n + tn;
+  if constexpr (!std::is_void_v<typename Loop::HalfEdge>) {
+    if (p.half_edge && t.m0 + kTile / 2 >= p.m_valid) {
+      store_tile<typename Loop::HalfEdge, kBlocks / 2>(g, p, t, tile, smem);
+      return;
     }
   }
+  store_tile<Loop, kBlocks>(g, p, t, tile, smem);
 }
 
 // out[n][m] = the sum over the parts of a split reduction, rounded to bf16: a streaming kernel, one thread per
@@ -953,6 +981,10 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float4* __restrict
                                                         __bf16* __restrict__ out, int64_t ld) {
   const int64_t stride = (int64_t)tiles_m * tiles_n * kTileAccVecs;
   const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;  // lane, then block (i, j), wavefront, tile
+  const int lane = (int)(q & 63), ij = (int)(q >> 6) & 63, wave = (int)(q >> 12) & 3, tile = (int)(q >> 14);
+  const int m = (tile / tiles_n) * kTile + (wave >> 1) * kWaveTile + (ij >> 3) * kBlk + 4 * (lane >> 4);
+  const int n = (tile % tiles_n) * kTile + (wave & 1) * kWaveTile + (ij & 7) * kBlk + (lane & 15);
+  if (m >= m_valid || n >= n_valid) return;
   const float4* src = parts + q;
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
   int s = 0;
@@ -967,10 +999,6 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float4* __restrict
     const float4 x = src[s * stride];
     v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
   }
-  const int lane = (int)(q & 63), ij = (int)(q >> 6) & 63, wave = (int)(q >> 12) & 3, tile = (int)(q >> 14);
-  const int m = (tile / tiles_n) * kTile + (wave >> 1) * kWaveTile + (ij >> 3) * kBlk + 4 * (lane >> 4);
-  const int n = (tile % tiles_n) * kTile + (wave & 1) * kWaveTile + (ij & 7) * kBlk + (lane & 15);
-  if (m >= m_valid || n >= n_valid) return;
   uint2 w;
   w.x = pack_bf16(v.x, v.y);
   w.y = pack_bf16(v.z, v.w);
@@ -1266,6 +1294,16 @@ SplitPlan split_plan(int64_t tiles, int64_t k) {
   }
   return best;
 }
+
+// Whether the half-filled last tiles of an output product are computed as half tiles.  What that saves falls with the
+// number of tiles beside them; what it costs grows with the reduction: a half tile runs ahead of the whole ones, with which
+// it no longer shares operand slices in the L2 (dWeight more than dHidden, whose parts keep an XCD on one part of k).
+// Whole / half, ms: dWeight hidden 896 (4 tiles) 3001 tokens (47 k-tiles) 0.671 / 0.611, 8192 1.67 / 1.58, 12288 2.53 / 2.45,
+// 16381 3.42 / 3.47; hidden 2880 (12 tiles) 700 tokens 0.847 / 0.789, 3001 2.60 / 2.57, 6007 4.92 / 4.96, 16381
+// 13.1 / 13.9.  dHidden 896 6007 tokens (297 k-tiles) 1.25 / 1.16, 16381 (792) 3.13 / 2.99; 2880 3001 tokens (629) 2.56 / 2.53,
+// 8192 (1571) 6.56 / 6.57, 16381 (3142) 13.0 / 13.2.
+constexpr int64_t kHalfEdgeDw = 768, kHalfEdgeDh = 12288;  // most k-tiles times tiles
+bool half_edge(int64_t k, int64_t tiles_m, int64_t most) { return (k + 63) / 64 * tiles_m <= most; }
 
 struct BwdWs {
   __bf16 *hT, *dl, *dlT;
@@ -1656,6 +1694,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       sp.m_valid = (int)h; sp.n_valid = (int)n;
       sp.tile_acc = (w.chunks > 1 || split) ? w.dh_acc : nullptr;
       sp.accumulate = (ci > 0); sp.keep_f32 = split || !last;
+      sp.half_edge = half_edge(sp.k_split, tiles_h, kHalfEdgeDh);
       // a shorter last chunk reaches the first parts only
       sp.k_split = plan.k_split;
       sp.splits = (int)((vc + sp.k_split - 1) / sp.k_split);
@@ -1689,6 +1728,8 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       sp.accumulate = blk.dw_mode == kDwAdd || blk.dw_mode == kDwLast;
       sp.keep_f32 = blk.dw_mode != kDwLast;
       sp.splits = 1; sp.k_split = g.k;
+      sp.half_edge = blk.dw_mode == kDwStore &&  // the carried sums hold whole tiles
+                     half_edge(g.k, tiles_h, kHalfEdgeDw);
       rc = launch_store_kmajor(g, sp, false, w.dl_kmajor, st);
       if (rc != AXON_OK) return rc;
     }
@@ -1878,7 +1919,7 @@ extern "C" int axon_gemm_nt_bf16(const void* a, int64_t lda, const void* b, int6
   StoreParams sp;
   sp.out_f32 = out; sp.ld_f32 = ldo; sp.out_bf16 = nullptr; sp.ld_bf16 = 0;
   sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 0; sp.tile_acc = nullptr;
-  sp.splits = 1; sp.k_split = (int)k;
+  sp.splits = 1; sp.k_split = (int)k; sp.half_edge = 0;
   return launch_store(g, sp, (hipStream_t)stream);
 }
 
@@ -1903,7 +1944,7 @@ extern "C" int axon_gemm_bf16(const void* a, int64_t lda, int a_kmajor, const vo
   StoreParams sp;
   sp.out_f32 = out; sp.ld_f32 = ldo; sp.out_bf16 = nullptr; sp.ld_bf16 = 0;
   sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 0; sp.tile_acc = nullptr;
-  sp.splits = 1; sp.k_split = (int)k;
+  sp.splits = 1; sp.k_split = (int)k; sp.half_edge = 0;
   return launch_store_kmajor(g, sp, a_kmajor != 0, b_kmajor != 0, (hipStream_t)stream);
 }
 

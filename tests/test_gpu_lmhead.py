@@ -1081,3 +1081,23 @@ def test_tiles_computed_in_halves_give_the_bits_of_whole_ones(h, v, cap):
     lp, ent, dh, dw = run(stash=True)
     assert torch.equal(lp, again[0]) and torch.equal(ent, again[1])
     assert rel_l2(dh, again[2]) < 5e-3 and rel_l2(dw, again[3]) < 5e-3
+
+
+@pytest.mark.parametrize("h", [288, 320, 384, 416, 640])
+@pytest.mark.parametrize("n,v,chunk", [(300, 8200, 0), (70, 1000, 512), (520, 777, 0)])
+def test_output_products_with_a_half_filled_last_tile(n, h, v, chunk):
+    """hidden sizes whose last 256-row tile holds 32, 64, 128 (half a tile each), 160 (a whole one) and 128 rows: the
+    reduction over the vocabulary in parts, carried over vocabulary chunks, and in one piece; the dlogits read as they
+    lie and (vocabulary of 777) from their vocab-major copy.  Every column against the oracle: a column beyond a
+    half tile's reach, or one that was never written, is off by its whole size."""
+    hid, w, lab = W.lmhead_inputs(n, h, v, seed=h + v)
+    w = (w.float() * 8).bfloat16()
+    g_lp, g_en = torch.randn(2, n, generator=torch.Generator().manual_seed(h))
+    hd, wd, ld = hid.to(DEV), w.to(DEV), lab.to(DEV)
+    _, _, lse, eb = _ops.lmhead_forward(hd, wd, ld, 1.0)[:4]
+    dh, dw = _ops.lmhead_backward(g_lp.to(DEV), g_en.to(DEV), hd, wd, ld, lse, eb, 1.0, vocab_chunk=chunk)
+    ref_dh, ref_dw = OM.backward(g_lp, g_en, hid, w, lab)
+    for a, ref in ((dh, ref_dh), (dw, ref_dw)):
+        err, size = (a.cpu().double() - ref.double()).norm(dim=0), ref.double().norm(dim=0)
+        # bf16 dlogits and bf16 results: 2^-9 each, and both norms over at least 70 entries of a column
+        assert (err < 2e-2 * size).all(), (err / size).max()
