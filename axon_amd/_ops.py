@@ -400,8 +400,9 @@ def _count_dev(x, dev, n=None, what="count"):
 
 def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, rows: Rows, *, token_reduce,
                 batch_reduce, ratio_lo, ratio_hi, clip_c, per_row_token_count=None, num_program_tokens=None,
-                num_program_steps=None, valid_count=None):
-    """Forward + gradient of the clipped policy loss.  Returns (acc[8], grad like log_probs).
+                num_program_steps=None, valid_count=None, acc=None):
+    """Forward + gradient of the clipped policy loss.  Returns (acc[8], grad like log_probs); ``acc``: where the
+    eight sums go (zeros when there are no slots), else a tensor of its own.
 
     acc[0] is the loss; acc[1:5] are the metric sums; acc[5] is the factor the returned
     gradient still has to be multiplied by (see axon_policy_loss).
@@ -418,7 +419,8 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
 
     valid = _count_dev(valid_count, dev)
     grad = torch.empty(rows.shape, device=dev, dtype=torch.float32)
-    acc = _acc8(rows.n_slots, dev)
+    if acc is None:
+        acc = _acc8(rows.n_slots, dev)
     # PPO with sum / token-mean needs no per-row quantity: one pass over the tokens, the
     # division by the token count happens when the last workgroup has the total.
     one_pass = kind != 1 and tr == 0 and br == 0

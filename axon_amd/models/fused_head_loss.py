@@ -127,7 +127,9 @@ class _BlockedHeadLoss(torch.autograd.Function):
         side = spec["side"]
         cu, cu_host, seq_mode = spec["cu"], spec["cu_host"], spec["seq_mode"]
 
-        if seq_mode:
+        if seq_mode and cu_host is None:  # one block
+            ranges = slots = [(0, n)]
+        elif seq_mode:
             row_blocks = spec["row_blocks"]
             ranges = slots = [(cu_host[r0], cu_host[r1]) for r0, r1 in row_blocks]  # a block's sequences
         else:
@@ -161,6 +163,8 @@ class _BlockedHeadLoss(torch.autograd.Function):
             scalars = [sums[:5].double(), side_sums[:5].double()]
             if spec.get("after_forward") is not None:  # more scalars from the whole-stream outputs (device tensors)
                 scalars += [t.double().reshape(-1) for t in spec["after_forward"](hb.logprobs, hb.entropy)]
+            if seq_mode and cu_host is None:  # the offsets' ends, checked when the step's scalars are read
+                scalars += [cu[:1].double(), cu[-1:].double()]
             spec["readback"] = _start_readback(torch.cat(scalars))
             out.update(loss=loss, sums=sums, side_sums=side_sums)
 
@@ -219,6 +223,11 @@ class _BlockedHeadLoss(torch.autograd.Function):
         return d_hidden, d_weight, None
 
 
+def _check_span(first, last, n):
+    if first != 0 or last != n:
+        raise ValueError(f"fused head loss: cu_seqlens spans {int(first)}..{int(last)}, the batch has {n} tokens")
+
+
 def blocked_spec(hidden, weight, packed_ids, cu_seqlens, data, loss_fn, loss_fn_args, temperature, *,
                  block_tokens=DEFAULT_BLOCK_TOKENS, vocab_chunk=0, dw_group=DEFAULT_DW_GROUP, logit_softcapping=None,
                  side_mask=None, cu_host=None):
@@ -247,13 +256,15 @@ def blocked_spec(hidden, weight, packed_ids, cu_seqlens, data, loss_fn, loss_fn_
     if seq_mode:
         if hp["token_reduce"] == "mean-norm":
             return None  # divides by the padded row length: not a packed-layout reduction
-        host = cu_host if cu_host is not None else cu.tolist()  # one readback: where the sequences end
-        if host[0] != 0 or host[-1] != n:
-            raise ValueError(f"fused head loss: cu_seqlens spans {host[0]}..{host[-1]}, the batch has {n} tokens")
-        spec["cu_host"] = host
-        spec["row_blocks"] = sequence_blocks(host, int(block_tokens))
-        if spec["row_blocks"] is None:
-            return None
+        if cu_host is None and n <= int(block_tokens) and rows_all.n_rows > 0:
+            spec["row_blocks"] = [(0, rows_all.n_rows)]  # one block, wherever the sequences end: nothing to read back
+        else:
+            host = cu_host if cu_host is not None else cu.tolist()  # one readback: where the sequences end
+            _check_span(host[0], host[-1], n)
+            spec["cu_host"] = host
+            spec["row_blocks"] = sequence_blocks(host, int(block_tokens))
+            if spec["row_blocks"] is None:
+                return None
     mask = tensors["response_mask"]
     spec["hp"]["valid_count"] = _global_count(mask, rows_all, hp["batch_reduce"], hp["valid_count"])
     if side_mask is not None:
@@ -293,13 +304,23 @@ def fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, *,
     ``data`` gets ``head_backward`` ("blocked-stash" or "recompute"), and for the blocked path ``stash_bytes``,
     ``head_workspace_bytes``, ``n_blocks`` and ``dw_group`` (blocks per weight-gradient GEMM).
 
-    ``cu_host``: the same offsets as a Python list, for a caller that has them (saves the one readback that the
-    sequence-cut blocks need)."""
+    ``cu_host``: the same offsets as a Python list, for a caller that has them (saves the one readback that
+    sequence-cut blocks need where a batch has several).
+
+    The host waits for the GPU once, for the step's scalars, while the last block's backward runs: the sums of the sampler
+    correction arrive with them, and nothing between them waits (waiting for the correction first left the GPU idle until
+    the host had enqueued the rest)."""
+    return _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, block_tokens, vocab_chunk, dw_group,
+                            logit_softcapping, cu_host)
+
+
+def _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, block_tokens, vocab_chunk, dw_group,
+                     logit_softcapping, cu_host, correct=True):
     from axon_amd.models.fsdp_models import loss_from_outputs
     from axon_amd.trainer.algos.loss.registry import _SAMPLER_SWITCHES
     from axon_amd.utils.fsdp.forward_utils import packed_logprobs
     from axon_amd.utils.rl.sampler import (compute_sampler_correction_and_add_to_batch, sampler_gap_metrics,
-                                           sampler_gap_sums)
+                                           sampler_gap_sums, start_sampler_correction)
 
     loss_fn = meta_info["loss_fn"]
     loss_fn_args = meta_info["loss_fn_args"] or {}
@@ -315,10 +336,12 @@ def fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, *,
     side_mask = b["response_mask"]  # before the correction can replace it
     spec = None
     if loss_fn in POLICY_LOSS_KINDS and hidden2.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
-        corr_metrics = {}
-        wanted = any(loss_fn_args.get(k, None) is not None for k in _SAMPLER_SWITCHES)
+        corr_metrics, in_flight = {}, None
+        wanted = correct and any(loss_fn_args.get(k, None) is not None for k in _SAMPLER_SWITCHES)
         if wanted and "sampler_log_probs" in b:
-            data, corr_metrics = compute_sampler_correction_and_add_to_batch(data, loss_fn_args)
+            in_flight = start_sampler_correction(data, loss_fn_args, readback=True)
+            if in_flight is None:
+                data, corr_metrics = compute_sampler_correction_and_add_to_batch(data, loss_fn_args)
             b = data.batch
         spec = blocked_spec(hidden2, weight, packed_ids, cu_seqlens, data, loss_fn, loss_fn_args, temperature,
                             block_tokens=block_tokens, vocab_chunk=vocab_chunk, dw_group=dw_group,
@@ -343,6 +366,16 @@ def fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, *,
     host, event = spec["readback"]  # the one readback of the step's scalars, started before the last block's backward
     event.synchronize()
     vals = host.tolist()
+    if spec["seq_mode"] and spec["cu_host"] is None:
+        _check_span(vals[-2], vals[-1], int(hidden2.shape[0]))
+    if in_flight is not None:
+        corr_metrics = in_flight.metrics()
+        if corr_metrics is None:  # no token to correct, and the batch is as it was
+            corr_metrics = {}
+            # weights under an all-zero mask change nothing, unless they are NaN: without them then
+            if not vals[0] == 0.0:
+                return _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, block_tokens, vocab_chunk,
+                                        dw_group, logit_softcapping, cu_host, correct=False)
     metrics = {**policy_loss_metrics(spec["kind"], vals[:5]), **corr_metrics}
     if sampler_log_prob is not None:
         metrics.update(sampler_gap_metrics(vals[10:], int(cu_seqlens.numel()) - 1))

@@ -138,41 +138,43 @@ POLICY_LOSS_KINDS = {"ppo": (_KIND_PPO, "sum"), "gspo": (_KIND_GSPO, "mean"), "r
                      "gpg": (_KIND_REINFORCE, "sum"), "cispo": (_KIND_CISPO, "sum")}
 
 
-def _run(kind: int, data, config, default_token_reduce: str):
+def _run(kind: int, data, config, default_token_reduce: str, corr=None):
     log_probs, rows, tensors, hp = policy_loss_spec(kind, data, config, default_token_reduce)
+    if corr is not None:
+        hp["acc"] = corr.loss_acc
     loss, acc = _ClippedPolicyLoss.apply(log_probs, kind, tensors, rows, hp)
-    sums = acc.tolist()  # the only host sync of the loss
+    sums = acc.tolist() if corr is None else corr.read()  # the only host sync of the loss
     return loss, policy_loss_metrics(kind, sums)
 
 
 @register_loss(LossFn.PPO)
-def ppo_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
+def ppo_loss_fn(data, config, corr=None) -> tuple[torch.Tensor, dict[str, Any]]:
     """Clipped PPO surrogate with dual clip (loss.py:47-111); defaults sum / token-mean."""
-    return _run(_KIND_PPO, data, config, "sum")
+    return _run(_KIND_PPO, data, config, "sum", corr)
 
 
 @register_loss(LossFn.GSPO)
-def gspo_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
+def gspo_loss_fn(data, config, corr=None) -> tuple[torch.Tensor, dict[str, Any]]:
     """GSPO sequence-level ratio loss (loss.py:114-180); code defaults mean / token-mean (:165-166)."""
-    return _run(_KIND_GSPO, data, config, "mean")
+    return _run(_KIND_GSPO, data, config, "mean", corr)
 
 
 @register_loss(LossFn.REINFORCE)
-def reinforce_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
+def reinforce_loss_fn(data, config, corr=None) -> tuple[torch.Tensor, dict[str, Any]]:
     """``-log_prob * A`` (times the sampler weights when present), loss.py:471-512; sum / token-mean."""
-    return _run(_KIND_REINFORCE, data, config, "sum")
+    return _run(_KIND_REINFORCE, data, config, "sum", corr)
 
 
 @register_loss(LossFn.GPG)
-def gpg_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
+def gpg_loss_fn(data, config, corr=None) -> tuple[torch.Tensor, dict[str, Any]]:
     """Same objective as REINFORCE; pairs with the GPG advantage (loss.py:183-197)."""
-    return reinforce_loss_fn(data, config)
+    return reinforce_loss_fn(data, config, corr)
 
 
 @register_loss(LossFn.CISPO)
-def cispo_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
+def cispo_loss_fn(data, config, corr=None) -> tuple[torch.Tensor, dict[str, Any]]:
     """Clipped, stop-gradient importance weight times ``A * log_prob`` (loss.py:411-468)."""
-    return _run(_KIND_CISPO, data, config, "sum")
+    return _run(_KIND_CISPO, data, config, "sum", corr)
 
 
 class _GmpoLoss(torch.autograd.Function):
@@ -291,3 +293,9 @@ def clip_cov_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
               cov_ub=config.get("clip_cov_ub", 5.0), seed=seed)
     loss, sums, denom = _run_cov(1, data, config, hp, "mean")
     return loss, {"pg_clipfrac": sums[1] / denom, "ppo_kl": sums[2] / denom}
+
+
+# These enqueue launches and read their sums back once, without a draw or another effect of their own, and take the
+# ``corr`` of a correction in flight, whose sums they read back with theirs.
+for _fn in (ppo_loss_fn, gspo_loss_fn, reinforce_loss_fn, gpg_loss_fn, cispo_loss_fn):
+    _fn.one_readback = True

@@ -59,8 +59,18 @@ def compute_loss_fn(data, loss_fn: str, loss_fn_args: dict | None = None) -> tup
     corr_metrics: dict[str, Any] = {}
     wants_correction = any(args.get(k, None) is not None for k in _SAMPLER_SWITCHES)
     if wants_correction and "sampler_log_probs" in data.batch:
-        from axon_amd.utils.rl.sampler import compute_sampler_correction_and_add_to_batch
+        from axon_amd.utils.rl.sampler import compute_sampler_correction_and_add_to_batch, start_sampler_correction
 
+        # a loss that only enqueues launches before its own readback takes the corrected batch without waiting for the
+        # correction's sums, which come back with its own: one wait for the GPU instead of two
+        in_flight = start_sampler_correction(data, args, readback=False) if getattr(fn, "one_readback", False) else None
+        if in_flight is not None:
+            loss, metrics = fn(data, args, corr=in_flight.corr)
+            corr_metrics = in_flight.metrics()
+            if corr_metrics is None:  # no token to correct: as if the correction had not been asked for
+                return fn(data, args)
+            metrics.update(corr_metrics)
+            return loss, metrics
         data, corr_metrics = compute_sampler_correction_and_add_to_batch(data, args)
 
     loss, metrics = fn(data, args)

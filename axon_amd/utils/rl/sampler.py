@@ -196,25 +196,83 @@ def _offpolicy_from_diag(d, n_rows) -> dict[str, float]:
     }
 
 
-# --- public API -------------------------------------------------------------------------------
+class _Correction:
+    """A correction whose kernels are enqueued: ``weights`` and ``new_mask`` are device tensors that later launches may
+    use at once; ``finish()`` waits for the sums and returns the metrics."""
 
-def compute_sampler_correction_and_rejection_mask(
-    old_log_prob: torch.Tensor,
-    sampler_log_prob: torch.Tensor,
-    response_mask: torch.Tensor,
-    sampler_is: str | None = None,
-    sampler_is_threshold: float | None = 2.0,
-    sampler_rs: str | None = None,
-    sampler_rs_threshold: float | None = 2.0,
-    sampler_rs_threshold_lower: float | None = None,
-    sampler_token_veto_threshold: float | None = None,
-    sampler_is_batch_normalize: bool = False,
-    cu_seqlens: torch.Tensor | None = None,
-) -> tuple[DataProto | None, torch.Tensor, dict[str, float]]:
-    """Returns ``(DataProto{"sampler_is_weights"} | None, modified_response_mask, metrics)``.
+    def __init__(self, old_log_prob, response_mask, rows, weights, new_mask, both, sampler_is, sampler_rs, log_veto,
+                 batch_normalize):
+        self.response_mask, self.rows, self.weights, self.new_mask, self.both = (response_mask, rows, weights, new_mask,
+                                                                                 both)
+        self.sampler_is, self.sampler_rs, self.log_veto = sampler_is, sampler_rs, log_veto
+        self.batch_normalize = batch_normalize
+        self.host = self.event = None
 
-    An all-zero ``response_mask`` is a no-op: ``(None, response_mask, {})``.
-    """
+    @property
+    def loss_acc(self):
+        """Eight more fp32 values behind the sums, for a loss whose own sums are to come back with them."""
+        return self.both[-4:].view(torch.float32)
+
+    def read(self):
+        """Wait for everything enqueued so far; the loss's eight values."""
+        self.host = self.both.cpu()
+        return self.host[-4:].view(torch.float32).tolist()
+
+    def start_readback(self):
+        """Start the copy of the sums to the host behind the launches enqueued so far; what is enqueued after it does
+        not delay ``finish``."""
+        self.host = torch.empty(self.both.numel(), dtype=torch.float64, pin_memory=True)
+        self.host.copy_(self.both, non_blocking=True)
+        self.event = torch.cuda.Event()
+        self.event.record()
+
+    def finish(self) -> dict[str, float] | None:
+        """The metrics, or None for an all-zero mask (the correction is then a no-op).  ``weights`` is the
+        normalised array after this when the caller asked for that."""
+        if self.event is not None:
+            self.event.synchronize()
+        elif self.host is None:
+            self.read()  # single readback: empty-mask test and every metric
+        host = self.host.numpy()
+        sums, d = host[:4].view(np.float32).tolist(), host[4:-4].tolist()
+        rows, n_valid = self.rows, sums[0]
+        if n_valid == 0:
+            return None
+        metrics: dict[str, float] = {}
+        soft = _soft(n_valid)
+        if self.weights is not None:
+            metrics.update(_weight_metrics("sampler_is", d, rows.n_rows, self.sampler_is, 1, 5, 6, 7, 8, 23, 31, 3, 4, 7))
+            if self.batch_normalize:
+                mean_w = sums[5] / soft
+                if self.sampler_is == "sequence":
+                    # mean over rows that have tokens of the row's (constant) weight
+                    cnt, per_row, _ = _ops.row_stats(self.weights, None, self.response_mask, rows)
+                    has = (cnt > 0).to(torch.float32)
+                    mean_w = float(((per_row / (cnt + 1e-8)) * has).sum() / has.sum().clamp_min(1e-8))
+                if mean_w > 1e-8:
+                    self.weights = self.weights / mean_w
+                    metrics["sampler_is_batch_norm_factor"] = mean_w
+                else:
+                    metrics["sampler_is_batch_norm_factor"] = 1.0
+        if self.sampler_rs is not None:
+            metrics.update(_weight_metrics("sampler_rs", d, rows.n_rows, self.sampler_rs, 1, 9, 10, 11, 12, 27, 36, 5, 6, 8))
+            metrics["sampler_rs_masked_fraction"] = sums[2] / soft
+            metrics["sampler_rs_seq_masked_fraction"] = d[41] / rows.n_rows
+        if self.log_veto is not None:
+            metrics["sampler_is_veto_fraction"] = sums[4] / max(rows.n_rows, 1)
+            metrics["sampler_is_catastrophic_token_fraction"] = sums[3] / soft
+        else:
+            metrics["sampler_is_veto_fraction"] = 0.0
+            metrics["sampler_is_catastrophic_token_fraction"] = 0.0
+        return {f"sampler_corr/{k}": v for k, v in metrics.items()}
+
+
+def _enqueue_correction(old_log_prob, sampler_log_prob, response_mask, sampler_is=None, sampler_is_threshold=2.0,
+                        sampler_rs=None, sampler_rs_threshold=2.0, sampler_rs_threshold_lower=None,
+                        sampler_token_veto_threshold=None, sampler_is_batch_normalize=False,
+                        cu_seqlens=None) -> _Correction | None:
+    """Check the arguments and enqueue the correction and its diagnostics.  None: bad arguments beside an all-zero mask,
+    which the reference lets pass."""
     use_is = sampler_is is not None and sampler_is_threshold is not None
     rs_lo = rs_hi = 0.0
     log_veto = None
@@ -241,14 +299,15 @@ def compute_sampler_correction_and_rejection_mask(
         # (sampler.py:368-370): a bad argument only raises when there is a token to correct.  The valid path keeps
         # its single readback; this one costs an extra one.
         if not bool(response_mask.any()):
-            return None, response_mask, {}
+            return None
         raise
 
     _ops.require_device(old_log_prob, "compute_sampler_correction_and_rejection_mask")
     rows = _ops.rows_of(old_log_prob, cu_seqlens)
-    # the eight fp32 sums of the correction (32 bytes), then the diagnostics: one buffer, one copy to the host
-    both = torch.zeros(4 + _ops.DIAG_OUT, device=old_log_prob.device, dtype=torch.float64) if rows.n_slots == 0 else \
-        torch.empty(4 + _ops.DIAG_OUT, device=old_log_prob.device, dtype=torch.float64)
+    # the eight fp32 sums of the correction (32 bytes), the diagnostics, eight fp32 sums of a loss: one buffer, one
+    # copy to the host
+    make = torch.zeros if rows.n_slots == 0 else torch.empty
+    both = make(4 + _ops.DIAG_OUT + 4, device=old_log_prob.device, dtype=torch.float64)
     weights, new_mask, _ = _ops.sampler_correction(
         old_log_prob, sampler_log_prob, response_mask, rows,
         is_mode=_ops.IS_MODES[sampler_is] if use_is else 0,
@@ -262,46 +321,42 @@ def compute_sampler_correction_and_rejection_mask(
         if sampler_rs is not None else 1.0
     tok_lo, tok_hi = (rs_lo, rs_hi) if sampler_rs == "token" else (-math.inf, math.inf)
     _ops.sampler_diag(
-        old_log_prob, sampler_log_prob, response_mask, rows, out=both[4:],
+        old_log_prob, sampler_log_prob, response_mask, rows, out=both[4:-4],
         is_mode=_ops.IS_MODES[sampler_is] if use_is else 0, is_lo=is_lo, is_hi=is_hi,
         rs_mode=_ops.RS_MODES[sampler_rs], rs_lo=rs_lo_t, rs_hi=rs_hi_t, rs_lr_lo=tok_lo, rs_lr_hi=tok_hi,
         log_is_lo=_log32(is_lo), log_is_hi=_log32(is_hi), log_rs_lo=_log32(rs_lo_t), log_rs_hi=_log32(rs_hi_t),
     )
-    host = both.cpu().numpy()  # single readback: empty-mask test and every metric
-    sums, d = host[:4].view(np.float32).tolist(), host[4:].tolist()
-    n_valid = sums[0]
-    if n_valid == 0:
+    return _Correction(old_log_prob, response_mask, rows, weights, new_mask, both, sampler_is, sampler_rs, log_veto,
+                       sampler_is_batch_normalize)
+
+
+# --- public API -------------------------------------------------------------------------------
+
+def compute_sampler_correction_and_rejection_mask(
+    old_log_prob: torch.Tensor,
+    sampler_log_prob: torch.Tensor,
+    response_mask: torch.Tensor,
+    sampler_is: str | None = None,
+    sampler_is_threshold: float | None = 2.0,
+    sampler_rs: str | None = None,
+    sampler_rs_threshold: float | None = 2.0,
+    sampler_rs_threshold_lower: float | None = None,
+    sampler_token_veto_threshold: float | None = None,
+    sampler_is_batch_normalize: bool = False,
+    cu_seqlens: torch.Tensor | None = None,
+) -> tuple[DataProto | None, torch.Tensor, dict[str, float]]:
+    """Returns ``(DataProto{"sampler_is_weights"} | None, modified_response_mask, metrics)``.
+
+    An all-zero ``response_mask`` is a no-op: ``(None, response_mask, {})``.
+    """
+    corr = _enqueue_correction(old_log_prob, sampler_log_prob, response_mask, sampler_is, sampler_is_threshold, sampler_rs,
+                               sampler_rs_threshold, sampler_rs_threshold_lower, sampler_token_veto_threshold,
+                               sampler_is_batch_normalize, cu_seqlens)
+    metrics = corr.finish() if corr is not None else None
+    if metrics is None:
         return None, response_mask, {}
-
-    metrics: dict[str, float] = {}
-    soft = _soft(n_valid)
-    if use_is:
-        metrics.update(_weight_metrics("sampler_is", d, rows.n_rows, sampler_is, 1, 5, 6, 7, 8, 23, 31, 3, 4, 7))
-        if sampler_is_batch_normalize:
-            mean_w = sums[5] / soft
-            if sampler_is == "sequence":
-                # mean over rows that have tokens of the row's (constant) weight
-                cnt, per_row, _ = _ops.row_stats(weights, None, response_mask, rows)
-                has = (cnt > 0).to(torch.float32)
-                mean_w = float(((per_row / (cnt + 1e-8)) * has).sum() / has.sum().clamp_min(1e-8))
-            if mean_w > 1e-8:
-                weights = weights / mean_w
-                metrics["sampler_is_batch_norm_factor"] = mean_w
-            else:
-                metrics["sampler_is_batch_norm_factor"] = 1.0
-    if sampler_rs is not None:
-        metrics.update(_weight_metrics("sampler_rs", d, rows.n_rows, sampler_rs, 1, 9, 10, 11, 12, 27, 36, 5, 6, 8))
-        metrics["sampler_rs_masked_fraction"] = sums[2] / soft
-        metrics["sampler_rs_seq_masked_fraction"] = d[41] / rows.n_rows
-    if log_veto is not None:
-        metrics["sampler_is_veto_fraction"] = sums[4] / max(rows.n_rows, 1)
-        metrics["sampler_is_catastrophic_token_fraction"] = sums[3] / soft
-    else:
-        metrics["sampler_is_veto_fraction"] = 0.0
-        metrics["sampler_is_catastrophic_token_fraction"] = 0.0
-
-    proto = DataProto.from_dict(tensors={"sampler_is_weights": weights}) if weights is not None else None
-    return proto, new_mask, {f"sampler_corr/{k}": v for k, v in metrics.items()}
+    proto = DataProto.from_dict(tensors={"sampler_is_weights": corr.weights}) if corr.weights is not None else None
+    return proto, corr.new_mask, metrics
 
 
 def compute_sampler_correction_weights(
@@ -394,24 +449,65 @@ def compute_sampler_corr_metrics_from_logprobs(log_prob, sampler_log_prob, respo
     return {f"sampler_corr/{k}": v for k, v in m.items()}
 
 
+def _correction_args(batch: DataProto, config: dict[str, Any]) -> dict[str, Any]:
+    return dict(
+        old_log_prob=batch.batch["old_log_probs"],
+        sampler_log_prob=batch.batch["sampler_log_probs"],
+        response_mask=batch.batch["response_mask"],
+        sampler_is=config.get("sampler_is", None),
+        sampler_is_threshold=config.get("sampler_is_threshold", 2.0),
+        sampler_rs=config.get("sampler_rs", None),
+        sampler_rs_threshold=config.get("sampler_rs_threshold", None),
+        sampler_rs_threshold_lower=config.get("sampler_rs_threshold_lower", None),
+        sampler_token_veto_threshold=config.get("sampler_token_veto_threshold", None),
+        sampler_is_batch_normalize=config.get("sampler_is_batch_normalize", False),
+        cu_seqlens=batch.meta_info.get("cu_seqlens", None) if batch.meta_info else None,
+    )
+
+
 def compute_sampler_correction_and_add_to_batch(batch: DataProto, config: dict[str, Any]) -> tuple[DataProto, dict]:
     """Overwrite ``batch.batch["response_mask"]`` and union ``sampler_is_weights`` into the batch
     (sampler.py:526-563); ``config`` is the loss_args dict."""
     with torch.no_grad():
-        weights, new_mask, metrics = compute_sampler_correction_and_rejection_mask(
-            old_log_prob=batch.batch["old_log_probs"],
-            sampler_log_prob=batch.batch["sampler_log_probs"],
-            response_mask=batch.batch["response_mask"],
-            sampler_is=config.get("sampler_is", None),
-            sampler_is_threshold=config.get("sampler_is_threshold", 2.0),
-            sampler_rs=config.get("sampler_rs", None),
-            sampler_rs_threshold=config.get("sampler_rs_threshold", None),
-            sampler_rs_threshold_lower=config.get("sampler_rs_threshold_lower", None),
-            sampler_token_veto_threshold=config.get("sampler_token_veto_threshold", None),
-            sampler_is_batch_normalize=config.get("sampler_is_batch_normalize", False),
-            cu_seqlens=batch.meta_info.get("cu_seqlens", None) if batch.meta_info else None,
-        )
+        weights, new_mask, metrics = compute_sampler_correction_and_rejection_mask(**_correction_args(batch, config))
     batch.batch["response_mask"] = new_mask
     if weights is not None:
         batch = batch.union(weights)
     return batch, metrics
+
+
+class CorrectionInFlight:
+    """``compute_sampler_correction_and_add_to_batch`` without its wait: the batch holds the new mask and the weights, the
+    caller enqueues what uses them, and ``metrics()`` (to be called when the caller has something to wait for anyway) gives the
+    correction's metrics.  An all-zero mask is known only then: ``metrics()`` puts the batch back as it was and returns
+    None, and the caller does its work again without a correction."""
+
+    def __init__(self, batch: DataProto, corr: _Correction):
+        self.batch, self.corr = batch, corr
+        batch.batch["response_mask"] = corr.new_mask
+        if corr.weights is not None:
+            batch.union(DataProto.from_dict(tensors={"sampler_is_weights": corr.weights}))
+
+    def metrics(self) -> dict[str, float] | None:
+        metrics = self.corr.finish()
+        if metrics is None:
+            self.batch.batch["response_mask"] = self.corr.response_mask
+            if self.corr.weights is not None:
+                self.batch.batch.pop("sampler_is_weights")
+        return metrics
+
+
+def start_sampler_correction(batch: DataProto, config: dict[str, Any], readback: bool) -> CorrectionInFlight | None:
+    """Enqueue the correction of ``batch`` (with ``readback`` also the copy of its sums to the host), or None where the
+    host needs them before anything else (weights normalised by their mean, weights that the batch already
+    has, a batch kept on the host): ``compute_sampler_correction_and_add_to_batch`` then."""
+    b = batch.batch
+    if config.get("sampler_is_batch_normalize", False) or "sampler_is_weights" in b or not b["old_log_probs"].is_cuda:
+        return None
+    with torch.no_grad():
+        corr = _enqueue_correction(**_correction_args(batch, config))
+        if corr is None:
+            return None
+        if readback:
+            corr.start_readback()
+        return CorrectionInFlight(batch, corr)

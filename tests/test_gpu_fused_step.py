@@ -414,3 +414,44 @@ def test_qwen3_8b_fused_step_vs_fp32_torch_and_oracle_loss():
     idx = torch.cat([torch.arange(0, n, 509), torch.tensor([8191, 8192, 16383, 16384, 24575, 24576, n - 1])])
     o_dh, _ = OM.backward(g_head[idx], None, hid[idx], w, torch.roll(ids, -1)[idx])
     assert rel_l2(got[3][idx.to(DEV)], o_dh) < 2e-2
+
+
+@pytest.mark.parametrize("nan", [False, True])
+@pytest.mark.parametrize("case", ["ppo", "gspo"])
+def test_fused_step_with_a_correction_in_flight(case, nan):
+    """The step does not wait for the sampler correction: an all-zero mask, known only at the end, leaves the batch as it
+    was, without correction metrics and with zero gradients, also where the sampler's log-probs are NaN."""
+    from axon_amd.models.fused_head_loss import fused_head_loss
+    lens = [40, 25, 63]
+    n, h, v = sum(lens), 64, 300
+    hid, w, ids, labels, rl, old, ref = _inputs(n, h, v, lens, seed=4)
+    name, args = {"ppo": ("ppo", PPO), "gspo": ("gspo", GSPO)}[case]
+    args = dict(args, sampler_is="token", sampler_is_threshold=2.0, sampler_token_veto_threshold=1e-4)
+    hd, wd = hid.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(True)
+    mask = torch.zeros(n, device=DEV)
+    samp = old.to(DEV) * (float("nan") if nan else 1.01)
+    data = DataProto.from_dict(tensors={"old_log_probs": old.to(DEV), "advantages": torch.ones(n, device=DEV),
+                                        "response_mask": mask, "sampler_log_probs": samp})
+    loss, metrics = fused_head_loss(hd, wd, ids.to(DEV), rl["cu_seqlens"].to(DEV), data,
+                                    {"loss_fn": name, "loss_fn_args": args, "temperature": 1.0, "dp_replicas": 1})
+    loss.backward()
+    assert loss.item() == 0.0 and (hd.grad == 0).all() and (wd.grad == 0).all()
+    assert data.batch["response_mask"] is mask and "sampler_is_weights" not in data.batch
+    assert not any(k.startswith("sampler_corr/") for k in metrics)
+
+
+def test_fused_step_of_one_block_checks_the_offsets_it_never_reads():
+    """A sequence-cut batch of one block does not read its offsets back first; offsets that do not span the batch are refused
+    all the same, with the step's one readback."""
+    from axon_amd.models.fused_head_loss import fused_head_loss
+    lens = [40, 25, 63]
+    n, h, v = sum(lens), 64, 300
+    hid, w, ids, labels, rl, old, ref = _inputs(n, h, v, lens, seed=4)
+    for cu in ([0, 40, 65, n - 1], [1, 40, 65, n], [0, 40, 65, n + 8]):
+        for kw in ({}, {"cu_host": cu}):
+            data = DataProto.from_dict(tensors={"old_log_probs": old.to(DEV), "advantages": torch.ones(n, device=DEV),
+                                                "response_mask": torch.ones(n, device=DEV)})
+            with pytest.raises(ValueError, match=f"spans {cu[0]}..{cu[-1]}, the batch has {n} tokens"):
+                fused_head_loss(hid.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(True), ids.to(DEV),
+                                torch.tensor(cu, dtype=torch.int32, device=DEV), data,
+                                {"loss_fn": "gspo", "loss_fn_args": GSPO, "temperature": 1.0, "dp_replicas": 1}, **kw)

@@ -1283,3 +1283,65 @@ def test_a_threads_run_in_the_streaming_losses_stays_at_sixteen_slots(chunks):
     assert abs(-acc[0].item() / lp[0, 0].item() - 1) < 2.5e-7 and acc[4].item() == n
     ent, _, _ = _ops.side_terms(lp, None, None, one, rows, token_reduce="sum", batch_reduce="token-mean")
     assert abs(ent[0].item() / lp[0, 0].item() - 1) < 2.5e-7
+
+
+_CORRECT = dict(sampler_is="token", sampler_is_threshold=2.0, sampler_rs="token", sampler_rs_threshold=1.5,
+                sampler_token_veto_threshold=1e-4)
+
+
+@pytest.mark.parametrize("loss_fn,extra", [("ppo", {}), ("gspo", {}), ("cispo", {}), ("reinforce", {}), ("gpg", {}), ("geo_mean", {}),
+                                           ("ppo", dict(sampler_is_batch_normalize=True)),
+                                           ("gspo", dict(sampler_is="sequence", sampler_rs="geometric"))])
+@pytest.mark.parametrize("packed", [False, True])
+def test_correction_read_back_with_the_loss(loss_fn, extra, packed):
+    """compute_loss_fn reads the correction's sums back with the loss's: loss, gradient, mask, weights and every metric
+    are those of the correction applied first and the loss after it."""
+    from axon_amd.utils.rl.sampler import compute_sampler_correction_and_add_to_batch
+    g = torch.Generator().manual_seed(5)
+    b, t = 6, 37
+    cu = (torch.arange(b + 1) * t).int().to(DEV) if packed else None
+    shape = (b * t,) if packed else (b, t)
+    old, adv = -torch.rand(shape, generator=g), torch.randn(shape, generator=g)
+    new, samp = old + 0.2 * torch.randn(shape, generator=g), old + 0.3 * torch.randn(shape, generator=g)
+    mask = (torch.rand(shape, generator=g) < 0.8).long()
+    args = dict(_CORRECT, **extra)
+
+    def batch():
+        lp = new.to(DEV).requires_grad_(True)
+        return lp, DataProto.from_dict(
+            tensors={"log_probs": lp, "old_log_probs": old.to(DEV), "advantages": adv.to(DEV),
+                     "response_mask": mask.to(DEV), "sampler_log_probs": samp.to(DEV)},
+            meta_info={"cu_seqlens": cu} if packed else {})
+
+    lp1, d1 = batch()
+    loss1, m1 = compute_loss_fn(d1, loss_fn, args)
+    loss1.backward()
+    lp2, d2 = batch()
+    d2, corr = compute_sampler_correction_and_add_to_batch(d2, args)
+    loss2, m2 = compute_loss_fn(d2, loss_fn, {})
+    loss2.backward()
+    m2.update(corr)
+    assert torch.equal(loss1, loss2) and torch.equal(lp1.grad, lp2.grad) and list(m1) == list(m2)
+    assert m1 == m2 and any(k.startswith("sampler_corr/") for k in m1)
+    assert all(torch.equal(d1.batch[k], d2.batch[k]) for k in ("response_mask", "sampler_is_weights"))
+
+
+@pytest.mark.parametrize("nan", [False, True])
+def test_correction_read_back_with_the_loss_of_an_empty_mask(nan):
+    """No token to correct: the batch keeps its mask and gets no weights, the loss is the uncorrected one and there are
+    no correction metrics; sampler log-probs that are NaN reach nothing."""
+    z = torch.zeros(2, 8, device=DEV)
+    mask = z.long()
+    lp = torch.randn(2, 8, generator=torch.Generator().manual_seed(1)).to(DEV).requires_grad_(True)
+    data = DataProto.from_dict(tensors={"log_probs": lp, "old_log_probs": z, "advantages": z + 1, "response_mask": mask,
+                                        "sampler_log_probs": z + (math.nan if nan else 0.5)})
+    loss, metrics = compute_loss_fn(data, "ppo", _CORRECT)
+    loss.backward()
+    assert loss.item() == 0.0 and (lp.grad == 0).all()
+    assert data.batch["response_mask"] is mask and "sampler_is_weights" not in data.batch
+    assert set(metrics) == {"ppo_kl", "pg_clipfrac", "pg_clipfrac_lower"}
+    # weights that the batch has already are not overwritten (the reference's union refuses other values)
+    full = DataProto.from_dict(tensors=dict(data.batch, response_mask=mask + 1, sampler_log_probs=z,
+                                            sampler_is_weights=z + 3.0))
+    with pytest.raises(AssertionError, match="sampler_is_weights"):
+        compute_loss_fn(full, "ppo", _CORRECT)
