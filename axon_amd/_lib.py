@@ -94,6 +94,10 @@ SIGNATURES: dict[str, tuple] = {
     "axon_kl_reward": (_i32, [_ptr, _ptr, _ptr, _ptr, _i32, _ptr, _i64, _i64, _i64, _i32, _f32, _ptr, _ptr, _ptr]),
     "axon_side_terms": (_i32, [_ptr, _ptr, _ptr, _ptr, _i32, _ptr, _i64, _i64, _i64, _ptr, _f32, _i32, _ptr, _i32,
                                _i32, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "axon_sampler_correction_diag_workspace_bytes": (_i64, [_i64, _i64]),
+    "axon_sampler_correction_diag": (_i32, [_ptr, _ptr, _ptr, _i32, _ptr, _i64, _i64, _i64, _i32, _f32, _i32, _f32, _f32,
+                                            _i32, _f32, _f32, _f32, _f32, _f32, _f32, _f32, _f32, _f32, _ptr, _ptr, _ptr,
+                                            _ptr, _ptr, _ptr, _ptr]),
     "axon_sampler_diag_workspace_bytes": (_i64, [_i64, _i64]),
     "axon_sampler_diag": (_i32, [_ptr, _ptr, _ptr, _i32, _ptr, _i64, _i64, _i64, _i32, _f32, _f32, _i32, _f32,
                                  _f32, _f32, _f32, _f32, _f32, _f32, _f32, _ptr, _ptr, _ptr]),

@@ -7,6 +7,7 @@ raises on a non-zero status.  Nothing here computes on the CPU.
 
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 
 import torch
@@ -357,6 +358,42 @@ def sampler_correction(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_thresho
 
 
 DIAG_OUT = 72
+
+
+def sampler_correction_diag(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_threshold, rs_mode, rs_lr_lo, rs_lr_hi,
+                            log_veto, is_lo, is_hi, rs_lo, rs_hi, log_is_lo, log_is_hi, log_rs_lo, log_rs_hi, acc, out):
+    """``sampler_correction`` into ``acc`` and the diagnostics of its metrics into ``out`` (DIAG_OUT float64 values, see
+    ``sampler_diag``; those that no metric of a correction reads may be left out).  Where a workgroup owns whole
+    rows one pass over the tokens serves both (axon_sampler_correction_diag)."""
+    if not ((is_mode == 2 or rs_mode >= 2 or log_veto is not None) and rows.n_rows > 0 and _own_rows(rows)):
+        isw, new_mask, _ = sampler_correction(old_lp, samp_lp, mask, rows, is_mode=is_mode, is_threshold=is_threshold,
+                                              rs_mode=rs_mode, rs_lr_lo=rs_lr_lo, rs_lr_hi=rs_lr_hi, log_veto=log_veto,
+                                              acc=acc)
+        tok_lo, tok_hi = (rs_lr_lo, rs_lr_hi) if rs_mode == 1 else (-math.inf, math.inf)
+        sampler_diag(old_lp, samp_lp, mask, rows, is_mode=is_mode, is_lo=is_lo, is_hi=is_hi, rs_mode=rs_mode, rs_lo=rs_lo,
+                     rs_hi=rs_hi, rs_lr_lo=tok_lo, rs_lr_hi=tok_hi, log_is_lo=log_is_lo, log_is_hi=log_is_hi,
+                     log_rs_lo=log_rs_lo, log_rs_hi=log_rs_hi, out=out)
+        return isw, new_mask
+    lib = _lib.load()
+    require_device(old_lp, "sampler_correction")
+    _same_len("sampler_correction", rows.n_slots, old_log_probs=old_lp, sampler_log_probs=samp_lp, mask=mask)
+    dev = old_lp.device
+    old_lp, samp_lp = f32(old_lp), f32(samp_lp)
+    mk, kind = mask_arg(mask)
+    isw = torch.empty(rows.shape, device=dev, dtype=torch.float32) if is_mode else None
+    new_mask = torch.empty(rows.shape, device=dev, dtype=torch.float32)
+    nbytes = lib.axon_sampler_correction_diag_workspace_bytes(rows.n_rows, rows.n_slots)
+    ws = torch.empty(nbytes // 4, device=dev, dtype=torch.float32)
+    check(
+        lib.axon_sampler_correction_diag(
+            ptr(old_lp), ptr(samp_lp), ptr(mk), kind, rows.cu_ptr, rows.n_rows, rows.n_slots, rows.uniform_len, is_mode,
+            float(is_threshold), rs_mode, float(rs_lr_lo), float(rs_lr_hi), int(log_veto is not None),
+            float(log_veto if log_veto is not None else 0.0), float(is_lo), float(is_hi), float(rs_lo), float(rs_hi),
+            float(log_is_lo), float(log_is_hi), float(log_rs_lo), float(log_rs_hi), ptr(isw), ptr(new_mask), ptr(acc),
+            ptr(_partials(rows.n_slots, dev)), ptr(ws), ptr(out), stream_ptr()),
+        "axon_sampler_correction_diag",
+    )
+    return isw, new_mask
 
 
 def sampler_diag(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_lo, is_hi, rs_mode, rs_lo, rs_hi, rs_lr_lo,

@@ -8,13 +8,10 @@
 // Pass 2 (one workgroup): adds the partials in a fixed order in double precision and walks the
 // rows for the sequence-level statistics.
 #include "common.h"
+#include "diag.h"
 
 namespace axon {
 
-constexpr int kDiagSums = 23;    // token-level sums, see axon_amd.h
-constexpr int kDiagMinMax = 6;   // max e, min e, max |pa-ps|, min |pa-ps|, max |lr|, min |lr|
-constexpr int kDiagStride = 32;  // floats per workgroup in `partials`
-constexpr int kDiagRowVals = 6;  // cnt, sum old, sum sampler, sum lr, sum e, sum token-rejected
 constexpr float kBound = 20.0f;  // axon/utils/rl/sampler.py:27
 
 __device__ __forceinline__ float clampf3(float x, float lo, float hi) {
@@ -171,12 +168,6 @@ constexpr int kOutSums = 50;  // out[0..49]: sums (0..22 token-level, 23..49 row
 constexpr int kOutMM = 10;    // out[50..59]: maxima, out[60..69]: minima
 constexpr int kDiagOut = 72;
 
-struct DiagCfg {
-  int is_mode, rs_mode;  // 0 off, 1 token, 2 sequence, 3 geometric (rs only)
-  float is_lo, is_hi, rs_lo, rs_hi;                  // ratio thresholds
-  float log_is_lo, log_is_hi, log_rs_lo, log_rs_hi;  // fp32 log of the same
-};
-
 // Four wavefronts per workgroup: what a wavefront spends here is mostly the 50 + 20 reductions at the end,
 // which cost the same for one row per lane as for four, and sixteen wavefronts would queue four deep on a SIMD.
 // Those reductions by DPP moves instead of LDS shuffles: 65536 tokens in 90 rows 9.6 us for 17.3, 8.4 M in 9000 15.3 for 21.9.
@@ -267,6 +258,7 @@ __global__ __launch_bounds__(kDiagRowThreads) void sampler_diag_rows_kernel(
       mx[5] = fmaxf(mx[5], x); mn[5] = fminf(mn[5], x);
       mx[6] = fmaxf(mx[6], fabsf(x - 1.f));
     }
+    if (!cfg.with_gap) continue;
     // off-policy diagnostics (sampler.py:476-517)
     const float a = so_a[r] / den, b = ss_a[r] / den;  // masked row means of old / sampler log-probs
     const float d = b - a;
@@ -333,11 +325,34 @@ __global__ __launch_bounds__(1024) void sampler_diag_final_kernel(const double* 
 
 using namespace axon;
 
-static inline int diag_row_blocks(int64_t n_rows, int64_t token_blocks) {
+static int diag_row_blocks(int64_t n_rows, int64_t token_blocks) {
   const int64_t work = n_rows > token_blocks ? n_rows : token_blocks;
   const int64_t b = (work + 1023) / 1024;
   return (int)(b < 1 ? 1 : (b > 128 ? 128 : b));
 }
+
+namespace axon {
+DiagWorkspace diag_workspace(float* base, int64_t n_rows, int64_t token_blocks) {
+  const int64_t floats = kDiagRowVals * n_rows + token_blocks * kDiagStride;
+  return DiagWorkspace{base, base + kDiagRowVals * n_rows, reinterpret_cast<double*>(base + (floats + 1) / 2 * 2)};
+}
+int64_t diag_workspace_bytes(int64_t n_rows, int64_t token_blocks) {
+  const int64_t floats = kDiagRowVals * n_rows + token_blocks * kDiagStride;
+  return ((floats + 1) / 2 * 2) * (int64_t)sizeof(float) +
+         (int64_t)diag_row_blocks(n_rows, token_blocks) * kDiagOut * (int64_t)sizeof(double);
+}
+int launch_diag_rows(const DiagWorkspace& w, int token_blocks, int64_t n_rows, const DiagCfg& cfg, double* out,
+                     hipStream_t st) {
+  const int rb = diag_row_blocks(n_rows, token_blocks);
+  hipLaunchKernelGGL(sampler_diag_rows_kernel, dim3(rb), dim3(kDiagRowThreads), 0, st, w.partials, token_blocks, w.row_vals,
+                     n_rows, cfg, rb == 1 ? out : w.parts);
+  AXON_CHECK_LAUNCH();
+  if (rb == 1) return AXON_OK;  // one workgroup's results are the totals
+  hipLaunchKernelGGL(sampler_diag_final_kernel, dim3(1), dim3(1024), 0, st, w.parts, rb, out);
+  AXON_CHECK_LAUNCH();
+  return AXON_OK;
+}
+}  // namespace axon
 
 // Steps of 1024 slots per workgroup of the token pass: one where longer chunks would leave compute units idle
 // (65536 slots in chunks of 4096 run on 16 of 256: 17.6 us, in chunks of 1024 8.6).
@@ -354,9 +369,7 @@ extern "C" int64_t axon_sampler_diag_workspace_bytes(int64_t n_rows, int64_t n_s
   const int64_t blocks = n_slots > 0 ? (int64_t)diag_grid(n_slots) : 1;
   // [6][n_rows] row sums (zero-filled by the caller), the per-workgroup token partials, then the
   // row pass's per-workgroup results (doubles, 8-byte aligned)
-  const int64_t floats = kDiagRowVals * n_rows + blocks * kDiagStride;
-  return ((floats + 1) / 2 * 2) * (int64_t)sizeof(float) +
-         (int64_t)diag_row_blocks(n_rows, blocks) * kDiagOut * (int64_t)sizeof(double);
+  return diag_workspace_bytes(n_rows, blocks);
 }
 
 extern "C" int axon_sampler_diag(const float* oldp, const float* samp, const void* mask, int mask_kind,
@@ -373,9 +386,9 @@ extern "C" int axon_sampler_diag(const float* oldp, const float* samp, const voi
   if (reinterpret_cast<uintptr_t>(workspace) & 7) return AXON_ERR_WORKSPACE;
   if (is_mode < 0 || is_mode > 2 || rs_mode < 0 || rs_mode > 3) return AXON_ERR_ARG;
   if (mask_kind != AXON_MASK_F32 && mask_kind != AXON_MASK_I64) return AXON_ERR_ARG;
-  float* row_vals = workspace;
-  float* partials = workspace + kDiagRowVals * n_rows;
   const dim3 g(diag_grid(n_slots)), blk(kBlock);
+  const DiagWorkspace w = diag_workspace(workspace, n_rows, g.x);
+  float *row_vals = w.row_vals, *partials = w.partials;
   const int iters = diag_iters(n_slots);
   const hipStream_t st = (hipStream_t)stream;
   if (mask_kind == AXON_MASK_F32)
@@ -388,18 +401,9 @@ extern "C" int axon_sampler_diag(const float* oldp, const float* samp, const voi
                        iters, row_vals, partials);
   AXON_CHECK_LAUNCH();
   DiagCfg cfg;
-  cfg.is_mode = is_mode; cfg.rs_mode = rs_mode;
+  cfg.is_mode = is_mode; cfg.rs_mode = rs_mode; cfg.with_gap = 1;
   cfg.is_lo = is_lo; cfg.is_hi = is_hi; cfg.rs_lo = rs_lo; cfg.rs_hi = rs_hi;
   cfg.log_is_lo = log_is_lo; cfg.log_is_hi = log_is_hi;
   cfg.log_rs_lo = log_rs_lo; cfg.log_rs_hi = log_rs_hi;
-  const int64_t floats = kDiagRowVals * n_rows + (int64_t)g.x * kDiagStride;
-  double* parts = reinterpret_cast<double*>(workspace + (floats + 1) / 2 * 2);
-  const int rb = diag_row_blocks(n_rows, g.x);
-  hipLaunchKernelGGL(sampler_diag_rows_kernel, dim3(rb), dim3(kDiagRowThreads), 0, st, partials, (int)g.x, row_vals,
-                     n_rows, cfg, rb == 1 ? out : parts);
-  AXON_CHECK_LAUNCH();
-  if (rb == 1) return AXON_OK;  // one workgroup's results are the totals
-  hipLaunchKernelGGL(sampler_diag_final_kernel, dim3(1), dim3(1024), 0, st, parts, rb, out);
-  AXON_CHECK_LAUNCH();
-  return AXON_OK;
+  return launch_diag_rows(w, (int)g.x, n_rows, cfg, out, st);
 }

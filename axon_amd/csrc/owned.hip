@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "diag.h"
 #include "token_math.h"
 
 namespace axon {
@@ -81,7 +82,9 @@ __device__ __forceinline__ float wave_total(float v) {  // the same value in eve
 //   load(p0, b, c)                    the vector of four slots starting at p0 into register set (b, c) (every input):
 //                                     a fixed number of 16-byte loads, p0 + 4 <= n_slots
 //   load_edge(p0, b, c)               the same for a vector that may reach beyond the last slot
-//   stat(b, c, j, s[])                add slot j of register set (b, c) to the thread's row sums
+//   stat(b, c, j, s[])                add slot j of register set (b, c) to the thread's row sums; every slot of every
+//                                     row once
+//   group_end()                       after the stat calls of a group (at most kRowHold * kVec of them)
 //   rows(r, tot[], first) -> RowVals  the per-row values from the row's sums (every thread the same)
 //   emit(p0, b, c, rv, t0, t1)        write the outputs of the vector in register set (b, c)
 //   fill_gap(a, b)                    zeros for slots that belong to no row
@@ -227,6 +230,7 @@ __device__ __forceinline__ void walk_owned_rows(const RowStarts& rs, int stride,
             if (p0 + j >= t0 && p0 + j < t1) op.stat(B, c, j, s[c]);
         }
       }
+      op.group_end();
     };
     auto emit_unit = [&](int c, int grp, const typename Op::RowVals& rv) {
       int p0, t0, t1;
@@ -393,6 +397,7 @@ struct OwnedLossOp {
     // masked sum: values outside the mask never reach it (NaN / Inf in padding)
     s[1] += (m != 0.f) ? (lv[b][c][j] - ov[b][c][j]) * m : 0.f;
   }
+  __device__ __forceinline__ void group_end() {}
   __device__ __forceinline__ RowVals rows(int64_t r, const float (&tot)[2], bool first) {
     const float c = tot[0];
     float td = 1.f;
@@ -463,17 +468,31 @@ struct OwnedCorrArgs {
   float *isw, *new_mask;
   float *row_cnt, *row_sum;  // optional per-row outputs (the sums the decisions were taken from)
   int32_t* row_flag;         // optional: 1 where the row was vetoed
+  // TOK kernels: per-row sums of the unclamped weights and of the rejected tokens, and what the token-level diagnostics
+  // clamp and count by (the arguments of axon_sampler_diag)
+  float *row_e, *row_rej;
+  float is_lo, is_hi, rs_lo, rs_hi, rs_lr_lo, rs_lr_hi;
+  float* diag_partials;      // [workgroups][kDiagStride], or null: no diagnostics
 };
 
-template <int MK>
+// TOK: also the token-level diagnostics (sampler_diag_tokens_kernel's) that the metrics of a correction with token-level
+// weights or rejection need; a correction by sequences needs none beyond the row sums.
+template <int MK, bool TOK>
 struct OwnedCorrOp {
-  static constexpr int kNV = 3;  // sum mask, sum (old - sampler) * mask, tokens under the veto threshold
+  // sum mask, sum (old - sampler) * mask, tokens under the veto threshold; sum weight * mask, sum rejected
+  static constexpr int kNV = TOK ? 5 : 3;
   typedef CorrRow RowVals;
   const OwnedCorrArgs& g;
   const RowStarts& rs;
   float ov[2][kRowHold][4], sv[2][kRowHold][4], mv[2][kRowHold][4];
   float a[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float vetoed_rows = 0.f;
+  // token-level diagnostics: a group's slots in fp32, the groups in double, so that no fp32 sum of a thread is longer than
+  // eight slots however many rows it walks
+  static constexpr int kTok = 9;  // e; e > is_hi, e < is_lo, clamped e, its square; the same by the rejection's bounds
+  float t[TOK ? kTok : 1] = {};
+  double td[TOK ? kTok : 1] = {};
+  float e_max = -__builtin_huge_valf(), e_min = __builtin_huge_valf();
 
   __device__ __forceinline__ OwnedCorrOp(const OwnedCorrArgs& g_, const RowStarts& rs_) : g(g_), rs(rs_) {}
 
@@ -489,20 +508,49 @@ struct OwnedCorrOp {
     row_load4_guard<KEEP>(g.samp, p0, rs.n_slots, sv[b][c]);
     row_load_mask4_guard<MK, KEEP>(g.mask, p0, rs.n_slots, mv[b][c]);
   }
-  __device__ __forceinline__ void stat(int b, int c, int j, float (&s)[3]) const {
+  __device__ __forceinline__ void stat(int b, int c, int j, float (&s)[kNV]) {
     const float m = mv[b][c][j];
     const float d = ov[b][c][j] - sv[b][c][j];
     s[0] += m;
     s[1] += (m != 0.f) ? d * m : 0.f;
     s[2] += (g.cfg.has_veto && m != 0.f && d < g.cfg.log_veto) ? 1.f : 0.f;
+    if (TOK && m != 0.f) {
+      const float e = __expf(clampf(d, -kSafetyBound, kSafetyBound));
+      const float ci = clampf(e, g.is_lo, g.is_hi), cr = clampf(e, g.rs_lo, g.rs_hi), em = e * m;
+      s[3] += em;
+      s[4] += (d >= g.rs_lr_lo && d <= g.rs_lr_hi) ? 0.f : m;
+      t[0] += em;
+      t[1] += (e > g.is_hi) ? m : 0.f;
+      t[2] += (e < g.is_lo) ? m : 0.f;
+      t[3] += ci * m;
+      t[4] += ci * ci * m;
+      t[5] += (e > g.rs_hi) ? m : 0.f;
+      t[6] += (e < g.rs_lo) ? m : 0.f;
+      t[7] += cr * m;
+      t[8] += cr * cr * m;
+      e_max = fmaxf(e_max, e);
+      e_min = fminf(e_min, e);
+    }
   }
-  __device__ __forceinline__ RowVals rows(int64_t r, const float (&tot)[3], bool first) {
+  __device__ __forceinline__ void group_end() {
+    if (!TOK) return;
+#pragma unroll
+    for (int k = 0; k < kTok; ++k) {
+      td[k] += (double)t[k];
+      t[k] = 0.f;
+    }
+  }
+  __device__ __forceinline__ RowVals rows(int64_t r, const float (&tot)[kNV], bool first) {
     const bool vetoed = tot[2] > 0.f;
     vetoed_rows += (first && g.cfg.has_veto && vetoed) ? 1.f : 0.f;
     if (first) {
       if (g.row_cnt) g.row_cnt[r] = tot[0];
       if (g.row_sum) g.row_sum[r] = tot[1];
       if (g.row_flag) g.row_flag[r] = vetoed ? 1 : 0;
+      if (TOK) {
+        g.row_e[r] = tot[3];
+        g.row_rej[r] = tot[4];
+      }
     }
     return corr_row(g.cfg, tot[1], tot[0], vetoed);
   }
@@ -526,12 +574,52 @@ struct OwnedCorrOp {
   }
 };
 
-template <int MK>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void owned_correction_kernel(OwnedCorrArgs g, RowStarts rs, int stride,
-                                                                  float* ws, float* __restrict__ acc) {
+// With `diag_partials` the launch takes the place of sampler_diag_tokens_kernel as well, which read the same three arrays
+// again, found every token's row and added the row sums up with atomics.  8.4 M tokens: 62 us for 59 + 43 and a fill of
+// the row sums where the diagnostics are the rows' only; 65536 tokens with token-level weights, rejection and veto 17.8 for
+// 13.4 + 8.6 and the fill.  Bound by the latency of a step of the walk (2.8 TB/s).  TOK at three workgroups per CU: 140
+// registers, four would spill.
+template <int MK, bool TOK>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(TOK ? 3 : 4))) void owned_correction_kernel(
+    OwnedCorrArgs g, RowStarts rs, int stride, float* ws, float* __restrict__ acc) {
   __shared__ float lds_red[kPartialStride * (kBlock / kWave)];
-  OwnedCorrOp<MK> op(g, rs);
+  OwnedCorrOp<MK, TOK> op(g, rs);
   walk_owned_rows(rs, stride, op);
+  if (g.diag_partials != nullptr) {
+    __shared__ float lds_tok[(OwnedCorrOp<MK, TOK>::kTok + 1) * (kBlock / kWave)], lds_mm[2 * (kBlock / kWave)];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    float v[OwnedCorrOp<MK, TOK>::kTok + 1];
+    v[0] = op.a[0];
+#pragma unroll
+    for (int k = 0; k < OwnedCorrOp<MK, TOK>::kTok; ++k) v[1 + k] = TOK ? (float)op.td[TOK ? k : 0] : 0.f;
+    const float hi = wave_max(op.e_max), lo = wave_min(op.e_min);
+    if (lane == 0) {
+      lds_mm[2 * wave] = hi;
+      lds_mm[2 * wave + 1] = lo;
+    }
+    block_sum<OwnedCorrOp<MK, TOK>::kTok + 1>(v, lds_tok);  // contains the barrier that also publishes lds_mm
+    __shared__ float lds_row[kDiagStride];
+    if (threadIdx.x == 0) {
+      // sums of nothing and extrema of nothing where a quantity is not formed
+      for (int k = 0; k < kDiagStride; ++k)
+        lds_row[k] = k < kDiagSums ? 0.f : ((k - kDiagSums) & 1) ? __builtin_huge_valf() : -__builtin_huge_valf();
+      lds_row[0] = v[0];
+      if (TOK) {
+        lds_row[1] = v[1];
+#pragma unroll
+        for (int k = 2; k < OwnedCorrOp<MK, TOK>::kTok + 1; ++k) lds_row[3 + k] = v[k];  // 5 .. 12
+        float mx = lds_mm[0], mn = lds_mm[1];
+        for (int w = 1; w < kBlock / kWave; ++w) {
+          mx = fmaxf(mx, lds_mm[2 * w]);
+          mn = fminf(mn, lds_mm[2 * w + 1]);
+        }
+        lds_row[kDiagSums] = mx;
+        lds_row[kDiagSums + 1] = mn;
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < kDiagStride) g.diag_partials[(size_t)blockIdx.x * kDiagStride + threadIdx.x] = lds_row[threadIdx.x];
+  }
   float part[6] = {op.a[0], op.a[1], op.a[2], op.a[3], op.vetoed_rows, op.a[5]};
   grid_finish<6>(part, lds_red, ws, [&](float (&tot)[kPartialStride]) {
     for (int k = 0; k < kPartialStride; ++k) acc[k] = tot[k];
@@ -567,6 +655,18 @@ OwnedLaunch owned_launch(int64_t n_slots, int resident) {
   stride = (stride + kVec - 1) / kVec * kVec;
   if (stride < kRowChunk) stride = kRowChunk;
   return OwnedLaunch{(int)stride, (unsigned)((n_slots + stride - 1) / stride)};
+}
+
+// At most this many workgroups for n_slots, whatever the device says about residency.
+int64_t owned_grid_bound(int64_t n_slots) { return (n_slots + kRowChunk - 1) / kRowChunk; }
+
+template <int MK, bool TOK>
+unsigned launch_correction(const OwnedCorrArgs& g, const RowStarts& rs, float* acc, float* partials, hipStream_t st) {
+  static const int resident = resident_blocks(owned_correction_kernel<MK, TOK>);
+  const OwnedLaunch ol = owned_launch(rs.n_slots, resident);
+  hipLaunchKernelGGL((owned_correction_kernel<MK, TOK>), dim3(ol.grid), dim3(kBlock), 0, st, g, rs, ol.stride, partials,
+                     acc);
+  return ol.grid;
 }
 
 int check_owned_rows(const int32_t* cu, int64_t n_rows, int64_t n_slots, int64_t uniform_len) {
@@ -657,17 +757,56 @@ extern "C" int axon_sampler_correction_rows(const float* oldp, const float* samp
   const OwnedCorrArgs g{oldp, samp, mask, CorrCfg{is_mode, is_thr, rs_mode, rs_lo, rs_hi, has_veto, log_veto},
                         isw, new_mask, row_cnt, row_sum, row_flag};
   const RowStarts rs{cu, uniform_len, n_rows, n_slots};
-  if (mask_kind == AXON_MASK_F32) {
-    static const int resident = resident_blocks(owned_correction_kernel<AXON_MASK_F32>);
-    const OwnedLaunch ol = owned_launch(n_slots, resident);
-    hipLaunchKernelGGL(owned_correction_kernel<AXON_MASK_F32>, dim3(ol.grid), dim3(kBlock), 0,
-                       (hipStream_t)stream, g, rs, ol.stride, partials, acc);
-  } else {
-    static const int resident = resident_blocks(owned_correction_kernel<AXON_MASK_I64>);
-    const OwnedLaunch ol = owned_launch(n_slots, resident);
-    hipLaunchKernelGGL(owned_correction_kernel<AXON_MASK_I64>, dim3(ol.grid), dim3(kBlock), 0,
-                       (hipStream_t)stream, g, rs, ol.stride, partials, acc);
-  }
+  if (mask_kind == AXON_MASK_F32) launch_correction<AXON_MASK_F32, false>(g, rs, acc, partials, (hipStream_t)stream);
+  else launch_correction<AXON_MASK_I64, false>(g, rs, acc, partials, (hipStream_t)stream);
   AXON_CHECK_LAUNCH();
   return AXON_OK;
+}
+
+extern "C" int64_t axon_sampler_correction_diag_workspace_bytes(int64_t n_rows, int64_t n_slots) {
+  if (n_rows < 0 || n_slots < 0) return AXON_ERR_ARG;
+  return diag_workspace_bytes(n_rows, owned_grid_bound(n_slots));
+}
+
+extern "C" int axon_sampler_correction_diag(const float* oldp, const float* samp, const void* mask, int mask_kind,
+                                            const int32_t* cu, int64_t n_rows, int64_t n_slots, int64_t uniform_len,
+                                            int is_mode, float is_thr, int rs_mode, float rs_lr_lo, float rs_lr_hi,
+                                            int has_veto, float log_veto, float is_lo, float is_hi, float rs_lo,
+                                            float rs_hi, float log_is_lo, float log_is_hi, float log_rs_lo,
+                                            float log_rs_hi, float* isw, float* new_mask, float* acc, float* partials,
+                                            float* workspace, double* out, void* stream) {
+  int rc = check_owned_rows(cu, n_rows, n_slots, uniform_len);
+  if (rc != AXON_OK) return rc;
+  if (n_rows == 0 || n_slots == 0) return AXON_ERR_ARG;
+  if (!oldp || !samp || !mask || !new_mask || !acc || !partials || !workspace || !out) return AXON_ERR_ARG;
+  if ((reinterpret_cast<uintptr_t>(oldp) | reinterpret_cast<uintptr_t>(samp) | reinterpret_cast<uintptr_t>(mask) |
+       reinterpret_cast<uintptr_t>(isw) | reinterpret_cast<uintptr_t>(new_mask)) & 15)
+    return AXON_ERR_ARG;
+  if (reinterpret_cast<uintptr_t>(workspace) & 7) return AXON_ERR_WORKSPACE;
+  if (is_mode < 0 || is_mode > 2 || rs_mode < 0 || rs_mode > 3) return AXON_ERR_ARG;
+  if (is_mode != 0 && isw == nullptr) return AXON_ERR_ARG;
+  if (mask_kind != AXON_MASK_F32 && mask_kind != AXON_MASK_I64) return AXON_ERR_ARG;
+  const bool tok = is_mode == 1 || rs_mode == 1;
+  const DiagWorkspace w = diag_workspace(workspace, n_rows, owned_grid_bound(n_slots));
+  const float inf = __builtin_huge_valf();
+  const OwnedCorrArgs g{oldp, samp, mask, CorrCfg{is_mode, is_thr, rs_mode, rs_lr_lo, rs_lr_hi, has_veto, log_veto},
+                        isw, new_mask, w.row_vals, w.row_vals + 3 * n_rows, nullptr, w.row_vals + 4 * n_rows,
+                        w.row_vals + 5 * n_rows, is_lo, is_hi, rs_lo, rs_hi, rs_mode == 1 ? rs_lr_lo : -inf,
+                        rs_mode == 1 ? rs_lr_hi : inf, w.partials};
+  const RowStarts rs{cu, uniform_len, n_rows, n_slots};
+  const hipStream_t st = (hipStream_t)stream;
+  unsigned grid;
+  if (mask_kind == AXON_MASK_F32)
+    grid = tok ? launch_correction<AXON_MASK_F32, true>(g, rs, acc, partials, st)
+               : launch_correction<AXON_MASK_F32, false>(g, rs, acc, partials, st);
+  else
+    grid = tok ? launch_correction<AXON_MASK_I64, true>(g, rs, acc, partials, st)
+               : launch_correction<AXON_MASK_I64, false>(g, rs, acc, partials, st);
+  AXON_CHECK_LAUNCH();
+  DiagCfg cfg;
+  cfg.is_mode = is_mode; cfg.rs_mode = rs_mode; cfg.with_gap = 0;
+  cfg.is_lo = is_lo; cfg.is_hi = is_hi; cfg.rs_lo = rs_lo; cfg.rs_hi = rs_hi;
+  cfg.log_is_lo = log_is_lo; cfg.log_is_hi = log_is_hi;
+  cfg.log_rs_lo = log_rs_lo; cfg.log_rs_hi = log_rs_hi;
+  return launch_diag_rows(w, (int)grid, n_rows, cfg, out, st);
 }

@@ -308,23 +308,18 @@ def _enqueue_correction(old_log_prob, sampler_log_prob, response_mask, sampler_i
     # copy to the host
     make = torch.zeros if rows.n_slots == 0 else torch.empty
     both = make(4 + _ops.DIAG_OUT + 4, device=old_log_prob.device, dtype=torch.float64)
-    weights, new_mask, _ = _ops.sampler_correction(
-        old_log_prob, sampler_log_prob, response_mask, rows,
-        is_mode=_ops.IS_MODES[sampler_is] if use_is else 0,
-        is_threshold=sampler_is_threshold if use_is else 1.0,
-        rs_mode=_ops.RS_MODES[sampler_rs], rs_lr_lo=rs_lo, rs_lr_hi=rs_hi, log_veto=log_veto, acc=both,
-    )
     is_hi = float(sampler_is_threshold) if use_is else 1.0
     is_lo = 1.0 / is_hi
     rs_hi_t = float(sampler_rs_threshold) if sampler_rs is not None else 1.0
     rs_lo_t = (float(sampler_rs_threshold_lower) if sampler_rs_threshold_lower is not None else 1.0 / rs_hi_t) \
         if sampler_rs is not None else 1.0
-    tok_lo, tok_hi = (rs_lo, rs_hi) if sampler_rs == "token" else (-math.inf, math.inf)
-    _ops.sampler_diag(
-        old_log_prob, sampler_log_prob, response_mask, rows, out=both[4:-4],
-        is_mode=_ops.IS_MODES[sampler_is] if use_is else 0, is_lo=is_lo, is_hi=is_hi,
-        rs_mode=_ops.RS_MODES[sampler_rs], rs_lo=rs_lo_t, rs_hi=rs_hi_t, rs_lr_lo=tok_lo, rs_lr_hi=tok_hi,
-        log_is_lo=_log32(is_lo), log_is_hi=_log32(is_hi), log_rs_lo=_log32(rs_lo_t), log_rs_hi=_log32(rs_hi_t),
+    weights, new_mask = _ops.sampler_correction_diag(
+        old_log_prob, sampler_log_prob, response_mask, rows,
+        is_mode=_ops.IS_MODES[sampler_is] if use_is else 0,
+        is_threshold=sampler_is_threshold if use_is else 1.0,
+        rs_mode=_ops.RS_MODES[sampler_rs], rs_lr_lo=rs_lo, rs_lr_hi=rs_hi, log_veto=log_veto,
+        is_lo=is_lo, is_hi=is_hi, rs_lo=rs_lo_t, rs_hi=rs_hi_t, log_is_lo=_log32(is_lo), log_is_hi=_log32(is_hi),
+        log_rs_lo=_log32(rs_lo_t), log_rs_hi=_log32(rs_hi_t), acc=both, out=both[4:-4],
     )
     return _Correction(old_log_prob, response_mask, rows, weights, new_mask, both, sampler_is, sampler_rs, log_veto,
                        sampler_is_batch_normalize)

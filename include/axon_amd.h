@@ -432,6 +432,19 @@ int axon_sampler_correction(const float* old_logp, const float* sampler_logp, co
  *   maxima [50] e  [51] |pa-ps|  [52] |lr|  [53] IS x  [54] IS |x-1|  [55] RS x  [56] RS |x-1|
  *          [57] IS L  [58] RS L  [59] b-a          minima [60..69]: the same slots ([64],[66] unused) */
 int64_t axon_sampler_diag_workspace_bytes(int64_t n_rows, int64_t n_slots);
+/* axon_sampler_correction_rows and the diagnostics that the metrics of a correction need, in one pass over the tokens and
+ * one over the rows: out[72] as above, of which [2..4], [13..22], [42..49] and the extrema in slots 1, 2 and 9 are not
+ * formed (zero, -inf and +inf), and [1], [5..12] and slot 0 only with token-level weights or rejection.  Restrictions
+ * as for axon_sampler_correction_rows; n_rows > 0 and n_slots > 0.  workspace: any contents,
+ * axon_sampler_correction_diag_workspace_bytes(n_rows, n_slots) bytes, 8-byte aligned. */
+int64_t axon_sampler_correction_diag_workspace_bytes(int64_t n_rows, int64_t n_slots);
+int axon_sampler_correction_diag(const float* old_logp, const float* sampler_logp, const void* mask, int mask_kind,
+                                 const int32_t* cu_seqlens, int64_t n_rows, int64_t n_slots, int64_t uniform_len,
+                                 int is_mode, float is_threshold, int rs_mode, float rs_lr_lo, float rs_lr_hi,
+                                 int has_veto, float log_veto, float is_lo, float is_hi, float rs_lo, float rs_hi,
+                                 float log_is_lo, float log_is_hi, float log_rs_lo, float log_rs_hi, float* is_weights,
+                                 float* new_mask, float* acc, float* partials, float* workspace, double* out,
+                                 void* stream);
 int axon_sampler_diag(const float* old_logp, const float* sampler_logp, const void* mask, int mask_kind,
                       const int32_t* cu_seqlens, int64_t n_rows, int64_t n_slots, int64_t uniform_len,
                       int is_mode, float is_lo, float is_hi, int rs_mode, float rs_lo, float rs_hi,

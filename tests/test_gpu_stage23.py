@@ -1345,3 +1345,50 @@ def test_correction_read_back_with_the_loss_of_an_empty_mask(nan):
                                             sampler_is_weights=z + 3.0))
     with pytest.raises(AssertionError, match="sampler_is_weights"):
         compute_loss_fn(full, "ppo", _CORRECT)
+
+
+# what each kind of metric reads of the 72 values
+_DIAG_ROWS = {"is": [23, 24, 25, 26], "rs": [27, 28, 29, 30, 41]}
+
+
+@pytest.mark.parametrize("is_mode,rs_mode,veto", [(1, 1, True), (1, 0, True), (0, 1, True), (2, 3, False), (2, 2, False),
+                                                  (2, 1, False), (1, 3, True), (0, 0, True), (0, 2, False)])
+@pytest.mark.parametrize("lens,mask_dtype", [([1500], torch.float32), ([7, 0, 3000, 1, 900, 0, 5001, 64, 33], torch.int64),
+                                             ([257] * 40, torch.float32), ([70000, 5, 2049, 2048, 1024, 1023], torch.int64)])
+def test_correction_and_its_diagnostics_in_one_pass(is_mode, rs_mode, veto, lens, mask_dtype):
+    """axon_sampler_correction_diag against the correction and the diagnostics in passes of their own: mask, weights and
+    the eight sums bit for bit, and every value that a correction's metrics read.  Rows of no slot, of less than a vector,
+    of exactly and one beyond a step of the walk, longer than what the registers hold, and a slot count that is no
+    multiple of four."""
+    g = torch.Generator().manual_seed(sum(lens) + is_mode)
+    n = sum(lens)
+    old = (-3 * torch.rand(n, generator=g)).to(DEV)
+    samp = old + (0.02 * torch.randn(n, generator=g) + (torch.rand(n, generator=g) < 0.01) * 3).to(DEV)
+    mask = (torch.rand(n, generator=g) < 0.8).to(mask_dtype).to(DEV)
+    samp[mask == 0] = math.nan  # reaches nothing but its own weight
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(DEV)
+    rows = _ops.rows_of(old, cu)
+    lr = dict(rs_lr_lo=-0.05, rs_lr_hi=0.05) if rs_mode == 1 else dict(rs_lr_lo=-0.01, rs_lr_hi=0.01)
+    kw = dict(is_mode=is_mode, is_threshold=1.02, rs_mode=rs_mode, log_veto=-2.9 if veto else None, **lr)
+    thr = dict(is_lo=1 / 1.02, is_hi=1.02, rs_lo=0.96, rs_hi=1.04, log_is_lo=-0.0198, log_is_hi=0.0198, log_rs_lo=-0.0408,
+               log_rs_hi=0.0392)
+    acc, out = torch.empty(8, device=DEV), torch.empty(72, device=DEV, dtype=torch.float64)
+    isw, nm = _ops.sampler_correction_diag(old, samp, mask, rows, **kw, **thr, acc=acc, out=out)
+    isw2, nm2, acc2 = _ops.sampler_correction(old, samp, mask, rows, **kw)
+    tok = lr if rs_mode == 1 else dict(rs_lr_lo=-math.inf, rs_lr_hi=math.inf)
+    ref = _ops.sampler_diag(old, samp, mask, rows, is_mode=is_mode, rs_mode=rs_mode, **thr, **tok)
+    assert torch.equal(nm, nm2) and torch.equal(acc[:6].nan_to_num(7.0), acc2[:6].nan_to_num(7.0))
+    assert (isw is None) == (isw2 is None) and (isw is None or torch.equal(isw.nan_to_num(7.0), isw2.nan_to_num(7.0)))
+    want = [0]
+    if is_mode == 1:
+        want += [1, 5, 6, 7, 8, 50, 60] + _DIAG_ROWS["is"] + [53, 63, 54]
+    if is_mode == 2:
+        want += _DIAG_ROWS["is"] + [53, 63, 54] + list(range(31, 36)) + [57, 67]
+    if rs_mode == 1:
+        want += [1, 9, 10, 11, 12, 50, 60] + _DIAG_ROWS["rs"] + [55, 65, 56]
+    if rs_mode >= 2:
+        want += _DIAG_ROWS["rs"] + [55, 65, 56] + list(range(36, 41)) + [58, 68]
+    a, b = out[want].cpu(), ref[want].cpu()
+    # fp32 partial sums: runs of at most 16 slots and trees here and there, row sums of up to 70000 slots in runs of
+    # 274; the squares' deviations cancel nothing (all terms are positive), log-ratio row sums do: an absolute bound
+    assert torch.isfinite(a).all() and ((a - b).abs() <= 3e-5 * b.abs() + 1e-6).all(), (want, a, b)
