@@ -619,9 +619,9 @@ def kl_reward(scores, old_log_probs, ref_log_probs, mask, rows: Rows, *, kl_type
 
 def side_terms(entropy, log_probs, ref_log_probs, mask, rows: Rows, *, token_reduce, batch_reduce, kl_type=0,
                kl_plus=0, per_row_token_count=None, num_program_tokens=None, num_program_steps=None,
-               valid_count=None):
+               valid_count=None, acc=None):
     """Aggregated entropy and KL penalty with their gradient arrays.  Returns (acc[8], agg_w | None,
-    grad_kl | None); see axon_side_terms."""
+    grad_kl | None); see axon_side_terms.  ``acc`` as in ``policy_loss``."""
     lib = _lib.load()
     anchor = entropy if entropy is not None else log_probs
     require_device(anchor, "side_terms")
@@ -649,7 +649,8 @@ def side_terms(entropy, log_probs, ref_log_probs, mask, rows: Rows, *, token_red
         )
     agg_w = torch.empty(rows.shape, device=dev, dtype=torch.float32) if ent is not None else None
     grad_kl = torch.empty(rows.shape, device=dev, dtype=torch.float32) if kl_type else None
-    acc = _acc8(rows.n_slots, dev)
+    if acc is None:
+        acc = _acc8(rows.n_slots, dev)
     check(
         lib.axon_side_terms(ptr(ent), ptr(lp), ptr(ref), ptr(mk), mkind, rows.cu_ptr, rows.n_rows, rows.n_slots,
                             rows.uniform_len, ptr(row_scale), 1.0, int(one_pass), ptr(valid if one_pass else None),
@@ -965,8 +966,10 @@ class HeadBlocks:
             raise ValueError(f"HeadBlocks: {len(self.keeps_stash)} stash choices for {len(self.ranges)} blocks")
         self.stash_bytes = self._keep_buffer(dev)
         self.stats = torch.empty(2, n_max, device=dev, dtype=torch.float32)  # lse, entropy_b of the current block
-        # whole-stream outputs; position 0 is a sequence start (the aligned layout writes it from the last row)
-        self.out = torch.zeros(2, max(self.n, 1), device=dev, dtype=torch.float32)
+        # whole-stream outputs; position 0 is a sequence start (the aligned layout writes it from the last row, which
+        # is a later block's where there are several)
+        make = torch.zeros if seq_start is not None and len(self.ranges) > 1 else torch.empty
+        self.out = make(2, max(self.n, 1), device=dev, dtype=torch.float32)
         self.d_hidden = torch.empty_like(hidden)
         self.d_weight = torch.empty_like(weight)
         self.one_block = self.n_groups == 1  # one weight-gradient GEMM: no partial sums to carry
@@ -1079,15 +1082,33 @@ def scale_f32(x, s1, s2=None):
     return out.view(x.shape)
 
 
-def scale_bf16_unless_one(x, scale):
-    """``x *= scale`` in place (bf16 ``x``, ``scale`` a device scalar); no memory traffic when it is exactly 1."""
+def scale_bf16_unless_one(x, y, scale):
+    """``x *= scale`` and ``y *= scale`` in place (bf16, ``scale`` a device scalar); no memory traffic when it is
+    exactly 1."""
     lib = _lib.load()
     require_device(x, "scale_bf16_unless_one")
-    if x.dtype != torch.bfloat16 or not x.is_contiguous():
-        raise ValueError("scale_bf16_unless_one: x must be contiguous bf16")
-    s = scale.detach().to(device=x.device, dtype=torch.float32).reshape(-1)[:1].contiguous()
-    check(lib.axon_scale_bf16_unless_one(ptr(x), int(x.numel()), ptr(s), stream_ptr()), "axon_scale_bf16_unless_one")
-    return x
+    for t in (x, y):
+        if t.dtype != torch.bfloat16 or not t.is_contiguous() or t.device != x.device:
+            raise ValueError("scale_bf16_unless_one: the arrays must be contiguous bf16 on one device")
+    s = scale.detach().reshape(1).to(device=x.device, dtype=torch.float32)
+    check(lib.axon_scale_bf16_pair_unless_one(ptr(x), int(x.numel()), ptr(y), int(y.numel()), ptr(s), stream_ptr()),
+          "axon_scale_bf16_pair_unless_one")
+
+
+def step_grads(grad, acc, agg_w, grad_kl, side, entropy_coef, kl_coef, g_lp, g_en):
+    """One block's upstream gradients into ``g_lp`` / ``g_en`` (slices of the step's arrays); see axon_step_grads."""
+    check(_lib.load().axon_step_grads(ptr(grad), ptr(acc), ptr(agg_w), ptr(grad_kl), ptr(side), float(entropy_coef),
+                                      float(kl_coef), int(g_lp.numel()), ptr(g_lp), ptr(g_en), stream_ptr()),
+          "axon_step_grads")
+
+
+def step_scalars(blocks, entropy_coef, kl_coef, cu, out):
+    """The loss of a step (0-d tensor), its totals into ``out`` (10 doubles); see axon_step_scalars."""
+    loss = torch.empty((), device=blocks.device, dtype=torch.float32)
+    check(_lib.load().axon_step_scalars(ptr(blocks), int(blocks.shape[0]), float(entropy_coef), float(kl_coef), ptr(cu),
+                                        0 if cu is None else int(cu.numel()) - 1, ptr(out), ptr(loss), stream_ptr()),
+          "axon_step_scalars")
+    return loss
 
 
 _LOGITS_DTYPES = {torch.float32: 0, torch.bfloat16: 1}

@@ -27,6 +27,8 @@ import torch
 
 from axon_amd import _lib, _ops
 from axon_amd.trainer.algos.loss.loss import POLICY_LOSS_KINDS, policy_loss_metrics, policy_loss_spec
+from axon_amd.utils.rl.sampler import (compute_sampler_correction_and_add_to_batch, sampler_gap_metrics, sampler_gap_sums,
+                                       start_sampler_correction)
 
 # Tokens per block.  One block's stash is 2 bytes x block x vocab (2.5 GB at 8192 x 151936).  The weight
 # gradient is formed once per group of DEFAULT_DW_GROUP blocks (their bf16 dlogits, 2 bytes x block x vocab
@@ -141,10 +143,15 @@ class _BlockedHeadLoss(torch.autograd.Function):
                              seq_start=spec["seq_start"], vocab_chunk=spec["vocab_chunk"], dw_group=spec["dw_group"],
                              stash=blocks_with_stash(ranges, n, hidden.shape[1], weight.shape[0]),
                              logits=hidden.shape[1] >= KEEP_LOGITS_MIN_HIDDEN, timing=_ops.TIMING)
-        g_lp = torch.zeros(n + 4, device=dev, dtype=torch.float32)
-        want_ent_grad = side is not None and side["entropy_coef"] != 0
-        g_en = torch.zeros(n + 4, device=dev, dtype=torch.float32) if want_ent_grad else None
-        accs, side_accs = [], []
+        # every position is some block's, and a block's backward reads its own
+        g_lp = torch.empty(n + 4, device=dev, dtype=torch.float32)
+        ent_coef = side["entropy_coef"] if side is not None else 0
+        kl_coef = side["kl_coef"] if side is not None and side["kl_type"] else 0
+        g_en = torch.empty(n + 4, device=dev, dtype=torch.float32) if ent_coef != 0 else None
+        # the blocks' sums, [block][loss, side terms][8]
+        accs = (torch.empty if side is not None else torch.zeros)(len(ranges), 16, device=dev, dtype=torch.float32)
+        gap = spec.get("sampler_gap")
+        scalars = torch.empty(10 + (_ops.DIAG_OUT if gap is not None else 0), device=dev, dtype=torch.float64)
 
         out = {}
 
@@ -152,28 +159,18 @@ class _BlockedHeadLoss(torch.autograd.Function):
             """After the last block's loss, before its backward: the step's scalars are complete.  Their readback
             starts here, so that the host can pick them up (and prepare whatever comes next) while the GPU still
             works through the last block's backward."""
-            sums = torch.stack(accs).sum(0) if accs else torch.zeros(8, device=dev)
-            side_sums = torch.stack(side_accs).sum(0) if side_accs else torch.zeros(8, device=dev)
-            loss = sums[0].clone()
-            if side is not None:
-                if side["entropy_coef"] != 0:
-                    loss = loss - side_sums[0] * side["entropy_coef"]
-                if side["kl_type"] and side["kl_coef"] != 0:
-                    loss = loss + side_sums[1] * side["kl_coef"]
-            scalars = [sums[:5].double(), side_sums[:5].double()]
-            if spec.get("after_forward") is not None:  # more scalars from the whole-stream outputs (device tensors)
-                scalars += [t.double().reshape(-1) for t in spec["after_forward"](hb.logprobs, hb.entropy)]
-            if seq_mode and cu_host is None:  # the offsets' ends, checked when the step's scalars are read
-                scalars += [cu[:1].double(), cu[-1:].double()]
-            spec["readback"] = _start_readback(torch.cat(scalars))
-            out.update(loss=loss, sums=sums, side_sums=side_sums)
+            out["loss"] = _ops.step_scalars(accs, ent_coef, kl_coef, cu, scalars)
+            if gap is not None:  # over the whole stream's log-probs
+                sampler_gap_sums(hb.logprobs, *gap, cu, out=scalars[10:])
+            spec["readback"] = _start_readback(scalars)
 
         for k, (lo, hi) in enumerate(slots):
             hb.forward(k)
             cut = lambda t: None if t is None else t.reshape(-1)[lo:hi]  # noqa: E731
             if seq_mode:
                 r0, r1 = spec["row_blocks"][k]
-                rows = _ops.Rows(r1 - r0, hi - lo, 0, (cu[r0:r1 + 1] - cu[r0:r0 + 1]).contiguous(), (hi - lo,))
+                cu_k = cu if len(slots) == 1 else (cu[r0:r1 + 1] - cu[r0:r0 + 1]).contiguous()
+                rows = _ops.Rows(r1 - r0, hi - lo, 0, cu_k, (hi - lo,))
                 per_row = {key: _rows_slice(hp[key], r0, r1)
                            for key in ("per_row_token_count", "num_program_tokens", "num_program_steps")}
             else:
@@ -184,24 +181,21 @@ class _BlockedHeadLoss(torch.autograd.Function):
                 kind, lp_b, cut(tensors["old_log_probs"]), cut(tensors["advantages"]), cut(tensors["response_mask"]),
                 cut(tensors["sampler_is_weights"]), rows, token_reduce=hp["token_reduce"],
                 batch_reduce=hp["batch_reduce"], ratio_lo=hp["ratio_lo"], ratio_hi=hp["ratio_hi"],
-                clip_c=hp["clip_c"], valid_count=hp["valid_count"], **per_row)
-            accs.append(acc)
-            torch.mul(grad.reshape(-1), acc[5], out=g_lp[lo:hi])
+                clip_c=hp["clip_c"], valid_count=hp["valid_count"], acc=accs[k, :8], **per_row)
+            s_acc = agg_w = grad_kl = None
             if side is not None:
                 s_acc, agg_w, grad_kl = _ops.side_terms(
                     hb.entropy[lo:hi], lp_b if side["kl_type"] else None, cut(side["ref"]), cut(side["mask"]), rows,
                     token_reduce=hp["token_reduce"], batch_reduce=hp["batch_reduce"], kl_type=side["kl_type"],
-                    kl_plus=side["kl_plus"], valid_count=side["valid_count"], **per_row)
-                side_accs.append(s_acc)
-                if want_ent_grad:
-                    torch.mul(agg_w.reshape(-1), s_acc[5] * (-side["entropy_coef"]), out=g_en[lo:hi])
-                if side["kl_type"] and side["kl_coef"] != 0:
-                    g_lp[lo:hi].addcmul_(grad_kl.reshape(-1), s_acc[5], value=side["kl_coef"])
+                    kl_plus=side["kl_plus"], valid_count=side["valid_count"], acc=accs[k, 8:], **per_row)
+            _ops.step_grads(grad, acc, agg_w, grad_kl if kl_coef != 0 else None, s_acc, ent_coef, kl_coef, g_lp[lo:hi],
+                            None if g_en is None else g_en[lo:hi])
             if k == len(slots) - 1:
                 finish()
             hb.backward(k, g_lp, g_en)
 
-        loss, sums, side_sums = out["loss"], out["sums"], out["side_sums"]
+        loss = out["loss"]
+        sums, side_sums = scalars[:4].view(torch.float32), scalars[4:8].view(torch.float32)
         ctx.grads = (hb.d_hidden, hb.d_weight)
         ctx.head_workspace_bytes = hb.workspace_bytes
         spec["stash_bytes"], spec["workspace_bytes"], spec["n_blocks"] = hb.stash_bytes, hb.workspace_bytes, len(ranges)
@@ -209,6 +203,7 @@ class _BlockedHeadLoss(torch.autograd.Function):
         log_probs, entropy = hb.logprobs, hb.entropy
         hb.d_hidden = hb.d_weight = None
         ctx.mark_non_differentiable(log_probs, entropy, sums, side_sums)
+        ctx.set_materialize_grads(False)  # no zeros for them in the backward
         return loss, log_probs, entropy, sums, side_sums
 
     @staticmethod
@@ -218,8 +213,9 @@ class _BlockedHeadLoss(torch.autograd.Function):
                                "over once: backward through it a second time is not possible")
         d_hidden, d_weight = ctx.grads
         ctx.grads = None
-        _ops.scale_bf16_unless_one(d_hidden, g_loss)
-        _ops.scale_bf16_unless_one(d_weight, g_loss)
+        if g_loss is None:
+            g_loss = torch.zeros((), device=d_hidden.device)
+        _ops.scale_bf16_unless_one(d_hidden, d_weight, g_loss)
         return d_hidden, d_weight, None
 
 
@@ -319,8 +315,6 @@ def _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, bl
     from axon_amd.models.fsdp_models import loss_from_outputs
     from axon_amd.trainer.algos.loss.registry import _SAMPLER_SWITCHES
     from axon_amd.utils.fsdp.forward_utils import packed_logprobs
-    from axon_amd.utils.rl.sampler import (compute_sampler_correction_and_add_to_batch, sampler_gap_metrics,
-                                           sampler_gap_sums, start_sampler_correction)
 
     loss_fn = meta_info["loss_fn"]
     loss_fn_args = meta_info["loss_fn_args"] or {}
@@ -357,7 +351,7 @@ def _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, bl
 
     sampler_log_prob = b.get("sampler_log_probs", None)
     if sampler_log_prob is not None:  # the gap between the current policy and the sampler (fsdp_models.py:232-241)
-        spec["after_forward"] = lambda lp, _ent: [sampler_gap_sums(lp, sampler_log_prob, side_mask, cu_seqlens)]
+        spec["sampler_gap"] = (sampler_log_prob, side_mask)
     loss, log_prob, entropy, _sums, _side_sums = blocked_head_loss(hidden2, weight, spec)
     b["log_probs"], b["entropys"] = log_prob, entropy
     data.meta_info.update(head_backward="blocked-stash", stash_bytes=spec["stash_bytes"],
@@ -366,23 +360,24 @@ def _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, bl
     host, event = spec["readback"]  # the one readback of the step's scalars, started before the last block's backward
     event.synchronize()
     vals = host.tolist()
+    sums = host[:8].view(torch.float32).tolist()  # eight of the loss, eight of the side terms
     if spec["seq_mode"] and spec["cu_host"] is None:
-        _check_span(vals[-2], vals[-1], int(hidden2.shape[0]))
+        _check_span(vals[8], vals[9], int(hidden2.shape[0]))
     if in_flight is not None:
         corr_metrics = in_flight.metrics()
         if corr_metrics is None:  # no token to correct, and the batch is as it was
             corr_metrics = {}
             # weights under an all-zero mask change nothing, unless they are NaN: without them then
-            if not vals[0] == 0.0:
+            if not sums[0] == 0.0:
                 return _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, block_tokens, vocab_chunk,
                                         dw_group, logit_softcapping, cu_host, correct=False)
-    metrics = {**policy_loss_metrics(spec["kind"], vals[:5]), **corr_metrics}
+    metrics = {**policy_loss_metrics(spec["kind"], sums[:5]), **corr_metrics}
     if sampler_log_prob is not None:
         metrics.update(sampler_gap_metrics(vals[10:], int(cu_seqlens.numel()) - 1))
-    metrics["pg_loss"] = vals[0] * n_micro_batches
-    metrics["entropy"] = vals[5] * n_micro_batches
-    metrics["entropy_token_mean"] = vals[7] / max(vals[9], 1.0)
+    metrics["pg_loss"] = sums[0] * n_micro_batches
+    metrics["entropy"] = sums[8] * n_micro_batches
+    metrics["entropy_token_mean"] = sums[10] / max(sums[12], 1.0)
     if spec["side"]["kl_coef"] != 0:
-        metrics["kl_loss"] = vals[6] * n_micro_batches
+        metrics["kl_loss"] = sums[9] * n_micro_batches
         metrics["kl_coef"] = spec["side"]["kl_coef"]
-    return loss * dp_replicas, metrics
+    return loss if dp_replicas == 1 else loss * dp_replicas, metrics

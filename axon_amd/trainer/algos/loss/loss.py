@@ -24,6 +24,11 @@ from axon_amd.trainer.algos.loss.registry import LossFn, register_loss
 _KIND_PPO, _KIND_GSPO, _KIND_REINFORCE, _KIND_CISPO, _KIND_VALUE = 0, 1, 2, 3, 4
 
 
+def _defined(g_loss, like):
+    """The upstream gradient of a loss whose node does not have undefined gradients filled with zeros."""
+    return torch.zeros((), device=like.device) if g_loss is None else g_loss
+
+
 class _ClippedPolicyLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, log_probs, kind, batch, rows, hp):
@@ -34,13 +39,14 @@ class _ClippedPolicyLoss(torch.autograd.Function):
         ctx.save_for_backward(grad, acc)
         ctx.in_dtype = log_probs.dtype
         ctx.mark_non_differentiable(acc)
+        ctx.set_materialize_grads(False)  # no zeros for it in the backward
         return acc[0].clone(), acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):
         grad, acc = ctx.saved_tensors
         # acc[5]: the 1/denominator a one-pass token-mean leaves to this multiply
-        return _ops.scale_f32(grad, g_loss, acc[5]).to(ctx.in_dtype), None, None, None, None
+        return _ops.scale_f32(grad, _defined(g_loss, grad), acc[5]).to(ctx.in_dtype), None, None, None, None
 
 
 class _ValueLoss(torch.autograd.Function):
@@ -54,12 +60,13 @@ class _ValueLoss(torch.autograd.Function):
         ctx.save_for_backward(grad, acc)
         ctx.in_dtype = vpreds.dtype
         ctx.mark_non_differentiable(acc)
+        ctx.set_materialize_grads(False)
         return 0.5 * acc[0], acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):
         grad, acc = ctx.saved_tensors
-        return _ops.scale_f32(grad, 0.5 * g_loss, acc[5]).to(ctx.in_dtype), None, None, None
+        return _ops.scale_f32(grad, 0.5 * _defined(g_loss, grad), acc[5]).to(ctx.in_dtype), None, None, None
 
 
 def _aggregation(b, config, default_token_reduce: str) -> dict:
@@ -185,12 +192,13 @@ class _GmpoLoss(torch.autograd.Function):
         ctx.save_for_backward(grad)
         ctx.in_dtype = log_probs.dtype
         ctx.mark_non_differentiable(acc)
+        ctx.set_materialize_grads(False)  # no zeros for it in the backward
         return acc[0].clone(), acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):
         (grad,) = ctx.saved_tensors
-        return _ops.scale_f32(grad, g_loss).to(ctx.in_dtype), None, None, None, None
+        return _ops.scale_f32(grad, _defined(g_loss, grad)).to(ctx.in_dtype), None, None, None, None
 
 
 @register_loss(LossFn.GEO_MEAN)
@@ -242,12 +250,13 @@ class _CovPolicyLoss(torch.autograd.Function):
         ctx.save_for_backward(grad, acc)
         ctx.in_dtype = log_probs.dtype
         ctx.mark_non_differentiable(acc)
+        ctx.set_materialize_grads(False)  # no zeros for it in the backward
         return acc[0].clone(), acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):
         grad, acc = ctx.saved_tensors
-        return _ops.scale_f32(grad, g_loss, acc[5]).to(ctx.in_dtype), None, None, None, None
+        return _ops.scale_f32(grad, _defined(g_loss, grad), acc[5]).to(ctx.in_dtype), None, None, None, None
 
 
 def _run_cov(kind: int, data, config, hp: dict, default_token_reduce: str):

@@ -420,13 +420,13 @@ def compute_offpolicy_metrics(old_log_prob, sampler_log_prob, response_mask,
     return _offpolicy_from_diag(d, n_rows)
 
 
-def sampler_gap_sums(log_prob, sampler_log_prob, response_mask, cu_seqlens=None):
+def sampler_gap_sums(log_prob, sampler_log_prob, response_mask, cu_seqlens=None, out=None):
     """The device half of ``compute_sampler_corr_metrics_from_logprobs``: the raw sums as a float64 device tensor
     (no readback), for a caller that collects them with other scalars; ``sampler_gap_metrics`` is the host half."""
     rows = _ops.rows_of(log_prob, cu_seqlens)
     return _ops.sampler_diag(log_prob.detach(), sampler_log_prob, response_mask, rows, is_mode=0, is_lo=1.0, is_hi=1.0,
                              rs_mode=0, rs_lo=1.0, rs_hi=1.0, rs_lr_lo=-math.inf, rs_lr_hi=math.inf, log_is_lo=0.0,
-                             log_is_hi=0.0, log_rs_lo=0.0, log_rs_hi=0.0)
+                             log_is_hi=0.0, log_rs_lo=0.0, log_rs_hi=0.0, out=out)
 
 
 def sampler_gap_metrics(sums: list, n_rows: int) -> dict[str, float]:

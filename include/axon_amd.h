@@ -98,7 +98,7 @@ int64_t axon_lmhead_fwd_workspace_bytes(int64_t n_tokens, int64_t hidden, int64_
  * an invalid shape.  The layout is private to the library and depends on the shape only. */
 int64_t axon_lmhead_stash_bytes(int64_t n_tokens, int64_t hidden, int64_t vocab);
 /* flags[p] = 1 where a non-empty sequence of cu_seqlens[n_seqs + 1] begins, else 0.
- * `flags` holds n_tokens bytes rounded up to a multiple of 4. */
+ * `flags` holds n_tokens bytes rounded up to a multiple of 4, on a 4-byte boundary. */
 int axon_seq_start_flags(const int32_t* cu_seqlens, int64_t n_seqs, int64_t n_tokens,
                          uint8_t* flags, void* stream);
 int axon_lmhead_fwd(const void* hidden_bf16, const void* weight_bf16, const void* labels,
@@ -277,6 +277,18 @@ int axon_lmhead_bwd_dlogit_copies(int64_t hidden, int64_t vocab, int64_t vocab_c
 int64_t axon_lmhead_bwd_dhidden_parts(int64_t n_tokens, int64_t ws_tokens, int64_t hidden, int64_t vocab,
                                       int64_t vocab_chunk, int64_t* reserved);
 int axon_scale_bf16_unless_one(void* x_bf16, int64_t n, const float* scale, void* stream);
+/* The same for two arrays in one launch (either may be empty). */
+int axon_scale_bf16_pair_unless_one(void* x_bf16, int64_t nx, void* y_bf16, int64_t ny, const float* scale, void* stream);
+/* One block of a step, n positions: g_lp = grad * acc[5] + kl_coef * grad_kl * side[5], g_en = -entropy_coef * agg_w * side[5],
+ * from the outputs of axon_policy_loss (grad, acc[8]) and axon_side_terms (agg_w, grad_kl, side[8]).  grad_kl or g_en may be
+ * NULL (no such term); no alignment beyond 4 bytes. */
+int axon_step_grads(const float* grad, const float* acc, const float* agg_w, const float* grad_kl, const float* side,
+                    float entropy_coef, float kl_coef, int64_t n, float* g_lp, float* g_en, void* stream);
+/* The scalars of a step from its blocks' sums [n_blocks][16] (acc[8] of axon_policy_loss, then acc[8] of axon_side_terms):
+ * out (10 doubles, 8-byte aligned): 16 floats, the sums over the blocks in order; [8], [9] the first and last of
+ * cu_seqlens[n_seqs + 1] (0 when NULL).  loss[0] = sum of [0] - entropy_coef * [8] + kl_coef * [9]. */
+int axon_step_scalars(const float* blocks, int64_t n_blocks, float entropy_coef, float kl_coef,
+                      const int32_t* cu_seqlens, int64_t n_seqs, double* out, float* loss, void* stream);
 
 /* Plain bf16 NT GEMM on the same MFMA main loop, out[n][m] = sum_k A[m][k]*B[n][k]
  * (fp32 accumulate, fp32 output).  No reference counterpart: it exists so tests
@@ -526,8 +538,8 @@ int axon_policy_loss(int kind, const float* logp, const float* old_logp, const f
  *   The per-token arrays (logp, old_logp, adv, mask, is_weights, grad; in axon_sampler_correction_rows
  *   old_logp, sampler_logp, mask, is_weights, new_mask) must start on 16-byte boundaries (AXON_ERR_ARG
  *   otherwise): every multiple of four slots is then a 16-byte vector.  cu_seqlens must be non-decreasing
- *   with 0 <= cu_seqlens[r] <= n_slots (not checked on the device: a row that runs backwards or past the
- *   arrays would be read out of bounds).
+ *   with 0 <= cu_seqlens[r] <= n_slots; offsets outside that are taken as the nearer end of it and a row that
+ *   runs backwards as empty, so that nothing is read out of bounds, but the results then mean nothing.
  * partials: workspace of axon_reduce_partials_bytes, ticket counters zero (see there). */
 int axon_policy_loss_rows(int kind, const float* logp, const float* old_logp, const float* adv,
                           const void* mask, int mask_kind, const float* is_weights,

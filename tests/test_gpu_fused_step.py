@@ -455,3 +455,41 @@ def test_fused_step_of_one_block_checks_the_offsets_it_never_reads():
                 fused_head_loss(hid.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(True), ids.to(DEV),
                                 torch.tensor(cu, dtype=torch.int32, device=DEV), data,
                                 {"loss_fn": "gspo", "loss_fn_args": GSPO, "temperature": 1.0, "dp_replicas": 1}, **kw)
+
+
+@pytest.mark.parametrize("n,blocks", [(1, 1), (255, 2), (256, 1), (1027, 5)])
+@pytest.mark.parametrize("ent,kl", [(0.0, 0.0), (0.01, 0.0), (0.0, 0.2), (0.01, 0.2)])
+def test_gradients_and_scalars_between_the_kernels_of_a_step(n, blocks, ent, kl):
+    """axon_step_grads / axon_step_scalars against torch, into slices that begin anywhere and leave their neighbours alone."""
+    from axon_amd import _ops
+    g = torch.Generator().manual_seed(n)
+    grad, agg_w, grad_kl = torch.randn(3, n, generator=g).to(DEV)
+    accs = torch.randn(blocks, 16, generator=g).to(DEV)
+    g_lp, g_en = torch.full((2, n + 7), 9.0, device=DEV)
+    _ops.step_grads(grad, accs[0, :8], agg_w, grad_kl if kl else None, accs[0, 8:], ent, kl, g_lp[3:n + 3],
+                    g_en[3:n + 3] if ent else None)
+    want = grad.double() * accs[0, 5].double() + kl * grad_kl.double() * accs[0, 13].double()
+    assert (g_lp[3:n + 3].double() - want).abs().max() < 1e-5
+    assert (g_lp[:3] == 9).all() and (g_lp[n + 3:] == 9).all() and (g_en[:3] == 9).all() and (g_en[n + 3:] == 9).all()
+    assert not ent or (g_en[3:n + 3].double() + ent * agg_w.double() * accs[0, 13].double()).abs().max() < 1e-6
+    out = torch.full((10,), 9.0, device=DEV, dtype=torch.float64)
+    cu = torch.tensor([0, 5, n + 11], dtype=torch.int32, device=DEV)
+    loss = _ops.step_scalars(accs, ent, kl, cu, out)
+    tot = accs.double().sum(0)
+    assert loss.shape == () and abs(loss.item() - (tot[0] - ent * tot[8] + kl * tot[9]).item()) < 1e-5
+    assert (out[:8].view(torch.float32).double() - tot).abs().max() < 1e-5 and out[8:].tolist() == [0.0, n + 11.0]
+
+
+@pytest.mark.parametrize("lens", [[1], [3, 0, 0, 1, 1, 1, 2, 9], [0, 0, 5], [4] * 300 + [0] * 700 + [1, 2, 3], [5000, 0]])
+def test_sequence_start_flags_and_paired_scaling(lens):
+    from axon_amd import _ops
+    n = sum(lens)
+    cu = torch.tensor([0] + lens).cumsum(0)
+    want = torch.zeros((n + 3) // 4 * 4, dtype=torch.uint8)
+    want[[int(a) for a, b in zip(cu[:-1], cu[1:]) if b > a]] = 1
+    assert torch.equal(_ops.seq_start_flags(cu.int().to(DEV), n).cpu(), want)
+    x, y = torch.randn(8 * n, device=DEV).bfloat16(), torch.randn(264, device=DEV).bfloat16()
+    for s in (1.0, 0.25, 0.0, 3.0):
+        a, b = x.clone(), y.clone()
+        _ops.scale_bf16_unless_one(a, b, torch.tensor(s, device=DEV))
+        assert torch.equal(a, (x.float() * s).bfloat16()) and torch.equal(b, (y.float() * s).bfloat16())
