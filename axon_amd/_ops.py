@@ -435,11 +435,17 @@ def _count_dev(x, dev, n=None, what="count"):
     return t.to(device=dev, dtype=torch.float64).reshape(-1).contiguous()
 
 
+def policy_loss_halves(*, token_reduce, batch_reduce, **_):
+    """Whether ``policy_loss(halve=True)`` returns half the loss: a factor of every token's term where no row has one."""
+    return token_reduce == "sum" and batch_reduce == "token-mean"
+
+
 def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, rows: Rows, *, token_reduce,
                 batch_reduce, ratio_lo, ratio_hi, clip_c, per_row_token_count=None, num_program_tokens=None,
-                num_program_steps=None, valid_count=None, acc=None):
+                num_program_steps=None, valid_count=None, acc=None, halve=False):
     """Forward + gradient of the clipped policy loss.  Returns (acc[8], grad like log_probs); ``acc``: where the
-    eight sums go (zeros when there are no slots), else a tensor of its own.
+    eight sums go (zeros when there are no slots), else a tensor of its own.  ``halve``: half the loss is wanted; a third
+    value says what is left to multiply loss and gradient by (1.0 where ``policy_loss_halves``, else 0.5).
 
     acc[0] is the loss; acc[1:5] are the metric sums; acc[5] is the factor the returned
     gradient still has to be multiplied by (see axon_policy_loss).
@@ -475,7 +481,7 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
                                       ptr(grad), ptr(acc), ptr(_partials(rows.n_slots, dev)), stream_ptr()),
             "axon_policy_loss_rows",
         )
-        return acc, grad
+        return (acc, grad, 0.5) if halve else (acc, grad)
     row_scale = row_mean = None
     if not one_pass:  # very large batches: row pass, row scales, token pass
         cnt, ssum, _ = row_stats(lp, old, mk, rows, want_sum=(kind == 1))
@@ -489,12 +495,12 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
         )
     check(
         lib.axon_policy_loss(kind, ptr(lp), ptr(old), ptr(adv), ptr(mk), mkind, ptr(isw), rows.cu_ptr, rows.n_rows,
-                             rows.n_slots, rows.uniform_len, ptr(row_scale), ptr(row_mean), 1.0, int(one_pass),
+                             rows.n_slots, rows.uniform_len, ptr(row_scale), ptr(row_mean), 0.5 if halve else 1.0, int(one_pass),
                              ptr(valid if one_pass else None), float(ratio_lo), float(ratio_hi), float(clip_c),
                              ptr(grad), ptr(acc), ptr(_partials(rows.n_slots, dev)), stream_ptr()),
         "axon_policy_loss",
     )
-    return acc, grad
+    return (acc, grad, 0.5 if row_scale is not None else 1.0) if halve else (acc, grad)
 
 
 def cov_policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, rows: Rows, *, select_ratio,

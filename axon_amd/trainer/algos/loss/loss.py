@@ -24,6 +24,12 @@ from axon_amd.trainer.algos.loss.registry import LossFn, register_loss
 _KIND_PPO, _KIND_GSPO, _KIND_REINFORCE, _KIND_CISPO, _KIND_VALUE = 0, 1, 2, 3, 4
 
 
+def _loss_of(acc):
+    """``acc[0]`` as a tensor of its own: no view (the caller may change it in place, and nothing reads it again), and
+    no launch that copies it."""
+    return torch.empty(0, device=acc.device, dtype=acc.dtype).set_(acc.untyped_storage(), acc.storage_offset(), ())
+
+
 def _defined(g_loss, like):
     """The upstream gradient of a loss whose node does not have undefined gradients filled with zeros."""
     return torch.zeros((), device=like.device) if g_loss is None else g_loss
@@ -40,7 +46,7 @@ class _ClippedPolicyLoss(torch.autograd.Function):
         ctx.in_dtype = log_probs.dtype
         ctx.mark_non_differentiable(acc)
         ctx.set_materialize_grads(False)  # no zeros for it in the backward
-        return acc[0].clone(), acc
+        return _loss_of(acc), acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):
@@ -50,23 +56,23 @@ class _ClippedPolicyLoss(torch.autograd.Function):
 
 
 class _ValueLoss(torch.autograd.Function):
-    """Half the aggregated value loss; one launch where a product behind ``_ClippedPolicyLoss`` is a copy, a product
-    and an autograd node more."""
+    """Half the aggregated value loss (the kernel halves the terms where it can, which is exact)."""
 
     @staticmethod
     def forward(ctx, vpreds, batch, rows, hp):
-        acc, grad = _ops.policy_loss(_KIND_VALUE, vpreds, batch["old_log_probs"], batch["advantages"],
-                                     batch["response_mask"], None, rows, **hp)
+        acc, grad, ctx.half = _ops.policy_loss(_KIND_VALUE, vpreds, batch["old_log_probs"], batch["advantages"],
+                                               batch["response_mask"], None, rows, halve=True, **hp)
         ctx.save_for_backward(grad, acc)
         ctx.in_dtype = vpreds.dtype
         ctx.mark_non_differentiable(acc)
         ctx.set_materialize_grads(False)
-        return 0.5 * acc[0], acc
+        return (_loss_of(acc) if ctx.half == 1.0 else ctx.half * acc[0]), acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):
         grad, acc = ctx.saved_tensors
-        return _ops.scale_f32(grad, 0.5 * _defined(g_loss, grad), acc[5]).to(ctx.in_dtype), None, None, None
+        g_loss = _defined(g_loss, grad)
+        return _ops.scale_f32(grad, g_loss if ctx.half == 1.0 else ctx.half * g_loss, acc[5]).to(ctx.in_dtype), None, None, None
 
 
 def _aggregation(b, config, default_token_reduce: str) -> dict:
@@ -193,7 +199,7 @@ class _GmpoLoss(torch.autograd.Function):
         ctx.in_dtype = log_probs.dtype
         ctx.mark_non_differentiable(acc)
         ctx.set_materialize_grads(False)  # no zeros for it in the backward
-        return acc[0].clone(), acc
+        return _loss_of(acc), acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):
@@ -237,7 +243,8 @@ def value_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
     loss, acc = _ValueLoss.apply(vpreds, tensors, rows, hp)
     sums = acc.tolist()
     denom = max(sums[4], 1.0)
-    return loss, {"vf_loss": 0.5 * sums[0], "vf_clipfrac": sums[1] / denom, "vpred_mean": sums[2] / denom}
+    half = 1.0 if _ops.policy_loss_halves(**agg) else 0.5
+    return loss, {"vf_loss": half * sums[0], "vf_clipfrac": sums[1] / denom, "vpred_mean": sums[2] / denom}
 
 
 class _CovPolicyLoss(torch.autograd.Function):
@@ -251,7 +258,7 @@ class _CovPolicyLoss(torch.autograd.Function):
         ctx.in_dtype = log_probs.dtype
         ctx.mark_non_differentiable(acc)
         ctx.set_materialize_grads(False)  # no zeros for it in the backward
-        return acc[0].clone(), acc
+        return _loss_of(acc), acc
 
     @staticmethod
     def backward(ctx, g_loss, _g_acc):

@@ -1392,3 +1392,40 @@ def test_correction_and_its_diagnostics_in_one_pass(is_mode, rs_mode, veto, lens
     # fp32 partial sums: runs of at most 16 slots and trees here and there, row sums of up to 70000 slots in runs of
     # 274; the squares' deviations cancel nothing (all terms are positive), log-ratio row sums do: an absolute bound
     assert torch.isfinite(a).all() and ((a - b).abs() <= 3e-5 * b.abs() + 1e-6).all(), (want, a, b)
+
+
+@pytest.mark.parametrize("loss_fn,args", [("ppo", {}), ("gspo", {}), ("geo_mean", {}), ("kl_cov", dict(kl_cov_ratio=0.1)), ("value", {}),
+                                          ("value", dict(token_reduce="mean", batch_reduce="step-mean")),
+                                          ("value", dict(token_reduce="mean"))])
+def test_loss_is_a_tensor_of_its_own(loss_fn, args):
+    """A caller may change the loss in place: the gradient follows, the metrics do not; the value loss is half the
+    aggregated loss, its metric and its gradient too, wherever the factor is applied."""
+    g = torch.Generator().manual_seed(3)
+    x, old, adv = (torch.randn(5, 33, generator=g) for _ in range(3))
+    mask = (torch.rand(5, 33, generator=g) < 0.7).float()
+
+    def run(scale):
+        lp = (old + 0.1 * x).to(DEV).requires_grad_(True)
+        data = DataProto.from_dict(tensors={"log_probs": lp, "old_log_probs": old.to(DEV), "advantages": adv.to(DEV),
+                                            "response_mask": mask.to(DEV), "vpreds": lp, "values": old.to(DEV),
+                                            "returns": adv.to(DEV)})
+        loss, metrics = compute_loss_fn(data, loss_fn, args)
+        assert loss._base is None and loss.shape == ()
+        if scale != 1.0:
+            loss *= scale
+        loss.backward()
+        return loss.item(), lp.grad, metrics
+
+    (l1, g1, m1), (l3, g3, m3) = run(1.0), run(4.0)
+    assert l3 == 4.0 * l1 and torch.equal(g3, 4.0 * g1) and m1 == m3
+    if loss_fn == "value":
+        v = (old + 0.1 * x).double().requires_grad_(True)
+        clip = old.double() + (v - old.double()).clamp(-0.5, 0.5)
+        per = torch.maximum((v - adv.double()) ** 2, (clip - adv.double()) ** 2) * mask.double()
+        if args.get("token_reduce"):
+            per = per.sum(1) / mask.double().sum(1).clamp_min(1.0)
+        den = 5.0 if args.get("batch_reduce") else mask.double().sum()  # every row has a token
+        ref = 0.5 * per.sum() / den
+        ref.backward()
+        assert l1 == pytest.approx(ref.item(), rel=1e-5) and m1["vf_loss"] == pytest.approx(ref.item(), rel=1e-5)
+        assert rel_l2(g1, v.grad) < 1e-5
