@@ -37,9 +37,10 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 // Forward: tile epilogue -> partial statistics
 // ----------------------------------------------------------------------------
 struct FwdParams {
-  float* pm;   // [parts][n_tokens] running max, in log2 units of the scaled logit
-  float* ps;   // sum 2^(x*c - max)
-  float* pe;   // sum (x*c - max) * 2^(x*c - max)
+  // [parts][n_tokens][3]: running max in log2 units of the scaled logit, sum 2^(x*c - max), sum (x*c - max) * 2^(x*c - max);
+  // side by side, so that sixteen tokens of a part are 192 contiguous bytes for the kernel that folds them
+  float* stats;
+  float* pm;   // [parts][n_tokens]: the max once more, where the backward reads it (null: it does not)
   int n_tokens, vocab;
   float c;     // inv_temperature * log2(e)
   float cap, inv_cap;  // logit soft-capping cap * tanh(logit / cap) (SOFTCAP kernels only)
@@ -95,8 +96,8 @@ __device__ __forceinline__ void merge_stats(float M, float& s, float& e, float M
                                             float e2, float Mn) {
   const float d1 = M - Mn, d2 = M2 - Mn;
   const float f1 = fast_exp2(d1), f2 = fast_exp2(d2);
-  e = f1 * fmaf(s, d1, e) + f2 * fmaf(s2, d2, e2);
-  s = s * f1 + s2 * f2;
+  e = fmaf(f1, fmaf(s, d1, e), f2 * fmaf(s2, d2, e2));  // written out: the same roundings wherever this is inlined
+  s = fmaf(s, f1, s2 * f2);
 }
 
 // All-reduce over the four 16-lane rows of the wavefront (lanes l, l^16, l^32, l^48: the four lanes that hold
@@ -145,10 +146,12 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
     e = rows_all_reduce(e, add);
     const int n = t.n0 + lp.n(j);
     if (lp.lq == 0 && n < p.n_tokens) {
-      const int64_t o = (int64_t)part * p.n_tokens + n;
-      p.pm[o] = M;
-      p.ps[o] = s;
-      p.pe[o] = e;
+      const int64_t at = (int64_t)part * p.n_tokens + n;
+      float* const o = p.stats + at * 3;
+      o[0] = M;
+      o[1] = s;
+      o[2] = e;
+      if (STASH) p.pm[at] = M;
     }
   };
   float* const mine = lds + lp.wave * 1024 + lp.lane;  // per wavefront: 8 x 64 of each of the two sums
@@ -337,77 +340,86 @@ __global__ __launch_bounds__(256) void seq_start_kernel(const int32_t* __restric
 
 // The last kernel of the forward: folds a token's partials into lse, entropy_b and entropy, forms the label's
 // logit and with it logprob[n] = softcap(hidden[n] . W[label[n]]) / T - lse[n].
-// A workgroup of 1024 threads owns 16 * PER consecutive tokens (a thread PER of them, 16 apart); its 64 thread groups each fold every 64th partial of a
-// token (four loads ahead of the fold), so that the chain of dependent folds is 19 long for 151936 vocabulary
-// rows (149 with eight groups of 32 tokens).  Groups of one wavefront are folded by lane exchanges, the wavefronts
-// through LDS in order: the same order whatever the number of tokens.  The label dots (one wavefront per token) run
-// before the barrier, beside the folds of the other wavefronts.  PER = 2 (both halves of a 128-byte line by the same
-// thread) once a workgroup per 16 tokens would be more than one per CU.
-// 187 tokens x 896 x 151936: 11.0 us where separate merge and label kernels took 18.7 + 5.2; 700 x 4096: 19.4 for
-// 26.0 + 7.4; 8192 x 4096: 51 for 33.2 + 23.3.
-constexpr int kFinishTokens = 16;
-template <int PER, typename LabelT>
+// A token's partials are folded in 256 groups, group c taking c, c + 256, ... (a chain of five for 151936 vocabulary rows); sixteen
+// neighbouring groups are folded as a tree, the sixteen results one after the other.  That order is the same whatever T and
+// PER, hence whatever the number of tokens.  A workgroup of 1024 threads owns T * PER consecutive tokens, a thread 256 * T / 1024
+// groups of PER tokens (T apart) with eight partials requested before the first is folded: T = 4 up to 1024 tokens, to put a
+// short call on as many compute units as there are; T = 16 beyond, PER = 2 once a workgroup per 16 tokens would be
+// more than one per CU.  The label dots (one wavefront per token) run before the barrier, beside the folds of the other wavefronts.
+// 187 tokens x 896 x 151936 5.9 us (11.0 with three arrays of partials, 64 groups and 16 tokens per workgroup), 700 x 4096 11.9
+// (19.0), 1500 x 896 9.8 (12.8), 3001 x 2880 x 201088 22.5 (31.4), 8192 x 4096 41.4 (49.0).
+template <int T, int PER, typename LabelT>
 __global__ __launch_bounds__(1024) void lmhead_finish_kernel(
-    const float* __restrict__ pm, const float* __restrict__ ps, const float* __restrict__ pe,
-    int parts, const __bf16* __restrict__ hidden, const __bf16* __restrict__ weight,
+    const float* __restrict__ stats, int parts, const __bf16* __restrict__ hidden, const __bf16* __restrict__ weight,
     const LabelT* __restrict__ labels, int n_tokens, int hidden_sz, int vocab, float inv_temp, float cap,
     float* __restrict__ lse, float* __restrict__ entropy_b, float* __restrict__ entropy,
     float* __restrict__ logprobs, const uint8_t* __restrict__ is_start, int last_dst) {
-  constexpr int TOK = kFinishTokens * PER, kGroups = 1024 / kFinishTokens, kWaves = 16;
+  constexpr int TOK = T * PER, kWaves = 16, kGroups = 256, SUB = kGroups * T / 1024;
+  constexpr int kDeep = 8 / (SUB * PER) < 1 ? 1 : 8 / (SUB * PER);
   __shared__ float red[3][kWaves][TOK];
   __shared__ float dots[TOK];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int grp = threadIdx.x / kFinishTokens;
+  const int grp = threadIdx.x / T * SUB;  // this thread's groups: grp .. grp + SUB - 1
   int nc[PER];
 #pragma unroll
   for (int t = 0; t < PER; ++t)  // a valid token; the results of those beyond the last are dropped below
-    nc[t] = min(blockIdx.x * TOK + t * kFinishTokens + (int)(threadIdx.x % kFinishTokens), n_tokens - 1);
+    nc[t] = min(blockIdx.x * TOK + t * T + (int)(threadIdx.x % T), n_tokens - 1);
+  // the first token's label is on its way while the partials are folded
+  int64_t lab = 0;
+  const int n_dot = blockIdx.x * TOK + wave;
+  if (wave < TOK && n_dot < n_tokens) lab = (int64_t)labels[aligned_pos(n_dot, n_tokens, is_start, last_dst)];
   // a group beyond the number of partials holds an empty set (s = 0 below any reference)
-  float M[PER], s[PER], e[PER];
+  float M[SUB][PER], s[SUB][PER], e[SUB][PER];
 #pragma unroll
-  for (int t = 0; t < PER; ++t) { M[t] = kEmptyMax; s[t] = 0.f; e[t] = 0.f; }
+  for (int g = 0; g < SUB; ++g)
+#pragma unroll
+    for (int t = 0; t < PER; ++t) { M[g][t] = kEmptyMax; s[g][t] = 0.f; e[g][t] = 0.f; }
   auto fold = [](float& M1, float& s1, float& e1, float M2, float s2, float e2) {
     const float Mn = fmaxf(M1, M2);
     merge_stats(M1, s1, e1, M2, s2, e2, Mn);
     M1 = Mn;
   };
-  int q = grp;
-  for (; q + 3 * kGroups < parts; q += 4 * kGroups) {
-    float M2[4][PER], s2[4][PER], e2[4][PER];
+  for (int q0 = grp; q0 < parts; q0 += kDeep * kGroups) {
+    float x[kDeep][SUB][PER][3];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < kDeep; ++u)
 #pragma unroll
-      for (int t = 0; t < PER; ++t) {
-        const int64_t o = (int64_t)(q + u * kGroups) * n_tokens + nc[t];
-        M2[u][t] = pm[o]; s2[u][t] = ps[o]; e2[u][t] = pe[o];
+      for (int g = 0; g < SUB; ++g)
+#pragma unroll
+        for (int t = 0; t < PER; ++t) {
+          const float* o = stats + ((int64_t)min(q0 + u * kGroups + g, parts - 1) * n_tokens + nc[t]) * 3;
+          x[u][g][t][0] = o[0]; x[u][g][t][1] = o[1]; x[u][g][t][2] = o[2];
+        }
+#pragma unroll
+    for (int u = 0; u < kDeep; ++u)
+#pragma unroll
+      for (int g = 0; g < SUB; ++g) {
+        if (q0 + u * kGroups + g >= parts) continue;
+#pragma unroll
+        for (int t = 0; t < PER; ++t)
+          fold(M[g][t], s[g][t], e[g][t], x[u][g][t][0], x[u][g][t][1], x[u][g][t][2]);
       }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int t = 0; t < PER; ++t) fold(M[t], s[t], e[t], M2[u][t], s2[u][t], e2[u][t]);
-  }
-  for (; q < parts; q += kGroups) {
-#pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int64_t o = (int64_t)q * n_tokens + nc[t];
-      fold(M[t], s[t], e[t], pm[o], ps[o], pe[o]);
-    }
   }
 #pragma unroll
   for (int t = 0; t < PER; ++t) {
 #pragma unroll
-    for (int off = kFinishTokens; off < 64; off <<= 1)
-      fold(M[t], s[t], e[t], __shfl_xor(M[t], off), __shfl_xor(s[t], off), __shfl_xor(e[t], off));
-    if (lane < kFinishTokens) {
-      const int tok = t * kFinishTokens + lane;
-      red[0][wave][tok] = M[t]; red[1][wave][tok] = s[t]; red[2][wave][tok] = e[t];
+    for (int off = 1; off < SUB; off <<= 1)
+#pragma unroll
+      for (int g = 0; g < SUB; g += 2 * off)
+        fold(M[g][t], s[g][t], e[g][t], M[g + off][t], s[g + off][t], e[g + off][t]);
+#pragma unroll
+    for (int off = T; off < 64; off <<= 1)
+      fold(M[0][t], s[0][t], e[0][t], __shfl_xor(M[0][t], off), __shfl_xor(s[0][t], off), __shfl_xor(e[0][t], off));
+    if (lane < T) {
+      const int tok = t * T + lane;
+      red[0][wave][tok] = M[0][t]; red[1][wave][tok] = s[0][t]; red[2][wave][tok] = e[0][t];
     }
   }
 
   for (int k = wave; k < TOK; k += kWaves) {  // label dots
     const int nk = blockIdx.x * TOK + k;
     if (nk >= n_tokens) break;
-    const int64_t lab = (int64_t)labels[aligned_pos(nk, n_tokens, is_start, last_dst)];
+    if (k != wave) lab = (int64_t)labels[aligned_pos(nk, n_tokens, is_start, last_dst)];
     float dot = 0.f;
     if (lab >= 0 && lab < vocab) {
       const uint4* h = reinterpret_cast<const uint4*>(hidden + (int64_t)nk * hidden_sz);
@@ -1229,19 +1241,15 @@ int set_lds(K kernel) {
   } while (0)
 
 struct FwdWs {
-  float *pm, *ps, *pe;
+  float* stats;
   int parts;
   int64_t bytes;
 };
 FwdWs fwd_ws(int64_t n, int64_t vocab, void* base) {
   FwdWs w;
   w.parts = (int)(round_up(vocab, kTile) / kTile) * 2;
-  const int64_t one = round_up((int64_t)w.parts * n * 4, kAlign);
-  char* p = static_cast<char*>(base);
-  w.pm = reinterpret_cast<float*>(p);
-  w.ps = reinterpret_cast<float*>(p + one);
-  w.pe = reinterpret_cast<float*>(p + 2 * one);
-  w.bytes = 3 * one;
+  w.stats = static_cast<float*>(base);
+  w.bytes = round_up((int64_t)w.parts * n * 12, kAlign);
   return w;
 }
 
@@ -1533,6 +1541,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
   if ((base - static_cast<char*>(workspace)) + w.bytes > ws_bytes) return AXON_ERR_WORKSPACE;
   const hipStream_t st = (hipStream_t)stream;
   StashWs sw{};
+  float* pm = nullptr;
   if (stash) {
     if (reinterpret_cast<uintptr_t>(stash) & 15) return AXON_ERR_ARG;
     if (keep == kKeepLogits) {
@@ -1544,7 +1553,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
       if (!is_block && !stash_of_all_tokens(n, h, v)) return AXON_ERR_SHAPE;
       sw = stash_ws(n, v, stash);
       if (sw.bytes > stash_bytes) return AXON_ERR_WORKSPACE;
-      w.pm = sw.pm;  // the backward needs the per-part maxima: they live in the stash
+      pm = sw.pm;  // the backward needs the per-part maxima as well: they live in the stash
     }
   }
 
@@ -1552,7 +1561,7 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
   g.a = static_cast<const __bf16*>(weight);  g.lda = h;  g.m_rows = (int)v;
   g.b = static_cast<const __bf16*>(hidden);  g.ldb = h;  g.n_rows = (int)n;
   g.k = (int)h;
-  FwdParams p{w.pm, w.ps, w.pe, (int)n, (int)v, inv_temp * kLog2e, softcap,
+  FwdParams p{w.stats, pm, (int)n, (int)v, inv_temp * kLog2e, softcap,
               softcap > 0.f ? 1.f / softcap : 0.f, sw.tiles, dma_ok(g) ? halved_tiles(n, v) : 0};
   {
     Span span(timer, 0);
@@ -1571,17 +1580,20 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
     }
   }
   Span span(timer, 1);
-#define AXON_FINISH(PER, LabelT)                                                                                 \
-  hipLaunchKernelGGL((lmhead_finish_kernel<PER, LabelT>),                                                        \
-                     dim3((unsigned)((n + kFinishTokens * PER - 1) / (kFinishTokens * PER))), dim3(1024), 0, st, \
-                     w.pm, w.ps, w.pe, w.parts, static_cast<const __bf16*>(hidden),                              \
-                     static_cast<const __bf16*>(weight), static_cast<const LabelT*>(labels), (int)n, (int)h,     \
-                     (int)v, inv_temp, softcap, lse, entropy_b, entropy, logprobs, is_start, (int)last_dst)
-  if (n > kFinishTokens * kCus) {
-    if (labels_i64) AXON_FINISH(2, int64_t); else AXON_FINISH(2, int32_t);
-  } else {
-    if (labels_i64) AXON_FINISH(1, int64_t); else AXON_FINISH(1, int32_t);
-  }
+#define AXON_FINISH(T, PER)                                                                                       \
+  do {                                                                                                           \
+    const dim3 grid((unsigned)((n + T * PER - 1) / (T * PER)));                                                  \
+    if (labels_i64) AXON_FINISH_L(T, PER, int64_t); else AXON_FINISH_L(T, PER, int32_t);                         \
+  } while (0)
+#define AXON_FINISH_L(T, PER, LabelT)                                                                            \
+  hipLaunchKernelGGL((lmhead_finish_kernel<T, PER, LabelT>), grid, dim3(1024), 0, st, w.stats, w.parts,          \
+                     static_cast<const __bf16*>(hidden), static_cast<const __bf16*>(weight),                     \
+                     static_cast<const LabelT*>(labels), (int)n, (int)h, (int)v, inv_temp, softcap, lse,         \
+                     entropy_b, entropy, logprobs, is_start, (int)last_dst)
+  if (n <= 4 * kCus) AXON_FINISH(4, 1);
+  else if (n <= 16 * kCus) AXON_FINISH(16, 1);
+  else AXON_FINISH(16, 2);
+#undef AXON_FINISH_L
 #undef AXON_FINISH
   AXON_CHECK_LAUNCH();
   return AXON_OK;

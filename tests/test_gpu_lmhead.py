@@ -1101,3 +1101,18 @@ def test_output_products_with_a_half_filled_last_tile(n, h, v, chunk):
         err, size = (a.cpu().double() - ref.double()).norm(dim=0), ref.double().norm(dim=0)
         # bf16 dlogits and bf16 results: 2^-9 each, and both norms over at least 70 entries of a column
         assert (err < 2e-2 * size).all(), (err / size).max()
+
+
+@pytest.mark.parametrize("v", [1000, 40000, 70001])
+def test_statistics_do_not_depend_on_the_number_of_tokens(v):
+    """The kernel that folds the partial statistics takes 4, 16 or 32 tokens per workgroup: a token's results are the same
+    bits in a call of 7, 1024, 1025, 4096 or 4097 tokens; vocabularies of 8, 314 and 548 partials (of 256 groups)."""
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(4097, 64, v, seed=v))
+    w = (w.float() * 6).bfloat16()
+    whole = _ops.lmhead_forward(hid, w, lab, 1.0 / 0.7)
+    for n in (7, 1024, 1025, 4096):
+        for a, b in zip(_ops.lmhead_forward(hid[:n], w, lab[:n], 1.0 / 0.7), whole):
+            assert torch.equal(a, b[:n]) and torch.isfinite(a).all()
+    logp = torch.log_softmax(hid[:64].double() @ w.double().T / 0.7, -1)
+    assert (whole[0][:64].double() - logp.gather(1, lab[:64, None].long())[:, 0]).abs().max() < 1e-4
+    assert (whole[1][:64].double() + (logp.exp() * logp).sum(-1)).abs().max() < 1e-4
