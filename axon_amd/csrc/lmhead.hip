@@ -472,6 +472,9 @@ struct DlogitParams {
   __bf16* dlT;   // [chunk_cols][n_pad]   vocab-major; null: not wanted (the dWeight GEMM reads dl as a K-major operand)
   int64_t ld_dl, ld_dlT;
   int n_tokens, vocab, v_begin;  // v_begin: first vocab row of this chunk
+  // Rows of dl from here on (a multiple of 64, at least n_tokens) are read by nobody and need not be written: sixty-four or
+  // a hundred and twenty-eight of them are left out together.  The zeros between n_tokens and n_end are k of the weight gradient.
+  int n_end;
   float inv_temp;
   float cap, inv_cap;  // soft-capping (SOFTCAP kernels only)
   const uint8_t* is_start;  // token-aligned packed layout (see aligned_pos), or null
@@ -600,8 +603,11 @@ __device__ __forceinline__ void dlogit_store(AccTile& acc, const DlogitParams& p
 // rows of a wavefront's sub-tile; staged row = token - 16 * j0.  SOFTCAP: the stash describes the capped
 // logit, whose derivative factor is 1 - (capped / cap)^2.  EDGE: entries beyond the last token or the last
 // vocabulary row are staged as zeros.
+// ENT: the entropies have a gradient.  Without one (and without soft-capping) the logit itself is not needed, and the
+// logarithm that recovers it is half of the vector work: 333 tokens x 1024 x 50257 36.8 us for 42.7, 300 x 896 x 151936 58.7
+// for 66.9 (rows beyond n_end left out as well), 700 x 4096 83 for 94; from some thousand tokens on memory bounds both.
 constexpr int kStashHalfBlocks = kBlocks / 2;
-template <bool SOFTCAP, bool EDGE>
+template <bool SOFTCAP, bool ENT, bool EDGE>
 __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashHalfBlocks], int j0,
                                                    const float* __restrict__ pm, int part,
                                                    const DlogitParams& p, const LanePos& lp,
@@ -626,8 +632,9 @@ __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashH
       for (int r = 0; r < 4; ++r) {
         const int mrel = lp.m(i, r);
         const float pr = wv[r] * scale;
-        const float raw = (__builtin_amdgcn_logf(fmaxf(wv[r], 1e-30f)) + Mp) * inv_c;
-        float v = pr * fmaf(k.cb, raw, k.ca);
+        float raw = 0.f;
+        if (SOFTCAP || ENT) raw = (__builtin_amdgcn_logf(fmaxf(wv[r], 1e-30f)) + Mp) * inv_c;
+        float v = pr * (ENT ? fmaf(k.cb, raw, k.ca) : k.ca);
         if (mrel == k.lab_rel) v += k.gl;
         if (SOFTCAP) {
           const float th = raw * p.inv_cap;
@@ -759,6 +766,7 @@ __device__ __forceinline__ void dlogit_body(const GemmOperands& g, const DlogitP
   __syncthreads();  // every wave is past its last main-loop LDS access
 
   const LanePos lp;
+  if (t.n0 + lp.wn * kWaveTile >= p.n_end) return;
   char* const stage = smem + lp.wave * 32768;
   if (t.n0 + kTile > p.n_tokens || p.v_begin + t.m0 + kTile > p.vocab)
     dlogit_store<SOFTCAP, true>(acc, p, lp, t, stage);
@@ -792,7 +800,7 @@ struct StashSource {
   int tiles_n, tm0;
 };
 
-template <bool SOFTCAP>
+template <bool SOFTCAP, bool ENT>
 __global__ __launch_bounds__(64) void lmhead_dlogit_stash_kernel(DlogitParams p, StashSource src) {
   __shared__ __align__(16) char stage[kStashHalfBlocks * kBlk * 256];  // 64 tokens x 128 bf16
   const int half = blockIdx.x & 1, wave = (blockIdx.x >> 1) & 3, tile = blockIdx.x >> 3;
@@ -803,6 +811,7 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_stash_kernel(DlogitParams p,
   lp.wm = wave >> 1;
   lp.wn = wave & 1;
   const int j0 = half * kStashHalfBlocks;
+  if (t.n0 + lp.wn * kWaveTile + j0 * kBlk >= p.n_end) return;
   const uint4* sv = src.stash + ((int64_t)(tm * src.tiles_n + tn) * 4 + wave) * kStashWaveVecs +
                     j0 * 4 * 64 + lp.lane;
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -816,9 +825,9 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_stash_kernel(DlogitParams p,
   t.m0 -= p.v_begin;
   const int part = tm * 2 + lp.wm;
   if (edge) {
-    dlogit_stage_stash<SOFTCAP, true>(st, j0, src.pm, part, p, lp, t, stage);
+    dlogit_stage_stash<SOFTCAP, ENT, true>(st, j0, src.pm, part, p, lp, t, stage);
   } else {
-    dlogit_stage_stash<SOFTCAP, false>(st, j0, src.pm, part, p, lp, t, stage);
+    dlogit_stage_stash<SOFTCAP, ENT, false>(st, j0, src.pm, part, p, lp, t, stage);
   }
   dlogit_copy_out_half(stage, j0, p, lp, t);
 }
@@ -835,6 +844,7 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_logits_kernel(DlogitParams p
   lp.wm = wave >> 1;
   lp.wn = wave & 1;
   const int j0 = half * kStashHalfBlocks;
+  if (t.n0 + lp.wn * kWaveTile + j0 * kBlk >= p.n_end) return;
   const uint4* sv = src.stash + ((int64_t)(tm * src.tiles_n + tn) * 4 + wave) * kLogitsWaveVecs +
                     j0 * kBlocks * 64 + lp.lane;
   float4 x[kStashHalfBlocks * kBlocks];
@@ -1676,7 +1686,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   for (int ci = 0; ci < w.chunks; ++ci) {
     const int64_t v0 = (int64_t)ci * w.chunk;
     const int64_t vc = (v - v0 < w.chunk) ? (v - v0) : w.chunk;  // valid vocab rows in this chunk
-    // B1: dlogit for vocab rows [v0, v0 + vc); whole tiles, zeros beyond the last token and vocabulary row
+    // B1: dlogit for vocab rows [v0, v0 + vc); zeros beyond the last token (up to n_end) and the last vocabulary row
     {
       Span span(timer, 1);
       GemmOperands g;
@@ -1691,12 +1701,17 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       p.cap = softcap; p.inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;
       p.is_start = is_start;
       p.last_dst = (int)blk.last_dst;
+      // a block with others behind it in the same weight-gradient GEMM: whole tiles, its rows lie between theirs
+      p.n_end = (int)(blk.dw_now ? n_red : n_tile);
       if (stash) {
         const StashSource src{sw.tiles, sw.pm, sw.tiles_n, (int)(v0 / kTile)};
         const unsigned blocks = (unsigned)(round_up(vc, kTile) / kTile) * (unsigned)sw.tiles_n * 8u;
         auto* const kernel = blk.keep == kKeepLogits
                                  ? (softcap > 0.f ? lmhead_dlogit_logits_kernel<true> : lmhead_dlogit_logits_kernel<false>)
-                                 : (softcap > 0.f ? lmhead_dlogit_stash_kernel<true> : lmhead_dlogit_stash_kernel<false>);
+                             : softcap > 0.f
+                                 ? (dentropy ? lmhead_dlogit_stash_kernel<true, true> : lmhead_dlogit_stash_kernel<true, false>)
+                                 : (dentropy ? lmhead_dlogit_stash_kernel<false, true>
+                                             : lmhead_dlogit_stash_kernel<false, false>);
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, st, p, src);
         AXON_CHECK_LAUNCH();
       } else if (softcap > 0.f) {

@@ -1116,3 +1116,32 @@ def test_statistics_do_not_depend_on_the_number_of_tokens(v):
     logp = torch.log_softmax(hid[:64].double() @ w.double().T / 0.7, -1)
     assert (whole[0][:64].double() - logp.gather(1, lab[:64, None].long())[:, 0]).abs().max() < 1e-4
     assert (whole[1][:64].double() + (logp.exp() * logp).sum(-1)).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("v", [2000, 1001])
+@pytest.mark.parametrize("keep", [dict(stash=True), dict(stash=False, logits=True), dict(stash=False)])
+@pytest.mark.parametrize("ranges,ent", [([(0, 300)], False), ([(0, 65)], True), ([(0, 300), (300, 520)], False),
+                                        ([(0, 130), (130, 200), (200, 264)], True)])
+def test_dlogit_rows_that_nobody_writes_are_read_by_nobody(ranges, ent, keep, v):
+    """dl rows beyond a block's tokens are written as far as a weight-gradient GEMM reads them: up to the next multiple of
+    64, or to the tile's end where other blocks of the group follow.  With NaN all over the workspace before each
+    backward the gradients are those of one over zeros; with and without a gradient of the entropies."""
+    n, h = ranges[-1][1], 256
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(n, h, v, seed=n))
+    w = (w.float() * 6).bfloat16()
+    g_lp, g_en = torch.randn(2, n + 4, generator=torch.Generator().manual_seed(n)).to(DEV)
+
+    def run(fill):
+        hb = _ops.HeadBlocks(hid, w, lab, 1.0, ranges, dw_group=len(ranges), **keep)
+        for k in range(len(ranges)):
+            if k == 0 or hb.dw_group == 1:
+                hb.bwd_ws.fill_(fill)
+            hb.forward(k)
+            hb.backward(k, g_lp, g_en if ent else None)
+        return hb.d_hidden, hb.d_weight
+
+    for a, b in zip(run(255), run(0)):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+    ref = OM.backward(g_lp[:n].cpu(), g_en[:n].cpu() if ent else None, hid.cpu(), w.cpu(), lab.cpu())
+    for a, r in zip(run(255), ref):
+        assert rel_l2(a, r) < 2e-2
