@@ -33,7 +33,7 @@
 //      and on the accumulators of dropped rows).
 //      Shifting edge tiles back inside the matrix instead needed 256 rows on both
 //      sides (a forward over 187 tokens, 896 x 151936, ran on RegLoop: 355 us per call
-//      against 89 now).
+//      against 89 with the DMA loop).
 //  * RegLoop<32>  (k % 64 == 32, which the 64-wide k-tiles above do not divide, and operands whose
 //      rows lie closer together than a k-tile or off a 16-byte boundary):
 //      loads through registers with per-row clamping.

@@ -7,7 +7,8 @@ the 6 that count.  Here the three stages run block of consecutive tokens by bloc
 vocabulary keeps 2 bytes per logit (``axon_lmhead_fwd``'s stash), the loss kernels run on the block's positions
 with the batch-wide denominators, the block's backward decodes its dlogits from the stash, and the next block
 reuses the same stash buffer.  What is held from a forward to its backward is one block's stash, a fixed number of
-bytes whatever the number of tokens, and no logit is computed twice.
+bytes whatever the number of tokens, and no logit is computed twice.  (A block without a stash, see
+``blocks_with_stash``, keeps its fp32 logits or recomputes them, see ``KEEP_LOGITS_MIN_HIDDEN``.)
 
 Everything the loss needs from outside a block is known before the first block: the sampler correction reads
 only ``old_log_probs`` / ``sampler_log_probs`` (it runs once, over the whole batch), and the denominators of
