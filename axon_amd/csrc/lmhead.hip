@@ -1516,10 +1516,13 @@ int launch_transpose(const void* in, int64_t ld_in, int rows, int cols, void* ou
 // The forward's tiles that are computed in halves of 128 vocabulary rows: those of a last round that would occupy at
 // most half of the compute units, so that it takes half as long.  594 tiles, 2.3 rounds: 187 tokens x 896 x 151936 87 us
 // for 80, 187 x 4096 305 for 288; 128 tiles (250 x 2048 x 32768) 44 for 35.  A last round over more than half of
-// them would become two.
+// them would become two.  Not behind many whole rounds, which then no longer split evenly over the XCDs' ranges of the
+// walk and read more from beyond the L2 (8192 x 4096 x 151936 18 to 21 GB for 15).  Whole / half, ms, at hidden 4096 x 151936:
+// 9.3 rounds 0.942 / 0.907, 16.2 1.574 / 1.545, 32.5 3.068 / 3.034, 37.1 3.581 / 3.609, 74.3 6.99 / 7.13.
+constexpr int64_t kHalvedRounds = 36;
 int halved_tiles(int64_t n, int64_t v) {
   const int64_t tiles = (round_up(v, kTile) / kTile) * (round_up(n, kTile) / kTile), rest = tiles % kCus;
-  return rest <= kCus / 2 ? (int)rest : 0;
+  return rest <= kCus / 2 && tiles < kHalvedRounds * kCus ? (int)rest : 0;
 }
 
 template <bool SOFTCAP>
