@@ -86,9 +86,12 @@ def _zeros(n, device, dtype=torch.float32):
     return torch.zeros(n, device=device, dtype=dtype)
 
 
-def _acc8(n_slots, device):
-    """The eight scalar sums a kernel returns; the library writes all of them unless there are no tokens.  Under
-    stream capture they start as NaN: a replay whose reduction never finished would then show."""
+def _acc8(n_slots, device, acc=None):
+    """The eight scalar sums a kernel returns, in ``acc`` where the caller has a place for them; the library writes all of
+    them unless there are no tokens.  Under stream capture they start as NaN: a replay whose reduction never finished
+    would then show."""
+    if acc is not None:
+        return acc.zero_() if n_slots == 0 else acc
     if n_slots == 0:
         return _zeros(8, device)
     if torch.cuda.is_current_stream_capturing():
@@ -462,8 +465,7 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
 
     valid = _count_dev(valid_count, dev)
     grad = torch.empty(rows.shape, device=dev, dtype=torch.float32)
-    if acc is None:
-        acc = _acc8(rows.n_slots, dev)
+    acc = _acc8(rows.n_slots, dev, acc)
     # PPO with sum / token-mean needs no per-row quantity: one pass over the tokens, the
     # division by the token count happens when the last workgroup has the total.
     one_pass = kind != 1 and tr == 0 and br == 0
@@ -655,8 +657,7 @@ def side_terms(entropy, log_probs, ref_log_probs, mask, rows: Rows, *, token_red
         )
     agg_w = torch.empty(rows.shape, device=dev, dtype=torch.float32) if ent is not None else None
     grad_kl = torch.empty(rows.shape, device=dev, dtype=torch.float32) if kl_type else None
-    if acc is None:
-        acc = _acc8(rows.n_slots, dev)
+    acc = _acc8(rows.n_slots, dev, acc)
     check(
         lib.axon_side_terms(ptr(ent), ptr(lp), ptr(ref), ptr(mk), mkind, rows.cu_ptr, rows.n_rows, rows.n_slots,
                             rows.uniform_len, ptr(row_scale), 1.0, int(one_pass), ptr(valid if one_pass else None),

@@ -493,3 +493,30 @@ def test_sequence_start_flags_and_paired_scaling(lens):
         a, b = x.clone(), y.clone()
         _ops.scale_bf16_unless_one(a, b, torch.tensor(s, device=DEV))
         assert torch.equal(a, (x.float() * s).bfloat16()) and torch.equal(b, (y.float() * s).bfloat16())
+
+
+@pytest.mark.parametrize("n,block_tokens,blocks", [(257, 256, 2), (1025, 512, 3)])
+@pytest.mark.parametrize("case", ["ppo", "dapo-entropy-kl"])
+def test_a_block_that_owns_no_position_adds_nothing(case, n, block_tokens, blocks, monkeypatch):
+    """Positions are shifted by one against rows: a last block of one row owns none of them, and no kernel writes its sums.
+    With NaN in every new tensor the step is that of one block: loss, metrics, outputs and gradients (the stash rounds
+    softmax numerators to fp16 where the odd single block has fp32 logits)."""
+    from axon_amd.models.fused_head_loss import token_blocks
+    assert token_blocks(n, block_tokens)[-1] == (n - 1, n) and len(token_blocks(n, block_tokens)) == blocks
+    lens = [n - 150, 50, 37, 63]
+    hid, w, ids, labels, rl, old, ref = _inputs(n, 64, 300, lens, seed=n, group=2)
+    args = {"ppo": PPO, "dapo-entropy-kl": DAPO_SIDE}[case]
+    want = fused_step(hid, w, ids, rl, old, ref, "ppo", args, 4096, adv_shift=0.5)
+    empty, empty_like = torch.empty, torch.empty_like
+    as_nan = lambda t: t.fill_(float("nan")) if t.is_cuda and t.is_floating_point() else t  # noqa: E731
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: as_nan(empty(*a, **k)))
+    monkeypatch.setattr(torch, "empty_like", lambda *a, **k: as_nan(empty_like(*a, **k)))
+    got = fused_step(hid, w, ids, rl, old, ref, "ppo", args, block_tokens, adv_shift=0.5)
+    assert got[2].meta_info["n_blocks"] == blocks and want[2].meta_info["n_blocks"] == 1
+    assert got[0].item() == pytest.approx(want[0].item(), rel=1e-4)
+    assert set(got[1]) == set(want[1])
+    for k, x in want[1].items():
+        assert got[1][k] == pytest.approx(x, rel=1e-4, abs=1e-6), k
+    for k in ("log_probs", "entropys"):
+        assert (got[2].batch[k] - want[2].batch[k]).abs().max() < 1e-5
+    assert rel_l2(got[3], want[3]) < 5e-3 and rel_l2(got[4], want[4]) < 5e-3
