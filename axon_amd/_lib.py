@@ -52,6 +52,7 @@ SIGNATURES: dict[str, tuple] = {
     "axon_lmhead_bwd_dlogit_copies": (_i32, [_i64, _i64, _i64]),
     "axon_lmhead_bwd_dlogit_copies_of": (_i32, [_i64, _i64, _i64, _i64]),
     "axon_lmhead_bwd_dhidden_parts": (_i64, [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
+    "axon_lmhead_bwd_half_tiles": (_i32, [_i64, _i64, _i64, _i64, _i64]),
     "axon_scale_bf16_unless_one": (_i32, [_ptr, _i64, _ptr, _ptr]),
     "axon_scale_bf16_pair_unless_one": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr]),
     "axon_step_grads": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _f32, _f32, _i64, _ptr, _ptr, _ptr]),

@@ -866,23 +866,23 @@ __global__ __launch_bounds__(64) void lmhead_dlogit_logits_kernel(DlogitParams p
 // Backward B2/B3 and the plain GEMM: store the tile as out[n][m]
 // ----------------------------------------------------------------------------
 struct StoreParams {
-  float* out_f32;     // [n][ld_f32] fp32 output (may be null)
-  __bf16* out_bf16;   // [n][ld_bf16] (may be null)
-  int64_t ld_f32, ld_bf16;
-  int m_valid, n_valid;
-  int accumulate;     // add the previous contents of tile_acc first
-  int keep_f32;       // write the sum back to tile_acc (0: it is only read, the sum leaves as bf16)
+  float* out_f32 = nullptr;    // [n][ld_f32] fp32 output (may be null)
+  __bf16* out_bf16 = nullptr;  // [n][ld_bf16] (may be null)
+  int64_t ld_f32 = 0, ld_bf16 = 0;
+  int m_valid = 0, n_valid = 0;
+  int accumulate = 0;  // add the previous contents of tile_acc first
+  int keep_f32 = 0;    // write the sum back to tile_acc (0: it is only read, the sum leaves as bf16)
   // fp32 partial sums (the weight gradient carried from one token block to the next, dHidden carried from one
   // vocabulary chunk to the next or formed in parts): kept per tile in the order the accumulators lie in the registers, so that every
   // wavefront load and store is one contiguous kilobyte.  float4 index =
   // ((tile * 4 + wave) * 64 + i * 8 + j) * 64 + lane, tile = tm * tiles_n + tn.  Null: not used.
-  float4* tile_acc;
+  float4* tile_acc = nullptr;
   // Split reduction: `splits` workgroups per tile, each over `k_split` (a multiple of 64) of the k; they leave their
   // partial sums in tile_acc, one array of tiles after the other, for split_sum_kernel.
-  int splits, k_split;
+  int splits = 1, k_split = 0;
   // The last tile of an m that fills at most half of it is computed as half a tile (DmaLoopT's BM).  Its rows lie in
   // tile_acc where a whole tile leaves them, the other half of the tile is left as it was.
-  int half_edge;
+  int half_edge = 0;
 };
 constexpr int64_t kTileAccVecs = 4 * kBlocks * kBlocks * 64;  // float4 per tile (256 KB)
 
@@ -1331,10 +1331,12 @@ SplitPlan split_plan(int64_t tiles, int64_t k) {
 // it no longer shares operand slices in the L2 (dWeight more than dHidden, whose parts keep an XCD on one part of k).
 // Whole / half, ms: dWeight hidden 896 (4 tiles) 3001 tokens (47 k-tiles) 0.671 / 0.611, 8192 1.67 / 1.58, 12288 2.53 / 2.45,
 // 16381 3.42 / 3.47; hidden 2880 (12 tiles) 700 tokens 0.847 / 0.789, 3001 2.60 / 2.57, 6007 4.92 / 4.96, 16381
-// 13.1 / 13.9.  dHidden 896 6007 tokens (297 k-tiles) 1.25 / 1.16, 16381 (792) 3.13 / 2.99; 2880 3001 tokens (629) 2.56 / 2.53,
-// 8192 (1571) 6.56 / 6.57, 16381 (3142) 13.0 / 13.2.
+// 13.1 / 13.9.  dHidden 896 6007 tokens (297 k-tiles) 1.28 / 1.20, 16381 (792) 3.26 / 3.13; 2880 3001 tokens (629) 2.66 / 2.64,
+// 6007 (1571) 6.21 / 6.22, 8192 (1571) 6.72 / 6.76, 16381 (3142) 13.3 / 13.5.
 constexpr int64_t kHalfEdgeDw = 768, kHalfEdgeDh = 12288;  // most k-tiles times tiles
-bool half_edge(int64_t k, int64_t tiles_m, int64_t most) { return (k + 63) / 64 * tiles_m <= most; }
+bool half_edge(int64_t k, int64_t h, int64_t most) {
+  return (h - 1) % kTile < kTile / 2 && (k + 63) / 64 * (round_up(h, kTile) / kTile) <= most;
+}
 
 struct BwdWs {
   __bf16 *hT, *dl, *dlT;
@@ -1400,6 +1402,15 @@ DhPlan dh_plan(const BwdWs& w, int64_t n, int64_t h, int64_t v) {
   const int64_t tiles = (round_up(h, kTile) / kTile) * (round_up(n, kTile) / kTile);
   const SplitPlan split = split_plan(tiles, w.chunks > 1 ? w.chunk : v);
   return DhPlan{split, (w.chunks > 1 || split.splits > 1) ? tiles * split.splits : 0};
+}
+
+// Which of the backward's two output products take half tiles: dHidden, each of whose parts reduces over k_split of the
+// vocabulary, and dWeight, which reduces over k_dw tokens (the partial sums that are carried from block to block hold
+// whole tiles: `carried`).  A hidden size below a tile has no half tiles, nor has dWeight from the vocab-major copy.
+struct HalfEdges { bool dh, dw; };
+HalfEdges half_edges(const BwdWs& w, const SplitPlan& dh, int64_t h, int64_t k_dw, bool carried) {
+  return HalfEdges{h >= kTile && half_edge(dh.k_split, h, kHalfEdgeDh),
+                   w.dl_kmajor && !carried && half_edge(k_dw, h, kHalfEdgeDw)};
 }
 
 // Bytes for a call over `n` tokens.  The default chunk shrinks in steps while n grows, so a shorter call can need a
@@ -1684,6 +1695,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
   }
   const int64_t n_red = round_up(n, 64);  // reduction length of B3 (from this block's first token)
   const int64_t tiles_h = round_up(h, kTile) / kTile;
+  const HalfEdges half = half_edges(w, plan, h, pos + n_red, blk.dw_mode != kDwStore);
   __bf16* const dl = w.dl + pos * w.ld_c;  // this block's rows
 
   for (int ci = 0; ci < w.chunks; ++ci) {
@@ -1732,12 +1744,11 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       g.k = (int)vc;
       const bool last = (ci == w.chunks - 1), split = plan.splits > 1;
       StoreParams sp;
-      sp.out_f32 = nullptr;  sp.ld_f32 = 0;
       sp.out_bf16 = (last && !split) ? static_cast<__bf16*>(d_hidden) : nullptr;  sp.ld_bf16 = h;
       sp.m_valid = (int)h; sp.n_valid = (int)n;
       sp.tile_acc = (w.chunks > 1 || split) ? w.dh_acc : nullptr;
       sp.accumulate = (ci > 0); sp.keep_f32 = split || !last;
-      sp.half_edge = half_edge(sp.k_split, tiles_h, kHalfEdgeDh);
+      sp.half_edge = half.dh;
       // a shorter last chunk reaches the first parts only
       sp.k_split = plan.k_split;
       sp.splits = (int)((vc + sp.k_split - 1) / sp.k_split);
@@ -1762,7 +1773,6 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       g.n_rows = (int)vc;
       g.k = (int)(pos + n_red);
       StoreParams sp;
-      sp.out_f32 = nullptr;  sp.ld_f32 = 0;
       sp.tile_acc = blk.dw_mode == kDwStore
                         ? nullptr
                         : reinterpret_cast<float4*>(blk.dw_acc) + (v0 / kTile) * tiles_h * kTileAccVecs;
@@ -1771,8 +1781,7 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       sp.accumulate = blk.dw_mode == kDwAdd || blk.dw_mode == kDwLast;
       sp.keep_f32 = blk.dw_mode != kDwLast;
       sp.splits = 1; sp.k_split = g.k;
-      sp.half_edge = blk.dw_mode == kDwStore &&  // the carried sums hold whole tiles
-                     half_edge(g.k, tiles_h, kHalfEdgeDw);
+      sp.half_edge = half.dw;
       rc = launch_store_kmajor(g, sp, false, w.dl_kmajor, st);
       if (rc != AXON_OK) return rc;
     }
@@ -1959,9 +1968,9 @@ extern "C" int axon_gemm_nt_bf16(const void* a, int64_t lda, const void* b, int6
   g.b = static_cast<const __bf16*>(b);  g.ldb = ldb;  g.n_rows = (int)n;
   g.k = (int)k;
   StoreParams sp;
-  sp.out_f32 = out; sp.ld_f32 = ldo; sp.out_bf16 = nullptr; sp.ld_bf16 = 0;
-  sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 0; sp.tile_acc = nullptr;
-  sp.splits = 1; sp.k_split = (int)k; sp.half_edge = 0;
+  sp.out_f32 = out; sp.ld_f32 = ldo;
+  sp.m_valid = (int)m; sp.n_valid = (int)n;
+  sp.k_split = (int)k;
   return launch_store(g, sp, (hipStream_t)stream);
 }
 
@@ -1984,9 +1993,9 @@ extern "C" int axon_gemm_bf16(const void* a, int64_t lda, int a_kmajor, const vo
   g.k = (int)k;
   if (!gemm_kmajor_domain(g, a_kmajor != 0, b_kmajor != 0)) return AXON_ERR_SHAPE;
   StoreParams sp;
-  sp.out_f32 = out; sp.ld_f32 = ldo; sp.out_bf16 = nullptr; sp.ld_bf16 = 0;
-  sp.m_valid = (int)m; sp.n_valid = (int)n; sp.accumulate = 0; sp.keep_f32 = 0; sp.tile_acc = nullptr;
-  sp.splits = 1; sp.k_split = (int)k; sp.half_edge = 0;
+  sp.out_f32 = out; sp.ld_f32 = ldo;
+  sp.m_valid = (int)m; sp.n_valid = (int)n;
+  sp.k_split = (int)k;
   return launch_store_kmajor(g, sp, a_kmajor != 0, b_kmajor != 0, (hipStream_t)stream);
 }
 
@@ -2030,6 +2039,16 @@ extern "C" int64_t axon_lmhead_bwd_dhidden_parts(int64_t n, int64_t ws_tokens, i
   const BwdWs w = bwd_ws(ws_tokens, h, v, chunk, nullptr);
   *reserved = w.dh_parts;
   return n > 0 ? dh_plan(w, n, h, v).parts : 0;
+}
+
+extern "C" int axon_lmhead_bwd_half_tiles(int64_t n, int64_t ws_tokens, int64_t h, int64_t v, int64_t chunk) {
+  int rc = check_head_shape(n, h, v);
+  if (rc == AXON_OK) rc = check_head_shape(ws_tokens, h, v);
+  if (rc != AXON_OK) return rc;
+  if (n == 0 || chunk < 0 || chunk % kTile != 0 || n > ws_tokens) return AXON_ERR_ARG;
+  const BwdWs w = bwd_ws(ws_tokens, h, v, chunk, nullptr);
+  const HalfEdges half = half_edges(w, dh_plan(w, n, h, v).split, h, round_up(n, 64), false);
+  return (half.dh ? 1 : 0) + (half.dw ? 2 : 0);
 }
 
 extern "C" int axon_lmhead_block_can_group(int64_t h, int64_t v, int64_t chunk) {

@@ -276,6 +276,9 @@ int axon_lmhead_bwd_dlogit_copies(int64_t hidden, int64_t vocab, int64_t vocab_c
  * fewer (a call would return AXON_ERR_WORKSPACE).  n_tokens <= ws_tokens; negative for an unsupported shape. */
 int64_t axon_lmhead_bwd_dhidden_parts(int64_t n_tokens, int64_t ws_tokens, int64_t hidden, int64_t vocab,
                                       int64_t vocab_chunk, int64_t* reserved);
+/* Which of the two output products of such a call over n_tokens > 0 computes a last tile of 256 hidden columns that is at
+ * most half filled as half a tile: 1 = dHidden, 2 = dWeight (where no sums are carried from another block), 3 = both. */
+int axon_lmhead_bwd_half_tiles(int64_t n_tokens, int64_t ws_tokens, int64_t hidden, int64_t vocab, int64_t vocab_chunk);
 int axon_scale_bf16_unless_one(void* x_bf16, int64_t n, const float* scale, void* stream);
 /* The same for two arrays in one launch (either may be empty). */
 int axon_scale_bf16_pair_unless_one(void* x_bf16, int64_t nx, void* y_bf16, int64_t ny, const float* scale, void* stream);

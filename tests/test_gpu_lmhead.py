@@ -14,7 +14,7 @@ import math
 import pytest
 import torch
 
-from axon_amd import _ops, workloads as W
+from axon_amd import _lib, _ops, workloads as W
 from axon_amd.utils.kernel.linear_cross_entropy import linear_cross_entropy
 from axon_amd.utils.torch.fused_linear import FusedLinearForPPO
 from oracle import lmhead as OM
@@ -1101,6 +1101,27 @@ def test_output_products_with_a_half_filled_last_tile(n, h, v, chunk):
         err, size = (a.cpu().double() - ref.double()).norm(dim=0), ref.double().norm(dim=0)
         # bf16 dlogits and bf16 results: 2^-9 each, and both norms over at least 70 entries of a column
         assert (err < 2e-2 * size).all(), (err / size).max()
+
+
+@pytest.mark.parametrize("n,v,chunk", [(300, 8200, 0), (70, 1000, 512), (520, 2056, 0)])
+@pytest.mark.parametrize("h", [320, 384, 640])
+def test_half_tiles_of_the_output_products_give_the_bits_of_whole_ones(n, v, chunk, h):
+    """The same call with hidden states that end in zeros up to whole tiles has the same dlogits, parts and order of
+    additions, and computes its last columns in whole tiles: every column of both gradients is equal bit for bit."""
+    whole = -(-h // 256) * 256
+    ask = lambda h: _lib.load().axon_lmhead_bwd_half_tiles(n, n, h, v, chunk)  # noqa: E731
+    assert ask(h) == 3 and ask(whole) == 0
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(n, whole, v, seed=h + v))
+    w = (w.float() * 8).bfloat16()
+    hid[:, h:] = 0
+    g_lp, g_en = torch.randn(2, n, generator=torch.Generator().manual_seed(h)).to(DEV)
+
+    def grads(hidden, weight):
+        _, _, lse, eb = _ops.lmhead_forward(hidden, weight, lab, 1.0)[:4]
+        return _ops.lmhead_backward(g_lp, g_en, hidden, weight, lab, lse, eb, 1.0, vocab_chunk=chunk)
+
+    for a, b in zip(grads(hid[:, :h].contiguous(), w[:, :h].contiguous()), grads(hid, w)):
+        assert torch.equal(a, b[:, :h]) and a.float().norm() > 0
 
 
 @pytest.mark.parametrize("v", [1000, 40000, 70001])

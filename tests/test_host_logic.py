@@ -376,6 +376,26 @@ def test_split_reduction_of_d_hidden_fits_its_workspace():
     assert parts_of(2, 1, 64, 4096, 0, ctypes.byref(room)) < 0 and parts_of(1, 1, 64, 4096, 100, ctypes.byref(room)) < 0
 
 
+def test_which_output_products_take_half_tiles():
+    """The rule that the backward launches by, on both sides of each of its limits: 12288 k-tiles times tiles for dHidden (12
+    tiles of hidden 2880: parts of 65536 vocabulary rows, four chunks with one answer), 768 for dWeight (4096 tokens; 12288
+    at the 4 tiles of hidden 896)."""
+    from axon_amd import _lib
+    ask = _lib.load().axon_lmhead_bwd_half_tiles
+    dh = lambda n, h, v, chunk=0: ask(n, n, h, v, chunk) & 1  # noqa: E731
+    dw = lambda n, h, v, chunk=0: ask(n, n, h, v, chunk) >> 1  # noqa: E731
+    assert dh(16384, 2880, 201088, 65536) == 1 and dh(16384, 2880, 201088, 65792) == 0
+    assert dh(16381, 2880, 201088, 201216) == 0 and dh(8192, 2880, 201088, 201216) == 0  # one chunk: 3142, 1571 k-tiles
+    assert dh(3001, 2880, 201088, 201216) == 1 and dh(16381, 896, 151936, 152064) == 1   # parts of 629 and 792
+    assert dw(4096, 2880, 50264) == 1 and dw(4097, 2880, 50264) == 0
+    assert dw(12288, 896, 151936) == 1 and dw(12289, 896, 151936) == 0
+    assert dw(700, 2880, 50257) == 0                                       # vocab-major copy of the dlogits
+    filled = {32: 0, 128: 0, 256: 0, 288: 3, 384: 3, 416: 0, 512: 0, 640: 3, 672: 0}
+    assert {h: ask(300, 300, h, 8200, 0) for h in filled} == filled
+    assert ask(300, 8192, 640, 8200, 8448) == 3                            # a block shorter than the workspace
+    assert ask(0, 0, 640, 8200, 0) < 0 and ask(2, 1, 640, 8200, 0) < 0 and ask(1, 1, 640, 8200, 100) < 0
+
+
 @pytest.mark.parametrize("h,v", [(896, 151936), (2880, 201088), (4096, 151936), (3072, 128264), (1024, 50257),
                                  (2048, 102400), (256, 262144), (1024, 65800), (128, 40000), (512, 1310720)])
 def test_default_backward_workspace_grows_with_the_tokens_and_stays_bounded(h, v):
