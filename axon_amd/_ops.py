@@ -759,6 +759,13 @@ def lmhead_stash_bytes(n: int, h: int, v: int) -> int:
     return max(0, int(_lib.load().axon_lmhead_stash_bytes(int(n), int(h), int(v))))
 
 
+def _fits_twice(need, dev) -> bool:
+    """Whether ``need`` bytes are at most half of what tensors on ``dev`` can still take: free there, or held by torch's
+    allocator without use (asked only where it matters: its statistics cost the host 80 us, the free memory 4)."""
+    free, _total = torch.cuda.mem_get_info(dev)
+    return 2 * need <= free or 2 * need <= free + torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
+
+
 def _want_stash(n, h, v, dev) -> int:
     """Bytes of the stash to allocate under the module's policy, or 0."""
     if LMHEAD_STASH is False or n == 0:
@@ -768,11 +775,8 @@ def _want_stash(n, h, v, dev) -> int:
         return need
     if need > LMHEAD_STASH_MAX_BYTES:
         return 0
-    if not torch.cuda.is_current_stream_capturing():
-        free, _total = torch.cuda.mem_get_info(dev)
-        reusable = torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
-        if need > (free + reusable) // 2:
-            return 0
+    if not torch.cuda.is_current_stream_capturing() and not _fits_twice(need, dev):
+        return 0
     return need
 
 
@@ -937,7 +941,8 @@ class HeadBlocks:
     dlogits are decoded from a stash (softmax numerators in 16 bits) or formed from logits in fp32, for all
     blocks or one truth value per block.  ``logits``: the same choice for the blocks without a stash, whether their fp32
     logits are kept from the forward (4 bytes x block x vocab, shared by the blocks as the stash is) or recomputed:
-    the same bits either way.  Recomputed where the device has no memory for them."""
+    the same bits either way.  Recomputed where they would take more than half of the memory that is left beside every other
+    buffer of the blocks."""
 
     def __init__(self, hidden, weight, labels, inv_temperature, ranges, *, softcap=0.0, seq_start=None,
                  vocab_chunk=0, stash=True, logits=False, dw_group=2, timing: "Timer | None" = None):
@@ -971,7 +976,6 @@ class HeadBlocks:
         self.keeps_stash, self.keeps_logits = per_block(stash), per_block(logits)
         if len(self.keeps_stash) != len(self.ranges) or len(self.keeps_logits) != len(self.ranges):
             raise ValueError(f"HeadBlocks: {len(self.keeps_stash)} stash choices for {len(self.ranges)} blocks")
-        self.stash_bytes = self._keep_buffer(dev)
         self.stats = torch.empty(2, n_max, device=dev, dtype=torch.float32)  # lse, entropy_b of the current block
         # whole-stream outputs; position 0 is a sequence start (the aligned layout writes it from the last row, which
         # is a later block's where there are several)
@@ -983,6 +987,7 @@ class HeadBlocks:
         self.dw_acc_bytes = 0 if self.one_block else int(self.lib.axon_lmhead_block_dw_acc_bytes(self.h, self.v))
         self.dw_acc = torch.empty(self.dw_acc_bytes // 4, device=dev, dtype=torch.float32) if self.dw_acc_bytes else None
         self.block_stash_bytes = self.block_logits_bytes = 0
+        self.stash_bytes = self._keep_buffer(dev)  # last: kept logits may not cost the step a buffer that it needs
         self.workspace_bytes = self.fwd_ws_bytes + self.bwd_ws_bytes + self.stash_bytes + self.dw_acc_bytes
 
     @property
@@ -1002,10 +1007,14 @@ class HeadBlocks:
         return int(self.lib.axon_lmhead_block_logits_bytes(n1 - n0, self.h, self.v)) if keep else 0
 
     def _keep_buffer(self, dev):
-        """Allocate what a block keeps from its forward to its backward, for the largest block; its size."""
+        """Allocate what a block keeps from its forward to its backward, for the largest block; its size.  Logits leave as
+        much memory as they take to what the step allocates after this (its loss arrays are a few bytes per token, the
+        logits 4 per token and vocabulary row)."""
         stash = max((self._stash_bytes(b - a) for (a, b), keep in zip(self.ranges, self.keeps_stash) if keep), default=0)
         size = max([stash] + [self._logits_bytes(k) for k in range(len(self.ranges))])
         try:
+            if size > stash and not torch.cuda.is_current_stream_capturing() and not _fits_twice(size, dev):
+                raise torch.OutOfMemoryError("no room for the logits")
             self.stash = torch.empty(size, device=dev, dtype=torch.uint8) if size else None
         except torch.OutOfMemoryError:
             if size == stash:

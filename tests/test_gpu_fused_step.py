@@ -520,3 +520,42 @@ def test_a_block_that_owns_no_position_adds_nothing(case, n, block_tokens, block
     for k in ("log_probs", "entropys"):
         assert (got[2].batch[k] - want[2].batch[k]).abs().max() < 1e-5
     assert rel_l2(got[3], want[3]) < 5e-3 and rel_l2(got[4], want[4]) < 5e-3
+
+
+@pytest.mark.parametrize("refused", ["later allocations", "the logits", "nothing"])
+def test_kept_logits_give_way_to_what_the_step_cannot_do_without(refused, monkeypatch):
+    """A step that fits without its blocks' fp32 logits fits with the choice to keep them: the other buffers are there before
+    them, and they are not kept where they would leave little room.  The same bits either way."""
+    import weakref
+    lens = [150, 50, 37, 64]
+    n, h, v = sum(lens), 768, 1000
+    hid, w, ids, labels, rl, old, ref = _inputs(n, h, v, lens, seed=9, group=2)
+    step = lambda: fused_step(hid, w, ids, rl, old, ref, "ppo", DAPO_SIDE, 8192)  # noqa: E731
+    want = step()
+    need = 4 * 2 * 262144  # four vocabulary tiles, two token tiles
+    assert want[2].meta_info["stash_bytes"] == need
+    if refused != "later allocations":  # half of the room is what they take, or a byte less
+        allocated = torch.cuda.memory_allocated
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev: (need, 4 * need))
+        monkeypatch.setattr(torch.cuda, "memory_reserved",
+                            lambda dev: allocated(dev) + need - (refused == "the logits"))
+    else:
+        kept = [None]
+
+        def guard(make):
+            def made(*a, **k):
+                t = make(*a, **k)
+                size = t.numel() * t.element_size()
+                if t.is_cuda and size >= 65536 and kept[0] is not None and kept[0]() is not None:
+                    raise torch.OutOfMemoryError("no room beside the logits")
+                if t.is_cuda and t.dtype == torch.uint8 and size == need:
+                    kept[0] = weakref.ref(t)
+                return t
+            return made
+
+        for name in ("empty", "empty_like", "zeros"):
+            monkeypatch.setattr(torch, name, guard(getattr(torch, name)))
+    got = step()
+    assert got[2].meta_info["stash_bytes"] == (0 if refused == "the logits" else need)
+    assert torch.equal(got[0], want[0]) and got[1] == want[1]
+    assert torch.equal(got[3], want[3]) and torch.equal(got[4], want[4])
