@@ -333,18 +333,26 @@ def _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, bl
     if loss_fn in POLICY_LOSS_KINDS and hidden2.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
         corr_metrics, in_flight = {}, None
         wanted = correct and any(loss_fn_args.get(k, None) is not None for k in _SAMPLER_SWITCHES)
+        had_weights = "sampler_is_weights" in b
+
+        def uncorrected():
+            if wanted and "sampler_log_probs" in b:
+                b["response_mask"] = side_mask
+                if not had_weights:
+                    b.pop("sampler_is_weights", None)
+
         if wanted and "sampler_log_probs" in b:
             in_flight = start_sampler_correction(data, loss_fn_args, readback=True)
             if in_flight is None:
                 data, corr_metrics = compute_sampler_correction_and_add_to_batch(data, loss_fn_args)
             b = data.batch
-        spec = blocked_spec(hidden2, weight, packed_ids, cu_seqlens, data, loss_fn, loss_fn_args, temperature,
-                            block_tokens=block_tokens, vocab_chunk=vocab_chunk, dw_group=dw_group,
-                            logit_softcapping=logit_softcapping, side_mask=side_mask, cu_host=cu_host)
-        if spec is None and wanted and "sampler_log_probs" in b:
-            # the unfused path applies the correction itself: hand it the batch as it was
-            b["response_mask"] = side_mask
-            b.pop("sampler_is_weights", None)
+        try:
+            spec = blocked_spec(hidden2, weight, packed_ids, cu_seqlens, data, loss_fn, loss_fn_args, temperature,
+                                block_tokens=block_tokens, vocab_chunk=vocab_chunk, dw_group=dw_group,
+                                logit_softcapping=logit_softcapping, side_mask=side_mask, cu_host=cu_host)
+        finally:
+            if spec is None:  # refused, or the unfused path, which applies the correction itself: the batch as it was
+                uncorrected()
     if spec is None:
         log_prob, entropy = packed_logprobs(hidden2, weight, packed_ids, cu_seqlens, temperature, logit_softcapping)
         data.meta_info["head_backward"] = "recompute"
@@ -354,16 +362,20 @@ def _fused_head_loss(hidden, weight, packed_ids, cu_seqlens, data, meta_info, bl
     if sampler_log_prob is not None:  # the gap between the current policy and the sampler (fsdp_models.py:232-241)
         spec["sampler_gap"] = (sampler_log_prob, side_mask)
     loss, log_prob, entropy, _sums, _side_sums = blocked_head_loss(hidden2, weight, spec)
-    b["log_probs"], b["entropys"] = log_prob, entropy
-    data.meta_info.update(head_backward="blocked-stash", stash_bytes=spec["stash_bytes"],
-                          head_workspace_bytes=spec["workspace_bytes"], n_blocks=spec["n_blocks"],
-                          dw_group=spec["dw_group_used"])
     host, event = spec["readback"]  # the one readback of the step's scalars, started before the last block's backward
     event.synchronize()
     vals = host.tolist()
     sums = host[:8].view(torch.float32).tolist()  # eight of the loss, eight of the side terms
     if spec["seq_mode"] and spec["cu_host"] is None:
-        _check_span(vals[8], vals[9], int(hidden2.shape[0]))
+        try:
+            _check_span(vals[8], vals[9], int(hidden2.shape[0]))
+        except ValueError:
+            uncorrected()
+            raise
+    b["log_probs"], b["entropys"] = log_prob, entropy
+    data.meta_info.update(head_backward="blocked-stash", stash_bytes=spec["stash_bytes"],
+                          head_workspace_bytes=spec["workspace_bytes"], n_blocks=spec["n_blocks"],
+                          dw_group=spec["dw_group_used"])
     if in_flight is not None:
         corr_metrics = in_flight.metrics()
         if corr_metrics is None:  # no token to correct, and the batch is as it was

@@ -559,3 +559,25 @@ def test_kept_logits_give_way_to_what_the_step_cannot_do_without(refused, monkey
     assert got[2].meta_info["stash_bytes"] == (0 if refused == "the logits" else need)
     assert torch.equal(got[0], want[0]) and got[1] == want[1]
     assert torch.equal(got[3], want[3]) and torch.equal(got[4], want[4])
+
+
+@pytest.mark.parametrize("block_tokens", [8192, 64], ids=["one-block", "blocks"])
+def test_refused_offsets_leave_the_batch_as_it_was(block_tokens):
+    """Offsets that do not span the batch: no log-probs or entropies of a step that was refused, no mask or weights of its
+    sampler correction, whether they are checked before the first launch or with the step's readback."""
+    from axon_amd.models.fused_head_loss import fused_head_loss
+    lens = [40, 25, 63]
+    n, h, v = sum(lens), 64, 300
+    hid, w, ids, labels, rl, old, ref = _inputs(n, h, v, lens, seed=4)
+    args = dict(GSPO, sampler_is="token", sampler_is_threshold=2.0, sampler_token_veto_threshold=1e-4)
+    tensors = {"old_log_probs": old.to(DEV), "advantages": torch.ones(n, device=DEV),
+               "response_mask": torch.ones(n, device=DEV), "sampler_log_probs": 1.01 * old.to(DEV)}
+    data = DataProto.from_dict(tensors=dict(tensors))
+    cu = [0, 40, 65, n - 1]
+    with pytest.raises(ValueError, match=f"spans 0..{n - 1}, the batch has {n} tokens"):
+        fused_head_loss(hid.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(True), ids.to(DEV),
+                        torch.tensor(cu, dtype=torch.int32, device=DEV), data,
+                        {"loss_fn": "gspo", "loss_fn_args": args, "temperature": 1.0, "dp_replicas": 1},
+                        block_tokens=block_tokens)
+    assert set(data.batch.keys()) == set(tensors) and all(data.batch[k] is t for k, t in tensors.items())
+    assert "head_backward" not in data.meta_info
