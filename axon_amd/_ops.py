@@ -90,13 +90,11 @@ def _acc8(n_slots, device, acc=None):
     """The eight scalar sums a kernel returns, in ``acc`` where the caller has a place for them; the library writes all of
     them unless there are no tokens.  Under stream capture they start as NaN: a replay whose reduction never finished
     would then show."""
-    if acc is not None:
-        return acc.zero_() if n_slots == 0 else acc
     if n_slots == 0:
-        return _zeros(8, device)
-    if torch.cuda.is_current_stream_capturing():
-        return torch.full((8,), float("nan"), device=device, dtype=torch.float32)
-    return torch.empty(8, device=device, dtype=torch.float32)
+        return _zeros(8, device) if acc is None else acc.zero_()
+    if acc is None:
+        acc = torch.empty(8, device=device, dtype=torch.float32)
+    return acc.fill_(float("nan")) if torch.cuda.is_current_stream_capturing() else acc
 
 
 _PARTIALS: dict = {}

@@ -82,6 +82,20 @@ def test_block_logits_room_and_refusals():
                                                 p, big, p, keep, None, None) == want
 
 
+def test_sums_start_as_zeros_without_tokens_and_as_nan_under_capture(monkeypatch):
+    """Whether the eight sums are the operator's own tensor or a place that the caller has for them (and nothing beside it)."""
+    from axon_amd import _ops
+    cpu = torch.device("cpu")
+    for capturing in (False, True):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        place = torch.full((3, 8), 5.0)
+        assert _ops._acc8(7, cpu, place[1]).data_ptr() == place[1].data_ptr()
+        assert (place[1].isnan() if capturing else place[1] == 5).all()
+        assert (_ops._acc8(0, cpu, place[1]) == 0).all() and (_ops._acc8(0, cpu) == 0).all()
+        assert (place[1] == 0).all() and (place[::2] == 5).all()
+        assert not capturing or _ops._acc8(7, cpu).isnan().all()
+
+
 def test_cpu_tensors_fail_loudly():
     x = torch.zeros(2, 4)
     with pytest.raises(_lib.AxonAmdError, match="no CPU fallback"):
