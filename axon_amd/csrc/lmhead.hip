@@ -322,8 +322,9 @@ __device__ __forceinline__ int aligned_pos(int n, int n_tokens, const uint8_t* i
 
 // Four positions per thread (the array is padded to that): one search for the sequence of the first, a walk from there.
 // In one launch; a fill followed by a store per sequence took two, 4.8 us each.
+typedef uint32_t AnyWord __attribute__((aligned(1)));  // the caller's array begins anywhere
 __global__ __launch_bounds__(256) void seq_start_kernel(const int32_t* __restrict__ cu, int n_seqs,
-                                                        int n_tokens, uint32_t* __restrict__ is_start) {
+                                                        int n_tokens, AnyWord* __restrict__ is_start) {
   const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x, p0 = v * 4;
   if (p0 >= n_tokens) return;
   int lo = 0, hi = n_seqs;  // the number of sequences that begin before p0
@@ -1798,10 +1799,9 @@ extern "C" int axon_seq_start_flags(const int32_t* cu_seqlens, int64_t n_seqs, i
     return AXON_ERR_SHAPE;
   if (n_tokens == 0) return AXON_OK;
   if (!flags || (n_seqs > 0 && !cu_seqlens)) return AXON_ERR_ARG;
-  if (reinterpret_cast<uintptr_t>(flags) & 3) return AXON_ERR_ARG;
   const int64_t words = (n_tokens + 3) / 4;
   hipLaunchKernelGGL(seq_start_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                     cu_seqlens, (int)n_seqs, (int)n_tokens, reinterpret_cast<uint32_t*>(flags));
+                     cu_seqlens, (int)n_seqs, (int)n_tokens, reinterpret_cast<AnyWord*>(flags));
   AXON_CHECK_LAUNCH();
   return AXON_OK;
 }

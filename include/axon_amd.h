@@ -98,7 +98,7 @@ int64_t axon_lmhead_fwd_workspace_bytes(int64_t n_tokens, int64_t hidden, int64_
  * an invalid shape.  The layout is private to the library and depends on the shape only. */
 int64_t axon_lmhead_stash_bytes(int64_t n_tokens, int64_t hidden, int64_t vocab);
 /* flags[p] = 1 where a non-empty sequence of cu_seqlens[n_seqs + 1] begins, else 0.
- * `flags` holds n_tokens bytes rounded up to a multiple of 4, on a 4-byte boundary. */
+ * `flags` holds n_tokens bytes rounded up to a multiple of 4. */
 int axon_seq_start_flags(const int32_t* cu_seqlens, int64_t n_seqs, int64_t n_tokens,
                          uint8_t* flags, void* stream);
 int axon_lmhead_fwd(const void* hidden_bf16, const void* weight_bf16, const void* labels,

@@ -495,6 +495,18 @@ def test_sequence_start_flags_and_paired_scaling(lens):
         assert torch.equal(a, (x.float() * s).bfloat16()) and torch.equal(b, (y.float() * s).bfloat16())
 
 
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [1, 4, 1027])
+def test_sequence_start_flags_at_any_address(n, offset):
+    from axon_amd import _lib, _ops
+    cu = torch.tensor([0, n // 3, n // 2, n], dtype=torch.int32, device=DEV)
+    words = (n + 3) // 4 * 4
+    buf = torch.full((words + 8,), 7, dtype=torch.uint8, device=DEV)
+    rc = _lib.load().axon_seq_start_flags(cu.data_ptr(), 3, n, buf.data_ptr() + offset, _ops.stream_ptr())
+    assert rc == 0 and torch.equal(buf[offset:offset + words], _ops.seq_start_flags(cu, n))
+    assert (buf[:offset] == 7).all() and (buf[offset + words:] == 7).all()
+
+
 @pytest.mark.parametrize("n,block_tokens,blocks", [(257, 256, 2), (1025, 512, 3)])
 @pytest.mark.parametrize("case", ["ppo", "dapo-entropy-kl"])
 def test_a_block_that_owns_no_position_adds_nothing(case, n, block_tokens, blocks, monkeypatch):
