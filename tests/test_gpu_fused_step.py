@@ -507,6 +507,33 @@ def test_sequence_start_flags_at_any_address(n, offset):
     assert (buf[:offset] == 7).all() and (buf[offset + words:] == 7).all()
 
 
+@pytest.mark.parametrize("n,at", [(1027, 1027), (1027, 513), (1026, 1), (5, 3)])
+def test_sequence_start_flags_of_offsets_padded_with_empty_sequences(n, at):
+    """20000 empty sequences at one place: the right flags, and no thread that goes through them one by one (which took
+    five hundred times as long as the call without them)."""
+    from axon_amd import _ops
+    real = torch.arange(0, n + 1, max(n // 40, 1))
+    real[-1] = n
+    padded = torch.sort(torch.cat([real, torch.full((20000,), at)]))[0]
+    want = torch.zeros((n + 3) // 4 * 4, dtype=torch.uint8)
+    want[padded[:-1][padded[1:] > padded[:-1]]] = 1
+
+    def timed(cu):
+        cu, best = cu.int().to(DEV), float("inf")
+        for _ in range(10):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                flags = _ops.seq_start_flags(cu, n)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return flags, best
+
+    (flags, t), (_, t0) = timed(padded), timed(real)
+    assert torch.equal(flags.cpu(), want) and t < 20 * t0
+
+
 @pytest.mark.parametrize("n,block_tokens,blocks", [(257, 256, 2), (1025, 512, 3)])
 @pytest.mark.parametrize("case", ["ppo", "dapo-entropy-kl"])
 def test_a_block_that_owns_no_position_adds_nothing(case, n, block_tokens, blocks, monkeypatch):
