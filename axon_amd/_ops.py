@@ -1046,7 +1046,7 @@ class HeadBlocks:
             self._at(self.seq_start, n0), last_dst, self._at(self.out[0], n0), self._at(self.out[1], n0),
             ptr(self.stats[0]), ptr(self.stats[1]), ptr(self.fwd_ws), self.fwd_ws_bytes,
             ptr(self.stash) if kept else None, kept, stream_ptr(), self.timing.handle if self.timing else None),
-            "axon_lmhead_block_fwd")
+            fwd.__name__)
 
     def backward(self, k, dlogprobs, dentropy):
         """Backward of block ``k`` (after its ``forward``; no other block's forward in between).  ``dlogprobs`` /
@@ -1073,7 +1073,7 @@ class HeadBlocks:
             ptr(self.d_weight), ptr(self.dw_acc), mode, 1, pos, int(dw_now), self.ws_tokens, self.chunk,
             ptr(self.bwd_ws), self.bwd_ws_bytes,
             ptr(self.stash) if kept else None, kept, st, th),
-            "axon_lmhead_block_bwd")
+            bwd.__name__)
 
 
 def scale_f32(x, s1, s2=None):
@@ -1159,7 +1159,7 @@ def logits_forward(logits, labels=None, want_entropy=True, backward_follows=Fals
         fwd(ptr(logits), _LOGITS_DTYPES[logits.dtype], ld, n, v, ptr(labels),
             int(labels is not None and labels.dtype == torch.int64), base if labels is not None else None,
             base + 4 * n if want_entropy else None, base + 8 * n, ptr(ws), stream_ptr()),
-        "axon_logits_fwd_ws",
+        fwd.__name__,
     )
     lp, ent, lse = out.unbind(0)
     return (lp if labels is not None else None), (ent if want_entropy else None), lse

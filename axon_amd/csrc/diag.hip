@@ -168,9 +168,9 @@ constexpr int kOutSums = 50;  // out[0..49]: sums (0..22 token-level, 23..49 row
 constexpr int kOutMM = 10;    // out[50..59]: maxima, out[60..69]: minima
 constexpr int kDiagOut = 72;
 
-// Four wavefronts per workgroup: what a wavefront spends here is mostly the 50 + 20 reductions at the end,
-// which cost the same for one row per lane as for four, and sixteen wavefronts would queue four deep on a SIMD.
-// Those reductions by DPP moves instead of LDS shuffles: 65536 tokens in 90 rows 9.6 us for 17.3, 8.4 M in 9000 15.3 for 21.9.
+// Four wavefronts per workgroup: what a wavefront spends here is mostly the 50 + 20 reductions at the end, which cost
+// the same for one row per lane as for four, and sixteen wavefronts would queue four deep on a SIMD. Those reductions
+// by DPP moves instead of LDS shuffles: 65536 tokens in 90 rows 9.6 us for 17.3, 8.4 M in 9000 15.3 for 21.9.
 constexpr int kDiagRowThreads = 256;
 // Workgroup b of the grid takes token partials b, b + gridDim.x, ... and rows likewise, and leaves its
 // 70 sums / maxima / minima in out[b][kDiagOut]; sampler_diag_final_kernel folds the workgroups where there are

@@ -220,10 +220,10 @@ struct DmaSide {
 };
 
 // kNarrow: the K-major A operand's rows are shorter than 512 bytes (see dma_kb).
-// BM: block rows per wave.  8 is the whole 256 x 256 tile; 4 computes its first 128 rows (64 per wave, half the matrix
-// instructions per k-tile) with the same slots and the same DMA instructions, of which those for the other rows
-// fetch nothing on a K-contiguous side (the descriptor ends): for the last tile of an m that fills at most half of it, and for
-// the tail of a walk whose tiles are halved to spread them over the compute units.
+// BM: block rows per wave.  8 is the whole 256 x 256 tile; 4 computes its first 128 rows (64 per wave, half the
+// matrix instructions per k-tile) with the same slots and the same DMA instructions, of which those for the other
+// rows fetch nothing on a K-contiguous side (the descriptor ends): for the last tile of an m that fills at most half
+// of it, and for the tail of a walk whose tiles are halved to spread them over the compute units.
 template <bool kAT, bool kBT, bool kNarrow = false, int BM = kBlocks>
 struct DmaLoopT {
   static_assert(BM == kBlocks || BM == kBlocks / 2, "");

@@ -117,13 +117,13 @@ __device__ __forceinline__ float rows_all_reduce(float v, Op op) {
   return op(c, d);
 }
 
-// Fold a logits tile of 32 * BM vocabulary rows x 256 tokens into per-token partials, one per 128 rows.  BM 8: a whole
-// tile, whose wavefronts have a part each; BM 4: the half `half` of one, whose part the wavefronts 0 and 2 (1 and 3) share:
-// its maximum and its sums go through LDS, in the order in which one wavefront of a whole tile adds them up (a lane
-// adds the first four and the last four 16-row blocks apart), so that the results do not depend on how a tile was computed.
-// MASKED: some rows of the tile lie beyond the vocabulary; they are excluded by predicate — their accumulators hold finite
-// values.  STASH: also store every 2^(y - M) for the backward (`stash_wave`: the 32 KB of the part and these
-// tokens, already offset by the lane).
+// Fold a logits tile of 32 * BM vocabulary rows x 256 tokens into per-token partials, one per 128 rows.  BM 8: a
+// whole tile, whose wavefronts have a part each; BM 4: the half `half` of one, whose part the wavefronts 0 and 2 (1
+// and 3) share: its maximum and its sums go through LDS, in the order in which one wavefront of a whole tile adds
+// them up (a lane adds the first four and the last four 16-row blocks apart), so that the results do not depend on
+// how a tile was computed. MASKED: some rows of the tile lie beyond the vocabulary; they are excluded by predicate —
+// their accumulators hold finite values.  STASH: also store every 2^(y - M) for the backward (`stash_wave`: the 32 KB
+// of the part and these tokens, already offset by the lane).
 template <bool MASKED, bool STASH, int BM>
 __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams& p, const LanePos& lp,
                                              const TilePos& t, int part, uint4* stash_wave, float* lds) {
@@ -322,8 +322,9 @@ __device__ __forceinline__ int aligned_pos(int n, int n_tokens, const uint8_t* i
 
 typedef uint32_t AnyWord __attribute__((aligned(1)));  // the caller's array of flags begins anywhere
 // Four positions per thread (the array is padded to that): one search for the sequence of the first, and from there a
-// gallop per position, so that offsets padded with empty sequences to a fixed number cost a thread a few steps more (one
-// sequence after the other 20000 of them took 2245 us for 5.1).  In one launch; a fill followed by a store per sequence took two, 4.8 us each.
+// gallop per position, so that offsets padded with empty sequences to a fixed number cost a thread a few steps more
+// (one sequence after the other 20000 of them took 2245 us for 5.1).  In one launch; a fill followed by a store per
+// sequence took two, 4.8 us each.
 __global__ __launch_bounds__(256) void seq_start_kernel(const int32_t* __restrict__ cu, int n_seqs,
                                                         int n_tokens, AnyWord* __restrict__ is_start) {
   const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x, p0 = v * 4;
@@ -355,16 +356,17 @@ __global__ __launch_bounds__(256) void seq_start_kernel(const int32_t* __restric
   is_start[v] = bits;
 }
 
-// The last kernel of the forward: folds a token's partials into lse, entropy_b and entropy, forms the label's
-// logit and with it logprob[n] = softcap(hidden[n] . W[label[n]]) / T - lse[n].
-// A token's partials are folded in 256 groups, group c taking c, c + 256, ... (a chain of five for 151936 vocabulary rows); sixteen
-// neighbouring groups are folded as a tree, the sixteen results one after the other.  That order is the same whatever T and
-// PER, hence whatever the number of tokens.  A workgroup of 1024 threads owns T * PER consecutive tokens, a thread 256 * T / 1024
-// groups of PER tokens (T apart) with eight partials requested before the first is folded: T = 4 up to 1024 tokens, to put a
-// short call on as many compute units as there are; T = 16 beyond, PER = 2 once a workgroup per 16 tokens would be
-// more than one per CU.  The label dots (one wavefront per token) run before the barrier, beside the folds of the other wavefronts.
-// 187 tokens x 896 x 151936 5.9 us (11.0 with three arrays of partials, 64 groups and 16 tokens per workgroup), 700 x 4096 11.9
-// (19.0), 1500 x 896 9.8 (12.8), 3001 x 2880 x 201088 22.5 (31.4), 8192 x 4096 41.4 (49.0).
+// The last kernel of the forward: folds a token's partials into lse, entropy_b and entropy, forms the label's logit
+// and with it logprob[n] = softcap(hidden[n] . W[label[n]]) / T - lse[n].
+// A token's partials are folded in 256 groups, group c taking c, c + 256, ... (a chain of five for 151936 vocabulary
+// rows); sixteen neighbouring groups are folded as a tree, the sixteen results one after the other.  That order is
+// the same whatever T and PER, hence whatever the number of tokens.  A workgroup of 1024 threads owns T * PER
+// consecutive tokens, a thread 256 * T / 1024 groups of PER tokens (T apart) with eight partials requested before the
+// first is folded: T = 4 up to 1024 tokens, to put a short call on as many compute units as there are; T = 16 beyond,
+// PER = 2 once a workgroup per 16 tokens would be more than one per CU.  The label dots (one wavefront per token) run
+// before the barrier, beside the folds of the other wavefronts. 187 tokens x 896 x 151936 5.9 us (11.0 with three
+// arrays of partials, 64 groups and 16 tokens per workgroup), 700 x 4096 11.9 (19.0), 1500 x 896 9.8 (12.8), 3001 x
+// 2880 x 201088 22.5 (31.4), 8192 x 4096 41.4 (49.0).
 template <int T, int PER, typename LabelT>
 __global__ __launch_bounds__(1024) void lmhead_finish_kernel(
     const float* __restrict__ stats, int parts, const __bf16* __restrict__ hidden, const __bf16* __restrict__ weight,
@@ -489,8 +491,9 @@ struct DlogitParams {
   __bf16* dlT;   // [chunk_cols][n_pad]   vocab-major; null: not wanted (the dWeight GEMM reads dl as a K-major operand)
   int64_t ld_dl, ld_dlT;
   int n_tokens, vocab, v_begin;  // v_begin: first vocab row of this chunk
-  // Rows of dl from here on (a multiple of 64, at least n_tokens) are read by nobody and need not be written: sixty-four or
-  // a hundred and twenty-eight of them are left out together.  The zeros between n_tokens and n_end are k of the weight gradient.
+  // Rows of dl from here on (a multiple of 64, at least n_tokens) are read by nobody and need not be written:
+  // sixty-four or a hundred and twenty-eight of them are left out together.  The zeros between n_tokens and n_end are
+  // k of the weight gradient.
   int n_end;
   float inv_temp;
   float cap, inv_cap;  // soft-capping (SOFTCAP kernels only)
@@ -615,14 +618,14 @@ __device__ __forceinline__ void dlogit_store(AccTile& acc, const DlogitParams& p
   }
 }
 
-// The same from a forward's stash (see StashLayout above FwdParams): softmax = w * 2^(M - lse), scaled
-// logit = log2(w) + M.  One call covers 64 tokens (four 16-token blocks, j0 .. j0 + 3) x 128 vocabulary
-// rows of a wavefront's sub-tile; staged row = token - 16 * j0.  SOFTCAP: the stash describes the capped
-// logit, whose derivative factor is 1 - (capped / cap)^2.  EDGE: entries beyond the last token or the last
-// vocabulary row are staged as zeros.
+// The same from a forward's stash (see StashLayout above FwdParams): softmax = w * 2^(M - lse), scaled logit =
+// log2(w) + M.  One call covers 64 tokens (four 16-token blocks, j0 .. j0 + 3) x 128 vocabulary rows of a wavefront's
+// sub-tile; staged row = token - 16 * j0.  SOFTCAP: the stash describes the capped logit, whose derivative factor is
+// 1 - (capped / cap)^2.  EDGE: entries beyond the last token or the last vocabulary row are staged as zeros.
 // ENT: the entropies have a gradient.  Without one (and without soft-capping) the logit itself is not needed, and the
-// logarithm that recovers it is half of the vector work: 333 tokens x 1024 x 50257 36.8 us for 42.7, 300 x 896 x 151936 58.7
-// for 66.9 (rows beyond n_end left out as well), 700 x 4096 83 for 94; from some thousand tokens on memory bounds both.
+// logarithm that recovers it is half of the vector work: 333 tokens x 1024 x 50257 36.8 us for 42.7, 300 x 896 x
+// 151936 58.7 for 66.9 (rows beyond n_end left out as well), 700 x 4096 83 for 94; from some thousand tokens on
+// memory bounds both.
 constexpr int kStashHalfBlocks = kBlocks / 2;
 template <bool SOFTCAP, bool ENT, bool EDGE>
 __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashHalfBlocks], int j0,
@@ -699,10 +702,10 @@ __device__ __forceinline__ void dlogit_stage_logits(const float4 (&x)[kStashHalf
   }
 }
 
-// A staged 64 x 128 half sub-tile (tokens 16 * j0 .. of the wavefront's sub-tile) -> dl and dlT.  Token-major
-// 32 lanes cover one 256-byte row, eight rows per trip (reads before writes); vocab-major: sixteen lanes cover the 64 tokens of one vocabulary row (one
-// 128-byte line), the four lane groups take units u, u + 8, u + 16, u + 24, whose permuted slots differ in
-// a bit that the rows' swizzles (a set with that bit fixed) cannot cancel.
+// A staged 64 x 128 half sub-tile (tokens 16 * j0 .. of the wavefront's sub-tile) -> dl and dlT.  Token-major 32
+// lanes cover one 256-byte row, eight rows per trip (reads before writes); vocab-major: sixteen lanes cover the 64
+// tokens of one vocabulary row (one 128-byte line), the four lane groups take units u, u + 8, u + 16, u + 24, whose
+// permuted slots differ in a bit that the rows' swizzles (a set with that bit fixed) cannot cancel.
 __device__ __forceinline__ void dlogit_copy_out_half(const char* stage, int j0, const DlogitParams& p,
                                                      const LanePos& lp, const TilePos& t) {
   const int l32 = lp.lane & 31, lhi = lp.lane >> 5;
@@ -806,11 +809,11 @@ __global__ __launch_bounds__(kGemmThreads) void lmhead_dlogit_softcap_kernel(Gem
   dlogit_body<Loop, true>(g, p, tiles_m, tiles_n);
 }
 
-// Backward B1 without the recompute: one wavefront per workgroup turns half (64 tokens x 128 rows) of a
-// sub-tile that a stashing forward stored into bf16 dlogits in both orientations (16 KB of LDS and few
-// registers: ten wavefronts per CU hide the latency of the loads and of the per-token operands).  A streaming kernel: 2 bytes
-// read and 4 written per logit.  Tiles are the forward's: `tm0` is the forward tile row of the chunk's
-// first vocabulary row, and t.m0 is made chunk-relative after the edge tests.
+// Backward B1 without the recompute: one wavefront per workgroup turns half (64 tokens x 128 rows) of a sub-tile that
+// a stashing forward stored into bf16 dlogits in both orientations (16 KB of LDS and few registers: ten wavefronts
+// per CU hide the latency of the loads and of the per-token operands).  A streaming kernel: 2 bytes read and 4
+// written per logit.  Tiles are the forward's: `tm0` is the forward tile row of the chunk's first vocabulary row, and
+// t.m0 is made chunk-relative after the edge tests.
 struct StashSource {
   const uint4* stash;
   const float* pm;
@@ -890,9 +893,9 @@ struct StoreParams {
   int accumulate = 0;  // add the previous contents of tile_acc first
   int keep_f32 = 0;    // write the sum back to tile_acc (0: it is only read, the sum leaves as bf16)
   // fp32 partial sums (the weight gradient carried from one token block to the next, dHidden carried from one
-  // vocabulary chunk to the next or formed in parts): kept per tile in the order the accumulators lie in the registers, so that every
-  // wavefront load and store is one contiguous kilobyte.  float4 index =
-  // ((tile * 4 + wave) * 64 + i * 8 + j) * 64 + lane, tile = tm * tiles_n + tn.  Null: not used.
+  // vocabulary chunk to the next or formed in parts): kept per tile in the order the accumulators lie in the
+  // registers, so that every wavefront load and store is one contiguous kilobyte.  float4 index = ((tile * 4 + wave)
+  // * 64 + i * 8 + j) * 64 + lane, tile = tm * tiles_n + tn.  Null: not used.
   float4* tile_acc = nullptr;
   // Split reduction: `splits` workgroups per tile, each over `k_split` (a multiple of 64) of the k; they leave their
   // partial sums in tile_acc, one array of tiles after the other, for split_sum_kernel.
@@ -1344,12 +1347,12 @@ SplitPlan split_plan(int64_t tiles, int64_t k) {
 }
 
 // Whether the half-filled last tiles of an output product are computed as half tiles.  What that saves falls with the
-// number of tiles beside them; what it costs grows with the reduction: a half tile runs ahead of the whole ones, with which
-// it no longer shares operand slices in the L2 (dWeight more than dHidden, whose parts keep an XCD on one part of k).
-// Whole / half, ms: dWeight hidden 896 (4 tiles) 3001 tokens (47 k-tiles) 0.671 / 0.611, 8192 1.67 / 1.58, 12288 2.53 / 2.45,
-// 16381 3.42 / 3.47; hidden 2880 (12 tiles) 700 tokens 0.847 / 0.789, 3001 2.60 / 2.57, 6007 4.92 / 4.96, 16381
-// 13.1 / 13.9.  dHidden 896 6007 tokens (297 k-tiles) 1.28 / 1.20, 16381 (792) 3.26 / 3.13; 2880 3001 tokens (629) 2.66 / 2.64,
-// 6007 (1571) 6.21 / 6.22, 8192 (1571) 6.72 / 6.76, 16381 (3142) 13.3 / 13.5.
+// number of tiles beside them; what it costs grows with the reduction: a half tile runs ahead of the whole ones, with
+// which it no longer shares operand slices in the L2 (dWeight more than dHidden, whose parts keep an XCD on one part
+// of k). Whole / half, ms: dWeight hidden 896 (4 tiles) 3001 tokens (47 k-tiles) 0.671 / 0.611, 8192 1.67 / 1.58,
+// 12288 2.53 / 2.45, 16381 3.42 / 3.47; hidden 2880 (12 tiles) 700 tokens 0.847 / 0.789, 3001 2.60 / 2.57, 6007 4.92
+// / 4.96, 16381 13.1 / 13.9.  dHidden 896 6007 tokens (297 k-tiles) 1.28 / 1.20, 16381 (2374) 3.26 / 3.13; 2880 3001
+// tokens (629) 2.66 / 2.64, 6007 (1571) 6.21 / 6.22, 8192 (1571) 6.72 / 6.76, 16381 (3142) 13.3 / 13.5.
 constexpr int64_t kHalfEdgeDw = 768, kHalfEdgeDh = 12288;  // most k-tiles times tiles
 bool half_edge(int64_t k, int64_t h, int64_t most) {
   return (h - 1) % kTile < kTile / 2 && (k + 63) / 64 * (round_up(h, kTile) / kTile) <= most;
@@ -1542,11 +1545,12 @@ int launch_transpose(const void* in, int64_t ld_in, int rows, int cols, void* ou
 }
 
 // The forward's tiles that are computed in halves of 128 vocabulary rows: those of a last round that would occupy at
-// most half of the compute units, so that it takes half as long.  594 tiles, 2.3 rounds: 187 tokens x 896 x 151936 87 us
-// for 80, 187 x 4096 305 for 288; 128 tiles (250 x 2048 x 32768) 44 for 35.  A last round over more than half of
-// them would become two.  Not behind many whole rounds, which then no longer split evenly over the XCDs' ranges of the
-// walk and read more from beyond the L2 (8192 x 4096 x 151936 18 to 21 GB for 15).  Whole / half, ms, at hidden 4096 x 151936:
-// 9.3 rounds 0.942 / 0.907, 16.2 1.574 / 1.545, 32.5 3.068 / 3.034, 37.1 3.581 / 3.609, 74.3 6.99 / 7.13.
+// most half of the compute units, so that it takes half as long.  594 tiles, 2.3 rounds: 187 tokens x 896 x 151936 87
+// us for 80, 187 x 4096 305 for 288; 128 tiles (250 x 2048 x 32768) 44 for 35.  A last round over more than half of
+// them would become two.  Not behind many whole rounds, which then no longer split evenly over the XCDs' ranges of
+// the walk and read more from beyond the L2 (8192 x 4096 x 151936 18 to 21 GB for 15).  Whole / half, ms, at hidden
+// 4096 x 151936: 9.3 rounds 0.942 / 0.907, 16.2 1.574 / 1.545, 32.5 3.068 / 3.034, 37.1 3.581 / 3.609, 74.3 6.99 /
+// 7.13.
 constexpr int64_t kHalvedRounds = 36;
 int halved_tiles(int64_t n, int64_t v) {
   const int64_t tiles = (round_up(v, kTile) / kTile) * (round_up(n, kTile) / kTile), rest = tiles % kCus;

@@ -102,8 +102,9 @@ __device__ __forceinline__ Stats merge(Stats a, Stats b) {
 constexpr float kFloor = -1e30f;  // below any logit; finite, so that differences stay finite
 
 // What one workgroup does of a row: the 16-byte vectors [q_lo, q_hi) of the row's aligned middle, counted from
-// element `head` on, and its share of the n_scalar elements outside it (before `head`, then behind the last vector).  An odd vocabulary puts every row on another boundary, so a row's first vector starts at its first
-// 16-byte boundary and not at its first element.
+// element `head` on, and its share of the n_scalar elements outside it (before `head`, then behind the last vector).
+// An odd vocabulary puts every row on another boundary, so a row's first vector starts at its first 16-byte boundary
+// and not at its first element.
 struct RowSpan {
   int head, n_vec, n_scalar, q_lo, q_hi;
   template <typename T>
@@ -218,12 +219,13 @@ __global__ __launch_bounds__(kWave) void logits_merge_kernel(
 }
 
 // dlogits[j] = g_lp (onehot_j - p_j) - g_ent p_j (log p_j + H),  p_j = exp(z_j - lse).
-// dlogits may be the logits' own storage: every element is read before it is written by the same thread.
-// Rows, and the vectors of a row, are walked from the last to the first: the end of what the forward read last is
-// still in the 256 MB cache in front of the memory (its cached_from), and the loads and stores here, which pass that
-// cache by, leave it there until it is read.  Bound by memory: 2047 x 151936 bf16 208 us for 247 with a forward that
-// leaves nothing, 4096 x 50257 151 for 186, 1600 x 151936 fp32 355 for 404; where a short batch is split into parts 32 x 151936 takes 9.3 us for 53, 187 x 151936 24 for 78;
-// rows of an odd vocabulary, read from their first 16-byte boundary on, 2047 x 50257 bf16 93 us for 166.
+// dlogits may be the logits' own storage: every element is read before it is written by the same thread.  Rows, and
+// the vectors of a row, are walked from the last to the first: the end of what the forward read last is still in the 256 MB cache in front of the
+// memory (its cached_from), and the loads and stores here, which pass that cache by, leave it there until it is
+// read.  Bound by memory: 2047 x 151936 bf16 208 us for 247 with a forward that leaves nothing, 4096 x 50257 151 for
+// 186, 1600 x 151936 fp32 355 for 404; where a short batch is split into parts 32 x 151936 takes 9.3 us for 53, 187 x
+// 151936 24 for 78; rows of an odd vocabulary, read from their first 16-byte boundary on, 2047 x 50257 bf16 93 us for
+// 166.
 template <typename T, typename LabelT>
 __global__ __launch_bounds__(kBlock) void logits_grad_kernel(
     const T* logits, int64_t ld, int vocab, const LabelT* __restrict__ labels,

@@ -487,8 +487,8 @@ struct OwnedCorrOp {
   float ov[2][kRowHold][4], sv[2][kRowHold][4], mv[2][kRowHold][4];
   float a[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float vetoed_rows = 0.f;
-  // token-level diagnostics: a group's slots in fp32, the groups in double, so that no fp32 sum of a thread is longer than
-  // eight slots however many rows it walks
+  // token-level diagnostics: a group's slots in fp32, the groups in double, so that no fp32 sum of a thread is longer
+  // than eight slots however many rows it walks
   static constexpr int kTok = 9;  // e; e > is_hi, e < is_lo, clamped e, its square; the same by the rejection's bounds
   float t[TOK ? kTok : 1] = {};
   double td[TOK ? kTok : 1] = {};
@@ -574,11 +574,11 @@ struct OwnedCorrOp {
   }
 };
 
-// With `diag_partials` the launch takes the place of sampler_diag_tokens_kernel as well, which read the same three arrays
-// again, found every token's row and added the row sums up with atomics.  8.4 M tokens: 62 us for 59 + 43 and a fill of
-// the row sums where the diagnostics are the rows' only; 65536 tokens with token-level weights, rejection and veto 17.8 for
-// 13.4 + 8.6 and the fill.  Bound by the latency of a step of the walk (2.8 TB/s).  TOK at three workgroups per CU: 140
-// registers, four would spill.
+// With `diag_partials` the launch takes the place of sampler_diag_tokens_kernel as well, which read the same three
+// arrays again, found every token's row and added the row sums up with atomics.  8.4 M tokens: 62 us for 59 + 43 and
+// a fill of the row sums where the diagnostics are the rows' only; 65536 tokens with token-level weights, rejection
+// and veto 17.8 for 13.4 + 8.6 and the fill.  Bound by the latency of a step of the walk (2.8 TB/s).  TOK at three
+// workgroups per CU: 140 registers, four would spill.
 template <int MK, bool TOK>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(TOK ? 3 : 4))) void owned_correction_kernel(
     OwnedCorrArgs g, RowStarts rs, int stride, float* ws, float* __restrict__ acc) {
