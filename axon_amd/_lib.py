@@ -53,6 +53,7 @@ SIGNATURES: dict[str, tuple] = {
     "axon_lmhead_bwd_dlogit_copies_of": (_i32, [_i64, _i64, _i64, _i64]),
     "axon_lmhead_bwd_dhidden_parts": (_i64, [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
     "axon_lmhead_bwd_half_tiles": (_i32, [_i64, _i64, _i64, _i64, _i64]),
+    "axon_lmhead_bwd_dweight_by_rows": (_i32, [_i64, _i64, _i64, _i64, _i64]),
     "axon_scale_bf16_unless_one": (_i32, [_ptr, _i64, _ptr, _ptr]),
     "axon_scale_bf16_pair_unless_one": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr]),
     "axon_step_grads": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _f32, _f32, _i64, _ptr, _ptr, _ptr]),
@@ -119,7 +120,7 @@ SIGNATURES: dict[str, tuple] = {
                                         _ptr, _ptr, _f32, _i32, _ptr, _f32, _f32, _f32, _ptr, _ptr, _ptr]),
 }
 
-ABI_VERSION = 22
+ABI_VERSION = 23
 MASK_F32, MASK_I64 = 0, 1
 
 _lock = threading.Lock()

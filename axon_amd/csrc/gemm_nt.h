@@ -105,12 +105,35 @@ __device__ __forceinline__ void zero_acc(AccTileOf<BM>& acc) {
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 }
 
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  // round-to-nearest-even in one instruction (v_cvt_pk_bf16_f32)
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const f32x2 v = {lo, hi};
+  const bf16x2 r = __builtin_convertvector(v, bf16x2);
+  return *reinterpret_cast<const uint32_t*>(&r);
+}
+
 // c += a * b on one 16x16 block, accumulator held in place in the AGPR file.  Written as an
 // instruction because the register allocator otherwise rotates the 64 four-register accumulators
 // through the VGPR file on every trip of the unrolled loop (hundreds of copies per k-tile).
 __device__ __forceinline__ void mfma_16x16x32(acc4& c, const bf16x8& a, const bf16x8& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
+
+// c = a * b, in the place of an accumulator that is no longer needed
+__device__ __forceinline__ void mfma_16x16x32_from_zero(acc4& c, const bf16x8& a, const bf16x8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+// The same with `a` in the accumulators' half of the register file.
+__device__ __forceinline__ void mfma_16x16x32_agpr(acc4& c, const bf16x8& a, const bf16x8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "a"(a), "v"(b));
+}
+
+// An accumulator is copied out for an epilogue behind this point; else the compiler copies all of them out at its head, and
+// spills them where the registers are few.
+__device__ __forceinline__ void pin_acc(acc4& c) { asm volatile("" : "+a"(c)); }
 
 // The compiler does not see the matrix instructions above, so it cannot count the wait states
 // between the last of them and the first read of an accumulator: spend them here.

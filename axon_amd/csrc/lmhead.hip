@@ -14,6 +14,7 @@
 // vocabularies that are no multiple of 8 get a second, vocab-major copy
 // dlT[vocab][token] from B1 for B3.
 #include "common.h"
+#include "dweight_rows.h"
 #include "gemm_nt.h"
 #include <vector>
 
@@ -23,15 +24,6 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-  // round-to-nearest-even in one instruction (v_cvt_pk_bf16_f32)
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  const f32x2 v = {lo, hi};
-  const bf16x2 r = __builtin_convertvector(v, bf16x2);
-  return *reinterpret_cast<const uint32_t*>(&r);
-}
 
 // ----------------------------------------------------------------------------
 // Forward: tile epilogue -> partial statistics
@@ -1433,6 +1425,13 @@ HalfEdges half_edges(const BwdWs& w, const SplitPlan& dh, int64_t h, int64_t k_d
                    w.dl_kmajor && !carried && half_edge(k_dw, h, kHalfEdgeDw)};
 }
 
+// Whether dWeight over k_dw tokens (padded to whole k-tiles) and vc vocabulary rows is formed from rows of hT held in
+// registers (dweight_rows.h): no partial sums carried, dlogits read as they lie, offsets in 32 bits, a long enough walk.
+bool dw_by_rows(const BwdWs& w, int64_t h, int64_t vc, int64_t k_dw, bool carried) {
+  return !carried && w.dl_kmajor && k_dw <= kDwRowsMaxK && h <= kDwRowsMaxHidden &&
+         h * w.ld_n * 2 < (int64_t(1) << 31) && dw_rows_worth(h, vc, k_dw);
+}
+
 // Bytes for a call over `n` tokens.  The default chunk shrinks in steps while n grows, so a shorter call can need a
 // little more: the most of any call over at most n tokens (beyond 32768 the chunk stays the same).
 int64_t bwd_ws_bytes(int64_t n, int64_t h, int64_t vocab, int64_t chunk) {
@@ -1803,7 +1802,8 @@ int bwd_impl(const float* dlogprobs, const float* dentropy, const void* hidden, 
       sp.keep_f32 = blk.dw_mode != kDwLast;
       sp.splits = 1; sp.k_split = g.k;
       sp.half_edge = half.dw;
-      rc = launch_store_kmajor(g, sp, false, w.dl_kmajor, st);
+      rc = dw_by_rows(w, h, vc, g.k, blk.dw_mode != kDwStore) ? launch_dw_rows(g, sp.out_bf16, sp.ld_bf16, st)
+                                                              : launch_store_kmajor(g, sp, false, w.dl_kmajor, st);
       if (rc != AXON_OK) return rc;
     }
   }
@@ -2068,7 +2068,16 @@ extern "C" int axon_lmhead_bwd_half_tiles(int64_t n, int64_t ws_tokens, int64_t 
   if (n == 0 || chunk < 0 || chunk % kTile != 0 || n > ws_tokens) return AXON_ERR_ARG;
   const BwdWs w = bwd_ws(ws_tokens, h, v, chunk, nullptr);
   const HalfEdges half = half_edges(w, dh_plan(w, n, h, v).split, h, round_up(n, 64), false);
-  return (half.dh ? 1 : 0) + (half.dw ? 2 : 0);
+  return (half.dh ? 1 : 0) + (half.dw && !dw_by_rows(w, h, v < w.chunk ? v : w.chunk, round_up(n, 64), false) ? 2 : 0);
+}
+
+extern "C" int axon_lmhead_bwd_dweight_by_rows(int64_t n, int64_t ws_tokens, int64_t h, int64_t v, int64_t chunk) {
+  int rc = check_head_shape(n, h, v);
+  if (rc == AXON_OK) rc = check_head_shape(ws_tokens, h, v);
+  if (rc != AXON_OK) return rc;
+  if (n == 0 || chunk < 0 || chunk % kTile != 0 || n > ws_tokens) return AXON_ERR_ARG;
+  const BwdWs w = bwd_ws(ws_tokens, h, v, chunk, nullptr);
+  return dw_by_rows(w, h, v < w.chunk ? v : w.chunk, round_up(n, 64), false) ? 1 : 0;
 }
 
 extern "C" int axon_lmhead_block_can_group(int64_t h, int64_t v, int64_t chunk) {

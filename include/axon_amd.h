@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define AXON_AMD_ABI_VERSION 22
+#define AXON_AMD_ABI_VERSION 23
 
 enum {
   AXON_OK = 0,
@@ -279,6 +279,10 @@ int64_t axon_lmhead_bwd_dhidden_parts(int64_t n_tokens, int64_t ws_tokens, int64
 /* Which of the two output products of such a call over n_tokens > 0 computes a last tile of 256 hidden columns that is at
  * most half filled as half a tile: 1 = dHidden, 2 = dWeight (where no sums are carried from another block), 3 = both. */
 int axon_lmhead_bwd_half_tiles(int64_t n_tokens, int64_t ws_tokens, int64_t hidden, int64_t vocab, int64_t vocab_chunk);
+/* Whether such a call (no sums carried from another block) forms dWeight of its whole vocabulary chunks from hidden rows
+ * that stay in registers instead of in 256 x 256 tiles: up to 768 tokens over a long vocabulary.  The same bits. */
+int axon_lmhead_bwd_dweight_by_rows(int64_t n_tokens, int64_t ws_tokens, int64_t hidden, int64_t vocab,
+                                    int64_t vocab_chunk);
 int axon_scale_bf16_unless_one(void* x_bf16, int64_t n, const float* scale, void* stream);
 /* The same for two arrays in one launch (either may be empty). */
 int axon_scale_bf16_pair_unless_one(void* x_bf16, int64_t nx, void* y_bf16, int64_t ny, const float* scale, void* stream);

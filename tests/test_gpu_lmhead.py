@@ -1124,6 +1124,24 @@ def test_half_tiles_of_the_output_products_give_the_bits_of_whole_ones(n, v, chu
         assert torch.equal(a, b[:, :h]) and a.float().norm() > 0
 
 
+@pytest.mark.parametrize("n,h", [(1, 896), (64, 1056), (65, 288), (128, 896), (150, 1056), (256, 320), (300, 896),
+                                 (384, 576), (400, 1056), (512, 896), (513, 576), (640, 1056), (641, 1248), (704, 992),
+                                 (768, 1216)])
+def test_dweight_from_resident_rows_gives_the_bits_of_tiles(n, h):
+    """Every number of k-tiles of the kernel for few tokens, with row tiles of 32 and 64 that end inside the matrix, wavefronts
+    without rows (896 = 14 x 64 on two groups of eight, 1056 = 33 x 32 on five) and a last tile of 8 columns, against the same call
+    in vocabulary chunks too short for it: the same dlogits, products and order of additions, equal bit for bit."""
+    v = 131080
+    ask = lambda chunk: _lib.load().axon_lmhead_bwd_dweight_by_rows(n, n, h, v, chunk)  # noqa: E731
+    assert ask(0) == 1 and ask(4096) == 0
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(n, h, v, seed=n + h))
+    w = (w.float() * 8).bfloat16()
+    g_lp, g_en = torch.randn(2, n, generator=torch.Generator().manual_seed(n)).to(DEV)
+    _, _, lse, eb = _ops.lmhead_forward(hid, w, lab, 1.0)[:4]
+    dw, ref = (_ops.lmhead_backward(g_lp, g_en, hid, w, lab, lse, eb, 1.0, vocab_chunk=c)[1] for c in (0, 4096))
+    assert torch.equal(dw, ref) and ref.float().norm() > 0
+
+
 @pytest.mark.parametrize("v", [1000, 40000, 70001])
 def test_statistics_do_not_depend_on_the_number_of_tokens(v):
     """The kernel that folds the partial statistics takes 4, 16 or 32 tokens per workgroup: a token's results are the same

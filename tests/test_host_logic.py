@@ -410,6 +410,29 @@ def test_which_output_products_take_half_tiles():
     assert ask(0, 0, 640, 8200, 0) < 0 and ask(2, 1, 640, 8200, 0) < 0 and ask(1, 1, 640, 8200, 100) < 0
 
 
+def test_which_calls_form_dweight_from_resident_rows():
+    """Both sides of each limit of the rule: 768 tokens, hidden 8192, the columns that a part of the vocabulary has (hidden 896:
+    two groups of 512 rows and 128 parts up to 320 tokens, four groups and 64 parts beyond), row tiles that fill 15 of 16
+    wavefronts beyond 640 tokens, a vocabulary that is read as it lies; no half tiles where the rows are resident."""
+    from axon_amd import _lib
+    ask = _lib.load().axon_lmhead_bwd_dweight_by_rows
+    by = lambda n, h, v, chunk=0: ask(n, n, h, v, chunk)  # noqa: E731
+    assert by(1, 4096, 151936) == 1 and by(768, 4096, 151936) == 1 and by(769, 4096, 151936) == 0
+    assert by(700, 8192, 151936) == 1 and by(700, 8224, 151936) == 0
+    assert by(1, 896, 32768) == 1 and by(256, 896, 32768) == 1 and by(256, 896, 32760) == 0
+    assert by(257, 896, 65536) == 1 and by(257, 896, 65528) == 0
+    assert by(321, 896, 65536) == 1 and by(640, 896, 65528) == 0
+    assert by(640, 896, 151936) == 1 and by(641, 896, 151936) == 0 and by(641, 1152, 151936) == 0
+    assert by(300, 4096, 50257) == 0 and by(300, 224, 151936) == 0  # vocab-major copies of the dlogits
+    assert by(700, 4096, 151936, 4096) == 0                          # short chunks of the vocabulary
+    assert ask(700, 40000, 4096, 151936, 152064) == 1                # a block shorter than the workspace
+    halves = _lib.load().axon_lmhead_bwd_half_tiles
+    assert by(700, 2880, 201088) == 1 and halves(700, 700, 2880, 201088, 0) & 2 == 0
+    assert by(769, 2880, 201088) == 0 and halves(769, 769, 2880, 201088, 0) & 2 == 2
+    assert by(700, 896, 151936) == 0 and halves(700, 700, 896, 151936, 0) & 2 == 2
+    assert ask(0, 0, 640, 8200, 0) < 0 and ask(2, 1, 640, 8200, 0) < 0 and ask(1, 1, 640, 8200, 100) < 0
+
+
 @pytest.mark.parametrize("h,v", [(896, 151936), (2880, 201088), (4096, 151936), (3072, 128264), (1024, 50257),
                                  (2048, 102400), (256, 262144), (1024, 65800), (128, 40000), (512, 1310720)])
 def test_default_backward_workspace_grows_with_the_tokens_and_stays_bounded(h, v):
