@@ -1,6 +1,7 @@
-"""Build recipe for libaxon_amd.so (HIP, gfx950 only).
+"""Build recipe for libaxon_amd.so (HIP, gfx950 only) and for _torch_ext.so, the native host side of the small
+operators (plain C++ against torch's headers, linked to the former).
 
-``build()`` always recompiles; ``ensure_built()`` compiles only when the
+``build()`` always recompiles; ``ensure_built()`` compiles only when a
 library is missing.  hipcc cross-compiles without a GPU.
 """
 
@@ -14,6 +15,7 @@ import tempfile
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(_HERE, "libaxon_amd.so")
+EXT_PATH = os.path.join(_HERE, "_torch_ext.so")
 SOURCES = ("capi.hip", "rows.hip", "loss.hip", "owned.hip", "diag.hip", "returns.hip", "cov.hip", "logits.hip", "step.hip", "lmhead.hip")
 
 HIPCC_FLAGS = (
@@ -47,9 +49,28 @@ def _run(cmd, cwd) -> str:
     return log
 
 
+def _ext_commands(obj: str, out: str, lib_dir: str):
+    """Compile and link commands of the torch extension; HIP's runtime is the one that torch brings."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    includes = [*include_paths("cuda"), sysconfig.get_paths()["include"]]
+    compile_cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1",
+                   "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                   "-DTORCH_EXTENSION_NAME=_torch_ext", *(a for i in includes for a in ("-isystem", i)),
+                   "-c", os.path.join(CSRC, "torch_ext.cpp"), "-o", obj]
+    link_cmd = ["g++", "-shared", "-o", out, obj, f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+                "-ltorch_python", f"-L{lib_dir}", "-l:libaxon_amd.so", "-Wl,-rpath,$ORIGIN"]
+    return compile_cmd, link_cmd
+
+
 def build(verbose: bool = False) -> str:
     """Compile every HIP source into ``axon_amd/libaxon_amd.so`` and return its path.  One hipcc per source,
-    side by side (the file with the most kernel instantiations takes a minute alone), then one link."""
+    side by side (the file with the most kernel instantiations takes a minute alone), then one link; the torch
+    extension beside them."""
     from concurrent.futures import ThreadPoolExecutor
 
     hipcc = _hipcc()
@@ -57,17 +78,22 @@ def build(verbose: bool = False) -> str:
     with tempfile.TemporaryDirectory(prefix="axon_amd_build_") as tmp:
         objs = [os.path.join(tmp, os.path.splitext(s)[0] + ".o") for s in SOURCES]
         cmds = [[hipcc, *compile_flags, "-c", os.path.join(CSRC, s), "-o", o] for s, o in zip(SOURCES, objs)]
+        ext = os.path.join(tmp, "_torch_ext.so")
+        ext_compile, ext_link = _ext_commands(os.path.join(tmp, "torch_ext.o"), ext, tmp)
+        cmds.append(ext_compile)
         with ThreadPoolExecutor(max_workers=min(len(cmds), os.cpu_count() or 1, 8)) as pool:
             logs = list(pool.map(lambda c: _run(c, tmp), cmds))
         out = os.path.join(tmp, "libaxon_amd.so")
         logs.append(_run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", "-o", out, *objs], tmp))
+        logs.append(_run(ext_link, tmp))
         if verbose and any(l.strip() for l in logs):
             print("\n".join(l for l in logs if l.strip()))
         shutil.move(out, LIB_PATH)
+        shutil.move(ext, EXT_PATH)
     return LIB_PATH
 
 
 def ensure_built() -> str:
-    if not os.path.exists(LIB_PATH):
+    if not (os.path.exists(LIB_PATH) and os.path.exists(EXT_PATH)):
         build()
     return LIB_PATH

@@ -125,6 +125,7 @@ MASK_F32, MASK_I64 = 0, 1
 
 _lock = threading.Lock()
 _lib = None
+_ext = None
 
 
 class AxonAmdError(RuntimeError):
@@ -157,6 +158,17 @@ def load() -> ctypes.CDLL:
             raise AxonAmdError(f"libaxon_amd.so ABI {got}, bindings expect {ABI_VERSION}")
         _lib = lib
     return _lib
+
+
+def native():
+    """The torch extension ``_torch_ext`` (csrc/torch_ext.cpp): the operators whose host side is native."""
+    global _ext
+    if _ext is None:
+        load()
+        import importlib
+
+        _ext = importlib.import_module("axon_amd._torch_ext")
+    return _ext
 
 
 def check(rc: int, what: str) -> None:

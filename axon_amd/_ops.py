@@ -27,6 +27,11 @@ class Rows:
     shape: tuple
 
     @property
+    def native(self):
+        """As the torch extension takes it; it refuses offsets that live in host memory."""
+        return self.n_rows, self.n_slots, self.uniform_len, self.cu, self.shape
+
+    @property
     def cu_ptr(self):
         # the kernels dereference this pointer: offsets that live in host memory would fault the GPU
         if self.cu is not None and not self.cu.is_cuda:
@@ -191,22 +196,9 @@ def group_advantage(rewards, mask, gidx, n_groups, rows: Rows, *, eps, mode, cla
     mask.  Two launches (axon_group_advantage) unless the rows are very short or long on average or there are more
     groups than fit in LDS; the row pass, group kernel and broadcast one by one then."""
     if 0 < n_groups <= GROUP_ADVANTAGE_MAX_GROUPS and _own_rows(rows):
-        lib = _lib.load()
         require_device(rewards, "group_advantage")
-        _same_len("group_advantage", rows.n_slots, rewards=rewards, mask=mask)
-        _same_len("group_advantage", rows.n_rows, gidx=gidx)
-        dev = rewards.device
-        rw = f32(rewards)
-        mk, kind = mask_arg(mask)
-        scratch = torch.empty(2 * rows.n_rows, device=dev, dtype=torch.float32)
-        out = torch.empty(rows.shape, device=dev, dtype=torch.float32)
-        check(
-            lib.axon_group_advantage(ptr(rw), ptr(mk), kind, rows.cu_ptr, rows.n_rows, rows.n_slots, rows.uniform_len,
-                                     ptr(gidx), int(n_groups), float(eps), int(mode), float(clamp_abs), ptr(scratch),
-                                     ptr(out), ptr(_partials(rows.n_slots, dev)), stream_ptr()),
-            "axon_group_advantage",
-        )
-        return out
+        return _lib.native().group_advantage(rewards, mask, gidx, int(n_groups), rows.native, float(eps), int(mode),
+                                             float(clamp_abs), _partials(rows.n_slots, rewards.device))
     _, scores, _ = row_stats(rewards, None, None, rows, want_cnt=False)
     _, _, _, scalar = group_stats(scores, gidx, n_groups, eps, mode)
     return row_broadcast_mask(scalar, mask, rows, clamp_abs=clamp_abs)
@@ -218,25 +210,9 @@ SCAN_GAE, SCAN_GAE_RESPONSE_ONLY, SCAN_DISCOUNTED, SCAN_SUFFIX_SUM = 0, 1, 2, 3
 def reverse_scan(mode, rewards, values, mask, rows: Rows, *, gamma=1.0, lam=1.0, row_baseline=None):
     """Time recurrence from each row's last token to its first; returns ``(adv | None, ret)``.  See
     axon_reverse_scan."""
-    lib = _lib.load()
     require_device(rewards, "reverse_scan")
-    _same_len("reverse_scan", rows.n_slots, rewards=rewards, values=values, mask=mask)
-    dev = rewards.device
-    rewards = f32(rewards)
-    values = f32(values) if values is not None else None
-    mk, kind = mask_arg(mask)
-    base = f32(row_baseline).reshape(-1) if row_baseline is not None else None
-    if base is not None and base.numel() != rows.n_rows:
-        raise ValueError(f"row_baseline has {base.numel()} entries, batch has {rows.n_rows} rows")
-    adv = None if mode == SCAN_DISCOUNTED else torch.empty(rows.shape, device=dev, dtype=torch.float32)
-    ret = torch.empty(rows.shape, device=dev, dtype=torch.float32)
-    check(
-        lib.axon_reverse_scan(mode, ptr(rewards), ptr(values), ptr(mk), kind, rows.cu_ptr, rows.n_rows, rows.n_slots,
-                              rows.uniform_len, float(gamma), float(lam), ptr(base), ptr(adv), ptr(ret),
-                              stream_ptr()),
-        "axon_reverse_scan",
-    )
-    return adv, ret
+    return _lib.native().reverse_scan(mode, rewards, values, mask, rows.native, float(gamma), float(lam), row_baseline,
+                                      mode != SCAN_DISCOUNTED)
 
 
 def masked_whiten(x, mask, *, remask=False, inplace=False, stats_only=False):
@@ -375,26 +351,12 @@ def sampler_correction_diag(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_th
                      rs_hi=rs_hi, rs_lr_lo=tok_lo, rs_lr_hi=tok_hi, log_is_lo=log_is_lo, log_is_hi=log_is_hi,
                      log_rs_lo=log_rs_lo, log_rs_hi=log_rs_hi, out=out)
         return isw, new_mask
-    lib = _lib.load()
     require_device(old_lp, "sampler_correction")
-    _same_len("sampler_correction", rows.n_slots, old_log_probs=old_lp, sampler_log_probs=samp_lp, mask=mask)
-    dev = old_lp.device
-    old_lp, samp_lp = f32(old_lp), f32(samp_lp)
-    mk, kind = mask_arg(mask)
-    isw = torch.empty(rows.shape, device=dev, dtype=torch.float32) if is_mode else None
-    new_mask = torch.empty(rows.shape, device=dev, dtype=torch.float32)
-    nbytes = lib.axon_sampler_correction_diag_workspace_bytes(rows.n_rows, rows.n_slots)
-    ws = torch.empty(nbytes // 4, device=dev, dtype=torch.float32)
-    check(
-        lib.axon_sampler_correction_diag(
-            ptr(old_lp), ptr(samp_lp), ptr(mk), kind, rows.cu_ptr, rows.n_rows, rows.n_slots, rows.uniform_len, is_mode,
-            float(is_threshold), rs_mode, float(rs_lr_lo), float(rs_lr_hi), int(log_veto is not None),
-            float(log_veto if log_veto is not None else 0.0), float(is_lo), float(is_hi), float(rs_lo), float(rs_hi),
-            float(log_is_lo), float(log_is_hi), float(log_rs_lo), float(log_rs_hi), ptr(isw), ptr(new_mask), ptr(acc),
-            ptr(_partials(rows.n_slots, dev)), ptr(ws), ptr(out), stream_ptr()),
-        "axon_sampler_correction_diag",
-    )
-    return isw, new_mask
+    return _lib.native().sampler_correction_diag(
+        old_lp, samp_lp, mask, rows.native, is_mode, float(is_threshold), rs_mode, float(rs_lr_lo), float(rs_lr_hi),
+        None if log_veto is None else float(log_veto), float(is_lo), float(is_hi), float(rs_lo), float(rs_hi),
+        float(log_is_lo), float(log_is_hi), float(log_rs_lo), float(log_rs_hi), acc, out,
+        _partials(rows.n_slots, old_lp.device))
 
 
 def sampler_diag(old_lp, samp_lp, mask, rows: Rows, *, is_mode, is_lo, is_hi, rs_mode, rs_lo, rs_hi, rs_lr_lo,
@@ -451,19 +413,10 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
     acc[0] is the loss; acc[1:5] are the metric sums; acc[5] is the factor the returned
     gradient still has to be multiplied by (see axon_policy_loss).
     """
-    lib = _lib.load()
     require_device(log_probs, "policy_loss")
-    _same_len("policy_loss", rows.n_slots, log_probs=log_probs, old_log_probs=old_log_probs, advantages=advantages,
-              mask=mask, is_weights=is_weights)
     dev = log_probs.device
-    lp, old, adv = f32(log_probs), f32(old_log_probs), f32(advantages)
-    mk, mkind = mask_arg(mask)
-    isw = f32(is_weights) if is_weights is not None else None
     tr, br = TOKEN_REDUCE[token_reduce], BATCH_REDUCE[batch_reduce]
-
     valid = _count_dev(valid_count, dev)
-    grad = torch.empty(rows.shape, device=dev, dtype=torch.float32)
-    acc = _acc8(rows.n_slots, dev, acc)
     # PPO with sum / token-mean needs no per-row quantity: one pass over the tokens, the
     # division by the token count happens when the last workgroup has the total.
     one_pass = kind != 1 and tr == 0 and br == 0
@@ -472,35 +425,45 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
     nps = _count_dev(num_program_steps, dev, rows.n_rows, "num_program_steps") if br == 2 else None
     if not one_pass and tr == 2 and not rows.uniform_len:
         raise ValueError("token_reduce='mean-norm' divides by the padded row length: needs a [batch, seq] layout")
-    if not one_pass and _own_rows(rows):
-        # a workgroup owns whole rows: one launch, still one pass over the tokens
-        check(
-            lib.axon_policy_loss_rows(kind, ptr(lp), ptr(old), ptr(adv), ptr(mk), mkind, ptr(isw), rows.cu_ptr,
-                                      rows.n_rows, rows.n_slots, rows.uniform_len, tr, br, ptr(prtc), ptr(npt),
-                                      ptr(nps), ptr(valid), float(ratio_lo), float(ratio_hi), float(clip_c),
-                                      ptr(grad), ptr(acc), ptr(_partials(rows.n_slots, dev)), stream_ptr()),
-            "axon_policy_loss_rows",
-        )
-        return (acc, grad, 0.5) if halve else (acc, grad)
-    row_scale = row_mean = None
-    if not one_pass:  # very large batches: row pass, row scales, token pass
-        cnt, ssum, _ = row_stats(lp, old, mk, rows, want_sum=(kind == 1))
-        row_scale = torch.empty(rows.n_rows, device=dev, dtype=torch.float32)
-        row_mean = torch.empty(rows.n_rows, device=dev, dtype=torch.float32) if kind == 1 else None
-        check(
-            lib.axon_loss_row_scale(ptr(cnt), ptr(ssum), rows.n_rows, rows.uniform_len if rows.uniform_len else 0, tr,
-                                    br, ptr(prtc), ptr(npt), ptr(nps), ptr(valid), ptr(row_scale), ptr(row_mean),
-                                    stream_ptr()),
-            "axon_loss_row_scale",
-        )
+    if one_pass or _own_rows(rows):
+        # one launch, one pass over the tokens; with per-row quantities a workgroup owns whole rows
+        scale = 0.5 if halve and one_pass else 1.0
+        acc, grad = _lib.native().policy_loss(
+            kind, log_probs, old_log_probs, advantages, mask, is_weights, rows.native, tr, br, prtc, npt, nps, valid,
+            float(ratio_lo), float(ratio_hi), float(clip_c), acc, scale, one_pass, _partials(rows.n_slots, dev))
+        return (acc, grad, 1.0 if one_pass else 0.5) if halve else (acc, grad)
+    # very large batches: row pass, row scales, token pass
+    lib = _lib.load()
+    _same_len("policy_loss", rows.n_slots, log_probs=log_probs, old_log_probs=old_log_probs, advantages=advantages,
+              mask=mask, is_weights=is_weights)
+    lp, old, adv = f32(log_probs), f32(old_log_probs), f32(advantages)
+    mk, mkind = mask_arg(mask)
+    isw = f32(is_weights) if is_weights is not None else None
+    grad = torch.empty(rows.shape, device=dev, dtype=torch.float32)
+    acc = _acc8(rows.n_slots, dev, acc)
+    cnt, ssum, _ = row_stats(lp, old, mk, rows, want_sum=(kind == 1))
+    row_scale = torch.empty(rows.n_rows, device=dev, dtype=torch.float32)
+    row_mean = torch.empty(rows.n_rows, device=dev, dtype=torch.float32) if kind == 1 else None
+    check(
+        lib.axon_loss_row_scale(ptr(cnt), ptr(ssum), rows.n_rows, rows.uniform_len if rows.uniform_len else 0, tr, br,
+                                ptr(prtc), ptr(npt), ptr(nps), ptr(valid), ptr(row_scale), ptr(row_mean), stream_ptr()),
+        "axon_loss_row_scale",
+    )
     check(
         lib.axon_policy_loss(kind, ptr(lp), ptr(old), ptr(adv), ptr(mk), mkind, ptr(isw), rows.cu_ptr, rows.n_rows,
-                             rows.n_slots, rows.uniform_len, ptr(row_scale), ptr(row_mean), 0.5 if halve else 1.0, int(one_pass),
-                             ptr(valid if one_pass else None), float(ratio_lo), float(ratio_hi), float(clip_c),
-                             ptr(grad), ptr(acc), ptr(_partials(rows.n_slots, dev)), stream_ptr()),
+                             rows.n_slots, rows.uniform_len, ptr(row_scale), ptr(row_mean), 0.5 if halve else 1.0, 0, None,
+                             float(ratio_lo), float(ratio_hi), float(clip_c), ptr(grad), ptr(acc),
+                             ptr(_partials(rows.n_slots, dev)), stream_ptr()),
         "axon_policy_loss",
     )
-    return (acc, grad, 0.5 if row_scale is not None else 1.0) if halve else (acc, grad)
+    return (acc, grad, 0.5) if halve else (acc, grad)
+
+
+def finished_loss(x, acc, grad, factor=1.0, slot=5):
+    """``factor * acc[0]`` as the loss of a kernel that has left its gradient with respect to ``x`` in ``grad``: a 0-d tensor
+    whose backward multiplies ``grad`` by the upstream gradient, by ``factor`` and by ``acc[slot]`` (the 1/denominator that
+    a one-pass token-mean leaves to this multiply; -1: nothing left)."""
+    return _lib.native().finished_loss(x, acc, grad, factor, slot)
 
 
 def cov_policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, rows: Rows, *, select_ratio,
@@ -1079,21 +1042,8 @@ class HeadBlocks:
 def scale_f32(x, s1, s2=None):
     """``x * s1 * s2`` for an fp32 array and one or two device scalars (0-d or 1-element fp32 tensors), in one
     launch; a new tensor shaped like ``x``."""
-    lib = _lib.load()
     require_device(x, "scale_f32")
-    xf = f32(x)
-
-    def scalar(t):
-        t = t.detach()
-        if t.dtype != torch.float32 or t.device != xf.device:
-            t = t.to(device=xf.device, dtype=torch.float32)
-        return t
-
-    a = scalar(s1)
-    b = scalar(s2) if s2 is not None else None
-    out = torch.empty_like(xf)
-    check(lib.axon_scale_f32(ptr(xf), ptr(a), ptr(b), ptr(out), int(xf.numel()), stream_ptr()), "axon_scale_f32")
-    return out.view(x.shape)
+    return _lib.native().scale_f32(x, s1, s2)
 
 
 def scale_bf16_unless_one(x, y, scale):

@@ -24,57 +24,6 @@ from axon_amd.trainer.algos.loss.registry import LossFn, register_loss
 _KIND_PPO, _KIND_GSPO, _KIND_REINFORCE, _KIND_CISPO, _KIND_VALUE = 0, 1, 2, 3, 4
 
 
-def _loss_of(acc):
-    """``acc[0]`` as a tensor of its own: no view (the caller may change it in place, and nothing reads it again), and
-    no launch that copies it."""
-    return torch.empty(0, device=acc.device, dtype=acc.dtype).set_(acc.untyped_storage(), acc.storage_offset(), ())
-
-
-def _defined(g_loss, like):
-    """The upstream gradient of a loss whose node does not have undefined gradients filled with zeros."""
-    return torch.zeros((), device=like.device) if g_loss is None else g_loss
-
-
-class _ClippedPolicyLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, log_probs, kind, batch, rows, hp):
-        acc, grad = _ops.policy_loss(
-            kind, log_probs, batch["old_log_probs"], batch["advantages"], batch["response_mask"],
-            batch["sampler_is_weights"], rows, **hp,
-        )
-        ctx.save_for_backward(grad, acc)
-        ctx.in_dtype = log_probs.dtype
-        ctx.mark_non_differentiable(acc)
-        ctx.set_materialize_grads(False)  # no zeros for it in the backward
-        return _loss_of(acc), acc
-
-    @staticmethod
-    def backward(ctx, g_loss, _g_acc):
-        grad, acc = ctx.saved_tensors
-        # acc[5]: the 1/denominator a one-pass token-mean leaves to this multiply
-        return _ops.scale_f32(grad, _defined(g_loss, grad), acc[5]).to(ctx.in_dtype), None, None, None, None
-
-
-class _ValueLoss(torch.autograd.Function):
-    """Half the aggregated value loss (the kernel halves the terms where it can, which is exact)."""
-
-    @staticmethod
-    def forward(ctx, vpreds, batch, rows, hp):
-        acc, grad, ctx.half = _ops.policy_loss(_KIND_VALUE, vpreds, batch["old_log_probs"], batch["advantages"],
-                                               batch["response_mask"], None, rows, halve=True, **hp)
-        ctx.save_for_backward(grad, acc)
-        ctx.in_dtype = vpreds.dtype
-        ctx.mark_non_differentiable(acc)
-        ctx.set_materialize_grads(False)
-        return (_loss_of(acc) if ctx.half == 1.0 else ctx.half * acc[0]), acc
-
-    @staticmethod
-    def backward(ctx, g_loss, _g_acc):
-        grad, acc = ctx.saved_tensors
-        g_loss = _defined(g_loss, grad)
-        return _ops.scale_f32(grad, g_loss if ctx.half == 1.0 else ctx.half * g_loss, acc[5]).to(ctx.in_dtype), None, None, None
-
-
 def _aggregation(b, config, default_token_reduce: str) -> dict:
     """The ``agg_loss`` arguments of a loss call (loss/utils.py:120-251), validated as the reference does."""
     token_reduce = config.get("token_reduce", default_token_reduce)
@@ -155,7 +104,9 @@ def _run(kind: int, data, config, default_token_reduce: str, corr=None):
     log_probs, rows, tensors, hp = policy_loss_spec(kind, data, config, default_token_reduce)
     if corr is not None:
         hp["acc"] = corr.loss_acc
-    loss, acc = _ClippedPolicyLoss.apply(log_probs, kind, tensors, rows, hp)
+    acc, grad = _ops.policy_loss(kind, log_probs, tensors["old_log_probs"], tensors["advantages"], tensors["response_mask"],
+                                 tensors["sampler_is_weights"], rows, **hp)
+    loss = _ops.finished_loss(log_probs, acc, grad)
     sums = acc.tolist() if corr is None else corr.read()  # the only host sync of the loss
     return loss, policy_loss_metrics(kind, sums)
 
@@ -190,23 +141,6 @@ def cispo_loss_fn(data, config, corr=None) -> tuple[torch.Tensor, dict[str, Any]
     return _run(_KIND_CISPO, data, config, "sum", corr)
 
 
-class _GmpoLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, log_probs, batch, rows, clip_low, clip_high):
-        acc, grad = _ops.gmpo_loss(log_probs, batch["old_log_probs"], batch["advantages"], batch["response_mask"],
-                                   batch["sampler_is_weights"], rows, clip_low=clip_low, clip_high=clip_high)
-        ctx.save_for_backward(grad)
-        ctx.in_dtype = log_probs.dtype
-        ctx.mark_non_differentiable(acc)
-        ctx.set_materialize_grads(False)  # no zeros for it in the backward
-        return _loss_of(acc), acc
-
-    @staticmethod
-    def backward(ctx, g_loss, _g_acc):
-        (grad,) = ctx.saved_tensors
-        return _ops.scale_f32(grad, _defined(g_loss, grad)).to(ctx.in_dtype), None, None, None, None
-
-
 @register_loss(LossFn.GEO_MEAN)
 def geo_mean_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
     """GMPO: sequence-level geometric-mean ratio with token-level clipping of the log-ratio
@@ -220,9 +154,9 @@ def geo_mean_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
     log_probs = b["log_probs"]
     _lib.require_device(log_probs, "policy loss")
     rows = _ops.rows_of(log_probs, data.meta_info.get("cu_seqlens", None) if data.meta_info else None)
-    tensors = {"old_log_probs": b["old_log_probs"], "advantages": b["advantages"], "response_mask": b["response_mask"],
-               "sampler_is_weights": b.get("sampler_is_weights", None)}
-    loss, acc = _GmpoLoss.apply(log_probs, tensors, rows, lo, hi)
+    acc, grad = _ops.gmpo_loss(log_probs, b["old_log_probs"], b["advantages"], b["response_mask"],
+                               b.get("sampler_is_weights", None), rows, clip_low=lo, clip_high=hi)
+    loss = _ops.finished_loss(log_probs, acc, grad, slot=-1)
     sums = acc.tolist()
     denom = max(sums[4], 1.0)
     return loss, {"pg_clipfrac": sums[1] / denom, "ppo_kl": sums[2] / denom, "pg_clipfrac_lower": sums[3] / denom}
@@ -238,32 +172,15 @@ def value_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
     agg = _aggregation(b, config, "sum")
     _lib.require_device(vpreds, "value loss")
     rows = _ops.rows_of(vpreds, data.meta_info.get("cu_seqlens", None) if data.meta_info else None)
-    tensors = {"old_log_probs": b["values"], "advantages": b["returns"], "response_mask": b["response_mask"]}
     hp = dict(ratio_lo=config.get("cliprange_value", 0.5), ratio_hi=0.0, clip_c=0.0, **agg)
-    loss, acc = _ValueLoss.apply(vpreds, tensors, rows, hp)
+    # half the aggregated loss: the kernel halves the terms where it can, which is exact
+    acc, grad, left = _ops.policy_loss(_KIND_VALUE, vpreds, b["values"], b["returns"], b["response_mask"], None, rows,
+                                       halve=True, **hp)
+    loss = _ops.finished_loss(vpreds, acc, grad, left)
     sums = acc.tolist()
     denom = max(sums[4], 1.0)
     half = 1.0 if _ops.policy_loss_halves(**agg) else 0.5
     return loss, {"vf_loss": half * sums[0], "vf_clipfrac": sums[1] / denom, "vpred_mean": sums[2] / denom}
-
-
-class _CovPolicyLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, log_probs, kind, batch, rows, hp):
-        acc, grad, _, _ = _ops.cov_policy_loss(
-            kind, log_probs, batch["old_log_probs"], batch["advantages"], batch["response_mask"],
-            batch["sampler_is_weights"], rows, **hp,
-        )
-        ctx.save_for_backward(grad, acc)
-        ctx.in_dtype = log_probs.dtype
-        ctx.mark_non_differentiable(acc)
-        ctx.set_materialize_grads(False)  # no zeros for it in the backward
-        return _loss_of(acc), acc
-
-    @staticmethod
-    def backward(ctx, g_loss, _g_acc):
-        grad, acc = ctx.saved_tensors
-        return _ops.scale_f32(grad, _defined(g_loss, grad), acc[5]).to(ctx.in_dtype), None, None, None, None
 
 
 def _run_cov(kind: int, data, config, hp: dict, default_token_reduce: str):
@@ -272,9 +189,9 @@ def _run_cov(kind: int, data, config, hp: dict, default_token_reduce: str):
     agg = _aggregation(b, config, default_token_reduce)
     _lib.require_device(log_probs, "policy loss")
     rows = _ops.rows_of(log_probs, data.meta_info.get("cu_seqlens", None) if data.meta_info else None)
-    tensors = {"old_log_probs": b["old_log_probs"], "advantages": b["advantages"],
-               "response_mask": b["response_mask"], "sampler_is_weights": b.get("sampler_is_weights", None)}
-    loss, acc = _CovPolicyLoss.apply(log_probs, kind, tensors, rows, dict(**hp, **agg))
+    acc, grad, _, _ = _ops.cov_policy_loss(kind, log_probs, b["old_log_probs"], b["advantages"], b["response_mask"],
+                                           b.get("sampler_is_weights", None), rows, **hp, **agg)
+    loss = _ops.finished_loss(log_probs, acc, grad)
     sums = acc.tolist()
     return loss, sums, max(sums[4], 1.0)
 

@@ -19,26 +19,6 @@ from axon_amd.trainer.algos.constants import VALID_BATCH_REDUCE, VALID_TOKEN_RED
 __all__ = ["agg_loss", "masked_mean"]
 
 
-class _WeightedRowSum(torch.autograd.Function):
-    """sum_t loss[t] * mask[t] * row_scale[row(t)] with gradient mask*row_scale: the entropy slot of
-    ``axon_side_terms`` (one pass for sum / token-mean, a row pass first otherwise)."""
-
-    @staticmethod
-    def forward(ctx, loss_mat, mask, rows, token_reduce, batch_reduce, extras):
-        prtc, npt, nps, valid = extras
-        acc, agg_w, _ = _ops.side_terms(loss_mat, None, None, mask, rows, token_reduce=token_reduce,
-                                        batch_reduce=batch_reduce, per_row_token_count=prtc, num_program_tokens=npt,
-                                        num_program_steps=nps, valid_count=valid)
-        ctx.save_for_backward(agg_w, acc)
-        ctx.in_dtype = loss_mat.dtype
-        return acc[0].clone()
-
-    @staticmethod
-    def backward(ctx, g):
-        agg_w, acc = ctx.saved_tensors
-        return _ops.scale_f32(agg_w, g, acc[5]).to(ctx.in_dtype), None, None, None, None, None
-
-
 def agg_loss(
     loss_mat: torch.Tensor,
     loss_mask: torch.Tensor,
@@ -71,10 +51,13 @@ def agg_loss(
         valid = valid_batch_size
     _lib.require_device(loss_mat, "agg_loss")
     rows = _ops.rows_of(loss_mat, cu_seqlens)
-    return _WeightedRowSum.apply(
-        loss_mat, loss_mask, rows, token_reduce, batch_reduce,
-        (per_row_token_count, num_program_tokens, num_program_steps, valid),
-    )
+    # sum_t loss[t] * mask[t] * row_scale[row(t)] with gradient mask*row_scale: the entropy slot of axon_side_terms
+    # (one pass for sum / token-mean, a row pass first otherwise)
+    acc, agg_w, _ = _ops.side_terms(loss_mat, None, None, loss_mask, rows, token_reduce=token_reduce,
+                                    batch_reduce=batch_reduce, per_row_token_count=per_row_token_count,
+                                    num_program_tokens=num_program_tokens, num_program_steps=num_program_steps,
+                                    valid_count=valid)
+    return _ops.finished_loss(loss_mat, acc, agg_w)
 
 
 def masked_mean(values: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:

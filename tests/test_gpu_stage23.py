@@ -939,6 +939,61 @@ def test_two_hip_graphs_replayed_in_the_other_order():
         _ops._PARTIALS.update(keep)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("loss_fn", ["ppo", "gspo", "geo_mean", "value"])
+def test_the_node_of_a_loss_is_an_autograd_function_like_any_other(loss_fn, dtype):
+    """Upstream factors, a second pass through a retained graph, a released graph, saved-tensor hooks, a loss changed in
+    place, a backward on another thread and stream, and what such a node refuses (forward mode, vmap)."""
+    import threading
+
+    g = torch.Generator(device=DEV).manual_seed(5)
+    b, t = 16, 130
+    old = -torch.empty(b, t, device=DEV).exponential_(1.0, generator=g)
+    new = (old + 0.05 * torch.randn(b, t, device=DEV, generator=g)).to(dtype)
+    batch = {"old_log_probs": old, "values": old, "advantages": torch.randn(b, t, device=DEV, generator=g),
+             "returns": torch.randn(b, t, device=DEV, generator=g), "response_mask": torch.ones(b, t, device=DEV)}
+
+    def loss_of(x):
+        data = DataProto.from_dict(tensors={**batch, "log_probs": x, "vpreds": x})
+        return compute_loss_fn(data, loss_fn, {})[0]
+
+    x = new.clone().requires_grad_(True)
+    (once,) = torch.autograd.grad(loss_of(x), x)
+    assert once.dtype == dtype and once.shape == x.shape and once.float().norm() > 0
+    loss = loss_of(x)
+    value = loss.item()
+    loss.backward(torch.tensor(4.0, device=DEV), retain_graph=True)
+    assert torch.equal(x.grad, 4 * once)  # a power of two
+    loss.backward()
+    torch.testing.assert_close(x.grad, 5 * once, rtol=2 ** -7 if dtype == torch.bfloat16 else 1e-6, atol=0)
+    with pytest.raises(RuntimeError, match="second time"):
+        loss.backward()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda s: packed.append(s) or s.cpu(), lambda s: s.to(DEV)):
+        loss = loss_of(x)
+    assert len(packed) >= 1
+    loss.mul_(2.0)  # a tensor of its own: twice the loss, twice the gradient
+    assert loss.item() == 2 * value and torch.equal(torch.autograd.grad(loss, x)[0], 2 * once)
+
+    side, got = torch.cuda.Stream(), []
+    side.wait_stream(torch.cuda.current_stream())
+
+    def work():
+        with torch.cuda.stream(side):
+            got.append(torch.autograd.grad(loss_of(x), x)[0])
+
+    thread = threading.Thread(target=work)
+    thread.start()
+    thread.join()
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(got[0], once)
+    assert loss_of(new).grad_fn is None
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):
+        loss_of(torch.autograd.forward_ad.make_dual(new, torch.ones_like(new)))
+    with pytest.raises(RuntimeError):
+        torch.vmap(loss_of)(new[None])
+
+
 # ---- kernels in which a workgroup owns whole rows (GSPO, per-row aggregation, veto, sequence level) --------
 def _awkward_packed(lens, seed):
     """Packed inputs over rows of the given lengths (zeros allowed), padded twins for the oracle."""
