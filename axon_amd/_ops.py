@@ -405,13 +405,15 @@ def policy_loss_halves(*, token_reduce, batch_reduce, **_):
 
 def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, rows: Rows, *, token_reduce,
                 batch_reduce, ratio_lo, ratio_hi, clip_c, per_row_token_count=None, num_program_tokens=None,
-                num_program_steps=None, valid_count=None, acc=None, halve=False):
+                num_program_steps=None, valid_count=None, acc=None, halve=False, post=None):
     """Forward + gradient of the clipped policy loss.  Returns (acc[8], grad like log_probs); ``acc``: where the
     eight sums go (zeros when there are no slots), else a tensor of its own.  ``halve``: half the loss is wanted; a third
     value says what is left to multiply loss and gradient by (1.0 where ``policy_loss_halves``, else 0.5).
 
     acc[0] is the loss; acc[1:5] are the metric sums; acc[5] is the factor the returned
     gradient still has to be multiplied by (see axon_policy_loss).
+
+    ``post``: a ``loss_sums_post`` that the launch sends the sums to, where it can.
     """
     require_device(log_probs, "policy_loss")
     dev = log_probs.device
@@ -430,7 +432,7 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
         scale = 0.5 if halve and one_pass else 1.0
         acc, grad = _lib.native().policy_loss(
             kind, log_probs, old_log_probs, advantages, mask, is_weights, rows.native, tr, br, prtc, npt, nps, valid,
-            float(ratio_lo), float(ratio_hi), float(clip_c), acc, scale, one_pass, _partials(rows.n_slots, dev))
+            float(ratio_lo), float(ratio_hi), float(clip_c), acc, scale, one_pass, _partials(rows.n_slots, dev), post)
         return (acc, grad, 1.0 if one_pass else 0.5) if halve else (acc, grad)
     # very large batches: row pass, row scales, token pass
     lib = _lib.load()
@@ -457,6 +459,18 @@ def policy_loss(kind, log_probs, old_log_probs, advantages, mask, is_weights, ro
         "axon_policy_loss",
     )
     return (acc, grad, 0.5) if halve else (acc, grad)
+
+
+def loss_sums_post(also=None):
+    """What ``policy_loss(post=)`` sends its eight sums to, for a host that waits for them: the launch writes them to pinned
+    memory (behind the words of ``also``, a device tensor that earlier work has written), without a copy or a wait for the
+    stream behind it."""
+    return _lib.native().Post(also)
+
+
+def loss_sums(post, acc):
+    """The eight sums of a loss as Python floats, once they have arrived."""
+    return post.sums() if post.sent else acc.tolist()
 
 
 def finished_loss(x, acc, grad, factor=1.0, slot=5):

@@ -195,9 +195,10 @@ __device__ __forceinline__ bool publish_row_take_ticket(float* row, const float 
 // that no counter is drawn from by thousands; the second level costs 3.5 us (its own stores, ticket and loads at the
 // level the XCDs share), as much as everything else in a launch over a micro-batch.  The order of every addition is
 // fixed by the grid size alone.  The counters must be zero when the kernel starts and are zero again when it ends.
+// True in the workgroup that has called `fin`.
 constexpr unsigned kOneLevelGrid = 1024;
 template <int NV, class Fin>
-__device__ __forceinline__ void grid_finish(float (&v)[NV], float* lds /* [8 * 4] */, float* ws,
+__device__ __forceinline__ bool grid_finish(float (&v)[NV], float* lds /* [8 * 4] */, float* ws,
                                             Fin&& fin) {
   static_assert(NV <= kPartialStride, "partials row too small");
   __shared__ int s_stage;
@@ -223,7 +224,7 @@ __device__ __forceinline__ void grid_finish(float (&v)[NV], float* lds /* [8 * 4
                                       one_level ? gridDim.x : in_group) ? 1 : 0;
   }
   __syncthreads();
-  if (s_stage == 0) return;
+  if (s_stage == 0) return false;
   // every row was acknowledged at the shared level before its ticket was drawn; drop
   // what this XCD's caches may still hold of those addresses (an earlier launch), then read them
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -238,7 +239,7 @@ __device__ __forceinline__ void grid_finish(float (&v)[NV], float* lds /* [8 * 4
                                           n_groups) ? 2 : 1;
     }
     __syncthreads();
-    if (s_stage != 2) return;
+    if (s_stage != 2) return false;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   float t[kPartialStride];
@@ -253,6 +254,33 @@ __device__ __forceinline__ void grid_finish(float (&v)[NV], float* lds /* [8 * 4
   }
   block_sum<kPartialStride>(t, lds);  // the barriers above separate this use of `lds` from the first
   if (threadIdx.x == 0) fin(t);
+  return true;
+}
+
+// Sums that a host thread waits for go to it from the launch that forms them: words of earlier launches (`also`), then
+// the eight sums, to pinned host memory from word kMailData on, then the sequence number to its first word.  A device to
+// host copy behind the launch and a wait for the stream take 22 us with the launch, this 10.  The words are stored at system scope, which
+// writes through, and every thread waits for its acknowledgements before the barrier that the last store stands behind
+// (a release fence would write back the XCD's whole L2 as well, see publish_row_take_ticket).
+struct Mail {
+  const uint32_t* also;
+  int n_also;
+  uint32_t* host;  // null: nobody waits
+  uint32_t seq;
+};
+constexpr int kMailData = 16;
+// `acc`: written by this workgroup's first thread (the `fin` of grid_finish).
+__device__ __forceinline__ void post_mail(const Mail& m, const float* acc) {
+  __syncthreads();
+  for (int i = threadIdx.x; i < m.n_also + 8; i += kBlock) {
+    const uint32_t v = i < m.n_also ? m.also[i] : __float_as_uint(acc[i - m.n_also]);
+    __hip_atomic_store(m.host + kMailData + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(m.host, m.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Workgroups of a streaming launch: beyond this many chunks a workgroup walks several (every

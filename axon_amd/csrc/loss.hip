@@ -196,7 +196,7 @@ __global__ __launch_bounds__(kBlock) void policy_loss_kernel(
     const float* __restrict__ row_mean, float uniform_scale, float lo, float hi, float clip_c,
     const uint32_t* __restrict__ sel_keys, const SelectState* __restrict__ sel_state,
     float* __restrict__ grad, float* partials, int norm_slots, const double* __restrict__ valid,
-    float* __restrict__ acc) {
+    float* acc, Mail mail) {
   __shared__ int32_t lds_cu[kLdsRows];
   __shared__ float lds_red[kPartialStride * (kBlock / kWave)];
   constexpr int kChunk = kBlock * kVec * IT;
@@ -299,8 +299,9 @@ __global__ __launch_bounds__(kBlock) void policy_loss_kernel(
   }
   }  // chunk
   if (blockIdx.x == 0 && threadIdx.x == 0) a[5] = 1.f;  // gradient factor unless post-normalised
-  grid_finish<6>(a, lds_red, partials,
-                 [&](float (&tot)[kPartialStride]) { write_acc(tot, norm_slots, valid, acc); });
+  const bool finished = grid_finish<6>(
+      a, lds_red, partials, [&](float (&tot)[kPartialStride]) { write_acc(tot, norm_slots, valid, acc); });
+  if (finished && mail.host) post_mail(mail, acc);
 }
 
 // KL penalty estimators of axon/utils/rl/kl.py:154-245 with PyTorch's gradient conventions.
@@ -731,7 +732,7 @@ static int policy_loss_impl(int kind, const float* logp, const float* oldp, cons
                             const float* row_scale, const float* row_mean, float uniform_scale,
                             int post_normalize, const double* valid, float ratio_lo,
                             float ratio_hi, float clip_c, float* grad, float* acc, float* partials,
-                            void* stream) {
+                            void* stream, const Mail& mail = Mail{}) {
   const bool need_row = (row_scale != nullptr) || (kind == 1);
   int rc = check_rows2(cu, n_rows, n_slots, uniform_len, need_row);
   if (rc != AXON_OK) return rc;
@@ -747,7 +748,7 @@ static int policy_loss_impl(int kind, const float* logp, const float* oldp, cons
                      dim3(kBlock), 0, st, logp, oldp, adv, mask, isw, cu, n_rows, n_slots, uniform_len,   \
                      row_scale, row_mean, uniform_scale, ratio_lo, ratio_hi, clip_c,                      \
                      (const uint32_t*)nullptr, (const SelectState*)nullptr, grad, partials,               \
-                     post_normalize ? 1 : 0, valid, acc)
+                     post_normalize ? 1 : 0, valid, acc, mail)
 #define AXON_LAUNCH_PL(MK, KD)                                          \
   do {                                                                  \
     if (n_slots <= 256 * kBlock * kVec) AXON_LAUNCH_PL_IT(MK, KD, 1);   \
@@ -783,6 +784,18 @@ extern "C" int axon_policy_loss(int kind, const float* logp, const float* oldp, 
   return policy_loss_impl(kind, logp, oldp, adv, mask, mask_kind, isw, cu, n_rows, n_slots,
                           uniform_len, row_scale, row_mean, uniform_scale, post_normalize, valid,
                           ratio_lo, ratio_hi, clip_c, grad, acc, partials, stream);
+}
+
+extern "C" int axon_policy_loss_post(int kind, const float* logp, const float* oldp, const float* adv, const void* mask,
+                                     int mask_kind, const float* isw, int64_t n_slots, float uniform_scale,
+                                     const double* valid, float ratio_lo, float ratio_hi, float clip_c, float* grad,
+                                     float* acc, float* partials, const void* also, int64_t n_also, void* host,
+                                     uint32_t seq, void* stream) {
+  if (n_slots <= 0 || kind == 1 || n_also < 0 || n_also > AXON_MAIL_MAX_WORDS || (n_also > 0 && !also) || !host)
+    return AXON_ERR_ARG;
+  return policy_loss_impl(kind, logp, oldp, adv, mask, mask_kind, isw, nullptr, 1, n_slots, n_slots, nullptr, nullptr,
+                          uniform_scale, 1, valid, ratio_lo, ratio_hi, clip_c, grad, acc, partials, stream,
+                          Mail{static_cast<const uint32_t*>(also), (int)n_also, static_cast<uint32_t*>(host), seq});
 }
 
 // ---- the entry point that allocates nothing ---------------------------------------------------
@@ -858,7 +871,7 @@ extern "C" int axon_cov_policy_loss(int kind, const float* logp, const float* ol
   hipLaunchKernelGGL((policy_loss_kernel<MK, KD, kIter>), g, blk, 0, st, logp, oldp, adv, mask, isw, cu, \
                      n_rows, n_slots, uniform_len, row_scale, (const float*)nullptr,              \
                      uniform_scale, ratio_lo, ratio_hi, kl_coef, keys, sel, grad, partials,           \
-                     post_normalize ? 1 : 0, valid, acc)
+                     post_normalize ? 1 : 0, valid, acc, Mail{})
   if (mask_kind == AXON_MASK_F32) {
     if (kind == 0) AXON_LAUNCH_CV(AXON_MASK_F32, 5);
     else AXON_LAUNCH_CV(AXON_MASK_F32, 6);

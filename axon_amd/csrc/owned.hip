@@ -434,7 +434,7 @@ struct OwnedLossOp {
 template <int MK, int KIND, bool HAS_W>
 // four workgroups per CU: the kernel is bound by the latencies of a step, which only other steps hide
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void owned_policy_loss_kernel(OwnedLossArgs g, RowStarts rs, int stride,
-                                                                   float* ws, float* __restrict__ acc) {
+                                                                   float* ws, float* acc, Mail mail) {
   __shared__ float lds_red[kPartialStride * (kBlock / kWave)];
   // a caller-supplied batch denominator (utils.py:224-229) is known before the first token
   const float bden = (g.valid != nullptr) ? fmaxf((float)g.valid[0], 1.f) : 1.f;
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
   float part[7] = {op.a[0], op.a[1], op.a[2], op.a[3], op.a[4], 0.f, op.rows_with_tokens};
   const int batch_reduce = g.batch_reduce;
   const bool known = (g.valid != nullptr);
-  grid_finish<7>(part, lds_red, ws, [&](float (&tot)[kPartialStride]) {
+  const bool finished = grid_finish<7>(part, lds_red, ws, [&](float (&tot)[kPartialStride]) {
     // without a supplied denominator the sums were formed without it: token-mean divides by the
     // number of mask tokens, step-mean by the number of rows that have one (utils.py:236-251); the
     // gradient array is left without that division and acc[5] carries the factor
@@ -456,6 +456,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     tot[5] = factor;
     for (int k = 0; k < kPartialStride; ++k) acc[k] = tot[k];
   });
+  if (finished && mail.host) post_mail(mail, acc);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -683,12 +684,11 @@ int check_owned_rows(const int32_t* cu, int64_t n_rows, int64_t n_slots, int64_t
 
 }  // namespace
 
-extern "C" int axon_policy_loss_rows(int kind, const float* logp, const float* oldp, const float* adv,
-                                     const void* mask, int mask_kind, const float* isw, const int32_t* cu,
-                                     int64_t n_rows, int64_t n_slots, int64_t uniform_len, int token_reduce,
-                                     int batch_reduce, const double* prtc, const double* npt, const double* nps,
-                                     const double* valid, float ratio_lo, float ratio_hi, float clip_c,
-                                     float* grad, float* acc, float* partials, void* stream) {
+static int policy_loss_rows_impl(int kind, const float* logp, const float* oldp, const float* adv, const void* mask,
+                                 int mask_kind, const float* isw, const int32_t* cu, int64_t n_rows, int64_t n_slots,
+                                 int64_t uniform_len, int token_reduce, int batch_reduce, const double* prtc,
+                                 const double* npt, const double* nps, const double* valid, float ratio_lo, float ratio_hi,
+                                 float clip_c, float* grad, float* acc, float* partials, void* stream, const Mail& mail) {
   int rc = check_owned_rows(cu, n_rows, n_slots, uniform_len);
   if (rc != AXON_OK) return rc;
   if (n_slots == 0) return AXON_OK;
@@ -712,7 +712,7 @@ extern "C" int axon_policy_loss_rows(int kind, const float* logp, const float* o
     static const int resident = resident_blocks(owned_policy_loss_kernel<MK, KD, HW>);                  \
     const OwnedLaunch ol = owned_launch(n_slots, resident);                                             \
     hipLaunchKernelGGL((owned_policy_loss_kernel<MK, KD, HW>), dim3(ol.grid), dim3(kBlock), 0, st, g,   \
-                       rs, ol.stride, partials, acc);                                                   \
+                       rs, ol.stride, partials, acc, mail);                                             \
   } while (0)
 #define AXON_LAUNCH_OWNED(MK, KD)                 \
   do {                                            \
@@ -736,6 +736,30 @@ extern "C" int axon_policy_loss_rows(int kind, const float* logp, const float* o
 #undef AXON_LAUNCH_OWNED_W
   AXON_CHECK_LAUNCH();
   return AXON_OK;
+}
+
+extern "C" int axon_policy_loss_rows(int kind, const float* logp, const float* oldp, const float* adv,
+                                     const void* mask, int mask_kind, const float* isw, const int32_t* cu,
+                                     int64_t n_rows, int64_t n_slots, int64_t uniform_len, int token_reduce,
+                                     int batch_reduce, const double* prtc, const double* npt, const double* nps,
+                                     const double* valid, float ratio_lo, float ratio_hi, float clip_c,
+                                     float* grad, float* acc, float* partials, void* stream) {
+  return policy_loss_rows_impl(kind, logp, oldp, adv, mask, mask_kind, isw, cu, n_rows, n_slots, uniform_len, token_reduce,
+                               batch_reduce, prtc, npt, nps, valid, ratio_lo, ratio_hi, clip_c, grad, acc, partials,
+                               stream, Mail{});
+}
+
+extern "C" int axon_policy_loss_rows_post(int kind, const float* logp, const float* oldp, const float* adv,
+                                          const void* mask, int mask_kind, const float* isw, const int32_t* cu,
+                                          int64_t n_rows, int64_t n_slots, int64_t uniform_len, int token_reduce,
+                                          int batch_reduce, const double* prtc, const double* npt, const double* nps,
+                                          const double* valid, float ratio_lo, float ratio_hi, float clip_c,
+                                          float* grad, float* acc, float* partials, const void* also, int64_t n_also,
+                                          void* host, uint32_t seq, void* stream) {
+  if (n_slots <= 0 || n_also < 0 || n_also > AXON_MAIL_MAX_WORDS || (n_also > 0 && !also) || !host) return AXON_ERR_ARG;
+  return policy_loss_rows_impl(kind, logp, oldp, adv, mask, mask_kind, isw, cu, n_rows, n_slots, uniform_len, token_reduce,
+                               batch_reduce, prtc, npt, nps, valid, ratio_lo, ratio_hi, clip_c, grad, acc, partials,
+                               stream, Mail{static_cast<const uint32_t*>(also), (int)n_also, static_cast<uint32_t*>(host), seq});
 }
 
 extern "C" int axon_sampler_correction_rows(const float* oldp, const float* samp, const void* mask, int mask_kind,

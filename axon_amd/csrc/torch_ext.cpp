@@ -10,12 +10,18 @@
 // Nothing here computes: the arithmetic is behind axon_amd.h.  The functions take what the Python wrappers of the same
 // names (axon_amd/_ops.py) have normalised, and run without the interpreter lock, as a call through ctypes does.
 #include <ATen/ATen.h>
+#include <hip/hip_runtime_api.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <atomic>
+#include <chrono>
+#include <cstring>
+#include <memory>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -98,13 +104,126 @@ Rows rows_of(const RowsTuple& t) {
   return r;
 }
 
+// The sums of a loss on their way to the host (axon_policy_loss_post): `also`, a tensor that earlier work of the stream has
+// written, and the loss's eight sums behind it.
+// One launch writes to a slot of pinned memory at a time; a slot goes back once its words have arrived.  The slots, one
+// kilobyte each, are as many as posts were ever under way together and live until the process ends.
+struct Slot {
+  uint32_t* host;
+  uint32_t* device;
+  uint32_t seq;
+};
+class Slots {
+ public:
+  static constexpr int kWords = 16 + AXON_MAIL_MAX_WORDS + 8, kBytes = 1024, kPerBlock = 64;
+  static_assert(kWords * 4 <= kBytes, "");
+  static Slots& get() {
+    static auto* const slots = new Slots;
+    return *slots;
+  }
+  Slot take() {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    if (free_.empty()) {
+      void *host = nullptr, *device = nullptr;
+      if (hipHostMalloc(&host, kBytes * kPerBlock, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
+              hipSuccess ||
+          hipHostGetDevicePointer(&device, host, 0) != hipSuccess)
+        throw AxonError("no pinned host memory for the sums of a loss");
+      std::memset(host, 0, kBytes * kPerBlock);
+      for (int i = 0; i < kPerBlock; ++i)
+        free_.push_back(Slot{static_cast<uint32_t*>(host) + i * (kBytes / 4), static_cast<uint32_t*>(device) + i * (kBytes / 4), 0});
+    }
+    Slot s = free_.back();
+    free_.pop_back();
+    ++s.seq;
+    return s;
+  }
+  void give(const Slot& s) {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    free_.push_back(s);
+  }
+
+ private:
+  std::mutex mutex_;
+  std::vector<Slot> free_;
+};
+
+class Post {
+ public:
+  explicit Post(OptTensor also) : also_(std::move(also)) {}
+  ~Post() {  // never waited for: the slot may not be written any more before another launch gets it
+    if (!sent_) return;
+    try {
+      arrive();
+      Slots::get().give(slot_);
+    } catch (...) {
+    }
+  }
+  const void* also() const { return also_ ? also_->data_ptr() : nullptr; }
+  int64_t n_also() const { return also_ ? (int64_t)also_->nbytes() / 4 : 0; }
+  const Slot& send(void* stream) {
+    if (sent_) throw AxonError("these sums are on their way already");
+    slot_ = Slots::get().take();
+    stream_ = (hipStream_t)stream;
+    return slot_;
+  }
+  void sent(int rc) {  // a refused launch writes nothing
+    if (rc == 0) sent_ = true;
+    else Slots::get().give(slot_);
+  }
+  bool is_sent() const { return sent_; }
+  // The loss's eight sums.
+  std::vector<double> sums() {
+    arrive();
+    float v[8];
+    std::memcpy(v, slot_.host + 16 + n_also(), sizeof v);
+    Slots::get().give(slot_);
+    return {v, v + 8};
+  }
+  // All words as an fp32 tensor on the host.
+  Tensor wait() {
+    arrive();
+    const int64_t words = n_also() + 8;
+    Tensor out = at::empty({words}, at::TensorOptions().dtype(at::kFloat));
+    std::memcpy(out.data_ptr(), slot_.host + 16, words * 4);
+    Slots::get().give(slot_);
+    return out;
+  }
+
+ private:
+  // Spins while the words can be expected at once, then leaves the waiting to the runtime; the stream's end or its error
+  // ends it in any case.
+  void arrive() {
+    if (!sent_) throw AxonError("no sums are on their way");
+    sent_ = false;
+    const auto arrived = [&] { return __atomic_load_n(slot_.host, __ATOMIC_ACQUIRE) == slot_.seq; };
+    const auto start = std::chrono::steady_clock::now();
+    for (int n = 1; !arrived(); ++n) {
+      if (n % 1024) {
+        __builtin_ia32_pause();
+        continue;
+      }
+      if (std::chrono::steady_clock::now() - start < std::chrono::milliseconds(2)) continue;
+      const hipError_t err = hipStreamSynchronize(stream_);
+      if (err == hipSuccess && arrived()) break;
+      // the slot is not used again: the device may be in any state
+      throw AxonError(std::string("the sums of a loss did not arrive: ") + hipGetErrorString(err));
+    }
+  }
+
+  OptTensor also_;
+  Slot slot_{};
+  hipStream_t stream_ = nullptr;
+  bool sent_ = false;
+};
+
 std::tuple<Tensor, Tensor> policy_loss(int kind, const Tensor& log_probs, const Tensor& old_log_probs,
                                        const Tensor& advantages, const Tensor& mask, const OptTensor& is_weights,
                                        const RowsTuple& rows_tuple, int token_reduce, int batch_reduce,
                                        const OptTensor& per_row_count, const OptTensor& program_tokens,
                                        const OptTensor& program_steps, const OptTensor& valid, double ratio_lo,
                                        double ratio_hi, double clip_c, const OptTensor& acc_place, double loss_scale,
-                                       bool one_pass, const Tensor& ws) {
+                                       bool one_pass, const Tensor& ws, Post* post) {
   const Rows rows = rows_of(rows_tuple);
   const int64_t n = rows.n_slots;
   same_len("policy_loss", "log_probs", n, log_probs);
@@ -115,20 +234,35 @@ std::tuple<Tensor, Tensor> policy_loss(int kind, const Tensor& log_probs, const 
   const Tensor lp = f32(log_probs), old = f32(old_log_probs), adv = f32(advantages), isw = f32(is_weights);
   const auto mk = mask_arg(mask);
   Tensor grad = at::empty(rows.shape, opts(lp)), acc = acc8(n, lp, acc_place);
-  if (one_pass)
-    check(axon_policy_loss(kind, (const float*)ptr(lp), (const float*)ptr(old), (const float*)ptr(adv), ptr(mk.first),
-                           mk.second, (const float*)ptr(isw), rows.offsets(), rows.n_rows, n, rows.uniform_len, nullptr,
-                           nullptr, (float)loss_scale, 1, (const double*)ptr(valid), (float)ratio_lo, (float)ratio_hi,
-                           (float)clip_c, grad.data_ptr<float>(), acc.data_ptr<float>(), ws.data_ptr<float>(), stream()),
+  const float *lp_p = (const float*)ptr(lp), *old_p = (const float*)ptr(old), *adv_p = (const float*)ptr(adv),
+              *isw_p = (const float*)ptr(isw);
+  float *grad_p = grad.data_ptr<float>(), *acc_p = acc.data_ptr<float>(), *ws_p = ws.data_ptr<float>();
+  const double *prtc_p = (const double*)ptr(per_row_count), *npt_p = (const double*)ptr(program_tokens),
+               *nps_p = (const double*)ptr(program_steps), *valid_p = (const double*)ptr(valid);
+  const float lo = (float)ratio_lo, hi = (float)ratio_hi, clip = (float)clip_c, scale = (float)loss_scale;
+  void* const st = stream();
+  // (nobody can wait inside a capture, and nothing is launched without tokens: the sums stay on the device then)
+  if (post != nullptr && n > 0 && !capturing()) {
+    const Slot& slot = post->send(st);
+    const int rc =
+        one_pass ? axon_policy_loss_post(kind, lp_p, old_p, adv_p, ptr(mk.first), mk.second, isw_p, n, scale, valid_p, lo, hi,
+                                         clip, grad_p, acc_p, ws_p, post->also(), post->n_also(), slot.device, slot.seq, st)
+                 : axon_policy_loss_rows_post(kind, lp_p, old_p, adv_p, ptr(mk.first), mk.second, isw_p, rows.offsets(),
+                                              rows.n_rows, n, rows.uniform_len, token_reduce, batch_reduce, prtc_p, npt_p,
+                                              nps_p, valid_p, lo, hi, clip, grad_p, acc_p, ws_p, post->also(),
+                                              post->n_also(), slot.device, slot.seq, st);
+    post->sent(rc);
+    check(rc, one_pass ? "axon_policy_loss" : "axon_policy_loss_rows");
+  } else if (one_pass) {
+    check(axon_policy_loss(kind, lp_p, old_p, adv_p, ptr(mk.first), mk.second, isw_p, rows.offsets(), rows.n_rows, n,
+                           rows.uniform_len, nullptr, nullptr, scale, 1, valid_p, lo, hi, clip, grad_p, acc_p, ws_p, st),
           "axon_policy_loss");
-  else
-    check(axon_policy_loss_rows(kind, (const float*)ptr(lp), (const float*)ptr(old), (const float*)ptr(adv),
-                                ptr(mk.first), mk.second, (const float*)ptr(isw), rows.offsets(), rows.n_rows, n,
-                                rows.uniform_len, token_reduce, batch_reduce, (const double*)ptr(per_row_count),
-                                (const double*)ptr(program_tokens), (const double*)ptr(program_steps),
-                                (const double*)ptr(valid), (float)ratio_lo, (float)ratio_hi, (float)clip_c,
-                                grad.data_ptr<float>(), acc.data_ptr<float>(), ws.data_ptr<float>(), stream()),
+  } else {
+    check(axon_policy_loss_rows(kind, lp_p, old_p, adv_p, ptr(mk.first), mk.second, isw_p, rows.offsets(), rows.n_rows, n,
+                                rows.uniform_len, token_reduce, batch_reduce, prtc_p, npt_p, nps_p, valid_p, lo, hi, clip,
+                                grad_p, acc_p, ws_p, st),
           "axon_policy_loss_rows");
+  }
   return {acc, grad};
 }
 
@@ -255,6 +389,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     }
   });
   const py::call_guard<py::gil_scoped_release> unlocked;
+  py::class_<Post>(m, "Post")
+      .def(py::init<OptTensor>())
+      .def_property_readonly("sent", &Post::is_sent)
+      .def("sums", &Post::sums, unlocked)
+      .def("wait", &Post::wait, unlocked);
   m.def("policy_loss", &policy_loss, unlocked);
   m.def("group_advantage", &group_advantage, unlocked);
   m.def("sampler_correction_diag", &sampler_correction_diag, unlocked);

@@ -104,10 +104,11 @@ def _run(kind: int, data, config, default_token_reduce: str, corr=None):
     log_probs, rows, tensors, hp = policy_loss_spec(kind, data, config, default_token_reduce)
     if corr is not None:
         hp["acc"] = corr.loss_acc
+    post = _ops.loss_sums_post(None if corr is None else corr.sums)
     acc, grad = _ops.policy_loss(kind, log_probs, tensors["old_log_probs"], tensors["advantages"], tensors["response_mask"],
-                                 tensors["sampler_is_weights"], rows, **hp)
+                                 tensors["sampler_is_weights"], rows, post=post, **hp)
     loss = _ops.finished_loss(log_probs, acc, grad)
-    sums = acc.tolist() if corr is None else corr.read()  # the only host sync of the loss
+    sums = _ops.loss_sums(post, acc) if corr is None else corr.read(post)  # the only host sync of the loss
     return loss, policy_loss_metrics(kind, sums)
 
 
@@ -174,10 +175,11 @@ def value_loss_fn(data, config) -> tuple[torch.Tensor, dict[str, Any]]:
     rows = _ops.rows_of(vpreds, data.meta_info.get("cu_seqlens", None) if data.meta_info else None)
     hp = dict(ratio_lo=config.get("cliprange_value", 0.5), ratio_hi=0.0, clip_c=0.0, **agg)
     # half the aggregated loss: the kernel halves the terms where it can, which is exact
+    post = _ops.loss_sums_post()
     acc, grad, left = _ops.policy_loss(_KIND_VALUE, vpreds, b["values"], b["returns"], b["response_mask"], None, rows,
-                                       halve=True, **hp)
+                                       halve=True, post=post, **hp)
     loss = _ops.finished_loss(vpreds, acc, grad, left)
-    sums = acc.tolist()
+    sums = _ops.loss_sums(post, acc)
     denom = max(sums[4], 1.0)
     half = 1.0 if _ops.policy_loss_halves(**agg) else 0.5
     return loss, {"vf_loss": half * sums[0], "vf_clipfrac": sums[1] / denom, "vpred_mean": sums[2] / denom}

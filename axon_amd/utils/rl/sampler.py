@@ -213,9 +213,14 @@ class _Correction:
         """Eight more fp32 values behind the sums, for a loss whose own sums are to come back with them."""
         return self.both[-4:].view(torch.float32)
 
-    def read(self):
+    @property
+    def sums(self):
+        """The correction's own sums, for a loss that sends them to the host with its own (``_ops.loss_sums_post``)."""
+        return self.both[:-4]
+
+    def read(self, post=None):
         """Wait for everything enqueued so far; the loss's eight values."""
-        self.host = self.both.cpu()
+        self.host = post.wait().view(torch.float64) if post is not None and post.sent else self.both.cpu()
         return self.host[-4:].view(torch.float32).tolist()
 
     def start_readback(self):

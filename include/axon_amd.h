@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define AXON_AMD_ABI_VERSION 23
+#define AXON_AMD_ABI_VERSION 24
 
 enum {
   AXON_OK = 0,
@@ -556,6 +556,26 @@ int axon_policy_loss_rows(int kind, const float* logp, const float* old_logp, co
                           const double* num_program_steps, const double* valid_count, float ratio_lo,
                           float ratio_hi, float clip_c, float* grad, float* acc, float* partials,
                           void* stream);
+
+/* The two calls above for a host thread that waits for the sums: the launch itself writes them to `host`, pinned and
+ * coherent host memory that the current device can write (hipHostMallocCoherent), so that neither a copy nor a wait for the stream
+ * is needed.  host, in 32-bit words: [0] = seq once everything else has arrived (the caller makes sure that it holds
+ * another value before), from word 16 on the n_also <= AXON_MAIL_MAX_WORDS words at `also` (device memory that earlier work
+ * of the stream has written) and then acc[0..7].  n_slots > 0.  axon_policy_loss_post is the call without a per-row
+ * quantity (kind != 1, post_normalize). */
+#define AXON_MAIL_MAX_WORDS 224
+int axon_policy_loss_post(int kind, const float* logp, const float* old_logp, const float* adv, const void* mask,
+                          int mask_kind, const float* is_weights, int64_t n_slots, float uniform_scale,
+                          const double* valid_count, float ratio_lo, float ratio_hi, float clip_c, float* grad,
+                          float* acc, float* partials, const void* also, int64_t n_also, void* host, uint32_t seq,
+                          void* stream);
+int axon_policy_loss_rows_post(int kind, const float* logp, const float* old_logp, const float* adv, const void* mask,
+                               int mask_kind, const float* is_weights, const int32_t* cu_seqlens, int64_t n_rows,
+                               int64_t n_slots, int64_t uniform_len, int token_reduce, int batch_reduce,
+                               const double* per_row_token_count, const double* num_program_tokens,
+                               const double* num_program_steps, const double* valid_count, float ratio_lo,
+                               float ratio_hi, float clip_c, float* grad, float* acc, float* partials, const void* also,
+                               int64_t n_also, void* host, uint32_t seq, void* stream);
 
 /* axon_sampler_correction for the modes that need a per-row quantity (the per-sequence veto,
  * sampler.py:413-428; sequence-level weights :210-214; sequence / geometric rejection :70-79), in ONE

@@ -994,6 +994,44 @@ def test_the_node_of_a_loss_is_an_autograd_function_like_any_other(loss_fn, dtyp
         torch.vmap(loss_of)(new[None])
 
 
+@pytest.mark.parametrize("kind,reduce", [(0, ("sum", "token-mean")), (1, ("mean", "step-mean"))])
+@pytest.mark.parametrize("n", [64, 4095, 70001, 1 << 21])
+def test_sums_that_the_launch_sends_to_the_host_are_those_on_the_device(kind, reduce, n):
+    """Grids of one and of two levels of reduction, with the words of an earlier launch in front and without; posts under way
+    together, one that nobody waits for, one that no launch was given."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    old, adv = torch.randn(2, n, device=DEV, generator=g)
+    new = old + 0.05 * torch.randn(n, device=DEV, generator=g)
+    mask = (torch.rand(n, device=DEV, generator=g) > 0.3).float()
+    rows = _ops.rows_of(new, torch.tensor([0, n // 3, n], device=DEV, dtype=torch.int32))
+    if kind == 1 and not _ops._own_rows(rows):
+        rows = _ops.rows_of(new, torch.arange(0, n + 1, min(n, 256), device=DEV, dtype=torch.int32))
+    kw = dict(token_reduce=reduce[0], batch_reduce=reduce[1], ratio_lo=0.8, ratio_hi=1.28, clip_c=3.0)
+    also = torch.randn(76, device=DEV, generator=g, dtype=torch.float64)
+    posts = []
+    for k in range(100):  # more than one block of slots
+        post = _ops.loss_sums_post(also + k if k % 2 else None)
+        acc, _ = _ops.policy_loss(kind, new, old, adv * (k + 1), mask, None, rows, post=post, **kw)
+        assert post.sent
+        if k % 10 == 3:
+            del post
+        else:
+            posts.append((k, post, acc))
+    for k, post, acc in reversed(posts):
+        if k % 2:
+            words = post.wait()
+            assert torch.equal(words[:-8].view(torch.float64), (also + k).cpu()) and torch.equal(words[-8:], acc.cpu())
+        else:
+            assert _ops.loss_sums(post, acc) == acc.tolist()
+        assert not post.sent and math.isfinite(acc[0].item())
+        with pytest.raises(_lib.AxonAmdError):
+            post.wait()
+    with pytest.raises(_lib.AxonAmdError):
+        _ops.loss_sums_post().wait()
+    with pytest.raises(_lib.AxonAmdError):  # more words than a slot holds: refused before anything is launched
+        _ops.policy_loss(kind, new, old, adv, mask, None, rows, post=_ops.loss_sums_post(torch.zeros(300, device=DEV)), **kw)
+
+
 # ---- kernels in which a workgroup owns whole rows (GSPO, per-row aggregation, veto, sequence level) --------
 def _awkward_packed(lens, seed):
     """Packed inputs over rows of the given lengths (zeros allowed), padded twins for the oracle."""
