@@ -135,6 +135,14 @@ __device__ __forceinline__ void mfma_16x16x32_agpr(acc4& c, const bf16x8& a, con
 // spills them where the registers are few.
 __device__ __forceinline__ void pin_acc(acc4& c) { asm volatile("" : "+a"(c)); }
 
+// Element r of an accumulator in a vector register, read where this stands: left to itself the compiler reads all of
+// them at an epilogue's head and spills.
+__device__ __forceinline__ float read_acc(const acc4& c, int r) {
+  float x;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(c[r]));
+  return x;
+}
+
 // The compiler does not see the matrix instructions above, so it cannot count the wait states
 // between the last of them and the first read of an accumulator: spend them here.
 __device__ __forceinline__ void settle_acc() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }

@@ -133,7 +133,7 @@ __device__ __forceinline__ void rows_spread4(float x, float (&o)[4]) {
 // and 3) share: its maximum and its sums go through LDS, in the order in which one wavefront of a whole tile adds
 // them up (a lane adds the first four and the last four 16-row blocks apart), so that the results do not depend on
 // how a tile was computed. MASKED: some rows of the tile lie beyond the vocabulary; they are excluded by predicate —
-// their accumulators hold finite values.  STASH: also store every 2^(y - M) for the backward (`stash_wave`: the 32 KB
+// their accumulators hold finite values.  STASH: also store every 2^(y - M) for the backward (`kept_wave`: the 32 KB
 // of the part and these tokens, already offset by the lane).
 //
 // Bound by the issue of vector instructions, one wavefront to a SIMD and the matrix pipes idle: five per logit (maximum
@@ -141,23 +141,34 @@ __device__ __forceinline__ void rows_spread4(float x, float (&o)[4]) {
 // long.  The exponentials of a block run between the sums of the block before it, so that none of its users waits for
 // one, and the reductions over lanes are done for four columns at a time: 1600 instructions where there were 2030 and 330
 // wait states.  8192 x 896 x 151936 forward 1866 -> 1818 us, 187 tokens 88.8 -> 85.5 (one card each).
-template <bool MASKED, bool SOFTCAP, bool STASH, int BM>
+template <bool MASKED, bool SOFTCAP, Keep KEEP, int BM>
 __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams& p, const LanePos& lp,
-                                             const TilePos& t, int part, uint4* stash_wave, float* lds) {
+                                             const TilePos& t, int part, uint4* kept_wave, float* lds) {
+  constexpr bool STASH = KEEP == kKeepStash;
   constexpr bool kHalf = BM < kBlocks;
   constexpr int kRun = kBlocks / 2;  // blocks that a lane adds up in one go
   constexpr int kGroups = kBlocks / 4;
   auto add = [](float a, float b) { return a + b; };
   auto row_ok = [&](int i, int r) { return !MASKED || t.m0 + lp.m<BM>(i, r) < p.vocab; };
-  // columns 4 g .. 4 g + 3 leave the accumulators; SOFTCAP: through cap * tanh(. / cap)
+  // logits for the backward: written once, read once, long after: past the caches
+  auto keep_logits = [&](int i, int j, const float (&z)[4]) {
+    const acc4 v = {z[0], z[1], z[2], z[3]};
+    __builtin_nontemporal_store(v, reinterpret_cast<acc4*>(kept_wave + (j * kBlocks + (kHalf ? lp.wm * BM + i : i)) * 64));
+  };
+  // columns 4 g .. 4 g + 3, read from the accumulators where they are needed (SOFTCAP: through cap * tanh(. / cap))
+  float x[kHalf ? kGroups : 1][BM][4][4];
   auto take = [&](int g) {
 #pragma unroll
     for (int i = 0; i < BM; ++i)
 #pragma unroll
-      for (int j = 4 * g; j < 4 * g + 4; ++j) {
-        if (SOFTCAP) {
+      for (int q = 0; q < 4; ++q) {
+        float(&z)[4] = x[kHalf ? g : 0][i][q];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][r] = p.cap * fast_tanh(acc[i][j][r] * p.inv_cap);
+        for (int r = 0; r < 4; ++r) z[r] = read_acc(acc[i][4 * g + q], r);
+        if (SOFTCAP) {
+          if (KEEP == kKeepLogits) keep_logits(i, 4 * g + q, z);  // what is kept is not capped
+#pragma unroll
+          for (int r = 0; r < 4; ++r) z[r] = p.cap * fast_tanh(z[r] * p.inv_cap);
         }
       }
   };
@@ -170,7 +181,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) mx[q] = row_ok(i, r) ? fmaxf(mx[q], acc[i][4 * g + q][r]) : mx[q];
+        for (int r = 0; r < 4; ++r) mx[q] = row_ok(i, r) ? fmaxf(mx[q], x[kHalf ? g : 0][i][q][r]) : mx[q];
     return rows_reduce4(mx, [](float a, float b) { return fmaxf(a, b); });
   };
   // columns 4 g .. 4 g + 3 are 64 consecutive tokens, one per lane
@@ -213,13 +224,15 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
       float s[2] = {0.f, 0.f}, e[2] = {0.f, 0.f};
       uint32_t hw[BM][2];
       float y[3][4], w[2][4];  // blocks i + 1, i, i - 1; i, i - 1
-      auto rel = [&](int i, int r) { return fmaf(acc[i][j][r], p.c, -M[q]); };  // scaled logit relative to the max, <= 0
+      auto rel = [&](int i, int r) { return fmaf(x[kHalf ? g : 0][i][q][r], p.c, -M[q]); };  // scaled logit relative to the max, <= 0
 #pragma unroll
       for (int r = 0; r < 4; ++r) y[0][r] = rel(0, r);
 #pragma unroll
       for (int i = 0; i <= BM; ++i) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+          // one store under the arithmetic of a block: all of them at the epilogue's head make it wait for their way out
+          if (KEEP == kKeepLogits && !SOFTCAP && i < BM && r == 0) keep_logits(i, j, x[kHalf ? g : 0][i][q]);
           if (i < BM) w[i % 2][r] = row_ok(i, r) ? fast_exp2(y[i % 3][r]) : 0.f;
           if (i > 0) {
             const int b = i - 1;
@@ -241,7 +254,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
           typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
           const u32x4 x = {hw[2 * ip][0], hw[2 * ip][1], hw[2 * ip + 1][0], hw[2 * ip + 1][1]};
           const int at = kHalf ? lp.wm * (BM / 2) + ip : ip;
-          __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(stash_wave + (j * 4 + at) * 64));
+          __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(kept_wave + (j * 4 + at) * 64));
         }
       }
       s4[q] = kHalf ? s[0] : s[0] + s[1];
@@ -281,22 +294,13 @@ __device__ __forceinline__ void fwd_tile(const GemmOperands& g, const FwdParams&
   const LanePos lp;
   const int wm = kHalf ? half : lp.wm;  // the 128-row part of the tile, and with it the place of what is kept
   const int64_t kept = (int64_t)tile * 4 + wm * 2 + lp.wn;
-  if (KEEP == kKeepLogits) {  // written once, read once by the backward, long after: past the caches
-    float4* const out = reinterpret_cast<float4*>(p.stash) + kept * kLogitsWaveVecs + lp.lane;
-#pragma unroll
-    for (int j = 0; j < kBlocks; ++j)
-#pragma unroll
-      for (int i = 0; i < BM; ++i)
-        __builtin_nontemporal_store(
-            acc[i][j], reinterpret_cast<acc4*>(out + (j * kBlocks + (kHalf ? lp.wm * BM + i : i)) * 64));
-  }
-  constexpr bool STASH = KEEP == kKeepStash;
-  uint4* const stash_wave = STASH ? p.stash + kept * kStashWaveVecs + lp.lane : nullptr;
+  uint4* const kept_wave =
+      KEEP == kKeepNone ? nullptr : p.stash + kept * (KEEP == kKeepStash ? kStashWaveVecs : kLogitsWaveVecs) + lp.lane;
   float* const lds = reinterpret_cast<float*>(smem);
   if (t.m0 + 2 * BM * kBlk > p.vocab)
-    fwd_epilogue<true, SOFTCAP, STASH, BM>(acc, p, lp, t, part0 + wm, stash_wave, lds);
+    fwd_epilogue<true, SOFTCAP, KEEP, BM>(acc, p, lp, t, part0 + wm, kept_wave, lds);
   else
-    fwd_epilogue<false, SOFTCAP, STASH, BM>(acc, p, lp, t, part0 + wm, stash_wave, lds);
+    fwd_epilogue<false, SOFTCAP, KEEP, BM>(acc, p, lp, t, part0 + wm, kept_wave, lds);
 }
 
 template <class Loop, bool SOFTCAP, Keep KEEP>
