@@ -91,16 +91,16 @@ struct LanePos {
   __device__ __forceinline__ int n(int j) const { return wn * kWaveTile + j * kBlk + l16; }
 };
 
-template <int BM>
-using AccTileOf = acc4[BM][kBlocks];
+template <int BM, int BN = kBlocks>
+using AccTileOf = acc4[BM][BN];
 typedef AccTileOf<kBlocks> AccTile;
 
-template <int BM>
-__device__ __forceinline__ void zero_acc(AccTileOf<BM>& acc) {
+template <int BM, int BN = kBlocks>
+__device__ __forceinline__ void zero_acc(AccTileOf<BM, BN>& acc) {
 #pragma unroll
   for (int i = 0; i < BM; ++i)
 #pragma unroll
-    for (int j = 0; j < kBlocks; ++j)
+    for (int j = 0; j < BN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 }
@@ -255,10 +255,14 @@ struct DmaSide {
 // matrix instructions per k-tile) with the same slots and the same DMA instructions, of which those for the other
 // rows fetch nothing on a K-contiguous side (the descriptor ends): for the last tile of an m that fills at most half
 // of it, and for the tail of a walk whose tiles are halved to spread them over the compute units.
-template <bool kAT, bool kBT, bool kNarrow = false, int BM = kBlocks>
+// BN: block columns per wave, the same on the other side: 8, 6 or 4, a tile of 256, 192 or 128 columns for a call that
+// has no more (both sides K-contiguous).
+template <bool kAT, bool kBT, bool kNarrow = false, int BM = kBlocks, int BN = kBlocks>
 struct DmaLoopT {
   static_assert(BM == kBlocks || BM == kBlocks / 2, "");
-  typedef DmaLoopT<kAT, kBT, kNarrow, kBlocks / 2> Half;
+  static_assert(BN == kBlocks || ((BN == 6 || BN == 4) && !kAT && !kBT), "");
+  typedef DmaLoopT<kAT, kBT, kNarrow, kBlocks / 2, BN> Half;
+  static constexpr int kBN = BN;
   typedef std::conditional_t<kAT != kBT && !kNarrow, Half, void> HalfEdge;  // for the forms of the output products
   static constexpr int kRows = 2 * BM * kBlk;  // tile rows computed
   static constexpr int kBK = 64;
@@ -313,38 +317,47 @@ struct DmaLoopT {
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   }
 
-  __device__ static __forceinline__ void run(const GemmOperands& g, const TilePos& t, AccTileOf<BM>& acc,
+  __device__ static __forceinline__ void run(const GemmOperands& g, const TilePos& t, AccTileOf<BM, BN>& acc,
                                              char* smem) {
     const LanePos lp;
     DmaSide<kAT, BM> sa;
-    DmaSide<kBT> sb;
+    DmaSide<kBT, BN> sb;
     sa.init(g.a, g.lda, BM < kBlocks ? min(g.m_rows, t.m0 + kRows) : g.m_rows, g.k, t.m0, lp.wm, lp, 0);
     sb.init(g.b, g.ldb, g.n_rows, g.k, t.n0, lp.wn, lp, kBBase);
     // wave-uniform, so the LDS destination of every DMA instruction is scalar arithmetic into M0
     char* const dst = smem + __builtin_amdgcn_readfirstlane(lp.wave) * 8192;
 
-    zero_acc<BM>(acc);
+    zero_acc<BM, BN>(acc);
     // fragments of two k-steps: whole (one 16-byte read) or as the two halves of a transpose read
-    bf16x8 af[2][BM], bf[2][kBlocks];
-    i16x4 aft[2][BM][2], bft[2][kBlocks][2];
+    bf16x8 af[2][BM], bf[2][BN];
+    i16x4 aft[2][BM][2], bft[2][BN][2];
     const int kt_n = (g.k + kBK - 1) / kBK;
     auto dma_a = [&](int slot_off, const __amdgpu_buffer_rsrc_t& r, int j) {
       dma_kb(r, sa.vo[DmaSide<kAT, BM>::variant(j)], sa.step, dst + slot_off, j);
     };
     auto dma_b = [&](int slot_off, const __amdgpu_buffer_rsrc_t& r, int j) {
-      dma_kb(r, sb.vo[DmaSide<kBT>::variant(j)], sb.step, dst + kBBase + slot_off, j);
+      dma_kb(r, sb.vo[DmaSide<kBT, BN>::variant(j)], sb.step, dst + kBBase + slot_off, j);
     };
     // LDS addresses of the fragments in the slots being read: slot + per-lane offset, formed well before the
     // reads that use them (a vector addition right before the read that needs its result delays the MFMA
     // behind the pair; sixteen such pairs per k-tile cost 3-4 % of the loop).  The reads under a tile's second
     // k-step (k-step 0 of the next tile) and under the next tile's first k-step (its k-step 1) go to the same
     // slots, so the addresses change once per k-tile: after the last read of a tile's first k-step.
-    constexpr int kAddrA = DmaSide<kAT, BM>::kFrag, kAddrB = DmaSide<kBT>::kFrag;
+    constexpr int kAddrA = DmaSide<kAT, BM>::kFrag, kAddrB = DmaSide<kBT, BN>::kFrag;
     // The schedule of a k-step: its MFMAs, one DMA instruction every kDmaGap of them, the fragment reads one per two
-    // MFMAs (BM 4: in every MFMA gap without a DMA instruction), then the address additions, kAdrPer to a gap.
-    constexpr bool kWhole = BM == kBlocks;
-    constexpr int kMfmas = BM * kBlocks, kDmaGap = kMfmas / 8, kReads = BM * kReadsA + kBlocks * kReadsB;
-    constexpr int kFirstAdr = kWhole ? 2 * kReads : (4 * kReads + 2) / 3, kAdrPer = kWhole ? 1 : 2;
+    // MFMAs (32 MFMAs and fewer: in every MFMA gap without a DMA instruction), then the address additions, kAdrPer to a
+    // gap.
+    constexpr int kMfmas = BM * BN, kDmaGap = kMfmas / 8, kReads = BM * kReadsA + BN * kReadsB;
+    constexpr bool kRoomy = kMfmas >= 48;
+    constexpr int kDmaAt = kRoomy ? 3 : kMfmas == 16 ? 0 : 1;
+    constexpr int kRdPer = kMfmas == 16 ? 2 : 1;  // reads to a gap
+    constexpr int kFirstAdr = kRoomy ? 2 * kReads : kMfmas == 32 ? (4 * kReads + 2) / 3 : kMfmas == 24 ? (3 * kReads + 1) / 2 : kReads;
+    constexpr int kAdrPer = kRoomy ? 1 : 2;
+    // where the scalar bookkeeping goes (`mid` below)
+    constexpr int kMid0 = kMfmas == 64 ? 37 : kMfmas == 48 ? 35 : kMfmas == 32 ? 18 : kMfmas == 24 ? 17 : 10;
+    constexpr int kMid1 = kMfmas == 24 ? 18 : kMfmas == 16 ? 11 : kMid0 + 2;
+    constexpr int kMid2 = kMfmas == 48 ? 40 : kMfmas == 24 ? 20 : kMfmas == 16 ? 13 : kMid0 + 4;
+    constexpr int kMid3 = kMfmas == 64 ? 61 : kMfmas >= 32 ? kMfmas - 2 : kMfmas - 1;
     // room for the additions behind the reads of a k-step (not with both operands K-major, whose reads fill it:
     // that form, which no kernel of the library uses, forms them in one piece after the barrier)
     constexpr bool kLateAdr = kFirstAdr + (kAddrA + kAddrB + kAdrPer - 1) / kAdrPer <= kMfmas;
@@ -381,27 +394,30 @@ struct DmaLoopT {
 #pragma unroll
       for (int i = 0; i < BM; ++i) {
 #pragma unroll
-        for (int j = 0; j < kBlocks; ++j) {
-          const int m = i * kBlocks + j;
+        for (int j = 0; j < BN; ++j) {
+          const int m = i * BN + j;
           // scalar bookkeeping for the coming k-tile, in pieces of at most four instructions, in slots without
           // other work (a wavefront issues in order: a dozen scalar instructions in one MFMA gap hold up the
           // MFMA behind them); pieces 3 and 4 come behind the step's last DMA instruction
-          if (m == (kWhole ? 37 : 18)) mid(std::integral_constant<int, 0>{});
-          if (m == (kWhole ? 39 : 20)) mid(std::integral_constant<int, 1>{});
-          if (m == (kWhole ? 41 : 22)) mid(std::integral_constant<int, 2>{});
-          if (m == kMfmas - (kWhole ? 3 : 2)) mid(std::integral_constant<int, 3>{});
+          if (m == kMid0) mid(std::integral_constant<int, 0>{});
+          if (m == kMid1) mid(std::integral_constant<int, 1>{});
+          if (m == kMid2) mid(std::integral_constant<int, 2>{});
+          if (m == kMid3) mid(std::integral_constant<int, 3>{});
           if (m == kMfmas - 1) mid(std::integral_constant<int, 4>{});
-          const bool dma_slot = (m % kDmaGap) == (kWhole ? 3 : 1);
+          const bool dma_slot = (m % kDmaGap) == kDmaAt;
           if (dma_slot) {
             if (NB) dma_b(b_slot, rsrc, m / kDmaGap);
             if (NA) dma_a(a_slot, rsrc, m / kDmaGap);
           }
-          if (kWhole ? (m & 1) == 0 : !dma_slot) {
-            const int s = kWhole ? m >> 1 : m - ((m + 2) >> 2);
-            if (s < RA) read_a(rd_kk, rd_set, 0, s);
-            else if (s < RA + kBlocks * RB) read_b(rd_kk, rd_set, (s - RA) / RB, (s - RA) % RB);
-            else if (s < kReads)
-              read_a(rd_kk, rd_set, 1 + (s - RA - kBlocks * RB) / RA, (s - RA - kBlocks * RB) % RA);
+          if (kRoomy ? (m & 1) == 0 : !dma_slot) {
+            const int gap = kRoomy ? m >> 1 : m - (m + kDmaGap - 1 - kDmaAt) / kDmaGap;
+#pragma unroll
+            for (int s = gap * kRdPer; s < (gap + 1) * kRdPer; ++s) {
+              if (s < RA) read_a(rd_kk, rd_set, 0, s);
+              else if (s < RA + BN * RB) read_b(rd_kk, rd_set, (s - RA) / RB, (s - RA) % RB);
+              else if (s < kReads)
+                read_a(rd_kk, rd_set, 1 + (s - RA - BN * RB) / RA, (s - RA - BN * RB) % RA);
+            }
           }
 #pragma unroll
           for (int q = (m - kFirstAdr) * kAdrPer; q < (m - kFirstAdr + 1) * kAdrPer; ++q) {
@@ -444,7 +460,8 @@ struct DmaLoopT {
       for (int h = 0; h < kReadsA; ++h)
         if (i < BM) read_a(0, 0, i, h);
 #pragma unroll
-      for (int h = 0; h < kReadsB; ++h) read_b(0, 0, i, h);
+      for (int h = 0; h < kReadsB; ++h)
+        if (i < BN) read_b(0, 0, i, h);
     }
     __builtin_amdgcn_sched_barrier(0);
     wait_lds_reads();
@@ -520,6 +537,7 @@ struct RegLoop {
   static constexpr int kBK = BK;
   static constexpr bool kAMajor = false, kBMajor = false;
   typedef void Half, HalfEdge;  // whole tiles only
+  static constexpr int kBN = kBlocks;
   static constexpr int kChunks = BK / 8;                 // 16-byte chunks per row
   static constexpr int kRowBytes = BK * 2;
   static constexpr int kRowsPerLine = 256 / kRowBytes;   // rows per 256-byte bank line

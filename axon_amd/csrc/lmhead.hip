@@ -133,27 +133,35 @@ __device__ __forceinline__ void rows_spread4(float x, float (&o)[4]) {
 // and 3) share: its maximum and its sums go through LDS, in the order in which one wavefront of a whole tile adds
 // them up (a lane adds the first four and the last four 16-row blocks apart), so that the results do not depend on
 // how a tile was computed. MASKED: some rows of the tile lie beyond the vocabulary; they are excluded by predicate —
-// their accumulators hold finite values.  STASH: also store every 2^(y - M) for the backward (`kept_wave`: the 32 KB
-// of the part and these tokens, already offset by the lane).
+// their accumulators hold finite values.  STASH: also store every 2^(y - M) for the backward (`kept_tile`: the part's
+// share of the tile, its two sub-tiles one behind the other, already offset by the lane).  BN: columns of 16 tokens per
+// wavefront, fewer than 8 where the call has no more (narrow tiles).
 //
 // Bound by the issue of vector instructions, one wavefront to a SIMD and the matrix pipes idle: five per logit (maximum
 // for two, read of the accumulator, fma, exponential, sum, product sum), of which the exponential takes four times as
 // long.  The exponentials of a block run between the sums of the block before it, so that none of its users waits for
 // one, and the reductions over lanes are done for four columns at a time: 1600 instructions where there were 2030 and 330
 // wait states.  8192 x 896 x 151936 forward 1866 -> 1818 us, 187 tokens 88.8 -> 85.5 (one card each).
-template <bool MASKED, bool SOFTCAP, Keep KEEP, int BM>
-__device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams& p, const LanePos& lp,
-                                             const TilePos& t, int part, uint4* kept_wave, float* lds) {
+template <bool MASKED, bool SOFTCAP, Keep KEEP, int BM, int BN>
+__device__ __forceinline__ void fwd_epilogue(AccTileOf<BM, BN>& acc, const FwdParams& p, const LanePos& lp,
+                                             const TilePos& t, int part, uint4* kept_tile, float* lds) {
   constexpr bool STASH = KEEP == kKeepStash;
   constexpr bool kHalf = BM < kBlocks;
   constexpr int kRun = kBlocks / 2;  // blocks that a lane adds up in one go
-  constexpr int kGroups = kBlocks / 4;
+  constexpr int kGroups = (BN + 3) / 4;
+  auto cols = [](int g) { return BN - 4 * g < 4 ? BN - 4 * g : 4; };  // of group g
   auto add = [](float a, float b) { return a + b; };
   auto row_ok = [&](int i, int r) { return !MASKED || t.m0 + lp.m<BM>(i, r) < p.vocab; };
+  // where column j of this wavefront is kept: the sub-tiles there are those of the whole tile, 128 columns each
+  auto kept_col = [&](int j) {
+    constexpr int kCol = (STASH ? kStashWaveVecs : kLogitsWaveVecs) / kBlocks;
+    const int at = BN == kBlocks ? j : lp.wn * BN + j;
+    return kept_tile + (int64_t)((BN == kBlocks ? lp.wn * kBlocks : 0) + at) * kCol;
+  };
   // logits for the backward: written once, read once, long after: past the caches
   auto keep_logits = [&](int i, int j, const float (&z)[4]) {
     const acc4 v = {z[0], z[1], z[2], z[3]};
-    __builtin_nontemporal_store(v, reinterpret_cast<acc4*>(kept_wave + (j * kBlocks + (kHalf ? lp.wm * BM + i : i)) * 64));
+    __builtin_nontemporal_store(v, reinterpret_cast<acc4*>(kept_col(j) + (kHalf ? lp.wm * BM + i : i) * 64));
   };
   // columns 4 g .. 4 g + 3, read from the accumulators where they are needed (SOFTCAP: through cap * tanh(. / cap))
   float x[kHalf ? kGroups : 1][BM][4][4];
@@ -162,6 +170,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
     for (int i = 0; i < BM; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
+        if (q >= cols(g)) continue;
         float(&z)[4] = x[kHalf ? g : 0][i][q];
 #pragma unroll
         for (int r = 0; r < 4; ++r) z[r] = read_acc(acc[i][4 * g + q], r);
@@ -181,14 +190,15 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) mx[q] = row_ok(i, r) ? fmaxf(mx[q], x[kHalf ? g : 0][i][q][r]) : mx[q];
+        for (int r = 0; r < 4; ++r)
+          if (q < cols(g)) mx[q] = row_ok(i, r) ? fmaxf(mx[q], x[kHalf ? g : 0][i][q][r]) : mx[q];
     return rows_reduce4(mx, [](float a, float b) { return fmaxf(a, b); });
   };
-  // columns 4 g .. 4 g + 3 are 64 consecutive tokens, one per lane
+  // columns 4 g .. 4 g + 3 are 64 consecutive tokens, one per lane (the last group of six columns has 32)
   auto write = [&](int g, float M, const float (&s)[4], const float (&e)[4]) {
     const float sum = rows_reduce4(s, add), prod = rows_reduce4(e, add);
-    const int n = t.n0 + lp.wn * kWaveTile + g * 64 + lp.lane;
-    if (n < p.n_tokens) {
+    const int n = t.n0 + lp.wn * BN * kBlk + g * 64 + lp.lane;
+    if (n < p.n_tokens && (cols(g) == 4 || lp.lane < cols(g) * kBlk)) {
       const int64_t at = (int64_t)part * p.n_tokens + n;
       float* const o = p.stats + at * 3;
       o[0] = M;
@@ -216,10 +226,11 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
     if (!kHalf) take(g);
     const float mx = kHalf ? mxs[g] : max_of(g);
     mxs[g] = (MASKED && mx == -INFINITY) ? kEmptyMax : mx * p.c;
-    float M[4], s4[4], e4[4];
+    float M[4], s4[4] = {}, e4[4] = {};
     rows_spread4(mxs[g], M);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
+      if (q >= cols(g)) continue;
       const int j = 4 * g + q;
       float s[2] = {0.f, 0.f}, e[2] = {0.f, 0.f};
       uint32_t hw[BM][2];
@@ -232,6 +243,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           // one store under the arithmetic of a block: all of them at the epilogue's head make it wait for their way out
+          // (GSPO step of 6007 x 896 x 151936 5443 -> 5362 us)
           if (KEEP == kKeepLogits && !SOFTCAP && i < BM && r == 0) keep_logits(i, j, x[kHalf ? g : 0][i][q]);
           if (i < BM) w[i % 2][r] = row_ok(i, r) ? fast_exp2(y[i % 3][r]) : 0.f;
           if (i > 0) {
@@ -254,7 +266,7 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
           typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
           const u32x4 x = {hw[2 * ip][0], hw[2 * ip][1], hw[2 * ip + 1][0], hw[2 * ip + 1][1]};
           const int at = kHalf ? lp.wm * (BM / 2) + ip : ip;
-          __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(kept_wave + (j * 4 + at) * 64));
+          __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(kept_col(j) + at * 64));
         }
       }
       s4[q] = kHalf ? s[0] : s[0] + s[1];
@@ -271,9 +283,10 @@ __device__ __forceinline__ void fwd_epilogue(AccTileOf<BM>& acc, const FwdParams
     if (lp.wm == 0) {
 #pragma unroll
       for (int g = 0; g < kGroups; ++g) {
-        float s4[4], e4[4];
+        float s4[4] = {}, e4[4] = {};
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
+          if (q >= cols(g)) continue;
           s4[q] = mine[(4 * g + q) * 64] + other[(4 * g + q) * 64];
           e4[q] = mine[(kBlocks + 4 * g + q) * 64] + other[(kBlocks + 4 * g + q) * 64];
         }
@@ -289,18 +302,19 @@ template <class Loop, int BM, bool SOFTCAP, Keep KEEP>
 __device__ __forceinline__ void fwd_tile(const GemmOperands& g, const FwdParams& p, const TilePos& t, int tile, int part0,
                                          int half, char* smem) {
   constexpr bool kHalf = BM < kBlocks;
-  AccTileOf<BM> acc;
+  constexpr int BN = Loop::kBN;
+  AccTileOf<BM, BN> acc;
   Loop::run(g, t, acc, smem);
   const LanePos lp;
   const int wm = kHalf ? half : lp.wm;  // the 128-row part of the tile, and with it the place of what is kept
-  const int64_t kept = (int64_t)tile * 4 + wm * 2 + lp.wn;
-  uint4* const kept_wave =
-      KEEP == kKeepNone ? nullptr : p.stash + kept * (KEEP == kKeepStash ? kStashWaveVecs : kLogitsWaveVecs) + lp.lane;
+  uint4* const kept_tile = KEEP == kKeepNone ? nullptr
+                                             : p.stash + ((int64_t)tile * 4 + wm * 2) *
+                                                             (KEEP == kKeepStash ? kStashWaveVecs : kLogitsWaveVecs) + lp.lane;
   float* const lds = reinterpret_cast<float*>(smem);
   if (t.m0 + 2 * BM * kBlk > p.vocab)
-    fwd_epilogue<true, SOFTCAP, KEEP, BM>(acc, p, lp, t, part0 + wm, kept_wave, lds);
+    fwd_epilogue<true, SOFTCAP, KEEP, BM, BN>(acc, p, lp, t, part0 + wm, kept_tile, lds);
   else
-    fwd_epilogue<false, SOFTCAP, KEEP, BM>(acc, p, lp, t, part0 + wm, kept_wave, lds);
+    fwd_epilogue<false, SOFTCAP, KEEP, BM, BN>(acc, p, lp, t, part0 + wm, kept_tile, lds);
 }
 
 template <class Loop, bool SOFTCAP, Keep KEEP>
@@ -1616,6 +1630,30 @@ int halved_tiles(int64_t n, int64_t v) {
   return rest <= kCus / 2 && tiles < kHalvedRounds * kCus ? (int)rest : 0;
 }
 
+// A call of few tokens has one column of tiles; up to 192 of them it is computed in tiles of 192 or 128 tokens, whose
+// products and statistics take three quarters or half of the time: what is left is reading the weight.  Forward with
+// 256 / these, us: hidden 896 x 151936 64 tokens 75 / 68, 128 79 / 68, 129 79.5 / 72.7, 192 87 / 81; 2880 x 201088 64
+// tokens 243 / 233, 128 250 / 236, 129 249 / 242, 192 262 / 253; 4096 x 151936 128 259 / 245, 192 275 / 270; 2048 x 32768
+// 128 35.2 / 33.7, 192 37.2 / 35.5; 1024 x 50257 the same within what runs differ.
+int narrow_columns(int64_t n) { return n <= 128 ? 4 : n <= 192 ? 6 : kBlocks; }
+
+template <bool SOFTCAP, Keep KEEP, int BN>
+__global__ __launch_bounds__(kGemmThreads) void lmhead_fwd_narrow_kernel(GemmOperands g, FwdParams p, int tiles_m,
+                                                                         int tiles_n) {
+  fwd_body<DmaLoopT<false, false, false, kBlocks, BN>, SOFTCAP, KEEP>(g, p, tiles_m, tiles_n);
+}
+
+template <bool SOFTCAP, Keep KEEP>
+int launch_fwd_narrow(const GemmOperands& g, const FwdParams& p, hipStream_t st) {
+  auto* const kernel = narrow_columns(g.n_rows) == 4 ? lmhead_fwd_narrow_kernel<SOFTCAP, KEEP, 4>
+                                                     : lmhead_fwd_narrow_kernel<SOFTCAP, KEEP, 6>;
+  const int tiles_m = (g.m_rows + kTile - 1) / kTile;
+  if (set_lds(kernel) != AXON_OK) return AXON_ERR_LAUNCH;
+  hipLaunchKernelGGL(kernel, dim3(tiles_m + p.halved), dim3(kGemmThreads), kGemmLdsBytes, st, g, p, tiles_m, 1);
+  AXON_CHECK_LAUNCH();
+  return AXON_OK;
+}
+
 template <bool SOFTCAP>
 int launch_fwd_logits(const GemmOperands& g, const FwdParams& p, hipStream_t st) {
   const int tiles_m = (g.m_rows + kTile - 1) / kTile, tiles_n = (g.n_rows + kTile - 1) / kTile;
@@ -1671,6 +1709,12 @@ int fwd_impl(const void* hidden, const void* weight, const void* labels, int lab
     Span span(timer, 0);
     if (stash && keep == kKeepLogits) {
       rc = softcap > 0.f ? launch_fwd_logits<true>(g, p, st) : launch_fwd_logits<false>(g, p, st);
+      if (rc != AXON_OK) return rc;
+    } else if (dma_ok(g) && narrow_columns(n) < kBlocks) {
+      rc = stash ? softcap > 0.f ? launch_fwd_narrow<true, kKeepStash>(g, p, st)
+                                 : launch_fwd_narrow<false, kKeepStash>(g, p, st)
+                 : softcap > 0.f ? launch_fwd_narrow<true, kKeepNone>(g, p, st)
+                                 : launch_fwd_narrow<false, kKeepNone>(g, p, st);
       if (rc != AXON_OK) return rc;
     } else if (stash) {
       if (softcap > 0.f)

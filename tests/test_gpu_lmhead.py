@@ -1001,6 +1001,29 @@ def test_rows_of_an_edge_tile_beyond_the_operand_are_zeros_in_the_accumulators()
     assert rel_l2(hb.d_weight, ref_dw) < 2e-2 and rel_l2(hb.d_hidden, ref_dh) < 2e-2
 
 
+@pytest.mark.parametrize("h,v,cap", [(64, 2000, 0.0), (192, 99 * 256 + 129, 0.0), (448, 99 * 256 + 1, 5.0)])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 96, 97, 127, 128, 129, 159, 160, 191, 192, 193])
+def test_forward_in_narrow_tiles_gives_the_bits_of_wide_ones(n, h, v, cap):
+    """Up to 128 and up to 192 tokens the forward's tiles are 128 and 192 tokens wide: the results are the bits of the same
+    tokens in a call of 512, in whole tiles and in halves, and the stash gives the recompute's gradients to its rounding."""
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(512, h, v, seed=h))
+    w = (w.float() * 6).bfloat16()
+    few, many = (_ops.lmhead_forward(hid[:k], w, lab[:k], 1.0 / 0.7, softcap=cap) for k in (n, 512))
+    for a, b in zip(few, many):
+        assert torch.equal(a, b[:n]) and torch.isfinite(a).all()
+    g_lp, g_en = torch.randn(2, n + 4, generator=torch.Generator().manual_seed(v)).to(DEV)
+
+    def run(**keep):
+        hb = _ops.HeadBlocks(hid[:n], w, lab[:n], 1.0 / 0.7, [(0, n)], softcap=cap, **keep)
+        hb.forward(0)
+        hb.backward(0, g_lp, g_en)
+        return hb.logprobs, hb.entropy, hb.d_hidden, hb.d_weight
+
+    (lp, ent, dh, dw), again = run(stash=True), run(stash=False)
+    assert torch.equal(lp, again[0]) and torch.equal(ent, again[1])
+    assert rel_l2(dh, again[2]) < 5e-3 and rel_l2(dw, again[3]) < 5e-3
+
+
 @pytest.mark.parametrize("n,h,v,chunk,cap,lens", [
     (257, 64, 256, 0, 0.0, None),              # one row into a second token tile, one vocabulary tile
     (301, 128, 1999, 0, 0.0, None),            # ragged on both sides
