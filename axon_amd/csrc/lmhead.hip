@@ -590,6 +590,20 @@ __device__ __forceinline__ int stage_off(int nw, int unit) {
   return nw * 256 + ((pu ^ ((nw & 31) ^ (nw >> 5))) << 3);
 }
 
+// The same where the row's lane part and the unit's are apart: accumulator block (i, j) of a wavefront (row 16 j + l16,
+// unit 4 i + lq), and the row 16 j + 2 u + lane / 32 that half a wavefront reads (unit lane % 32).  Per lane, then
+// constants: an exclusive or and an offset per access, where the compiler spent four instructions.
+__device__ __forceinline__ int stage_block_base(const LanePos& lp) {
+  return lp.l16 * 256 + (((((lp.lq & 1) << 4) | ((lp.lq & 2) << 2)) ^ lp.l16) << 3);
+}
+__device__ __forceinline__ int stage_block(int base, int i, int j) {
+  return (base ^ ((i ^ (j >> 1) ^ ((j & 1) << 4)) << 3)) + j * kBlk * 256;
+}
+__device__ __forceinline__ int stage_row_base(const LanePos& lp) { return stage_off(lp.lane >> 5, lp.lane & 31); }
+__device__ __forceinline__ int stage_row(int base, int j, int u) {
+  return (base ^ (((2 * u) ^ (j >> 1) ^ ((j & 1) << 4)) << 3)) + (j * kBlk + 2 * u) * 256;
+}
+
 // Per-token factors of dlogit = softmax * (ca + cb * logit) + onehot * gl for tile-relative token
 // row nr; lab_rel is the label's row inside the tile whose first vocabulary row is m0_abs (-1: not
 // in this tile).
@@ -620,7 +634,7 @@ struct TokenCoef {
 // The dlogit of one logit (the accumulator, before temperature and soft-capping), row mrel of the tile.  SOFTCAP:
 // the logit goes through cap * tanh(. / cap) and the gradient is multiplied by the derivative 1 - tanh^2
 // (fused_linear.py:80-83).
-template <bool SOFTCAP>
+template <bool SOFTCAP, bool LABEL = true>
 __device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef& k, const DlogitParams& p, float c) {
   float dcap = 1.f;
   if (SOFTCAP) {
@@ -630,7 +644,7 @@ __device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef&
   }
   const float pr = fast_exp2(fmaf(raw, c, -k.lse2));
   float v = pr * fmaf(k.cb, raw, k.ca);
-  if (mrel == k.lab_rel) v += k.gl;
+  if (LABEL && mrel == k.lab_rel) v += k.gl;
   if (SOFTCAP) v *= dcap;
   return v;
 }
@@ -640,7 +654,10 @@ __device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef&
 // written as zeros.  Sixteen tokens at a time, and all tokens' scalars requested before the first: the main loop ends for
 // all workgroups of the chip at about the same time, so that this is a burst of 33 MB of stores, which the arithmetic
 // of the next sixteen tokens now runs under (whole sub-tile first, then its copy: 6007 x 896 x 151936 1.98 ms for
-// 1.79, 3001 x 1024 x 50257 0.408 for 0.380, 8192 x 4096 x 151936 7.43 for 7.27).
+// 1.79, 3001 x 1024 x 50257 0.408 for 0.380, 8192 x 4096 x 151936 7.43 for 7.27).  Bound by the issue of vector
+// instructions: 1900 where no label is among the wavefront's logits, 3470 with the label's two per logit and the staging
+// addresses formed anew for each access (us, before / after: 6007 x 896 x 151936 1791 / 1686, 3001 x 2880 x 201088 2645 / 2583,
+// 2048 x 3072 x 128264 1206 / 1176, 333 x 896 x 151936 164 / 158).
 template <bool SOFTCAP, bool MASKED>
 __device__ __forceinline__ void dlogit_store(AccTile& acc, const DlogitParams& p, const LanePos& lp,
                                              const TilePos& t, char* stage) {
@@ -653,35 +670,43 @@ __device__ __forceinline__ void dlogit_store(AccTile& acc, const DlogitParams& p
   TokenCoef k[kBlocks];
 #pragma unroll
   for (int j = 0; j < kBlocks; ++j) k[j] = TokenCoef(p, n_wave + j * kBlk + lp.l16, (int64_t)p.v_begin + t.m0);
-#pragma unroll
-  for (int j = 0; j < kBlocks; ++j) {
-    const int nw = j * kBlk + lp.l16;  // token row inside the wave's sub-tile
-    const int m_end = MASKED ? (k[j].n_ok ? p.vocab - p.v_begin - t.m0 : 0) : kTile;  // rows that count
-#pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
-      float v[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int mrel = lp.m(i, r);
-        const float x = dlogit_of<SOFTCAP>(acc[i][j][r], mrel, k[j], p, c);
-        v[r] = (!MASKED || mrel < m_end) ? x : 0.f;
-      }
-      uint2 w;
-      w.x = pack_bf16(v[0], v[1]);
-      w.y = pack_bf16(v[2], v[3]);
-      *reinterpret_cast<uint2*>(stage + stage_off(nw, i * 4 + lp.lq)) = w;
-    }
-    // these sixteen tokens are complete: their rows leave while the next sixteen are computed
-    uint2 o[kBlocks];
-#pragma unroll
-    for (int u = 0; u < kBlocks; ++u)
-      o[u] = *reinterpret_cast<const uint2*>(stage + stage_off(j * kBlk + 2 * u + lhi, l32));
+  const int block = stage_block_base(lp), row = stage_row_base(lp);
+  uint2 o[kBlocks];  // sixteen complete tokens on their way from LDS to memory, under the arithmetic of the next sixteen
+  auto put = [&]() {
 #pragma unroll
     for (int u = 0; u < kBlocks; ++u) {
       *reinterpret_cast<uint2*>(d) = o[u];
       d += dstep;
     }
+  };
+#pragma unroll
+  for (int j = 0; j < kBlocks; ++j) {
+    const int m_end = MASKED ? (k[j].n_ok ? p.vocab - p.v_begin - t.m0 : 0) : kTile;  // rows that count
+    auto compute = [&](auto label) {
+#pragma unroll
+      for (int i = 0; i < kBlocks; ++i) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int mrel = lp.m(i, r);
+          const float x = dlogit_of<SOFTCAP, decltype(label)::value>(read_acc(acc[i][j], r), mrel, k[j], p, c);
+          v[r] = (!MASKED || mrel < m_end) ? x : 0.f;
+        }
+        uint2 w;
+        w.x = pack_bf16(v[0], v[1]);
+        w.y = pack_bf16(v[2], v[3]);
+        *reinterpret_cast<uint2*>(stage + stage_block(block, i, j)) = w;
+      }
+    };
+    // of sixteen tokens one in a hundred wavefronts holds a label: the others leave its two instructions per logit out
+    const unsigned at = (unsigned)(k[j].lab_rel - lp.wm * kWaveTile);
+    if (__builtin_amdgcn_ballot_w64(at < (unsigned)kWaveTile) != 0) compute(std::true_type{});
+    else compute(std::false_type{});
+    if (j > 0) put();
+#pragma unroll
+    for (int u = 0; u < kBlocks; ++u) o[u] = *reinterpret_cast<const uint2*>(stage + stage_row(row, j, u));
   }
+  put();
 }
 
 // The same from a forward's stash (see StashLayout above FwdParams): softmax = w * 2^(M - lse), scaled logit =
@@ -997,32 +1022,11 @@ __device__ __forceinline__ void store_tile(const GemmOperands& g, const StorePar
   AccTileOf<BM> acc;
   Loop::run(g, t, acc, smem);
   const LanePos lp;
-  if (p.tile_acc) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    f32x4* ta = reinterpret_cast<f32x4*>(p.tile_acc) +
-                (tile * 4 + (kHalf ? lp.wn : lp.wave)) * (kBlocks * kBlocks * 64) +
-                (kHalf ? lp.wm * BM * kBlocks * 64 : 0) + lp.lane;
-#pragma unroll
-    for (int i = 0; i < BM; ++i) {
-      f32x4 old[kBlocks];
-      if (p.accumulate) {
-#pragma unroll
-        for (int j = 0; j < kBlocks; ++j) old[j] = __builtin_nontemporal_load(ta + (i * kBlocks + j) * 64);
-      }
-#pragma unroll
-      for (int j = 0; j < kBlocks; ++j) {
-        if (p.accumulate) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][r] += old[j][r];
-        }
-        if (p.keep_f32) {
-          const f32x4 v = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-          __builtin_nontemporal_store(v, ta + (i * kBlocks + j) * 64);
-        }
-      }
-    }
-  }
-  if (p.out_f32) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  auto value = [&](int i, int j) {
+    return f32x4{read_acc(acc[i][j], 0), read_acc(acc[i][j], 1), read_acc(acc[i][j], 2), read_acc(acc[i][j], 3)};
+  };
+  if (p.out_f32) {  // the plain product
 #pragma unroll
     for (int j = 0; j < kBlocks; ++j) {
       const int n = t.n0 + lp.n(j);
@@ -1031,27 +1035,59 @@ __device__ __forceinline__ void store_tile(const GemmOperands& g, const StorePar
       for (int i = 0; i < BM; ++i) {
         const int m = t.m0 + lp.m<BM>(i, 0);
         if (m >= p.m_valid) continue;  // m_valid % 4 == 0: a quad is all in or all out
-        *reinterpret_cast<float4*>(p.out_f32 + (int64_t)n * p.ld_f32 + m) =
-            make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+        *reinterpret_cast<f32x4*>(p.out_f32 + (int64_t)n * p.ld_f32 + m) = value(i, j);
       }
     }
+    return;
   }
-  if (!p.out_bf16) return;
   // bf16 rows leave through the wavefront's own 32 KB of LDS, so that a store instruction writes four rows of 256
   // contiguous bytes (whole cache lines) instead of sixteen pieces of 32: the main loop has ended with a barrier, and
   // LDS operations of one wave complete in order.  Two half-waves' reads touch 32 distinct slots each (rows 16
   // apart, see stage_off).  dWeight of 700 tokens (11 k-tiles; 151936 x 4096 written) 979 us before, 832 with the
-  // staging, 809 with the non-temporal hint on top; long reductions do not notice.
+  // staging, 809 with the non-temporal hint on top; long reductions do not notice.  Accumulators are read on their way
+  // out (read_acc): read at the head and written back around the branches below they cost 600 instructions more
+  // (us, before / after: dHidden 1201 x 1024 x 50257 115 / 109.5, 1500 x 2048 x 32768 129 / 124, 6007 x 896 x 151936
+  // 1119 / 1107; dWeight 1201 x 1024 x 50257 133 / 127.5, 6007 x 896 x 151936 1148 / 1138).
   char* const stage = smem + lp.wave * 32768;
-#pragma unroll
-  for (int j = 0; j < kBlocks; ++j)
+  const int block = stage_block_base(lp);
+  auto to_stage = [&](int i, int j, const f32x4& v) {
+    uint2 w;
+    w.x = pack_bf16(v[0], v[1]);
+    w.y = pack_bf16(v[2], v[3]);
+    *reinterpret_cast<uint2*>(stage + stage_block(block, i, j)) = w;
+  };
+  if (p.tile_acc) {
+    f32x4* ta = reinterpret_cast<f32x4*>(p.tile_acc) +
+                (tile * 4 + (kHalf ? lp.wn : lp.wave)) * (kBlocks * kBlocks * 64) +
+                (kHalf ? lp.wm * BM * kBlocks * 64 : 0) + lp.lane;
 #pragma unroll
     for (int i = 0; i < BM; ++i) {
-      uint2 w;
-      w.x = pack_bf16(acc[i][j][0], acc[i][j][1]);
-      w.y = pack_bf16(acc[i][j][2], acc[i][j][3]);
-      *reinterpret_cast<uint2*>(stage + stage_off(j * kBlk + lp.l16, i * 4 + lp.lq)) = w;
+      f32x4 v[kBlocks];
+      if (p.accumulate) {
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) v[j] = __builtin_nontemporal_load(ta + (i * kBlocks + j) * 64);
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) v[j] = value(i, j) + v[j];
+      } else {
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) v[j] = value(i, j);
+      }
+      if (p.keep_f32) {
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) __builtin_nontemporal_store(v[j], ta + (i * kBlocks + j) * 64);
+      }
+      if (p.out_bf16) {
+#pragma unroll
+        for (int j = 0; j < kBlocks; ++j) to_stage(i, j, v[j]);
+      }
     }
+    if (!p.out_bf16) return;
+  } else {
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j)
+#pragma unroll
+      for (int i = 0; i < BM; ++i) to_stage(i, j, value(i, j));
+  }
   if (kHalf) {  // 64 values of m per wavefront: eight rows of 128 contiguous bytes per store instruction
     const int row0 = lp.lane >> 3, col = lp.lane & 7, m = t.m0 + lp.wm * BM * kBlk + col * 8;
     if (m >= p.m_valid) return;
