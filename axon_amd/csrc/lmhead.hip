@@ -649,6 +649,17 @@ __device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef&
   return v;
 }
 
+// f(true_type) where one of the lanes' sixteen tokens has its label among the wavefront's 128 vocabulary rows, one
+// wavefront in a hundred and more; else f(false_type), without the label's two instructions per logit.  Decode of a stash
+// or of kept logits, us, before / after: 300 x 896 x 151936 59.2 / 55.3, 1000 x 4096 x 151936 with an entropy gradient
+// 137.6 / 130.4, 333 x 2880 x 201088 102.3 / 97.5, 6007 x 896 x 151936 (memory-bound) 1056 / 1048.
+template <class F>
+__device__ __forceinline__ void with_label_or_not(const TokenCoef& k, const LanePos& lp, F&& f) {
+  const unsigned at = (unsigned)(k.lab_rel - lp.wm * kWaveTile);
+  if (__builtin_amdgcn_ballot_w64(at < (unsigned)kWaveTile) != 0) f(std::true_type{});
+  else f(std::false_type{});
+}
+
 // Accumulators -> bf16 dlogits, token-major to dl through the wave's staging area, where they stay for the
 // vocab-major copy.  MASKED: the tile reaches past the last token or the last vocabulary row; those entries are
 // written as zeros.  Sixteen tokens at a time, and all tokens' scalars requested before the first: the main loop ends for
@@ -698,10 +709,7 @@ __device__ __forceinline__ void dlogit_store(AccTile& acc, const DlogitParams& p
         *reinterpret_cast<uint2*>(stage + stage_block(block, i, j)) = w;
       }
     };
-    // of sixteen tokens one in a hundred wavefronts holds a label: the others leave its two instructions per logit out
-    const unsigned at = (unsigned)(k[j].lab_rel - lp.wm * kWaveTile);
-    if (__builtin_amdgcn_ballot_w64(at < (unsigned)kWaveTile) != 0) compute(std::true_type{});
-    else compute(std::false_type{});
+    with_label_or_not(k[j], lp, compute);
     if (j > 0) put();
 #pragma unroll
     for (int u = 0; u < kBlocks; ++u) o[u] = *reinterpret_cast<const uint2*>(stage + stage_row(row, j, u));
@@ -724,41 +732,42 @@ __device__ __forceinline__ void dlogit_stage_stash(const uint4 (&st)[4 * kStashH
                                                    const DlogitParams& p, const LanePos& lp,
                                                    const TilePos& t, char* stage) {
   const float inv_c = 1.f / (p.inv_temp * kLog2e);
+  const int block = stage_block_base(lp);
 #pragma unroll
   for (int jl = 0; jl < kStashHalfBlocks; ++jl) {
-    const int nw = jl * kBlk + lp.l16;
-    const int nr = lp.wn * kWaveTile + j0 * kBlk + nw;
-    const TokenCoef k(p, t.n0 + nr, (int64_t)p.v_begin + t.m0);
+    const TokenCoef k(p, t.n0 + lp.wn * kWaveTile + (j0 + jl) * kBlk + lp.l16, (int64_t)p.v_begin + t.m0);
     const float Mp = pm[(int64_t)part * p.n_tokens + k.nn];
     const float scale = fast_exp2(Mp - k.lse2);
     const bool n_counts = !EDGE || k.n_ok;
+    with_label_or_not(k, lp, [&](auto label) {
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
-      const uint4 q = st[jl * 4 + (i >> 1)];
-      float wv[4];
-      unpack_f16((i & 1) ? q.z : q.x, wv[0], wv[1]);
-      unpack_f16((i & 1) ? q.w : q.y, wv[2], wv[3]);
-      float d[4];
+      for (int i = 0; i < kBlocks; ++i) {
+        const uint4 q = st[jl * 4 + (i >> 1)];
+        float wv[4];
+        unpack_f16((i & 1) ? q.z : q.x, wv[0], wv[1]);
+        unpack_f16((i & 1) ? q.w : q.y, wv[2], wv[3]);
+        float d[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int mrel = lp.m(i, r);
-        const float pr = wv[r] * scale;
-        float raw = 0.f;
-        if (SOFTCAP || ENT) raw = (__builtin_amdgcn_logf(fmaxf(wv[r], 1e-30f)) + Mp) * inv_c;
-        float v = pr * (ENT ? fmaf(k.cb, raw, k.ca) : k.ca);
-        if (mrel == k.lab_rel) v += k.gl;
-        if (SOFTCAP) {
-          const float th = raw * p.inv_cap;
-          v *= fmaf(-th, th, 1.f);
+        for (int r = 0; r < 4; ++r) {
+          const int mrel = lp.m(i, r);
+          const float pr = wv[r] * scale;
+          float raw = 0.f;
+          if (SOFTCAP || ENT) raw = (__builtin_amdgcn_logf(fmaxf(wv[r], 1e-30f)) + Mp) * inv_c;
+          float v = pr * (ENT ? fmaf(k.cb, raw, k.ca) : k.ca);
+          if (decltype(label)::value && mrel == k.lab_rel) v += k.gl;
+          if (SOFTCAP) {
+            const float th = raw * p.inv_cap;
+            v *= fmaf(-th, th, 1.f);
+          }
+          const bool ok = !EDGE || (n_counts && p.v_begin + t.m0 + mrel < p.vocab);
+          d[r] = ok ? v : 0.f;
         }
-        const bool ok = !EDGE || (n_counts && p.v_begin + t.m0 + mrel < p.vocab);
-        d[r] = ok ? v : 0.f;
+        uint2 w;
+        w.x = pack_bf16(d[0], d[1]);
+        w.y = pack_bf16(d[2], d[3]);
+        *reinterpret_cast<uint2*>(stage + stage_block(block, i, jl)) = w;
       }
-      uint2 w;
-      w.x = pack_bf16(d[0], d[1]);
-      w.y = pack_bf16(d[2], d[3]);
-      *reinterpret_cast<uint2*>(stage + stage_off(nw, i * 4 + lp.lq)) = w;
-    }
+    });
   }
 }
 
@@ -769,27 +778,29 @@ __device__ __forceinline__ void dlogit_stage_logits(const float4 (&x)[kStashHalf
                                                     const DlogitParams& p, const LanePos& lp, const TilePos& t,
                                                     char* stage) {
   const float c = p.inv_temp * kLog2e;
+  const int block = stage_block_base(lp);
 #pragma unroll
   for (int jl = 0; jl < kStashHalfBlocks; ++jl) {
-    const int nw = jl * kBlk + lp.l16;
-    const TokenCoef k(p, t.n0 + lp.wn * kWaveTile + j0 * kBlk + nw, (int64_t)p.v_begin + t.m0);
+    const TokenCoef k(p, t.n0 + lp.wn * kWaveTile + (j0 + jl) * kBlk + lp.l16, (int64_t)p.v_begin + t.m0);
     const int m_end = EDGE ? (k.n_ok ? p.vocab - p.v_begin - t.m0 : 0) : kTile;  // rows that count
+    with_label_or_not(k, lp, [&](auto label) {
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
-      const float4 q = x[jl * kBlocks + i];
-      const float raw[4] = {q.x, q.y, q.z, q.w};
-      float d[4];
+      for (int i = 0; i < kBlocks; ++i) {
+        const float4 q = x[jl * kBlocks + i];
+        const float raw[4] = {q.x, q.y, q.z, q.w};
+        float d[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int mrel = lp.m(i, r);
-        const float v = dlogit_of<SOFTCAP>(raw[r], mrel, k, p, c);
-        d[r] = (!EDGE || mrel < m_end) ? v : 0.f;
+        for (int r = 0; r < 4; ++r) {
+          const int mrel = lp.m(i, r);
+          const float v = dlogit_of<SOFTCAP, decltype(label)::value>(raw[r], mrel, k, p, c);
+          d[r] = (!EDGE || mrel < m_end) ? v : 0.f;
+        }
+        uint2 w;
+        w.x = pack_bf16(d[0], d[1]);
+        w.y = pack_bf16(d[2], d[3]);
+        *reinterpret_cast<uint2*>(stage + stage_block(block, i, jl)) = w;
       }
-      uint2 w;
-      w.x = pack_bf16(d[0], d[1]);
-      w.y = pack_bf16(d[2], d[3]);
-      *reinterpret_cast<uint2*>(stage + stage_off(nw, i * 4 + lp.lq)) = w;
-    }
+    });
   }
 }
 
