@@ -172,7 +172,10 @@ def native():
         load()
         import importlib
 
-        _ext = importlib.import_module("axon_amd._torch_ext")
+        try:
+            _ext = importlib.import_module("axon_amd._torch_ext")
+        except ImportError as e:
+            raise AxonAmdError(f"axon_amd/_torch_ext.so cannot be loaded ({e}); build it with __graft_entry__.build()") from e
     return _ext
 
 
