@@ -132,12 +132,13 @@ __global__ __launch_bounds__(kDwRowsWaves * 64, 2) void dw_rows_kernel(GemmOpera
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = acc4{0.f, 0.f, 0.f, 0.f};
   // Where this lane's sixteen bytes go: row l16 of a block of columns, and of a pair of row blocks the eight values that
-  // the lane holds after the swap below; -1 (beyond the descriptor's end: dropped) where the matrix has no such row.
+  // the lane holds after the swap below.  Where the matrix has no such row: an offset that stays beyond the descriptor's
+  // end (2 MB at most) for every block of columns, so that the store is dropped.
   int vo[MB / 2];
 #pragma unroll
   for (int h = 0; h < MB / 2; ++h) {
     const int m = mt * P::kRows + 32 * h + 16 * (lp.lq & 1) + 8 * (lp.lq >> 1);
-    vo[h] = m < g.m_rows ? lp.l16 * ldo2 + m * 2 : -1;
+    vo[h] = m < g.m_rows ? lp.l16 * ldo2 + m * 2 : INT32_MIN;
   }
   __builtin_amdgcn_s_waitcnt(vmcnt(0));
 
@@ -193,7 +194,9 @@ __global__ __launch_bounds__(kDwRowsWaves * 64, 2) void dw_rows_kernel(GemmOpera
         __builtin_amdgcn_sched_barrier(0);
       }
       settle_acc();
-      // the tile leaves: the two 16-row blocks of a pair trade halves so that a lane holds sixteen contiguous bytes
+      // the tile leaves: the two 16-row blocks of a pair trade halves so that a lane holds sixteen contiguous bytes.  The
+      // rows of the last tile that the result does not have end at the descriptor; a block's offset is added to the
+      // lane's, which is what the hardware compares with the descriptor's size whatever it does with a scalar one.
       const int n0 = t * P::kCols;
       const __amdgpu_buffer_rsrc_t ro = DmaSide<false>::rsrc_of(reinterpret_cast<const char*>(out + (int64_t)n0 * ld_out),
                                                                 min(g.n_rows - n0, P::kCols) * ldo2);
@@ -210,7 +213,9 @@ __global__ __launch_bounds__(kDwRowsWaves * 64, 2) void dw_rows_kernel(GemmOpera
                        : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1));
           typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
           const u32x4 v = {x0, x1, y0, y1};
-          __builtin_amdgcn_raw_buffer_store_b128(v, ro, vo[h], j * kBlk * ldo2, 0);
+          int at;  // an instruction: the compiler would keep the offsets of all blocks in registers of their own
+          asm volatile("v_add_u32 %0, %1, %2" : "=v"(at) : "s"(j * kBlk * ldo2), "v"(vo[h]));
+          __builtin_amdgcn_raw_buffer_store_b128(v, ro, at, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
         }
     }

@@ -1165,6 +1165,27 @@ def test_dweight_from_resident_rows_gives_the_bits_of_tiles(n, h):
     assert torch.equal(dw, ref) and ref.float().norm() > 0
 
 
+@pytest.mark.parametrize("v", [131080, 131112])
+@pytest.mark.parametrize("n,h", [(64, 1056), (150, 1056), (300, 896), (641, 1248)])
+def test_dweight_from_resident_rows_leaves_what_lies_behind_the_last_row(n, h, v):
+    """Tiles of 128, 64, 32 and 32 columns of which the last has 8 or 40: its other blocks of columns and the lanes without
+    a row are kept inside the result by the descriptor alone.  The rows that a whole tile would have stay as they were."""
+    lib = _lib.load()
+    assert lib.axon_lmhead_bwd_dweight_by_rows(n, n, h, v, 0) == 1
+    hid, w, lab = (x.to(DEV) for x in W.lmhead_inputs(n, h, v, seed=n + h))
+    w = (w.float() * 8).bfloat16()
+    g_lp, g_en = torch.randn(2, n, generator=torch.Generator().manual_seed(n)).to(DEV)
+    _, _, lse, eb = _ops.lmhead_forward(hid, w, lab, 1.0)[:4]
+    dh, ref = _ops.lmhead_backward(g_lp, g_en, hid, w, lab, lse, eb, 1.0)
+    room, dh2 = torch.full((v + 128, h), -7.0, device=DEV, dtype=torch.bfloat16), torch.empty_like(dh)
+    ws = torch.empty(lib.axon_lmhead_bwd_workspace_bytes(n, h, v, 0), device=DEV, dtype=torch.uint8)
+    p = _lib.ptr
+    _lib.check(lib.axon_lmhead_bwd(p(g_lp), p(g_en), p(hid), p(w), p(lab), int(lab.dtype == torch.int64), p(lse), p(eb), n, h,
+                                   v, 1.0, 0.0, None, p(dh2), p(room), 0, p(ws), ws.numel(), None, 0,
+                                   _lib.stream_ptr()), "axon_lmhead_bwd")
+    assert torch.equal(room[:v], ref) and (room[v:] == -7.0).all()
+
+
 @pytest.mark.parametrize("v", [1000, 40000, 70001])
 def test_statistics_do_not_depend_on_the_number_of_tokens(v):
     """The kernel that folds the partial statistics takes 4, 16 or 32 tokens per workgroup: a token's results are the same
