@@ -1056,7 +1056,6 @@ class HeadBlocks:
 def scale_f32(x, s1, s2=None):
     """``x * s1 * s2`` for an fp32 array and one or two device scalars (0-d or 1-element fp32 tensors), in one
     launch; a new tensor shaped like ``x``."""
-    require_device(x, "scale_f32")
     return _lib.native().scale_f32(x, s1, s2)
 
 

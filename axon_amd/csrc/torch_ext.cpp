@@ -13,6 +13,7 @@
 #include <hip/hip_runtime_api.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/utils/pybind.h>
@@ -34,12 +35,20 @@ using OptTensor = std::optional<Tensor>;
 namespace {
 
 PyObject* g_error = nullptr;  // axon_amd._lib.AxonAmdError
-struct AxonError : std::runtime_error {
-  using std::runtime_error::runtime_error;
+struct AxonError : torch::PyTorchError {  // the autograd engine hands it on as what it is
+  using PyTorchError::PyTorchError;
+  PyObject* python_type() override { return g_error; }
 };
 
 void check(int rc, const char* what) {
   if (rc != 0) throw AxonError(std::string(what) + ": " + axon_amd_error_string(rc) + " (code " + std::to_string(rc) + ")");
+}
+
+// The HIP path only.  (The Python wrappers look at the first operand of every other function.)
+void require_device(const Tensor& t, const char* what) {
+  if (!t.is_cuda())
+    throw AxonError(std::string(what) + ": tensor is on " + t.device().str() +
+                    "; the axon_amd path runs on MI355X only and has no CPU fallback");
 }
 
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
@@ -337,6 +346,7 @@ std::tuple<OptTensor, Tensor> reverse_scan(int mode, const Tensor& rewards, cons
 
 // x * s1 * s2 (device scalars, s2 may be missing) as a new fp32 tensor shaped like x
 Tensor scale_f32(const Tensor& x, const Tensor& s1, const OptTensor& s2) {
+  require_device(x, "scale_f32");  // a backward comes here without Python, with what a saved-tensor hook has handed back
   const Tensor xf = f32(x);
   const auto scalar = [&](const Tensor& s) {
     Tensor t = s.detach();

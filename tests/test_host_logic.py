@@ -410,6 +410,18 @@ def test_which_output_products_take_half_tiles():
     assert ask(0, 0, 640, 8200, 0) < 0 and ask(2, 1, 640, 8200, 0) < 0 and ask(1, 1, 640, 8200, 100) < 0
 
 
+def test_a_loss_whose_saved_gradient_left_the_gpu_refuses_its_backward():
+    """What a saved-tensor hook hands back goes to a kernel: a tensor in host memory is refused, with the package's error."""
+    from axon_amd import _lib, _ops
+    x = torch.randn(4, requires_grad=True)
+    for factor, slot in ((1.0, 5), (0.5, -1)):
+        loss = _ops.finished_loss(x, torch.arange(8.0), torch.ones(4), factor, slot)
+        with pytest.raises(_lib.AxonAmdError, match="scale_f32: tensor is on cpu"):
+            loss.backward()
+    with pytest.raises(_lib.AxonAmdError, match="scale_f32: tensor is on cpu"):
+        _ops.scale_f32(x, torch.ones(1))
+
+
 def test_which_calls_form_dweight_from_resident_rows():
     """Both sides of each limit of the rule: 768 tokens, hidden 8192, the columns that a part of the vocabulary has (hidden 896:
     two groups of 512 rows and 128 parts up to 320 tokens, four groups and 64 parts beyond), row tiles that fill 15 of 16
