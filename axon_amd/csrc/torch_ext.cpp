@@ -159,7 +159,13 @@ class Slots {
 
 class Post {
  public:
-  explicit Post(OptTensor also) : also_(std::move(also)) {}
+  explicit Post(OptTensor also) : also_(std::move(also)) {
+    if (!also_) return;  // the launch reads nbytes() / 4 words from data_ptr() on
+    require_device(*also_, "the words in front of a loss's sums");
+    if (!also_->is_contiguous() || also_->nbytes() % 4 != 0 || also_->nbytes() > 4 * AXON_MAIL_MAX_WORDS)
+      throw AxonError("the words in front of a loss's sums must be a contiguous tensor of whole words, at most " +
+                      std::to_string(AXON_MAIL_MAX_WORDS) + "; got " + std::to_string(also_->nbytes()) + " bytes");
+  }
   ~Post() {  // never waited for: the slot may not be written any more before another launch gets it
     if (!sent_) return;
     try {

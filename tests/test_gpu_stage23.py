@@ -1032,6 +1032,15 @@ def test_sums_that_the_launch_sends_to_the_host_are_those_on_the_device(kind, re
         _ops.policy_loss(kind, new, old, adv, mask, None, rows, post=_ops.loss_sums_post(torch.zeros(300, device=DEV)), **kw)
 
 
+@pytest.mark.parametrize("words", [lambda: torch.zeros(16, device=DEV)[::2], lambda: torch.zeros(8, 4, device=DEV).t(),
+                                   lambda: torch.zeros(6, device=DEV, dtype=torch.uint8),
+                                   lambda: torch.zeros(225, device=DEV)], ids=["strided", "transposed", "6 bytes", "225 words"])
+def test_words_that_a_launch_cannot_send_as_they_lie_are_refused(words):
+    with pytest.raises(_lib.AxonAmdError, match="contiguous tensor of whole words"):
+        _ops.loss_sums_post(words())
+    assert not _ops.loss_sums_post(torch.zeros(224, device=DEV)).sent
+
+
 # ---- kernels in which a workgroup owns whole rows (GSPO, per-row aggregation, veto, sequence level) --------
 def _awkward_packed(lens, seed):
     """Packed inputs over rows of the given lengths (zeros allowed), padded twins for the oracle."""

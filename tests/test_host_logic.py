@@ -422,6 +422,12 @@ def test_a_loss_whose_saved_gradient_left_the_gpu_refuses_its_backward():
         _ops.scale_f32(x, torch.ones(1))
 
 
+def test_words_sent_with_a_loss_have_to_be_on_the_gpu():
+    from axon_amd import _lib, _ops
+    with pytest.raises(_lib.AxonAmdError, match="tensor is on cpu"):
+        _ops.loss_sums_post(torch.zeros(8))
+
+
 def test_which_calls_form_dweight_from_resident_rows():
     """Both sides of each limit of the rule: 768 tokens, hidden 8192, the columns that a part of the vocabulary has (hidden 896:
     two groups of 512 rows and 128 parts up to 320 tokens, four groups and 64 parts beyond), row tiles that fill 15 of 16
