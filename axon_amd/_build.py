@@ -60,7 +60,7 @@ def _ext_commands(obj: str, out: str, lib_dir: str):
     includes = [*include_paths("cuda"), sysconfig.get_paths()["include"]]
     compile_cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1",
                    "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-                   "-DTORCH_EXTENSION_NAME=_torch_ext", *(a for i in includes for a in ("-isystem", i)),
+                   "-DTORCH_EXTENSION_NAME=_torch_ext", f'-DAXON_TORCH_VERSION="{torch.__version__}"', *(a for i in includes for a in ("-isystem", i)),
                    "-c", os.path.join(CSRC, "torch_ext.cpp"), "-o", obj]
     link_cmd = ["g++", "-shared", "-o", out, obj, f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
                 "-ltorch_python", f"-L{lib_dir}", "-l:libaxon_amd.so", "-Wl,-rpath,$ORIGIN"]

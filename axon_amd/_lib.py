@@ -172,10 +172,19 @@ def native():
         load()
         import importlib
 
+        import torch
+
         try:
-            _ext = importlib.import_module("axon_amd._torch_ext")
+            ext = importlib.import_module("axon_amd._torch_ext")
         except ImportError as e:
             raise AxonAmdError(f"axon_amd/_torch_ext.so cannot be loaded ({e}); build it with __graft_entry__.build()") from e
+        # it passes pointers by the argument lists of the header it was compiled with, and tensors by torch's C++ ABI
+        got = getattr(ext, "abi_version", None), getattr(ext, "torch_version", None)
+        here = ABI_VERSION, str(torch.__version__)
+        if got != here:
+            raise AxonAmdError(f"_torch_ext.so was compiled against ABI {got[0]} and torch {got[1]}, this is ABI {here[0]} and "
+                               f"torch {here[1]}; build it with __graft_entry__.build()")
+        _ext = ext
     return _ext
 
 

@@ -404,6 +404,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       PyErr_SetString(g_error, err.what());
     }
   });
+  // what this file was compiled against: axon_amd/_lib.py refuses another
+  m.attr("abi_version") = AXON_AMD_ABI_VERSION;
+  m.attr("torch_version") = AXON_TORCH_VERSION;
   const py::call_guard<py::gil_scoped_release> unlocked;
   py::class_<Post>(m, "Post")
       .def(py::init<OptTensor>())

@@ -428,6 +428,24 @@ def test_words_sent_with_a_loss_have_to_be_on_the_gpu():
         _ops.loss_sums_post(torch.zeros(8))
 
 
+@pytest.mark.parametrize("stale", [{"abi_version": -1}, {"torch_version": "1.0.0"}, {"abi_version": None},
+                                   {"torch_version": None}])
+def test_an_extension_of_another_abi_or_torch_is_refused(monkeypatch, stale):
+    """As the other library is: its calls would pass the wrong arguments."""
+    import sys
+    import types
+
+    from axon_amd import _lib
+    now = {"abi_version": _lib.ABI_VERSION, "torch_version": str(torch.__version__)}
+    monkeypatch.setattr(_lib, "_ext", None)
+    monkeypatch.setitem(sys.modules, "axon_amd._torch_ext", types.SimpleNamespace(**{**now, **stale}))
+    with pytest.raises(_lib.AxonAmdError, match="_torch_ext.so was compiled against"):
+        _lib.native()
+    assert _lib._ext is None
+    monkeypatch.setitem(sys.modules, "axon_amd._torch_ext", types.SimpleNamespace(**now))
+    assert _lib.native().abi_version == _lib.ABI_VERSION
+
+
 def test_which_calls_form_dweight_from_resident_rows():
     """Both sides of each limit of the rule: 768 tokens, hidden 8192, the columns that a part of the vocabulary has (hidden 896:
     two groups of 512 rows and 128 parts up to 320 tokens, four groups and 64 parts beyond), row tiles that fill 15 of 16
