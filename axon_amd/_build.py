@@ -1,8 +1,8 @@
 """Build recipe for libaxon_amd.so (HIP, gfx950 only) and for _torch_ext.so, the native host side of the small
 operators (plain C++ against torch's headers, linked to the former).
 
-``build()`` always recompiles; ``ensure_built()`` compiles only when a
-library is missing.  hipcc cross-compiles without a GPU.
+``build()`` always recompiles both; ``ensure_built()`` compiles only when libaxon_amd.so is missing, and
+``ensure_extension_built()`` the extension alone when that is what is missing.  hipcc cross-compiles without a GPU.
 """
 
 from __future__ import annotations
@@ -45,7 +45,7 @@ def _run(cmd, cwd) -> str:
         if "is not a recognized feature" not in line  # host pass does not know the GPU feature
     )
     if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({proc.returncode}): {' '.join(cmd)}\n{log}")
+        raise RuntimeError(f"{cmd[0]} failed ({proc.returncode}): {' '.join(cmd)}\n{log}")
     return log
 
 
@@ -60,7 +60,8 @@ def _ext_commands(obj: str, out: str, lib_dir: str):
     includes = [*include_paths("cuda"), sysconfig.get_paths()["include"]]
     compile_cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1",
                    "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-                   "-DTORCH_EXTENSION_NAME=_torch_ext", f'-DAXON_TORCH_VERSION="{torch.__version__}"', *(a for i in includes for a in ("-isystem", i)),
+                   "-DTORCH_EXTENSION_NAME=_torch_ext", f'-DAXON_TORCH_VERSION="{torch.__version__}"',
+                   *(a for i in includes for a in ("-isystem", i)),
                    "-c", os.path.join(CSRC, "torch_ext.cpp"), "-o", obj]
     link_cmd = ["g++", "-shared", "-o", out, obj, f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
                 "-ltorch_python", f"-L{lib_dir}", "-l:libaxon_amd.so", "-Wl,-rpath,$ORIGIN"]
@@ -94,6 +95,17 @@ def build(verbose: bool = False) -> str:
 
 
 def ensure_built() -> str:
-    if not (os.path.exists(LIB_PATH) and os.path.exists(EXT_PATH)):
+    if not os.path.exists(LIB_PATH):
         build()
     return LIB_PATH
+
+
+def ensure_extension_built() -> str:
+    """The extension beside a library that is there: g++ and torch's headers, no hipcc."""
+    if not os.path.exists(EXT_PATH):
+        with tempfile.TemporaryDirectory(prefix="axon_amd_build_") as tmp:
+            ext = os.path.join(tmp, "_torch_ext.so")
+            for cmd in _ext_commands(os.path.join(tmp, "torch_ext.o"), ext, os.path.dirname(LIB_PATH)):
+                _run(cmd, tmp)
+            shutil.move(ext, EXT_PATH)
+    return EXT_PATH

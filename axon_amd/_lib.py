@@ -175,8 +175,10 @@ def native():
         import torch
 
         try:
+            with _lock:
+                _build.ensure_extension_built()
             ext = importlib.import_module("axon_amd._torch_ext")
-        except ImportError as e:
+        except (ImportError, OSError, RuntimeError) as e:  # no such file and no compiler, or not for this torch
             raise AxonAmdError(f"axon_amd/_torch_ext.so cannot be loaded ({e}); build it with __graft_entry__.build()") from e
         # it passes pointers by the argument lists of the header it was compiled with, and tensors by torch's C++ ABI
         got = getattr(ext, "abi_version", None), getattr(ext, "torch_version", None)

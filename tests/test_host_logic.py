@@ -412,7 +412,7 @@ def test_which_output_products_take_half_tiles():
 
 def test_a_loss_whose_saved_gradient_left_the_gpu_refuses_its_backward():
     """What a saved-tensor hook hands back goes to a kernel: a tensor in host memory is refused, with the package's error."""
-    from axon_amd import _lib, _ops
+    from axon_amd import _ops
     x = torch.randn(4, requires_grad=True)
     for factor, slot in ((1.0, 5), (0.5, -1)):
         loss = _ops.finished_loss(x, torch.arange(8.0), torch.ones(4), factor, slot)
@@ -423,7 +423,7 @@ def test_a_loss_whose_saved_gradient_left_the_gpu_refuses_its_backward():
 
 
 def test_words_sent_with_a_loss_have_to_be_on_the_gpu():
-    from axon_amd import _lib, _ops
+    from axon_amd import _ops
     with pytest.raises(_lib.AxonAmdError, match="tensor is on cpu"):
         _ops.loss_sums_post(torch.zeros(8))
 
@@ -434,8 +434,6 @@ def test_an_extension_of_another_abi_or_torch_is_refused(monkeypatch, stale):
     """As the other library is: its calls would pass the wrong arguments."""
     import sys
     import types
-
-    from axon_amd import _lib
     now = {"abi_version": _lib.ABI_VERSION, "torch_version": str(torch.__version__)}
     monkeypatch.setattr(_lib, "_ext", None)
     monkeypatch.setitem(sys.modules, "axon_amd._torch_ext", types.SimpleNamespace(**{**now, **stale}))
@@ -444,6 +442,29 @@ def test_an_extension_of_another_abi_or_torch_is_refused(monkeypatch, stale):
     assert _lib._ext is None
     monkeypatch.setitem(sys.modules, "axon_amd._torch_ext", types.SimpleNamespace(**now))
     assert _lib.native().abi_version == _lib.ABI_VERSION
+
+
+def test_a_missing_extension_is_built_alone_and_only_when_it_is_asked_for(monkeypatch, tmp_path):
+    """A library without the extension beside it loads without a compiler; the extension is compiled by g++ and linked to it."""
+    from axon_amd import _build
+    ran = []
+
+    def run(cmd, cwd):
+        ran.append(cmd)
+        if "-shared" in cmd:
+            open(cmd[cmd.index("-o") + 1], "w").close()
+        return ""
+
+    ext = str(tmp_path / "_torch_ext.so")
+    monkeypatch.setattr(_build, "EXT_PATH", ext)
+    monkeypatch.setattr(_build, "_run", run)
+    monkeypatch.setattr(_build, "_hipcc", lambda: pytest.fail("hipcc asked for"))
+    assert _build.ensure_built() == _build.LIB_PATH and not ran
+    monkeypatch.setattr(_lib, "_lib", None)
+    assert _lib.load() is not None and not ran
+    assert _build.ensure_extension_built() == ext and os.path.exists(ext)
+    assert [c[0] for c in ran] == ["g++", "g++"] and f"-L{os.path.dirname(_build.LIB_PATH)}" in ran[1]
+    assert _build.ensure_extension_built() == ext and len(ran) == 2
 
 
 def test_which_calls_form_dweight_from_resident_rows():
