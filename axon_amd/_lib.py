@@ -113,8 +113,8 @@ SIGNATURES: dict[str, tuple] = {
                                 _ptr]),
     "axon_policy_loss_rows": (_i32, [_i32, _ptr, _ptr, _ptr, _ptr, _i32, _ptr, _ptr, _i64, _i64, _i64, _i32, _i32,
                                      _ptr, _ptr, _ptr, _ptr, _f32, _f32, _f32, _ptr, _ptr, _ptr, _ptr]),
-    "axon_policy_loss_post": (_i32, [_i32, _ptr, _ptr, _ptr, _ptr, _i32, _ptr, _i64, _f32, _ptr, _f32, _f32, _f32, _ptr,
-                                     _ptr, _ptr, _ptr, _i64, _ptr, ctypes.c_uint32, _ptr]),
+    "axon_policy_loss_post": (_i32, [_i32, _ptr, _ptr, _ptr, _ptr, _i32, _ptr, _ptr, _i64, _i64, _i64, _f32, _ptr, _f32,
+                                     _f32, _f32, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, ctypes.c_uint32, _ptr]),
     "axon_policy_loss_rows_post": (_i32, [_i32, _ptr, _ptr, _ptr, _ptr, _i32, _ptr, _ptr, _i64, _i64, _i64, _i32, _i32,
                                           _ptr, _ptr, _ptr, _ptr, _f32, _f32, _f32, _ptr, _ptr, _ptr, _ptr, _i64, _ptr,
                                           ctypes.c_uint32, _ptr]),
@@ -125,7 +125,7 @@ SIGNATURES: dict[str, tuple] = {
                                         _ptr, _ptr, _f32, _i32, _ptr, _f32, _f32, _f32, _ptr, _ptr, _ptr]),
 }
 
-ABI_VERSION = 24
+ABI_VERSION = 25
 MASK_F32, MASK_I64 = 0, 1
 
 _lock = threading.Lock()

@@ -787,13 +787,13 @@ extern "C" int axon_policy_loss(int kind, const float* logp, const float* oldp, 
 }
 
 extern "C" int axon_policy_loss_post(int kind, const float* logp, const float* oldp, const float* adv, const void* mask,
-                                     int mask_kind, const float* isw, int64_t n_slots, float uniform_scale,
-                                     const double* valid, float ratio_lo, float ratio_hi, float clip_c, float* grad,
-                                     float* acc, float* partials, const void* also, int64_t n_also, void* host,
-                                     uint32_t seq, void* stream) {
+                                     int mask_kind, const float* isw, const int32_t* cu, int64_t n_rows, int64_t n_slots,
+                                     int64_t uniform_len, float uniform_scale, const double* valid, float ratio_lo,
+                                     float ratio_hi, float clip_c, float* grad, float* acc, float* partials,
+                                     const void* also, int64_t n_also, void* host, uint32_t seq, void* stream) {
   if (n_slots <= 0 || kind == 1 || n_also < 0 || n_also > AXON_MAIL_MAX_WORDS || (n_also > 0 && !also) || !host)
     return AXON_ERR_ARG;
-  return policy_loss_impl(kind, logp, oldp, adv, mask, mask_kind, isw, nullptr, 1, n_slots, n_slots, nullptr, nullptr,
+  return policy_loss_impl(kind, logp, oldp, adv, mask, mask_kind, isw, cu, n_rows, n_slots, uniform_len, nullptr, nullptr,
                           uniform_scale, 1, valid, ratio_lo, ratio_hi, clip_c, grad, acc, partials, stream,
                           Mail{static_cast<const uint32_t*>(also), (int)n_also, static_cast<uint32_t*>(host), seq});
 }

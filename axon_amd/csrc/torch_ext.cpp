@@ -260,8 +260,9 @@ std::tuple<Tensor, Tensor> policy_loss(int kind, const Tensor& log_probs, const 
   if (post != nullptr && n > 0 && !capturing()) {
     const Slot& slot = post->send(st);
     const int rc =
-        one_pass ? axon_policy_loss_post(kind, lp_p, old_p, adv_p, ptr(mk.first), mk.second, isw_p, n, scale, valid_p, lo, hi,
-                                         clip, grad_p, acc_p, ws_p, post->also(), post->n_also(), slot.device, slot.seq, st)
+        one_pass ? axon_policy_loss_post(kind, lp_p, old_p, adv_p, ptr(mk.first), mk.second, isw_p, rows.offsets(), rows.n_rows,
+                                         n, rows.uniform_len, scale, valid_p, lo, hi, clip, grad_p, acc_p, ws_p,
+                                         post->also(), post->n_also(), slot.device, slot.seq, st)
                  : axon_policy_loss_rows_post(kind, lp_p, old_p, adv_p, ptr(mk.first), mk.second, isw_p, rows.offsets(),
                                               rows.n_rows, n, rows.uniform_len, token_reduce, batch_reduce, prtc_p, npt_p,
                                               nps_p, valid_p, lo, hi, clip, grad_p, acc_p, ws_p, post->also(),

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define AXON_AMD_ABI_VERSION 24
+#define AXON_AMD_ABI_VERSION 25
 
 enum {
   AXON_OK = 0,
@@ -562,13 +562,13 @@ int axon_policy_loss_rows(int kind, const float* logp, const float* old_logp, co
  * is needed.  host, in 32-bit words: [0] = seq once everything else has arrived (the caller makes sure that it holds
  * another value before), from word 16 on the n_also <= AXON_MAIL_MAX_WORDS words at `also` (device memory that earlier work
  * of the stream has written) and then acc[0..7].  n_slots > 0.  axon_policy_loss_post is the call without a per-row
- * quantity (kind != 1, post_normalize). */
+ * quantity (kind != 1, post_normalize); it takes and refuses the rows that axon_policy_loss does. */
 #define AXON_MAIL_MAX_WORDS 224
 int axon_policy_loss_post(int kind, const float* logp, const float* old_logp, const float* adv, const void* mask,
-                          int mask_kind, const float* is_weights, int64_t n_slots, float uniform_scale,
-                          const double* valid_count, float ratio_lo, float ratio_hi, float clip_c, float* grad,
-                          float* acc, float* partials, const void* also, int64_t n_also, void* host, uint32_t seq,
-                          void* stream);
+                          int mask_kind, const float* is_weights, const int32_t* cu_seqlens, int64_t n_rows,
+                          int64_t n_slots, int64_t uniform_len, float uniform_scale, const double* valid_count,
+                          float ratio_lo, float ratio_hi, float clip_c, float* grad, float* acc, float* partials,
+                          const void* also, int64_t n_also, void* host, uint32_t seq, void* stream);
 int axon_policy_loss_rows_post(int kind, const float* logp, const float* old_logp, const float* adv, const void* mask,
                                int mask_kind, const float* is_weights, const int32_t* cu_seqlens, int64_t n_rows,
                                int64_t n_slots, int64_t uniform_len, int token_reduce, int batch_reduce,

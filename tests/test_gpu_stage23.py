@@ -1041,6 +1041,17 @@ def test_words_that_a_launch_cannot_send_as_they_lie_are_refused(words):
     assert not _ops.loss_sums_post(torch.zeros(224, device=DEV)).sent
 
 
+@pytest.mark.parametrize("loss_fn", ["ppo", "cispo", "value"])
+def test_a_loss_over_offsets_without_an_entry_is_refused(loss_fn):
+    """Packed tokens whose cu_seqlens are empty (no [0, ..., n] at all) do not have -1 rows."""
+    x = torch.zeros(64, device=DEV)
+    names = ("log_probs", "old_log_probs", "advantages", "response_mask", "vpreds", "values", "returns")
+    data = DataProto.from_dict(tensors={k: x for k in names},
+                               meta_info={"cu_seqlens": torch.empty(0, device=DEV, dtype=torch.int32)})
+    with pytest.raises(_lib.AxonAmdError):
+        compute_loss_fn(data, loss_fn, {})
+
+
 # ---- kernels in which a workgroup owns whole rows (GSPO, per-row aggregation, veto, sequence level) --------
 def _awkward_packed(lens, seed):
     """Packed inputs over rows of the given lengths (zeros allowed), padded twins for the oracle."""
