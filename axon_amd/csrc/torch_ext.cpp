@@ -18,6 +18,7 @@
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cstring>
@@ -115,12 +116,15 @@ Rows rows_of(const RowsTuple& t) {
 
 // The sums of a loss on their way to the host (axon_policy_loss_post): `also`, a tensor that earlier work of the stream has
 // written, and the loss's eight sums behind it.
-// One launch writes to a slot of pinned memory at a time; a slot goes back once its words have arrived.  The slots, one
-// kilobyte each, are as many as posts were ever under way together and live until the process ends.
+// One launch writes to a slot of pinned memory at a time; a slot goes back once its words have arrived.  One that nobody
+// waits for any more (its loss raised behind the launch) is set aside until they have, which the next taker finds out: to wait
+// in a destructor would hold the interpreter lock for the rest of the queue.  The slots, one kilobyte each, are as many as
+// posts were ever under way together and live until the process ends.
 struct Slot {
   uint32_t* host;
   uint32_t* device;
   uint32_t seq;
+  bool arrived() const { return __atomic_load_n(host, __ATOMIC_ACQUIRE) == seq; }
 };
 class Slots {
  public:
@@ -132,6 +136,9 @@ class Slots {
   }
   Slot take() {
     const std::lock_guard<std::mutex> lock(mutex_);
+    const auto back = std::partition(aside_.begin(), aside_.end(), [](const Slot& s) { return !s.arrived(); });
+    free_.insert(free_.end(), back, aside_.end());
+    aside_.erase(back, aside_.end());
     if (free_.empty()) {
       void *host = nullptr, *device = nullptr;
       if (hipHostMalloc(&host, kBytes * kPerBlock, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
@@ -141,6 +148,7 @@ class Slots {
       std::memset(host, 0, kBytes * kPerBlock);
       for (int i = 0; i < kPerBlock; ++i)
         free_.push_back(Slot{static_cast<uint32_t*>(host) + i * (kBytes / 4), static_cast<uint32_t*>(device) + i * (kBytes / 4), 0});
+      made_ += kPerBlock;
     }
     Slot s = free_.back();
     free_.pop_back();
@@ -151,10 +159,19 @@ class Slots {
     const std::lock_guard<std::mutex> lock(mutex_);
     free_.push_back(s);
   }
+  void set_aside(const Slot& s) {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    aside_.push_back(s);
+  }
+  int made() {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    return made_;
+  }
 
  private:
   std::mutex mutex_;
-  std::vector<Slot> free_;
+  std::vector<Slot> free_, aside_;
+  int made_ = 0;
 };
 
 class Post {
@@ -166,12 +183,11 @@ class Post {
       throw AxonError("the words in front of a loss's sums must be a contiguous tensor of whole words, at most " +
                       std::to_string(AXON_MAIL_MAX_WORDS) + "; got " + std::to_string(also_->nbytes()) + " bytes");
   }
-  ~Post() {  // never waited for: the slot may not be written any more before another launch gets it
+  ~Post() {  // never waited for
     if (!sent_) return;
     try {
-      arrive();
-      Slots::get().give(slot_);
-    } catch (...) {
+      Slots::get().set_aside(slot_);
+    } catch (...) {  // no memory for the list: the slot is not used again
     }
   }
   const void* also() const { return also_ ? also_->data_ptr() : nullptr; }
@@ -211,16 +227,15 @@ class Post {
   void arrive() {
     if (!sent_) throw AxonError("no sums are on their way");
     sent_ = false;
-    const auto arrived = [&] { return __atomic_load_n(slot_.host, __ATOMIC_ACQUIRE) == slot_.seq; };
     const auto start = std::chrono::steady_clock::now();
-    for (int n = 1; !arrived(); ++n) {
+    for (int n = 1; !slot_.arrived(); ++n) {
       if (n % 1024) {
         __builtin_ia32_pause();
         continue;
       }
       if (std::chrono::steady_clock::now() - start < std::chrono::milliseconds(2)) continue;
       const hipError_t err = hipStreamSynchronize(stream_);
-      if (err == hipSuccess && arrived()) break;
+      if (err == hipSuccess && slot_.arrived()) break;
       // the slot is not used again: the device may be in any state
       throw AxonError(std::string("the sums of a loss did not arrive: ") + hipGetErrorString(err));
     }
@@ -414,6 +429,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def_property_readonly("sent", &Post::is_sent)
       .def("sums", &Post::sums, unlocked)
       .def("wait", &Post::wait, unlocked);
+  m.def("post_slots", [] { return Slots::get().made(); });
   m.def("policy_loss", &policy_loss, unlocked);
   m.def("group_advantage", &group_advantage, unlocked);
   m.def("sampler_correction_diag", &sampler_correction_diag, unlocked);

@@ -1041,6 +1041,35 @@ def test_words_that_a_launch_cannot_send_as_they_lie_are_refused(words):
     assert not _ops.loss_sums_post(torch.zeros(224, device=DEV)).sent
 
 
+def test_sums_that_nobody_waits_for_hold_up_neither_the_host_nor_the_slots():
+    """A post dropped behind its launch does not wait for the GPU; its slot comes back once the words have arrived."""
+    x = torch.ones(64, device=DEV)
+    rows = _ops.rows_of(x, torch.tensor([0, 64], device=DEV, dtype=torch.int32))
+    kw = dict(token_reduce="sum", batch_reduce="token-mean", ratio_lo=0.8, ratio_hi=1.28, clip_c=3.0)
+    work = torch.zeros(1 << 28, device=DEV)
+
+    def drop():
+        post = _ops.loss_sums_post()
+        _ops.policy_loss(0, x, x, x, x, None, rows, post=post, **kw)
+        assert post.sent
+
+    drop()
+    torch.cuda.synchronize()
+    for _ in range(200):  # 400 GB of traffic: some 80 ms
+        work.add_(1.0)
+    drop()
+    assert not torch.cuda.current_stream().query()
+    torch.cuda.synchronize()
+    made = _lib.native().post_slots()
+    for _ in range(made + 8):
+        drop()
+        torch.cuda.synchronize()
+    assert _lib.native().post_slots() == made
+    post = _ops.loss_sums_post()
+    acc, _ = _ops.policy_loss(0, x, x, x, x, None, rows, post=post, **kw)
+    assert _ops.loss_sums(post, acc) == acc.tolist()
+
+
 @pytest.mark.parametrize("loss_fn", ["ppo", "cispo", "value"])
 def test_a_loss_over_offsets_without_an_entry_is_refused(loss_fn):
     """Packed tokens whose cu_seqlens are empty (no [0, ..., n] at all) do not have -1 rows."""
