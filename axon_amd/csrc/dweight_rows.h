@@ -10,11 +10,12 @@
 // of a tile have until the ring comes round to drain, and a wave never waits for a load that is younger than its
 // last tile's stores.  Each accumulator takes the same products in the same order as in DmaLoop: the same bits.
 //
-// Measured (us, 256 x 256 tiles before / this kernel), vocabulary 151936 x hidden 4096: 64 tokens 390 / 247, 128 424 / 285,
-// 192 480 / 330, 256 540 / 375, 300 585 / 427, 384 645 / 505, 448 715 / 560, 512 750 / 610, 640 845 / 735, 700 905 / 845, 768
-// 965 / 905; 100 x 2880 x 201088 367 / 290, 500 x 2880 x 201088 680 / 590, 600 x 896 x 151936 197 / 185, 500 x 2048 x 32768
-// 81 / 73.  What bounds it: the stores and the products of a tile still add up in part (all CUs are in the same phase), and from 704
-// tokens on the tiles are 32 columns wide, where a fragment from LDS serves two MFMAs and the barrier comes every 88.
+// Measured (us between events, 256 x 256 tiles / this kernel, both on one card), vocabulary 151936 x hidden 4096: 64 tokens
+// 362 / 232, 128 398 / 282, 192 455 / 321, 256 508 / 366, 300 556 / 419, 384 604 / 500, 448 658 / 528, 512 715 / 585, 640 804 / 710,
+// 700 860 / 819, 768 917 / 877; 100 x 2880 x 201088 346 / 284, 333 532 / 495, 500 629 / 570; 300 x 896 x 151936 128 / 109, 600
+// 185 / 180; 500 x 2048 x 32768 78 / 69, of which a loop over that call gives back most (dHidden, which follows, 72 / 80).
+// What bounds it: the stores and the products of a tile still add up in part (all CUs are in the same phase); beyond 320 tokens a
+// fragment from LDS serves two MFMAs, and beyond 640 the tiles are 32 columns wide, with a barrier every 88 or 96 MFMAs.
 // Beyond 768 tokens the rows no longer fit in the registers.  Tried: the barrier in the middle of a tile, so that the
 // next one's fragments are read ahead (64 tokens 252, 700 860), half of the wavefronts storing a tile later (264, 856),
 // non-temporal stores (64-byte pieces of rows: 372), four wavefronts with twice the registers (700 tokens 974).
@@ -29,8 +30,8 @@ constexpr int kDwRowsCus = 256, kDwRowsWaves = 8;
 // 16-row blocks of hT per wavefront for a reduction of kt k-tiles of 64 tokens: four are whole 128-byte lines of the
 // result and halve the LDS reads per MFMA (64 tokens 300 us with two), two where four would not fit in the registers.
 constexpr int dw_rows_mb(int kt) { return kt <= 5 ? 4 : 2; }
-// 16-column blocks of a tile: as many as the registers and two slots in LDS allow (448 tokens 636 us with two, 574 with
-// four).
+// 16-column blocks of a tile: as many as the registers and two slots in LDS allow: eight up to 128 tokens, two for 257 to
+// 320 and beyond 640, else four (448 tokens 636 us with two, 574 with four).
 constexpr int dw_rows_nb(int kt) { return kt <= 2 ? 8 : kt == 5 || kt > 10 ? 2 : 4; }
 // Workgroups that share the rows of hT; each takes one of kDwRowsCus / groups parts of the vocabulary's tiles (up to 8192
 // hidden at least 90 % of the compute units then have work).
@@ -224,15 +225,32 @@ __global__ __launch_bounds__(kDwRowsWaves * 64, 2) void dw_rows_kernel(GemmOpera
   __builtin_amdgcn_s_waitcnt(vmcnt(0));  // loads past the range must not land in the next workgroup's LDS
 }
 
-// Whether that is the faster way: each workgroup loads its rows (up to 32 KB per wavefront) and fills the ring before its
-// first tile, which a long enough walk makes up for, and beyond 640 tokens, where little is gained, the row tiles have to
-// fill the groups.  256 x 256 tiles / this kernel, us, by columns walked: 192 tokens 256 columns 26 / 25, 512 46 / 36;
-// 256 tokens 256 28 / 29; 320 tokens 256 30 / 33, 512 57 / 51; 384 to 640 tokens 512 38 / 40, 768 62 / 64 to 48 / 45,
-// 1024 72 / 68 and 92 / 85.  Hidden 896 (7 of 8 wavefronts have rows) 704 tokens 172 / 184, 1152 (90 %) 256 / 257, 2880
-// (15 of 16) 829 / 824, 3072 555 / 536.
+// Whether that is the faster way.  A workgroup loads its rows (up to 32 KB per wavefront) and fills the ring before its
+// first tile, which a long enough walk makes up for.  Its time is that of eight wavefronts also where some have no rows,
+// while a tile of 256 x 256 whose rows end in its first half is computed as half a tile: the more rows are computed here
+// against there (`mine` / `theirs`), the longer that takes.  256 x 256 tiles / this kernel, us, by columns walked:
+//   192 tokens: 256 columns, hidden 896 25.5 / 25.3, 576 24.2 / 21.6, 2880 28.0 / 27.4.
+//   256 tokens: 256 columns, hidden 896 28.0 / 29.4, 2880 30.8 / 31.8; 384 columns 39.1 / 36.6 and 42.4 / 39.4, hidden 576 (1024
+//     rows for 640) 30.4 / 30.8; 512 columns 49.4 / 43.7, 54.5 / 47.8 and 39.2 / 37.0.
+//   320 tokens: 512 columns, hidden 896 54.7 / 51.2, 2880 59.3 / 52.7, 576 42.9 / 44.2; 1024 columns, hidden 576 74.3 / 74.4.
+//   384 to 576 tokens: 512 columns 38 / 40, 768 62 / 64 to 48 / 45, 1024 60.8 / 56.3 and 75.4 / 75.7 (hidden 896), 52.4 / 48.4 and
+//     66.0 / 66.6 (288).
+//   640 tokens: 1024 columns, hidden 2880 (3072 rows for 2944) 89.2 / 84.7, 1056 (1280 for 1152) 75.9 / 74.3, 288 (512 for 384) 69.9 / 72.4;
+//     hidden 896 (1024 for 896) 1536 columns 120.5 / 123.8, 2048 159.6 / 163.9, 2374 189.9 / 189.1.
+//   704 and 768 tokens: 1024 columns, hidden 512 102.4 / 105.3 and 109.0 / 110.8, 3072 98.1 / 99.7 and 101.1 / 107.0; 2048 columns, hidden
+//     512 191.0 / 187.9 and 210.6 / 200.5, 2048 197.9 / 191.7, 3072 192.9 / 193.0, 4096 195.7 / 186.9; and only where the row tiles fill 15 of
+//     16 wavefronts (hidden 896, 7 of 8, 172 / 184 at 151936 columns of vocabulary).
 constexpr bool dw_rows_worth(int64_t h, int64_t vc, int64_t k) {
   const int kt = (int)(k / 64);
-  const int64_t groups = dw_rows_groups(h, kt), walk = kt <= 4 ? 256 : kt == 5 ? 512 : 1024;
+  const int64_t groups = dw_rows_groups(h, kt);
+  const int64_t mine = groups * kDwRowsWaves * dw_rows_mb(kt) * kBlk, theirs = (h + 127) / 128 * 128;
+  const bool sparse = 2 * mine > 3 * theirs, over = 8 * mine > 9 * theirs;
+  const int64_t walk = kt <= 3    ? 256
+                       : kt == 4  ? (sparse ? 512 : 384)
+                       : kt == 5  ? (sparse ? 1024 : 512)
+                       : kt <= 9  ? 1024
+                       : kt == 10 ? (over ? 2304 : 1024)
+                                  : 2048;
   const bool full = (h + 31) / 32 * 16 >= groups * kDwRowsWaves * 15;
   return vc >= walk * (kDwRowsCus / groups) && (kt <= 10 || full);
 }

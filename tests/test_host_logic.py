@@ -476,10 +476,16 @@ def test_which_calls_form_dweight_from_resident_rows():
     by = lambda n, h, v, chunk=0: ask(n, n, h, v, chunk)  # noqa: E731
     assert by(1, 4096, 151936) == 1 and by(768, 4096, 151936) == 1 and by(769, 4096, 151936) == 0
     assert by(700, 8192, 151936) == 1 and by(700, 8224, 151936) == 0
-    assert by(1, 896, 32768) == 1 and by(256, 896, 32768) == 1 and by(256, 896, 32760) == 0
+    assert by(1, 896, 32768) == 1 and by(192, 896, 32768) == 1 and by(192, 896, 32760) == 0
+    assert by(256, 896, 49152) == 1 and by(256, 896, 49144) == 0
+    assert by(256, 576, 65536) == 1 and by(256, 576, 65528) == 0      # 1024 rows computed for 640
+    assert by(320, 576, 131072) == 1 and by(320, 576, 131064) == 0
     assert by(257, 896, 65536) == 1 and by(257, 896, 65528) == 0
-    assert by(321, 896, 65536) == 1 and by(640, 896, 65528) == 0
+    assert by(321, 896, 65536) == 1 and by(576, 896, 65536) == 1 and by(576, 896, 65528) == 0
+    assert by(577, 2880, 21504) == 1 and by(577, 2880, 21496) == 0    # 3072 rows computed for 2944
+    assert by(577, 896, 147456) == 1 and by(640, 896, 147448) == 0    # 1024 for 896
     assert by(640, 896, 151936) == 1 and by(641, 896, 151936) == 0 and by(641, 1152, 151936) == 0
+    assert by(641, 512, 262144) == 1 and by(641, 512, 262136) == 0 and by(768, 512, 131072) == 0
     assert by(300, 4096, 50257) == 0 and by(300, 224, 151936) == 0  # vocab-major copies of the dlogits
     assert by(700, 4096, 151936, 4096) == 0                          # short chunks of the vocabulary
     assert ask(700, 40000, 4096, 151936, 152064) == 1                # a block shorter than the workspace
