@@ -228,30 +228,35 @@ __global__ __launch_bounds__(kDwRowsWaves * 64, 2) void dw_rows_kernel(GemmOpera
 // Whether that is the faster way.  A workgroup loads its rows (up to 32 KB per wavefront) and fills the ring before its
 // first tile, which a long enough walk makes up for.  Its time is that of eight wavefronts also where some have no rows,
 // while a tile of 256 x 256 whose rows end in its first half is computed as half a tile: the more rows are computed here
-// against there (`mine` / `theirs`), the longer that takes.  256 x 256 tiles / this kernel, us, by columns walked:
-//   192 tokens: 256 columns, hidden 896 25.5 / 25.3, 576 24.2 / 21.6, 2880 28.0 / 27.4.
-//   256 tokens: 256 columns, hidden 896 28.0 / 29.4, 2880 30.8 / 31.8; 384 columns 39.1 / 36.6 and 42.4 / 39.4, hidden 576 (1024
-//     rows for 640) 30.4 / 30.8; 512 columns 49.4 / 43.7, 54.5 / 47.8 and 39.2 / 37.0.
-//   320 tokens: 512 columns, hidden 896 54.7 / 51.2, 2880 59.3 / 52.7, 576 42.9 / 44.2; 1024 columns, hidden 576 74.3 / 74.4.
-//   384 to 576 tokens: 512 columns 38 / 40, 768 62 / 64 to 48 / 45, 1024 60.8 / 56.3 and 75.4 / 75.7 (hidden 896), 52.4 / 48.4 and
-//     66.0 / 66.6 (288).
-//   640 tokens: 1024 columns, hidden 2880 (3072 rows for 2944) 89.2 / 84.7, 1056 (1280 for 1152) 75.9 / 74.3, 288 (512 for 384) 69.9 / 72.4;
-//     hidden 896 (1024 for 896) 1536 columns 120.5 / 123.8, 2048 159.6 / 163.9, 2374 189.9 / 189.1.
-//   704 and 768 tokens: 1024 columns, hidden 512 102.4 / 105.3 and 109.0 / 110.8, 3072 98.1 / 99.7 and 101.1 / 107.0; 2048 columns, hidden
-//     512 191.0 / 187.9 and 210.6 / 200.5, 2048 197.9 / 191.7, 3072 192.9 / 193.0, 4096 195.7 / 186.9; and only where the row tiles fill 15 of
-//     16 wavefronts (hidden 896, 7 of 8, 172 / 184 at 151936 columns of vocabulary).
+// than there (`mine`, `theirs`), the longer that takes.  Beyond 640 tokens little is gained, and nothing where rows are computed
+// for nothing or compute units go without a part of the vocabulary.  256 x 256 tiles / this kernel, us, on the same buffers
+// (between buffers at other addresses either differs by up to 5 %), by columns walked:
+//   192 tokens: hidden 896 192 columns 22.6 / 21.2, 256 23.9 / 23.6; 576 (1024 rows for 640) 192 17.0 / 18.6, 256 23.2 / 20.6; 2880 256
+//     26.8 / 25.7.
+//   256 tokens: hidden 896 256 columns 27.0 / 27.8, 384 36.8 / 34.3; 2880 256 29.3 / 29.5, 384 40.1 / 36.7; 576 384 28.6 / 29.2, 512 36.9 / 35.1.
+//   320 tokens: hidden 896 384 columns 41.0 / 40.8, 512 53.6 / 50.7; 2880 512 56.0 / 49.9; 576 768 55.6 / 56.6, 1024 76.0 / 73.8.
+//   384 and 576 tokens: hidden 896 1024 columns 57.1 / 54.7 and 71.8 / 70.3 (768: 54.9 / 56.8 for 576); 288 1024 65.6 / 66.2 for 576.
+//   640 tokens: 1024 columns, hidden 2880 (3072 rows for 2944) 81.6 / 79.4, 1056 (1280 for 1152) 77.6 / 75.8, 288 (512 for 384)
+//     69.2 / 73.8; 896 (1024 for 896) 1536 113.3 / 116.7, 1600 118.6 / 112.6, 2004 149.2 / 138.2, 2374 177.6 / 167.8.
+//   704 tokens, 151936 vocabulary rows: hidden 896 188 / 194, 1248 254 / 246, 1504 (252 of 256 compute units) 300 / 296, 2560 (250) 514 / 521,
+//     2880 579 / 599, 3072 (252) 623 / 624, 3584 (252, fourteen groups) 713 / 728, 4096 862 / 819, 5120 (240) 1045 / 1083.  By columns: hidden
+//     512 1536 146.1 / 146.7, 2048 192.9 / 190.0, but 1571, where the tiles are 6.14 rounds, 154.5 / 139.1 and 1187 (4.64) 112 / 111;
+//     992 1600 (6.25 rounds) 145 / 137, 2004 171 / 167; 2048 1536 136.2 / 139.1, 2048 187.1 / 185.9.
 constexpr bool dw_rows_worth(int64_t h, int64_t vc, int64_t k) {
   const int kt = (int)(k / 64);
   const int64_t groups = dw_rows_groups(h, kt);
   const int64_t mine = groups * kDwRowsWaves * dw_rows_mb(kt) * kBlk, theirs = (h + 127) / 128 * 128;
   const bool sparse = 2 * mine > 3 * theirs, over = 8 * mine > 9 * theirs;
+  // half tiles of the other way, 512 to a round: its last round leaves a twentieth of all of them unused
+  const int64_t halves = (vc + 255) / 256 * (theirs / 128), rounds = (halves + 511) / 512;
+  const bool ends_empty = 100 * 512 * rounds > 105 * halves;
   const int64_t walk = kt <= 3    ? 256
                        : kt == 4  ? (sparse ? 512 : 384)
                        : kt == 5  ? (sparse ? 1024 : 512)
                        : kt <= 9  ? 1024
-                       : kt == 10 ? (over ? 2304 : 1024)
-                                  : 2048;
-  const bool full = (h + 31) / 32 * 16 >= groups * kDwRowsWaves * 15;
+                       : kt == 10 ? (over ? 1600 : 1024)
+                                  : (ends_empty ? 1024 : 2000);
+  const bool full = mine == theirs && kDwRowsCus % groups <= (groups <= 12 ? 4 : 1);
   return vc >= walk * (kDwRowsCus / groups) && (kt <= 10 || full);
 }
 

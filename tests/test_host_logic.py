@@ -469,8 +469,8 @@ def test_a_missing_extension_is_built_alone_and_only_when_it_is_asked_for(monkey
 
 def test_which_calls_form_dweight_from_resident_rows():
     """Both sides of each limit of the rule: 768 tokens, hidden 8192, the columns that a part of the vocabulary has (hidden 896:
-    two groups of 512 rows and 128 parts up to 320 tokens, four groups and 64 parts beyond), row tiles that fill 15 of 16
-    wavefronts beyond 640 tokens, a vocabulary that is read as it lies; no half tiles where the rows are resident."""
+    two groups of 512 rows and 128 parts up to 320 tokens, four groups and 64 parts beyond), beyond 640 tokens rows and
+    compute units without waste, a vocabulary that is read as it lies; no half tiles where the rows are resident."""
     from axon_amd import _lib
     ask = _lib.load().axon_lmhead_bwd_dweight_by_rows
     by = lambda n, h, v, chunk=0: ask(n, n, h, v, chunk)  # noqa: E731
@@ -483,14 +483,18 @@ def test_which_calls_form_dweight_from_resident_rows():
     assert by(257, 896, 65536) == 1 and by(257, 896, 65528) == 0
     assert by(321, 896, 65536) == 1 and by(576, 896, 65536) == 1 and by(576, 896, 65528) == 0
     assert by(577, 2880, 21504) == 1 and by(577, 2880, 21496) == 0    # 3072 rows computed for 2944
-    assert by(577, 896, 147456) == 1 and by(640, 896, 147448) == 0    # 1024 for 896
+    assert by(577, 896, 102400) == 1 and by(640, 896, 102392) == 0    # 1024 for 896
     assert by(640, 896, 151936) == 1 and by(641, 896, 151936) == 0 and by(641, 1152, 151936) == 0
-    assert by(641, 512, 262144) == 1 and by(641, 512, 262136) == 0 and by(768, 512, 131072) == 0
+    assert by(641, 512, 256000) == 1 and by(641, 512, 255992) == 0    # 7.8 rounds of tiles
+    assert by(641, 512, 131080) == 1 and by(768, 512, 131072) == 0    # 4.01 and 4
+    assert by(641, 1248, 151936) == 1 and by(641, 1120, 151936) == 0  # 1280 rows computed for 1152
+    assert by(641, 2880, 201088) == 0 and by(641, 1504, 201088) == 1  # 3072 for 2944; 252 of 256 compute units
+    assert by(641, 2560, 201088) == 0 and by(641, 3584, 201088) == 0  # 250; 252, fourteen groups
     assert by(300, 4096, 50257) == 0 and by(300, 224, 151936) == 0  # vocab-major copies of the dlogits
     assert by(700, 4096, 151936, 4096) == 0                          # short chunks of the vocabulary
     assert ask(700, 40000, 4096, 151936, 152064) == 1                # a block shorter than the workspace
     halves = _lib.load().axon_lmhead_bwd_half_tiles
-    assert by(700, 2880, 201088) == 1 and halves(700, 700, 2880, 201088, 0) & 2 == 0
+    assert by(640, 2880, 201088) == 1 and halves(640, 640, 2880, 201088, 0) & 2 == 0
     assert by(769, 2880, 201088) == 0 and halves(769, 769, 2880, 201088, 0) & 2 == 2
     assert by(700, 896, 151936) == 0 and halves(700, 700, 896, 151936, 0) & 2 == 2
     assert ask(0, 0, 640, 8200, 0) < 0 and ask(2, 1, 640, 8200, 0) < 0 and ask(1, 1, 640, 8200, 100) < 0
