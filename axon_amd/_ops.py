@@ -2,7 +2,9 @@
 
 Each function validates on the host, allocates outputs/workspace with torch,
 passes raw device pointers and the current stream to ``libaxon_amd.so`` and
-raises on a non-zero status.  Nothing here computes on the CPU.
+raises on a non-zero status; ``policy_loss``, ``group_advantage``, ``reverse_scan``,
+``sampler_correction_diag``, ``scale_f32`` and a loss's autograd node do so in native
+code (``_lib.native()``, csrc/torch_ext.cpp).  Nothing here computes on the CPU.
 """
 
 from __future__ import annotations

@@ -649,8 +649,8 @@ __device__ __forceinline__ float dlogit_of(float raw, int mrel, const TokenCoef&
   return v;
 }
 
-// f(true_type) where one of the lanes' sixteen tokens has its label among the wavefront's 128 vocabulary rows, one
-// wavefront in a hundred and more; else f(false_type), without the label's two instructions per logit.  Decode of a stash
+// f(true_type) where one of the lanes' sixteen tokens has its label among the wavefront's 128 vocabulary rows (2048 / V of
+// the cases: one in 74 at 151936, one in 16 at 32768); else f(false_type), without the label's two instructions per logit.  Decode of a stash
 // or of kept logits, us, before / after: 300 x 896 x 151936 59.2 / 55.3, 1000 x 4096 x 151936 with an entropy gradient
 // 137.6 / 130.4, 333 x 2880 x 201088 102.3 / 97.5, 6007 x 896 x 151936 (memory-bound) 1056 / 1048.
 template <class F>
@@ -1054,11 +1054,12 @@ __device__ __forceinline__ void store_tile(const GemmOperands& g, const StorePar
   // bf16 rows leave through the wavefront's own 32 KB of LDS, so that a store instruction writes four rows of 256
   // contiguous bytes (whole cache lines) instead of sixteen pieces of 32: the main loop has ended with a barrier, and
   // LDS operations of one wave complete in order.  Two half-waves' reads touch 32 distinct slots each (rows 16
-  // apart, see stage_off).  dWeight of 700 tokens (11 k-tiles; 151936 x 4096 written) 979 us before, 832 with the
-  // staging, 809 with the non-temporal hint on top; long reductions do not notice.  Accumulators are read on their way
-  // out (read_acc): read at the head and written back around the branches below they cost 600 instructions more
-  // (us, before / after: dHidden 1201 x 1024 x 50257 115 / 109.5, 1500 x 2048 x 32768 129 / 124, 6007 x 896 x 151936
-  // 1119 / 1107; dWeight 1201 x 1024 x 50257 133 / 127.5, 6007 x 896 x 151936 1148 / 1138).
+  // apart, see stage_off).  dWeight of 700 tokens in these tiles (11 k-tiles; 151936 x 4096 written, inside a step) 979 us
+  // before, 832 with the staging, 809 with the non-temporal hint on top; long reductions do not notice.  Accumulators are
+  // read on their way out (read_acc): read at the head and written back around the branches below they cost 600
+  // instructions more (us between events, medians of three processes of each, before / after: dHidden 1201 x 1024 x 50257
+  // 138 / 132, 1500 x 2048 x 32768 168 / 164, 6007 x 896 x 151936 1207 / 1193; the dWeight of the same calls 146 / 143, 168 / 166,
+  // 1223 / 1229, within what processes differ).
   char* const stage = smem + lp.wave * 32768;
   const int block = stage_block_base(lp);
   auto to_stage = [&](int i, int j, const f32x4& v) {

@@ -4,8 +4,8 @@
 // A call of such an operator takes the GPU 5 to 20 us and took the host 18 to 30 us in Python, and a Python backward
 // some 40 us more than a native one: the engine's device thread has to get the interpreter lock from the thread that
 // waits for it.  Per call: policy_loss 18 -> 9 us, group_advantage 28 -> 13, reverse_scan 24 -> 7; whole passes
-// (advantage, loss, backward): GRPO + PPO on 128 x 1024 162 -> 98, sampler correction + GSPO on 65536 tokens 232 -> 165, GAE +
-// value loss on 2.1 M tokens 177 -> 121.
+// (advantage, loss, backward), with the sums that the launch sends to the host itself: GRPO + PPO on 128 x 1024 165 -> 94 us,
+// sampler correction + GSPO on 65536 tokens 254 -> 166, correction + PPO on 8.4 M 402 -> 352, GAE + value loss on 2.1 M 176 -> 115.
 //
 // Nothing here computes: the arithmetic is behind axon_amd.h.  The functions take what the Python wrappers of the same
 // names (axon_amd/_ops.py) have normalised, and run without the interpreter lock, as a call through ctypes does.
